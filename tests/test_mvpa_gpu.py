@@ -83,6 +83,23 @@ def test_fp32_generic_shapes(cfg):
     assert (out.cpu().double() - _oracle(inp)).abs().max().item() <= F32_MAX_ABS
 
 
+@pytest.mark.parametrize("cfg", [
+    dict(B=1, C=1, T=1, H=1, Dh=16),                      # one key: seven of the eight waves see none
+    dict(B=1, C=31, T=9, H=2, Dh=32, Hkv=1),              # query blocks and key tiles straddle time steps
+    dict(B=2, C=33, T=2, H=1, Dh=64, validity=True),      # a last key tile of two keys, absent channels
+    dict(B=1, C=150, T=3, H=1, Dh=128),                   # more channels than the bf16 kernels take
+    dict(B=1, C=1, T=1216, H=1, Dh=16),                   # the longest tables the tile kernel holds ...
+    dict(B=1, C=1, T=1217, H=1, Dh=16),                   # ... and one row more: the row-per-lane kernel
+])
+def test_fp32_tile_kernel_edges(cfg):
+    """The fp32 matrix-instruction kernel where its tiles end: fp32 sums against float64."""
+    inp = make_mvpa_inputs(seed=4, **cfg)
+    out, lse = _gpu(inp, torch.float32, return_lse=True)
+    ref, ref_lse = _oracle(inp, return_lse=True)
+    assert (out.cpu().double() - ref).abs().max().item() <= F32_MAX_ABS
+    assert (lse.cpu().double() - ref_lse).abs().max().item() <= 1e-4
+
+
 def test_fp32_flags_and_key_bias():
     inp = make_mvpa_inputs(B=2, C=4, T=15, H=2, Dh=32, seed=4, table_std=0.3)
     d = inp.to("cuda", torch.float32)
