@@ -402,6 +402,71 @@ int mvpa_ring_append_bf16(const void* k_new, const void* v_new, void* k_ring, vo
                           int32_t steps, int64_t stride_b, int64_t stride_h, int64_t stride_c,
                           void* stream);
 
+/* The segment encoder up to its projection in one pass: db4 analysis of fp32 rows x[M,L]
+ * (models/fftencoder.py:80-88), RMSNorm of the coefficients (:93, weight fp32 [dwt_size]) and the
+ * rounding to bf16, y[M,ldy] with columns dwt_size .. ldy-1 set to zero (ldy a multiple of 8, y
+ * 16-byte aligned): coefficients never reach memory in fp32.  Every level's input must hold at
+ * least 8 samples and a row must fit the LDS (L up to about 16000), else MVPA_ERR_UNSUPPORTED. */
+int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64_t M, int32_t L, int32_t levels,
+                             int32_t dwt_size, int64_t ldy, float eps, void* stream);
+
+/* out[g] = mean over its `rows` rows of a group of bf16 rows (fp32 sum, one rounding): the mean over
+ * the channels of the last segment's hidden state (models/mvpformer.py:947-953).  Group g starts at
+ * x + g * group_stride (elements), rows are ldx elements apart; cols a multiple of 8. */
+int mvpa_mean_rows_bf16(const void* x, void* out, int64_t groups, int64_t rows, int32_t cols, int64_t ldx,
+                        int64_t group_stride, void* stream);
+
+/* ---- the stack of parallel blocks as one call ---------------------------------------------------
+ * models/mvpformer.py:296-381: every block x + attn(ln_1(x)) + mlp(ln_1(x)), then ln_f, on bf16 rows.
+ * The launches are the library's own (mvpa_forward and the products around it); one call enqueues
+ * all of them, so that a short window or one step of a stream is not bound by its caller. */
+typedef struct mvpa_stack_block {
+  const void* w_qkv;          /* [E + 2*Hkv*Dh, E] rows of q_attn, then keys, then values         */
+  const void* w_gate_up;      /* [2*inner, E] gate rows, then up rows                             */
+  const void* w_qkv_normed;   /* nullable; the same two with ln_1's weight in their columns (see   */
+  const void* w_gate_up_normed; /* sumsq below)                                                   */
+  const void* w_tail;         /* [E, E + inner]: c_proj | down_proj                               */
+  const float* ln_weight;     /* ln_1, fp32 [E]                                                   */
+  const void* bias_u;         /* as in mvpa_fwd_args                                              */
+  const void* bias_v;
+  const void* bias_z;
+  const void* k_time;         /* [Hkv,T,Dh]                                                       */
+  const void* k_chan;         /* [Hkv,C,Dh]                                                       */
+  const uint8_t* chan_valid;  /* nullable [B,C]                                                   */
+  void* k_cache;              /* a step only: [B][Hkv][steps][C][Dh], the first live step          */
+  void* v_cache;
+  int64_t cache_stride_b, cache_stride_g;   /* elements                                           */
+  float ln_eps, sm_scale;
+  uint32_t flags;             /* MVPA_FLAG_CONTENT | MVPA_FLAG_FP8_QK                             */
+  int32_t window;
+} mvpa_stack_block;
+
+typedef struct mvpa_stack_args {
+  uint32_t struct_size;       /* sizeof(mvpa_stack_args)                                          */
+  int32_t n_blocks;
+  int32_t B, T, C;            /* T: time steps of the keys                                        */
+  int32_t H, Hkv, Dh, E, inner;
+  int32_t step;               /* 0: x, y hold B*T*C rows; 1: B*C rows, one new time step whose keys
+                                 and values are written into the caches (slot T-1 from k_cache, or
+                                 *ring_head) before the attention reads them                      */
+  float lnf_eps;
+  const mvpa_stack_block* blocks;
+  const void* x;              /* [rows, E] bf16, contiguous                                       */
+  void* y;                    /* [rows, E] bf16: ln_f of the last block's output                  */
+  const float* lnf_weight;    /* fp32 [E]                                                         */
+  const float* sumsq;         /* nullable [rows]: sums of squares of x's rows (mvpa_row_sumsq_bf16).
+                                 With it, and with every block's *_normed weights, ln_1 is applied
+                                 in the epilogue of the products; without, by itself              */
+  const int32_t* ring_head;   /* nullable; a step on rings, as MVPA_FLAG_RING                     */
+  void* ws;                   /* mvpa_stack_ws_bytes(args), 256-byte aligned                      */
+  size_t ws_bytes;
+} mvpa_stack_args;
+
+/* MVPA_ERR_UNSUPPORTED for shapes it does not take (E and E + inner multiples of 64, at most 4096
+ * columns; a matrix-core attention shape); ws_bytes is 0 for those. */
+size_t mvpa_stack_ws_bytes(const mvpa_stack_args* args);
+int mvpa_stack_forward(const mvpa_stack_args* args, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -151,9 +151,7 @@ def flash_mvpa(
             k_chan.reshape(kv_heads, chan_ctx, dh), v, bool(causal), sm_scale, int(window_size),
             bool(rel_bias_time), bool(rel_bias_chan), chan_valid)
     return mvpa_hip.mvpa_forward(
-        q, k_glob, v,
-        q_bias.reshape(kv_heads, dh), q_btime.reshape(kv_heads, dh), q_bchan.reshape(kv_heads, dh),
-        k_time.reshape(kv_heads, time_ctx, dh), k_chan.reshape(kv_heads, chan_ctx, dh),
+        q, k_glob, v, q_bias, q_btime, q_bchan, k_time, k_chan,
         sm_scale=sm_scale, window=int(window_size), causal=bool(causal), content=True,
         time_bias=bool(rel_bias_time), chan_bias=bool(rel_bias_chan), chan_valid=chan_valid,
         out=out, kernel=kernel)

@@ -1524,6 +1524,119 @@ __global__ __launch_bounds__(256) void wavedec_db4_kernel(const float* __restric
   for (int k = threadIdx.x; k < n; k += 256) out[row * ldc + k] = cur[k];
 }
 
+// -----------------------------------------------------------------------------------------
+// The encoder up to its projection in one pass: db4 analysis, RMSNorm of the coefficients, bf16.
+// A row's samples, running approximations and coefficients live in LDS; memory sees 4 bytes in per
+// sample and 2 bytes out per coefficient (as three launches through fp32 coefficients: 98 us for
+// 16384 rows of 512, of which the row-per-workgroup analysis with a barrier per level took 72).
+// G threads own a row: one wave for short rows (no workgroup barrier at all), a workgroup for long
+// ones.  Periodic wrap by copies of 8 samples on either side of an approximation, so that the taps of
+// output k are the 8 consecutive samples 2k-6 .. 2k+1 without an index modulo n.
+// -----------------------------------------------------------------------------------------
+template <int G>
+__global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* __restrict__ x,
+                                                                  const float* __restrict__ w,
+                                                                  bf16_t* __restrict__ y, int64_t M, int L,
+                                                                  int levels, int dwt_size, int64_t ldy, float eps,
+                                                                  int row_floats) {
+  extern __shared__ __attribute__((aligned(16))) float wd_lds[];
+  __shared__ float red[4];
+  const int sub = threadIdx.x / G, t = threadIdx.x % G;
+  const int64_t row = (int64_t)blockIdx.x * (256 / G) + sub;
+  if (G == 64 && row >= M) return;                  // (G == 256: one row per workgroup, the grid is M)
+  auto sync = [&]() {
+    if (G == 256) {
+      __syncthreads();
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+  };
+  constexpr int PAD = 8;
+  const int half = (L + 7) / 2;
+  float* cur = wd_lds + sub * row_floats + PAD;     // [PAD | L | PAD]
+  float* nxt = cur + ((L + 2 * PAD + 3) & ~3);      // [PAD | half | PAD]
+  float* coef = nxt + ((half + 2 * PAD + 3) & ~3) - PAD;
+  const float* xr = x + row * L;
+  for (int i = t; i < L; i += G) cur[i] = xr[i];
+  int n = L, tail = dwt_size;
+  float ss = 0.f;
+  for (int lv = 1; lv <= levels; ++lv) {
+    sync();
+    if (t < PAD) {
+      cur[t - PAD] = cur[n + t - PAD];
+      cur[n + t] = cur[t];
+    }
+    sync();
+    const int m = (n + 7) >> 1;
+    tail -= m;
+    for (int k = t; k < m; k += G) {
+      float lo = 0.f, hi = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float v = cur[2 * k + 1 - j];
+        lo += kDb4Lo[j] * v;
+        hi += ((j & 1) ? kDb4Lo[7 - j] : -kDb4Lo[7 - j]) * v;
+      }
+      nxt[k] = lo;
+      coef[tail + k] = hi;
+      ss += hi * hi;
+    }
+    float* sw = cur;
+    cur = nxt;
+    nxt = sw;
+    n = m;
+  }
+  sync();
+  for (int k = t; k < n; k += G) {
+    const float v = cur[k];
+    coef[k] = v;
+    ss += v * v;
+  }
+  ss = wave_sum(ss);
+  if (G == 256) {
+    if ((t & 63) == 0) red[t >> 6] = ss;
+    __syncthreads();
+    ss = red[0] + red[1] + red[2] + red[3];
+  } else {
+    sync();
+  }
+  const float inv = rsqrtf(ss / (float)dwt_size + eps);
+  for (int c = t * 8; c < ldy; c += G * 8) {
+    float v[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = c + i < dwt_size ? coef[c + i] * inv * w[c + i] : 0.f;
+    vec8<bf16_t>::store(y + row * ldy + c, v);
+  }
+}
+
+// Means of groups of rows: a workgroup takes 64 columns of a group, 32 row lanes of 8 columns each.
+__global__ __launch_bounds__(256) void mean_rows_bf16_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ out,
+                                                             int64_t rows, int cols, int64_t ldx, int64_t group_stride) {
+  __shared__ float red[32][65];
+  const int cl = threadIdx.x & 7, rl = threadIdx.x >> 3;
+  const int c = blockIdx.x * 64 + cl * 8;
+  const bf16_t* xg = x + blockIdx.y * group_stride;
+  float s[8] = {};
+  if (c < cols)
+    for (int64_t r = rl; r < rows; r += 32) {
+      float v[8];
+      vec8<bf16_t>::load(xg + r * ldx + c, v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s[i] += v[i];
+    }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) red[rl][cl * 8 + i] = s[i];
+  __syncthreads();
+  if (threadIdx.x < 64 && blockIdx.x * 64 + threadIdx.x < cols) {
+    float v = 0.f;
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v += red[r][threadIdx.x];
+    out[(int64_t)blockIdx.y * cols + blockIdx.x * 64 + threadIdx.x] = f32_to_bf16(v / (float)rows);
+  }
+}
+
 // One new time step of keys and values into the slot *head of two ring buffers
 // [B,Hkv,steps,C,Dh]: k_new / v_new are [B,Hkv,C,Dh] views (element strides sb, sh, sc, unit
 // last stride) of the projection output.  One thread per 16 bytes.
@@ -1959,5 +2072,40 @@ extern "C" int mvpa_wavedec_db4(const float* x, float* coeffs, int64_t M, int32_
     mvpa::want_dynamic_lds((const void*)wavedec_db4_kernel, (int)(2 * L * sizeof(float)));
   MVPA_LAUNCH(wavedec_db4_kernel, dim3((unsigned)M), dim3(256), 2 * L * sizeof(float),
                      (hipStream_t)stream, x, coeffs, L, levels, dwt_size, ldc);
+  return mvpa::take_launch_status();
+}
+
+extern "C" int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64_t M, int32_t L,
+                                        int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream) {
+  if (!x || !weight || !y) return MVPA_ERR_NULL;
+  if (M <= 0 || L < 8 || levels < 1 || ldy < dwt_size) return MVPA_ERR_SHAPE;
+  if ((ldy & 7) || ((uintptr_t)y & 15)) return MVPA_ERR_ALIGN;
+  int n = L, total = 0;
+  for (int lv = 0; lv < levels; ++lv) {
+    if (n < 8) return MVPA_ERR_UNSUPPORTED;
+    n = (n + 7) >> 1;
+    total += n;
+  }
+  if (total + n != dwt_size) return MVPA_ERR_SHAPE;
+  // per row: samples and first approximation with their wrap copies, coefficients
+  const int row_floats = ((L + 16 + 3) & ~3) + (((L + 7) / 2 + 16 + 3) & ~3) + ((dwt_size + 3) & ~3);
+  // one wave per row while four rows leave room for two workgroups per CU
+  const bool wave = row_floats * 4 * 4 <= 80 * 1024;
+  const int lds = row_floats * 4 * (wave ? 4 : 1);
+  if (lds > 156 * 1024) return MVPA_ERR_UNSUPPORTED;
+  auto kern = wave ? wavedec_db4_rmsnorm_kernel<64> : wavedec_db4_rmsnorm_kernel<256>;
+  if (lds > 64 * 1024) mvpa::want_dynamic_lds((const void*)kern, lds);
+  MVPA_LAUNCH(kern, dim3((unsigned)(wave ? (M + 3) / 4 : M)), dim3(256), lds, (hipStream_t)stream, x, weight, (bf16_t*)y,
+              M, L, levels, dwt_size, ldy, eps, row_floats);
+  return mvpa::take_launch_status();
+}
+
+extern "C" int mvpa_mean_rows_bf16(const void* x, void* out, int64_t groups, int64_t rows, int32_t cols, int64_t ldx,
+                                   int64_t group_stride, void* stream) {
+  if (!x || !out) return MVPA_ERR_NULL;
+  if (groups <= 0 || rows <= 0 || cols <= 0 || ldx < cols) return MVPA_ERR_SHAPE;
+  if ((cols & 7) || (ldx & 7) || (group_stride & 7) || ((uintptr_t)x & 15)) return MVPA_ERR_ALIGN;
+  MVPA_LAUNCH(mean_rows_bf16_kernel, dim3((unsigned)((cols + 63) / 64), (unsigned)groups), dim3(256), 0,
+              (hipStream_t)stream, (const bf16_t*)x, (bf16_t*)out, rows, cols, ldx, group_stride);
   return mvpa::take_launch_status();
 }

@@ -1,0 +1,393 @@
+// Python binding of the launch-bound paths: tensors in, launches of libmvpa_hip.so out.
+//
+// A call through ctypes takes apart its tensors in the interpreter, one attribute at a time (about 18 us
+// for the attention operator, and 100 us per block of a stack); here it costs a few.  Nothing is
+// computed in this file: every function fills an argument block of the C ABI (include/mvpa_hip.h),
+// allocates the results with torch's caching allocator and enqueues on torch's current stream.
+// Functions return an int status where the library refused, for the Python layer to raise on.
+#include <ATen/ATen.h>
+#include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/grad_mode.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <cmath>
+#include <cstring>
+#include <string>
+#include <vector>
+
+#include "mvpa_hip.h"
+
+namespace {
+
+using at::Tensor;
+
+void* current_stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
+
+bool is_none(PyObject* o) { return o == nullptr || o == Py_None; }
+
+const Tensor& tensor_of(PyObject* o) {
+  TORCH_CHECK_TYPE(THPVariable_Check(o), "expected a tensor");
+  return THPVariable_Unpack(o);
+}
+
+int dtype_code(at::ScalarType t) {
+  if (t == at::kFloat) return MVPA_F32;
+  if (t == at::kBFloat16) return MVPA_BF16;
+  TORCH_CHECK_TYPE(t == at::kHalf, "libmvpa_hip supports float32, bfloat16 and float16");
+  return MVPA_F16;
+}
+
+void on_gpu(const Tensor& t) {
+  TORCH_CHECK(t.is_cuda(), "libmvpa_hip ops need tensors in GPU memory (there is no CPU path)");
+}
+
+// t itself where it already has the type and is contiguous
+Tensor as_operand(const Tensor& t, at::ScalarType dt) {
+  on_gpu(t);
+  if (t.scalar_type() == dt && t.is_contiguous()) return t;
+  return t.to(dt).contiguous();
+}
+
+// ---- the attention operator -----------------------------------------------------------------
+// forward(q, k, v, u, vb, z, k_time, k_chan, out, chan_valid, key_bias, sm_scale, window, flags,
+//         kernel, return_lse) -> out | (out, lse) | status
+PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 16, "forward takes 16 arguments");
+  const Tensor &q = tensor_of(args[0]), &k = tensor_of(args[1]), &v = tensor_of(args[2]);
+  on_gpu(q);
+  on_gpu(k);
+  on_gpu(v);
+  TORCH_CHECK(q.dim() == 4 && k.dim() == 4 && v.dim() == 4, "q, k and v have four dimensions");
+  const Tensor &kt0 = tensor_of(args[6]), &kc0 = tensor_of(args[7]);
+  TORCH_CHECK(kt0.dim() >= 2 && kc0.dim() >= 2, "k_time and k_chan are [.., T, Dh] and [.., C, Dh]");
+  const int64_t rows = kt0.size(-2) * kc0.size(-2), hkv = k.size(1), dh = q.size(3);
+  auto require = [](bool ok, const char* what) {
+    if (!ok) PyErr_SetString(PyExc_AssertionError, what);
+    return ok;
+  };
+  if (!require(k.size(3) == dh && v.size(3) == dh, "head dims of q, k, v differ") ||
+      !require(k.size(2) == rows && v.size(2) == rows, "k and v must hold T*C rows") ||
+      !require(q.size(2) == rows, "q must hold T*C rows (C with last_step_only)") ||
+      !require(v.size(1) == hkv && k.size(0) == q.size(0) && v.size(0) == q.size(0), "q, k, v disagree on B or Hkv") ||
+      !require(kt0.numel() == hkv * kt0.size(-2) * dh && kc0.numel() == hkv * kc0.size(-2) * dh,
+               "k_time and k_chan must hold Hkv tables of Dh columns"))
+    return nullptr;
+  for (int i = 3; i < 6; ++i)
+    if (!require(tensor_of(args[i]).numel() == hkv * dh, "u, vb, z must hold Hkv rows of Dh")) return nullptr;
+  if (!is_none(args[8])) {
+    const Tensor& o = tensor_of(args[8]);
+    on_gpu(o);
+    if (!require(o.dim() == 4 && o.sizes() == q.sizes() && o.scalar_type() == q.scalar_type(), "out must match q")) return nullptr;
+  }
+  if (!is_none(args[9]) &&
+      !require(tensor_of(args[9]).dim() == 2 && tensor_of(args[9]).size(0) == q.size(0) && tensor_of(args[9]).size(1) == kc0.size(-2),
+               "chan_valid is [B, C]"))
+    return nullptr;
+  if (!is_none(args[10]) &&
+      !require(tensor_of(args[10]).dim() == 2 && tensor_of(args[10]).size(0) == q.size(0) && tensor_of(args[10]).size(1) == rows,
+               "key_bias is [B, N]"))
+    return nullptr;
+  const auto dt = q.scalar_type();
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor u = as_operand(tensor_of(args[3]), dt), vb = as_operand(tensor_of(args[4]), dt),
+               z = as_operand(tensor_of(args[5]), dt), kt = as_operand(tensor_of(args[6]), dt),
+               kc = as_operand(tensor_of(args[7]), dt);
+  mvpa_fwd_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.dtype = dtype_code(dt);
+  a.window = (int32_t)PyLong_AsLong(args[12]);
+  a.flags = (uint32_t)PyLong_AsUnsignedLong(args[13]);
+  a.kernel = (int32_t)PyLong_AsLong(args[14]);
+  a.sm_scale = (float)PyFloat_AsDouble(args[11]);
+  if (PyErr_Occurred()) return nullptr;
+  a.B = (int32_t)q.size(0);
+  a.H = (int32_t)q.size(1);
+  a.Dh = (int32_t)q.size(3);
+  a.Hkv = (int32_t)k.size(1);
+  a.T = (int32_t)kt.size(-2);
+  a.C = (int32_t)kc.size(-2);
+  Tensor out = is_none(args[8]) ? at::empty(q.sizes(), q.options(), at::MemoryFormat::Contiguous) : tensor_of(args[8]);
+  TORCH_CHECK_VALUE(q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1 && out.stride(3) == 1,
+                    "q, k, v, out: last dim must be contiguous");
+  a.q = q.data_ptr();
+  a.k = k.data_ptr();
+  a.v = v.data_ptr();
+  a.o = out.data_ptr();
+  a.q_stride_b = q.stride(0); a.q_stride_h = q.stride(1); a.q_stride_n = q.stride(2);
+  a.k_stride_b = k.stride(0); a.k_stride_h = k.stride(1); a.k_stride_n = k.stride(2);
+  a.v_stride_b = v.stride(0); a.v_stride_h = v.stride(1); a.v_stride_n = v.stride(2);
+  a.o_stride_b = out.stride(0); a.o_stride_h = out.stride(1); a.o_stride_n = out.stride(2);
+  a.bias_u = u.data_ptr();
+  a.bias_v = vb.data_ptr();
+  a.bias_z = z.data_ptr();
+  a.k_time = kt.data_ptr();
+  a.k_chan = kc.data_ptr();
+  Tensor cv, kb, lse;
+  if (!is_none(args[9])) {
+    cv = as_operand(tensor_of(args[9]), tensor_of(args[9]).scalar_type() == at::kBool ? at::kBool : at::kByte);
+    a.chan_valid = (const uint8_t*)cv.data_ptr();
+  }
+  if (!is_none(args[10])) {
+    kb = as_operand(tensor_of(args[10]), at::kFloat);
+    a.key_bias = (const float*)kb.data_ptr();
+  }
+  const bool want_lse = args[15] == Py_True;
+  if (want_lse) {
+    lse = at::empty({q.size(0), q.size(1), q.size(2)}, q.options().dtype(at::kFloat));
+    a.lse = (float*)lse.data_ptr();
+  }
+  const int st = mvpa_forward(&a, current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  if (!want_lse) return THPVariable_Wrap(out);
+  PyObject* r = PyTuple_New(2);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(out));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(lse));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- dense ops ------------------------------------------------------------------------------
+// linear(x, w) -> x @ w^T, bf16, plain product | status
+PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 2, "linear takes x and w");
+  Tensor x = tensor_of(args[0]);
+  const Tensor& w = tensor_of(args[1]);
+  on_gpu(x);
+  on_gpu(w);
+  TORCH_CHECK_TYPE(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16, "linear: bf16 only");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const int64_t K = x.size(-1), N = w.size(0);
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && w.stride(1) == 1, "linear: w is [N, K] with unit last stride");
+  std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
+  shape.back() = N;
+  if (!(x.dim() == 2 && x.stride(1) == 1)) x = x.contiguous();
+  const int64_t M = x.numel() / K, ldx = x.dim() == 2 ? x.stride(0) : K;
+  Tensor y = at::empty(shape, x.options());
+  int st;
+  if (M <= 128 && K >= 1536 && N <= 4096) {
+    Tensor ws = at::empty({(int64_t)mvpa_linear_splitk_ws_bytes(M, N, K, 0)}, x.options().dtype(at::kByte));
+    st = mvpa_linear_bf16_splitk(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, w.stride(0), N, 0,
+                                 ws.data_ptr(), (size_t)ws.numel(), current_stream());
+  } else {
+    st = mvpa_linear_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, ldx, w.stride(0), N, 0, current_stream());
+  }
+  return st == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
+// encode(x [M, L] fp32, norm weight fp32, levels, dwt_size, pitch, eps) -> [M, pitch] bf16 | status
+PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 6, "encode takes 6 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor x = as_operand(tensor_of(args[0]), at::kFloat), w = as_operand(tensor_of(args[1]), at::kFloat);
+  const long levels = PyLong_AsLong(args[2]), dwt = PyLong_AsLong(args[3]), pitch = PyLong_AsLong(args[4]);
+  const double eps = PyFloat_AsDouble(args[5]);
+  if (PyErr_Occurred()) return nullptr;
+  Tensor y = at::empty({x.size(0), pitch}, x.options().dtype(at::kBFloat16));
+  const int st = mvpa_wavedec_db4_rmsnorm((const float*)x.data_ptr(), (const float*)w.data_ptr(), y.data_ptr(), x.size(0),
+                                          (int32_t)x.size(1), (int32_t)levels, (int32_t)dwt, pitch, (float)eps,
+                                          current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
+// mean_rows(x [G, R, E] bf16, unit last stride) -> [G, E] | status
+PyObject* py_mean_rows(PyObject*, PyObject* arg) {
+  HANDLE_TH_ERRORS
+  const Tensor& x = tensor_of(arg);
+  on_gpu(x);
+  TORCH_CHECK(x.dim() == 3 && x.stride(2) == 1 && x.scalar_type() == at::kBFloat16, "mean_rows: bf16 [G, R, E]");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor y = at::empty({x.size(0), x.size(2)}, x.options());
+  const int st = mvpa_mean_rows_bf16(x.data_ptr(), y.data_ptr(), x.size(0), x.size(1), (int32_t)x.size(2), x.stride(1),
+                                     x.stride(0), current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- the stack of blocks ----------------------------------------------------------------------
+// What a model's weights looked like when a plan was made from them: entries of modules' parameter and
+// sub-module tables (identity), and the storages and versions of the tensors found there.
+struct Watch {
+  struct Entry { PyObject *dict, *key, *value; };
+  std::vector<Entry> entries;
+  std::vector<Tensor> tensors;
+  std::vector<std::pair<const void*, uint32_t>> seen;
+
+  bool unchanged() const {
+    for (const auto& e : entries)
+      if (PyDict_GetItem(e.dict, e.key) != e.value) return false;
+    for (size_t i = 0; i < tensors.size(); ++i)
+      if (tensors[i].const_data_ptr() != seen[i].first || tensors[i]._version() != (int64_t)seen[i].second) return false;
+    return true;
+  }
+  ~Watch() {
+    for (auto& e : entries) {
+      Py_DECREF(e.dict);
+      Py_DECREF(e.key);
+      Py_DECREF(e.value);
+    }
+  }
+};
+
+struct Plan {
+  Watch watch;
+  std::vector<Tensor> keep;                  // every operand, alive as long as the plan
+  std::vector<mvpa_stack_block> blocks;
+  std::vector<char> honours_mask;
+  mvpa_stack_args args;
+};
+
+const char* kPlanName = "mvpa_stack_plan";
+
+Plan* plan_of(PyObject* o) { return (Plan*)PyCapsule_GetPointer(o, kPlanName); }
+
+void free_plan(PyObject* o) { delete plan_of(o); }
+
+// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks, watched entries, watched tensors)
+//   a block: (w_qkv, w_gu, w_qkv_normed|None, w_gu_normed|None, w_tail, ln_weight, u, vb, z, k_time, k_chan,
+//             ln_eps, sm_scale, flags, window, honours_mask)
+PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 6, "plan takes 6 arguments");
+  auto plan = std::make_unique<Plan>();
+  mvpa_stack_args& a = plan->args;
+  std::memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  int32_t* dims[7] = {&a.T, &a.C, &a.H, &a.Hkv, &a.Dh, &a.E, &a.inner};
+  for (int i = 0; i < 7; ++i) *dims[i] = (int32_t)PyLong_AsLong(PyTuple_GetItem(args[0], i));
+  auto operand = [&](PyObject* o, at::ScalarType dt) -> const void* {
+    if (is_none(o)) return nullptr;
+    const Tensor& t = tensor_of(o);
+    on_gpu(t);
+    TORCH_CHECK(t.scalar_type() == dt && t.is_contiguous(), "plan: operands are contiguous and of the stack's type");
+    plan->keep.push_back(t);
+    return t.const_data_ptr();
+  };
+  a.lnf_weight = (const float*)operand(args[1], at::kFloat);
+  a.lnf_eps = (float)PyFloat_AsDouble(args[2]);
+  const Py_ssize_t nb = PyList_Size(args[3]);
+  for (Py_ssize_t i = 0; i < nb; ++i) {
+    PyObject* t = PyList_GetItem(args[3], i);
+    mvpa_stack_block b;
+    std::memset(&b, 0, sizeof(b));
+    const void** ops[11] = {&b.w_qkv, &b.w_gate_up, &b.w_qkv_normed, &b.w_gate_up_normed, &b.w_tail,
+                            (const void**)&b.ln_weight, &b.bias_u, &b.bias_v, &b.bias_z, &b.k_time, &b.k_chan};
+    for (int j = 0; j < 11; ++j) *ops[j] = operand(PyTuple_GetItem(t, j), j == 5 ? at::kFloat : at::kBFloat16);
+    b.ln_eps = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 11));
+    b.sm_scale = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 12));
+    b.flags = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GetItem(t, 13));
+    b.window = (int32_t)PyLong_AsLong(PyTuple_GetItem(t, 14));
+    plan->honours_mask.push_back(PyTuple_GetItem(t, 15) == Py_True);
+    plan->blocks.push_back(b);
+  }
+  for (Py_ssize_t i = 0; i < PyList_Size(args[4]); ++i) {
+    PyObject* t = PyList_GetItem(args[4], i);
+    Watch::Entry e{PyTuple_GetItem(t, 0), PyTuple_GetItem(t, 1), PyTuple_GetItem(t, 2)};
+    Py_INCREF(e.dict);
+    Py_INCREF(e.key);
+    Py_INCREF(e.value);
+    plan->watch.entries.push_back(e);
+  }
+  for (Py_ssize_t i = 0; i < PyList_Size(args[5]); ++i) {
+    const Tensor& t = tensor_of(PyList_GetItem(args[5], i));
+    plan->watch.tensors.push_back(t);
+    plan->watch.seen.emplace_back(t.const_data_ptr(), (uint32_t)t._version());
+  }
+  if (PyErr_Occurred()) return nullptr;
+  a.n_blocks = (int32_t)nb;
+  a.blocks = plan->blocks.data();
+  return PyCapsule_New(plan.release(), kPlanName, free_plan);
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_plan_current(PyObject*, PyObject* o) {
+  Plan* p = plan_of(o);
+  if (!p) return nullptr;
+  return PyBool_FromLong(p->watch.unchanged());
+}
+
+// run(plan, x [B, T|1, C, E] bf16 contiguous, chan_valid [B,C]|None, caches|None, ring_head|None, sumsq|None)
+//   caches, one step: (k tensors, v tensors, first live steps), the tensors [B,Hkv,steps,C,Dh] contiguous;
+//   returns the normed output, shaped like x | status
+PyObject* py_run(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 6, "run takes 6 arguments");
+  Plan* p = plan_of(args[0]);
+  if (!p) return nullptr;
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor x = as_operand(tensor_of(args[1]), at::kBFloat16);
+  mvpa_stack_args& a = p->args;
+  TORCH_CHECK(x.dim() == 4 && x.size(3) == a.E && x.size(2) == a.C, "run: x is [B, T, C, E]");
+  a.B = (int32_t)x.size(0);
+  a.step = is_none(args[3]) ? 0 : 1;
+  TORCH_CHECK(x.size(1) == (a.step ? 1 : a.T), "run: x and the plan disagree on T");
+  Tensor cv;
+  if (!is_none(args[2])) cv = as_operand(tensor_of(args[2]), at::kBool);
+  for (size_t i = 0; i < p->blocks.size(); ++i)
+    p->blocks[i].chan_valid = cv.defined() && p->honours_mask[i] ? (const uint8_t*)cv.const_data_ptr() : nullptr;
+  a.ring_head = nullptr;
+  if (a.step) {
+    PyObject *ks = PyTuple_GetItem(args[3], 0), *vs = PyTuple_GetItem(args[3], 1), *st = PyTuple_GetItem(args[3], 2);
+    TORCH_CHECK(ks && vs && st && PyList_Size(ks) == (Py_ssize_t)p->blocks.size(), "run: one cache per block");
+    for (size_t i = 0; i < p->blocks.size(); ++i) {
+      const Tensor &k = tensor_of(PyList_GetItem(ks, i)), &v = tensor_of(PyList_GetItem(vs, i));
+      const int64_t first = PyLong_AsLong(PyList_GetItem(st, i));
+      TORCH_CHECK(k.dim() == 5 && k.sizes() == v.sizes() && k.is_contiguous() && v.is_contiguous() &&
+                      k.scalar_type() == at::kBFloat16 && v.scalar_type() == at::kBFloat16 && k.size(0) == a.B &&
+                      k.size(1) == a.Hkv && k.size(3) == a.C && k.size(4) == a.Dh && first >= 0 &&
+                      first + a.T <= k.size(2),
+                  "run: caches are contiguous bf16 [B, Hkv, steps, C, Dh] with room for the step");
+      mvpa_stack_block& b = p->blocks[i];
+      const int64_t slot = (int64_t)a.C * a.Dh;
+      b.k_cache = (char*)k.data_ptr() + first * slot * 2;
+      b.v_cache = (char*)v.data_ptr() + first * slot * 2;
+      b.cache_stride_b = k.stride(0);
+      b.cache_stride_g = k.stride(1);
+    }
+    if (!is_none(args[4])) {
+      const Tensor& h = tensor_of(args[4]);
+      TORCH_CHECK(h.is_cuda() && h.scalar_type() == at::kInt && h.numel() == 1, "run: ring_head is one int32 on the GPU");
+      a.ring_head = (const int32_t*)h.data_ptr();
+    }
+  }
+  a.sumsq = nullptr;
+  if (!is_none(args[5])) {
+    const Tensor& ss = tensor_of(args[5]);
+    TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.is_contiguous() && ss.numel() * a.E == x.numel(),
+                "run: sumsq holds one fp32 value per row");
+    a.sumsq = (const float*)ss.data_ptr();
+  }
+  Tensor y = at::empty(x.sizes(), x.options());
+  const int64_t bytes = (int64_t)mvpa_stack_ws_bytes(&a);
+  if (bytes == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+  a.x = x.data_ptr();
+  a.y = y.data_ptr();
+  a.ws = ws.data_ptr();
+  a.ws_bytes = (size_t)bytes;
+  const int status = mvpa_stack_forward(&a, current_stream());
+  return status == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(status);
+  END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef kMethods[] = {
+    {"forward", (PyCFunction)(void*)py_forward, METH_FASTCALL, "fused MVPA forward"},
+    {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
+    {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
+    {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
+    {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
+    {"plan_current", (PyCFunction)py_plan_current, METH_O, "whether the weights a plan was made from are unchanged"},
+    {"run", (PyCFunction)(void*)py_run, METH_FASTCALL, "a stack of blocks on one plan"},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_mvpa_ext", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__mvpa_ext(void) { return PyModule_Create(&kModule); }

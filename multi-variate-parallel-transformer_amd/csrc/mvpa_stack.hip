@@ -1,0 +1,241 @@
+// The stack of parallel blocks as one call: a host-side sequence of the library's launches.
+//
+// A block is four or five short launches; driven one by one from the caller's language a window of 525
+// rows or one step of a stream is bound by that caller (1.2 ms of host time for twelve blocks), not
+// by the GPU.  Three sequences, by the number of rows:
+//   many rows      [q/k/v | gate/up] on raw rows with ln_1 in the epilogue -> attention -> tail product
+//                  with residual and the next norm's row statistics (mvpa_dense.hip, 256-row tiles)
+//   few rows       [q/k/v | gate/up] on small tiles, of raw rows (ln_1 in the epilogue) or of normed ones ->
+//                  attention -> split-K tail -> sum + residual + the row statistics or the normed rows
+//                  that the next block wants (mvpa_tiles.hip)
+//   a step         the latter with the new keys and values written straight into the caches by the
+//                  product's epilogue, and the attention of the last time step only
+#include "mvpa_mfma_tools.h"
+#include "mvpa_tiles.h"
+
+namespace mvpa {
+
+// The 256-row tiles are the better ones once [q/k/v | gate/up] is this many of them, about a round and
+// a half of the chip (us per block, 256-row against small tiles: a model of 768 columns at
+// 1600 / 3200 / 4096 rows 105 : 68, 126 : 130, 150 : 173; of 2048 columns at 1024 / 1536 / 2048 rows
+// 258 : 203, 313 : 295, 331 : 361).
+constexpr int64_t kManyTiles = 352;
+
+static int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }
+
+struct stack_ws {
+  char* base;
+  int64_t used;
+  void* take(int64_t bytes) {
+    void* p = base ? base + used : nullptr;
+    used += up256(bytes);
+    return p;
+  }
+};
+
+struct stack_plan {
+  bool many, raw;                      // 256-row tiles; ln_1 inside the products
+  int64_t rows;
+  tile_split split_k;
+  int runs;
+  bf16_t *qkv, *both, *hidden[2], *normed;
+  float *partial, *sumsq[2];
+  float *q_scale, *k_scale;
+  void *k_fp8, *split;
+  int32_t parts;
+};
+
+static bool stack_supported(const mvpa_stack_args* a) {
+  if (a->E != a->H * a->Dh || a->E % 64 || a->inner <= 0 || a->inner % 64 || a->E > 4096) return false;
+  if (a->Dh != 32 && a->Dh != 64 && a->Dh != 128) return false;
+  if (a->C > 128) return false;
+  const int64_t nw = (int64_t)a->E + 2 * a->Hkv * a->Dh;
+  const int64_t widest = 2 * (int64_t)a->inner > nw ? 2 * (int64_t)a->inner : nw;
+  if (widest * a->E >= ((int64_t)1 << 30) || (int64_t)a->E * (a->E + a->inner) >= ((int64_t)1 << 30)) return false;
+  return true;
+}
+
+static int default_runs(const mvpa_stack_args* a) {      // key runs of a step: see default_key_splits
+  int n = 256 / (a->B * a->H);
+  if (n > a->T / 8) n = a->T / 8;
+  if (n < 1) n = 1;
+  while (n > 1 && (int64_t)(n - 1) * ((a->T + n - 1) / n) >= a->T) --n;
+  return n;
+}
+
+static void stack_layout(const mvpa_stack_args* a, stack_plan& p, stack_ws& w) {
+  const int64_t E = a->E, kv = (int64_t)a->Hkv * a->Dh, inner = a->inner;
+  p.rows = (int64_t)a->B * a->C * (a->step ? 1 : a->T);
+  p.raw = !a->step && a->sumsq;
+  for (int i = 0; i < a->n_blocks; ++i) p.raw = p.raw && a->blocks[i].w_qkv_normed && a->blocks[i].w_gate_up_normed;
+  const int64_t tiles = (p.rows + 255) / 256 * ((inner + 127) / 128 + (E + 2 * kv + 255) / 256);
+  p.many = p.raw && p.rows >= 512 && tiles >= kManyTiles && E >= 128;
+  p.qkv = (bf16_t*)w.take(p.rows * (a->step ? E : E + 2 * kv) * 2);
+  p.both = (bf16_t*)w.take(p.rows * (E + inner) * 2);
+  p.hidden[0] = (bf16_t*)w.take(p.rows * E * 2);
+  p.hidden[1] = p.normed = nullptr;
+  p.sumsq[0] = p.sumsq[1] = nullptr;
+  p.partial = nullptr;
+  if (p.many) {
+    p.hidden[1] = (bf16_t*)w.take(p.rows * E * 2);
+    p.parts = mvpa_linear_sumsq_parts(p.rows, E);
+    for (int i = 0; i < 2; ++i) p.sumsq[i] = (float*)w.take(p.rows * p.parts * 4);
+  } else {
+    if (p.raw) p.sumsq[0] = (float*)w.take(p.rows * 4);
+    else p.normed = (bf16_t*)w.take(p.rows * E * 2);
+    p.split_k = make_tile_split(p.rows, E, E + inner, p.raw ? 0 : E);
+    p.partial = (float*)w.take((int64_t)p.split_k.total() * p.rows * E * 4);
+  }
+  p.runs = 1;
+  p.split = nullptr;
+  if (a->step) {
+    p.runs = default_runs(a);
+    if (p.runs > 1) p.split = w.take((int64_t)p.runs * a->B * a->H * a->C * (a->Dh * 2 + 4));
+  }
+  p.q_scale = p.k_scale = nullptr;
+  p.k_fp8 = nullptr;
+  bool fp8 = false;
+  for (int i = 0; i < a->n_blocks; ++i) fp8 |= (a->blocks[i].flags & MVPA_FLAG_FP8_QK) != 0;
+  if (fp8) {
+    p.q_scale = (float*)w.take(a->H * 4);
+    p.k_scale = (float*)w.take(a->Hkv * 4);
+    if (!a->step && a->C > 32 && (a->Dh == 64 || a->Dh == 128)) p.k_fp8 = w.take((int64_t)a->B * a->T * a->C * kv);
+  }
+}
+
+static int stack_check(const mvpa_stack_args* a) {
+  if (!a) return MVPA_ERR_NULL;
+  if (a->struct_size != sizeof(mvpa_stack_args)) return MVPA_ERR_STRUCT;
+  if (a->n_blocks <= 0 || a->B <= 0 || a->H <= 0 || a->Hkv <= 0 || a->E <= 0) return MVPA_ERR_SHAPE;
+  if (a->T <= 0 || a->C <= 0) return MVPA_ERR_CTX;
+  if (a->H % a->Hkv) return MVPA_ERR_HEAD_RATIO;
+  if (!a->blocks) return MVPA_ERR_NULL;
+  return stack_supported(a) ? MVPA_OK : MVPA_ERR_UNSUPPORTED;
+}
+
+}  // namespace mvpa
+
+using namespace mvpa;
+
+extern "C" size_t mvpa_stack_ws_bytes(const mvpa_stack_args* a) {
+  if (stack_check(a) != MVPA_OK) return 0;
+  stack_plan p;
+  stack_ws w{nullptr, 0};
+  stack_layout(a, p, w);
+  return (size_t)w.used;
+}
+
+extern "C" int mvpa_stack_forward(const mvpa_stack_args* a, void* stream) {
+  int st = stack_check(a);
+  if (st != MVPA_OK) return st;
+  if (!a->x || !a->y || !a->lnf_weight || !a->ws) return MVPA_ERR_NULL;
+  if (((uintptr_t)a->ws & 255) || ((uintptr_t)a->x & 15) || ((uintptr_t)a->y & 15)) return MVPA_ERR_ALIGN;
+  stack_plan p;
+  stack_ws w{(char*)a->ws, 0};
+  stack_layout(a, p, w);
+  if ((size_t)w.used > a->ws_bytes) return MVPA_ERR_WS_SIZE;
+  hipStream_t s = (hipStream_t)stream;
+  const int64_t E = a->E, kv = (int64_t)a->Hkv * a->Dh, inner = a->inner, wide = E + inner, nw = E + 2 * kv;
+  const int64_t n = a->step ? a->C : (int64_t)a->T * a->C;
+
+  // the attention of a block, from p.qkv (and the caches) to the first E columns of p.both
+  auto attend = [&](const mvpa_stack_block& blk) -> int {
+    mvpa_fwd_args f = {};
+    f.struct_size = sizeof(f);
+    f.dtype = MVPA_BF16;
+    f.kernel = MVPA_KERNEL_AUTO;
+    f.flags = MVPA_FLAG_CAUSAL | MVPA_FLAG_TIME_BIAS | MVPA_FLAG_CHAN_BIAS |
+              (blk.flags & (MVPA_FLAG_CONTENT | MVPA_FLAG_FP8_QK));
+    f.B = a->B; f.H = a->H; f.Hkv = a->Hkv; f.T = a->T; f.C = a->C; f.Dh = a->Dh;
+    f.window = blk.window;
+    f.sm_scale = blk.sm_scale;
+    const int64_t row = a->step ? E : nw;
+    f.q = p.qkv;
+    f.q_stride_b = n * row; f.q_stride_h = a->Dh; f.q_stride_n = row;
+    if (a->step) {
+      f.flags |= MVPA_FLAG_LAST_STEP | (a->ring_head ? MVPA_FLAG_RING : 0);
+      f.ring_head = a->ring_head;
+      f.k = blk.k_cache;
+      f.v = blk.v_cache;
+      f.k_stride_b = f.v_stride_b = blk.cache_stride_b;
+      f.k_stride_h = f.v_stride_h = blk.cache_stride_g;
+      f.k_stride_n = f.v_stride_n = a->Dh;
+    } else {
+      f.k = p.qkv + E;
+      f.v = p.qkv + E + kv;
+      f.k_stride_b = f.v_stride_b = n * row;
+      f.k_stride_h = f.v_stride_h = a->Dh;
+      f.k_stride_n = f.v_stride_n = row;
+    }
+    f.o = p.both;
+    f.o_stride_b = n * wide; f.o_stride_h = a->Dh; f.o_stride_n = wide;
+    f.bias_u = blk.bias_u; f.bias_v = blk.bias_v; f.bias_z = blk.bias_z;
+    f.k_time = blk.k_time; f.k_chan = blk.k_chan;
+    f.chan_valid = blk.chan_valid;
+    if (f.flags & MVPA_FLAG_FP8_QK) {
+      f.fp8_q_scale = p.q_scale;
+      f.fp8_k_scale = p.k_scale;
+      f.k_fp8 = p.k_fp8;
+      const int e = mvpa_fp8_prepare(&f, p.q_scale, p.k_scale, p.k_fp8, stream);
+      if (e != MVPA_OK) return e;
+    }
+    if (a->step && p.runs > 1) {
+      f.n_split = p.runs;
+      f.split_ws = p.split;
+    }
+    return mvpa_forward(&f, stream);
+  };
+
+  const bf16_t* x = (const bf16_t*)a->x;
+  if (p.many) {
+    const float* ss = a->sumsq;
+    int32_t parts = 1;
+    for (int i = 0; i < a->n_blocks; ++i) {
+      const mvpa_stack_block& blk = a->blocks[i];
+      if ((st = mvpa_linear_bf16_dual_normed(x, blk.w_qkv_normed, p.qkv, blk.w_gate_up_normed, p.both + E, p.rows, nw,
+                                             inner, E, E, E, nw, E, wide, ss, parts, blk.ln_eps,
+                                             stream)) != MVPA_OK) return st;
+      if ((st = attend(blk)) != MVPA_OK) return st;
+      bf16_t* out = p.hidden[i & 1];
+      if ((st = mvpa_linear_bf16_residual_sumsq(p.both, blk.w_tail, x, out, p.sumsq[(i + 1) & 1], p.rows, E, wide, wide,
+                                                wide, E, E, stream)) != MVPA_OK) return st;
+      ss = p.sumsq[(i + 1) & 1];
+      parts = p.parts;
+      x = out;
+    }
+    return mvpa_rmsnorm(x, a->lnf_weight, a->y, p.rows, (int32_t)E, E, E, a->lnf_eps, MVPA_BF16, MVPA_BF16, stream);
+  }
+
+  if (!p.raw && (st = mvpa_rmsnorm(x, a->blocks[0].ln_weight, p.normed, p.rows, (int32_t)E, E, E, a->blocks[0].ln_eps, MVPA_BF16,
+                         MVPA_BF16, stream)) != MVPA_OK) return st;
+  for (int i = 0; i < a->n_blocks; ++i) {
+    const mvpa_stack_block& blk = a->blocks[i];
+    tile_out out = {};
+    out.y = p.qkv;
+    out.ldy = a->step ? E : nw;
+    out.n_y = (int32_t)(a->step ? E : nw);
+    if (a->step) {
+      out.n_kv = (int32_t)kv;
+      out.Dh = a->Dh;
+      out.C = a->C;
+      out.k = (bf16_t*)blk.k_cache;
+      out.v = (bf16_t*)blk.v_cache;
+      out.stride_b = blk.cache_stride_b;
+      out.stride_g = blk.cache_stride_g;
+      out.slot = a->T - 1;
+      out.head = a->ring_head;
+    }
+    const tile_gated gated{(const bf16_t*)(p.raw ? blk.w_gate_up_normed : blk.w_gate_up), p.both + E, E, wide, (int32_t)inner};
+    const tile_norm norm{p.raw ? (i ? p.sumsq[0] : a->sumsq) : nullptr, 1, blk.ln_eps};
+    if ((st = launch_tile_dual(p.raw ? x : p.normed, p.rows, E, E, (const bf16_t*)(p.raw ? blk.w_qkv_normed : blk.w_qkv), nw,
+                               E, out, gated, norm, s)) != MVPA_OK) return st;
+    if ((st = attend(blk)) != MVPA_OK) return st;
+    if ((st = launch_tile_partial(p.both, p.rows, wide, wide, (const bf16_t*)blk.w_tail, E, wide, p.partial, p.split_k, s)) != MVPA_OK) return st;
+    const bool last = i + 1 == a->n_blocks;
+    if ((st = launch_tail_reduce(p.partial, p.split_k, x, p.hidden[0], last ? (bf16_t*)a->y : p.normed,
+                                 last ? a->lnf_weight : a->blocks[i + 1].ln_weight, last ? a->lnf_eps : a->blocks[i + 1].ln_eps,
+                                 p.raw && !last ? p.sumsq[0] : nullptr, p.rows, E, s)) != MVPA_OK) return st;
+    x = p.hidden[0];
+  }
+  return MVPA_OK;
+}

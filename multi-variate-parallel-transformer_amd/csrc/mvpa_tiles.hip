@@ -1,0 +1,369 @@
+// Small-tile bf16 GEMM (y = x w^T): products whose x has few rows.
+//
+// The 256-row tiles of mvpa_dense.hip give such a product a handful of workgroups (525 rows x 768
+// columns: 18 of them on 256 CUs, 50 us for 2 GFLOP).  Here a workgroup is 32 * WM rows of x by 64 rows
+// of w, and a product with a long contraction and a narrow output is split over K as well.  The
+// time of such a product is the latency of its chain of k-blocks, so the operands come through a ring
+// of STAGES direct-to-LDS blocks of 64: STAGES - 1 blocks are in flight at any time.
+//   4 waves.  WM = 4: a wave owns 32 rows of x and all 64 columns.  WM = 2 / 1: two / four waves share
+//   the rows and take 32 / 16 of every 64 k each; their sums meet in LDS at the end, so that a wave
+//   always holds two 32 x 32 tiles (for the gated product: the gate and the up columns of an output).
+//   Rows are 128 bytes with the 16-byte chunks XOR-swizzled as in mvpa_dense.hip.
+#include "mvpa_tiles.h"
+
+#include "mvpa_mfma_tools.h"
+
+namespace mvpa {
+
+constexpr int TL_BN = 64, TL_BK = 64, TL_ROWB = TL_BK * 2;
+
+template <int WM, int STAGES>
+struct tile_cfg {
+  static constexpr int BM = 32 * WM, KH = 4 / WM, LPW = WM + 2;      // 1 KiB loads per wave and block
+  static constexpr int STAGE = (BM + TL_BN) * TL_ROWB;
+  static constexpr int LDS = STAGES * STAGE;
+  static_assert((KH - 1) * WM * 8192 <= LDS, "the sums of the k-parts fit the ring");
+};
+
+// acc[j] = rows 32j.. of the w tile times the wave's 32 rows of x, k-blocks [kb0, kb1); complete in the
+// waves of k-part 0 only.  wrow(r): which row of W feeds row r of the tile.
+template <int WM, int STAGES, typename WRow>
+__device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* __restrict__ X, int64_t ldx, int64_t m0,
+                                             int64_t M, const bf16_t* __restrict__ W, int64_t ldw, WRow wrow,
+                                             int kb0, int kb1, f32x16 (&acc)[2]) {
+  using G = tile_cfg<WM, STAGES>;
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, kh = wave / WM;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))lds;
+
+  // load i of a wave: rows (wave + 4i) * 8 .. + 7 of the block, x rows first (i < WM), then w rows
+  uint32_t off[G::LPW];
+  {
+    const int rsub = lane >> 3, phys = lane & 7;
+#pragma unroll
+    for (int i = 0; i < G::LPW; ++i) {
+      const int row = (wave + 4 * i) * 8 + rsub;
+      const int chunk = (phys ^ ((row >> 1) & 7)) << 3;
+      if (i < WM) {
+        const int64_t m = m0 + row;
+        off[i] = (uint32_t)((((m < M ? m : M - 1) - m0) * ldx + chunk) * 2);
+      } else {
+        off[i] = (uint32_t)((wrow(row - G::BM) * ldw + chunk) * 2);
+      }
+    }
+  }
+  const bf16_t* xs = X + m0 * ldx + (int64_t)kb0 * TL_BK;
+  const bf16_t* ws = W + (int64_t)kb0 * TL_BK;
+  uint32_t dst = lds0;
+  auto issue = [&]() {
+#pragma unroll
+    for (int i = 0; i < G::LPW; ++i)
+      load_to_lds_16(i < WM ? (const void*)xs : (const void*)ws, off[i], dst + (wave + 4 * i) * 1024);
+    xs += TL_BK;
+    ws += TL_BK;
+    dst = dst + G::STAGE == lds0 + G::LDS ? lds0 : dst + G::STAGE;
+  };
+
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
+  const int nkb = kb1 - kb0;
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nkb) issue();
+
+  constexpr int SL = 4 / G::KH;                     // 16-wide k-slices of a block per wave
+  int frag[SL];
+#pragma unroll
+  for (int s = 0; s < SL; ++s) frag[s] = ln * TL_ROWB + (((2 * (kh * SL + s) + hh) ^ ((ln >> 1) & 7)) << 4);
+  const unsigned char* st = lds;
+  for (int kb = 0; kb < nkb; ++kb) {
+    // block kb has landed once only the loads of the younger blocks are still out
+    const int younger = min(STAGES - 2, nkb - 1 - kb);
+    if (younger == STAGES - 2) wait_vmcnt_imm<(STAGES - 2) * G::LPW>();
+    else if (STAGES > 3 && younger == STAGES - 3) wait_vmcnt_imm<(STAGES > 3 ? STAGES - 3 : 0) * G::LPW>();
+    else if (STAGES > 4 && younger == STAGES - 4) wait_vmcnt_imm<(STAGES > 4 ? STAGES - 4 : 0) * G::LPW>();
+    else if (STAGES > 5 && younger == STAGES - 5) wait_vmcnt_imm<(STAGES > 5 ? STAGES - 5 : 0) * G::LPW>();
+    else wait_vmcnt_imm<0>();
+    lds_barrier();                                  // ... for every wave; and block kb - 1 is read by all
+    if (kb + STAGES - 1 < nkb) issue();
+    const unsigned char* xb = st + wm * 32 * TL_ROWB;
+    const unsigned char* wb = st + G::BM * TL_ROWB;
+    bf16x8 xf[SL], wf[SL][2];
+#pragma unroll
+    for (int s = 0; s < SL; ++s) {
+      xf[s] = *(const bf16x8*)(xb + frag[s]);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) wf[s][j] = *(const bf16x8*)(wb + j * 32 * TL_ROWB + frag[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < SL; ++s)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s], acc[j], 0, 0, 0);
+    st = st + G::STAGE == lds + G::LDS ? lds : st + G::STAGE;
+  }
+  if (G::KH > 1) {
+    lds_barrier();
+    float* red = (float*)lds + lane;
+    if (kh > 0) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[((((kh - 1) * WM + wm) * 2 + j) * 16 + r) * 64] = acc[j][r];
+    }
+    lds_barrier();
+    if (kh == 0) {
+#pragma unroll
+      for (int p = 0; p < G::KH - 1; ++p)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) acc[j][r] += red[(((p * WM + wm) * 2 + j) * 16 + r) * 64];
+    }
+  }
+}
+
+__device__ inline void store_quad(bf16_t* p, float a, float b, float c, float d) {
+  bf16x4 o = {(__bf16)a, (__bf16)b, (__bf16)c, (__bf16)d};
+  *(bf16x4*)p = o;
+}
+
+// Workgroup id -> (column tile, row tile): ids equal mod 8 share an XCD and its L2; the row tiles of a
+// column tile are neighbours there, so the panel of w enters one L2 once.
+__device__ inline bool tile_coords(int id, int ct, int mt, int& col, int& row) {
+  const int xcd = id & 7, s = id >> 3;
+  col = (s / mt) * 8 + xcd;
+  row = s % mt;
+  return col < ct;
+}
+
+template <int WM, int STAGES>
+__global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+                                                        const bf16_t* __restrict__ W0, int N0, int64_t ldw0,
+                                                        tile_out out, tile_gated gt, tile_norm nrm, int gated_ct,
+                                                        int ct, int mt) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
+  int col, row;
+  if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
+  const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t m0 = (int64_t)row * 32 * WM;
+  const int64_t m = m0 + (wave % WM) * 32 + ln;
+  f32x16 acc[2];
+  float rn = 1.f;                                   // this lane's row factor
+  if (nrm.ss) {
+    const float* pp = nrm.ss + min(m, M - 1) * nrm.parts;
+    float ss = 0.f;
+    for (int p = 0; p < nrm.parts; ++p) ss += pp[p];
+    rn = rsqrtf(ss / (float)K + nrm.eps);
+  }
+  if (col < gated_ct) {
+    const int n0 = col * 32, N = gt.N;
+    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, gt.w, gt.ldw,
+                             [&](int r) { return (int64_t)((r >> 5) * N + min(n0 + (r & 31), N - 1)); }, 0, K / TL_BK, acc);
+    if (wave >= WM || m >= M) return;
+#pragma unroll
+    for (int a4 = 0; a4 < 4; ++a4) {
+      const int n = n0 + a4 * 8 + hh * 4;
+      if (n >= N) continue;
+      float o[4];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float g = acc[0][a4 * 4 + r] * rn;
+        o[r] = g / (1.f + __expf(-g)) * (acc[1][a4 * 4 + r] * rn);
+      }
+      store_quad(gt.y + m * gt.ldy + n, o[0], o[1], o[2], o[3]);
+    }
+    return;
+  }
+  const int n0 = (col - gated_ct) * TL_BN;
+  tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W0, ldw0, [&](int r) { return (int64_t)min(n0 + r, N0 - 1); }, 0,
+                           K / TL_BK, acc);
+  if (wave >= WM || m >= M) return;
+  const int slot = out.k ? (out.head ? *out.head : out.slot) : 0;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int a4 = 0; a4 < 4; ++a4) {
+      const int n = n0 + j * 32 + a4 * 8 + hh * 4;
+      if (n >= N0) continue;
+      bf16_t* dst;
+      if (n < out.n_y) {
+        dst = out.y + m * out.ldy + n;
+      } else {
+        const int i = n - out.n_y, is_v = i >= out.n_kv, e = is_v ? i - out.n_kv : i;
+        const int g = e / out.Dh, d = e - g * out.Dh;
+        const int b = (int)m / out.C, c = (int)m - b * out.C;
+        dst = (is_v ? out.v : out.k) + b * out.stride_b + g * out.stride_g + ((int64_t)slot * out.C + c) * out.Dh + d;
+      }
+      store_quad(dst, acc[j][a4 * 4] * rn, acc[j][a4 * 4 + 1] * rn, acc[j][a4 * 4 + 2] * rn, acc[j][a4 * 4 + 3] * rn);
+    }
+}
+
+template <int WM, int STAGES>
+__global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+                                                           const bf16_t* __restrict__ W, int N, int64_t ldw,
+                                                           float* __restrict__ P, tile_split sp, int ct, int mt) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
+  int cz, row;
+  const int splits = sp.a + sp.b;
+  if (!tile_coords(blockIdx.x, ct * splits, mt, cz, row)) return;
+  const int col = cz / splits, z = cz - col * splits;
+  const int kb0 = z < sp.a ? z * sp.per_a : sp.nkb_a + (z - sp.a) * sp.per_b;
+  const int kb1 = z < sp.a ? min(kb0 + sp.per_a, sp.nkb_a) : min(kb0 + sp.per_b, K / TL_BK);
+  const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t m0 = (int64_t)row * 32 * WM;
+  const int64_t m = m0 + (wave % WM) * 32 + ln;
+  const int n0 = col * TL_BN;
+  f32x16 acc[2];
+  tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0,
+                           kb1, acc);
+  if (wave >= WM || m >= M) return;
+  float* prow = P + ((int64_t)z * M + m) * N;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int a4 = 0; a4 < 4; ++a4) {
+      const int n = n0 + j * 32 + a4 * 8 + hh * 4;
+      if (n < N)
+        *(float4*)(prow + n) = make_float4(acc[j][a4 * 4], acc[j][a4 * 4 + 1], acc[j][a4 * 4 + 2], acc[j][a4 * 4 + 3]);
+    }
+}
+
+// One workgroup per row: the partial sums of a split-K tail product, the residual, one rounding, and
+// the RMSNorm that the next product wants, while the row is in registers (8 columns per lane and chunk).
+template <int CHUNKS>
+__global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restrict__ P, int split_a, int split_b,
+                                                          const bf16_t* __restrict__ R, bf16_t* __restrict__ S,
+                                                          bf16_t* __restrict__ Y, const float* __restrict__ w,
+                                                          float eps, float* __restrict__ ss_out, int64_t M, int N) {
+  __shared__ float red[4];
+  const int64_t m = blockIdx.x;
+  float v[CHUNKS][8], ss = 0.f;
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int n = (c * 256 + threadIdx.x) * 8;
+    if (n < N) {
+      const u32x4 rr = *(const u32x4*)(R + m * N + n);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        v[c][2 * i] = __uint_as_float(rr[i] << 16);
+        v[c][2 * i + 1] = __uint_as_float(rr[i] & 0xffff0000u);
+      }
+      auto add_part = [&](int z0, int z1) {
+        float s[8] = {};
+        for (int z = z0; z < z1; ++z) {
+          const float* p = P + ((int64_t)z * M + m) * N + n;
+          const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
+          s[0] += a.x; s[1] += a.y; s[2] += a.z; s[3] += a.w;
+          s[4] += b.x; s[5] += b.y; s[6] += b.z; s[7] += b.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[c][i] += (float)(__bf16)s[i];
+      };
+      add_part(split_a, split_a + split_b);
+      if (split_a) add_part(0, split_a);
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        o[i] = (__bf16)v[c][i];
+        v[c][i] = (float)o[i];
+        ss += v[c][i] * v[c][i];
+      }
+      *(bf16x8*)(S + m * N + n) = o;
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const float tot = red[0] + red[1] + red[2] + red[3];
+  if (ss_out && threadIdx.x == 0) ss_out[m] = tot;
+  if (!Y) return;
+  const float inv = rsqrtf(tot / (float)N + eps);
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {
+    const int n = (c * 256 + threadIdx.x) * 8;
+    if (n < N) {
+      const float4 a = *(const float4*)(w + n), b = *(const float4*)(w + n + 4);
+      const float g[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      bf16x8 o;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = (__bf16)(v[c][i] * inv * g[i]);
+      *(bf16x8*)(Y + m * N + n) = o;
+    }
+  }
+}
+
+template <int WM, int STAGES>
+static int launch_dual_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,
+                         const tile_out& out, const tile_gated& gated, const tile_norm& norm, hipStream_t s) {
+  using G = tile_cfg<WM, STAGES>;
+  auto kern = tile_dual_kernel<WM, STAGES>;
+  want_dynamic_lds((const void*)kern, G::LDS);
+  const int gct = gated.w ? (gated.N + 31) / 32 : 0;
+  const int ct = gct + (w0 ? (int)((N0 + TL_BN - 1) / TL_BN) : 0), mt = (int)((M + G::BM - 1) / G::BM);
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w0, (int)N0, ldw0,
+              out, gated, norm, gct, ct, mt);
+  return take_launch_status();
+}
+
+int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,
+                     const tile_out& out, const tile_gated& gated, const tile_norm& norm, hipStream_t s) {
+  if (M <= 32) return launch_dual_t<1, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  if (M <= 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  if (M <= 128) return launch_dual_t<4, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  return launch_dual_t<4, 3>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+}
+
+// Partial sums per output element: enough workgroups for every CU, about 4 k-blocks each or more, at most
+// 8 or 9 (every one of them is 4 bytes written and read again per output element).
+tile_split make_tile_split(int64_t M, int64_t N, int64_t K, int64_t Ka) {
+  const int64_t wgs = ((N + TL_BN - 1) / TL_BN) * ((M + 127) / 128), nkb = K / TL_BK, na = Ka / TL_BK, nb = nkb - na;
+  int64_t z = (256 + wgs / 2) / wgs;
+  if (z > nkb / 4) z = nkb / 4;
+  if (z > 8) z = 8;
+  if (z < 1) z = 1;
+  const int64_t per = (nkb + z - 1) / z;
+  tile_split sp;
+  sp.nkb_a = (int32_t)na;
+  sp.a = (int32_t)((na + per - 1) / per);
+  sp.per_a = sp.a ? (int32_t)((na + sp.a - 1) / sp.a) : 0;
+  sp.b = (int32_t)((nb + per - 1) / per);
+  sp.per_b = sp.b ? (int32_t)((nb + sp.b - 1) / sp.b) : 0;
+  if (sp.a) sp.a = (int32_t)((na + sp.per_a - 1) / sp.per_a);
+  if (sp.b) sp.b = (int32_t)((nb + sp.per_b - 1) / sp.per_b);
+  return sp;
+}
+
+template <int WM, int STAGES>
+static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw,
+                            float* P, const tile_split& sp, hipStream_t s) {
+  using G = tile_cfg<WM, STAGES>;
+  auto kern = tile_partial_kernel<WM, STAGES>;
+  want_dynamic_lds((const void*)kern, G::LDS);
+  const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct * sp.total() + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w,
+              (int)N, ldw, P, sp, ct, mt);
+  return take_launch_status();
+}
+
+int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw,
+                        float* P, const tile_split& splits, hipStream_t s) {
+  if (M <= 32) return launch_partial_t<1, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
+  if (M <= 64) return launch_partial_t<2, 5>(x, M, K, ldx, w, N, ldw, P, splits, s);
+  if (M <= 128) return launch_partial_t<4, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
+  return launch_partial_t<4, 3>(x, M, K, ldx, w, N, ldw, P, splits, s);
+}
+
+int launch_tail_reduce(const float* P, const tile_split& split, const bf16_t* r, bf16_t* sum, bf16_t* norm, const float* w,
+                       float eps, float* ss, int64_t M, int64_t N, hipStream_t s) {
+  if (N <= 2048) MVPA_LAUNCH(tail_reduce_kernel<1>, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
+  else MVPA_LAUNCH(tail_reduce_kernel<2>, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
+  return take_launch_status();
+}
+
+}  // namespace mvpa

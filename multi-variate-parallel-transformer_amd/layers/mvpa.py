@@ -48,8 +48,10 @@ class MvpaKVCache:
         self.start = 0            # first live time step in the buffers
         self.length = 0           # live time steps
 
-    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
-        """Add one time step ([B,Hkv,C,Dh] each); returns views [B,Hkv,T,C,Dh] of the live steps."""
+    def advance(self) -> int:
+        """Room for one more time step: the oldest leaves a full window, live steps move back to the front
+        of a full buffer.  Returns the slot that the new step's keys and values belong in; the step
+        counts as live from here on."""
         if self.length == self.max_steps:                 # the oldest step leaves the window
             self.start += 1
             self.length -= 1
@@ -59,10 +61,14 @@ class MvpaKVCache:
             self.k[:, :, :self.length] = live_k
             self.v[:, :, :self.length] = live_v
             self.start = 0
-        pos = self.start + self.length
+        self.length += 1
+        return self.start + self.length - 1
+
+    def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
+        """Add one time step ([B,Hkv,C,Dh] each); returns views [B,Hkv,T,C,Dh] of the live steps."""
+        pos = self.advance()
         self.k[:, :, pos] = k_new
         self.v[:, :, pos] = v_new
-        self.length += 1
         return self.views()
 
     def views(self) -> Tuple[torch.Tensor, torch.Tensor]:

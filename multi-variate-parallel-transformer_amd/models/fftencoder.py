@@ -81,14 +81,8 @@ class WaveEncoder(BrainEncoder):
                          torch.nn.functional.pad(self.proj.weight.to(torch.bfloat16), (0, pad)))
 
     def _forward_fused(self, x: Tensor) -> Tensor:
-        m = x.shape[0]
-        kp = self._padded_k()
-        coeffs = mvpa_hip.wavedec_db4(x.float(), pitch=kp, zero_pad=False)   # [M, dwt] view, pitch kp
-        normed = torch.empty((m, kp), dtype=torch.bfloat16, device=x.device)
-        normed[:, self.dwt_size:].zero_()
-        mvpa_hip.rmsnorm(coeffs, self.ln.weight, 1e-5, out=normed[:, : self.dwt_size])
-        w = self._padded_weight()
-        return mvpa_hip.linear(normed, w)          # the zero padding contributes nothing
+        normed = mvpa_hip.wavedec_db4_rmsnorm(x, self.ln.weight, self._padded_k())
+        return mvpa_hip.linear(normed, self._padded_weight())       # the zero padding contributes nothing
 
     def encode(self, x: Tensor) -> Tensor:
         return self.forward(x)

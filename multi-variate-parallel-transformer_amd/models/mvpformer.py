@@ -290,6 +290,8 @@ class MVPFormerModel(nn.Module):
         self.positional_embedding = nn.Embedding(config.max_position_embeddings, self.embed_dim)
         self.channel_embedding = nn.Embedding(config.max_channel_embeddings, self.embed_dim)
         self.gradient_checkpointing = gradient_checkpointing
+        self._plan = None                # operands of the native stack, see _native_plan
+        self._plan_key = None
         self.apply(self._init_weights)
 
     def _init_weights(self, module):
@@ -341,6 +343,102 @@ class MVPFormerModel(nn.Module):
             return self._forward(past_key_values, inputs_embeds, attention_mask, use_cache, position_end,
                                  channel_validity)
 
+    def _native_plan(self, t_len, c_len, pos_lo, normed):
+        """The operands of every block for the library's stack call, collected once per shape and kept
+        until a weight changes (its tensor, storage or version).  normed: with the weights that carry
+        ln_1 in their columns.  None where a block is not what that call computes."""
+        key = (t_len, c_len, pos_lo, normed)
+        ext = mvpa_hip.load_ext()
+        if self._plan_key == key and self._plan is not None and ext.plan_current(self._plan):
+            return self._plan
+        self._plan = None
+        first = self.h[0].attn
+        inner = self.h[0].mlp.down_proj.in_features
+        bf16, entries, tensors = torch.bfloat16, [], []
+
+        def watch(module, *names):
+            for name in names:
+                table = module._modules if name in module._modules else \
+                    module._parameters if name in module._parameters else module.__dict__
+                entries.append((table, name, table[name]))
+                if isinstance(table[name], torch.Tensor):
+                    tensors.append(table[name])
+
+        watch(self, "h", "ln_f", "positional_embedding", "channel_embedding")
+        for m in (self.ln_f, self.positional_embedding, self.channel_embedding):
+            watch(m, "weight")
+        watch(self.ln_f, "eps")
+        pos = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
+        chan = self.channel_embedding.weight[:c_len][None]
+        blocks = []
+        for name, blk in self.h._modules.items():
+            attn, mlp = blk.attn, blk.mlp
+            if (type(blk) is not MVPFormerBlock or type(mlp) is not GatedMLP
+                    or type(attn) not in (MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
+                    or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != (first.num_heads, first.num_kv_heads, first.head_dim)
+                    or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != bf16):
+                return None
+            watch(self.h, name)
+            watch(blk, "ln_1", "attn", "mlp")
+            watch(blk.ln_1, "weight", "eps")
+            watch(attn, "q_attn", "c_attn", "c_proj", "position_net", "channel_net", "attn_bias", "fp8_qk", "global_att",
+                  "scale_attn_weights", "scale_attn_by_inverse_layer_idx", "layer_idx")
+            watch(mlp, "gate_proj", "up_proj", "down_proj")
+            for m in (attn.q_attn, attn.c_attn, attn.c_proj, attn.position_net, attn.channel_net, mlp.gate_proj,
+                      mlp.up_proj, mlp.down_proj):
+                watch(m, *m._parameters)
+            k_time, k_chan = attn._key_tables(pos, chan)
+            bias = attn.attn_bias.detach().to(bf16).contiguous()
+            u, vb, z = (b.contiguous() for b in bias.split(attn.embed_kv_dim))
+            wq, wg = blk._folded_weights() if normed else (None, None)
+            flags = ((mvpa_hip.FLAG_CONTENT if attn._content() else 0) | (mvpa_hip.FLAG_FP8_QK if attn.fp8_qk else 0))
+            blocks.append((attn.qkv_weight(bf16), mlp.gate_up_weight(), wq, wg, blk._tail_weight(),
+                           mvpa_hip._as_f32_weight(blk.ln_1.weight), u, vb, z, k_time.to(bf16), k_chan.to(bf16),
+                           float(blk.ln_1.eps), attn._scale(), flags, 10, attn._honours_masks))
+        self._plan = ext.plan((t_len, c_len, first.num_heads, first.num_kv_heads, first.head_dim, self.embed_dim, inner),
+                              mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks, entries, tensors)
+        self._plan_key = key
+        return self._plan
+
+    def _native(self, hidden_states, past_key_values, mask, t_len, pos_lo):
+        """The whole stack as one call of the library, for the whole-sequence forward and for one step
+        on caches; None where that call does not apply (an additive key bias, caches of another
+        kind, shapes outside the matrix-core kernels) and the blocks go one by one."""
+        bsz, t_new, c_len, e = hidden_states.shape
+        attn, inner = self.h[0].attn, self.h[0].mlp.down_proj.in_features
+        if e % 64 or inner % 64 or e > 4096 or c_len > 128 or attn.head_dim not in (32, 64, 128) or bsz == 0:
+            return None
+        valid = None
+        if mask is not None:
+            valid, bias = mask.resolve(bsz, t_len, c_len)
+            if bias is not None:
+                return None
+        caches = head = sumsq = None
+        rows = bsz * t_new * c_len
+        if past_key_values is not None:
+            kinds = {type(c) for c in past_key_values}
+            if kinds == {MvpaKVCache}:
+                if any(c.k.dtype != torch.bfloat16 or c.max_steps != past_key_values[0].max_steps
+                       or c.length != past_key_values[0].length for c in past_key_values):
+                    return None
+            elif kinds == {MvpaRingCache}:
+                clock = past_key_values[0].clock
+                if any(c.own_clock or c.clock is not clock or c.k.dtype != torch.bfloat16 for c in past_key_values):
+                    return None
+                head = clock.head32
+            else:
+                return None
+        normed = past_key_values is None and self.h[0].norm_fused_supported(rows)
+        plan = self._native_plan(t_len, c_len, pos_lo, normed)
+        if plan is None:
+            return None
+        if past_key_values is not None:
+            first = [0 if head is not None else c.advance() - (t_len - 1) for c in past_key_values]
+            caches = ([c.k for c in past_key_values], [c.v for c in past_key_values], first)
+        elif normed:
+            sumsq = mvpa_hip.row_sumsq(hidden_states.reshape(rows, e))
+        return mvpa_hip._taken(mvpa_hip.load_ext().run(plan, hidden_states, valid, caches, head, sumsq))
+
     def _forward(self, past_key_values, inputs_embeds, attention_mask, use_cache, position_end,
                  channel_validity):
         use_cache = bool(use_cache)      # None = off whatever config.use_cache says: a tensor comes back
@@ -379,6 +477,11 @@ class MVPFormerModel(nn.Module):
         pos_lo = 0 if position_end is None else position_end - t_len
         if pos_lo < 0 or pos_lo + t_len > self.positional_embedding.num_embeddings:
             raise IndexError("position_end leaves fewer than T rows of the position embedding")
+        if (not torch.is_grad_enabled() and inputs_embeds.is_cuda and inputs_embeds.dtype == torch.bfloat16
+                and len(self.h) > 0 and (past_key_values is not None or not use_cache)):
+            out = self._native(inputs_embeds, past_key_values, attention_mask, t_len, pos_lo)
+            if out is not None:
+                return (out, tuple(past_key_values)) if past_key_values is not None else out
         position_embeds = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
         channel_embeds = self.channel_embedding.weight[:c_len][None]
         hidden_states, normed = inputs_embeds, None
@@ -505,7 +608,7 @@ class HMVPFormer(BrainModel):
             out, past = self._first_step(embeds, past)
         else:
             out, past = self.mvpformer(inputs_embeds=embeds, past_key_values=past)
-        return self.head(out[:, -1].float().mean(dim=1).to(out.dtype)), past
+        return self.head(_channel_mean(out)), past
 
     def capture_stream(self, past, segment_like: torch.Tensor, predict: bool = False):
         """Turn a stream whose window is full into a replayable HIP graph.  `past` is what
@@ -533,7 +636,7 @@ class HMVPFormer(BrainModel):
                 sim = torch.cosine_similarity(embeds[:, 0].float(), forecast.float(), dim=-1)
                 forecast.copy_(self.head(out[:, -1]))
                 return sim, forecast
-            return self.head(out[:, -1].float().mean(dim=1).to(out.dtype))
+            return self.head(_channel_mean(out))
 
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
@@ -615,7 +718,15 @@ class HMVPFormer(BrainModel):
         last segment's hidden state)."""
         with self._grad_mode():
             out, _ = self._common_forward(batch)
-            return self.head(out[:, -1].float().mean(dim=1).to(out.dtype))
+            return self.head(_channel_mean(out))
+
+
+def _channel_mean(out: torch.Tensor) -> torch.Tensor:
+    """Mean over the channels of the last time step of [B, T, C, E], in fp32, in out's dtype."""
+    last = out[:, -1]
+    if last.is_cuda and out.dtype == torch.bfloat16 and out.shape[-1] % 8 == 0 and not torch.is_grad_enabled():
+        return mvpa_hip.mean_rows(last)
+    return last.float().mean(dim=1).to(out.dtype)
 
 
 def _load_weights(path: str):

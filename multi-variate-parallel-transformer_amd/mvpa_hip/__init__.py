@@ -3,10 +3,14 @@
 PyTorch is used only for device memory and streams: every op here hands raw device
 pointers and the current HIP stream to the library.  There is no fallback: if the shared
 library is missing or an entry point reports an error, the call raises.
+
+The calls that are bound by their launches (the attention operator, the encoder, a stack of blocks)
+go through `_mvpa_ext.so`, a binding of the same entry points in C++ (csrc/mvpa_ext.cpp).
 """
 from __future__ import annotations
 
 import ctypes
+import functools
 import os
 from typing import Optional
 
@@ -149,6 +153,32 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+_ext = None
+
+
+def load_ext():
+    """The C++ binding of the launch-bound paths, built beside the library; raises if it is missing."""
+    global _ext
+    if _ext is None:
+        load_library()
+        import importlib.util
+        path = os.path.join(_HERE, "_mvpa_ext.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing - build it with `python __graft_entry__.py`; there is no fallback path")
+        spec = importlib.util.spec_from_file_location("_mvpa_ext", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        _ext = mod
+    return _ext
+
+
+def _taken(result):
+    """A result of the C++ binding: a tensor (or a tuple of them), or the status the library refused with."""
+    if type(result) is int:
+        _check(result)
+    return result
+
+
 def error_string(status: int) -> str:
     return load_library().mvpa_error_string(status).decode()
 
@@ -267,6 +297,12 @@ def mvpa_forward(q, k, v, u, vb, z, k_time, k_chan, *, sm_scale: Optional[float]
     the workspace built into the library (mvpa_forward_last_step_static) instead of one allocated
     here; with `out` given the call then allocates no device memory at all.
     """
+    if not (last_step_only or fp8_qk or static_ws or ring_head is not None) and q.is_cuda:
+        flags = ((FLAG_CAUSAL if causal else 0) | (FLAG_CONTENT if content else 0) |
+                 (FLAG_TIME_BIAS if time_bias else 0) | (FLAG_CHAN_BIAS if chan_bias else 0))
+        s = q.shape[-1] ** -0.5 if sm_scale is None else float(sm_scale)
+        return _taken((_ext or load_ext()).forward(q, k, v, u, vb, z, k_time, k_chan, out, chan_valid, key_bias, s,
+                                                   window, flags, kernel, return_lse))
     lib = load_library()
     _need_cuda(q, k, v, u, vb, z, k_time, k_chan, chan_valid, key_bias)
     B, H, Nq, Dh = q.shape
@@ -484,6 +520,19 @@ def row_sumsq(x: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def mean_rows(x: torch.Tensor) -> torch.Tensor:
+    """Mean over dim 1 of a bf16 [groups, rows, cols] tensor (unit last stride, cols a multiple of 8)
+    in fp32, rounded to bf16."""
+    return _taken((_ext or load_ext()).mean_rows(x))
+
+
+def wavedec_db4_rmsnorm(x: torch.Tensor, weight: torch.Tensor, pitch: int, eps: float = 1e-5) -> torch.Tensor:
+    """RMSNorm of the db4 coefficients of x [M, L] in bf16, [M, pitch] with zeros past the coefficients:
+    wavedec_db4 and rmsnorm in one pass."""
+    levels, total = _dwt_shape(x.shape[-1])
+    return _taken((_ext or load_ext()).encode(x, _as_f32_weight(weight), levels, total, pitch, eps))
+
+
 def linear_norm_fused_supported(M: int, K: int, N: int) -> bool:
     """Shapes for which the tail product can write row statistics (linear(..., sumsq_out=True))
     and the dual product can consume them (linear_dual(sumsq=...))."""
@@ -501,6 +550,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, out: Optional[torch.Tensor] = 
     linear_residual_supported holds; otherwise MvpaError).
     sumsq_out (with residual): also returns the partial sums of squares of the output rows,
     [rows, parts] fp32 - (out, sumsq) comes back - for a later linear_dual(sumsq=...)."""
+    if out is None and not gated and split_k is None and residual is None and not sumsq_out and x.is_cuda:
+        return _taken((_ext or load_ext()).linear(x, weight))
     lib = load_library()
     _need_cuda(x, weight)
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
@@ -695,6 +746,12 @@ def dwt_sizes(size_input: int):
         sizes.append(n)
     sizes.append(n)
     return levels, sizes
+
+
+@functools.lru_cache(maxsize=64)
+def _dwt_shape(size_input: int):
+    levels, sizes = dwt_sizes(size_input)
+    return levels, sum(sizes)
 
 
 def wavedec_db4(x: torch.Tensor, pitch: Optional[int] = None, zero_pad: bool = True) -> torch.Tensor:

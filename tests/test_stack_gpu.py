@@ -1,0 +1,115 @@
+"""The stack of blocks as one library call (small-tile products, caches written by their epilogue) against
+the same blocks one by one, and the one-pass encoder against its separate kernels, at the sizes where
+tiles, splits and rows end."""
+import pytest
+import torch
+
+import mvpa_hip
+from models.mvpformer import MVPFormerConfig, MVPFormerModel
+
+pytestmark = pytest.mark.gpu
+
+# Both sides multiply bf16 operands with fp32 accumulation; the library call keeps the attention and MLP
+# outputs of a block in fp32 until one rounding where the blocks one by one round three times.  Two
+# blocks, a handful of roundings of 2^-9 each: 1e-2 relative.
+REL = 1e-2
+
+
+def _model(**kw):
+    torch.manual_seed(3)
+    dims = dict(n_positions=40, n_channels=128, n_embd=128, n_layer=2, n_head=2, n_head_kv=1, n_inner=192)
+    dims.update(kw)
+    model = MVPFormerModel(MVPFormerConfig(**dims)).to(device="cuda", dtype=torch.bfloat16).eval()
+    for n, p in model.named_parameters():
+        p.data.copy_(1.0 + 0.2 * torch.randn_like(p)) if "ln" in n else p.data.mul_(3.0)
+    return model
+
+
+def _rel(a, b):
+    return ((a.float() - b.float()).norm() / b.float().norm()).item()
+
+
+@pytest.mark.parametrize("dims", [{}, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=64),      # ragged column tiles
+                                  dict(n_embd=256, n_head=2, n_head_kv=1, n_inner=640)],        # head size 128
+                         ids=["E128", "E320", "D128"])
+@pytest.mark.parametrize("B,C,T", [(1, 1, 1), (1, 31, 1), (1, 33, 1), (1, 64, 1), (1, 13, 5), (1, 128, 1), (3, 43, 1),
+                                   (1, 64, 8), (2, 37, 7)],     # row tiles of 32, 64, 128; rows from which ln_1 is fused
+                         ids=lambda v: str(v))
+def test_whole_sequence(monkeypatch, dims, B, C, T):
+    model = _model(**dims)
+    x = torch.randn(B, T, C, model.embed_dim, device="cuda").bfloat16()
+    valid = torch.rand(B, C, device="cuda") < 0.8
+    valid[:, 0] = True
+    with torch.no_grad():
+        a = model(inputs_embeds=x, channel_validity=valid)
+        monkeypatch.setattr(MVPFormerModel, "_native", lambda *args: None)
+        b = model(inputs_embeds=x, channel_validity=valid)
+    assert a.shape == b.shape and _rel(a, b) <= REL
+
+
+@pytest.mark.parametrize("B,C", [(1, 5), (1, 64), (2, 100)])
+def test_steps_on_caches(monkeypatch, B, C):
+    """A stream that fills its window and slides on: outputs, and every cached key and value."""
+    model = _model()
+    xs = torch.randn(12, B, 1, C, model.embed_dim, device="cuda").bfloat16()
+    runs = []
+    for native in (True, False):
+        with monkeypatch.context() as m:
+            if not native:
+                m.setattr(MVPFormerModel, "_native", lambda *args: None)
+            caches = model.new_cache(B, C, max_steps=8)
+            with torch.no_grad():
+                out = [model(inputs_embeds=x, past_key_values=caches)[0] for x in xs]
+            runs.append((out, [t.clone() for c in caches for t in c.views()]))
+    for a, b in zip(runs[0][0] + runs[0][1], runs[1][0] + runs[1][1]):
+        assert a.shape == b.shape and _rel(a, b) <= REL
+
+
+def test_plan_follows_the_weights():
+    """A changed weight - in place, by a new storage, by a new parameter, by a new sub-module - is seen."""
+    model = _model()
+    x = torch.randn(1, 3, 8, 128, device="cuda").bfloat16()
+
+    def out():
+        with torch.no_grad():
+            return model(inputs_embeds=x)
+    seen = [out()]
+    blk = model.h[1]
+    with torch.no_grad():
+        blk.mlp.down_proj.weight.mul_(2.0)
+    seen.append(out())
+    blk.attn.q_attn.weight.data = blk.attn.q_attn.weight.data * 2.0
+    seen.append(out())
+    blk.attn.c_proj.weight = torch.nn.Parameter(blk.attn.c_proj.weight.detach() * 2.0)
+    seen.append(out())
+    new = torch.nn.Linear(128, 192, bias=False, device="cuda", dtype=torch.bfloat16)
+    blk.mlp.up_proj = new
+    seen.append(out())
+    blk.ln_1.eps = 0.5
+    seen.append(out())
+    for a, b in zip(seen, seen[1:]):
+        assert not torch.equal(a, b)
+    assert torch.equal(out(), seen[-1])
+
+
+@pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560])
+@pytest.mark.parametrize("M", [1, 5])
+def test_encoder_in_one_pass(L, M):
+    """Analysis, norm and rounding in one kernel against the two kernels: the same fp32 formula, summed
+    in another order, so at most one bf16 step apart."""
+    _, sizes = mvpa_hip.dwt_sizes(L)
+    total = sum(sizes)
+    pitch = (total + 63) // 64 * 64
+    x = torch.randn(M, L, device="cuda")
+    w = 1.0 + 0.1 * torch.randn(total, device="cuda")
+    got = mvpa_hip.wavedec_db4_rmsnorm(x, w, pitch).float()
+    ref = mvpa_hip.rmsnorm(mvpa_hip.wavedec_db4(x), w, 1e-5, out=torch.empty(M, total, device="cuda"))
+    assert (got[:, total:] == 0).all()
+    assert ((got[:, :total] - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
+def test_mean_rows():
+    x = torch.randn(3, 77, 136, device="cuda").bfloat16()
+    got = mvpa_hip.mean_rows(x[:, 5:]).float()
+    ref = x[:, 5:].float().mean(1)
+    assert ((got - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
