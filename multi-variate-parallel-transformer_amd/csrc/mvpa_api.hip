@@ -116,6 +116,15 @@ extern "C" int mvpa_forward(const mvpa_fwd_args* a, void* stream) {
     if (a->kernel == MVPA_KERNEL_MFMA_SPLIT) return mvpa_launch_mfma128(a, st);
     if (a->kernel == MVPA_KERNEL_MFMA) return mvpa_launch_mfma(a, st);
     // AUTO: the specialised builds where they are the faster ones.
+    // Launches that leave the chip idle: the build whose waves split the keys of a query tile, up to two
+    // workgroups per CU, and further with one query tile per step, where the other kernel's time is one
+    // chain over the steps whatever the batch (us, general -> this: H12 C21 T25 24 -> 13 at B1, 24.5 -> 20
+    // at B2, 25 -> 35 at B4; C21 T50 35 -> 23; C32 T64 54 -> 28; C21 T110 84 -> 58; C64 T12 17.5 -> 13,
+    // C64 T25 24.4 -> 25; H4 C8 T32 Dh32 22 -> 8; H16 Dh128 C21 T25 35 -> 25).
+    if (!(a->flags & MVPA_FLAG_LAST_STEP) && a->C <= (a->Dh == 128 ? 32 : 64) && mvpa_wave_supported(a)) {
+      const int64_t wgs = (int64_t)a->B * a->H * ((a->C + 31) / 32) * a->T;
+      if (wgs <= 512 || (a->C <= 32 && a->T <= 128 && wgs <= 24 * (int64_t)a->T)) return mvpa_launch_wave(a, st);
+    }
     // 65..128 channels at head size 64 or 128: the build of csrc/mvpa_mfma128.hip wins at every
     // length and channel count measured (Dh 128, B1 H16: C128 T 16 .. 1024 13 .. 20 % less time than
     // the general kernel, C 80 .. 100 21 .. 40 %; Dh 64, H16: B8 C117 T256 11.14 -> 8.58 ms,

@@ -143,6 +143,12 @@ int mvpa_mfma_supported(const mvpa_fwd_args* a);
 // the build of it in which a wave owns a whole time step (head size 64, 33..64 channels)
 int mvpa_mfma64_supported(const mvpa_fwd_args* a);
 int mvpa_launch_mfma64(const mvpa_fwd_args* a, hipStream_t stream);
+// the build whose waves split the keys of one query tile (launches that do not fill the chip)
+int mvpa_wave_supported(const mvpa_fwd_args* a);
+int mvpa_launch_wave(const mvpa_fwd_args* a, hipStream_t stream);
+// one decoding step in runs, 65..128 channels: the query tiles of a workgroup share the K and V of a run
+int mvpa_step_supported(const mvpa_fwd_args* a);
+int mvpa_launch_step(const mvpa_fwd_args* a, hipStream_t stream);
 int mvpa_mfma128_supported(const mvpa_fwd_args* a);
 int mvpa_launch_mfma128(const mvpa_fwd_args* a, hipStream_t stream);
 // backward, query pass on MFMA (bf16, Dh = 64, C <= 64)

@@ -827,17 +827,38 @@ __global__ __launch_bounds__(256) void mvpa_split_merge_kernel(mvpa_fwd_args a) 
   if (row >= rows) return;
   const bf16_t* po = (const bf16_t*)a.split_ws;
   const float* plse = (const float*)(po + (int64_t)a.n_split * rows * DH);
-  float m = -INFINITY;
-  for (int r = 0; r < a.n_split; ++r) m = fmaxf(m, plse[(int64_t)r * rows + row]);
-  float l = 0.f, acc[8];
+  // eight runs at a time, all of their loads in flight together (one run after the other: 16 runs took
+  // 10.5 us, the latency of 32 dependent round trips)
+  float m = -INFINITY, l = 0.f, acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-  for (int r = 0; r < a.n_split; ++r) {
-    const float w = fast_exp2(plse[(int64_t)r * rows + row] - m);
-    l += w;
-    const x8 v = *(const x8*)(po + ((int64_t)r * rows + row) * DH + 8 * sub);
+  for (int r0 = 0; r0 < a.n_split; r0 += 8) {
+    float e[8];
+    x8 v[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] += w * (float)v[i];
+    for (int j = 0; j < 8; ++j) {
+      const int64_t at = (int64_t)min(r0 + j, a.n_split - 1) * rows + row;
+      e[j] = plse[at];
+      v[j] = *(const x8*)(po + at * DH + 8 * sub);
+    }
+    float mc = m;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (r0 + j >= a.n_split) e[j] = -INFINITY;
+      mc = fmaxf(mc, e[j]);
+    }
+    const float keep = fast_exp2(m - mc);
+    m = mc;
+    l *= keep;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] *= keep;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float w = fast_exp2(e[j] - m);
+      l += w;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i] += w * (float)v[j][i];
+    }
   }
   const int bh = row / C_, cq = row % C_, b = bh / a.H, h = bh % a.H;
   const float inv = 1.f / l;
@@ -846,6 +867,14 @@ __global__ __launch_bounds__(256) void mvpa_split_merge_kernel(mvpa_fwd_args a) 
   for (int i = 0; i < 8; ++i) w8[i] = E::cvt(acc[i] * inv);
   *(x8*)((bf16_t*)a.o + b * a.o_stride_b + h * a.o_stride_h + (int64_t)cq * a.o_stride_n + 8 * sub) = w8;
   if (a.lse && sub == 0) a.lse[row] = m + log2f(l);
+}
+
+template <typename E>
+static void launch_merge(const mvpa_fwd_args* a, hipStream_t stream) {
+  const int rows = a->B * a->H * a->C, rpb = 2048 / a->Dh;
+  auto kern = a->Dh == 32 ? mvpa_split_merge_kernel<32, E> : a->Dh == 64 ? mvpa_split_merge_kernel<64, E>
+                                                                          : mvpa_split_merge_kernel<128, E>;
+  MVPA_LAUNCH(kern, dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, stream, *a);
 }
 
 template <int DH, int NCT, int NW, int STAGES, int MINB, bool FP8, int KH, typename E>
@@ -865,10 +894,7 @@ static int launch_one(const mvpa_fwd_args* a, hipStream_t stream) {
   const int nt = (G::TQW == 2 && STAGES == 4 && KH == 1) ? 1 + a->T / 2 : (a->T + G::TQW - 1) / G::TQW;   // as in the kernel
   dim3 grid((unsigned)((last ? n_split : nt) * a->B * a->H));
   MVPA_LAUNCH(kern, grid, dim3(G::THREADS), G::LDS_BYTES, stream, *a);
-  if (n_split > 1) {
-    const int rows = a->B * a->H * a->C;
-    MVPA_LAUNCH((mvpa_split_merge_kernel<DH, E>), dim3((unsigned)((rows + 2048 / DH - 1) / (2048 / DH))), dim3(256), 0, stream, *a);
-  }
+  if (n_split > 1) launch_merge<E>(a, stream);
   return mvpa::take_launch_status();
 }
 
@@ -906,6 +932,17 @@ int mvpa_mfma_supported(const mvpa_fwd_args* a) {
 
 int mvpa_launch_mfma(const mvpa_fwd_args* a, hipStream_t stream) {
   using namespace mvpa;
+  // a decoding step cut into runs: the builds made for it, by the number of channels (us with the merge, this
+  // kernel -> those: B1 H12 C64 T64 Dh64 8 runs 17.8 -> 11.2, H12 C21 16.5 -> 9.7, H16 C128 T110 Dh128 16 runs
+  // 50 -> 28, T512 108 -> 82); fp8 and the lengths they have no LDS for stay here
+  if ((a->flags & MVPA_FLAG_LAST_STEP) && a->split_ws && a->n_split > 1 && (a->flags & MVPA_FLAG_CONTENT) &&
+      (mvpa_wave_supported(a) || mvpa_step_supported(a))) {
+    const int st = mvpa_step_supported(a) ? mvpa_launch_step(a, stream) : mvpa_launch_wave(a, stream);
+    if (st != MVPA_OK) return st;
+    if (a->dtype == MVPA_F16) launch_merge<el_f16>(a, stream);
+    else launch_merge<el_bf16>(a, stream);
+    return take_launch_status();
+  }
   const int nct = a->C <= 32 ? 1 : a->C <= 64 ? 2 : 4;
   switch (a->Dh) {
     case 32:

@@ -163,6 +163,15 @@ struct el_bf16 {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
   }
   static __device__ inline x8 qfrag(u32x4 raw, const bf16_t* __restrict__ bias, float scale) { return make_qfrag(raw, bias, scale); }
+  // the same in two parts, for kernels that form several fragments of a q row: fma instead of add and
+  // multiply, the unpacked q and the scaled bias each formed once
+  static __device__ inline void unpack(u32x4 w, float (&f)[8]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      f[2 * i] = __uint_as_float(w[i] << 16);
+      f[2 * i + 1] = __uint_as_float(w[i] & 0xffff0000u);
+    }
+  }
   static __device__ inline x8 as8(u32x4 v) { return as_bf16x8(v); }
   static __device__ inline x8 pack(const f32x16& v, int base) { return pack8(v, base); }
   static __device__ inline float add_pair(x2 p, float acc) { return __builtin_amdgcn_fdot2_f32_bf16(p, kOnes2, acc, false); }
@@ -187,6 +196,12 @@ struct el_f16 {
     for (int i = 0; i < 8; ++i) out[i] = (_Float16)(((float)r.h[i] + (float)b.h[i]) * scale);
     return out;
   }
+  static __device__ inline void unpack(u32x4 w, float (&f)[8]) {
+    union { u32x4 u; x8 h; } c;
+    c.u = w;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) f[i] = (float)c.h[i];
+  }
   static __device__ inline x8 as8(u32x4 v) {
     union { u32x4 u; x8 h; } c;
     c.u = v;
@@ -209,6 +224,17 @@ struct el_f16 {
   }
   static __device__ inline _Float16 cvt(float f) { return (_Float16)f; }
 };
+
+// (q + bias) * scale of 8 elements, from unpacked q and packed bias
+template <typename E>
+__device__ inline typename E::x8 qfrag_fma(const float (&q)[8], u32x4 bias, float scale) {
+  float b[8];
+  E::unpack(bias, b);
+  typename E::x8 out;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) out[i] = E::cvt(__builtin_fmaf(q[i], scale, b[i] * scale));
+  return out;
+}
 
 // XOR swizzles of the 16-byte chunk index within a K / V row, chosen so that the lanes that
 // read LDS together (16 consecutive rows at one chunk for K; 4 consecutive rows x 4 chunks for
@@ -274,6 +300,43 @@ __host__ __device__ inline void map_block(int L, int nbh, int nt, int grp, int& 
   }
   bh = xcd * per_xcd + unit * u + i % u;
   tile = nt - 2 - i / u;
+}
+
+// The order of the workgroups of mvpa_wave.hip and mvpa_step.hip.  Everything that reads one run of a kv
+// head's K and V - its query heads, and their query tiles where those are workgroups of their own - sits
+// on one XCD (ids equal mod 8) side by side, so that the run enters one L2, once.  The grid is three
+// dimensional, x fastest: x the XCD, y the item (head of the group, query tile), z the run, so that a
+// workgroup finds its place without a division (a kernel of 8 us spent 1 of them on divisions).
+//   n_bg (batch x kv heads) a multiple of 8: z also walks the pairs an XCD owns; n_bg a divisor of 8: the runs
+//   of a pair are dealt over the XCDs it has; else x is the pair itself.
+struct step_geom {
+  int32_t n_bg, grp, runs, len;            // pairs, query heads per kv head, runs, key steps per run
+  int32_t sub_shift;                       // n_bg a divisor of 8: log2 of n_bg, else -1
+};
+inline step_geom make_step_geom(int n_bg, int grp, int runs, int T) {
+  step_geom g{n_bg, grp, runs, (T + runs - 1) / runs, -1};
+  if (n_bg < 8 && 8 % n_bg == 0) g.sub_shift = n_bg == 1 ? 0 : n_bg == 2 ? 1 : 2;
+  return g;
+}
+inline dim3 step_grid(const step_geom& g, int items) {
+  if (g.n_bg % 8 == 0) return dim3(8, (unsigned)items, (unsigned)(g.runs * (g.n_bg / 8)));
+  if (g.sub_shift >= 0) return dim3(8, (unsigned)items, (unsigned)((g.runs + (8 >> g.sub_shift) - 1) >> (3 - g.sub_shift)));
+  return dim3((unsigned)g.n_bg, (unsigned)items, (unsigned)g.runs);
+}
+// the workgroup's pair and run (false: no such run)
+__device__ inline bool step_block(const step_geom& g, int& bg, int& run) {
+  const int x = blockIdx.x, z = blockIdx.z;
+  bg = x;
+  run = z;
+  if (g.sub_shift >= 0) {
+    bg = x & ((1 << g.sub_shift) - 1);
+    run = (z << (3 - g.sub_shift)) + (x >> g.sub_shift);
+  } else if (g.n_bg > 8 && (g.n_bg & 7) == 0) {
+    const int p = z / g.runs;
+    run = z - p * g.runs;
+    bg = x + 8 * p;
+  }
+  return run < g.runs;
 }
 
 }  // namespace mvpa

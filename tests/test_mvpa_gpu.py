@@ -1053,3 +1053,49 @@ def test_bf16_base_attention_shape_full_size(kern):
     o82 = mvpa_hip.mvpa_forward(d.q, d.k, v2, d.u, d.vb, d.z, d.k_time, d.k_chan, chan_valid=d.chan_valid,
                                 kernel=kern, fp8_qk=True)
     assert torch.equal(o82[:, :, :-40 * C], o8[:, :, :-40 * C])
+
+
+@pytest.mark.parametrize("cfg,kw", [
+    (dict(B=1, C=1, T=1, H=1, Dh=64), {}),                                   # one key, one wave of eight
+    (dict(B=1, C=21, T=25, H=12, Hkv=4, Dh=64), {}),                         # one tile per step, pairs that divide 8
+    (dict(B=2, C=33, T=9, H=6, Hkv=3, Dh=64, validity=True), {}),            # two tiles, one nearly empty; 6 pairs
+    (dict(B=1, C=64, T=13, H=8, Hkv=8, Dh=64), dict(window=3)),              # 8 pairs; steps outside the window
+    (dict(B=2, C=32, T=40, H=8, Hkv=8, Dh=32, validity=True), dict(window=2)),   # 16 pairs, two tiles of time rows
+    (dict(B=1, C=17, T=33, H=4, Hkv=2, Dh=128), dict(window=0)),
+], ids=lambda v: "-".join(f"{k}{x}" for k, x in v.items()) or "-")
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_wave_split_build_shapes(cfg, kw, dtype):
+    """The build whose waves split the keys of one query tile (what small launches run on)."""
+    inp = make_mvpa_inputs(seed=61, table_std=0.3, qkv_unit=True, **cfg).round_to(dtype)
+    out, lse = _gpu(inp, dtype, return_lse=True, **kw)
+    ref, ref_lse = _oracle(inp, return_lse=True, **kw)
+    err, rel = (out.float().cpu() - ref.float()).abs().max().item(), _rel_l2(out.float().cpu(), ref.float())
+    assert err <= BF16_MAX_ABS and rel <= BF16_REL_L2, (err, rel)
+    assert (lse.cpu().double() - ref_lse).abs().max().item() <= 3e-2
+
+
+@pytest.mark.parametrize("cfg,n,head", [
+    (dict(B=1, C=65, T=9, H=2, Hkv=1, Dh=64), 9, None),          # a second key half of one channel, one step per run
+    (dict(B=2, C=96, T=40, H=8, Hkv=4, Dh=64), 2, 5),            # 8 pairs, a ring
+    (dict(B=1, C=128, T=33, H=3, Hkv=3, Dh=128), 3, None),       # 3 pairs
+    (dict(B=2, C=128, T=64, H=16, Hkv=8, Dh=128), 2, 63),        # 16 pairs; runs of 32 steps, the longest it takes
+    (dict(B=1, C=100, T=70, H=2, Hkv=1, Dh=128), 2, None),       # runs of 35: left to the other builds
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+def test_decoding_step_in_runs_wide(cfg, n, head, dtype):
+    """65..128 channels, a step cut into runs (the build whose query tiles share K and V), with absent
+    channels: against the oracle's last rows."""
+    inp = make_mvpa_inputs(seed=67, table_std=0.3, qkv_unit=True, validity=True, **cfg).round_to(dtype)
+    ref = _oracle(inp)[:, :, -cfg["C"]:].float()
+    d = inp.to("cuda", dtype)
+    k, v, ring = d.k, d.v, None
+    if head is not None:
+        B, Hkv, T, C, Dh = cfg["B"], cfg.get("Hkv", cfg["H"]), cfg["T"], cfg["C"], cfg["Dh"]
+        step = T - 1 - (head - torch.arange(T, device="cuda")) % T
+        k, v = (t.view(B, Hkv, T, C, Dh)[:, :, step].reshape(B, Hkv, T * C, Dh).contiguous() for t in (k, v))
+        ring = torch.tensor([head], dtype=torch.int32, device="cuda")
+        if dtype == torch.float16:
+            pytest.skip("rings are tested in bf16")
+    out = mvpa_hip.mvpa_forward(d.q[:, :, -cfg["C"]:], k, v, d.u, d.vb, d.z, d.k_time, d.k_chan, chan_valid=d.chan_valid,
+                                last_step_only=True, key_splits=n, ring_head=ring).float().cpu()
+    assert (out - ref).abs().max().item() <= BF16_MAX_ABS and _rel_l2(out, ref) <= BF16_REL_L2
