@@ -257,6 +257,26 @@ typedef struct mvpa_bwd_args {
  * products that autograd applies to attentions/attn.py:1305-1314. */
 int mvpa_backward(const mvpa_bwd_args* args, void* stream);
 
+/* The backward up to the gradients of the operator's inputs in bf16: mvpa_backward and what autograd makes of
+ * its table gradients (attentions/attn.py:1305-1314), for the shapes of the matrix-core backward (bf16, Dh 64 or
+ * 128, C <= 128, causal, no key bias; MVPA_ERR_UNSUPPORTED otherwise).  Of `args` the input fields are read
+ * (through lse); its gradient and workspace fields are taken from `ws`
+ * (mvpa_backward_full_ws_bytes(args), 256-byte aligned).  dq, dk, dv at element strides that are multiples
+ * of 8; the rest contiguous. */
+typedef struct mvpa_bwd_grads {
+  uint32_t struct_size;      /* = sizeof(mvpa_bwd_grads)                                      */
+  uint32_t reserved0;
+  void *dq, *dk, *dv;        /* [B,H,N,Dh], [B,Hkv,N,Dh] x 2                                  */
+  int64_t dq_stride_b, dq_stride_h, dq_stride_n;
+  int64_t dk_stride_b, dk_stride_h, dk_stride_n;
+  int64_t dv_stride_b, dv_stride_h, dv_stride_n;
+  void *dbias_u, *dbias_v, *dbias_z;   /* [Hkv,Dh]                                            */
+  void *dk_time, *dk_chan;             /* [Hkv,T,Dh], [Hkv,C,Dh]                              */
+} mvpa_bwd_grads;
+size_t mvpa_backward_full_ws_bytes(const mvpa_bwd_args* args);
+int mvpa_backward_full(const mvpa_bwd_args* args, const mvpa_bwd_grads* grads, void* ws, size_t ws_bytes,
+                       void* stream);
+
 /* Which kernel mvpa_forward would run for these arguments: MVPA_KERNEL_GENERIC or
  * MVPA_KERNEL_MFMA (or a negative status). */
 int mvpa_select_kernel(const mvpa_fwd_args* args);

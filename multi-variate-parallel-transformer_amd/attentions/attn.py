@@ -39,6 +39,14 @@ class FlashMVPA(torch.autograd.Function):
     def backward(ctx, d_out):
         q, u, vb, z, k, k_time, k_chan, v, out, lse = ctx.saved_tensors
         causal, sm_scale, window, time_bias, chan_bias, chan_valid, content, key_bias = ctx.conf
+        if (q.dtype == k.dtype == v.dtype == torch.bfloat16 and q.shape[-1] in (64, 128) and k_chan.shape[-2] <= 128
+                and causal and key_bias is None):
+            grads = mvpa_hip.mvpa_backward_full(q, k, v, out, d_out, lse, u, vb, z, k_time, k_chan, sm_scale=sm_scale,
+                                                window=window, content=content, time_bias=time_bias,
+                                                chan_bias=chan_bias, chan_valid=chan_valid)
+            if grads is not None:
+                return (*(g.to(t.dtype) for g, t in zip(grads, (q, u, vb, z, k, k_time, k_chan, v))),
+                        None, None, None, None, None, None, None, None)
         dq_c, dk, dv, dbt, dbc = mvpa_hip.mvpa_backward(
             q, k, v, out, d_out.contiguous(), lse, u, vb, z, k_time, k_chan, sm_scale=sm_scale,
             window=window, causal=causal, content=content, time_bias=time_bias, chan_bias=chan_bias,

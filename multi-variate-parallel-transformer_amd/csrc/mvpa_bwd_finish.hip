@@ -1,0 +1,431 @@
+// From the backward's fp32 results to the gradients of the operator's inputs (bf16, head size 64 or 128).
+//
+// mvpa_backward leaves the content share of dq, dk and dv in fp32 and the gradients G of the two bias
+// tables [B,H,N,T], [B,H,N,C]; what autograd makes of attentions/attn.py:1305-1314 turns them into
+//     dq          = dq_content + G_time k_time + G_chan k_chan          (per kv head, rows of its heads)
+//     d k_time[j] = sum_rows G_time[:, j] (q + v),   d k_chan likewise with z
+//     dv          = sum_rows G_time k_time = (column sums of G_time) k_time,  dz likewise,  du = sum_rows dq_content
+// As tensor operations this is some twenty passes over the largest tensors of the backward (casts, two
+// batched products each way, sums: 0.85 ms beside 1.7 ms of kernels at B4 H16 C64 T128).  Here G is read
+// twice, once by rows and once by columns, and nothing of its size is written:
+//   finish_rows     128 query rows per workgroup: products with the tables on MFMA, dq to bf16 where the
+//                   caller wants it, partial column sums of dq_content
+//   finish_tables   128 table rows per workgroup over a share of the query rows: G^T q on MFMA (both
+//                   operands by transposing LDS reads), column sums of G; fp32 partial results
+//   finish_reduce   the partial results to dk_time, dk_chan; finish_biases: du, dv, dz
+// Columns of G_time that the causal mask empties (j < T-1-tq) are skipped in both.  HBM bound: 0.45 ms at that
+// size (rows 187 us, tables 189, dk and dv 60), G being 400 MB.
+#include "mvpa_mfma_tools.h"
+
+namespace mvpa {
+namespace fin {
+
+constexpr int ROWS = 128;            // query rows per workgroup of finish_rows
+constexpr int JB = 64;               // table rows per step of finish_rows
+constexpr int TJ = 128, TN = 64;     // table rows per workgroup, query rows per step of finish_tables
+
+struct fin_args {
+  int32_t B, H, Hkv, T, C, N;
+  const bf16_t* q;
+  int64_t q_sb, q_sh, q_sn;
+  const bf16_t *bias_v, *bias_z, *k_time, *k_chan;
+  const float *dq, *dk, *dv, *gt, *gc;
+  bf16_t *dq_out, *dk_out, *dv_out;
+  int64_t dq_sb, dq_sh, dq_sn, dk_sb, dk_sh, dk_sn, dv_sb, dv_sh, dv_sn;
+  float *p_du, *p_tab, *p_col;       // partial results: [b,h][row tile][Dh], [part][T + C][Dh], [part][T + C]
+  float* csum;                       // [Hkv][T + C] column sums of G
+  bf16_t *du, *dvb, *dz, *dk_time, *dk_chan;
+  int32_t tj_t, tj_c, n_split, split_len;   // column tiles of the two tables; row shares and their length
+};
+
+// four consecutive fp32 of a table-gradient row as bf16; zeros past the end
+__device__ inline bf16x4 load4(const float* row, int col, int cols, bool vec) {
+  float v[4] = {0.f, 0.f, 0.f, 0.f};
+  if (vec && col + 3 < cols) {
+    const float4 x = *(const float4*)(row + col);
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (col + i < cols) v[i] = row[col + i];
+  }
+  return bf16x4{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+}
+
+// fragment of a [rows][columns] tile for a product contracted over its rows: column 32 mt + ln, rows
+// 16 s + 8 rd + 4 hh + e in element 4 rd + e (row pitch ROWB, swizzle swz_v<DH>)
+template <int DH>
+struct tr_tile {
+  static constexpr int ROWB = DH * 2;
+  static __device__ inline bf16x8 frag(const unsigned char* tile, int s, int mt, int lane) {
+    const int ln = lane & 31, hh = lane >> 5, e = (ln & 15) >> 2, aa = ln & 3, grp = ln >> 4, row0 = 4 * hh + e;
+    const unsigned char* p = tile + (16 * s + row0) * ROWB + (((4 * mt + 2 * grp + (aa >> 1)) ^ swz_v<DH>(row0)) << 4) + ((aa & 1) << 3);
+    const bf16x4 lo = el_bf16::read_tr(p), hi = el_bf16::read_tr(p + 8 * ROWB);
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  }
+  static __device__ inline int offset(int row, int col) {          // byte offset of element (row, col), col a multiple of 4
+    return row * ROWB + (((col >> 3) ^ swz_v<DH>(row)) << 4) + ((col & 4) << 1);
+  }
+};
+
+template <int DH>
+__global__ __launch_bounds__(256) void finish_rows_kernel(fin_args a) {
+  constexpr int MT = DH / 32, ROWB = DH * 2, GP = JB + 8;
+  __shared__ __attribute__((aligned(16))) bf16_t Gs[4][32 * GP];
+  __shared__ __attribute__((aligned(16))) unsigned char Ts[JB * ROWB];
+  __shared__ float red[256];
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H, g = h / (a.H / a.Hkv);
+  const int n0 = blockIdx.x * ROWS, nw = n0 + wave * 32;
+  const int64_t rbase = (int64_t)bh * a.N;
+  f32x16 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[mt][i] = 0.f;
+  const int tq_hi = min(n0 + ROWS - 1, a.N - 1) / a.C;
+#pragma unroll 1
+  for (int which = 0; which < 2; ++which) {
+    const float* G = which ? a.gc : a.gt;
+    if (!G) continue;
+    const int cols = which ? a.C : a.T;
+    const bf16_t* tab = (which ? a.k_chan : a.k_time) + (int64_t)g * cols * DH;
+    const bool vec = (cols & 3) == 0;
+    const int j_first = which ? 0 : (a.T - 1 - tq_hi) / JB * JB;
+#pragma unroll 1
+    for (int j0 = j_first; j0 < cols; j0 += JB) {
+      __syncthreads();
+      // table rows j0 .. (shared), G rows of the wave (its own): 16 lanes x 4 columns, 4 rows at a time;
+      // the four-column groups of 16 in the order 0 2 1 3, so that a lane's 8 operand elements are together
+#pragma unroll
+      for (int i = 0; i < JB * DH / 8 / 256; ++i) {
+        const int c = i * 256 + tid, r = c / (DH / 8), ch = c % (DH / 8);
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (j0 + r < cols) v = *(const u32x4*)(tab + (int64_t)(j0 + r) * DH + ch * 8);
+        *(u32x4*)(Ts + r * ROWB + ((ch ^ swz_v<DH>(r)) << 4)) = v;
+      }
+      const int c16 = lane & 15, grp4 = (c16 & 12) | ((c16 & 1) << 1) | ((c16 >> 1) & 1);
+      bf16x4 gv[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int r = i * 4 + (lane >> 4), n = nw + r;
+        gv[i] = n < a.N ? load4(G + (rbase + n) * cols, j0 + c16 * 4, cols, vec) : bf16x4{};
+      }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) *(bf16x4*)(&Gs[wave][(i * 4 + (lane >> 4)) * GP + grp4 * 4]) = gv[i];
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < JB / 16; ++s) {
+        const bf16x8 gf = *(const bf16x8*)(&Gs[wave][ln * GP + s * 16 + hh * 8]);
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_tile<DH>::frag(Ts, s, mt, lane), gf, acc[mt], 0, 0, 0);
+      }
+    }
+  }
+  // dq = content share + table shares; lane: row nw + ln, columns 32 mt + 8 a4 + 4 hh + 0..3
+  const int n = nw + ln;
+  if (n < a.N) {
+    const float* src = a.dq + (rbase + n) * DH;
+    bf16_t* dst = a.dq_out + b * a.dq_sb + h * a.dq_sh + (int64_t)n * a.dq_sn;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        const int d = mt * 32 + a4 * 8 + hh * 4;
+        const float4 c = *(const float4*)(src + d);
+        *(bf16x4*)(dst + d) = bf16x4{(__bf16)(c.x + acc[mt][a4 * 4]), (__bf16)(c.y + acc[mt][a4 * 4 + 1]),
+                                     (__bf16)(c.z + acc[mt][a4 * 4 + 2]), (__bf16)(c.w + acc[mt][a4 * 4 + 3])};
+      }
+  }
+  // column sums of the content share (the rows are in the L2 by now)
+  {
+    const int d = tid % DH;
+    float s = 0.f;
+    for (int r = tid / DH; r < ROWS; r += 256 / DH)
+      if (n0 + r < a.N) s += a.dq[(rbase + n0 + r) * DH + d];
+    red[tid] = s;
+    __syncthreads();
+    if (tid < DH) {
+#pragma unroll
+      for (int i = 1; i < 256 / DH; ++i) s += red[tid + i * DH];
+      a.p_du[((int64_t)bh * gridDim.x + blockIdx.x) * DH + d] = s;
+    }
+  }
+}
+
+// dk, dv: fp32 [B,Hkv,N,Dh] to bf16 rows at the caller's strides
+template <int DH>
+__global__ __launch_bounds__(256) void finish_kv_kernel(fin_args a) {
+  const int64_t per = (int64_t)a.B * a.Hkv * a.N * (DH / 8);
+  int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const bool is_v = i >= per;
+  if (is_v) i -= per;
+  if (i >= per) return;
+  const int ch = (int)(i % (DH / 8));
+  const int64_t r = i / (DH / 8);
+  const int n = (int)(r % a.N), bg = (int)(r / a.N), b = bg / a.Hkv, g = bg % a.Hkv;
+  const float* src = (is_v ? a.dv : a.dk) + r * DH + ch * 8;
+  bf16_t* dst = is_v ? a.dv_out + b * a.dv_sb + g * a.dv_sh + (int64_t)n * a.dv_sn
+                     : a.dk_out + b * a.dk_sb + g * a.dk_sh + (int64_t)n * a.dk_sn;
+  const float4 x = *(const float4*)src, y = *(const float4*)(src + 4);
+  *(bf16x8*)(dst + ch * 8) = bf16x8{(__bf16)x.x, (__bf16)x.y, (__bf16)x.z, (__bf16)x.w,
+                                    (__bf16)y.x, (__bf16)y.y, (__bf16)y.z, (__bf16)y.w};
+}
+
+template <int DH>
+__global__ __launch_bounds__(256) void finish_tables_kernel(fin_args a) {
+  constexpr int MT = DH / 32, GB = TJ * 2;           // bytes per G row in LDS
+  __shared__ __attribute__((aligned(16))) unsigned char Gs[TN * GB];
+  __shared__ __attribute__((aligned(16))) unsigned char Qs[TN * DH * 2];
+  __shared__ float cred[8][TJ];
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tile = blockIdx.x, split = blockIdx.y, bh = blockIdx.z, b = bh / a.H, h = bh % a.H;
+  const bool chan = tile >= a.tj_t;
+  const float* G = chan ? a.gc : a.gt;
+  const int cols = chan ? a.C : a.T, j0 = (chan ? tile - a.tj_t : tile) * TJ;
+  const int row_out = (chan ? a.T : 0) + j0;          // first row of this tile in the [T + C] tables
+  const bool vec = (cols & 3) == 0;
+  const int64_t rbase = (int64_t)bh * a.N;
+  const bf16_t* qbase = a.q + b * a.q_sb + h * a.q_sh;
+  int lo = split * a.split_len, hi = min(lo + a.split_len, a.N);
+  // query rows that reach a column of this tile: tq >= T-1-(j0+TJ-1)
+  if (!chan) lo = max(lo, max(0, a.T - j0 - TJ) * a.C / TN * TN);
+  f32x16 acc[MT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[mt][i] = 0.f;
+  float cs[4] = {0.f, 0.f, 0.f, 0.f};
+  const int gc4 = (tid & 31) * 4, gr = tid >> 5;
+  float4 gv[TN / 8];
+  u32x4 qv[TN * DH / 8 / 256];
+  auto request = [&](int n1) {
+#pragma unroll
+    for (int i = 0; i < TN / 8; ++i) {
+      const int n = n1 + gr + 8 * i;
+      gv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+      if (n < hi && G) {
+        const float* row = G + (rbase + n) * cols + j0;
+        if (vec && j0 + gc4 + 3 < cols) gv[i] = *(const float4*)(row + gc4);
+        else {
+          if (j0 + gc4 < cols) gv[i].x = row[gc4];
+          if (j0 + gc4 + 1 < cols) gv[i].y = row[gc4 + 1];
+          if (j0 + gc4 + 2 < cols) gv[i].z = row[gc4 + 2];
+          if (j0 + gc4 + 3 < cols) gv[i].w = row[gc4 + 3];
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < TN * DH / 8 / 256; ++i) {
+      const int c = i * 256 + tid, r = c / (DH / 8), ch = c % (DH / 8);
+      qv[i] = *(const u32x4*)(qbase + (int64_t)min(n1 + r, a.N - 1) * a.q_sn + ch * 8);   // G is 0 past the end
+    }
+  };
+  if (lo < hi) request(lo);
+#pragma unroll 1
+  for (int n1 = lo; n1 < hi; n1 += TN) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TN / 8; ++i) {
+      cs[0] += gv[i].x; cs[1] += gv[i].y; cs[2] += gv[i].z; cs[3] += gv[i].w;
+      *(bf16x4*)(Gs + tr_tile<128>::offset(gr + 8 * i, gc4)) =
+          bf16x4{(__bf16)gv[i].x, (__bf16)gv[i].y, (__bf16)gv[i].z, (__bf16)gv[i].w};
+    }
+#pragma unroll
+    for (int i = 0; i < TN * DH / 8 / 256; ++i) {
+      const int c = i * 256 + tid, r = c / (DH / 8), ch = c % (DH / 8);
+      *(u32x4*)(Qs + r * DH * 2 + ((ch ^ swz_v<DH>(r)) << 4)) = qv[i];
+    }
+    __syncthreads();
+    if (n1 + TN < hi) request(n1 + TN);
+#pragma unroll
+    for (int s = 0; s < TN / 16; ++s) {
+      const bf16x8 gf = tr_tile<128>::frag(Gs, s, wave, lane);
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+        acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gf, tr_tile<DH>::frag(Qs, s, mt, lane), acc[mt], 0, 0, 0);
+    }
+  }
+  const int64_t part = (int64_t)bh * a.n_split + split;
+  float* P = a.p_tab + part * (a.T + a.C) * DH;
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int j = wave * 32 + (i >> 2) * 8 + hh * 4 + (i & 3);
+      if (j0 + j < cols) P[(int64_t)(row_out + j) * DH + mt * 32 + ln] = acc[mt][i];
+    }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) cred[gr][gc4 + i] = cs[i];
+  __syncthreads();
+  if (tid < TJ && j0 + tid < cols) {
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) s += cred[i][tid];
+    a.p_col[part * (a.T + a.C) + row_out + tid] = s;
+  }
+}
+
+// one workgroup per 256 / DH table rows of a kv head
+template <int DH>
+__global__ __launch_bounds__(256) void finish_reduce_kernel(fin_args a) {
+  const int g = blockIdx.y, rows = a.T + a.C, j = blockIdx.x * (256 / DH) + threadIdx.x / DH, d = threadIdx.x % DH;
+  if (j >= rows) return;
+  const int grp = a.H / a.Hkv;
+  float s = 0.f, c = 0.f;
+  for (int b = 0; b < a.B; ++b) {
+    const int64_t p0 = ((int64_t)b * a.H + g * grp) * a.n_split;
+    const int np = grp * a.n_split;
+#pragma unroll 4
+    for (int p = 0; p < np; ++p) {
+      s += a.p_tab[((p0 + p) * rows + j) * DH + d];
+      c += a.p_col[(p0 + p) * rows + j];
+    }
+  }
+  const bool chan = j >= a.T;
+  s += c * bf16_to_f32((chan ? a.bias_z : a.bias_v)[g * DH + d]);
+  bf16_t* dst = chan ? a.dk_chan + ((int64_t)g * a.C + j - a.T) * DH : a.dk_time + ((int64_t)g * a.T + j) * DH;
+  dst[d] = f32_to_bf16(s);
+  if (d == 0) a.csum[(int64_t)g * rows + j] = c;
+}
+
+// du, dv, dz of a kv head: blockIdx.y = 0, 1, 2
+template <int DH>
+__global__ __launch_bounds__(1024) void finish_biases_kernel(fin_args a, int row_tiles) {
+  __shared__ float red[1024];
+  const int g = blockIdx.x, d = threadIdx.x % DH, sub = threadIdx.x / DH;
+  constexpr int SUBS = 1024 / DH;
+  const int grp = a.H / a.Hkv;
+  float s = 0.f;
+  if (blockIdx.y == 0) {
+    const int per = grp * row_tiles;
+    for (int i = sub; i < a.B * per; i += SUBS)
+      s += a.p_du[(((int64_t)(i / per) * a.H + g * grp) * row_tiles + i % per) * DH + d];
+  } else {
+    const bool chan = blockIdx.y == 2;
+    const int cols = chan ? a.C : a.T;
+    const bf16_t* tab = (chan ? a.k_chan : a.k_time) + (int64_t)g * cols * DH;
+    const float* c = a.csum + (int64_t)g * (a.T + a.C) + (chan ? a.T : 0);
+    for (int j = sub; j < cols; j += SUBS) s += c[j] * bf16_to_f32(tab[(int64_t)j * DH + d]);
+  }
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (sub == 0) {
+#pragma unroll
+    for (int i = 1; i < SUBS; ++i) s += red[threadIdx.x + i * DH];
+    (blockIdx.y == 0 ? a.du : blockIdx.y == 1 ? a.dvb : a.dz)[g * DH + d] = f32_to_bf16(s);
+  }
+}
+
+struct layout {
+  int64_t used = 0;
+  char* base;
+  template <typename T> T* take(int64_t n) {
+    T* p = base ? (T*)(base + used) : nullptr;
+    used += (n * (int64_t)sizeof(T) + 255) & ~(int64_t)255;
+    return p;
+  }
+};
+
+// row shares of finish_tables: enough workgroups for two rounds of the chip, whole TN-row steps
+static void row_split(const mvpa_bwd_args* b, int* n_split, int* len) {
+  const int64_t N = (int64_t)b->T * b->C;
+  const int tiles = (b->T + TJ - 1) / TJ + (b->C + TJ - 1) / TJ;
+  int64_t s = 512 / ((int64_t)tiles * b->B * b->H);
+  const int64_t most = (N + 4 * TN - 1) / (4 * TN);
+  if (s > most) s = most;
+  if (s < 1) s = 1;
+  *len = (int)(((N + s - 1) / s + TN - 1) / TN * TN);
+  *n_split = (int)((N + *len - 1) / *len);
+}
+
+static void lay_out(const mvpa_bwd_args* b, fin_args& f, mvpa_bwd_args& w, layout& l) {
+  const int64_t N = (int64_t)b->T * b->C, bhn = (int64_t)b->B * b->H * N, bgn = (int64_t)b->B * b->Hkv * N, Dh = b->Dh;
+  w = *b;
+  w.dq = l.take<float>(bhn * Dh);
+  w.dk = l.take<float>(bgn * Dh);
+  w.dv = l.take<float>(bgn * Dh);
+  w.dbias_time = l.take<float>(bhn * b->T);
+  w.dbias_chan = l.take<float>(bhn * b->C);
+  w.ws_delta = l.take<float>(bhn);
+  w.ws_time = l.take<float>(bhn * b->T);
+  w.ws_chan = l.take<float>(bhn * ((b->C + 3) / 4 * 4));
+  w.ws_qu = l.take<bf16_t>(bhn * Dh);
+  int n_split, len;
+  row_split(b, &n_split, &len);
+  f.n_split = n_split;
+  f.split_len = len;
+  f.tj_t = (b->T + TJ - 1) / TJ;
+  f.tj_c = (b->C + TJ - 1) / TJ;
+  const int64_t parts = (int64_t)b->B * b->H * n_split, rows = b->T + b->C;
+  f.p_du = l.take<float>((int64_t)b->B * b->H * ((N + ROWS - 1) / ROWS) * Dh);
+  f.p_tab = l.take<float>(parts * rows * Dh);
+  f.p_col = l.take<float>(parts * rows);
+  f.csum = l.take<float>(b->Hkv * rows);
+}
+
+template <int DH>
+static int launch_finish(const fin_args& f, hipStream_t s) {
+  const int row_tiles = (f.N + ROWS - 1) / ROWS;
+  MVPA_LAUNCH(finish_rows_kernel<DH>, dim3((unsigned)row_tiles, (unsigned)(f.B * f.H)), dim3(256), 0, s, f);
+  MVPA_LAUNCH(finish_tables_kernel<DH>, dim3((unsigned)(f.tj_t + f.tj_c), (unsigned)f.n_split, (unsigned)(f.B * f.H)),
+              dim3(256), 0, s, f);
+  const int64_t kv = 2 * (int64_t)f.B * f.Hkv * f.N * (DH / 8);
+  MVPA_LAUNCH(finish_kv_kernel<DH>, dim3((unsigned)((kv + 255) / 256)), dim3(256), 0, s, f);
+  MVPA_LAUNCH(finish_reduce_kernel<DH>, dim3((unsigned)((f.T + f.C + 256 / DH - 1) / (256 / DH)), (unsigned)f.Hkv), dim3(256), 0, s, f);
+  MVPA_LAUNCH(finish_biases_kernel<DH>, dim3((unsigned)f.Hkv, 3), dim3(1024), 0, s, f, row_tiles);
+  return take_launch_status();
+}
+
+}  // namespace fin
+}  // namespace mvpa
+
+using namespace mvpa;
+
+extern "C" size_t mvpa_backward_full_ws_bytes(const mvpa_bwd_args* a) {
+  if (!a || a->struct_size != sizeof(mvpa_bwd_args) || a->B <= 0 || a->H <= 0 || a->Hkv <= 0 || a->T <= 0 || a->C <= 0) return 0;
+  fin::fin_args f;
+  mvpa_bwd_args w;
+  fin::layout l{0, nullptr};
+  fin::lay_out(a, f, w, l);
+  return (size_t)l.used;
+}
+
+extern "C" int mvpa_backward_full(const mvpa_bwd_args* a, const mvpa_bwd_grads* o, void* ws, size_t ws_bytes, void* stream) {
+  if (!a || !o || !ws) return MVPA_ERR_NULL;
+  if (a->struct_size != sizeof(mvpa_bwd_args) || o->struct_size != sizeof(mvpa_bwd_grads)) return MVPA_ERR_STRUCT;
+  if (a->dtype != MVPA_BF16 || (a->Dh != 64 && a->Dh != 128)) return MVPA_ERR_UNSUPPORTED;
+  if (!o->dq || !o->dk || !o->dv || !o->dbias_u || !o->dbias_v || !o->dbias_z || !o->dk_time || !o->dk_chan) return MVPA_ERR_NULL;
+  if ((uintptr_t)ws & 255) return MVPA_ERR_ALIGN;
+  if (((uintptr_t)o->dq | (uintptr_t)o->dk | (uintptr_t)o->dv) & 15) return MVPA_ERR_ALIGN;
+  if ((o->dq_stride_b | o->dq_stride_h | o->dq_stride_n | o->dk_stride_b | o->dk_stride_h | o->dk_stride_n |
+       o->dv_stride_b | o->dv_stride_h | o->dv_stride_n) & 7) return MVPA_ERR_ALIGN;
+  fin::fin_args f = {};
+  mvpa_bwd_args w;
+  fin::layout l{0, (char*)ws};
+  fin::lay_out(a, f, w, l);
+  if ((size_t)l.used > ws_bytes) return MVPA_ERR_WS_SIZE;
+  if (!mvpa_bwd_query_mfma_supported(&w)) return MVPA_ERR_UNSUPPORTED;
+  const int st = mvpa_backward(&w, stream);
+  if (st != MVPA_OK) return st;
+  f.B = a->B; f.H = a->H; f.Hkv = a->Hkv; f.T = a->T; f.C = a->C; f.N = a->T * a->C;
+  f.q = (const bf16_t*)a->q;
+  f.q_sb = a->q_stride_b; f.q_sh = a->q_stride_h; f.q_sn = a->q_stride_n;
+  f.bias_v = (const bf16_t*)a->bias_v; f.bias_z = (const bf16_t*)a->bias_z;
+  f.k_time = (const bf16_t*)a->k_time; f.k_chan = (const bf16_t*)a->k_chan;
+  f.dq = w.dq; f.dk = w.dk; f.dv = w.dv;
+  // a bias term that is switched off takes no part in the forward: its table, its query bias and the query
+  // get nothing through it
+  f.gt = (a->flags & MVPA_FLAG_TIME_BIAS) ? w.dbias_time : nullptr;
+  f.gc = (a->flags & MVPA_FLAG_CHAN_BIAS) ? w.dbias_chan : nullptr;
+  f.dq_out = (bf16_t*)o->dq; f.dk_out = (bf16_t*)o->dk; f.dv_out = (bf16_t*)o->dv;
+  f.dq_sb = o->dq_stride_b; f.dq_sh = o->dq_stride_h; f.dq_sn = o->dq_stride_n;
+  f.dk_sb = o->dk_stride_b; f.dk_sh = o->dk_stride_h; f.dk_sn = o->dk_stride_n;
+  f.dv_sb = o->dv_stride_b; f.dv_sh = o->dv_stride_h; f.dv_sn = o->dv_stride_n;
+  f.du = (bf16_t*)o->dbias_u; f.dvb = (bf16_t*)o->dbias_v; f.dz = (bf16_t*)o->dbias_z;
+  f.dk_time = (bf16_t*)o->dk_time; f.dk_chan = (bf16_t*)o->dk_chan;
+  return a->Dh == 64 ? fin::launch_finish<64>(f, (hipStream_t)stream) : fin::launch_finish<128>(f, (hipStream_t)stream);
+}

@@ -149,6 +149,84 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, chan_valid, sm_scale, window, flags)
+//   -> (dq, du, dvb, dz, dk, dk_time, dk_chan, dv) in bf16 | status
+PyObject* py_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 15, "backward takes 15 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const auto dt = at::kBFloat16;
+  const Tensor &q = tensor_of(args[0]), &k = tensor_of(args[1]), &v = tensor_of(args[2]), &o = tensor_of(args[3]);
+  Tensor d_o = tensor_of(args[4]);
+  for (const Tensor* t : {&q, &k, &v, &o, (const Tensor*)&d_o}) {
+    on_gpu(*t);
+    TORCH_CHECK(t->dim() == 4 && t->scalar_type() == dt, "backward: q, k, v, o, d_o are bf16 with four dimensions");
+  }
+  TORCH_CHECK(o.sizes() == q.sizes() && d_o.sizes() == q.sizes() && k.sizes() == v.sizes(), "backward: shapes differ");
+  if (d_o.stride(3) != 1 || ((d_o.stride(0) | d_o.stride(1) | d_o.stride(2)) & 7)) d_o = d_o.contiguous();
+  const Tensor lse = as_operand(tensor_of(args[5]), at::kFloat);
+  const Tensor u = as_operand(tensor_of(args[6]), dt), vb = as_operand(tensor_of(args[7]), dt),
+               z = as_operand(tensor_of(args[8]), dt), kt = as_operand(tensor_of(args[9]), dt),
+               kc = as_operand(tensor_of(args[10]), dt);
+  mvpa_bwd_args a;
+  std::memset(&a, 0, sizeof(a));
+  a.struct_size = sizeof(a);
+  a.dtype = MVPA_BF16;
+  a.sm_scale = (float)PyFloat_AsDouble(args[12]);
+  a.window = (int32_t)PyLong_AsLong(args[13]);
+  a.flags = (uint32_t)PyLong_AsUnsignedLong(args[14]);
+  if (PyErr_Occurred()) return nullptr;
+  a.B = (int32_t)q.size(0);
+  a.H = (int32_t)q.size(1);
+  a.Dh = (int32_t)q.size(3);
+  a.Hkv = (int32_t)k.size(1);
+  a.T = (int32_t)kt.size(-2);
+  a.C = (int32_t)kc.size(-2);
+  TORCH_CHECK(q.size(2) == (int64_t)a.T * a.C && k.size(2) == q.size(2) && lse.numel() == q.numel() / a.Dh &&
+                  u.numel() == (int64_t)a.Hkv * a.Dh && kt.numel() == (int64_t)a.Hkv * a.T * a.Dh &&
+                  kc.numel() == (int64_t)a.Hkv * a.C * a.Dh,
+              "backward: shapes differ");
+  TORCH_CHECK_VALUE(q.stride(3) == 1 && k.stride(3) == 1 && v.stride(3) == 1 && o.stride(3) == 1,
+                    "q, k, v, o: last dim must be contiguous");
+  a.q = q.data_ptr(); a.k = k.data_ptr(); a.v = v.data_ptr(); a.o = o.data_ptr(); a.d_o = d_o.data_ptr();
+  a.q_stride_b = q.stride(0); a.q_stride_h = q.stride(1); a.q_stride_n = q.stride(2);
+  a.k_stride_b = k.stride(0); a.k_stride_h = k.stride(1); a.k_stride_n = k.stride(2);
+  a.v_stride_b = v.stride(0); a.v_stride_h = v.stride(1); a.v_stride_n = v.stride(2);
+  a.o_stride_b = o.stride(0); a.o_stride_h = o.stride(1); a.o_stride_n = o.stride(2);
+  a.do_stride_b = d_o.stride(0); a.do_stride_h = d_o.stride(1); a.do_stride_n = d_o.stride(2);
+  a.bias_u = u.data_ptr(); a.bias_v = vb.data_ptr(); a.bias_z = z.data_ptr();
+  a.k_time = kt.data_ptr(); a.k_chan = kc.data_ptr();
+  a.lse = (const float*)lse.data_ptr();
+  Tensor cv;
+  if (!is_none(args[11])) {
+    cv = as_operand(tensor_of(args[11]), tensor_of(args[11]).scalar_type() == at::kBool ? at::kBool : at::kByte);
+    a.chan_valid = (const uint8_t*)cv.data_ptr();
+  }
+  const auto opt = q.options();
+  Tensor dq = at::empty(q.sizes(), opt, at::MemoryFormat::Contiguous), dk = at::empty(k.sizes(), opt, at::MemoryFormat::Contiguous),
+         dv = at::empty(v.sizes(), opt, at::MemoryFormat::Contiguous);
+  Tensor du = at::empty(u.sizes(), opt), dvb = at::empty(vb.sizes(), opt), dz = at::empty(z.sizes(), opt),
+         dkt = at::empty(kt.sizes(), opt), dkc = at::empty(kc.sizes(), opt);
+  mvpa_bwd_grads g;
+  std::memset(&g, 0, sizeof(g));
+  g.struct_size = sizeof(g);
+  g.dq = dq.data_ptr(); g.dk = dk.data_ptr(); g.dv = dv.data_ptr();
+  g.dq_stride_b = dq.stride(0); g.dq_stride_h = dq.stride(1); g.dq_stride_n = dq.stride(2);
+  g.dk_stride_b = dk.stride(0); g.dk_stride_h = dk.stride(1); g.dk_stride_n = dk.stride(2);
+  g.dv_stride_b = dv.stride(0); g.dv_stride_h = dv.stride(1); g.dv_stride_n = dv.stride(2);
+  g.dbias_u = du.data_ptr(); g.dbias_v = dvb.data_ptr(); g.dbias_z = dz.data_ptr();
+  g.dk_time = dkt.data_ptr(); g.dk_chan = dkc.data_ptr();
+  const int64_t bytes = (int64_t)mvpa_backward_full_ws_bytes(&a);
+  Tensor ws = at::empty({bytes}, opt.dtype(at::kByte));
+  const int st = mvpa_backward_full(&a, &g, ws.data_ptr(), (size_t)bytes, current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* r = PyTuple_New(8);
+  int i = 0;
+  for (Tensor* t : {&dq, &du, &dvb, &dz, &dk, &dkt, &dkc, &dv}) PyTuple_SET_ITEM(r, i++, THPVariable_Wrap(*t));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
 // ---- dense ops ------------------------------------------------------------------------------
 // linear(x, w) -> x @ w^T, bf16, plain product | status
 PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
@@ -378,6 +456,7 @@ PyObject* py_run(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 PyMethodDef kMethods[] = {
     {"forward", (PyCFunction)(void*)py_forward, METH_FASTCALL, "fused MVPA forward"},
+    {"backward", (PyCFunction)(void*)py_backward, METH_FASTCALL, "backward of the fused MVPA forward, bf16"},
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},

@@ -25,7 +25,7 @@ FLAG_LAST_STEP = 32
 FLAG_RING = 64
 FLAG_CAUSAL, FLAG_CONTENT, FLAG_TIME_BIAS, FLAG_CHAN_BIAS, FLAG_FP8_QK = 1, 2, 4, 8, 16
 
-ERR_HEAD_DIM, ERR_HEAD_RATIO, ERR_CTX, ERR_SHAPE = -2, -3, -4, -5
+ERR_HEAD_DIM, ERR_HEAD_RATIO, ERR_CTX, ERR_SHAPE, ERR_UNSUPPORTED = -2, -3, -4, -5, -8
 
 
 class MvpaFwdArgs(ctypes.Structure):
@@ -440,6 +440,21 @@ def mvpa_backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, *,
     a.ws_qu = ws_qu.data_ptr()
     _check(lib.mvpa_backward(ctypes.byref(a), _stream()))
     return dq, dk, dv, dbt, dbc
+
+
+def mvpa_backward_full(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, *, sm_scale: float, window: int = 10,
+                       content: bool = True, time_bias: bool = True, chan_bias: bool = True,
+                       chan_valid: Optional[torch.Tensor] = None):
+    """Gradients of mvpa_forward's inputs in bf16, (dq, du, dvb, dz, dk, dk_time, dk_chan, dv): mvpa_backward
+    and the products that finish its table gradients, all in the library.  None for shapes or layouts that
+    the matrix-core backward does not take."""
+    flags = (FLAG_CAUSAL | (FLAG_CONTENT if content else 0) | (FLAG_TIME_BIAS if time_bias else 0) |
+             (FLAG_CHAN_BIAS if chan_bias else 0))
+    r = (_ext or load_ext()).backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, chan_valid, float(sm_scale),
+                                      window, flags)
+    if type(r) is int and r == ERR_UNSUPPORTED:
+        return None
+    return _taken(r)
 
 
 def debug_maps(T: int, C: int, window: int = 10, flags: int = 15, chan_valid=None,

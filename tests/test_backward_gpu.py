@@ -146,6 +146,27 @@ def test_backward_bf16_mfma_query_pass(case):
         assert rel <= 2e-2, (n, rel)
 
 
+@pytest.mark.parametrize("cfg", [
+    dict(B=1, C=5, T=130, H=2, Hkv=1, Dh=64, window=4),       # a second tile of 2 time-table rows; GQA
+    dict(B=2, C=4, T=129, H=1, Hkv=1, Dh=128, window=10),     # one row in it; rows of 516 bytes (no 16-byte loads)
+    # one ragged step of everything.  Not fewer rows: delta = rowsum(d_o o) takes o in bf16 and is off by up to
+    # 2^-9 sum |d_o o| ~ 2^-9 * 64 * 0.6 = 0.08, a fiftieth of a row's dP - delta (~ 4 for unit inputs) before
+    # rows average out; T = 2, C = 1 read 2.05e-2
+    dict(B=1, C=3, T=4, H=1, Hkv=1, Dh=64, window=0),
+], ids=lambda c: "B{B}C{C}T{T}H{H}g{Hkv}D{Dh}".format(**c))
+def test_backward_finish_tile_edges(cfg):
+    """Tiles of 128 table rows and 128 query rows, 64 columns a step; the bound is the file's for bf16."""
+    cfg = dict(cfg)
+    window = cfg.pop("window")
+    inp = make_mvpa_inputs(seed=17, qkv_unit=True, **cfg).round_to(torch.bfloat16)
+    d_out = torch.randn(inp.q.shape, generator=torch.Generator().manual_seed(8)).bfloat16().float()
+    _, ref = _oracle_grads(inp, d_out, window)
+    _, got = _gpu_grads(inp, d_out, window, torch.bfloat16)
+    for n in NAMES:
+        rel = (got[n].double() - ref[n]).norm().item() / max(ref[n].norm().item(), 1e-30)
+        assert rel <= 2e-2, (n, rel)
+
+
 def test_backward_rows_are_causal():
     """do confined to the first time steps must leave dk/dv of later keys exactly zero."""
     inp = make_mvpa_inputs(B=1, C=4, T=10, H=2, Hkv=2, Dh=32, seed=1, qkv_unit=True)
