@@ -436,6 +436,20 @@ int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64
 int mvpa_mean_rows_bf16(const void* x, void* out, int64_t groups, int64_t rows, int32_t cols, int64_t ldx,
                         int64_t group_stride, void* stream);
 
+/* Backward of y = RMSNorm(x) * weight over contiguous rows [rows, cols], cols <= 4096 (else
+ * MVPA_ERR_UNSUPPORTED): dx = the input's gradient (+ res, the gradient that reaches the rows past the
+ * norm, where given), dw = the weight's.  dy is bf16; x, res and dx are fp32 with x_f32 and bf16 otherwise,
+ * weight and dw likewise with w_f32.  dx or dw may be null; dw needs ws
+ * (mvpa_rmsnorm_backward_ws_bytes(rows, cols) bytes, 16-byte aligned). */
+size_t mvpa_rmsnorm_backward_ws_bytes(int64_t rows, int32_t cols);
+int mvpa_rmsnorm_backward(const void* x, const void* weight, const void* dy, const void* res, void* dx, void* dw,
+                          void* ws, int64_t rows, int32_t cols, float eps, int32_t x_f32, int32_t w_f32, void* stream);
+
+/* out = silu(gate) * up for contiguous bf16 rows gu = [gate | up] of 2 n columns, and its backward
+ * dgu = [dgate | dup] (models/mvpformer.py:114); n a multiple of 8, 16-byte aligned pointers. */
+int mvpa_silu_gate_bf16(const void* gu, void* out, int64_t rows, int32_t n, void* stream);
+int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void* dgu, int64_t rows, int32_t n, void* stream);
+
 /* ---- the stack of parallel blocks as one call ---------------------------------------------------
  * models/mvpformer.py:296-381: every block x + attn(ln_1(x)) + mlp(ln_1(x)), then ln_f, on bf16 rows.
  * The launches are the library's own (mvpa_forward and the products around it); one call enqueues

@@ -47,46 +47,99 @@ class FlashMVPA(torch.autograd.Function):
             if grads is not None:
                 return (*(g.to(t.dtype) for g, t in zip(grads, (q, u, vb, z, k, k_time, k_chan, v))),
                         None, None, None, None, None, None, None, None)
-        dq_c, dk, dv, dbt, dbc = mvpa_hip.mvpa_backward(
-            q, k, v, out, d_out.contiguous(), lse, u, vb, z, k_time, k_chan, sm_scale=sm_scale,
-            window=window, causal=causal, content=content, time_bias=time_bias, chan_bias=chan_bias,
-            chan_valid=chan_valid, key_bias=key_bias)
-        B, H, N, Dh = q.shape
-        Hkv = k.shape[1]
-        grp = H // Hkv
-        rows = grp * N                                  # the query rows of a kv head, heads side by side
-        dq = dq_c.view(B, Hkv, rows, Dh)
-        du = dq.sum(dim=(0, 2)) if content else torch.zeros_like(u, dtype=torch.float32)
-        # bf16 runs take these products in bf16 (fp32 accumulation), as the kernels take theirs
-        cd = torch.bfloat16 if q.dtype == torch.bfloat16 else torch.float32
-        q2 = q.reshape(B, Hkv, rows, Dh)
-
-        # Per kv head g the table is (q + bias) @ table[g]^T, so with its gradient G [rows, J]:
-        #   d(q + bias) = G @ table[g]            - one batched product over (b, g), and
-        #   d table[g]  = sum_b G^T @ (q + bias)  - one batched product with G read transposed in
-        # place, then a sum over b (an einsum over (b, r, n) would first copy G, the largest tensor
-        # of the backward, into a [g, (b r n), J] layout).  A bias term that is switched off takes
-        # no part in the forward: its table, its query bias and the query get nothing through it.
-        def finish(grad_table, table, bias):
-            g2 = grad_table.view(B, Hkv, rows, -1).to(cd)
-            dq_share = torch.matmul(g2, table.to(cd)).float()          # [B,Hkv,rows,Dh]
-            qb = (q2.float() + bias.float()[None, :, None, :]).to(cd)
-            dtab = torch.matmul(g2.transpose(2, 3), qb).float().sum(0)  # [Hkv,J,Dh]
-            return dq_share, dq_share.sum(dim=(0, 2)), dtab
-
-        if time_bias:
-            dq_t, dvb, dk_time = finish(dbt, k_time, vb)
-            dq = dq + dq_t
-        else:
-            dvb, dk_time = torch.zeros_like(vb, dtype=torch.float32), torch.zeros_like(k_time, dtype=torch.float32)
-        if chan_bias:
-            dq_ch, dz, dk_chan = finish(dbc, k_chan, z)
-            dq = dq + dq_ch
-        else:
-            dz, dk_chan = torch.zeros_like(z, dtype=torch.float32), torch.zeros_like(k_chan, dtype=torch.float32)
-        return (dq.view(B, H, N, Dh).to(q.dtype), du.to(u.dtype), dvb.to(vb.dtype), dz.to(z.dtype),
-                dk.to(k.dtype), dk_time.to(k_time.dtype), dk_chan.to(k_chan.dtype), dv.to(v.dtype),
+        return (*_operator_grads(q, u, vb, z, k, k_time, k_chan, v, out, lse, d_out, *ctx.conf),
                 None, None, None, None, None, None, None, None)
+
+
+def _operator_grads(q, u, vb, z, k, k_time, k_chan, v, out, lse, d_out, causal, sm_scale, window, time_bias, chan_bias,
+                    chan_valid, content, key_bias):
+    """Gradients of the operator's tensors for every shape and type: mvpa_backward and the products of its
+    table gradients as tensor operations."""
+    dq_c, dk, dv, dbt, dbc = mvpa_hip.mvpa_backward(
+        q, k, v, out, d_out.contiguous(), lse, u, vb, z, k_time, k_chan, sm_scale=sm_scale,
+        window=window, causal=causal, content=content, time_bias=time_bias, chan_bias=chan_bias,
+        chan_valid=chan_valid, key_bias=key_bias)
+    B, H, N, Dh = q.shape
+    Hkv = k.shape[1]
+    grp = H // Hkv
+    rows = grp * N                                  # the query rows of a kv head, heads side by side
+    dq = dq_c.view(B, Hkv, rows, Dh)
+    du = dq.sum(dim=(0, 2)) if content else torch.zeros_like(u, dtype=torch.float32)
+    # bf16 runs take these products in bf16 (fp32 accumulation), as the kernels take theirs
+    cd = torch.bfloat16 if q.dtype == torch.bfloat16 else torch.float32
+    q2 = q.reshape(B, Hkv, rows, Dh)
+
+    # Per kv head g the table is (q + bias) @ table[g]^T, so with its gradient G [rows, J]:
+    #   d(q + bias) = G @ table[g]            - one batched product over (b, g), and
+    #   d table[g]  = sum_b G^T @ (q + bias)  - one batched product with G read transposed in
+    # place, then a sum over b (an einsum over (b, r, n) would first copy G, the largest tensor
+    # of the backward, into a [g, (b r n), J] layout).  A bias term that is switched off takes
+    # no part in the forward: its table, its query bias and the query get nothing through it.
+    def finish(grad_table, table, bias):
+        g2 = grad_table.view(B, Hkv, rows, -1).to(cd)
+        dq_share = torch.matmul(g2, table.to(cd)).float()          # [B,Hkv,rows,Dh]
+        qb = (q2.float() + bias.float()[None, :, None, :]).to(cd)
+        dtab = torch.matmul(g2.transpose(2, 3), qb).float().sum(0)  # [Hkv,J,Dh]
+        return dq_share, dq_share.sum(dim=(0, 2)), dtab
+
+    if time_bias:
+        dq_t, dvb, dk_time = finish(dbt, k_time, vb)
+        dq = dq + dq_t
+    else:
+        dvb, dk_time = torch.zeros_like(vb, dtype=torch.float32), torch.zeros_like(k_time, dtype=torch.float32)
+    if chan_bias:
+        dq_ch, dz, dk_chan = finish(dbc, k_chan, z)
+        dq = dq + dq_ch
+    else:
+        dz, dk_chan = torch.zeros_like(z, dtype=torch.float32), torch.zeros_like(k_chan, dtype=torch.float32)
+    return (dq.view(B, H, N, Dh).to(q.dtype), du.to(u.dtype), dvb.to(vb.dtype), dz.to(z.dtype),
+            dk.to(k.dtype), dk_time.to(k_time.dtype), dk_chan.to(k_chan.dtype), dv.to(v.dtype))
+
+
+class FlashMVPAPacked(torch.autograd.Function):
+    """FlashMVPA on the rows of one projection: qkv [B,N,(H + 2 Hkv) Dh] holds query, key and value heads
+    side by side, the result [B,N,H,Dh] the merged heads, and the gradient of qkv is written in its own
+    layout (as slices of a tensor, each of the three would be copied into rows of zeros and added)."""
+
+    @staticmethod
+    def supported(qkv, dh, c_len) -> bool:
+        return (qkv.is_cuda and qkv.dtype == torch.bfloat16 and dh in (64, 128) and c_len <= 128
+                and qkv.is_contiguous())
+
+    @staticmethod
+    def _heads(rows, h, hkv, dh):
+        q, k, v = rows.unflatten(-1, (h + 2 * hkv, dh)).split((h, hkv, hkv), 2)
+        return q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2)
+
+    @staticmethod
+    def forward(ctx, qkv, u, vb, z, k_time, k_chan, heads, sm_scale, window, chan_valid, content):
+        hkv, dh = u.shape
+        q, k, v = FlashMVPAPacked._heads(qkv, heads, hkv, dh)
+        merged = torch.empty((qkv.shape[0], qkv.shape[1], heads, dh), dtype=qkv.dtype, device=qkv.device)
+        _, lse = mvpa_hip.mvpa_forward(q, k, v, u, vb, z, k_time, k_chan, sm_scale=sm_scale, window=window,
+                                       content=content, chan_valid=chan_valid, out=merged.transpose(1, 2),
+                                       return_lse=True)
+        ctx.save_for_backward(qkv, u, vb, z, k_time, k_chan, merged, lse)
+        ctx.conf = (heads, sm_scale, window, chan_valid, content)
+        return merged
+
+    @staticmethod
+    def backward(ctx, d_merged):
+        qkv, u, vb, z, k_time, k_chan, merged, lse = ctx.saved_tensors
+        heads, sm_scale, window, chan_valid, content = ctx.conf
+        q, k, v = FlashMVPAPacked._heads(qkv, heads, *u.shape)
+        d_qkv = torch.empty_like(qkv)
+        out, d_out = merged.transpose(1, 2), d_merged.transpose(1, 2)
+        grads = mvpa_hip.mvpa_backward_full(q, k, v, out, d_out, lse, u, vb, z, k_time, k_chan, sm_scale=sm_scale,
+                                            window=window, content=content, chan_valid=chan_valid,
+                                            out=FlashMVPAPacked._heads(d_qkv, heads, *u.shape))
+        if grads is None:                                   # a shape the matrix-core backward refuses
+            grads = _operator_grads(q, u, vb, z, k, k_time, k_chan, v, out, lse, d_out, True, sm_scale, window,
+                                    True, True, chan_valid, content, None)
+            d_qkv = torch.cat([grads[i] for i in (0, 4, 7)], 1).transpose(1, 2).reshape(qkv.shape)
+        _, du, dvb, dz, _, dk_time, dk_chan, _ = grads
+        return (d_qkv, *(g.to(t.dtype) for g, t in zip((du, dvb, dz, dk_time, dk_chan), (u, vb, z, k_time, k_chan))),
+                None, None, None, None, None)
 
 
 def dropout_key_scale(p_drop, time_ctx, chan_ctx, device, generator=None, time_keep=None, chan_keep=None):

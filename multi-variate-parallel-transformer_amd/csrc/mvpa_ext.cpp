@@ -11,6 +11,7 @@
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <string>
@@ -149,11 +150,11 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, chan_valid, sm_scale, window, flags)
-//   -> (dq, du, dvb, dz, dk, dk_time, dk_chan, dv) in bf16 | status
+// backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, chan_valid, sm_scale, window, flags[, dq, dk, dv])
+//   -> (dq, du, dvb, dz, dk, dk_time, dk_chan, dv) in bf16 | status.  dq, dk, dv: views that receive the gradients
 PyObject* py_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK(n == 15, "backward takes 15 arguments");
+  TORCH_CHECK(n == 15 || n == 18, "backward takes 15 or 18 arguments");
   at::AutoDispatchBelowADInplaceOrView guard;
   const auto dt = at::kBFloat16;
   const Tensor &q = tensor_of(args[0]), &k = tensor_of(args[1]), &v = tensor_of(args[2]), &o = tensor_of(args[3]);
@@ -203,8 +204,19 @@ PyObject* py_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
     a.chan_valid = (const uint8_t*)cv.data_ptr();
   }
   const auto opt = q.options();
-  Tensor dq = at::empty(q.sizes(), opt, at::MemoryFormat::Contiguous), dk = at::empty(k.sizes(), opt, at::MemoryFormat::Contiguous),
-         dv = at::empty(v.sizes(), opt, at::MemoryFormat::Contiguous);
+  Tensor dq, dk, dv;
+  if (n == 18) {
+    dq = tensor_of(args[15]); dk = tensor_of(args[16]); dv = tensor_of(args[17]);
+    for (const Tensor* t : {(const Tensor*)&dq, (const Tensor*)&dk, (const Tensor*)&dv}) {
+      on_gpu(*t);
+      TORCH_CHECK(t->scalar_type() == dt && t->dim() == 4 && t->stride(3) == 1, "backward: dq, dk, dv are bf16 with unit last stride");
+    }
+    TORCH_CHECK(dq.sizes() == q.sizes() && dk.sizes() == k.sizes() && dv.sizes() == k.sizes(), "backward: shapes differ");
+  } else {
+    dq = at::empty(q.sizes(), opt, at::MemoryFormat::Contiguous);
+    dk = at::empty(k.sizes(), opt, at::MemoryFormat::Contiguous);
+    dv = at::empty(v.sizes(), opt, at::MemoryFormat::Contiguous);
+  }
   Tensor du = at::empty(u.sizes(), opt), dvb = at::empty(vb.sizes(), opt), dz = at::empty(z.sizes(), opt),
          dkt = at::empty(kt.sizes(), opt), dkc = at::empty(kc.sizes(), opt);
   mvpa_bwd_grads g;
@@ -284,6 +296,67 @@ PyObject* py_mean_rows(PyObject*, PyObject* arg) {
   Tensor y = at::empty({x.size(0), x.size(2)}, x.options());
   const int st = mvpa_mean_rows_bf16(x.data_ptr(), y.data_ptr(), x.size(0), x.size(1), (int32_t)x.size(2), x.stride(1),
                                      x.stride(0), current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
+// ---- row operations of the training path -------------------------------------------------------
+bool f32_or_bf16(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+
+// norm_backward(x, weight, dy, res | None, eps, need_dx, need_dw) -> (dx | None, dw | None) | status
+PyObject* py_norm_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 7, "norm_backward takes 7 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor x = as_operand(tensor_of(args[0]), tensor_of(args[0]).scalar_type());
+  const Tensor w = as_operand(tensor_of(args[1]), tensor_of(args[1]).scalar_type());
+  const Tensor dy = as_operand(tensor_of(args[2]), at::kBFloat16);
+  TORCH_CHECK_TYPE(f32_or_bf16(x) && f32_or_bf16(w), "norm_backward: fp32 or bf16");
+  const int64_t cols = x.size(-1), rows = x.numel() / std::max<int64_t>(cols, 1);
+  Tensor res, dx, dw, ws;
+  if (!is_none(args[3])) res = as_operand(tensor_of(args[3]), x.scalar_type());
+  TORCH_CHECK(dy.sizes() == x.sizes() && w.numel() == cols && (!res.defined() || res.sizes() == x.sizes()),
+              "norm_backward: shapes differ");
+  const double eps = PyFloat_AsDouble(args[4]);
+  if (PyErr_Occurred()) return nullptr;
+  if (args[5] == Py_True) dx = at::empty_like(x);
+  if (args[6] == Py_True) {
+    dw = at::empty(w.sizes(), w.options());
+    ws = at::empty({(int64_t)mvpa_rmsnorm_backward_ws_bytes(rows, (int32_t)cols)}, x.options().dtype(at::kByte));
+  }
+  const int st = mvpa_rmsnorm_backward(x.data_ptr(), w.data_ptr(), dy.data_ptr(), res.defined() ? res.data_ptr() : nullptr,
+                                       dx.defined() ? dx.data_ptr() : nullptr, dw.defined() ? dw.data_ptr() : nullptr,
+                                       ws.defined() ? ws.data_ptr() : nullptr, rows, (int32_t)cols, (float)eps,
+                                       x.scalar_type() == at::kFloat, w.scalar_type() == at::kFloat, current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* r = PyTuple_New(2);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(dx));           // an undefined tensor comes out as None
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(dw));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// silu_gate(gu [.., 2n]) -> [.., n];  silu_gate(gu, d [.., n]) -> the gradient of gu | status
+PyObject* py_silu_gate(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 1 || n == 2, "silu_gate takes gu and, for the backward, the gradient");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor gu = as_operand(tensor_of(args[0]), at::kBFloat16);
+  TORCH_CHECK(gu.dim() >= 1 && gu.size(-1) % 2 == 0 && gu.numel() > 0, "silu_gate: rows of gate and up");
+  const int64_t cols = gu.size(-1) / 2, rows = gu.numel() / (2 * cols);
+  std::vector<int64_t> shape(gu.sizes().begin(), gu.sizes().end());
+  shape.back() = cols;
+  Tensor y;
+  int st;
+  if (n == 1) {
+    y = at::empty(shape, gu.options());
+    st = mvpa_silu_gate_bf16(gu.data_ptr(), y.data_ptr(), rows, (int32_t)cols, current_stream());
+  } else {
+    const Tensor d = as_operand(tensor_of(args[1]), at::kBFloat16);
+    TORCH_CHECK(d.sizes() == at::IntArrayRef(shape), "silu_gate: shapes differ");
+    y = at::empty_like(gu);
+    st = mvpa_silu_gate_backward_bf16(gu.data_ptr(), d.data_ptr(), y.data_ptr(), rows, (int32_t)cols, current_stream());
+  }
   return st == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(st);
   END_HANDLE_TH_ERRORS
 }
@@ -460,6 +533,8 @@ PyMethodDef kMethods[] = {
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
+    {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},
+    {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
     {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
     {"plan_current", (PyCFunction)py_plan_current, METH_O, "whether the weights a plan was made from are unchanged"},
     {"run", (PyCFunction)(void*)py_run, METH_FASTCALL, "a stack of blocks on one plan"},

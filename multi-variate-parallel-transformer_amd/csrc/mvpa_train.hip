@@ -1,0 +1,285 @@
+// Row operations of the training path: backward of RMSNorm with the residual's gradient, and the gated
+// activation of the MLP with its backward (models/mvpformer.py:132-147).
+//
+// All are bound by HBM: each input is read once and each result written once, where the tensor
+// expressions they stand for walked fp32 copies of their operands (RMSNorm backward: a dozen passes).
+// 6400 rows: norm backward with residual 768 columns 20 us, gate of 2048 columns 18 us (4.5 TB/s), its
+// backward 23 us (5.6 TB/s).  A fine-tuning pass of twelve such blocks 21.8 -> 15.9 ms.
+#include "mvpa_common.h"
+
+namespace mvpa {
+namespace train {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2;
+
+constexpr int MAX_COLS = 4096;       // 16 chunks of 4 columns per lane
+constexpr int MAX_GROUPS = 512;      // workgroups of the row pass = partial sums per column of the weight gradient
+
+__device__ inline float wave_sum(float x) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
+  return x;
+}
+
+__device__ inline void load4(const float* p, float (&v)[4]) {
+  const f32x4 x = *(const f32x4*)p;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = x[i];
+}
+__device__ inline void load4(const bf16_t* p, float (&v)[4]) {
+  const u32x2 x = *(const u32x2*)p;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    v[2 * i] = __uint_as_float(x[i] << 16);
+    v[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
+  }
+}
+__device__ inline uint32_t pack2(float lo, float hi) { return (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16); }
+__device__ inline void store4(float* p, const float (&v)[4]) { *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]}; }
+__device__ inline void store4(bf16_t* p, const float (&v)[4]) { *(u32x2*)p = u32x2{pack2(v[0], v[1]), pack2(v[2], v[3])}; }
+
+// four columns of a row, guarded at the end of the row where rows are not whole chunks
+template <bool VEC, typename T>
+__device__ inline void get4(const T* row, int c, int cols, float (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = 0.f;
+  if (VEC) {
+    if (c < cols) load4(row + c, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c + i < cols) v[i] = io<T>::load(row + c + i);
+  }
+}
+template <bool VEC, typename T>
+__device__ inline void put4(T* row, int c, int cols, const float (&v)[4]) {
+  if (VEC) {
+    if (c < cols) store4(row + c, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (c + i < cols) io<T>::store(row + c + i, v[i]);
+  }
+}
+
+// y = x r w with r = rsqrt(mean(x^2) + eps):   dx = r w dy - x r^3 mean(x w dy) (+ res),   dw = sum_rows dy x r
+// A wave owns whole rows, a lane the same columns of each of them: the row is in registers between its
+// two sums and its result, and the lane's share of dw stays there over all rows.  HBM bound.  512 workgroups:
+// with one per four rows the partial sums of dw are as many bytes as a row operand.
+template <typename TX, typename TW, int NCH, bool VEC>
+__global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restrict__ x, const TW* __restrict__ w,
+                                                               const bf16_t* __restrict__ dy, const TX* __restrict__ res,
+                                                               TX* __restrict__ dx, float* __restrict__ part,
+                                                               int64_t rows, int cols, float eps) {
+  __shared__ float red[3][256];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  float wv[NCH][4], acc[NCH][4];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    get4<VEC>(w, (i * 64 + lane) * 4, cols, wv[i]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+  }
+  const float rcols = 1.f / (float)cols;
+  for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
+    float xv[NCH][4], gv[NCH][4];
+    float ss = 0.f, dot = 0.f;
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      get4<VEC>(x + row * cols, (i * 64 + lane) * 4, cols, xv[i]);
+      get4<VEC>(dy + row * cols, (i * 64 + lane) * 4, cols, gv[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        ss += xv[i][j] * xv[i][j];
+        dot += xv[i][j] * (gv[i][j] * wv[i][j]);
+      }
+    ss = wave_sum(ss);
+    dot = wave_sum(dot);
+    const float r = rsqrtf(ss * rcols + eps), k = r * r * r * (dot * rcols);
+#pragma unroll
+    for (int i = 0; i < NCH; ++i) {
+      const int c = (i * 64 + lane) * 4;
+      if (dx) {
+        float o[4], add[4] = {0.f, 0.f, 0.f, 0.f};
+        if (res) get4<VEC>(res + row * cols, c, cols, add);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) o[j] = r * (gv[i][j] * wv[i][j]) - xv[i][j] * k + add[j];
+        put4<VEC>(dx + row * cols, c, cols, o);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] += gv[i][j] * xv[i][j] * r;
+    }
+  }
+  if (!part) return;
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) {
+    __syncthreads();
+    if (wave > 0)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) red[wave - 1][lane * 4 + j] = acc[i][j];
+    __syncthreads();
+    if (wave == 0)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = (i * 64 + lane) * 4 + j;
+        const float s = (acc[i][j] + red[0][lane * 4 + j]) + (red[1][lane * 4 + j] + red[2][lane * 4 + j]);
+        if (c < cols) part[(int64_t)blockIdx.x * cols + c] = s;
+      }
+  }
+}
+
+// column sums of part [n][cols]: 64 columns per workgroup, 16 of its waves each every 16th row
+template <typename TW>
+__global__ __launch_bounds__(1024) void column_sum_kernel(const float* __restrict__ part, TW* __restrict__ out, int n, int cols) {
+  __shared__ float red[16][64];
+  const int lane = threadIdx.x & 63, sub = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (c < cols) {
+#pragma unroll 8
+    for (int i = sub; i < n; i += 16) s += part[(int64_t)i * cols + c];
+  }
+  red[sub][lane] = s;
+  __syncthreads();
+  if (sub == 0 && c < cols) {
+#pragma unroll
+    for (int i = 1; i < 16; ++i) s += red[i][lane];
+    io<TW>::store(out + c, s);
+  }
+}
+
+__device__ inline void load8(const bf16_t* p, float (&v)[8]) {
+  const u32x4 x = *(const u32x4*)p;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    v[2 * i] = __uint_as_float(x[i] << 16);
+    v[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
+  }
+}
+__device__ inline void store8(bf16_t* p, const float (&v)[8]) {
+  *(u32x4*)p = u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
+}
+
+constexpr int GATE_ROWS = 4;         // rows per thread: their loads go out together
+
+// out = silu(gate) up for rows [gate | up] of 2 n columns; a thread takes 8 columns of GATE_ROWS rows
+__global__ __launch_bounds__(256) void silu_gate_kernel(const bf16_t* __restrict__ gu, bf16_t* __restrict__ out, int64_t rows, int n) {
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (c >= n) return;
+#pragma unroll
+  for (int i = 0; i < GATE_ROWS; ++i) {
+    const int64_t row = (int64_t)blockIdx.x * GATE_ROWS + i;
+    if (row >= rows) break;
+    float g[8], u[8];
+    load8(gu + row * 2 * n + c, g);
+    load8(gu + row * 2 * n + n + c, u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) g[j] = g[j] / (1.f + expf(-g[j])) * u[j];
+    store8(out + row * n + c, g);
+  }
+}
+
+// dgate = d up s (1 + gate (1 - s)), dup = d gate s, s the sigmoid of gate
+__global__ __launch_bounds__(256) void silu_gate_backward_kernel(const bf16_t* __restrict__ gu, const bf16_t* __restrict__ d,
+                                                                 bf16_t* __restrict__ dgu, int64_t rows, int n) {
+  const int c = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (c >= n) return;
+#pragma unroll
+  for (int i = 0; i < GATE_ROWS; ++i) {
+    const int64_t row = (int64_t)blockIdx.x * GATE_ROWS + i;
+    if (row >= rows) break;
+    float g[8], u[8], dv[8];
+    load8(gu + row * 2 * n + c, g);
+    load8(gu + row * 2 * n + n + c, u);
+    load8(d + row * n + c, dv);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float s = 1.f / (1.f + expf(-g[j]));
+      const float du = dv[j] * g[j] * s;
+      g[j] = dv[j] * u[j] * (s * (1.f + g[j] * (1.f - s)));
+      u[j] = du;
+    }
+    store8(dgu + row * 2 * n + c, g);
+    store8(dgu + row * 2 * n + n + c, u);
+  }
+}
+
+static int row_groups(int64_t rows) { return (int)(rows >= 4 * MAX_GROUPS ? MAX_GROUPS : (rows + 3) / 4); }
+
+template <typename TX, typename TW>
+static void launch_norm(const void* x, const void* w, const void* dy, const void* res, void* dx, float* part, int64_t rows,
+                        int cols, float eps, bool vec, hipStream_t s) {
+  auto go = [&](auto kern) {
+    MVPA_LAUNCH(kern, dim3((unsigned)row_groups(rows)), dim3(256), 0, s, (const TX*)x, (const TW*)w, (const bf16_t*)dy,
+                (const TX*)res, (TX*)dx, part, rows, cols, eps);
+  };
+  if (!vec) {
+    if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, false>);
+    else go(rmsnorm_backward_kernel<TX, TW, 16, false>);
+  } else if (cols <= 768) go(rmsnorm_backward_kernel<TX, TW, 3, true>);
+  else if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, true>);
+  else if (cols <= 2048) go(rmsnorm_backward_kernel<TX, TW, 8, true>);
+  else go(rmsnorm_backward_kernel<TX, TW, 16, true>);
+}
+
+}  // namespace train
+}  // namespace mvpa
+
+using namespace mvpa;
+
+extern "C" size_t mvpa_rmsnorm_backward_ws_bytes(int64_t rows, int32_t cols) {
+  return rows > 0 && cols > 0 ? (size_t)train::row_groups(rows) * cols * sizeof(float) : 0;
+}
+
+extern "C" int mvpa_rmsnorm_backward(const void* x, const void* weight, const void* dy, const void* res, void* dx, void* dw,
+                                     void* ws, int64_t rows, int32_t cols, float eps, int32_t x_f32, int32_t w_f32,
+                                     void* stream) {
+  if (!x || !weight || !dy || (!dx && !dw) || (dw && !ws)) return MVPA_ERR_NULL;
+  if (rows <= 0 || cols <= 0) return MVPA_ERR_SHAPE;
+  if (cols > train::MAX_COLS) return MVPA_ERR_UNSUPPORTED;
+  const uintptr_t low = (uintptr_t)x | (uintptr_t)weight | (uintptr_t)dy | (uintptr_t)res | (uintptr_t)dx;
+  const bool vec = cols % 4 == 0 && (low & 15) == 0;
+  float* part = dw ? (float*)ws : nullptr;
+  hipStream_t s = (hipStream_t)stream;
+  if (x_f32 && w_f32) train::launch_norm<float, float>(x, weight, dy, res, dx, part, rows, cols, eps, vec, s);
+  else if (x_f32) train::launch_norm<float, bf16_t>(x, weight, dy, res, dx, part, rows, cols, eps, vec, s);
+  else if (w_f32) train::launch_norm<bf16_t, float>(x, weight, dy, res, dx, part, rows, cols, eps, vec, s);
+  else train::launch_norm<bf16_t, bf16_t>(x, weight, dy, res, dx, part, rows, cols, eps, vec, s);
+  if (dw) {
+    const dim3 grid((unsigned)((cols + 63) / 64));
+    const int n = train::row_groups(rows);
+    if (w_f32) MVPA_LAUNCH(train::column_sum_kernel<float>, grid, dim3(1024), 0, s, part, (float*)dw, n, cols);
+    else MVPA_LAUNCH(train::column_sum_kernel<bf16_t>, grid, dim3(1024), 0, s, part, (bf16_t*)dw, n, cols);
+  }
+  return take_launch_status();
+}
+
+static int gate_check(const void* a, const void* b, const void* c, int64_t rows, int32_t n) {
+  if (!a || !b || !c) return MVPA_ERR_NULL;
+  if (rows <= 0 || n <= 0 || n > (1 << 24) || rows > ((int64_t)1 << 31)) return MVPA_ERR_SHAPE;
+  if (n % 8 != 0 || (((uintptr_t)a | (uintptr_t)b | (uintptr_t)c) & 15)) return MVPA_ERR_ALIGN;
+  return MVPA_OK;
+}
+
+static dim3 gate_grid(int64_t rows, int32_t n) {
+  return dim3((unsigned)((rows + train::GATE_ROWS - 1) / train::GATE_ROWS), (unsigned)((n + 2047) / 2048));
+}
+
+extern "C" int mvpa_silu_gate_bf16(const void* gu, void* out, int64_t rows, int32_t n, void* stream) {
+  const int st = gate_check(gu, out, out, rows, n);
+  if (st != MVPA_OK) return st;
+  MVPA_LAUNCH(train::silu_gate_kernel, gate_grid(rows, n), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gu, (bf16_t*)out, rows, n);
+  return take_launch_status();
+}
+
+extern "C" int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void* dgu, int64_t rows, int32_t n, void* stream) {
+  const int st = gate_check(gu, d, dgu, rows, n);
+  if (st != MVPA_OK) return st;
+  MVPA_LAUNCH(train::silu_gate_backward_kernel, gate_grid(rows, n), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gu,
+              (const bf16_t*)d, (bf16_t*)dgu, rows, n);
+  return take_launch_status();
+}

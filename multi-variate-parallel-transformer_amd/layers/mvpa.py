@@ -419,7 +419,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
         projections and c_proj through the library's GEMM (backward: two more GEMMs each), the
         attention through FlashMVPA (backward: mvpa_backward).  Same kernels as the inference path,
         launched one by one instead of fused."""
-        from attentions.attn import FlashMVPA
+        from attentions.attn import FlashMVPA, FlashMVPAPacked
         from mvpa_hip import autograd as AG
         bsz, t_len, c_len, e = hidden_states.shape
         h, hkv, dh, kv = self.num_heads, self.num_kv_heads, self.head_dim, self.embed_kv_dim
@@ -439,9 +439,14 @@ class MVPFormerGQAAttention(torch.nn.Module):
             # soft-max sum ignores the masks, so the values carry them (attentions.attn)
             from attentions.attn import dropout_key_scale
             v = v * dropout_key_scale(self.attn_dropout.p, t_len, c_len, v.device).to(dt)[None, None, :, None]
-        out = FlashMVPA.apply(q, u, vb, z, k, k_time.contiguous(), k_chan.contiguous(), v, True,
-                              self._scale(), window, True, True, chan_valid, self._content(), key_bias)
-        merged = out.permute(0, 2, 1, 3)                                      # [B,N,H,Dh]
+        k_time, k_chan = k_time.contiguous(), k_chan.contiguous()
+        if v is v_plain and key_bias is None and FlashMVPAPacked.supported(qkv, dh, c_len):
+            merged = FlashMVPAPacked.apply(qkv, u, vb, z, k_time, k_chan, h, self._scale(), window, chan_valid,
+                                           self._content())
+        else:
+            out = FlashMVPA.apply(q, u, vb, z, k, k_time, k_chan, v, True,
+                                  self._scale(), window, True, True, chan_valid, self._content(), key_bias)
+            merged = out.permute(0, 2, 1, 3)                                  # [B,N,H,Dh]
         if head_mask is not None:                                            # layers/mvpa.py:274-275
             if head_mask.numel() != h:
                 raise NotImplementedError("head_mask must hold one factor per head")

@@ -80,6 +80,12 @@ class MVPFormerConfig:
         return cls(**doc["model"]["init_args"]["gpt_config"]["init_args"])
 
 
+def _unhooked(norm: nn.Module) -> bool:
+    """A plain RMSNorm whose call nobody watches or replaces: its weight may be used without calling it."""
+    return (type(norm) is RMSNorm and "forward" not in norm.__dict__
+            and not (norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks))
+
+
 class GatedMLP(nn.Module):
     """down(silu(gate(x)) * up(x)), bias-free: the MLP the reference takes from the Llama family
     (models/mvpformer.py:114).  gate and up run as ONE GEMM with the SiLU-multiply fused."""
@@ -103,6 +109,11 @@ class GatedMLP(nn.Module):
 
     def forward(self, x):
         if torch.is_grad_enabled() and (x.requires_grad or self.training):
+            wg, wu = self.gate_proj.weight, self.up_proj.weight
+            if x.is_cuda and x.dtype == torch.bfloat16 and wg.shape == wu.shape and wg.shape[0] % 8 == 0 and x.numel():
+                # frozen weights keep their stacked copy, others are stacked inside the graph
+                w = torch.cat([wg, wu], 0) if wg.requires_grad or wu.requires_grad else self._gate_up()
+                return AG.linear(AG.gated_mid(x, w), self.down_proj.weight)
             mid = torch.nn.functional.silu(AG.linear(x, self.gate_proj.weight)) * AG.linear(x, self.up_proj.weight)
             return AG.linear(mid, self.down_proj.weight)
         with torch.no_grad():
@@ -214,9 +225,15 @@ class MVPFormerBlock(nn.Module):
             attn_outputs = self.attn(normed, positional_embedding, channel_embedding,
                                      attention_mask=attention_mask, head_mask=head_mask,
                                      use_cache=use_cache, output_attentions=output_attentions)
-            hidden_states = hidden_states + self.mlp(normed) + attn_outputs[0]
-            outputs = (hidden_states,) + (attn_outputs[1:] if use_cache else attn_outputs[2:])
-            return outputs, (next_norm(hidden_states) if next_norm is not None else None)
+            mlp_output = self.mlp(normed)
+            both = None
+            if next_norm is not None and _unhooked(next_norm):
+                both = AG.add3_rmsnorm(hidden_states, mlp_output, attn_outputs[0], next_norm.weight, next_norm.eps)
+            if both is None:
+                hidden_states = hidden_states + mlp_output + attn_outputs[0]
+                both = hidden_states, (next_norm(hidden_states) if next_norm is not None else None)
+            outputs = (both[0],) + (attn_outputs[1:] if use_cache else attn_outputs[2:])
+            return outputs, both[1]
         residual = hidden_states
         if normed is None:
             normed = self.ln_1(hidden_states)

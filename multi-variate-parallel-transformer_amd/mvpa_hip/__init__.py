@@ -444,14 +444,14 @@ def mvpa_backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, *,
 
 def mvpa_backward_full(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, *, sm_scale: float, window: int = 10,
                        content: bool = True, time_bias: bool = True, chan_bias: bool = True,
-                       chan_valid: Optional[torch.Tensor] = None):
+                       chan_valid: Optional[torch.Tensor] = None, out=()):
     """Gradients of mvpa_forward's inputs in bf16, (dq, du, dvb, dz, dk, dk_time, dk_chan, dv): mvpa_backward
-    and the products that finish its table gradients, all in the library.  None for shapes or layouts that
-    the matrix-core backward does not take."""
+    and the products that finish its table gradients, all in the library.  out: three views that receive dq,
+    dk, dv.  None for shapes or layouts that the matrix-core backward does not take."""
     flags = (FLAG_CAUSAL | (FLAG_CONTENT if content else 0) | (FLAG_TIME_BIAS if time_bias else 0) |
              (FLAG_CHAN_BIAS if chan_bias else 0))
     r = (_ext or load_ext()).backward(q, k, v, o, d_o, lse, u, vb, z, k_time, k_chan, chan_valid, float(sm_scale),
-                                      window, flags)
+                                      window, flags, *out)
     if type(r) is int and r == ERR_UNSUPPORTED:
         return None
     return _taken(r)
@@ -533,6 +533,20 @@ def row_sumsq(x: torch.Tensor) -> torch.Tensor:
     out = torch.empty((x.shape[0], 1), dtype=torch.float32, device=x.device)
     _check(lib.mvpa_row_sumsq_bf16(x.data_ptr(), out.data_ptr(), x.shape[0], x.shape[1], x.stride(0), _stream()))
     return out
+
+
+def norm_backward(x, weight, dy, res, eps: float, need_x: bool = True, need_w: bool = True):
+    """(dx, dw) of y = RMSNorm(x) * weight for dy in bf16; dx with `res`, the gradient that reaches the rows
+    past the norm, added (None: nothing to add).  What is not needed comes back as None."""
+    if not (need_x or need_w):
+        return None, None
+    return _taken((_ext or load_ext()).norm_backward(x, weight, dy, res, float(eps), bool(need_x), bool(need_w)))
+
+
+def silu_gate(gu: torch.Tensor, d: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """silu(gate) * up of bf16 rows [gate | up]; with d, the gradient of gu for the gradient d of that."""
+    ext = _ext or load_ext()
+    return _taken(ext.silu_gate(gu) if d is None else ext.silu_gate(gu, d))
 
 
 def mean_rows(x: torch.Tensor) -> torch.Tensor:

@@ -4,8 +4,8 @@ modules (the reference trains through layers/mvpa.py:280-337 and models/mvpforme
 Forward passes are the library's kernels.  The backward passes of the bf16 products are the two
 plain products dX = dY W and dW = dY^T X on the vendor library through torch.matmul: it reads
 the transposed operand in place and splits the long contraction of a weight gradient (a small
-[N,K] output over all rows), which this library's GEMM would run on a few dozen tiles.  The
-norm's backward is a few fp32 tensor ops.  The attention operator itself is
+[N,K] output over all rows), which this library's GEMM would run on a few dozen tiles.  Norm,
+gated activation and residual sums run on kernels of the library both ways (csrc/mvpa_train.hip).  The attention operator itself is
 `attentions.attn.FlashMVPA` (mvpa_backward kernels).
 """
 from __future__ import annotations
@@ -76,8 +76,30 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return torch.nn.functional.linear(x, w.to(x.dtype))
 
 
+MAX_NORM_COLS = 4096          # the longest row of the library's RMSNorm backward
+
+
+def _norm_backward(ctx, x, w, dy, res, need_x, need_w):
+    """(dx, dw) of y = RMSNorm(x) w, dx with the gradient `res` of the rows themselves added where given."""
+    if (x.is_cuda and dy.dtype == torch.bfloat16 and x.dtype in (torch.bfloat16, torch.float32) and x.numel()
+            and w.dtype in (torch.bfloat16, torch.float32) and x.shape[-1] <= MAX_NORM_COLS
+            and not torch.is_grad_enabled()):
+        return mvpa_hip.norm_backward(x, w, dy, res, ctx.eps, need_x, need_w)
+    # other types, and a backward that is differentiated itself (create_graph)
+    xf, wf, g = x.float(), w.float(), dy.float()
+    r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)
+    gw = g * wf
+    dx = dw = None
+    if need_x:
+        dx = r * gw - xf * r.pow(3) * (xf * gw).mean(-1, keepdim=True)
+        dx = (dx if res is None else dx + res.float()).to(x.dtype)
+    if need_w:
+        dw = (g * xf * r).reshape(-1, x.shape[-1]).sum(0).to(w.dtype)
+    return dx, dw
+
+
 class _RMSNormFn(torch.autograd.Function):
-    """y = x * rsqrt(mean(x^2) + eps) * w; forward on the library's kernel, backward in fp32."""
+    """y = x * rsqrt(mean(x^2) + eps) * w, forward and backward on the library's kernels."""
 
     @staticmethod
     def forward(ctx, x, w, eps, out_dtype):
@@ -88,18 +110,64 @@ class _RMSNormFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         x, w = ctx.saved_tensors
-        xf, wf, g = x.float(), w.float(), dy.float()
-        r = torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + ctx.eps)
-        gw = g * wf
-        dx = dw = None
-        if ctx.needs_input_grad[0]:
-            dx = (r * gw - xf * r.pow(3) * (xf * gw).mean(-1, keepdim=True)).to(x.dtype)
-        if ctx.needs_input_grad[1]:
-            dw = (g * xf * r).reshape(-1, x.shape[-1]).sum(0).to(w.dtype)
-        return dx, dw, None, None
+        return (*_norm_backward(ctx, x, w, dy, None, *ctx.needs_input_grad[:2]), None, None)
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype=None) -> torch.Tensor:
     if wants_grad(x, w):
         return _RMSNormFn.apply(x, w, eps, out_dtype)
     return mvpa_hip.rmsnorm(x, w, eps, out_dtype=out_dtype)
+
+
+class _Add3RMSNormFn(torch.autograd.Function):
+    """(s, RMSNorm(s) w) with s = a + b + c: the residual update of a block and the norm behind it."""
+
+    @staticmethod
+    def forward(ctx, a, b, c, w, eps):
+        ctx.set_materialize_grads(False)
+        total, normed = mvpa_hip.add3_rmsnorm(a, b, c, w, eps)
+        ctx.save_for_backward(total, w)
+        ctx.eps = eps
+        return total, normed
+
+    @staticmethod
+    def backward(ctx, d_total, d_normed):
+        total, w = ctx.saved_tensors
+        d, dw = d_total, None
+        if d_normed is not None:
+            d, dw = _norm_backward(ctx, total, w, d_normed, d_total, any(ctx.needs_input_grad[:3]),
+                                   ctx.needs_input_grad[3])
+        return d, d, d, dw, None
+
+
+def add3_rmsnorm(a, b, c, w, eps):
+    """(a + b + c, RMSNorm(a + b + c) * w) in one pass each way, or None where the operands are not bf16
+    rows of whole 16-byte chunks on the GPU."""
+    if (not a.is_cuda or not a.dtype == b.dtype == c.dtype == torch.bfloat16 or not a.shape == b.shape == c.shape
+            or a.shape[-1] % 8 or a.shape[-1] > MAX_NORM_COLS or not a.numel()
+            or w.dtype not in (torch.bfloat16, torch.float32)):
+        return None
+    return _Add3RMSNormFn.apply(a, b, c, w, eps)
+
+
+class _SiluGateFn(torch.autograd.Function):
+    """silu(gate) * up of rows [gate | up], one pass each way."""
+
+    @staticmethod
+    def forward(ctx, gu):
+        ctx.save_for_backward(gu)
+        return mvpa_hip.silu_gate(gu)
+
+    @staticmethod
+    def backward(ctx, d):
+        gu, = ctx.saved_tensors
+        if not torch.is_grad_enabled():
+            return mvpa_hip.silu_gate(gu, d)
+        gate, up = gu.float().chunk(2, -1)                   # a backward that is differentiated itself
+        s, df = torch.sigmoid(gate), d.float()
+        return torch.cat([df * up * s * (1 + gate * (1 - s)), df * gate * s], -1).to(gu.dtype)
+
+
+def gated_mid(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
+    """silu(x @ gate^T) * (x @ up^T) for w_gate_up = [gate; up]: one product, one pass over its result."""
+    return _SiluGateFn.apply(linear(x, w_gate_up))

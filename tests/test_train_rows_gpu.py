@@ -1,0 +1,112 @@
+"""Row operations of the training path (csrc/mvpa_train.hip) against the same formulas in 64 bits, and the
+attention on packed projection rows against the operator on separate tensors."""
+import pytest
+import torch
+
+import mvpa_hip
+from attentions.attn import FlashMVPA, FlashMVPAPacked
+from mvpa_hip import autograd as AG
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, ref, terms=1):
+    """One rounding to the type of the result (half an ulp: 2^-8 of bf16 with its 8 significant bits, 2^-24 of fp32)
+    terms whose roundings add up to at most 2^-24 sqrt(terms) of the result's scale, 8 sigma."""
+    half = 2.0 ** -8 if got.dtype == torch.bfloat16 else 2.0 ** -24
+    ref = ref.double()
+    scale = ref.pow(2).mean().sqrt()
+    bound = half * 1.01 * ref.abs() + 8 * 2.0 ** -24 * (max(terms, 16) ** 0.5) * (ref.abs() + scale)
+    assert ((got.double() - ref).abs() <= bound).all()
+
+
+# columns: one chunk, rows that are no whole chunks, the edges of each build; rows: one, fewer than a
+# workgroup's, a second round of rows for some workgroups only
+@pytest.mark.parametrize("cols", [4, 7, 768, 772, 1024, 1030, 2048, 4092, 4096])
+@pytest.mark.parametrize("rows,xt,wt,res", [(1, torch.bfloat16, torch.bfloat16, True), (5, torch.float32, torch.float32, False),
+                                            (2051, torch.bfloat16, torch.float32, True),
+                                            (2050, torch.float32, torch.bfloat16, True)])
+def test_norm_backward(cols, rows, xt, wt, res):
+    g = torch.Generator(device="cuda").manual_seed(cols * 31 + rows)
+
+    def rn(*s):
+        return torch.randn(s, generator=g, device="cuda")
+    x, w, dy = rn(rows, cols).to(xt), (1 + 0.1 * rn(cols)).to(wt), rn(rows, cols).bfloat16()
+    r = rn(rows, cols).to(xt) if res else None
+    dx, dw = mvpa_hip.norm_backward(x, w, dy, r, 1e-5)
+    xd, wd, gd = x.double(), w.double(), dy.double()
+    inv = (xd.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+    parts = inv * gd * wd, xd * inv ** 3 * (xd * gd * wd).mean(-1, keepdim=True)
+    ref = parts[0] - parts[1] + (r.double() if res else 0)
+    half = 2.0 ** -8 if xt == torch.bfloat16 else 2.0 ** -24
+    bound = half * 1.01 * ref.abs() + 2.0 ** -18 * (parts[0].abs() + parts[1].abs() + inv * wd.abs() + 1)
+    assert ((dx.double() - ref).abs() <= bound).all()
+    _close(dw, (gd * xd * inv).sum(0), rows * 4)
+    only_x, none = mvpa_hip.norm_backward(x, w, dy, r, 1e-5, True, False)
+    assert none is None and torch.equal(only_x, dx)
+    none, only_w = mvpa_hip.norm_backward(x, w, dy, r, 1e-5, False, True)
+    assert none is None and torch.equal(only_w, dw)
+
+
+@pytest.mark.parametrize("rows,n", [(1, 8), (3, 2040), (4, 2048), (5, 2056), (33, 344), (130, 5632)])
+def test_silu_gate(rows, n):
+    g = torch.Generator(device="cuda").manual_seed(rows * n)
+    gu = (torch.randn((rows, 2 * n), generator=g, device="cuda") * 4).bfloat16()
+    gu[0, 0], gu[-1, n - 1] = -200.0, 200.0            # exp(-gate) overflows, underflows
+    d = torch.randn((rows, n), generator=g, device="cuda").bfloat16()
+    gate, up = gu.double().chunk(2, -1)
+    s = torch.sigmoid(gate)
+    _close(mvpa_hip.silu_gate(gu), gate * s * up)
+    dgate, dup = mvpa_hip.silu_gate(gu, d).chunk(2, -1)
+    _close(dgate, d.double() * up * s * (1 + gate * (1 - s)))
+    _close(dup, d.double() * gate * s)
+
+
+@pytest.mark.parametrize("cols", [8, 768])
+def test_add3_norm_gradients(cols):
+    """Gradients through both results, through one of them, and of a gradient (the tensor expressions)."""
+    def leaf(*s):
+        return torch.randn(s, device="cuda").bfloat16().requires_grad_(True)
+    torch.manual_seed(cols)
+    a, b, c, w = leaf(70, cols), leaf(70, cols), leaf(70, cols), leaf(cols)
+    ds, dn = torch.randn(70, cols, device="cuda").bfloat16(), torch.randn(70, cols, device="cuda").bfloat16()
+    total, normed = AG.add3_rmsnorm(a, b, c, w, 1e-5)
+    t64, w64 = total.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
+    n64 = t64 * (t64.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt() * w64
+    for outs, grads, ref_outs in (((total, normed), (ds, dn), (t64 + 0, n64)), ((normed,), (dn,), (n64,))):
+        got = torch.autograd.grad(outs, (a, b, c, w), grads, retain_graph=True)
+        ref = torch.autograd.grad(ref_outs, (t64, w64), [g.double() for g in grads], retain_graph=True)
+        assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+        for x, y in ((got[0], ref[0]), (got[3], ref[1])):
+            assert (x.double() - y).norm() <= 2.0 ** -8 * y.norm()
+    first, = torch.autograd.grad(normed, (a,), dn, create_graph=True)
+    second, = torch.autograd.grad(first.float().pow(2).sum(), (w,))
+    assert torch.isfinite(second).all() and second.abs().sum() > 0
+
+
+@pytest.mark.parametrize("B,C,T,H,Hkv,Dh,masked", [(1, 1, 1, 2, 1, 64, False), (2, 5, 13, 4, 2, 64, True),
+                                                   (1, 33, 14, 6, 2, 64, False), (1, 70, 12, 2, 2, 128, True)])
+def test_packed_attention(B, C, T, H, Hkv, Dh, masked):
+    """Rows of one projection against separate tensors: the same kernels on other strides."""
+    g = torch.Generator(device="cuda").manual_seed(C * T)
+
+    def rn(*s, std=1.0):
+        return (torch.randn(s, generator=g, device="cuda") * std).bfloat16().requires_grad_(True)
+    N, row = T * C, (H + 2 * Hkv) * Dh
+    qkv, tabs = rn(B, N, row), [rn(Hkv, Dh, std=0.1) for _ in range(3)] + [rn(Hkv, T, Dh, std=0.1), rn(Hkv, C, Dh, std=0.1)]
+    valid = None
+    if masked:
+        valid = torch.ones(B, C, dtype=torch.bool, device="cuda")
+        valid[:, C // 2] = False
+    d = torch.randn((B, N, H, Dh), generator=g, device="cuda").bfloat16()
+    scale = Dh ** -0.5
+    out = FlashMVPAPacked.apply(qkv, *tabs, H, scale, 10, valid, True)
+    got = torch.autograd.grad(out, [qkv, *tabs], d)
+    q, k, v = FlashMVPAPacked._heads(qkv, H, Hkv, Dh)
+    ref_out = FlashMVPA.apply(q, *tabs[:3], k, tabs[3], tabs[4], v, True, scale, 10, True, True, valid)
+    ref = torch.autograd.grad(ref_out, [qkv, *tabs], d.transpose(1, 2))
+    # bf16 rounding of the probabilities and of the result where the two take kernels of another split
+    assert (out.transpose(1, 2).double() - ref_out.double()).norm() <= 2.0 ** -7 * ref_out.double().norm()
+    for x, y in zip(got, ref):
+        assert x.shape == y.shape
+        assert (x.double() - y.double()).norm() <= 2.0 ** -6 * y.double().norm() + 1e-6
