@@ -12,7 +12,7 @@
 //     dq^T += K^T dS^T                     (inside the window)
 //     dbias_time[q, tk] = sum_ck dS,       dbias_chan[q, |cq-ck|] += dS.
 // Outputs are those of mvpa_backward (include/mvpa_hip.h): the content share of dq and the two
-// bias-table gradients.  For the key pass the workspace receives, in base-2 score units, delta,
+// bias-table gradients.  For the key pass the workspace receives, in base-2 score units, -delta,
 // the channel-table rows, (time bias - L) laid out [b,h,tq,tk,cq] and (q+u) * scale in bf16.
 // K and V tiles come through a ring of LDS stages filled by direct-to-LDS loads two key steps
 // ahead, K in two copies (row fragments for K Q^T, transposed fragments for K^T dS^T); far key
@@ -126,6 +126,7 @@ template <int DH, int NCT>
 __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
   constexpr int NW = QUERY_WAVES<DH, NCT>;
+  constexpr bool SOLO = NW == 4;                  // one wave per SIMD
   constexpr int CP = NCT * 32, TQW = NW / NCT, TILE = CP * ROWB;
   static_assert(64 * 32 <= WAVE_SCRATCH && 32 * (CP + 1) <= WAVE_SCRATCH, "channel tables overlay the slabs");
   constexpr int STAGES = QSTAGES<DH, NCT>, STAGE_BYTES = 3 * TILE;   // stage: V | K | K (transposing)
@@ -346,7 +347,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
             *(float4*)(wc + ci) = make_float4(Ec[t][a4 * 4], Ec[t][a4 * 4 + 1], Ec[t][a4 * 4 + 2], Ec[t][a4 * 4 + 3]);
         }
     }
-    if (qok && hh == 0) a.ws_delta[row] = delta;
+    if (qok && hh == 0) a.ws_delta[row] = -delta;
   }
 
   f32x16 dq[MT], dSc[NCT];
@@ -405,7 +406,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
 #pragma unroll 8
     for (int it = 0; it < 16; ++it) {
       const int q = 2 * it + hh;
-      const float g = Gtb[ln * GP + q];
+      const float g = Gtb[ln * GP + q] * a.sm_scale;
       if (q < nq_live && ln < nj) {
         float* dst = a.dbias_time + (wrow0 + q) * T_ + j0 + ln;
         // launches of one stream: the key parts add up.  An atomic add without a return value,
@@ -469,8 +470,9 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
 
   // A far key step (content term dropped): P^T = Ec et with et = exp2(time bias - L + mc) one
   // scalar per query, so with dP^T = V dO^T
-  //     dbias_time[q, tk]  = scale et (sum_keys Ec dP - delta sumEc)
-  //     dbias_chan share   = Ec (sum_tk scale et dP - delta sum_tk scale et)   (formed after the loop)
+  //     dbias_time[q, tk]  = et (sum_keys Ec dP - delta sumEc)
+  //     dbias_chan share   = Ec (sum_tk et dP - delta sum_tk et)   (formed after the loop)
+  // (all of them, like dS below, times the score scale where they are written)
   // costs two FMAs per element and no exponential per element.
   // The loop is software-pipelined: the products of step tk are issued to the matrix cores, and
   // the vector work on the products of step tk-1 runs meanwhile.
@@ -478,7 +480,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   // reduces the products of far step tkp (none if tkp < 0)
   auto far_reduce = [&](const f32x16 (&dP)[NCT], int tkp) {
     if (tkp < 0) return;
-    const float et = __builtin_amdgcn_exp2f(Stb[(tkp & 31) * 32 + ln] - lse + mc) * a.sm_scale;
+    const float et = __builtin_amdgcn_exp2f(Stb[(tkp & 31) * 32 + ln] - lse + mc);
     float dot[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < NCT; ++t)
@@ -527,19 +529,40 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
     float gt = 0.f;
 #pragma unroll
     for (int t = 0; t < NCT; ++t) {               // one key-channel tile at a time: fewer live tiles
-      f32x16 S = Bc[t], dP;
+      // A wave that has its SIMD to itself sends out every LDS read of a phase before the first product or
+      // exponential of it: read where they are used, each pair of fragments waits out the LDS latency (last time
+      // step of 512: 512 such steps, the longest chain of the launch; 4.92 -> 4.64 ms at B1 H16 C64 of 128 Dh128).
+      // Two waves cover each other's waits, and 256 registers do not hold the fragments (78 spilled, 0.90 -> 1.23 ms).
+      const unsigned char *Kt = Krow + t * 32 * ROWB, *Vt = Vrow + t * 32 * ROWB;
+      bf16x8 kf[KS], vf[KS], kt[2][MT];
+      if constexpr (SOLO) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) dP[i] = 0.f;
+        for (int ks = 0; ks < KS; ++ks) {
+          kf[ks] = *(const bf16x8*)(Kt + r_lane[ks]);
+          vf[ks] = *(const bf16x8*)(Vt + r_lane[ks]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      f32x16 S = Bc[t], dP;
+      // dP - delta: the subtraction is the product's C operand (16 registers more)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dP[i] = SOLO ? -delta : 0.f;
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        const int off = r_lane[ks] + t * 32 * ROWB;
-        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Krow + off), Qu[ks], S, 0, 0, 0);
-        dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Vrow + off), dOf[ks], dP, 0, 0, 0);
+        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(SOLO ? kf[ks] : *(const bf16x8*)(Kt + r_lane[ks]), Qu[ks], S, 0, 0, 0);
+        dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(SOLO ? vf[ks] : *(const bf16x8*)(Vt + r_lane[ks]), dOf[ks], dP, 0, 0, 0);
+      }
+      if constexpr (SOLO) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) kt[s][mt] = tr_frag(Ktr, t, s, mt);
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float p = __builtin_amdgcn_exp2f(S[i] + off2);        // masked keys: exp2(-inf) = 0
-        const float ds = p * (dP[i] - delta) * a.sm_scale;
+        const float ds = p * (SOLO ? dP[i] : dP[i] - delta);
         S[i] = ds;
         dSc[t][i] += ds;
         gt += ds;
@@ -549,7 +572,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
         const bf16x8 dsf = pack8(S, 8 * s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          dq[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Ktr, t, s, mt), dsf, dq[mt], 0, 0, 0);
+          dq[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(SOLO ? kt[s][mt] : tr_frag(Ktr, t, s, mt), dsf, dq[mt], 0, 0, 0);
       }
     }
     gt = xhalf_sum(gt);
@@ -610,7 +633,8 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
       for (int a4 = 0; a4 < 4; ++a4)
       {
         float4* dst = (float4*)(dqo + mt * 32 + a4 * 8 + hh * 4);
-        float4 val = make_float4(dq[mt][a4 * 4], dq[mt][a4 * 4 + 1], dq[mt][a4 * 4 + 2], dq[mt][a4 * 4 + 3]);
+        float4 val = make_float4(dq[mt][a4 * 4] * a.sm_scale, dq[mt][a4 * 4 + 1] * a.sm_scale,
+                                 dq[mt][a4 * 4 + 2] * a.sm_scale, dq[mt][a4 * 4 + 3] * a.sm_scale);
         if (accum) {
           const float4 old = *dst;
           val = make_float4(val.x + old.x, val.y + old.y, val.z + old.z, val.w + old.w);
@@ -627,7 +651,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
 #pragma unroll
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) scr[ln * PC + t * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i];
+    for (int i = 0; i < 16; ++i) scr[ln * PC + t * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i] * a.sm_scale;
   wave_sync_lds();
   for (int c0 = 0; c0 < C_; c0 += 64) {
     const int col = c0 + lane;
@@ -954,28 +978,37 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
     const float* De = (const float*)(base + OFF_SC) + KT * 64;
 #pragma unroll
     for (int qt = 0; qt < NCT; ++qt) {
-      f32x16 S, dP, dS;
-#pragma unroll
-      for (int i = 0; i < 16; ++i) { S[i] = 0.f; dP[i] = 0.f; }
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        const int off = r_lane[ks] + qt * 32 * ROWB;
-        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Qrow + off), Kf[ks], S, 0, 0, 0);
-        dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Drow + off), Vf[ks], dP, 0, 0, 0);
-      }
+      // the exponent and -delta are the products' C operands; dk takes its factor 1 / log2(e) where it is written
+      f32x16 S, dP;
 #pragma unroll
       for (int a4 = 0; a4 < 4; ++a4) {
         const int rb = qt * 32 + a4 * 8 + hh * 4;
         const float4 tl = *(const float4*)(TL + rb);
         const float4 de = *(const float4*)(De + rb);
-        const float tls[4] = {tl.x, tl.y, tl.z, tl.w}, des[4] = {de.x, de.y, de.z, de.w};
+        S[a4 * 4] = tl.x; S[a4 * 4 + 1] = tl.y; S[a4 * 4 + 2] = tl.z; S[a4 * 4 + 3] = tl.w;
+        dP[a4 * 4] = de.x; dP[a4 * 4 + 1] = de.y; dP[a4 * 4 + 2] = de.z; dP[a4 * 4 + 3] = de.w;
+      }
+      bf16x8 qf[KS], df[KS];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int i = a4 * 4 + j;
-          const float p = __builtin_amdgcn_exp2f(S[i] + tls[j]) * Ecs[(rb + j) * CP];
-          S[i] = p;
-          dS[i] = p * (dP[i] - des[j]) * (1.f / kLog2e);
-        }
+      for (int ks = 0; ks < KS; ++ks) {
+        qf[ks] = *(const bf16x8*)(Qrow + r_lane[ks] + qt * 32 * ROWB);
+        df[ks] = *(const bf16x8*)(Drow + r_lane[ks] + qt * 32 * ROWB);
+      }
+      __builtin_amdgcn_sched_barrier(0);          // every read out before the first product
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qf[ks], Kf[ks], S, 0, 0, 0);
+        dP = __builtin_amdgcn_mfma_f32_32x32x16_bf16(df[ks], Vf[ks], dP, 0, 0, 0);
+      }
+      float ec[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ec[i] = Ecs[(qt * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)) * CP];
+      __builtin_amdgcn_sched_barrier(0);
+      f32x16& dS = dP;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        S[i] = __builtin_amdgcn_exp2f(S[i]) * ec[i];
+        dS[i] = S[i] * dP[i];
       }
 #pragma unroll
       for (int s = 0; s < 2; ++s) {
@@ -1018,7 +1051,8 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
 #pragma unroll
       for (int a4 = 0; a4 < 4; ++a4) {
         const int d = mt * 32 + a4 * 8 + hh * 4;
-        float4 vk = make_float4(dK[mt][a4 * 4], dK[mt][a4 * 4 + 1], dK[mt][a4 * 4 + 2], dK[mt][a4 * 4 + 3]);
+        constexpr float f = 1.f / kLog2e;
+        float4 vk = make_float4(dK[mt][a4 * 4] * f, dK[mt][a4 * 4 + 1] * f, dK[mt][a4 * 4 + 2] * f, dK[mt][a4 * 4 + 3] * f);
         float4 vv = make_float4(dV[mt][a4 * 4], dV[mt][a4 * 4 + 1], dV[mt][a4 * 4 + 2], dV[mt][a4 * 4 + 3]);
         if (accum) {                              // launches of one stream: the query parts add up
           const float4 ok = *(const float4*)(a.dk + o + d), ov = *(const float4*)(a.dv + o + d);
