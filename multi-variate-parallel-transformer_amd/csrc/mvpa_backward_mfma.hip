@@ -737,7 +737,8 @@ namespace bwdq {
 // SIMD holds two waves
 template <int NCT> constexpr int KEY_WAVES = NCT == 2 ? 8 : 4;
 
-template <int DH, int NCT, bool MASKED>
+// NEAR: the far steps are left to mvpa_bwd_far_kernel, which has written dv before.
+template <int DH, int NCT, bool MASKED, bool NEAR>
 __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
   constexpr int NW = KEY_WAVES<NCT>;
@@ -902,8 +903,10 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
-  // steps: query heads of the group, and for each the query steps T-1 .. tk0
-  const int span = T_ - tk0, nsteps = grp * span;
+  // steps: query heads of the group, and for each the query steps T-1 .. tk0; NEAR: T-1, then top .. tk0,
+  // top the last step in the window of one of the waves
+  const int top = NEAR ? min(T_ - 2, tk0 + KT - 1 + W) : T_ - 2;
+  const int span = top < tk0 ? 1 : top - tk0 + 2, nsteps = grp * span;
   int ihq = 0, itq = T_ - 1;                      // the step the ring fetches next
   rebase(0);
   auto next_issue = [&]() {
@@ -916,6 +919,15 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
       p_ec -= d_ec;
       p_sc -= d_sc;
       p_de -= C_;
+      if (NEAR && itq == T_ - 2) {                // over the steps that are far for every wave
+        const int64_t n = T_ - 2 - top;
+        p_do -= n * d_do;
+        p_qu -= n * d_qu;
+        p_ec -= n * d_ec;
+        p_sc -= n * d_sc;
+        p_de -= n * C_;
+        itq = top;
+      }
     }
   };
 #pragma unroll
@@ -926,7 +938,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   // advances the ring by one step and returns the stage that holds its data
   auto ring_step = [&]() -> const unsigned char* {
     // the step has landed once only the loads of the one younger step are in flight
-    const int next_tq = ring_tq - 1 < tk0 ? T_ - 1 : ring_tq - 1;
+    const int next_tq = ring_tq - 1 < tk0 ? T_ - 1 : ring_tq == T_ - 1 ? top : ring_tq - 1;
     if (it + 1 >= nsteps) wait_vmcnt_imm<0>();
     else if (wg_near(next_tq)) wait_vmcnt_imm<LPS_NEAR>();
     else wait_vmcnt_imm<LPS_FAR>();
@@ -1025,10 +1037,15 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
 
   // this wave's steps of one head, walking down from tq = T-1: the last query step keeps the
   // content term, then the steps beyond the window, then the window, then the steps before tk
-  int n_last = 0, n_far = 0, n_win = 0;
+  int n_last = 0, n_far = 0, n_win = 0, n_over = 0;
   if (wave_on) {
     const int live = T_ - tk;
-    if (!has_content) n_far = live;
+    if (NEAR) {
+      const int win_top = min(T_ - 2, tk + W);
+      n_last = 1;
+      n_over = max(0, top - win_top);             // far for this wave, inside the window of another
+      n_win = win_top - tk + 1;
+    } else if (!has_content) n_far = live;
     else if (W <= 0) n_win = live;
     else {
       n_last = 1;
@@ -1036,10 +1053,11 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
       n_win = live - 1 - n_far;
     }
   }
-  const int n_idle = span - n_last - n_far - n_win;
+  const int n_idle = span - n_last - n_over - n_far - n_win;
   for (int hq = 0; hq < grp; ++hq) {
     for (int n = n_last; n > 0; --n) near_step(ring_step());
-    for (int n = n_far; n > 0; --n) far_step(ring_step());
+    if (NEAR) for (int n = n_over; n > 0; --n) (void)ring_step();
+    else for (int n = n_far; n > 0; --n) far_step(ring_step());
     for (int n = n_win; n > 0; --n) near_step(ring_step());
     for (int n = n_idle; n > 0; --n) (void)ring_step();
   }
@@ -1055,8 +1073,11 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
         float4 vk = make_float4(dK[mt][a4 * 4] * f, dK[mt][a4 * 4 + 1] * f, dK[mt][a4 * 4 + 2] * f, dK[mt][a4 * 4 + 3] * f);
         float4 vv = make_float4(dV[mt][a4 * 4], dV[mt][a4 * 4 + 1], dV[mt][a4 * 4 + 2], dV[mt][a4 * 4 + 3]);
         if (accum) {                              // launches of one stream: the query parts add up
-          const float4 ok = *(const float4*)(a.dk + o + d), ov = *(const float4*)(a.dv + o + d);
+          const float4 ok = *(const float4*)(a.dk + o + d);
           vk = make_float4(vk.x + ok.x, vk.y + ok.y, vk.z + ok.z, vk.w + ok.w);
+        }
+        if (NEAR || accum) {
+          const float4 ov = *(const float4*)(a.dv + o + d);
           vv = make_float4(vv.x + ov.x, vv.y + ov.y, vv.z + ov.z, vv.w + ov.w);
         }
         *(float4*)(a.dk + o + d) = vk;
@@ -1065,17 +1086,218 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   }
 }
 
+
+// ==========================================================================================
+// The far share of dv: dv^T[d][key] += dO^T[d][q] Ec[q][ck] et[q][tk] over the (query, key) steps outside
+// the content window, for 64 query and 64 key channels of a launch.  Nothing else of a far pair enters the key
+// pass, so that a wave holds the dv tiles of FR key steps at once: per query step it reads the Ec tile and
+// the dO fragments once for all of them.  In the key pass the wave of each key step reads both, three LDS
+// cycles for one of the matrix cores: 1.4 us a step with 0.1 us of products at Dh 128.  (Key pass of B1 C128
+// T512 Dh128 21.3 -> 11.5 ms, of B4 C64 T128 Dh64 820 -> 690 us; this kernel runs at 0.5 of the matrix cores'
+// rate there.)  The scalars et of a key step are one register per 32 queries: lane n of a row of 16 holds the
+// n-th query of the tile's register order, and the multiplication takes its operand from there by DPP.
+// ==========================================================================================
+constexpr int FR = 4;                                            // key steps per wave
+template <int DH> constexpr int FAR_WAVES = DH == 64 ? 8 : 4;    // FR tiles of Dh 128 are 256 registers
+template <int DH> constexpr int FAR_STAGES = DH == 64 ? 5 : 4;
+template <int DH> constexpr int FAR_STAGE_BYTES = 64 * 2 * DH + 64 * 64 * 4 + FR * FAR_WAVES<DH> / 2 * 256;
+
+// x * (the value of lane I of this lane's row of 16)
+template <int I>
+__device__ inline float times_row_lane(float x, float row) {
+  return x * __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(row), 0x150 + I, 0xf, 0xf, true));
+}
+template <int... I>
+__device__ inline f32x16 times_row(const float (&x)[16], float row, std::integer_sequence<int, I...>) {
+  f32x16 r;
+  ((r[I] = times_row_lane<I>(x[I], row)), ...);
+  return r;
+}
+
+template <int DH>
+__global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_bwd_args a, int k0, int q0, int accum) {
+  constexpr int MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8, CP = 64, NW = FAR_WAVES<DH>, KT = FR * NW / 2;
+  constexpr int TILE = CP * ROWB, OFF_EC = TILE, OFF_SC = TILE + CP * CP * 4;
+  constexpr int STAGES = FAR_STAGES<DH>, STAGE_BYTES = FAR_STAGE_BYTES<DH>;
+  constexpr int LPW = TILE / 1024 / NW, CS_LPW = CP * CP * 4 / 1024 / NW, SC_LPW = KT / NW, LPS = LPW + CS_LPW + SC_LPW;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ln = lane & 31, hh = lane >> 5;
+  const int kt = wave & 1, set = wave >> 1;       // key-channel tile, and which FR key steps
+  const int T_ = a.T, C_ = a.C, N = a.T * a.C, CW = (C_ + 3) & ~3;
+  const int Wf = a.window, tq_top = T_ - 2;       // far: tq - tk > Wf and tq <= tq_top
+  const int nbg = a.B * a.Hkv;
+  // the longest walks (early key steps) first, over all (b, kv head); those of one (b, kv head) on one XCD
+  const int bg = blockIdx.x % nbg, tile = blockIdx.x / nbg;
+  const int b = bg / a.Hkv, g = bg % a.Hkv, grp = a.H / a.Hkv;
+  const int tk0 = tile * KT, tkw = tk0 + set * FR;
+  const int span = max(0, tq_top - (tk0 + Wf)), nsteps = grp * span;   // query steps tq_top .. tk0 + Wf + 1
+
+  int d_off[LPW], cs_off[CS_LPW], sc_off[SC_LPW];
+#pragma unroll
+  for (int i = 0; i < LPW; ++i) {
+    const int pc = (wave + NW * i) * 64 + lane, r = pc / CPR, phys = pc % CPR;
+    d_off[i] = min(q0 + r, C_ - 1) * (int)a.do_stride_n + ((phys ^ swz_tr<DH>(r)) << 3);
+  }
+#pragma unroll
+  for (int i = 0; i < CS_LPW; ++i) {
+    const int pc = (wave + NW * i) * 64 + lane;
+    cs_off[i] = min(q0 + pc / (CP / 4), C_ - 1) * CW + k0 + min((pc % (CP / 4)) * 4, max(CW - k0 - 4, 0));
+  }
+#pragma unroll
+  for (int i = 0; i < SC_LPW; ++i) sc_off[i] = min(tk0 + wave + NW * i, T_ - 1) * C_ + min(q0 + lane, C_ - 1);
+  const uint32_t ring_lds = (uint32_t)(uintptr_t)(BWD_LDS_PTR(unsigned char))smem;
+  // source pointers of the step the ring fetches next: re-based at each head, stepped down otherwise
+  const bf16_t* p_do = nullptr;
+  const float *p_ec = nullptr, *p_sc = nullptr;
+  const int64_t d_do = (int64_t)C_ * a.do_stride_n, d_sc = (int64_t)T_ * C_;
+  const int d_ec = C_ * CW;
+  int ihq = 0, itq = tq_top;
+  auto rebase = [&]() {
+    const int h = g * grp + ihq;
+    const int64_t bhq = (int64_t)b * a.H + h;
+    p_do = (const bf16_t*)a.d_o + b * a.do_stride_b + h * a.do_stride_h + (int64_t)tq_top * d_do;
+    p_ec = a.ws_chan + (bhq * N + (int64_t)tq_top * C_) * CW;
+    p_sc = a.ws_time + (bhq * T_ + tq_top) * d_sc;
+  };
+  auto issue_next = [&](int stage_idx) {
+    const uint32_t st = ring_lds + stage_idx * STAGE_BYTES;
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) dma16(p_do + d_off[i], st + (wave + NW * i) * 1024);
+#pragma unroll
+    for (int i = 0; i < CS_LPW; ++i) dma16(p_ec + cs_off[i], st + OFF_EC + (wave + NW * i) * 1024);
+#pragma unroll
+    for (int i = 0; i < SC_LPW; ++i) dma4(p_sc + sc_off[i], st + OFF_SC + (wave + NW * i) * 256);
+    if (--itq <= tk0 + Wf) {
+      itq = tq_top;
+      if (++ihq < grp) rebase();
+    } else {
+      p_do -= d_do;
+      p_ec -= d_ec;
+      p_sc -= d_sc;
+    }
+  };
+
+  f32x16 dV[FR][MT];
+#pragma unroll
+  for (int r = 0; r < FR; ++r)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dV[r][mt][i] = 0.f;
+
+  int t_lane[MT];
+  {
+    const int e = (ln & 15) >> 2, aa = ln & 3, grp16 = ln >> 4, row0 = 4 * hh + e;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp16 + (aa >> 1)) ^ swz_tr<DH>(row0)) << 4) + ((aa & 1) << 3);
+  }
+  auto tr_frag = [&](const unsigned char* tile_p, int qt, int s, int mt) -> bf16x8 {
+    const unsigned char* p = tile_p + t_lane[mt] + (32 * qt + 16 * s) * ROWB;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))p);
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  };
+  // the query whose scalar this lane holds: register n = lane & 15 of the product layout
+  const int qn = (((lane & 15) >> 2) << 3) + hh * 4 + (lane & 3);
+  uint32_t q_mask[2];
+#pragma unroll
+  for (int qt = 0; qt < 2; ++qt) q_mask[qt] = q0 + qt * 32 + qn < C_ ? 0xffffffffu : 0u;
+
+  rebase();
+#pragma unroll
+  for (int s = 0; s < STAGES - 1; ++s)
+    if (s < nsteps) issue_next(s);
+  int stage = 0, tq = tq_top;
+  for (int it = 0; it < nsteps; ++it) {
+    // the step has landed once only the loads of the younger ones are in flight
+    const int left = nsteps - 1 - it;
+    if (left >= STAGES - 2) wait_vmcnt_imm<(STAGES - 2) * LPS>();
+    else if (left >= 2) wait_vmcnt_imm<2 * LPS>();
+    else if (left == 1) wait_vmcnt_imm<LPS>();
+    else wait_vmcnt_imm<0>();
+    lds_barrier();            // the stage visible to all; the previous one is free
+    if (left >= STAGES - 1) issue_next(stage == 0 ? STAGES - 1 : stage - 1);
+    const unsigned char* base = smem + stage * STAGE_BYTES;
+    const float* Ecs = (const float*)(base + OFF_EC) + kt * 32 + ln;
+    const float* Sc = (const float*)(base + OFF_SC) + set * FR * 64 + qn;
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+      float ec[16], et[FR];
+#pragma unroll
+      for (int r = 0; r < FR; ++r) {
+        // 0 for padded queries and for the pairs of this step that are not far (their slot holds something else)
+        const uint32_t m = tq - (tkw + r) > Wf ? q_mask[qt] : 0u;
+        et[r] = __uint_as_float(__float_as_uint(Sc[r * 64 + qt * 32]) & m);
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) ec[i] = Ecs[(qt * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)) * CP];
+      bf16x8 df[2][MT];
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) df[s][mt] = tr_frag(base, qt, s, mt);
+#pragma unroll
+      for (int r = 0; r < FR; ++r) {
+        const f32x16 P = times_row(ec, et[r], std::make_integer_sequence<int, 16>{});
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const bf16x8 pf = pack8(P, 8 * s);
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+            dV[r][mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(df[s][mt], pf, dV[r][mt], 0, 0, 0);
+        }
+      }
+    }
+    stage = stage + 1 == STAGES ? 0 : stage + 1;
+    if (--tq <= tk0 + Wf) tq = tq_top;
+  }
+
+  const int ck = k0 + kt * 32 + ln;
+#pragma unroll
+  for (int r = 0; r < FR; ++r) {
+    if (tkw + r >= T_ || ck >= C_) continue;
+    float* o = a.dv + ((((int64_t)b * a.Hkv + g) * N) + (int64_t)(tkw + r) * C_ + ck) * DH;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        float4* dst = (float4*)(o + mt * 32 + a4 * 8 + hh * 4);
+        float4 v = make_float4(dV[r][mt][a4 * 4], dV[r][mt][a4 * 4 + 1], dV[r][mt][a4 * 4 + 2], dV[r][mt][a4 * 4 + 3]);
+        if (accum) {
+          const float4 old = *dst;
+          v = make_float4(v.x + old.x, v.y + old.y, v.z + old.z, v.w + old.w);
+        }
+        *dst = v;
+      }
+  }
+}
+
 }  // namespace bwdq
 }  // namespace mvpa
 
-template <int DH, int NCT, bool MASKED>
+template <int DH>
+static void launch_far(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum) {
+  using namespace mvpa::bwdq;
+  constexpr int nw = FAR_WAVES<DH>, kt = FR * nw / 2;
+  constexpr size_t lds = (size_t)FAR_STAGES<DH> * FAR_STAGE_BYTES<DH>;
+  static_assert(lds <= 160 * 1024, "far-pass ring exceeds the LDS");
+  dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * a->Hkv));
+  auto kern = mvpa_bwd_far_kernel<DH>;
+  mvpa::want_dynamic_lds((const void*)kern, (int)lds);
+  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum);
+}
+
+template <int DH, int NCT, bool MASKED, bool NEAR>
 static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum) {
   using namespace mvpa::bwdq;
   constexpr int nw = KEY_WAVES<NCT>, cp = NCT * 32, kt = nw / NCT, ROWB = 2 * DH;
   static_assert((size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256) <= 160 * 1024, "key-pass ring exceeds the LDS");
   const size_t lds = (size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256);
   dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * a->Hkv));
-  auto kern = mvpa_bwd_key_mfma_kernel<DH, NCT, MASKED>;
+  auto kern = mvpa_bwd_key_mfma_kernel<DH, NCT, MASKED, NEAR>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
   MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum);
 }
@@ -1091,21 +1313,36 @@ static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 // (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).
 template <int DH>
 static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
-  const int C = a->C;
+  using namespace mvpa::bwdq;
+  const int C = a->C, T = a->T;
   constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
+  // Far query steps (outside the content window and not the last step) in a kernel of their own where its
+  // workgroups, of four times as many key steps, still fill the chip.  Forward and backward, far kernel / without:
+  // Dh 64, C 64, T 128: 384 workgroups 1794 / 1825 us, 256: 1265 / 1220, 128: 811 / 707;
+  // Dh 128, C 128: T 128, 128 workgroups 5.77 / 6.15 ms, T 512, 512 workgroups 40.9 / 50.7.
+  constexpr int FAR_KT = FR * FAR_WAVES<DH> / 2;
+  const int64_t far_groups = (int64_t)a->B * a->Hkv * ((T + FAR_KT - 1) / FAR_KT);
+  const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= FAR_KT &&
+                   far_groups >= (DH == 64 ? 384 : 128);
+  auto key_launch = [&](auto near, int kk, int qq, int accum) {
+    constexpr bool NEAR = decltype(near)::value;
+    const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
+    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, stream, kk, qq, accum);
+    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, stream, kk, qq, accum);
+  };
   auto key_launches = [&](int q0, int k0, int span, bool first_q) {
+    if (far) launch_far<DH>(a, stream, k0, q0, !first_q);
     for (int kk = k0; kk < min(k0 + span, C); kk += KEY_CP)
       for (int qq = q0; qq < min(q0 + span, C); qq += KEY_CP) {
         const int accum = !(first_q && qq == q0);
-        const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
-        if (full) launch_key<DH, KEY_CP / 32, false>(a, stream, kk, qq, accum);
-        else launch_key<DH, KEY_CP / 32, true>(a, stream, kk, qq, accum);
+        if (far) key_launch(std::true_type{}, kk, qq, accum);
+        else key_launch(std::false_type{}, kk, qq, accum);
       }
   };
   if (C <= 32) {
     launch_query<DH, 1>(a, stream, 0, 0, 0);
-    if (C == 32) launch_key<DH, 1, false>(a, stream, 0, 0, 0);
-    else launch_key<DH, 1, true>(a, stream, 0, 0, 0);
+    if (C == 32) launch_key<DH, 1, false, false>(a, stream, 0, 0, 0);
+    else launch_key<DH, 1, true, false>(a, stream, 0, 0, 0);
   } else {
     const int parts = (C + 63) / 64;
     for (int kp = 0; kp < parts; ++kp)

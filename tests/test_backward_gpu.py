@@ -258,3 +258,36 @@ def test_backward_bf16_strided_inputs_match_contiguous():
     got = mvpa_hip.mvpa_backward(q, k, v, o, g, lse, *tabs)
     for a, b in zip(got, ref):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("B,C,T,H,Hkv,Dh,window,masked", [
+    (48, 33, 21, 8, 4, 64, 3, True),       # 384 workgroups of 16 key steps, the second holds 5; one live channel in tile 2
+    (32, 64, 33, 4, 4, 64, 1, False),      # a third group of one key step; whole tiles
+    (24, 65, 40, 16, 8, 64, 20, True),     # four launches, parts of 64 and 1 channels; the far steps end inside a group
+    (32, 40, 13, 2, 2, 128, 3, True),      # 128 workgroups of 8 key steps, the second has no far step
+    (8, 100, 25, 8, 4, 128, 10, False),    # parts of 64 and 36 channels, GQA
+])
+def test_far_steps_in_their_own_kernel(B, C, T, H, Hkv, Dh, window, masked):
+    """A batch whose far query steps get a kernel of their own against its samples one at a time, which do
+    not: the same sums in another order (fp32), rounded to bf16 once on either side."""
+    from attentions import flashmvpa
+    g = torch.Generator(device="cuda").manual_seed(C * T)
+
+    def rn(*s, std=1.0):
+        return (torch.randn(s, generator=g, device="cuda") * std).bfloat16()
+    q, k, v, d = rn(B, H, T * C, Dh), rn(B, Hkv, T * C, Dh, std=Dh ** -0.5), rn(B, Hkv, T * C, Dh), rn(B, H, T * C, Dh)
+    tabs = [rn(1, Hkv, 1, Dh, std=0.1) for _ in range(3)] + [rn(1, Hkv, T, Dh, std=0.1), rn(1, Hkv, C, Dh, std=0.1)]
+    valid = None
+    if masked:
+        valid = torch.rand((B, C), generator=g, device="cuda") < 0.8
+        valid[:, 0] = True
+
+    def grads(b):
+        leaves = [x[b].clone().requires_grad_(True) for x in (q, k, v)]
+        out = flashmvpa(leaves[0], *tabs[:3], leaves[1], *tabs[3:], leaves[2], True, Dh ** -0.5, window_size=window,
+                        chan_valid=valid[b] if masked else None)
+        return torch.autograd.grad(out, leaves, d[b])
+    whole = grads(slice(0, B))
+    for b in range(0, B, 5):
+        for x, y in zip(whole, grads(slice(b, b + 1))):
+            assert (x[b].double() - y[0].double()).norm() <= 2.0 ** -8 * y.double().norm()
