@@ -122,14 +122,23 @@ __device__ inline float xhalf_sum(float x) { return x + __shfl_xor(x, 32); }
 template <int DH> __device__ inline int swz_row(int row) { return DH == 64 ? ((row >> 1) & 7) : (row & 15); }
 template <int DH> __device__ inline int swz_tr(int row) { return DH == 64 ? (((row >> 1) & 1) << 2) : ((row & 3) << 2); }
 
-template <int DH, int NCT>
-__global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
+// ONE: the whole walk.  FAR, WIN: the steps before a wave's content window and those from it on, as a launch
+// each, FAR first.  At Dh 128 a wave of the whole walk takes 475 registers and has its SIMD to itself: the far steps'
+// LDS reads, products, reductions and table slabs simply add up (0.89 us a step of 2 x 64 queries at T 512, 0.25 of
+// them products).  FAR alone fits in 256, and two waves cover each other's waits (1.3 us a step of 4 x 64 queries).
+enum query_phase { ONE, FAR, WIN };
+template <int DH, int NCT, int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : QUERY_WAVES<DH, NCT>;
+template <int DH, int NCT, int PHASE> constexpr int PHASE_STAGES = PHASE == FAR ? 5 : QSTAGES<DH, NCT>;
+
+template <int DH, int NCT, int PHASE>
+__global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
-  constexpr int NW = QUERY_WAVES<DH, NCT>;
+  constexpr int NW = PHASE_WAVES<DH, NCT, PHASE>;
   constexpr bool SOLO = NW == 4;                  // one wave per SIMD
   constexpr int CP = NCT * 32, TQW = NW / NCT, TILE = CP * ROWB;
   static_assert(64 * 32 <= WAVE_SCRATCH && 32 * (CP + 1) <= WAVE_SCRATCH, "channel tables overlay the slabs");
-  constexpr int STAGES = QSTAGES<DH, NCT>, STAGE_BYTES = 3 * TILE;   // stage: V | K | K (transposing)
+  // stage: V | K | K (transposing); FAR reads V only
+  constexpr int STAGES = PHASE_STAGES<DH, NCT, PHASE>, STAGE_BYTES = PHASE == FAR ? TILE : 3 * TILE;
   constexpr int LPW = TILE / 1024 / NW;           // 1 KiB wave loads per wave and tile copy
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   float* wave_base = (float*)(smem + STAGES * STAGE_BYTES);
@@ -209,6 +218,13 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   }
   // first key step whose K is needed: the band of the earliest query step of the workgroup
   const int tk_near = !has_content ? tq_hi + 1 : (W <= 0 || tq_hi == T_ - 1) ? 0 : max(0, tq0 - W);
+  // this wave's far steps are those before far_end (none for the last time step, whose queries keep the content
+  // term everywhere); the workgroup walks the key steps tk_lo .. tk_hi
+  const int far_end = !active ? 0 : !has_content ? tq + 1 : (W <= 0 || tq == T_ - 1) ? 0 : max(0, tq - W);
+  const int far_top = tq_hi == T_ - 1 ? T_ - 2 : tq_hi;           // FAR: the latest query step with far steps
+  const int tk_lo = PHASE == WIN ? tk_near : 0;
+  const int tk_hi = PHASE == FAR ? (far_top < tq0 ? -1 : far_top - W - 1) : tq_hi;
+  const int tk_first = PHASE == WIN ? far_end : 0;                // slabs of 32 steps count from here
   const uint32_t ring_lds = (uint32_t)(uintptr_t)(BWD_LDS_PTR(unsigned char))smem;
   auto issue_tile = [&](int tk, int stage_idx, bool with_k) {
     const uint32_t st = ring_lds + stage_idx * STAGE_BYTES;
@@ -226,7 +242,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   };
 #pragma unroll
   for (int s = 0; s < STAGES - 1; ++s)
-    if (s <= tq_hi) issue_tile(s, s, s >= tk_near);
+    if (tk_lo + s <= tk_hi) issue_tile(tk_lo + s, s, PHASE != FAR && tk_lo + s >= tk_near);
 
   // ---- set-up: operand fragments, delta, channel-bias tile
   bf16x8 dOf[KS];            // (q+u), (q+v) fragments are re-formed where needed, not kept
@@ -259,7 +275,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
     for (int ks = 0; ks < KS; ++ks) {
       const int d0 = ks * 16 + hh * 8;
       const u32x4 raw = raw_[ks], draw = draw_[ks], oraw = oraw_[ks];
-      if (qok) *(bf16x8*)((bf16_t*)a.ws_qu + row * DH + d0) = qfrag(raw, bu + d0, sc2);   // for the key pass
+      if (PHASE != WIN && qok) *(bf16x8*)((bf16_t*)a.ws_qu + row * DH + d0) = qfrag(raw, bu + d0, sc2);   // for the key pass
       qz[ks] = qfrag(raw, bz + d0, sc2);
       dOf[ks] = as_frag(draw);
 #pragma unroll
@@ -336,7 +352,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
     sumEc = xhalf_sum(sumEc);
     // for the key pass: (q+u) * scale, delta, and the tile exp2(channel bias - mc) by
     // [query][key channel]; and the rows of dbias_time that no key step reaches
-    if (qok) {
+    if (PHASE != WIN && qok) {
       float* wc = a.ws_chan + row * CW + k0;      // rows of CW floats: 16-byte aligned for any C
 #pragma unroll
       for (int t = 0; t < NCT; ++t)
@@ -347,7 +363,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
             *(float4*)(wc + ci) = make_float4(Ec[t][a4 * 4], Ec[t][a4 * 4 + 1], Ec[t][a4 * 4 + 2], Ec[t][a4 * 4 + 3]);
         }
     }
-    if (qok && hh == 0) a.ws_delta[row] = -delta;
+    if (PHASE != WIN && qok && hh == 0) a.ws_delta[row] = -delta;
   }
 
   f32x16 dq[MT], dSc[NCT];
@@ -367,7 +383,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   const int64_t wrow0 = ((int64_t)b * a.H + h) * N + (int64_t)(active ? tq : 0) * C_ + cq0;
 
   // the columns of dbias_time that no key step reaches (once: by the launch that does not add)
-  if (!accum)
+  if (PHASE != WIN && !accum)
     for (int q = hh; q < nq_live; q += 2)
       for (int j = ln; j < T_ - 1 - tq; j += 32) a.dbias_time[(wrow0 + q) * T_ + j] = 0.f;
 
@@ -392,7 +408,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   // writes the gradients of the slab that started at key step tks, and its per-pair scalars for
   // the key pass (the exponent e = time bias - L + mc for pairs inside the window, else exp2(e))
   auto flush_slab = [&](int tks) {
-    const int nj = min(32, tq - tks + 1);
+    const int nj = min(32, (PHASE == FAR ? far_end : tq + 1) - tks);
     // fixed trip counts with predicates: the LDS reads of several iterations go out together
 #pragma unroll 8
     for (int it = 0; it < 16; ++it) {
@@ -422,18 +438,19 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   auto ring_step = [&](int tk) -> const unsigned char* {
     // tile tk has landed once at most the loads of the younger tiles are in flight (a count that
     // is too small only waits longer)
-    if (tk + 1 >= tk_near && tk + STAGES - 2 <= tq_hi) {
-      wait_vmcnt_imm<(STAGES - 2) * 3 * LPW>();
+    constexpr int WITH_K = PHASE == FAR ? 1 : 3;  // tiles of a step from tk_near on
+    if ((PHASE == FAR || tk + 1 >= tk_near) && tk + STAGES - 2 <= tk_hi) {
+      wait_vmcnt_imm<(STAGES - 2) * WITH_K * LPW>();
     } else {
       int younger = 0;
 #pragma unroll
       for (int d = 1; d <= STAGES - 2; ++d)
-        if (tk + d <= tq_hi) younger += LPW * (tk + d >= tk_near ? 3 : 1);
+        if (tk + d <= tk_hi) younger += LPW * (tk + d >= tk_near ? WITH_K : 1);
       wait_vmcnt(younger);
     }
     lds_barrier();            // tile tk visible to all; everyone is done with tile tk-1's stage
-    if (tk + STAGES - 1 <= tq_hi)
-      issue_tile(tk + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1, tk + STAGES - 1 >= tk_near);
+    if (tk + STAGES - 1 <= tk_hi)
+      issue_tile(tk + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1, PHASE != FAR && tk + STAGES - 1 >= tk_near);
     const unsigned char* Vrow = smem + stage * STAGE_BYTES;
     stage = stage + 1 == STAGES ? 0 : stage + 1;
     return Vrow;
@@ -441,8 +458,8 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
 
   // every 32 key steps: write the finished slab, form the next slab of time-bias scores
   auto time_slab = [&](int tk) {
-    if ((tk & 31) == 0) {
-      if (tk > 0) {
+    if (((tk - tk_first) & 31) == 0) {
+      if (tk > tk_first) {
         wave_sync_lds();
         flush_slab(tk - 32);
         wave_sync_lds();
@@ -525,7 +542,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   auto near_step = [&](const unsigned char* Vrow, int tk) {
     const unsigned char* Krow = Vrow + TILE;
     const unsigned char* Ktr = Vrow + 2 * TILE;
-    const float off2 = Stb[(tk & 31) * 32 + ln] - lse;
+    const float off2 = Stb[((tk - tk_first) & 31) * 32 + ln] - lse;
     float gt = 0.f;
 #pragma unroll
     for (int t = 0; t < NCT; ++t) {               // one key-channel tile at a time: fewer live tiles
@@ -576,14 +593,28 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
       }
     }
     gt = xhalf_sum(gt);
-    if (hh == 0) Gtb[(tk & 31) * GP + ln] = gt;
+    if (hh == 0) Gtb[((tk - tk_first) & 31) * GP + ln] = gt;
   };
 
-  // far steps first (none for the last time step, whose queries keep the content term everywhere),
-  // then the steps inside the window; waves that are done keep the ring and the barriers going
-  const int far_end = !active ? 0 : !has_content ? tq + 1 : (W <= 0 || tq == T_ - 1) ? 0 : max(0, tq - W);
-  int tk = 0;
-  {
+  // far steps first, then the steps inside the window; waves that are done keep the ring and the barriers going
+  int tk = tk_lo;
+  if constexpr (PHASE == FAR) {
+    f32x16 dP[NCT];
+    for (; tk < far_end; ++tk) {
+      const unsigned char* Vrow = ring_step(tk);
+      time_slab(tk);
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dP[t][i] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+          dP[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB), dOf[ks], dP[t], 0, 0, 0);
+      }
+      far_reduce(dP, tk);
+    }
+    for (; tk <= tk_hi; ++tk) (void)ring_step(tk);
+  } else if constexpr (PHASE == ONE) {
     f32x16 dPa[NCT], dPb[NCT];
     int tkp = -1;
     for (; tk + 1 < far_end; tk += 2) {
@@ -603,6 +634,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dSc[t][i] = Ec[t][i] * (dSc[t][i] - delta * esum);
+  if constexpr (PHASE != FAR) {
   // Bc = mc + log2(Ec): the table it was gathered from lies under the slabs by now (-inf where
   // Ec = 0: masked keys, and biases more than 126 octaves below the row's largest)
 #pragma unroll
@@ -614,18 +646,20 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
     Qu[ks] = qfrag(*(const u32x4*)(qrow + ks * 16 + hh * 8), bu + ks * 16 + hh * 8, sc2);
   for (; tk <= tq_hi; ++tk) {
     const unsigned char* Vrow = ring_step(tk);
-    if (active && tk <= tq) {
+    if (active && tk >= far_end && tk <= tq) {
       time_slab(tk);
       near_step(Vrow, tk);
     }
   }
+  }
 
   if (!active) return;
   wave_sync_lds();
-  flush_slab(tq & ~31);
+  const int tk_end = PHASE == FAR ? far_end : tq + 1;
+  if (tk_end > tk_first) flush_slab(tk_first + ((tk_end - 1 - tk_first) & ~31));
 
   // dq^T[d][q]: this lane's query, d = 32mt + 8a4 + 4hh + 0..3
-  if (qok) {
+  if (PHASE != FAR && qok) {
     float* dqo = a.dq + row * DH;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
@@ -665,7 +699,7 @@ __global__ __launch_bounds__((QUERY_WAVES<DH, NCT> * 64)) void mvpa_bwd_query_mf
       if (d > 0 && hi >= 0 && hi < CP) g += g2;
       if (q < nq_live && col < C_) {
         float* dst = a.dbias_chan + (wrow0 + q) * C_ + col;
-        if (accum) atomicAdd(dst, g);
+        if (accum || PHASE == WIN) atomicAdd(dst, g);
         else *dst = g;
       }
     }
@@ -698,14 +732,16 @@ int mvpa_bwd_query_mfma_supported(const mvpa_bwd_args* a) {
   return 1;
 }
 
-template <int DH, int NCT>
+template <int DH, int NCT, int PHASE>
 static void launch_query(const mvpa_bwd_args* a, hipStream_t stream, int q0, int k0, int accum) {
   using namespace mvpa::bwdq;
-  constexpr int nw = QUERY_WAVES<DH, NCT>, tqw = nw / NCT, cp = NCT * 32, ROWB = 2 * DH;
+  constexpr int nw = PHASE_WAVES<DH, NCT, PHASE>, tqw = nw / NCT, cp = NCT * 32, ROWB = 2 * DH;
   const int nt = (a->T + tqw - 1) / tqw;
-  const size_t lds = (size_t)QSTAGES<DH, NCT> * 3 * cp * ROWB + (size_t)nw * WAVE_SCRATCH * sizeof(float);
+  constexpr size_t lds = (size_t)PHASE_STAGES<DH, NCT, PHASE> * (PHASE == FAR ? 1 : 3) * cp * ROWB +
+                         (size_t)nw * WAVE_SCRATCH * sizeof(float);
+  static_assert(lds <= 160 * 1024, "query-pass ring exceeds the LDS");
   dim3 grid((unsigned)(nt * a->B * a->H));
-  auto kern = mvpa_bwd_query_mfma_kernel<DH, NCT>;
+  auto kern = mvpa_bwd_query_mfma_kernel<DH, NCT, PHASE>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
   MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, q0, k0, accum);
 }
@@ -1311,6 +1347,10 @@ static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 // At Dh 128 a key-pass stage of 64 channels does not fit the LDS three times: the key pass then
 // takes the (query part, key part) pair of a query-pass launch in quarters of 32 x 32 channels
 // (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).
+// far steps of the longest walk from which the two phases of the query pass are a launch each (Dh 128): the
+// set-up of a workgroup is paid twice.  Forward and backward, one launch / two: T 128 5.77 / 5.95 ms (C 128, B 1),
+// T 512 40.8 / 39.3 (query pass 18.5 / 16.3).
+constexpr int SPLIT_STEPS = 256;
 template <int DH>
 static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
   using namespace mvpa::bwdq;
@@ -1324,6 +1364,7 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
   const int64_t far_groups = (int64_t)a->B * a->Hkv * ((T + FAR_KT - 1) / FAR_KT);
   const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= FAR_KT &&
                    far_groups >= (DH == 64 ? 384 : 128);
+  const bool split_query = DH == 128 && (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && T - 2 - a->window >= SPLIT_STEPS;
   auto key_launch = [&](auto near, int kk, int qq, int accum) {
     constexpr bool NEAR = decltype(near)::value;
     const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
@@ -1340,14 +1381,20 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
       }
   };
   if (C <= 32) {
-    launch_query<DH, 1>(a, stream, 0, 0, 0);
+    launch_query<DH, 1, ONE>(a, stream, 0, 0, 0);
     if (C == 32) launch_key<DH, 1, false, false>(a, stream, 0, 0, 0);
     else launch_key<DH, 1, true, false>(a, stream, 0, 0, 0);
   } else {
     const int parts = (C + 63) / 64;
     for (int kp = 0; kp < parts; ++kp)
       for (int qp = 0; qp < parts; ++qp) {
-        launch_query<DH, 2>(a, stream, qp * 64, kp * 64, kp > 0);
+        if constexpr (DH == 128) {
+          if (split_query) {
+            launch_query<DH, 2, FAR>(a, stream, qp * 64, kp * 64, kp > 0);
+            launch_query<DH, 2, WIN>(a, stream, qp * 64, kp * 64, kp > 0);
+          }
+        }
+        if (!split_query) launch_query<DH, 2, ONE>(a, stream, qp * 64, kp * 64, kp > 0);
         key_launches(qp * 64, kp * 64, 64, qp == 0);
       }
   }

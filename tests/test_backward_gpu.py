@@ -266,6 +266,7 @@ def test_backward_bf16_strided_inputs_match_contiguous():
     (24, 65, 40, 16, 8, 64, 20, True),     # four launches, parts of 64 and 1 channels; the far steps end inside a group
     (32, 40, 13, 2, 2, 128, 3, True),      # 128 workgroups of 8 key steps, the second has no far step
     (8, 100, 25, 8, 4, 128, 10, False),    # parts of 64 and 36 channels, GQA
+    (4, 33, 268, 2, 1, 128, 10, True),     # 256 far steps: two launches of the query pass; 136 workgroups
 ])
 def test_far_steps_in_their_own_kernel(B, C, T, H, Hkv, Dh, window, masked):
     """A batch whose far query steps get a kernel of their own against its samples one at a time, which do
@@ -291,3 +292,29 @@ def test_far_steps_in_their_own_kernel(B, C, T, H, Hkv, Dh, window, masked):
     for b in range(0, B, 5):
         for x, y in zip(whole, grads(slice(b, b + 1))):
             assert (x[b].double() - y[0].double()).norm() <= 2.0 ** -8 * y.double().norm()
+
+
+@pytest.mark.parametrize("T,C,Dh,window,masked", [(267, 5, 128, 10, False), (268, 33, 128, 10, False), (269, 40, 128, 11, True),
+                                                  (290, 70, 128, 2, False)])
+def test_long_walks_against_the_fp32_kernels(T, C, Dh, window, masked):
+    """Both sides of the line where the query pass becomes two launches, slabs that end inside and at the end of
+    a walk, against the fp32 kernels on the same (bf16) inputs."""
+    from attentions import flashmvpa
+    g = torch.Generator(device="cuda").manual_seed(C * T)
+
+    def rn(*s, std=1.0):
+        return (torch.randn(s, generator=g, device="cuda") * std).bfloat16()
+    args = [rn(1, 2, T * C, Dh)] + [rn(1, 1, 1, Dh, std=0.1) for _ in range(3)] + \
+           [rn(1, 1, T * C, Dh, std=Dh ** -0.5), rn(1, 1, T, Dh, std=0.1), rn(1, 1, C, Dh, std=0.1), rn(1, 1, T * C, Dh)]
+    d = rn(1, 2, T * C, Dh)
+    valid = None
+    if masked:
+        valid = torch.ones((1, C), dtype=torch.bool, device="cuda")
+        valid[0, 1::3] = False
+
+    def grads(dtype):
+        leaves = [x.to(dtype).requires_grad_(True) for x in args]
+        out = flashmvpa(*leaves, True, Dh ** -0.5, window_size=window, chan_valid=valid)
+        return torch.autograd.grad(out, leaves, d.to(dtype))
+    for n, x, y in zip(NAMES, grads(torch.bfloat16), grads(torch.float32)):
+        assert (x.double() - y.double()).norm() <= 2e-2 * y.double().norm(), n      # the bf16 bound of this file
