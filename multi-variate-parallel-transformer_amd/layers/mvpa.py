@@ -344,10 +344,11 @@ class MVPFormerGQAAttention(torch.nn.Module):
         return bool(self.global_att)                       # layers/mvpa.py:188-222, 230
 
     def _attend(self, hidden_states, positional_embedding, channel_embedding, attention_mask,
-                head_mask, use_cache, window, layer_past=None, merged_out=None, qkv=None):
+                head_mask, use_cache, window, layer_past=None, merged_out=None, qkv=None, key_tables=None):
         """merged_out: a [B, T*C, H, Dh] view (unit last stride, any row pitch) that receives the
         merged heads; c_proj is then left to the caller and merged_out is what comes back.
-        qkv: hidden_states @ [q_attn; c_attn]^T when the caller has already formed it."""
+        qkv: hidden_states @ [q_attn; c_attn]^T when the caller has already formed it.  key_tables: the two
+        bias tables ([Hkv,T,Dh], [Hkv,C,Dh]) when the caller has formed them, for a differentiable pass."""
         if self.training and (self.attn_dropout.p > 0 or self.resid_dropout.p > 0):
             # dropout lives on the differentiable path (one launch per op); the fused inference
             # path has none
@@ -374,7 +375,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
                                      attention_mask, head_mask, use_cache, window, layer_past)
         if merged_out is None and qkv is None and self._wants_grad(hidden_states):
             return self._attend_autograd(hidden_states, positional_embedding, channel_embedding,
-                                         attention_mask, head_mask, use_cache, window)
+                                         attention_mask, head_mask, use_cache, window, key_tables)
         with torch.no_grad():
             if qkv is None:
                 qkv = _linear(hidden_states, self._qkv_weight(dt))      # [B,T,C,E+2kvE]
@@ -414,7 +415,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
         return torch.is_grad_enabled() and (hidden_states.requires_grad or self.training)
 
     def _attend_autograd(self, hidden_states, positional_embedding, channel_embedding, attention_mask,
-                         head_mask, use_cache, window):
+                         head_mask, use_cache, window, key_tables=None):
         """The whole-sequence forward of layers/mvpa.py:280-337 as a differentiable graph: the four
         projections and c_proj through the library's GEMM (backward: two more GEMMs each), the
         attention through FlashMVPA (backward: mvpa_backward).  Same kernels as the inference path,
@@ -430,8 +431,11 @@ class MVPFormerGQAAttention(torch.nn.Module):
         q = qkv[:, :, :e].reshape(bsz, n, h, dh).permute(0, 2, 1, 3)
         k = qkv[:, :, e:e + kv].reshape(bsz, n, hkv, dh).permute(0, 2, 1, 3)
         v = v_plain = qkv[:, :, e + kv:].reshape(bsz, n, hkv, dh).permute(0, 2, 1, 3)
-        k_time = AG.linear(positional_embedding, self.position_net.weight).reshape(t_len, hkv, dh).permute(1, 0, 2)
-        k_chan = AG.linear(channel_embedding, self.channel_net.weight).reshape(c_len, hkv, dh).permute(1, 0, 2)
+        if key_tables is None:
+            k_time = AG.linear(positional_embedding, self.position_net.weight).reshape(t_len, hkv, dh).permute(1, 0, 2)
+            k_chan = AG.linear(channel_embedding, self.channel_net.weight).reshape(c_len, hkv, dh).permute(1, 0, 2)
+        else:
+            k_time, k_chan = key_tables
         u, vb, z = (b.reshape(hkv, dh).to(dt) for b in self.attn_bias.split(kv, dim=0))
         chan_valid, key_bias = self._resolve_mask(attention_mask, bsz, t_len, c_len)
         if self.training and self.attn_dropout.p > 0:
@@ -537,6 +541,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
         encoder_attention_mask: Optional[torch.Tensor] = None,
         use_cache: Optional[bool] = False,
         output_attentions: Optional[bool] = False,
+        key_tables=None,
     ):
         if encoder_hidden_states is not None:
             raise NotImplementedError("MVPA HIP layer: cross attention is not implemented")
@@ -547,7 +552,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
                 "MVPA HIP layer: the fused kernel never forms the [B,H,N,N] attention weights")
         out, present = self._attend(hidden_states, positional_embedding, channel_embedding,
                                     attention_mask, head_mask, use_cache, window=10,
-                                    layer_past=layer_past)
+                                    layer_past=layer_past, key_tables=key_tables)
         outputs = (out, present)
         if output_attentions:
             outputs += (None,)                            # layers/mvpa.py:407-408
@@ -591,9 +596,9 @@ class MVPFormerGQAFlashAttention(MVPFormerGQAAttention):
 
     def forward(self, hidden_states, positional_embedding, channel_embedding, layer_past=None,
                 attention_mask=None, head_mask=None, encoder_hidden_states=None,
-                encoder_attention_mask=None, use_cache=False, output_attentions=False):
+                encoder_attention_mask=None, use_cache=False, output_attentions=False, key_tables=None):
         out, present = self._attend(hidden_states, positional_embedding, channel_embedding,
-                                    None, None, use_cache, window=10, layer_past=layer_past)
+                                    None, None, use_cache, window=10, layer_past=layer_past, key_tables=key_tables)
         outputs = (out, present)
         if output_attentions:
             outputs += (None,)

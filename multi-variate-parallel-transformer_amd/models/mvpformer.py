@@ -213,7 +213,7 @@ class MVPFormerBlock(nn.Module):
 
     def forward_fused(self, hidden_states, normed, next_norm, positional_embedding,
                       channel_embedding, layer_past=None, attention_mask=None, head_mask=None,
-                      use_cache=False, output_attentions=False):
+                      use_cache=False, output_attentions=False, key_tables=None):
         """The block with its norms at the seams: `normed` is ln_1(hidden_states) when the caller
         already has it, `next_norm` the RMSNorm that will consume this block's output (the next
         block's ln_1, or ln_f).  Returns (outputs, next_norm(output) or None); the residual sum and
@@ -222,9 +222,10 @@ class MVPFormerBlock(nn.Module):
             # differentiable path (models/mvpformer.py:132-147 op by op; both branches read ln_1(x))
             if normed is None:
                 normed = self.ln_1(hidden_states)
+            tables = {} if key_tables is None else dict(key_tables=key_tables)
             attn_outputs = self.attn(normed, positional_embedding, channel_embedding,
                                      attention_mask=attention_mask, head_mask=head_mask,
-                                     use_cache=use_cache, output_attentions=output_attentions)
+                                     use_cache=use_cache, output_attentions=output_attentions, **tables)
             mlp_output = self.mlp(normed)
             both = None
             if next_norm is not None and _unhooked(next_norm):
@@ -359,6 +360,25 @@ class MVPFormerModel(nn.Module):
         with torch.set_grad_enabled(grad):
             return self._forward(past_key_values, inputs_embeds, attention_mask, use_cache, position_end,
                                  channel_validity)
+
+    def _all_key_tables(self, position_embeds, channel_embeds):
+        """The two bias tables of every block as one product each (position_net and channel_net of all blocks
+        stacked), for a differentiable pass: a block's own are two small products, and four more backward.
+        A list of (k_time [Hkv,T,Dh], k_chan [Hkv,C,Dh]), or Nones where a block is not of the plain kind."""
+        none = [None] * len(self.h)
+        if not (position_embeds.is_cuda and position_embeds.dtype == channel_embeds.dtype == torch.bfloat16):
+            return none
+        attns = [blk.attn for blk in self.h if type(blk) is MVPFormerBlock]
+        if len(attns) < 2 or len(attns) != len(self.h) or any(
+                type(a) not in (MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or "forward" in a.__dict__
+                or a.embed_kv_dim != attns[0].embed_kv_dim or a.head_dim != attns[0].head_dim for a in attns):
+            return none
+
+        def tables(embeds, nets):
+            out = AG.linear(embeds, torch.cat([n.weight for n in nets], 0))                 # [1, J, L Hkv Dh]
+            return out.view(-1, len(nets), attns[0].num_kv_heads, attns[0].head_dim).permute(1, 2, 0, 3).contiguous().unbind(0)
+        return list(zip(tables(position_embeds, [a.position_net for a in attns]),
+                        tables(channel_embeds, [a.channel_net for a in attns])))
 
     def _native_plan(self, t_len, c_len, pos_lo, normed):
         """The operands of every block for the library's stack call, collected once per shape and kept
@@ -522,12 +542,15 @@ class MVPFormerModel(nn.Module):
                     presents = presents + (outputs[1],)
             out = self.ln_f(hidden_states).view(bsz, inputs_embeds.shape[1], c_len, -1)
             return (out, presents) if use_cache else out
+        grad = past_key_values is None and torch.is_grad_enabled() and (hidden_states.requires_grad or self.training)
+        tables = self._all_key_tables(position_embeds, channel_embeds) if grad else [None] * n_layers
         for i, block in enumerate(self.h):
             next_norm = self.h[i + 1].ln_1 if i + 1 < n_layers else self.ln_f
             layer_past = past_key_values[i] if past_key_values is not None else None
             outputs, normed = block.forward_fused(hidden_states, normed, next_norm, position_embeds,
                                                   channel_embeds, layer_past=layer_past,
-                                                  attention_mask=attention_mask, use_cache=use_cache)
+                                                  attention_mask=attention_mask, use_cache=use_cache,
+                                                  key_tables=tables[i])
             hidden_states = outputs[0]
             if use_cache:
                 presents = presents + (outputs[1],)              # models/mvpformer.py:366-367
