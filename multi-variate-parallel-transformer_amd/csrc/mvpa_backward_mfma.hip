@@ -775,7 +775,7 @@ template <int NCT> constexpr int KEY_WAVES = NCT == 2 ? 8 : 4;
 
 // NEAR: the far steps are left to mvpa_bwd_far_kernel, which has written dv before.
 template <int DH, int NCT, bool MASKED, bool NEAR>
-__global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum) {
+__global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum, int per_head) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
   constexpr int NW = KEY_WAVES<NCT>;
   constexpr int CP = NCT * 32, KT = NW / NCT, TILE = CP * ROWB;
@@ -797,7 +797,8 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   const int T_ = a.T, C_ = a.C, W = a.window, N = a.T * a.C;
   const int CW = (C_ + 3) & ~3;                   // row pitch of the Ec tiles in the workspace
   const bool has_content = a.flags & MVPA_FLAG_CONTENT;
-  const int nbg = a.B * a.Hkv, ntk = (T_ + KT - 1) / KT;
+  // per_head: a workgroup takes one query head and dk, dv come per query head ([B,H,N,Dh])
+  const int out_heads = per_head ? a.H : a.Hkv, nbg = a.B * out_heads, ntk = (T_ + KT - 1) / KT;
   int bg, tile;
   {
     const int L = blockIdx.x;
@@ -810,8 +811,8 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
       tile = L % ntk;
     }
   }
-  const int b = bg / a.Hkv, g = bg % a.Hkv;
-  const int grp = a.H / a.Hkv;
+  const int b = bg / out_heads, g = per_head ? bg % out_heads / (a.H / a.Hkv) : bg % out_heads;
+  const int grp = per_head ? 1 : a.H / a.Hkv, h0 = per_head ? bg % out_heads : g * grp;
   const int tk0 = tile * KT;
   const int tk = tk0 + ktw;
   const bool wave_on = tk < T_;
@@ -887,7 +888,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   const int64_t d_do = (int64_t)C_ * a.do_stride_n, d_sc = (int64_t)T_ * C_;
   const int d_ec = C_ * CW, d_qu = C_ * DH;
   auto rebase = [&](int hq) {
-    const int h = g * grp + hq;
+    const int h = h0 + hq;
     const int64_t bhq = (int64_t)b * a.H + h;
     const int64_t r0 = bhq * N + (int64_t)(T_ - 1) * C_;    // first query row of step T-1
     p_do = (const bf16_t*)a.d_o + b * a.do_stride_b + h * a.do_stride_h + (int64_t)(T_ - 1) * d_do;
@@ -1099,7 +1100,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   }
 
   if (wave_on && ck < C_) {
-    const int64_t o = ((((int64_t)b * a.Hkv + g) * N) + (int64_t)tk * C_ + ck) * DH;
+    const int64_t o = (((int64_t)bg * N) + (int64_t)tk * C_ + ck) * DH;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -1151,7 +1152,7 @@ __device__ inline f32x16 times_row(const float (&x)[16], float row, std::integer
 }
 
 template <int DH>
-__global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_bwd_args a, int k0, int q0, int accum) {
+__global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_bwd_args a, int k0, int q0, int accum, int per_head) {
   constexpr int MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8, CP = 64, NW = FAR_WAVES<DH>, KT = FR * NW / 2;
   constexpr int TILE = CP * ROWB, OFF_EC = TILE, OFF_SC = TILE + CP * CP * 4;
   constexpr int STAGES = FAR_STAGES<DH>, STAGE_BYTES = FAR_STAGE_BYTES<DH>;
@@ -1163,10 +1164,10 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
   const int kt = wave & 1, set = wave >> 1;       // key-channel tile, and which FR key steps
   const int T_ = a.T, C_ = a.C, N = a.T * a.C, CW = (C_ + 3) & ~3;
   const int Wf = a.window, tq_top = T_ - 2;       // far: tq - tk > Wf and tq <= tq_top
-  const int nbg = a.B * a.Hkv;
+  const int out_heads = per_head ? a.H : a.Hkv, nbg = a.B * out_heads;
   // the longest walks (early key steps) first, over all (b, kv head); those of one (b, kv head) on one XCD
   const int bg = blockIdx.x % nbg, tile = blockIdx.x / nbg;
-  const int b = bg / a.Hkv, g = bg % a.Hkv, grp = a.H / a.Hkv;
+  const int b = bg / out_heads, grp = per_head ? 1 : a.H / a.Hkv, h0 = bg % out_heads * grp;
   const int tk0 = tile * KT, tkw = tk0 + set * FR;
   const int span = max(0, tq_top - (tk0 + Wf)), nsteps = grp * span;   // query steps tq_top .. tk0 + Wf + 1
 
@@ -1191,7 +1192,7 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
   const int d_ec = C_ * CW;
   int ihq = 0, itq = tq_top;
   auto rebase = [&]() {
-    const int h = g * grp + ihq;
+    const int h = h0 + ihq;
     const int64_t bhq = (int64_t)b * a.H + h;
     p_do = (const bf16_t*)a.d_o + b * a.do_stride_b + h * a.do_stride_h + (int64_t)tq_top * d_do;
     p_ec = a.ws_chan + (bhq * N + (int64_t)tq_top * C_) * CW;
@@ -1295,7 +1296,7 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
 #pragma unroll
   for (int r = 0; r < FR; ++r) {
     if (tkw + r >= T_ || ck >= C_) continue;
-    float* o = a.dv + ((((int64_t)b * a.Hkv + g) * N) + (int64_t)(tkw + r) * C_ + ck) * DH;
+    float* o = a.dv + (((int64_t)bg * N) + (int64_t)(tkw + r) * C_ + ck) * DH;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -1315,27 +1316,27 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
 }  // namespace mvpa
 
 template <int DH>
-static void launch_far(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum) {
+static void launch_far(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum, int per_head) {
   using namespace mvpa::bwdq;
   constexpr int nw = FAR_WAVES<DH>, kt = FR * nw / 2;
   constexpr size_t lds = (size_t)FAR_STAGES<DH> * FAR_STAGE_BYTES<DH>;
   static_assert(lds <= 160 * 1024, "far-pass ring exceeds the LDS");
-  dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * a->Hkv));
+  dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * (per_head ? a->H : a->Hkv)));
   auto kern = mvpa_bwd_far_kernel<DH>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
-  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum);
+  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum, per_head);
 }
 
 template <int DH, int NCT, bool MASKED, bool NEAR>
-static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum) {
+static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum, int per_head) {
   using namespace mvpa::bwdq;
   constexpr int nw = KEY_WAVES<NCT>, cp = NCT * 32, kt = nw / NCT, ROWB = 2 * DH;
   static_assert((size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256) <= 160 * 1024, "key-pass ring exceeds the LDS");
   const size_t lds = (size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256);
-  dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * a->Hkv));
+  dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * (per_head ? a->H : a->Hkv)));
   auto kern = mvpa_bwd_key_mfma_kernel<DH, NCT, MASKED, NEAR>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
-  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum);
+  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum, per_head);
 }
 
 // Both passes.  Up to 32 channels: one launch each with one channel tile per wave; up to 64: one
@@ -1352,7 +1353,7 @@ static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 // T 512 40.8 / 39.3 (query pass 18.5 / 16.3).
 constexpr int SPLIT_STEPS = 256;
 template <int DH>
-static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
+static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per_head) {
   using namespace mvpa::bwdq;
   const int C = a->C, T = a->T;
   constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
@@ -1361,18 +1362,18 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
   // Dh 64, C 64, T 128: 384 workgroups 1794 / 1825 us, 256: 1265 / 1220, 128: 811 / 707;
   // Dh 128, C 128: T 128, 128 workgroups 5.77 / 6.15 ms, T 512, 512 workgroups 40.9 / 50.7.
   constexpr int FAR_KT = FR * FAR_WAVES<DH> / 2;
-  const int64_t far_groups = (int64_t)a->B * a->Hkv * ((T + FAR_KT - 1) / FAR_KT);
+  const int64_t far_groups = (int64_t)a->B * (per_head ? a->H : a->Hkv) * ((T + FAR_KT - 1) / FAR_KT);
   const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= FAR_KT &&
                    far_groups >= (DH == 64 ? 384 : 128);
   const bool split_query = DH == 128 && (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && T - 2 - a->window >= SPLIT_STEPS;
   auto key_launch = [&](auto near, int kk, int qq, int accum) {
     constexpr bool NEAR = decltype(near)::value;
     const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
-    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, stream, kk, qq, accum);
-    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, stream, kk, qq, accum);
+    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, stream, kk, qq, accum, per_head);
+    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, stream, kk, qq, accum, per_head);
   };
   auto key_launches = [&](int q0, int k0, int span, bool first_q) {
-    if (far) launch_far<DH>(a, stream, k0, q0, !first_q);
+    if (far) launch_far<DH>(a, stream, k0, q0, !first_q, per_head);
     for (int kk = k0; kk < min(k0 + span, C); kk += KEY_CP)
       for (int qq = q0; qq < min(q0 + span, C); qq += KEY_CP) {
         const int accum = !(first_q && qq == q0);
@@ -1382,8 +1383,8 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
   };
   if (C <= 32) {
     launch_query<DH, 1, ONE>(a, stream, 0, 0, 0);
-    if (C == 32) launch_key<DH, 1, false, false>(a, stream, 0, 0, 0);
-    else launch_key<DH, 1, true, false>(a, stream, 0, 0, 0);
+    if (C == 32) launch_key<DH, 1, false, false>(a, stream, 0, 0, 0, per_head);
+    else launch_key<DH, 1, true, false>(a, stream, 0, 0, 0, per_head);
   } else {
     const int parts = (C + 63) / 64;
     for (int kp = 0; kp < parts; ++kp)
@@ -1400,8 +1401,8 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream) {
   }
 }
 
-int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream) {
-  if (a->Dh == 64) launch_bwd_parts<64>(a, stream);
-  else launch_bwd_parts<128>(a, stream);
+int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head) {
+  if (a->Dh == 64) launch_bwd_parts<64>(a, stream, per_head);
+  else launch_bwd_parts<128>(a, stream, per_head);
   return mvpa::take_launch_status();
 }

@@ -35,6 +35,7 @@ struct fin_args {
   float *p_du, *p_tab, *p_col;       // partial results: [b,h][row tile][Dh], [part][T + C][Dh], [part][T + C]
   float* csum;                       // [Hkv][T + C] column sums of G
   bf16_t *du, *dvb, *dz, *dk_time, *dk_chan;
+  int32_t kv_parts;                  // query heads whose partial dk, dv make one kv head's (1: summed already)
   int32_t tj_t, tj_c, n_split, split_len;   // column tiles of the two tables; row shares and their length
 };
 
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(256) void finish_rows_kernel(fin_args a) {
   }
 }
 
-// dk, dv: fp32 [B,Hkv,N,Dh] to bf16 rows at the caller's strides
+// dk, dv: fp32 [B,Hkv,kv_parts,N,Dh] summed over the parts, to bf16 rows at the caller's strides
 template <int DH>
 __global__ __launch_bounds__(256) void finish_kv_kernel(fin_args a) {
   const int64_t per = (int64_t)a.B * a.Hkv * a.N * (DH / 8);
@@ -166,10 +167,16 @@ __global__ __launch_bounds__(256) void finish_kv_kernel(fin_args a) {
   const int ch = (int)(i % (DH / 8));
   const int64_t r = i / (DH / 8);
   const int n = (int)(r % a.N), bg = (int)(r / a.N), b = bg / a.Hkv, g = bg % a.Hkv;
-  const float* src = (is_v ? a.dv : a.dk) + r * DH + ch * 8;
+  const float* src = (is_v ? a.dv : a.dk) + ((int64_t)bg * a.kv_parts * a.N + n) * DH + ch * 8;
   bf16_t* dst = is_v ? a.dv_out + b * a.dv_sb + g * a.dv_sh + (int64_t)n * a.dv_sn
                      : a.dk_out + b * a.dk_sb + g * a.dk_sh + (int64_t)n * a.dk_sn;
-  const float4 x = *(const float4*)src, y = *(const float4*)(src + 4);
+  float4 x = *(const float4*)src, y = *(const float4*)(src + 4);
+  for (int part = 1; part < a.kv_parts; ++part) {
+    src += (int64_t)a.N * DH;
+    const float4 x1 = *(const float4*)src, y1 = *(const float4*)(src + 4);
+    x.x += x1.x; x.y += x1.y; x.z += x1.z; x.w += x1.w;
+    y.x += y1.x; y.y += y1.y; y.z += y1.z; y.w += y1.w;
+  }
   *(bf16x8*)(dst + ch * 8) = bf16x8{(__bf16)x.x, (__bf16)x.y, (__bf16)x.z, (__bf16)x.w,
                                     (__bf16)y.x, (__bf16)y.y, (__bf16)y.z, (__bf16)y.w};
 }
@@ -342,12 +349,22 @@ static void row_split(const mvpa_bwd_args* b, int* n_split, int* len) {
   *n_split = (int)((N + *len - 1) / *len);
 }
 
+// A workgroup of the key pass walks the query heads of a kv head one after the other.  Where its workgroups (of four
+// key steps) are less than two rounds of the chip, each query head gets its own, and finish_kv adds up their dk, dv.
+// Forward and backward without / with, us: B4 C64 T25 H12/4 (112 workgroups) 342 / 293, B1 C64 T64 (64) 468 / 329,
+// B2 C64 T128 (256) 1091 / 1022, B1 C128 T128 H16/8 Dh128 (256) 5810 / 5350, B4 C128 T64 H16/8 Dh128 (512) 7430 / 7870.
+constexpr int64_t KEY_GROUPS_FULL = 512;
+static bool per_head(const mvpa_bwd_args* b) {
+  return b->H > b->Hkv && (int64_t)b->B * b->Hkv * ((b->T + 3) / 4) < KEY_GROUPS_FULL;
+}
+
 static void lay_out(const mvpa_bwd_args* b, fin_args& f, mvpa_bwd_args& w, layout& l) {
   const int64_t N = (int64_t)b->T * b->C, bhn = (int64_t)b->B * b->H * N, bgn = (int64_t)b->B * b->Hkv * N, Dh = b->Dh;
   w = *b;
   w.dq = l.take<float>(bhn * Dh);
-  w.dk = l.take<float>(bgn * Dh);
-  w.dv = l.take<float>(bgn * Dh);
+  f.kv_parts = per_head(b) ? b->H / b->Hkv : 1;
+  w.dk = l.take<float>(bgn * f.kv_parts * Dh);
+  w.dv = l.take<float>(bgn * f.kv_parts * Dh);
   w.dbias_time = l.take<float>(bhn * b->T);
   w.dbias_chan = l.take<float>(bhn * b->C);
   w.ws_delta = l.take<float>(bhn);
@@ -409,7 +426,7 @@ extern "C" int mvpa_backward_full(const mvpa_bwd_args* a, const mvpa_bwd_grads* 
   fin::lay_out(a, f, w, l);
   if ((size_t)l.used > ws_bytes) return MVPA_ERR_WS_SIZE;
   if (!mvpa_bwd_query_mfma_supported(&w)) return MVPA_ERR_UNSUPPORTED;
-  const int st = mvpa_backward(&w, stream);
+  const int st = mvpa_backward_checked(&w, (hipStream_t)stream, f.kv_parts > 1);
   if (st != MVPA_OK) return st;
   f.B = a->B; f.H = a->H; f.Hkv = a->Hkv; f.T = a->T; f.C = a->C; f.N = a->T * a->C;
   f.q = (const bf16_t*)a->q;

@@ -153,4 +153,6 @@ int mvpa_mfma128_supported(const mvpa_fwd_args* a);
 int mvpa_launch_mfma128(const mvpa_fwd_args* a, hipStream_t stream);
 // backward, query pass on MFMA (bf16, Dh = 64, C <= 64)
 int mvpa_bwd_query_mfma_supported(const mvpa_bwd_args* a);
-int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream);
+// per_head: dk and dv come per query head ([B,H,N,Dh]), for the caller to add up
+int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head);
+int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_head);
