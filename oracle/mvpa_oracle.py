@@ -38,6 +38,9 @@ Pinning status (what independent evidence fixes each function):
                                models/mvpformer.py:104-147, 246-283, 380 state it (parallel
                                block, both branches read ln_1(x), ln_2 unused, ln_f last), with
                                and without a token mask; a sequential block is shown to differ.
+  stack_forward              : equality with mvpformer_forward on its embeddings.
+  stream_steps               : equality with stack_forward while the content window holds every
+                               segment; with more segments, on one block.
   wavedec_db4_periodic       : the reference delegates to ptwt.wavedec (ptwt==0.1.9 with
                                PyWavelets' db4 filters, models/fftencoder.py:62, 70-88), not
                                installed here.  Its published algorithm - circular pad of
@@ -489,3 +492,94 @@ def mvpformer_forward(x: torch.Tensor, params: dict, cfg: dict,
         h = h + mlp + a                                             # :146-147
     h = rmsnorm(h, params["mvpformer.ln_f.weight"], eps)            # :380
     return h, embeds
+
+
+# --------------------------------------------------------------------------------------
+# the stack in 64 bits, whole windows and one segment at a time
+# --------------------------------------------------------------------------------------
+
+
+def _rmsnorm64(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
+    return x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps) * weight
+
+
+def _block64(h, p, cfg, attend):
+    """One parallel block (models/mvpformer.py:133-147) on rows h; attend(q, k, v) -> merged heads."""
+    e = h.shape[-1]
+    hn = _rmsnorm64(h, p["ln_1.weight"], cfg.get("layer_norm_epsilon", 1e-5))
+    q = hn @ p["attn.q_attn.weight"].T
+    k, v = (hn @ p["attn.c_attn.weight"].T).split(e // cfg["n_head"] * cfg["n_head_kv"], dim=-1)
+    act = torch.nn.functional.silu(hn @ p["mlp.gate_proj.weight"].T) * (hn @ p["mlp.up_proj.weight"].T)
+    return h + act @ p["mlp.down_proj.weight"].T + attend(q, k, v) @ p["attn.c_proj.weight"].T
+
+
+def _block_params(params: dict, i: int) -> dict:
+    pre = f"h.{i}."
+    return {n[len(pre):]: t for n, t in params.items() if n.startswith(pre)}
+
+
+def _tables64(p, cfg, e, pos, chan):
+    """u, v, z [Hkv,Dh] and the two bias tables [Hkv,J,Dh] (layers/mvpa.py:185-187, 307-313)."""
+    g, dh = cfg["n_head_kv"], e // cfg["n_head"]
+    rows = [b.view(g, dh) for b in p["attn.attn_bias"].split(g * dh)]
+    return rows + [(t @ p[f"attn.{n}.weight"].T).view(-1, g, dh).transpose(0, 1)
+                   for t, n in ((pos, "position_net"), (chan, "channel_net"))]
+
+
+def stack_forward(embeds: torch.Tensor, params: dict, cfg: dict, chan_valid: Optional[torch.Tensor] = None):
+    """mvpformer_forward without the encoder, in 64 bits: embeds [B,T,C,E], params under the names of
+    the stack alone (h.{i}.*, ln_f.weight, ...), chan_valid [B,C] -> [B,T,C,E]."""
+    params = {n: t.double() for n, t in params.items()}
+    b, t, c, e = embeds.shape
+    nh, g = cfg["n_head"], cfg["n_head_kv"]
+    h = embeds.double().reshape(b, t * c, e)
+    for i in range(cfg["n_layer"]):
+        p = _block_params(params, i)
+        tabs = _tables64(p, cfg, e, params["positional_embedding.weight"][:t], params["channel_embedding.weight"][:c])
+
+        def attend(q, k, v):
+            heads = (x.view(b, t * c, n, e // nh).transpose(1, 2) for x, n in ((q, nh), (k, g), (v, g)))
+            out = mvpa_direct(*heads, *tabs, chan_valid=chan_valid)
+            return out.transpose(1, 2).reshape(b, t * c, e)
+        h = _block64(h, p, cfg, attend)
+    return _rmsnorm64(h, params["ln_f.weight"], cfg.get("layer_norm_epsilon", 1e-5)).view(b, t, c, e)
+
+
+def stream_steps(embeds: torch.Tensor, params: dict, cfg: dict, max_steps: int):
+    """The segments of embeds [S,C,E] one at a time in 64 bits, on whatever device they are: each is the
+    newest step of a window of at most max_steps segments whose keys and values are those of the time they
+    arrived (layers/mvpa.py:314-321, along the time axis).  The newest step keeps the content term for every
+    key (layers/mvpa.py:244) and the positions end at row max_steps.  Returns (last hidden states [S,C,E],
+    keys [L,T,C,Hkv,Dh], values)."""
+    params = {n: t.double() for n, t in params.items()}
+    steps, c, e = embeds.shape
+    nh, g = cfg["n_head"], cfg["n_head_kv"]
+    dh = e // nh
+    at = torch.arange(c, device=embeds.device)
+    dist = c - 1 - (at[:, None] - at[None]).abs()
+    keys, values = ([[] for _ in range(cfg["n_layer"])] for _ in range(2))
+    out = []
+
+    def heads(x):
+        return x.repeat_interleave(nh // g, -2)                  # the kv head of each query head
+    for s in range(steps):
+        h = embeds[s].double()
+        for i in range(cfg["n_layer"]):
+            p = _block_params(params, i)
+
+            def attend(q, k, v):
+                for held, new in ((keys, k), (values, v)):
+                    held[i] = (held[i] + [new.view(c, g, dh)])[-max_steps:]
+                t = len(keys[i])
+                u, vb, z, kt, kc = _tables64(p, cfg, e, params["positional_embedding.weight"][max_steps - t:max_steps],
+                                             params["channel_embedding.weight"][:c])
+                q = q.view(c, nh, dh)
+                content = torch.einsum("qhd,tkhd->hqtk", q + heads(u), heads(torch.stack(keys[i])))
+                time = torch.einsum("qhd,thd->hqt", q + heads(vb), heads(kt.transpose(0, 1)))
+                chan = torch.einsum("qhd,khd->hqk", q + heads(z), heads(kc.transpose(0, 1)))
+                chan = chan.gather(2, dist.expand(nh, c, c))
+                w = ((content + time[..., None] + chan[:, :, None]) / math.sqrt(dh)).flatten(2).softmax(-1)
+                return torch.einsum("hqn,nhd->qhd", w, heads(torch.stack(values[i])).flatten(0, 1)).reshape(c, e)
+            h = _block64(h, p, cfg, attend)
+        out.append(_rmsnorm64(h, params["ln_f.weight"], cfg.get("layer_norm_epsilon", 1e-5)))
+    return torch.stack(out), *(torch.stack([torch.stack(held) for held in kv]) for kv in (keys, values))

@@ -350,3 +350,53 @@ def test_mvpformer_forward_matches_module_composition(masked):
             h = a + blk.mlp(blk.ln_2(a))
         seq = model.ln_f(h)
     assert (seq - want).abs().max().item() > 1e-2
+
+
+# --------------------------------------------------------------------------------------
+# the stack in 64 bits (stack_forward, stream_steps)
+# --------------------------------------------------------------------------------------
+
+def _stack64(n_layer, n_positions, C):
+    cfg = dict(n_embd=24, n_inner=40, n_layer=n_layer, n_head=6, n_head_kv=2, n_positions=n_positions,
+               n_channels=C + 2, layer_norm_epsilon=1e-5)
+    model = _StackByModules(cfg, 97).double()
+    with torch.no_grad():
+        for name, p in model.named_parameters():
+            if ".ln_" in name or name.startswith("ln_f"):
+                p.copy_(1.0 + 0.3 * torch.randn_like(p))
+            else:
+                p.copy_(torch.randn_like(p) * (0.2 if p.dim() == 1 else 1.5 / math.sqrt(p.shape[1])))
+    params = {n[len("mvpformer."):]: t for n, t in _oracle_params(model).items() if n.startswith("mvpformer.")}
+    return model, params, cfg
+
+
+def _oracle_heads(params, rows):
+    """params with the position rows `rows` in front: what a window whose positions end elsewhere uses."""
+    return dict(params, **{"positional_embedding.weight": params["positional_embedding.weight"][rows]})
+
+
+def test_stack_forward_is_mvpformer_forward():
+    torch.manual_seed(11)
+    model, params, cfg = _stack64(2, 9, 4)
+    valid = torch.tensor([[1, 1, 0, 1], [0, 1, 1, 1]], dtype=torch.bool)
+    x = torch.randn(2, 6, 4, 97, dtype=torch.float64)
+    am = valid[:, None, :].expand(2, 6, 4).reshape(2, 24).double()
+    for kw, mask in ((None, None), (valid, am)):
+        want, emb = O.mvpformer_forward(x, _oracle_params(model), cfg, attention_mask=mask)
+        got = O.stack_forward(emb, params, cfg, chan_valid=kw)
+        assert (got - want).abs().max().item() <= 2e-4          # the former's norms compute in fp32
+
+
+@pytest.mark.parametrize("n_layer,steps,max_steps", [(3, 12, 12), (1, 20, 15)])
+def test_stream_steps_are_last_rows_of_windows(n_layer, steps, max_steps):
+    """While the content window holds every segment (12), and with one block at any length, a step is the
+    last row of the window it closes, positions ending at max_steps."""
+    torch.manual_seed(12)
+    _, params, cfg = _stack64(n_layer, max_steps + 3, 3)
+    x = torch.randn(steps, 3, 24, dtype=torch.float64)
+    got, keys, values = O.stream_steps(x, params, cfg, max_steps)
+    assert keys.shape == values.shape == (n_layer, min(steps, max_steps), 3, 2, 4)
+    for s in range(steps):
+        t = min(s + 1, max_steps)
+        want = O.stack_forward(x[None, s + 1 - t:s + 1], _oracle_heads(params, slice(max_steps - t, max_steps)), cfg)[0, -1]
+        assert (got[s] - want).abs().max().item() <= 1e-10
