@@ -7,6 +7,7 @@
 // Functions return an int status where the library refused, for the Python layer to raise on.
 #include <ATen/ATen.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/util/accumulate.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/grad_mode.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -255,7 +256,7 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   if (!(x.dim() == 2 && x.stride(1) == 1)) x = x.contiguous();
-  const int64_t M = x.numel() / K, ldx = x.dim() == 2 ? x.stride(0) : K;
+  const int64_t M = c10::multiply_integers(x.sizes().slice(0, x.dim() - 1)), ldx = x.dim() == 2 ? x.stride(0) : K;
   Tensor y = at::empty(shape, x.options());
   int st;
   if (M <= 128 && K >= 1536 && N <= 4096) {

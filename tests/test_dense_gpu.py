@@ -119,6 +119,15 @@ def test_two_products_of_one_launch_refuse_small_shapes():
         mvpa_hip.linear_dual(x, w, w)
 
 
+@pytest.mark.parametrize("shape", [(4, 0), (2, 3, 0), (0, 64), (2, 0, 64)], ids=str)
+def test_linear_refuses_empty_products(shape):
+    """No columns to sum over, or no rows: an error of the library, whatever the number of dimensions."""
+    x = torch.empty(shape, dtype=torch.bfloat16, device="cuda")
+    w = torch.empty((16, shape[-1]), dtype=torch.bfloat16, device="cuda")
+    with pytest.raises((AssertionError, mvpa_hip.MvpaError)):
+        mvpa_hip.linear(x, w)
+
+
 def test_linear_into_a_column_slice():
     """The gated product written into a column slice of a wider buffer (the block's tail operand)."""
     g = torch.Generator().manual_seed(9)
