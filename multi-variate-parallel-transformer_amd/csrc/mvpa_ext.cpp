@@ -51,6 +51,12 @@ Tensor as_operand(const Tensor& t, at::ScalarType dt) {
   return t.to(dt).contiguous();
 }
 
+// false, with an AssertionError set, where a shape is refused
+bool require(bool ok, const char* what) {
+  if (!ok) PyErr_SetString(PyExc_AssertionError, what);
+  return ok;
+}
+
 // ---- the attention operator -----------------------------------------------------------------
 // forward(q, k, v, u, vb, z, k_time, k_chan, out, chan_valid, key_bias, sm_scale, window, flags,
 //         kernel, return_lse) -> out | (out, lse) | status
@@ -65,10 +71,6 @@ PyObject* py_forward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   const Tensor &kt0 = tensor_of(args[6]), &kc0 = tensor_of(args[7]);
   TORCH_CHECK(kt0.dim() >= 2 && kc0.dim() >= 2, "k_time and k_chan are [.., T, Dh] and [.., C, Dh]");
   const int64_t rows = kt0.size(-2) * kc0.size(-2), hkv = k.size(1), dh = q.size(3);
-  auto require = [](bool ok, const char* what) {
-    if (!ok) PyErr_SetString(PyExc_AssertionError, what);
-    return ok;
-  };
   if (!require(k.size(3) == dh && v.size(3) == dh, "head dims of q, k, v differ") ||
       !require(k.size(2) == rows && v.size(2) == rows, "k and v must hold T*C rows") ||
       !require(q.size(2) == rows, "q must hold T*C rows (C with last_step_only)") ||
@@ -252,7 +254,7 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_CHECK_TYPE(x.scalar_type() == at::kBFloat16 && w.scalar_type() == at::kBFloat16, "linear: bf16 only");
   at::AutoDispatchBelowADInplaceOrView guard;
   const int64_t K = x.size(-1), N = w.size(0);
-  TORCH_CHECK(w.dim() == 2 && w.size(1) == K && w.stride(1) == 1, "linear: w is [N, K] with unit last stride");
+  if (!require(w.dim() == 2 && w.size(1) == K && w.stride(1) == 1, "linear: w is [N, K] with unit last stride")) return nullptr;
   std::vector<int64_t> shape(x.sizes().begin(), x.sizes().end());
   shape.back() = N;
   if (!(x.dim() == 2 && x.stride(1) == 1)) x = x.contiguous();

@@ -128,6 +128,15 @@ def test_linear_refuses_empty_products(shape):
         mvpa_hip.linear(x, w)
 
 
+def test_linear_refuses_other_weights():
+    """A weight of another width or one that is not row-major is an AssertionError, with every way to call."""
+    x, w = (torch.zeros(n, 64, dtype=torch.bfloat16, device="cuda") for n in (8, 16))
+    for other in (w[:, :56], w.view(64, 16).t()):
+        for kw in ({}, dict(split_k=False), dict(gated=True)):
+            with pytest.raises(AssertionError):
+                mvpa_hip.linear(x, other, **kw)
+
+
 def test_linear_into_a_column_slice():
     """The gated product written into a column slice of a wider buffer (the block's tail operand)."""
     g = torch.Generator().manual_seed(9)
