@@ -124,7 +124,7 @@ def test_plan_follows_the_weights():
     assert torch.equal(out(), seen[-1])
 
 
-@pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560])
+@pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560, 15930, 15931, 16384])    # the longest in one pass, and beyond
 @pytest.mark.parametrize("M", [1, 5])
 def test_encoder_in_one_pass(L, M):
     """Analysis, norm and rounding in one kernel against the two kernels: the same fp32 formula, summed
