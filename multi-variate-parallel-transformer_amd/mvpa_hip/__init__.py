@@ -558,7 +558,9 @@ def mean_rows(x: torch.Tensor) -> torch.Tensor:
 def wavedec_db4_rmsnorm(x: torch.Tensor, weight: torch.Tensor, pitch: int, eps: float = 1e-5) -> torch.Tensor:
     """RMSNorm of the db4 coefficients of x [M, L] in bf16, [M, pitch] with zeros past the coefficients:
     wavedec_db4 and rmsnorm, in one pass where a row fits the LDS (up to about 15 900 samples)."""
-    levels, total = _dwt_shape(x.shape[-1])
+    _, length = x.shape
+    levels, total = _dwt_shape(length)
+    assert weight.numel() == total, "wavedec_db4_rmsnorm: one weight per coefficient"
     y = (_ext or load_ext()).encode(x, _as_f32_weight(weight), levels, total, pitch, eps)
     if type(y) is int and y == ERR_UNSUPPORTED:          # rows too long for the one pass: coefficients through memory
         coeffs = wavedec_db4(x, pitch=pitch, zero_pad=False)

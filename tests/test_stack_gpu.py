@@ -140,6 +140,15 @@ def test_encoder_in_one_pass(L, M):
     assert ((got[:, :total] - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
 
 
+def test_encoder_refuses_other_shapes():
+    """Rows in more than two dimensions (also where their sizes agree) and a weight of another length."""
+    w = torch.ones(mvpa_hip._dwt_shape(512)[1], device="cuda")
+    with pytest.raises(ValueError):
+        mvpa_hip.wavedec_db4_rmsnorm(torch.zeros(2, 512, 512, device="cuda"), w, 576)
+    with pytest.raises(AssertionError):
+        mvpa_hip.wavedec_db4_rmsnorm(torch.zeros(2, 512, device="cuda"), w[:-1], 576)
+
+
 def test_mean_rows():
     x = torch.randn(3, 77, 136, device="cuda").bfloat16()
     got = mvpa_hip.mean_rows(x[:, 5:]).float()
