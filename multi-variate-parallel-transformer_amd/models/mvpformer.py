@@ -312,6 +312,19 @@ class MVPFormerModel(nn.Module):
         self._plan_key = None
         self.apply(self._init_weights)
 
+    # A plan points at this object's operands: it stays behind when the model is copied, pickled or
+    # replicated, and a file of a model that had none loads
+    def __getstate__(self):
+        return {**self.__dict__, "_plan": None, "_plan_key": None}
+
+    def __setstate__(self, state):
+        super().__setstate__({"_plan": None, "_plan_key": None, **state})
+
+    def _replicate_for_data_parallel(self):
+        replica = super()._replicate_for_data_parallel()
+        replica._plan = replica._plan_key = None
+        return replica
+
     def _init_weights(self, module):
         std = self.config.initializer_range                      # models/mvpformer.py:179-188
         if isinstance(module, (nn.Linear, nn.Embedding)):

@@ -1,6 +1,8 @@
 """The stack of blocks as one library call (small-tile products, caches written by their epilogue) against
 the same blocks one by one, and the one-pass encoder against its separate kernels, at the sizes where
 tiles, splits and rows end."""
+import copy
+
 import pytest
 import torch
 
@@ -122,6 +124,18 @@ def test_plan_follows_the_weights():
     for a, b in zip(seen, seen[1:]):
         assert not torch.equal(a, b)
     assert torch.equal(out(), seen[-1])
+
+
+def test_a_used_model_is_copied():
+    """A copy of a model that has run is a model of its own: same results, and its own weights."""
+    model = _model()
+    x = torch.randn(1, 3, 8, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        first = model(inputs_embeds=x)
+        other = copy.deepcopy(model)
+        assert torch.equal(other(inputs_embeds=x), first)
+        other.h[0].mlp.down_proj.weight.mul_(2.0)
+        assert not torch.equal(other(inputs_embeds=x), first) and torch.equal(model(inputs_embeds=x), first)
 
 
 @pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560, 15930, 15931, 16384])    # the longest in one pass, and beyond

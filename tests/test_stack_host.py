@@ -1,0 +1,56 @@
+"""What the stack keeps between calls, as far as it shows without a GPU: copies, files, replicas."""
+import copy
+import ctypes
+import io
+import pickle
+
+import pytest
+import torch
+
+from models.mvpformer import MVPFormerConfig, MVPFormerModel
+
+
+def _model(**kw):
+    torch.manual_seed(0)
+    dims = dict(n_positions=8, n_channels=6, n_embd=64, n_layer=2, n_head=2, n_head_kv=1, n_inner=64)
+    dims.update(kw)
+    return MVPFormerModel(MVPFormerConfig(**dims)).eval()
+
+
+def _capsule():
+    """What a plan is to Python: an opaque pointer that neither copies nor pickles."""
+    new = ctypes.pythonapi.PyCapsule_New
+    new.restype, new.argtypes = ctypes.py_object, (ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p)
+    return new(1, None, None)
+
+
+def _through_file(model):
+    buf = io.BytesIO()
+    torch.save(model, buf)
+    buf.seek(0)
+    return torch.load(buf, weights_only=False)
+
+
+@pytest.mark.parametrize("how", [copy.copy, copy.deepcopy, lambda m: pickle.loads(pickle.dumps(m)), _through_file],
+                         ids=["copy", "deepcopy", "pickle", "save"])
+def test_a_model_with_a_plan_is_copied(how):
+    model = _model()
+    model._plan, model._plan_key = _capsule(), (1, 2, 3, True)
+    other = how(model)
+    assert other._plan is None and other._plan_key is None and model._plan is not None
+    assert all(torch.equal(a, b) for a, b in zip(model.state_dict().values(), other.state_dict().values()))
+
+
+def test_a_model_saved_without_plans_loads():
+    model = _model()
+    state = {n: v for n, v in model.__getstate__().items() if not n.startswith("_plan")}
+    other = MVPFormerModel.__new__(MVPFormerModel)
+    other.__setstate__(state)
+    assert other._plan is None and other._plan_key is None
+
+
+def test_a_replica_has_no_plan():
+    model = _model()
+    model._plan, model._plan_key = _capsule(), (1, 2, 3, True)
+    replica = model._replicate_for_data_parallel()
+    assert replica._plan is None and replica._plan_key is None and model._plan is not None
