@@ -365,17 +365,21 @@ PyObject* py_silu_gate(PyObject*, PyObject* const* args, Py_ssize_t n) {
 }
 
 // ---- the stack of blocks ----------------------------------------------------------------------
-// What a model's weights looked like when a plan was made from them: entries of modules' parameter and
-// sub-module tables (identity), and the storages and versions of the tensors found there.
+// What a model looked like when a plan was made from it: entries of modules' parameter and sub-module tables
+// (identity), the storages and versions of the tensors found there, and the sizes of the tables that grow
+// when a method is replaced on an object or a hook is registered.
 struct Watch {
   struct Entry { PyObject *dict, *key, *value; };
   std::vector<Entry> entries;
   std::vector<Tensor> tensors;
   std::vector<std::pair<const void*, uint32_t>> seen;
+  std::vector<std::pair<PyObject*, Py_ssize_t>> sized;
 
   bool unchanged() const {
     for (const auto& e : entries)
       if (PyDict_GetItem(e.dict, e.key) != e.value) return false;
+    for (const auto& [dict, n] : sized)
+      if (PyDict_Size(dict) != n) return false;
     for (size_t i = 0; i < tensors.size(); ++i)
       if (tensors[i].const_data_ptr() != seen[i].first || tensors[i]._version() != (int64_t)seen[i].second) return false;
     return true;
@@ -386,6 +390,7 @@ struct Watch {
       Py_DECREF(e.key);
       Py_DECREF(e.value);
     }
+    for (auto& [dict, n] : sized) Py_DECREF(dict);
   }
 };
 
@@ -403,12 +408,13 @@ Plan* plan_of(PyObject* o) { return (Plan*)PyCapsule_GetPointer(o, kPlanName); }
 
 void free_plan(PyObject* o) { delete plan_of(o); }
 
-// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks, watched entries, watched tensors)
+// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks, watched entries, watched tensors,
+//      dicts watched by their size)
 //   a block: (w_qkv, w_gu, w_qkv_normed|None, w_gu_normed|None, w_tail, ln_weight, u, vb, z, k_time, k_chan,
 //             ln_eps, sm_scale, flags, window, honours_mask)
 PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK(n == 6, "plan takes 6 arguments");
+  TORCH_CHECK(n == 7, "plan takes 7 arguments");
   auto plan = std::make_unique<Plan>();
   mvpa_stack_args& a = plan->args;
   std::memset(&a, 0, sizeof(a));
@@ -452,6 +458,12 @@ PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
     const Tensor& t = tensor_of(PyList_GetItem(args[5], i));
     plan->watch.tensors.push_back(t);
     plan->watch.seen.emplace_back(t.const_data_ptr(), (uint32_t)t._version());
+  }
+  for (Py_ssize_t i = 0; i < PyList_Size(args[6]); ++i) {
+    PyObject* d = PyList_GetItem(args[6], i);
+    TORCH_CHECK(PyDict_Check(d), "plan: a dict");
+    Py_INCREF(d);
+    plan->watch.sized.emplace_back(d, PyDict_Size(d));
   }
   if (PyErr_Occurred()) return nullptr;
   a.n_blocks = (int32_t)nb;

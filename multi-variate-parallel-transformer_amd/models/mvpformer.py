@@ -12,6 +12,7 @@ parameter as they do through models/mvpformer.py:132-147 and layers/mvpa.py:280-
 """
 from __future__ import annotations
 
+import functools
 from typing import Optional
 
 import torch
@@ -80,10 +81,29 @@ class MVPFormerConfig:
         return cls(**doc["model"]["init_args"]["gpt_config"]["init_args"])
 
 
+_GLOBAL_HOOKS = tuple(getattr(torch.nn.modules.module, f"_global_{n}_hooks")
+                      for n in ("forward", "forward_pre", "backward", "backward_pre"))
+
+
+@functools.lru_cache(maxsize=None)
+def _class_names(cls: type) -> frozenset:
+    return frozenset(dir(cls))
+
+
+def _as_built(module: nn.Module, *kinds: type) -> bool:
+    """One of the given classes itself, with no method of it replaced on the object."""
+    return type(module) in kinds and _class_names(type(module)).isdisjoint(module.__dict__)
+
+
+def _plain(module: nn.Module, *kinds: type) -> bool:
+    """_as_built, and with nobody watching its calls: it may be computed without calling it."""
+    return _as_built(module, *kinds) and not (module._forward_hooks or module._forward_pre_hooks)
+
+
 def _unhooked(norm: nn.Module) -> bool:
-    """A plain RMSNorm whose call nobody watches or replaces: its weight may be used without calling it."""
-    return (type(norm) is RMSNorm and "forward" not in norm.__dict__
-            and not (norm._forward_hooks or norm._forward_pre_hooks or norm._backward_hooks or norm._backward_pre_hooks))
+    """A plain RMSNorm whose call nobody watches or replaces, backward included: its weight may be used
+    without calling it."""
+    return _plain(norm, RMSNorm) and not (norm._backward_hooks or norm._backward_pre_hooks or any(_GLOBAL_HOOKS))
 
 
 class GatedMLP(nn.Module):
@@ -395,8 +415,9 @@ class MVPFormerModel(nn.Module):
 
     def _native_plan(self, t_len, c_len, pos_lo, normed):
         """The operands of every block for the library's stack call, collected once per shape and kept
-        until a weight changes (its tensor, storage or version).  normed: with the weights that carry
-        ln_1 in their columns.  None where a block is not what that call computes."""
+        until a weight changes (its tensor, storage or version), a module is replaced, or somebody hooks
+        into a module that would not be called.  normed: with the weights that carry ln_1 in their columns.
+        None where a block is not what that call computes."""
         key = (t_len, c_len, pos_lo, normed)
         ext = mvpa_hip.load_ext()
         if self._plan_key == key and self._plan is not None and ext.plan_current(self._plan):
@@ -405,6 +426,12 @@ class MVPFormerModel(nn.Module):
         first = self.h[0].attn
         inner = self.h[0].mlp.down_proj.in_features
         bf16, entries, tensors = torch.bfloat16, [], []
+        sized = list(_GLOBAL_HOOKS[:2])          # tables of hooks and of a module's own attributes: by their sizes
+        if any(sized) or not _plain(self.ln_f, RMSNorm):
+            return None
+
+        def uncalled(module):
+            sized.extend((module.__dict__, module._forward_hooks, module._forward_pre_hooks))
 
         def watch(module, *names):
             for name in names:
@@ -418,18 +445,22 @@ class MVPFormerModel(nn.Module):
         for m in (self.ln_f, self.positional_embedding, self.channel_embedding):
             watch(m, "weight")
         watch(self.ln_f, "eps")
+        uncalled(self.ln_f)
         pos = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
         chan = self.channel_embedding.weight[:c_len][None]
         blocks = []
         for name, blk in self.h._modules.items():
             attn, mlp = blk.attn, blk.mlp
-            if (type(blk) is not MVPFormerBlock or type(mlp) is not GatedMLP
-                    or type(attn) not in (MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
+            if (not _as_built(blk, MVPFormerBlock) or not _plain(mlp, GatedMLP) or not _plain(blk.ln_1, RMSNorm)
+                    or not _plain(attn, MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
                     or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != (first.num_heads, first.num_kv_heads, first.head_dim)
                     or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != bf16):
                 return None
             watch(self.h, name)
             watch(blk, "ln_1", "attn", "mlp")
+            sized.append(blk.__dict__)
+            for m in (blk.ln_1, attn, mlp):
+                uncalled(m)
             watch(blk.ln_1, "weight", "eps")
             watch(attn, "q_attn", "c_attn", "c_proj", "position_net", "channel_net", "attn_bias", "fp8_qk", "global_att",
                   "scale_attn_weights", "scale_attn_by_inverse_layer_idx", "layer_idx")
@@ -446,7 +477,7 @@ class MVPFormerModel(nn.Module):
                            mvpa_hip._as_f32_weight(blk.ln_1.weight), u, vb, z, k_time.to(bf16), k_chan.to(bf16),
                            float(blk.ln_1.eps), attn._scale(), flags, 10, attn._honours_masks))
         self._plan = ext.plan((t_len, c_len, first.num_heads, first.num_kv_heads, first.head_dim, self.embed_dim, inner),
-                              mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks, entries, tensors)
+                              mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks, entries, tensors, sized)
         self._plan_key = key
         return self._plan
 

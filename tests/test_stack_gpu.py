@@ -126,6 +126,51 @@ def test_plan_follows_the_weights():
     assert torch.equal(out(), seen[-1])
 
 
+WATCHED = {"ln_f": lambda m: m.ln_f, "attn": lambda m: m.h[1].attn, "mlp": lambda m: m.h[0].mlp, "ln_1": lambda m: m.h[0].ln_1}
+
+
+@pytest.mark.parametrize("name,C,T", [("ln_f", 64, 8), ("attn", 13, 5), ("mlp", 13, 5), ("ln_1", 13, 5), ("attn", 13, 0),
+                                      ("mlp", 13, 0)], ids=str)
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "global", "replaced"])
+def test_watched_modules_are_called(name, C, T, how):
+    """Whoever hooks into a module that the blocks one by one call, or replaces its forward, is heard: the hook
+    runs, its output counts, and the stack call comes back when it is gone.  (T = 0: a step on caches.)"""
+    model = _model()
+    module = WATCHED[name](model)
+    caches = model.new_cache(1, C, max_steps=4)
+    x = torch.randn(1, max(T, 1), C, 128, device="cuda").bfloat16()
+
+    def out():
+        with torch.no_grad():
+            if T:
+                return model(inputs_embeds=x)
+            for c in caches:
+                c.reset()
+            return model(inputs_embeds=x, past_key_values=caches)[0]
+    before, heard = out(), []
+
+    def louder(result):
+        heard.append(1)
+        return (result[0] * 2, *result[1:]) if isinstance(result, tuple) else result * 2
+    if how == "hook":
+        handle = module.register_forward_hook(lambda m, i, o: louder(o))
+    elif how == "pre-hook":
+        handle = module.register_forward_pre_hook(lambda m, i: (louder(i[0]), *i[1:]))
+    elif how == "global":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda m, i, o: louder(o) if m is module else None)
+    else:
+        plain = module.forward
+        module.forward = lambda *a, **kw: louder(plain(*a, **kw))
+    try:
+        changed = out()
+    finally:
+        handle.remove() if how != "replaced" else module.__dict__.pop("forward")
+    # twice the rows into a norm are the same rows out of it
+    assert heard and (_rel(changed, before) <= REL) == (name.startswith("ln") and how == "pre-hook")
+    n = len(heard)
+    assert torch.equal(out(), before) and len(heard) == n
+
+
 def test_a_used_model_is_copied():
     """A copy of a model that has run is a model of its own: same results, and its own weights."""
     model = _model()
