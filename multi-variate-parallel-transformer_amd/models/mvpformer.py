@@ -295,7 +295,7 @@ class MVPFormerBlock(nn.Module):
         outputs = attn_outputs[1:]
         mlp_output = self.mlp(normed)
         next_normed = None
-        if next_norm is not None and residual.dtype == torch.bfloat16:
+        if next_norm is not None and residual.dtype == torch.bfloat16 and _plain(next_norm, RMSNorm):
             hidden_states, next_normed = mvpa_hip.add3_rmsnorm(residual, mlp_output, attn_output,
                                                                next_norm.weight, next_norm.eps)
         else:
@@ -430,6 +430,10 @@ class MVPFormerModel(nn.Module):
         if any(sized) or not _plain(self.ln_f, RMSNorm):
             return None
 
+        def own(*modules):
+            """Weights that are the modules' own parameters, not computed on each access (parametrizations)."""
+            return all(isinstance(m._parameters.get("weight"), torch.Tensor) for m in modules)
+
         def uncalled(module):
             sized.extend((module.__dict__, module._forward_hooks, module._forward_pre_hooks))
 
@@ -441,6 +445,8 @@ class MVPFormerModel(nn.Module):
                 if isinstance(table[name], torch.Tensor):
                     tensors.append(table[name])
 
+        if not own(self.ln_f, self.positional_embedding, self.channel_embedding):
+            return None
         watch(self, "h", "ln_f", "positional_embedding", "channel_embedding")
         for m in (self.ln_f, self.positional_embedding, self.channel_embedding):
             watch(m, "weight")
@@ -456,6 +462,10 @@ class MVPFormerModel(nn.Module):
                     or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != (first.num_heads, first.num_kv_heads, first.head_dim)
                     or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != bf16):
                 return None
+            weights = (attn.q_attn, attn.c_attn, attn.c_proj, attn.position_net, attn.channel_net, mlp.gate_proj,
+                       mlp.up_proj, mlp.down_proj)
+            if not own(blk.ln_1, *weights) or "attn_bias" not in attn._parameters:
+                return None
             watch(self.h, name)
             watch(blk, "ln_1", "attn", "mlp")
             sized.append(blk.__dict__)
@@ -465,8 +475,7 @@ class MVPFormerModel(nn.Module):
             watch(attn, "q_attn", "c_attn", "c_proj", "position_net", "channel_net", "attn_bias", "fp8_qk", "global_att",
                   "scale_attn_weights", "scale_attn_by_inverse_layer_idx", "layer_idx")
             watch(mlp, "gate_proj", "up_proj", "down_proj")
-            for m in (attn.q_attn, attn.c_attn, attn.c_proj, attn.position_net, attn.channel_net, mlp.gate_proj,
-                      mlp.up_proj, mlp.down_proj):
+            for m in weights:
                 watch(m, *m._parameters)
             k_time, k_chan = attn._key_tables(pos, chan)
             bias = attn.attn_bias.detach().to(bf16).contiguous()
@@ -570,7 +579,8 @@ class MVPFormerModel(nn.Module):
         presents = () if use_cache else None
         rows = bsz * t_len * c_len
         if (n_layers > 0 and past_key_values is None and not torch.is_grad_enabled() and hidden_states.is_cuda
-                and hidden_states.dtype == torch.bfloat16 and self.h[0].norm_fused_supported(rows)):
+                and hidden_states.dtype == torch.bfloat16 and self.h[0].norm_fused_supported(rows)
+                and all(_plain(blk.ln_1, RMSNorm) for blk in self.h)):
             # every ln_1 inside the products around it: the statistics of a block's input come out of
             # the previous block's tail product (of one small pass for the first block)
             e = self.embed_dim

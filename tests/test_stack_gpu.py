@@ -5,6 +5,7 @@ import copy
 
 import pytest
 import torch
+import torch.nn.utils.parametrize
 
 import mvpa_hip
 from models.configs import MVPFORMER_S
@@ -169,6 +170,38 @@ def test_watched_modules_are_called(name, C, T, how):
     assert heard and (_rel(changed, before) <= REL) == (name.startswith("ln") and how == "pre-hook")
     n = len(heard)
     assert torch.equal(out(), before) and len(heard) == n
+
+
+@pytest.mark.parametrize("C,T", [(64, 8), (13, 5), (13, 0)], ids=["rows512", "rows65", "step"])
+def test_other_norms_are_called(C, T):
+    """Norms of another class are computed as what they are, on many rows, on few and on a step."""
+    model = _model()
+    model.ln_f, model.h[1].ln_1 = (torch.nn.LayerNorm(128, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    for norm in (model.ln_f, model.h[1].ln_1):
+        torch.nn.init.normal_(norm.bias)
+    x = torch.randn(1, max(T, 1), C, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = model(inputs_embeds=x) if T else model(inputs_embeds=x, past_key_values=model.new_cache(1, C, max_steps=1))[0]
+        h, pos, chan = x, model.positional_embedding.weight[:max(T, 1)][None], model.channel_embedding.weight[:C][None]
+        for blk in model.h:
+            n = blk.ln_1(h)
+            h = h + blk.mlp(n) + blk.attn(n, pos, chan)[0]
+        assert _rel(got, model.ln_f(h)) <= REL
+
+
+def test_weights_that_are_computed():
+    """An embedding whose rows are computed on access is no operand to keep: the blocks go one by one."""
+    class Twice(torch.nn.Module):
+        def forward(self, w):
+            return 2 * w
+    model = _model()
+    x = torch.randn(1, 3, 8, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        plain = model(inputs_embeds=x)
+        torch.nn.utils.parametrize.register_parametrization(model.channel_embedding, "weight", Twice())
+        twice = model(inputs_embeds=x)
+        model.channel_embedding.parametrizations.weight.original.mul_(0.5)
+        assert not torch.equal(twice, plain) and _rel(model(inputs_embeds=x), plain) <= REL
 
 
 def test_a_used_model_is_copied():
