@@ -478,38 +478,55 @@ PyObject* py_plan_current(PyObject*, PyObject* o) {
   return PyBool_FromLong(p->watch.unchanged());
 }
 
-// run(plan, x [B, T|1, C, E] bf16 contiguous, chan_valid [B,C]|None, caches|None, ring_head|None, sumsq|None)
-//   caches, one step: (k tensors, v tensors, first live steps), the tensors [B,Hkv,steps,C,Dh] contiguous;
-//   returns the normed output, shaped like x | status
-PyObject* py_run(PyObject*, PyObject* const* args, Py_ssize_t n) {
+// One pass over the blocks of a plan: its arguments, checked, and every buffer it needs.
+struct Run {
+  std::vector<Tensor> keep;
+  std::vector<mvpa_stack_block> blocks;
+  mvpa_stack_args args;
+  Tensor y;
+  PyObject* plan;
+  ~Run() { Py_XDECREF(plan); }
+};
+
+const char* kRunName = "mvpa_stack_run";
+
+// begin(plan, x [B, T|1, C, E] bf16 contiguous, chan_valid [B,C]|None, caches|None, ring_head|None, sumsq|None)
+//   caches, one step: (k tensors, v tensors, first live steps), the tensors [B,Hkv,steps,C,Dh] contiguous.
+//   Checks and allocates; nothing is enqueued.  Returns the pass | status
+PyObject* py_begin(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK(n == 6, "run takes 6 arguments");
-  Plan* p = plan_of(args[0]);
+  TORCH_CHECK(n == 6, "begin takes 6 arguments");
+  const Plan* p = plan_of(args[0]);
   if (!p) return nullptr;
   at::AutoDispatchBelowADInplaceOrView guard;
-  const Tensor x = as_operand(tensor_of(args[1]), at::kBFloat16);
-  mvpa_stack_args& a = p->args;
-  TORCH_CHECK(x.dim() == 4 && x.size(3) == a.E && x.size(2) == a.C, "run: x is [B, T, C, E]");
+  auto run = std::make_unique<Run>();
+  run->args = p->args;
+  run->blocks = p->blocks;
+  run->plan = Py_NewRef(args[0]);
+  mvpa_stack_args& a = run->args;
+  a.blocks = run->blocks.data();
+  auto held = [&](const Tensor& t) -> const Tensor& { return run->keep.emplace_back(t); };
+  const Tensor& x0 = tensor_of(args[1]);
+  run->keep.reserve(5 + 2 * run->blocks.size());
+  const Tensor& x = held(as_operand(x0, at::kBFloat16));
+  TORCH_CHECK(x.dim() == 4 && x.size(3) == a.E && x.size(2) == a.C, "begin: x is [B, T, C, E]");
   a.B = (int32_t)x.size(0);
   a.step = is_none(args[3]) ? 0 : 1;
-  TORCH_CHECK(x.size(1) == (a.step ? 1 : a.T), "run: x and the plan disagree on T");
-  Tensor cv;
-  if (!is_none(args[2])) cv = as_operand(tensor_of(args[2]), at::kBool);
-  for (size_t i = 0; i < p->blocks.size(); ++i)
-    p->blocks[i].chan_valid = cv.defined() && p->honours_mask[i] ? (const uint8_t*)cv.const_data_ptr() : nullptr;
-  a.ring_head = nullptr;
+  TORCH_CHECK(x.size(1) == (a.step ? 1 : a.T), "begin: x and the plan disagree on T");
+  const uint8_t* valid = is_none(args[2]) ? nullptr : (const uint8_t*)held(as_operand(tensor_of(args[2]), at::kBool)).const_data_ptr();
+  for (size_t i = 0; i < run->blocks.size(); ++i) run->blocks[i].chan_valid = p->honours_mask[i] ? valid : nullptr;
   if (a.step) {
     PyObject *ks = PyTuple_GetItem(args[3], 0), *vs = PyTuple_GetItem(args[3], 1), *st = PyTuple_GetItem(args[3], 2);
-    TORCH_CHECK(ks && vs && st && PyList_Size(ks) == (Py_ssize_t)p->blocks.size(), "run: one cache per block");
-    for (size_t i = 0; i < p->blocks.size(); ++i) {
-      const Tensor &k = tensor_of(PyList_GetItem(ks, i)), &v = tensor_of(PyList_GetItem(vs, i));
+    TORCH_CHECK(ks && vs && st && PyList_Size(ks) == (Py_ssize_t)run->blocks.size(), "begin: one cache per block");
+    for (size_t i = 0; i < run->blocks.size(); ++i) {
+      const Tensor &k = held(tensor_of(PyList_GetItem(ks, i))), &v = held(tensor_of(PyList_GetItem(vs, i)));
       const int64_t first = PyLong_AsLong(PyList_GetItem(st, i));
-      TORCH_CHECK(k.dim() == 5 && k.sizes() == v.sizes() && k.is_contiguous() && v.is_contiguous() &&
+      TORCH_CHECK(k.dim() == 5 && k.sizes() == v.sizes() && k.is_cuda() && v.is_cuda() && k.is_contiguous() && v.is_contiguous() &&
                       k.scalar_type() == at::kBFloat16 && v.scalar_type() == at::kBFloat16 && k.size(0) == a.B &&
                       k.size(1) == a.Hkv && k.size(3) == a.C && k.size(4) == a.Dh && first >= 0 &&
                       first + a.T <= k.size(2),
-                  "run: caches are contiguous bf16 [B, Hkv, steps, C, Dh] with room for the step");
-      mvpa_stack_block& b = p->blocks[i];
+                  "begin: caches are contiguous bf16 [B, Hkv, steps, C, Dh] with room for the step");
+      mvpa_stack_block& b = run->blocks[i];
       const int64_t slot = (int64_t)a.C * a.Dh;
       b.k_cache = (char*)k.data_ptr() + first * slot * 2;
       b.v_cache = (char*)v.data_ptr() + first * slot * 2;
@@ -517,28 +534,37 @@ PyObject* py_run(PyObject*, PyObject* const* args, Py_ssize_t n) {
       b.cache_stride_g = k.stride(1);
     }
     if (!is_none(args[4])) {
-      const Tensor& h = tensor_of(args[4]);
-      TORCH_CHECK(h.is_cuda() && h.scalar_type() == at::kInt && h.numel() == 1, "run: ring_head is one int32 on the GPU");
+      const Tensor& h = held(tensor_of(args[4]));
+      TORCH_CHECK(h.is_cuda() && h.scalar_type() == at::kInt && h.numel() == 1, "begin: ring_head is one int32 on the GPU");
       a.ring_head = (const int32_t*)h.data_ptr();
     }
   }
-  a.sumsq = nullptr;
   if (!is_none(args[5])) {
-    const Tensor& ss = tensor_of(args[5]);
+    const Tensor& ss = held(tensor_of(args[5]));
     TORCH_CHECK(ss.is_cuda() && ss.scalar_type() == at::kFloat && ss.is_contiguous() && ss.numel() * a.E == x.numel(),
-                "run: sumsq holds one fp32 value per row");
+                "begin: sumsq holds one fp32 value per row");
     a.sumsq = (const float*)ss.data_ptr();
   }
-  Tensor y = at::empty(x.sizes(), x.options());
+  if (PyErr_Occurred()) return nullptr;
   const int64_t bytes = (int64_t)mvpa_stack_ws_bytes(&a);
   if (bytes == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
-  Tensor ws = at::empty({bytes}, x.options().dtype(at::kByte));
+  run->y = at::empty(x.sizes(), x.options());
+  const Tensor& ws = held(at::empty({bytes}, x.options().dtype(at::kByte)));
   a.x = x.data_ptr();
-  a.y = y.data_ptr();
+  a.y = run->y.data_ptr();
   a.ws = ws.data_ptr();
   a.ws_bytes = (size_t)bytes;
-  const int status = mvpa_stack_forward(&a, current_stream());
-  return status == MVPA_OK ? THPVariable_Wrap(y) : PyLong_FromLong(status);
+  return PyCapsule_New(run.release(), kRunName, [](PyObject* o) { delete (Run*)PyCapsule_GetPointer(o, kRunName); });
+  END_HANDLE_TH_ERRORS
+}
+
+// enqueue(pass) -> the normed output, shaped like x | status
+PyObject* py_enqueue(PyObject*, PyObject* o) {
+  HANDLE_TH_ERRORS
+  Run* run = (Run*)PyCapsule_GetPointer(o, kRunName);
+  if (!run) return nullptr;
+  const int status = mvpa_stack_forward(&run->args, current_stream());
+  return status == MVPA_OK ? THPVariable_Wrap(run->y) : PyLong_FromLong(status);
   END_HANDLE_TH_ERRORS
 }
 
@@ -552,7 +578,8 @@ PyMethodDef kMethods[] = {
     {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
     {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
     {"plan_current", (PyCFunction)py_plan_current, METH_O, "whether the weights a plan was made from are unchanged"},
-    {"run", (PyCFunction)(void*)py_run, METH_FASTCALL, "a stack of blocks on one plan"},
+    {"begin", (PyCFunction)(void*)py_begin, METH_FASTCALL, "a pass over a plan's blocks, checked"},
+    {"enqueue", (PyCFunction)py_enqueue, METH_O, "launch a pass"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_mvpa_ext", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -48,27 +48,36 @@ class MvpaKVCache:
         self.start = 0            # first live time step in the buffers
         self.length = 0           # live time steps
 
-    def advance(self) -> int:
+    def _live(self) -> Tuple[int, int]:
+        """First slot and number of the steps that stay live beside a new one: the oldest leaves a full window."""
+        full = self.length == self.max_steps
+        return self.start + full, self.length - full
+
+    def next_slot(self) -> int:
+        """The slot of the step that comes next, after make_room().  Changes nothing."""
+        first, live = self._live()
+        return live if first + live == self.capacity else first + live
+
+    def make_room(self) -> int:
         """Room for one more time step: the oldest leaves a full window, live steps move back to the front
-        of a full buffer.  Returns the slot that the new step's keys and values belong in; the step
-        counts as live from here on."""
-        if self.length == self.max_steps:                 # the oldest step leaves the window
-            self.start += 1
-            self.length -= 1
-        if self.start + self.length == self.capacity:     # out of room: live steps back to the front
-            live_k = self.k[:, :, self.start:self.start + self.length].clone()
-            live_v = self.v[:, :, self.start:self.start + self.length].clone()
-            self.k[:, :, :self.length] = live_k
-            self.v[:, :, :self.length] = live_v
-            self.start = 0
-        self.length += 1
-        return self.start + self.length - 1
+        of a full buffer.  Returns the slot that the new step's keys and values belong in; whoever writes them
+        counts the step (`length`) afterwards."""
+        first, live = self._live()
+        if first + live == self.capacity:                 # out of room: live steps back to the front
+            live_k = self.k[:, :, first:first + live].clone()
+            live_v = self.v[:, :, first:first + live].clone()
+            self.k[:, :, :live] = live_k
+            self.v[:, :, :live] = live_v
+            first = 0
+        self.start, self.length = first, live
+        return first + live
 
     def append(self, k_new: torch.Tensor, v_new: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor]:
         """Add one time step ([B,Hkv,C,Dh] each); returns views [B,Hkv,T,C,Dh] of the live steps."""
-        pos = self.advance()
+        pos = self.make_room()
         self.k[:, :, pos] = k_new
         self.v[:, :, pos] = v_new
+        self.length += 1
         return self.views()
 
     def views(self) -> Tuple[torch.Tensor, torch.Tensor]:

@@ -523,11 +523,19 @@ class MVPFormerModel(nn.Module):
         if plan is None:
             return None
         if past_key_values is not None:
-            first = [0 if head is not None else c.advance() - (t_len - 1) for c in past_key_values]
+            first = [0 if head is not None else c.next_slot() - (t_len - 1) for c in past_key_values]
             caches = ([c.k for c in past_key_values], [c.v for c in past_key_values], first)
         elif normed:
             sumsq = mvpa_hip.row_sumsq(hidden_states.reshape(rows, e))
-        return mvpa_hip._taken(mvpa_hip.load_ext().run(plan, hidden_states, valid, caches, head, sumsq))
+        ext = mvpa_hip.load_ext()
+        run = mvpa_hip._taken(ext.begin(plan, hidden_states, valid, caches, head, sumsq))
+        grown = past_key_values if caches is not None and head is None else ()
+        for c in grown:                     # only now: what begin() refuses leaves the caches as they were
+            c.make_room()
+        out = mvpa_hip._taken(ext.enqueue(run))
+        for c in grown:
+            c.length += 1
+        return out
 
     def _forward(self, past_key_values, inputs_embeds, attention_mask, use_cache, position_end,
                  channel_validity):

@@ -100,6 +100,26 @@ def test_step_error_against_64_bits(monkeypatch, C, W, steps):
     assert (a <= 1.05 * b).all() and (a <= 2e-2).all()
 
 
+@pytest.mark.parametrize("steps", [3, 5, 9])            # a window that fills, a full one, a full buffer
+def test_a_refused_step_leaves_the_caches(steps):
+    model = _model()
+    xs = torch.randn(steps + 3, 1, 1, 5, 128, device="cuda").bfloat16()
+    two, one = model.new_cache(1, 5, max_steps=4), model.new_cache(1, 5, max_steps=4)
+    assert two[0].capacity == 5
+    with torch.no_grad():
+        for i, x in enumerate(xs):
+            if i >= steps:
+                held = [(c.start, c.length, c.k.clone(), c.v.clone()) for c in two]
+                with pytest.raises((RuntimeError, ValueError)):
+                    model(inputs_embeds=x.expand(2, -1, -1, -1).contiguous(), past_key_values=two)
+                for c, (start, length, k, v) in zip(two, held):
+                    first = slice(start, start + length)
+                    assert (c.start, c.length) == (start, length)
+                    assert torch.equal(c.k[:, :, first], k[:, :, first]) and torch.equal(c.v[:, :, first], v[:, :, first])
+            a, b = (model(inputs_embeds=x, past_key_values=c)[0] for c in (two, one))
+            assert torch.equal(a, b)
+
+
 def test_plan_follows_the_weights():
     """A changed weight - in place, by a new storage, by a new parameter, by a new sub-module - is seen."""
     model = _model()

@@ -7,6 +7,7 @@ import pickle
 import pytest
 import torch
 
+from layers import MvpaKVCache
 from models.mvpformer import MVPFormerConfig, MVPFormerModel
 
 
@@ -54,3 +55,21 @@ def test_a_replica_has_no_plan():
     model._plan, model._plan_key = _capsule(), (1, 2, 3, True)
     replica = model._replicate_for_data_parallel()
     assert replica._plan is None and replica._plan_key is None and model._plan is not None
+
+
+@pytest.mark.parametrize("max_steps,slack", [(1, 0), (3, 0), (3, 1), (4, 2)])
+def test_a_cache_counts_a_step_once_it_is_written(max_steps, slack):
+    """next_slot() names make_room()'s slot and changes nothing; a step that is never counted costs a full
+    window its oldest step and nothing else, however often it is tried."""
+    cache = MvpaKVCache(1, 1, 1, 4, max_steps, dtype=torch.float32, device="cpu", slack=slack)
+    held = []
+    for step in range(4 * max_steps + 7):
+        before = (cache.start, cache.length, cache.k.clone())
+        slot = cache.next_slot()
+        assert (cache.start, cache.length) == before[:2] and torch.equal(cache.k, before[2])
+        for _ in range(1 + step % 2):                                 # tried again where a step did not come about
+            assert cache.make_room() == cache.next_slot() == slot
+            assert cache.views()[0][0, 0, :, 0, 0].tolist() == held[max(0, len(held) - max_steps + 1):]
+        cache.append(*(torch.full((1, 1, 1, 4), float(step)) for _ in range(2)))
+        held = (held + [float(step)])[-max_steps:]
+        assert cache.views()[0][0, 0, :, 0, 0].tolist() == held
