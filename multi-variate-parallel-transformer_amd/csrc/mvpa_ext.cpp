@@ -513,8 +513,12 @@ PyObject* py_begin(PyObject*, PyObject* const* args, Py_ssize_t n) {
   a.B = (int32_t)x.size(0);
   a.step = is_none(args[3]) ? 0 : 1;
   TORCH_CHECK(x.size(1) == (a.step ? 1 : a.T), "begin: x and the plan disagree on T");
-  const uint8_t* valid = is_none(args[2]) ? nullptr : (const uint8_t*)held(as_operand(tensor_of(args[2]), at::kBool)).const_data_ptr();
-  for (size_t i = 0; i < run->blocks.size(); ++i) run->blocks[i].chan_valid = p->honours_mask[i] ? valid : nullptr;
+  if (!is_none(args[2]) && std::count(p->honours_mask.begin(), p->honours_mask.end(), 1)) {
+    const Tensor& cv = held(as_operand(tensor_of(args[2]), at::kBool));
+    if (!require(cv.dim() == 2 && cv.size(0) == a.B && cv.size(1) == a.C, "chan_valid is [B, C]")) return nullptr;
+    for (size_t i = 0; i < run->blocks.size(); ++i)
+      if (p->honours_mask[i]) run->blocks[i].chan_valid = (const uint8_t*)cv.const_data_ptr();
+  }
   if (a.step) {
     PyObject *ks = PyTuple_GetItem(args[3], 0), *vs = PyTuple_GetItem(args[3], 1), *st = PyTuple_GetItem(args[3], 2);
     TORCH_CHECK(ks && vs && st && PyList_Size(ks) == (Py_ssize_t)run->blocks.size(), "begin: one cache per block");

@@ -20,11 +20,11 @@ pytestmark = pytest.mark.gpu
 REL = 1e-2
 
 
-def _model(**kw):
+def _model(flash=True, **kw):
     torch.manual_seed(3)
     dims = dict(n_positions=40, n_channels=128, n_embd=128, n_layer=2, n_head=2, n_head_kv=1, n_inner=192)
     dims.update(kw)
-    model = MVPFormerModel(MVPFormerConfig(**dims)).to(device="cuda", dtype=torch.bfloat16).eval()
+    model = MVPFormerModel(MVPFormerConfig(**dims), flash=flash).to(device="cuda", dtype=torch.bfloat16).eval()
     for n, p in model.named_parameters():
         p.data.copy_(1.0 + 0.2 * torch.randn_like(p)) if "ln" in n else p.data.mul_(3.0)
     return model
@@ -118,6 +118,19 @@ def test_a_refused_step_leaves_the_caches(steps):
                     assert torch.equal(c.k[:, :, first], k[:, :, first]) and torch.equal(c.v[:, :, first], v[:, :, first])
             a, b = (model(inputs_embeds=x, past_key_values=c)[0] for c in (two, one))
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(1, 7), (2, 6), (2, 8), (14,)], ids=str)
+def test_validity_of_another_shape_is_refused(shape):
+    """The class that honours masks reads B x C bytes of it; the flash class none, whatever the shape."""
+    x = torch.randn(2, 3, 7, 128, device="cuda").bfloat16()
+    valid = torch.ones(shape, dtype=torch.bool, device="cuda")
+    with torch.no_grad():
+        model = _model(flash=False)
+        with pytest.raises(AssertionError):
+            model(inputs_embeds=x, channel_validity=valid)
+        flash = _model()
+        assert torch.equal(flash(inputs_embeds=x, channel_validity=valid), flash(inputs_embeds=x))
 
 
 def test_plan_follows_the_weights():
