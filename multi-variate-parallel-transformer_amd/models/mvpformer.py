@@ -717,7 +717,8 @@ class HMVPFormer(BrainModel):
         classify_step returned once max_steps segments were in (MvpaKVCache per block);
         segment_like a tensor shaped like one segment batch [B, ch, len].  Returns a callable
         step(segment) -> logits that copies the segment into a fixed buffer and replays the graph
-        of one classify_step on ring caches (the caches are copied; `past` is left alone).  The
+        of one classify_step on ring caches (the caches are copied; `past` is left alone).  The graph
+        reads the weights as they were captured, and step keeps those alive.  The
         returned logits tensor is overwritten by the next call.  predict=True captures predict_step
         instead (`past` as predict_step returned it): step(segment) -> (similarity, prediction),
         the similarity scoring the forecast of the call before."""
@@ -765,8 +766,19 @@ class HMVPFormer(BrainModel):
             graph.replay()
             return logits
 
-        step.rings, step.graph = rings, graph
+        step.rings, step.graph, step.operands = rings, graph, self._operands()
         return step
+
+    def _operands(self) -> list:
+        """What a step reads besides its caches, for whoever replays it: the parameters' storages, what the
+        modules derived from them, and the plan.  A replay finds them where they were whatever the model
+        does meanwhile (another shape, a new weight, none of which it follows)."""
+        held = [self.mvpformer._plan, getattr(self.encoder, "_proj_padded", None)]
+        held += [p.detach() for p in self.parameters()]
+        held += [mvpa_hip._as_f32_weight(m.weight) for m in self.modules() if isinstance(m, RMSNorm)]
+        for blk in self.mvpformer.h:
+            held += [blk.attn._fused_w, blk.attn._tables, blk.mlp._gu, blk._tail_w]
+        return held
 
     def _first_step(self, embeds, caches):
         """The first segment of a stream through the full forward; its keys and values seed the

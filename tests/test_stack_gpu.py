@@ -9,7 +9,8 @@ import torch.nn.utils.parametrize
 
 import mvpa_hip
 from models.configs import MVPFORMER_S
-from models.mvpformer import MVPFormerConfig, MVPFormerModel
+from models.fftencoder import WaveEncoder
+from models.mvpformer import HMVPFormer, MVPFormerConfig, MVPFormerHead, MVPFormerModel
 from oracle import mvpa_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -235,6 +236,37 @@ def test_weights_that_are_computed():
         twice = model(inputs_embeds=x)
         model.channel_embedding.parametrizations.weight.original.mul_(0.5)
         assert not torch.equal(twice, plain) and _rel(model(inputs_embeds=x), plain) <= REL
+
+
+def test_a_captured_step_keeps_what_it_reads():
+    """A replay after the model has scored other shapes and got other weights, with what it may have freed
+    meanwhile allocated again and overwritten, is the replay of before."""
+    torch.manual_seed(4)
+    cfg = MVPFormerConfig(n_positions=6, n_channels=16, n_embd=128, n_layer=2, n_head=2, n_head_kv=1, n_inner=192)
+    model = HMVPFormer(cfg, WaveEncoder(100, 128), MVPFormerHead(128, 2)).to("cuda", torch.bfloat16).eval()
+    xs = torch.randn(12, 1, 5, 100, device="cuda")
+    past = None
+    for x in xs[:6]:
+        _, past = model.classify_step(x, past)
+    results = []
+    for meanwhile in (False, True):
+        step = model.capture_stream(past, xs[6])
+        if meanwhile:
+            with torch.no_grad():
+                for c, t in ((3, 6), (16, 4), (9, 2)) * 4:
+                    model.classify(torch.randn(1, t, c, 100, device="cuda"))
+                model.encoder.ln.weight.mul_(3.0)
+                for p in model.parameters():
+                    p.data = p.data * 2.0
+                model.classify(torch.randn(1, 5, 4, 100, device="cuda"))
+            dirt = [torch.full((n,), float("nan"), device="cuda") for n in (64, 1 << 10, 1 << 14, 1 << 18) for _ in range(64)]
+        out = []
+        for x in xs[6:]:
+            out.append(step(x).clone())
+            torch.cuda.synchronize()
+        results.append(out)
+    del dirt
+    assert all(torch.equal(a, b) for a, b in zip(*results))
 
 
 def test_a_used_model_is_copied():
