@@ -62,6 +62,7 @@ def test_a_cache_counts_a_step_once_it_is_written(max_steps, slack):
     """next_slot() names make_room()'s slot and changes nothing; a step that is never counted costs a full
     window its oldest step and nothing else, however often it is tried."""
     cache = MvpaKVCache(1, 1, 1, 4, max_steps, dtype=torch.float32, device="cpu", slack=slack)
+    cache.k.zero_()                                                   # so that it can be compared with itself
     held = []
     for step in range(4 * max_steps + 7):
         before = (cache.start, cache.length, cache.k.clone())
