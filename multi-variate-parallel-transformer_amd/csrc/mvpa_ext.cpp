@@ -394,8 +394,39 @@ struct Watch {
   }
 };
 
+const char* kWatchName = "mvpa_stack_watch";
+
+// watch(entries (dict, key, value), tensors, dicts watched by their size)
+PyObject* py_watch(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 3, "watch takes 3 arguments");
+  auto watch = std::make_unique<Watch>();
+  for (Py_ssize_t i = 0; i < PyList_Size(args[0]); ++i) {
+    PyObject* t = PyList_GetItem(args[0], i);
+    TORCH_CHECK(PyTuple_Check(t) && PyTuple_Size(t) == 3 && PyDict_Check(PyTuple_GetItem(t, 0)), "watch: (dict, key, value)");
+    watch->entries.push_back({Py_NewRef(PyTuple_GetItem(t, 0)), Py_NewRef(PyTuple_GetItem(t, 1)), Py_NewRef(PyTuple_GetItem(t, 2))});
+  }
+  for (Py_ssize_t i = 0; i < PyList_Size(args[1]); ++i) {
+    const Tensor& t = tensor_of(PyList_GetItem(args[1], i));
+    watch->tensors.push_back(t);
+    watch->seen.emplace_back(t.const_data_ptr(), (uint32_t)t._version());
+  }
+  for (Py_ssize_t i = 0; i < PyList_Size(args[2]); ++i) {
+    PyObject* d = PyList_GetItem(args[2], i);
+    TORCH_CHECK(PyDict_Check(d), "watch: a dict");
+    watch->sized.emplace_back(Py_NewRef(d), PyDict_Size(d));
+  }
+  if (PyErr_Occurred()) return nullptr;
+  return PyCapsule_New(watch.release(), kWatchName, [](PyObject* o) { delete (Watch*)PyCapsule_GetPointer(o, kWatchName); });
+  END_HANDLE_TH_ERRORS
+}
+
+PyObject* py_watch_current(PyObject*, PyObject* o) {
+  const Watch* w = (const Watch*)PyCapsule_GetPointer(o, kWatchName);
+  return w ? PyBool_FromLong(w->unchanged()) : nullptr;
+}
+
 struct Plan {
-  Watch watch;
   std::vector<Tensor> keep;                  // every operand, alive as long as the plan
   std::vector<mvpa_stack_block> blocks;
   std::vector<char> honours_mask;
@@ -408,13 +439,12 @@ Plan* plan_of(PyObject* o) { return (Plan*)PyCapsule_GetPointer(o, kPlanName); }
 
 void free_plan(PyObject* o) { delete plan_of(o); }
 
-// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks, watched entries, watched tensors,
-//      dicts watched by their size)
+// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks)
 //   a block: (w_qkv, w_gu, w_qkv_normed|None, w_gu_normed|None, w_tail, ln_weight, u, vb, z, k_time, k_chan,
 //             ln_eps, sm_scale, flags, window, honours_mask)
 PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK(n == 7, "plan takes 7 arguments");
+  TORCH_CHECK(n == 4, "plan takes 4 arguments");
   auto plan = std::make_unique<Plan>();
   mvpa_stack_args& a = plan->args;
   std::memset(&a, 0, sizeof(a));
@@ -446,36 +476,11 @@ PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
     plan->honours_mask.push_back(PyTuple_GetItem(t, 15) == Py_True);
     plan->blocks.push_back(b);
   }
-  for (Py_ssize_t i = 0; i < PyList_Size(args[4]); ++i) {
-    PyObject* t = PyList_GetItem(args[4], i);
-    Watch::Entry e{PyTuple_GetItem(t, 0), PyTuple_GetItem(t, 1), PyTuple_GetItem(t, 2)};
-    Py_INCREF(e.dict);
-    Py_INCREF(e.key);
-    Py_INCREF(e.value);
-    plan->watch.entries.push_back(e);
-  }
-  for (Py_ssize_t i = 0; i < PyList_Size(args[5]); ++i) {
-    const Tensor& t = tensor_of(PyList_GetItem(args[5], i));
-    plan->watch.tensors.push_back(t);
-    plan->watch.seen.emplace_back(t.const_data_ptr(), (uint32_t)t._version());
-  }
-  for (Py_ssize_t i = 0; i < PyList_Size(args[6]); ++i) {
-    PyObject* d = PyList_GetItem(args[6], i);
-    TORCH_CHECK(PyDict_Check(d), "plan: a dict");
-    Py_INCREF(d);
-    plan->watch.sized.emplace_back(d, PyDict_Size(d));
-  }
   if (PyErr_Occurred()) return nullptr;
   a.n_blocks = (int32_t)nb;
   a.blocks = plan->blocks.data();
   return PyCapsule_New(plan.release(), kPlanName, free_plan);
   END_HANDLE_TH_ERRORS
-}
-
-PyObject* py_plan_current(PyObject*, PyObject* o) {
-  Plan* p = plan_of(o);
-  if (!p) return nullptr;
-  return PyBool_FromLong(p->watch.unchanged());
 }
 
 // One pass over the blocks of a plan: its arguments, checked, and every buffer it needs.
@@ -581,7 +586,8 @@ PyMethodDef kMethods[] = {
     {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},
     {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
     {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
-    {"plan_current", (PyCFunction)py_plan_current, METH_O, "whether the weights a plan was made from are unchanged"},
+    {"watch", (PyCFunction)(void*)py_watch, METH_FASTCALL, "what a model looks like now"},
+    {"watch_current", (PyCFunction)py_watch_current, METH_O, "whether it still looks like that"},
     {"begin", (PyCFunction)(void*)py_begin, METH_FASTCALL, "a pass over a plan's blocks, checked"},
     {"enqueue", (PyCFunction)py_enqueue, METH_O, "launch a pass"},
     {nullptr, nullptr, 0, nullptr}};

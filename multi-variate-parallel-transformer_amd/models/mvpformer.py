@@ -12,6 +12,7 @@ parameter as they do through models/mvpformer.py:132-147 and layers/mvpa.py:280-
 """
 from __future__ import annotations
 
+import collections
 import functools
 from typing import Optional
 
@@ -309,6 +310,20 @@ class MVPFormerBlock(nn.Module):
         return outputs, next_normed
 
 
+class _StackOperands:
+    """What the library's stack call was given of a model, as long as `watch` finds the model unchanged.
+
+    weights: the operands of each block that no shape enters, {with ln_1 in the columns: [tuple per block]};
+    plans: the last SHAPES shapes in use, the one used last at the end - the bias tables of each (24 blocks of
+    the base model at 128 channels and 512 positions: 31 MB) beside the weights they share.  A recording's
+    shape, those of a few others and of a stream beside them stay; a stream that fills its window passes through."""
+
+    SHAPES = 8
+
+    def __init__(self, watch):
+        self.watch, self.weights, self.plans = watch, {}, collections.OrderedDict()
+
+
 class MVPFormerModel(nn.Module):
     """models/mvpformer.py:155-402 without the HF base class: h, ln_f, positional_embedding,
     channel_embedding; forward(inputs_embeds=[B,T,C,E]) -> last_hidden_state [B,T,C,E]."""
@@ -328,21 +343,20 @@ class MVPFormerModel(nn.Module):
         self.positional_embedding = nn.Embedding(config.max_position_embeddings, self.embed_dim)
         self.channel_embedding = nn.Embedding(config.max_channel_embeddings, self.embed_dim)
         self.gradient_checkpointing = gradient_checkpointing
-        self._plan = None                # operands of the native stack, see _native_plan
-        self._plan_key = None
+        self._stack = None               # operands of the native stack, see _native_plan
         self.apply(self._init_weights)
 
-    # A plan points at this object's operands: it stays behind when the model is copied, pickled or
+    # Plans point at this object's operands: they stay behind when the model is copied, pickled or
     # replicated, and a file of a model that had none loads
     def __getstate__(self):
-        return {**self.__dict__, "_plan": None, "_plan_key": None}
+        return {**self.__dict__, "_stack": None}
 
     def __setstate__(self, state):
-        super().__setstate__({"_plan": None, "_plan_key": None, **state})
+        super().__setstate__({"_stack": None, **state})
 
     def _replicate_for_data_parallel(self):
         replica = super()._replicate_for_data_parallel()
-        replica._plan = replica._plan_key = None
+        replica._stack = None
         return replica
 
     def _init_weights(self, module):
@@ -413,20 +427,13 @@ class MVPFormerModel(nn.Module):
         return list(zip(tables(position_embeds, [a.position_net for a in attns]),
                         tables(channel_embeds, [a.channel_net for a in attns])))
 
-    def _native_plan(self, t_len, c_len, pos_lo, normed):
-        """The operands of every block for the library's stack call, collected once per shape and kept
-        until a weight changes (its tensor, storage or version), a module is replaced, or somebody hooks
-        into a module that would not be called.  normed: with the weights that carry ln_1 in their columns.
-        None where a block is not what that call computes."""
-        key = (t_len, c_len, pos_lo, normed)
-        ext = mvpa_hip.load_ext()
-        if self._plan_key == key and self._plan is not None and ext.plan_current(self._plan):
-            return self._plan
-        self._plan = None
+    def _survey(self):
+        """What the stack call's operands depend on: entries of the modules' tables (by identity), tensors (by
+        storage and version), and the tables of hooks and of a module's own attributes (by their sizes).  None
+        where a block is not what that call computes, or somebody hooks into a module that would not be called."""
         first = self.h[0].attn
         inner = self.h[0].mlp.down_proj.in_features
-        bf16, entries, tensors = torch.bfloat16, [], []
-        sized = list(_GLOBAL_HOOKS[:2])          # tables of hooks and of a module's own attributes: by their sizes
+        entries, tensors, sized = [], [], list(_GLOBAL_HOOKS[:2])
         if any(sized) or not _plain(self.ln_f, RMSNorm):
             return None
 
@@ -452,15 +459,12 @@ class MVPFormerModel(nn.Module):
             watch(m, "weight")
         watch(self.ln_f, "eps")
         uncalled(self.ln_f)
-        pos = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
-        chan = self.channel_embedding.weight[:c_len][None]
-        blocks = []
         for name, blk in self.h._modules.items():
             attn, mlp = blk.attn, blk.mlp
             if (not _as_built(blk, MVPFormerBlock) or not _plain(mlp, GatedMLP) or not _plain(blk.ln_1, RMSNorm)
                     or not _plain(attn, MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
                     or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != (first.num_heads, first.num_kv_heads, first.head_dim)
-                    or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != bf16):
+                    or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != torch.bfloat16):
                 return None
             weights = (attn.q_attn, attn.c_attn, attn.c_proj, attn.position_net, attn.channel_net, mlp.gate_proj,
                        mlp.up_proj, mlp.down_proj)
@@ -477,18 +481,52 @@ class MVPFormerModel(nn.Module):
             watch(mlp, "gate_proj", "up_proj", "down_proj")
             for m in weights:
                 watch(m, *m._parameters)
-            k_time, k_chan = attn._key_tables(pos, chan)
-            bias = attn.attn_bias.detach().to(bf16).contiguous()
-            u, vb, z = (b.contiguous() for b in bias.split(attn.embed_kv_dim))
-            wq, wg = blk._folded_weights() if normed else (None, None)
+        return entries, tensors, sized
+
+    def _native_plan(self, t_len, c_len, pos_lo, normed):
+        """The operands of every block for the library's stack call at one shape.  Those that depend on the
+        weights alone are collected once and kept until the model changes, and so are the last few shapes.
+        normed: with the weights that carry ln_1 in their columns.  None: not for that call (_survey)."""
+        ext = mvpa_hip.load_ext()
+        held = self._stack
+        if held is None or not ext.watch_current(held.watch):
+            held = self._stack = None
+            seen = self._survey()
+            if seen is None:
+                return None
+            held = self._stack = _StackOperands(ext.watch(*seen))
+        key = (t_len, c_len, pos_lo, normed)
+        plan = held.plans.pop(key, None)
+        if plan is None:
+            plan = self._make_plan(held, *key)
+        held.plans[key] = plan                   # the last used one at the end
+        while len(held.plans) > held.SHAPES:
+            held.plans.popitem(last=False)
+        return plan
+
+    def _make_plan(self, held, t_len, c_len, pos_lo, normed):
+        bf16, first = torch.bfloat16, self.h[0].attn
+        if normed not in held.weights:
+            held.weights[normed] = [self._block_operands(blk, normed) for blk in self.h]
+        pos = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
+        chan = self.channel_embedding.weight[:c_len][None]
+        blocks = []
+        for blk, weights in zip(self.h, held.weights[normed]):
+            attn = blk.attn
+            tables = (t.to(bf16) for t in attn._key_tables(pos, chan))
             flags = ((mvpa_hip.FLAG_CONTENT if attn._content() else 0) | (mvpa_hip.FLAG_FP8_QK if attn.fp8_qk else 0))
-            blocks.append((attn.qkv_weight(bf16), mlp.gate_up_weight(), wq, wg, blk._tail_weight(),
-                           mvpa_hip._as_f32_weight(blk.ln_1.weight), u, vb, z, k_time.to(bf16), k_chan.to(bf16),
-                           float(blk.ln_1.eps), attn._scale(), flags, 10, attn._honours_masks))
-        self._plan = ext.plan((t_len, c_len, first.num_heads, first.num_kv_heads, first.head_dim, self.embed_dim, inner),
-                              mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks, entries, tensors, sized)
-        self._plan_key = key
-        return self._plan
+            blocks.append((*weights, *tables, float(blk.ln_1.eps), attn._scale(), flags, 10, attn._honours_masks))
+        return mvpa_hip.load_ext().plan((t_len, c_len, first.num_heads, first.num_kv_heads, first.head_dim, self.embed_dim,
+                                         self.h[0].mlp.down_proj.in_features),
+                                        mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks)
+
+    @staticmethod
+    def _block_operands(blk, normed):
+        attn = blk.attn
+        bias = attn.attn_bias.detach().to(torch.bfloat16).contiguous()
+        wq, wg = blk._folded_weights() if normed else (None, None)
+        return (attn.qkv_weight(torch.bfloat16), blk.mlp.gate_up_weight(), wq, wg, blk._tail_weight(),
+                mvpa_hip._as_f32_weight(blk.ln_1.weight), *(b.contiguous() for b in bias.split(attn.embed_kv_dim)))
 
     def _native(self, hidden_states, past_key_values, mask, t_len, pos_lo):
         """The whole stack as one call of the library, for the whole-sequence forward and for one step
@@ -771,9 +809,10 @@ class HMVPFormer(BrainModel):
 
     def _operands(self) -> list:
         """What a step reads besides its caches, for whoever replays it: the parameters' storages, what the
-        modules derived from them, and the plan.  A replay finds them where they were whatever the model
+        modules derived from them, and the plans.  A replay finds them where they were whatever the model
         does meanwhile (another shape, a new weight, none of which it follows)."""
-        held = [self.mvpformer._plan, getattr(self.encoder, "_proj_padded", None)]
+        stack = self.mvpformer._stack
+        held = [list(stack.plans.values()) if stack else None, getattr(self.encoder, "_proj_padded", None)]
         held += [p.detach() for p in self.parameters()]
         held += [mvpa_hip._as_f32_weight(m.weight) for m in self.modules() if isinstance(m, RMSNorm)]
         for blk in self.mvpformer.h:

@@ -10,7 +10,7 @@ import torch.nn.utils.parametrize
 import mvpa_hip
 from models.configs import MVPFORMER_S
 from models.fftencoder import WaveEncoder
-from models.mvpformer import HMVPFormer, MVPFormerConfig, MVPFormerHead, MVPFormerModel
+from models.mvpformer import HMVPFormer, MVPFormerConfig, MVPFormerHead, MVPFormerModel, _StackOperands
 from oracle import mvpa_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -236,6 +236,55 @@ def test_weights_that_are_computed():
         twice = model(inputs_embeds=x)
         model.channel_embedding.parametrizations.weight.original.mul_(0.5)
         assert not torch.equal(twice, plain) and _rel(model(inputs_embeds=x), plain) <= REL
+
+
+def test_shapes_in_turn_share_weights_and_keep_their_plans(monkeypatch):
+    """Shapes in turn, a stream beside them, and a stream that fills: each shape is prepared once, the weights
+    once in all, results are those of a model that sees one shape only, and no more than SHAPES plans are held."""
+    model, made, collected = _model(), [], []
+    make, collect = MVPFormerModel._make_plan, MVPFormerModel._block_operands
+    monkeypatch.setattr(MVPFormerModel, "_make_plan", lambda self, held, *key: made.append(key) or make(self, held, *key))
+    monkeypatch.setattr(MVPFormerModel, "_block_operands", staticmethod(lambda *a: collected.append(a) or collect(*a)))
+    xs = [torch.randn(1, t, c, 128, device="cuda").bfloat16() for t, c in ((3, 8), (5, 8), (8, 64), (5, 9), (3, 8))]
+    seg = torch.randn(1, 1, 8, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        alone = [copy.deepcopy(model)(inputs_embeds=x) for x in xs]
+        caches = model.new_cache(1, 8, max_steps=2)
+        for _ in range(2):
+            model(inputs_embeds=seg, past_key_values=caches)
+        made.clear(), collected.clear()
+        model._stack.plans.clear()
+        model._stack.weights.clear()
+        for _ in range(3):
+            for x, want in zip(xs, alone):
+                assert torch.equal(model(inputs_embeds=x), want)
+                model(inputs_embeds=seg, past_key_values=caches)
+        assert len(made) == len(set(made)) == 5              # four windows and the stream
+        assert len(collected) == 2 * len(model.h)            # plain, and with ln_1 in the columns
+        caches = model.new_cache(1, 8, max_steps=20)         # every step of a filling window is a shape of its own
+        for _ in range(20):
+            model(inputs_embeds=seg, past_key_values=caches)
+            assert len(model._stack.plans) <= _StackOperands.SHAPES
+            assert torch.equal(model(inputs_embeds=xs[0]), alone[0])
+        assert made.count((3, 8, 0, False)) == 1
+
+
+def test_adapters_reach_the_stack_call():
+    """A model with adapters: their product is part of the weight, and follows them."""
+    model = _model(lora=True, lora_rank=4, lora_alpha=8)
+    x = torch.randn(1, 5, 9, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        before = model(inputs_embeds=x)
+        for blk in model.h:
+            blk.attn.q_attn.lora_B.normal_(std=0.1)
+            blk.attn.c_attn.lora_B.normal_(std=0.1)
+        got = model(inputs_embeds=x)
+        plain = copy.deepcopy(model)
+        for blk in plain.h:
+            for m in (blk.attn.q_attn, blk.attn.c_attn):
+                m.weight.copy_(m.effective_weight())
+                m.lora_B.zero_()
+        assert torch.equal(got, plain(inputs_embeds=x)) and _rel(got, before) > REL
 
 
 def test_a_captured_step_keeps_what_it_reads():

@@ -8,7 +8,7 @@ import pytest
 import torch
 
 from layers import MvpaKVCache
-from models.mvpformer import MVPFormerConfig, MVPFormerModel
+from models.mvpformer import MVPFormerConfig, MVPFormerModel, _StackOperands
 
 
 def _model(**kw):
@@ -19,7 +19,7 @@ def _model(**kw):
 
 
 def _capsule():
-    """What a plan is to Python: an opaque pointer that neither copies nor pickles."""
+    """What watch and plans are to Python: an opaque pointer that neither copies nor pickles."""
     new = ctypes.pythonapi.PyCapsule_New
     new.restype, new.argtypes = ctypes.py_object, (ctypes.c_void_p, ctypes.c_char_p, ctypes.c_void_p)
     return new(1, None, None)
@@ -36,25 +36,25 @@ def _through_file(model):
                          ids=["copy", "deepcopy", "pickle", "save"])
 def test_a_model_with_a_plan_is_copied(how):
     model = _model()
-    model._plan, model._plan_key = _capsule(), (1, 2, 3, True)
+    model._stack = _StackOperands(_capsule())
     other = how(model)
-    assert other._plan is None and other._plan_key is None and model._plan is not None
+    assert other._stack is None and model._stack is not None
     assert all(torch.equal(a, b) for a, b in zip(model.state_dict().values(), other.state_dict().values()))
 
 
 def test_a_model_saved_without_plans_loads():
     model = _model()
-    state = {n: v for n, v in model.__getstate__().items() if not n.startswith("_plan")}
+    state = {n: v for n, v in model.__getstate__().items() if n != "_stack"}
     other = MVPFormerModel.__new__(MVPFormerModel)
     other.__setstate__(state)
-    assert other._plan is None and other._plan_key is None
+    assert other._stack is None
 
 
 def test_a_replica_has_no_plan():
     model = _model()
-    model._plan, model._plan_key = _capsule(), (1, 2, 3, True)
+    model._stack = _StackOperands(_capsule())
     replica = model._replicate_for_data_parallel()
-    assert replica._plan is None and replica._plan_key is None and model._plan is not None
+    assert replica._stack is None and model._stack is not None
 
 
 @pytest.mark.parametrize("max_steps,slack", [(1, 0), (3, 0), (3, 1), (4, 2)])
