@@ -500,6 +500,11 @@ typedef struct mvpa_stack_args {
  * columns; a matrix-core attention shape); ws_bytes is 0 for those. */
 size_t mvpa_stack_ws_bytes(const mvpa_stack_args* args);
 int mvpa_stack_forward(const mvpa_stack_args* args, void* stream);
+/* Blocks [first, end) of it, for a caller that prepares the operands of one block while the launches of the
+ * one before run: the parts in order, on one stream and with the same arguments and workspace (what lies
+ * between two blocks stays there).  A part reads the operands of its own blocks and ln_weight of block `end`;
+ * of the others only whether the *_normed weights are there and the flags.  ln_f comes with the last. */
+int mvpa_stack_forward_blocks(const mvpa_stack_args* args, int32_t first, int32_t end, void* stream);
 
 #ifdef __cplusplus
 }

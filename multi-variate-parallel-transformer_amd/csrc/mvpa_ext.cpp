@@ -430,6 +430,7 @@ struct Plan {
   std::vector<Tensor> keep;                  // every operand, alive as long as the plan
   std::vector<mvpa_stack_block> blocks;
   std::vector<char> honours_mask;
+  long set = 0;                              // blocks whose operands are there
   mvpa_stack_args args;
 };
 
@@ -439,9 +440,18 @@ Plan* plan_of(PyObject* o) { return (Plan*)PyCapsule_GetPointer(o, kPlanName); }
 
 void free_plan(PyObject* o) { delete plan_of(o); }
 
-// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks)
-//   a block: (w_qkv, w_gu, w_qkv_normed|None, w_gu_normed|None, w_tail, ln_weight, u, vb, z, k_time, k_chan,
-//             ln_eps, sm_scale, flags, window, honours_mask)
+// The pointer of a plan's operand, which the plan keeps; null for None
+const void* operand(Plan* plan, PyObject* o, at::ScalarType dt) {
+  if (is_none(o)) return nullptr;
+  const Tensor& t = tensor_of(o);
+  on_gpu(t);
+  TORCH_CHECK(t.scalar_type() == dt && t.is_contiguous(), "plan: operands are contiguous and of the stack's type");
+  plan->keep.push_back(t);
+  return t.const_data_ptr();
+}
+
+// plan(dims (T, C, H, Hkv, Dh, E, inner), lnf_weight, lnf_eps, blocks): a block is what no tensor is needed for,
+//   (ln_eps, sm_scale, flags, window, honours_mask)
 PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 4, "plan takes 4 arguments");
@@ -451,35 +461,49 @@ PyObject* py_plan(PyObject*, PyObject* const* args, Py_ssize_t n) {
   a.struct_size = sizeof(a);
   int32_t* dims[7] = {&a.T, &a.C, &a.H, &a.Hkv, &a.Dh, &a.E, &a.inner};
   for (int i = 0; i < 7; ++i) *dims[i] = (int32_t)PyLong_AsLong(PyTuple_GetItem(args[0], i));
-  auto operand = [&](PyObject* o, at::ScalarType dt) -> const void* {
-    if (is_none(o)) return nullptr;
-    const Tensor& t = tensor_of(o);
-    on_gpu(t);
-    TORCH_CHECK(t.scalar_type() == dt && t.is_contiguous(), "plan: operands are contiguous and of the stack's type");
-    plan->keep.push_back(t);
-    return t.const_data_ptr();
-  };
-  a.lnf_weight = (const float*)operand(args[1], at::kFloat);
+  a.lnf_weight = (const float*)operand(plan.get(), args[1], at::kFloat);
   a.lnf_eps = (float)PyFloat_AsDouble(args[2]);
-  const Py_ssize_t nb = PyList_Size(args[3]);
-  for (Py_ssize_t i = 0; i < nb; ++i) {
+  a.n_blocks = (int32_t)PyList_Size(args[3]);
+  for (int32_t i = 0; i < a.n_blocks; ++i) {
     PyObject* t = PyList_GetItem(args[3], i);
     mvpa_stack_block b;
     std::memset(&b, 0, sizeof(b));
-    const void** ops[11] = {&b.w_qkv, &b.w_gate_up, &b.w_qkv_normed, &b.w_gate_up_normed, &b.w_tail,
-                            (const void**)&b.ln_weight, &b.bias_u, &b.bias_v, &b.bias_z, &b.k_time, &b.k_chan};
-    for (int j = 0; j < 11; ++j) *ops[j] = operand(PyTuple_GetItem(t, j), j == 5 ? at::kFloat : at::kBFloat16);
-    b.ln_eps = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 11));
-    b.sm_scale = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 12));
-    b.flags = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GetItem(t, 13));
-    b.window = (int32_t)PyLong_AsLong(PyTuple_GetItem(t, 14));
-    plan->honours_mask.push_back(PyTuple_GetItem(t, 15) == Py_True);
+    b.ln_eps = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 0));
+    b.sm_scale = (float)PyFloat_AsDouble(PyTuple_GetItem(t, 1));
+    b.flags = (uint32_t)PyLong_AsUnsignedLong(PyTuple_GetItem(t, 2));
+    b.window = (int32_t)PyLong_AsLong(PyTuple_GetItem(t, 3));
+    plan->honours_mask.push_back(PyTuple_GetItem(t, 4) == Py_True);
     plan->blocks.push_back(b);
   }
   if (PyErr_Occurred()) return nullptr;
-  a.n_blocks = (int32_t)nb;
-  a.blocks = plan->blocks.data();
   return PyCapsule_New(plan.release(), kPlanName, free_plan);
+  END_HANDLE_TH_ERRORS
+}
+
+// set_block(plan, i, (w_qkv, w_gu, w_qkv_normed|None, w_gu_normed|None, w_tail, ln_weight, u, vb, z, k_time, k_chan),
+//           ln_weight of the block behind it|None)
+//   in the order of the blocks; once block 0 is set a pass can begin(), and every block that is set be enqueued
+PyObject* py_set_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 4, "set_block takes 4 arguments");
+  Plan* p = plan_of(args[0]);
+  if (!p) return nullptr;
+  const long at = PyLong_AsLong(args[1]);
+  TORCH_CHECK(at >= 0 && at < (long)p->blocks.size() && at == p->set && PyTuple_Check(args[2]) && PyTuple_Size(args[2]) == 11,
+              "set_block: the next block's operands");
+  TORCH_CHECK(is_none(args[3]) == (at + 1 == (long)p->blocks.size()), "set_block: the norm of the block behind it");
+  mvpa_stack_block& b = p->blocks[at];
+  const void** ops[11] = {&b.w_qkv, &b.w_gate_up, &b.w_qkv_normed, &b.w_gate_up_normed, &b.w_tail,
+                          (const void**)&b.ln_weight, &b.bias_u, &b.bias_v, &b.bias_z, &b.k_time, &b.k_chan};
+  for (int j = 0; j < 11; ++j) *ops[j] = operand(p, PyTuple_GetItem(args[2], j), j == 5 ? at::kFloat : at::kBFloat16);
+  if (!is_none(args[3])) p->blocks[at + 1].ln_weight = (const float*)operand(p, args[3], at::kFloat);
+  ++p->set;
+  if (at == 0)                                // sizes are asked for before the others are set: as many weights as here
+    for (auto& other : p->blocks) {
+      other.w_qkv_normed = b.w_qkv_normed;
+      other.w_gate_up_normed = b.w_gate_up_normed;
+    }
+  Py_RETURN_NONE;
   END_HANDLE_TH_ERRORS
 }
 
@@ -489,7 +513,8 @@ struct Run {
   std::vector<mvpa_stack_block> blocks;
   mvpa_stack_args args;
   Tensor y;
-  PyObject* plan;
+  PyObject* plan = nullptr;
+  long done = 0;                             // blocks enqueued
   ~Run() { Py_XDECREF(plan); }
 };
 
@@ -567,13 +592,31 @@ PyObject* py_begin(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// enqueue(pass) -> the normed output, shaped like x | status
-PyObject* py_enqueue(PyObject*, PyObject* o) {
+// enqueue(pass, first, end): blocks [first, end), which the parts of a pass take in order -> the normed output,
+// shaped like x, with the last | None | status
+PyObject* py_enqueue(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  Run* run = (Run*)PyCapsule_GetPointer(o, kRunName);
+  TORCH_CHECK(n == 3, "enqueue takes 3 arguments");
+  Run* run = (Run*)PyCapsule_GetPointer(args[0], kRunName);
   if (!run) return nullptr;
-  const int status = mvpa_stack_forward(&run->args, current_stream());
-  return status == MVPA_OK ? THPVariable_Wrap(run->y) : PyLong_FromLong(status);
+  const Plan* p = plan_of(run->plan);
+  const long first = PyLong_AsLong(args[1]), end = PyLong_AsLong(args[2]), blocks = (long)run->blocks.size();
+  TORCH_CHECK(first == run->done && first < end && end <= blocks && end <= p->set, "enqueue: the next blocks, set");
+  for (long i = first; i < std::min(end + 1, blocks); ++i) {       // operands set since begin()
+    mvpa_stack_block b = p->blocks[i];
+    const mvpa_stack_block& own = run->blocks[i];
+    b.chan_valid = own.chan_valid;
+    b.k_cache = own.k_cache;
+    b.v_cache = own.v_cache;
+    b.cache_stride_b = own.cache_stride_b;
+    b.cache_stride_g = own.cache_stride_g;
+    run->blocks[i] = b;
+  }
+  const int status = mvpa_stack_forward_blocks(&run->args, (int32_t)first, (int32_t)end, current_stream());
+  if (status != MVPA_OK) return PyLong_FromLong(status);
+  run->done = end;
+  if (end < blocks) Py_RETURN_NONE;
+  return THPVariable_Wrap(run->y);
   END_HANDLE_TH_ERRORS
 }
 
@@ -588,8 +631,9 @@ PyMethodDef kMethods[] = {
     {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
     {"watch", (PyCFunction)(void*)py_watch, METH_FASTCALL, "what a model looks like now"},
     {"watch_current", (PyCFunction)py_watch_current, METH_O, "whether it still looks like that"},
+    {"set_block", (PyCFunction)(void*)py_set_block, METH_FASTCALL, "operands of one block"},
     {"begin", (PyCFunction)(void*)py_begin, METH_FASTCALL, "a pass over a plan's blocks, checked"},
-    {"enqueue", (PyCFunction)py_enqueue, METH_O, "launch a pass"},
+    {"enqueue", (PyCFunction)(void*)py_enqueue, METH_FASTCALL, "launch blocks of a pass"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_mvpa_ext", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -129,8 +129,13 @@ extern "C" size_t mvpa_stack_ws_bytes(const mvpa_stack_args* a) {
 }
 
 extern "C" int mvpa_stack_forward(const mvpa_stack_args* a, void* stream) {
+  return mvpa_stack_forward_blocks(a, 0, a ? a->n_blocks : 0, stream);
+}
+
+extern "C" int mvpa_stack_forward_blocks(const mvpa_stack_args* a, int32_t first, int32_t end, void* stream) {
   int st = stack_check(a);
   if (st != MVPA_OK) return st;
+  if (first < 0 || end <= first || end > a->n_blocks) return MVPA_ERR_SHAPE;
   if (!a->x || !a->y || !a->lnf_weight || !a->ws) return MVPA_ERR_NULL;
   if (((uintptr_t)a->ws & 255) || ((uintptr_t)a->x & 15) || ((uintptr_t)a->y & 15)) return MVPA_ERR_ALIGN;
   stack_plan p;
@@ -189,30 +194,28 @@ extern "C" int mvpa_stack_forward(const mvpa_stack_args* a, void* stream) {
     return mvpa_forward(&f, stream);
   };
 
-  const bf16_t* x = (const bf16_t*)a->x;
   if (p.many) {
-    const float* ss = a->sumsq;
-    int32_t parts = 1;
-    for (int i = 0; i < a->n_blocks; ++i) {
+    for (int i = first; i < end; ++i) {
       const mvpa_stack_block& blk = a->blocks[i];
+      const bf16_t* x = i ? p.hidden[(i - 1) & 1] : (const bf16_t*)a->x;
+      const float* ss = i ? p.sumsq[i & 1] : a->sumsq;
+      const int32_t parts = i ? p.parts : 1;
       if ((st = mvpa_linear_bf16_dual_normed(x, blk.w_qkv_normed, p.qkv, blk.w_gate_up_normed, p.both + E, p.rows, nw,
                                              inner, E, E, E, nw, E, wide, ss, parts, blk.ln_eps,
                                              stream)) != MVPA_OK) return st;
       if ((st = attend(blk)) != MVPA_OK) return st;
-      bf16_t* out = p.hidden[i & 1];
-      if ((st = mvpa_linear_bf16_residual_sumsq(p.both, blk.w_tail, x, out, p.sumsq[(i + 1) & 1], p.rows, E, wide, wide,
+      if ((st = mvpa_linear_bf16_residual_sumsq(p.both, blk.w_tail, x, p.hidden[i & 1], p.sumsq[(i + 1) & 1], p.rows, E, wide, wide,
                                                 wide, E, E, stream)) != MVPA_OK) return st;
-      ss = p.sumsq[(i + 1) & 1];
-      parts = p.parts;
-      x = out;
     }
-    return mvpa_rmsnorm(x, a->lnf_weight, a->y, p.rows, (int32_t)E, E, E, a->lnf_eps, MVPA_BF16, MVPA_BF16, stream);
+    if (end < a->n_blocks) return MVPA_OK;
+    return mvpa_rmsnorm(p.hidden[(end - 1) & 1], a->lnf_weight, a->y, p.rows, (int32_t)E, E, E, a->lnf_eps, MVPA_BF16, MVPA_BF16, stream);
   }
 
-  if (!p.raw && (st = mvpa_rmsnorm(x, a->blocks[0].ln_weight, p.normed, p.rows, (int32_t)E, E, E, a->blocks[0].ln_eps, MVPA_BF16,
+  if (first == 0 && !p.raw && (st = mvpa_rmsnorm(a->x, a->blocks[0].ln_weight, p.normed, p.rows, (int32_t)E, E, E, a->blocks[0].ln_eps, MVPA_BF16,
                          MVPA_BF16, stream)) != MVPA_OK) return st;
-  for (int i = 0; i < a->n_blocks; ++i) {
+  for (int i = first; i < end; ++i) {
     const mvpa_stack_block& blk = a->blocks[i];
+    const bf16_t* x = i ? p.hidden[0] : (const bf16_t*)a->x;
     tile_out out = {};
     out.y = p.qkv;
     out.ldy = a->step ? E : nw;
@@ -238,7 +241,6 @@ extern "C" int mvpa_stack_forward(const mvpa_stack_args* a, void* stream) {
     if ((st = launch_tail_reduce(p.partial, p.split_k, x, p.hidden[0], last ? (bf16_t*)a->y : p.normed,
                                  last ? a->lnf_weight : a->blocks[i + 1].ln_weight, last ? a->lnf_eps : a->blocks[i + 1].ln_eps,
                                  p.raw && !last ? p.sumsq[0] : nullptr, p.rows, E, s)) != MVPA_OK) return st;
-    x = p.hidden[0];
   }
   return MVPA_OK;
 }

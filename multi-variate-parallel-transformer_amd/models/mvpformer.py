@@ -107,6 +107,13 @@ def _unhooked(norm: nn.Module) -> bool:
     return _plain(norm, RMSNorm) and not (norm._backward_hooks or norm._backward_pre_hooks or any(_GLOBAL_HOOKS))
 
 
+def _weighted(blk) -> tuple:
+    """The modules of a block whose weights the stack call uses, without the norm."""
+    attn, mlp = blk._modules["attn"]._modules, blk._modules["mlp"]._modules
+    return (*map(attn.__getitem__, ("q_attn", "c_attn", "c_proj", "position_net", "channel_net")),
+            *map(mlp.__getitem__, ("gate_proj", "up_proj", "down_proj")))
+
+
 class GatedMLP(nn.Module):
     """down(silu(gate(x)) * up(x)), bias-free: the MLP the reference takes from the Llama family
     (models/mvpformer.py:114).  gate and up run as ONE GEMM with the SiLU-multiply fused."""
@@ -186,9 +193,9 @@ class MVPFormerBlock(nn.Module):
         wq, wg, ln = self.attn.qkv_weight(), self.mlp.gate_up_weight(), self.ln_1.weight
         key = (wq.data_ptr(), wq._version, wg.data_ptr(), wg._version, ln.data_ptr(), ln._version)
         if self._fold_key != key:
-            scale = ln.detach().float()[None, :]
-            self._fold_w = ((wq.float() * scale).to(torch.bfloat16).contiguous(),
-                            (wg.float() * scale).to(torch.bfloat16).contiguous())
+            # one pass each: the product of two bf16 values is formed in fp32 and rounded once, and a norm
+            # weight in fp32 makes the product fp32
+            self._fold_w = tuple((w * ln.detach()).to(torch.bfloat16) for w in (wq, wg))
             self._fold_key = key
         return self._fold_w
 
@@ -313,14 +320,14 @@ class MVPFormerBlock(nn.Module):
 class _StackOperands:
     """What the library's stack call was given of a model, as long as `watch` finds the model unchanged.
 
-    weights: the operands of each block that no shape enters, {with ln_1 in the columns: [tuple per block]};
+    weights: the operands of each block that no shape enters, by (block, with ln_1 in the columns or without);
     plans: the last SHAPES shapes in use, the one used last at the end - the bias tables of each (24 blocks of
     the base model at 128 channels and 512 positions: 31 MB) beside the weights they share.  A recording's
     shape, those of a few others and of a stream beside them stay; a stream that fills its window passes through."""
 
     SHAPES = 8
 
-    def __init__(self, watch):
+    def __init__(self, watch=None):
         self.watch, self.weights, self.plans = watch, {}, collections.OrderedDict()
 
 
@@ -343,7 +350,7 @@ class MVPFormerModel(nn.Module):
         self.positional_embedding = nn.Embedding(config.max_position_embeddings, self.embed_dim)
         self.channel_embedding = nn.Embedding(config.max_channel_embeddings, self.embed_dim)
         self.gradient_checkpointing = gradient_checkpointing
-        self._stack = None               # operands of the native stack, see _native_plan
+        self._stack = None               # operands of the native stack, see _native
         self.apply(self._init_weights)
 
     # Plans point at this object's operands: they stay behind when the model is copied, pickled or
@@ -427,22 +434,35 @@ class MVPFormerModel(nn.Module):
         return list(zip(tables(position_embeds, [a.position_net for a in attns]),
                         tables(channel_embeds, [a.channel_net for a in attns])))
 
+    def _stack_computes(self) -> bool:
+        """Whether the stack call computes what the modules do: every block of the plain kind, weights that are
+        the modules' own parameters and not computed on each access (parametrizations), and nobody hooked into a
+        module that would not be called."""
+        def own(module):
+            return isinstance(module._parameters.get("weight"), torch.Tensor)
+
+        first, inner = self.h[0].attn, self.h[0].mlp.down_proj.in_features
+        shape = (first.num_heads, first.num_kv_heads, first.head_dim)
+        if (_GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1] or not _plain(self.ln_f, RMSNorm)
+                or not all(map(own, (self.ln_f, self.positional_embedding, self.channel_embedding)))):
+            return False
+        for blk in self.h:                       # in front of a first pass's first launch: few attribute look-ups
+            if not _as_built(blk, MVPFormerBlock):
+                return False
+            ln, attn, mlp = map(blk._modules.get, ("ln_1", "attn", "mlp"))
+            if (not _plain(ln, RMSNorm) or not _plain(mlp, GatedMLP)
+                    or not _plain(attn, MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
+                    or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != shape
+                    or not all(map(own, (ln, *_weighted(blk)))) or "attn_bias" not in attn._parameters
+                    or mlp._modules["down_proj"].in_features != inner or ln._parameters["weight"].dtype != torch.bfloat16):
+                return False
+        return True
+
     def _survey(self):
-        """What the stack call's operands depend on: entries of the modules' tables (by identity), tensors (by
-        storage and version), and the tables of hooks and of a module's own attributes (by their sizes).  None
-        where a block is not what that call computes, or somebody hooks into a module that would not be called."""
-        first = self.h[0].attn
-        inner = self.h[0].mlp.down_proj.in_features
+        """What the stack call's operands, and _stack_computes, depend on: entries of the modules' tables (by
+        identity), tensors (by storage and version), and the tables of hooks and of a module's own attributes
+        (by their sizes)."""
         entries, tensors, sized = [], [], list(_GLOBAL_HOOKS[:2])
-        if any(sized) or not _plain(self.ln_f, RMSNorm):
-            return None
-
-        def own(*modules):
-            """Weights that are the modules' own parameters, not computed on each access (parametrizations)."""
-            return all(isinstance(m._parameters.get("weight"), torch.Tensor) for m in modules)
-
-        def uncalled(module):
-            sized.extend((module.__dict__, module._forward_hooks, module._forward_pre_hooks))
 
         def watch(module, *names):
             for name in names:
@@ -452,73 +472,48 @@ class MVPFormerModel(nn.Module):
                 if isinstance(table[name], torch.Tensor):
                     tensors.append(table[name])
 
-        if not own(self.ln_f, self.positional_embedding, self.channel_embedding):
-            return None
+        def uncalled(module):
+            sized.extend((module.__dict__, module._forward_hooks, module._forward_pre_hooks))
+
         watch(self, "h", "ln_f", "positional_embedding", "channel_embedding")
         for m in (self.ln_f, self.positional_embedding, self.channel_embedding):
             watch(m, "weight")
         watch(self.ln_f, "eps")
         uncalled(self.ln_f)
         for name, blk in self.h._modules.items():
-            attn, mlp = blk.attn, blk.mlp
-            if (not _as_built(blk, MVPFormerBlock) or not _plain(mlp, GatedMLP) or not _plain(blk.ln_1, RMSNorm)
-                    or not _plain(attn, MVPFormerGQAAttention, MVPFormerGQAFlashAttention) or attn.is_cross_attention
-                    or (attn.num_heads, attn.num_kv_heads, attn.head_dim) != (first.num_heads, first.num_kv_heads, first.head_dim)
-                    or mlp.down_proj.in_features != inner or blk.ln_1.weight.dtype != torch.bfloat16):
-                return None
-            weights = (attn.q_attn, attn.c_attn, attn.c_proj, attn.position_net, attn.channel_net, mlp.gate_proj,
-                       mlp.up_proj, mlp.down_proj)
-            if not own(blk.ln_1, *weights) or "attn_bias" not in attn._parameters:
-                return None
             watch(self.h, name)
             watch(blk, "ln_1", "attn", "mlp")
             sized.append(blk.__dict__)
-            for m in (blk.ln_1, attn, mlp):
+            for m in (blk.ln_1, blk.attn, blk.mlp):
                 uncalled(m)
             watch(blk.ln_1, "weight", "eps")
-            watch(attn, "q_attn", "c_attn", "c_proj", "position_net", "channel_net", "attn_bias", "fp8_qk", "global_att",
+            watch(blk.attn, "q_attn", "c_attn", "c_proj", "position_net", "channel_net", "attn_bias", "fp8_qk", "global_att",
                   "scale_attn_weights", "scale_attn_by_inverse_layer_idx", "layer_idx")
-            watch(mlp, "gate_proj", "up_proj", "down_proj")
-            for m in weights:
+            watch(blk.mlp, "gate_proj", "up_proj", "down_proj")
+            for m in _weighted(blk):
                 watch(m, *m._parameters)
         return entries, tensors, sized
 
-    def _native_plan(self, t_len, c_len, pos_lo, normed):
-        """The operands of every block for the library's stack call at one shape.  Those that depend on the
-        weights alone are collected once and kept until the model changes, and so are the last few shapes.
-        normed: with the weights that carry ln_1 in their columns.  None: not for that call (_survey)."""
-        ext = mvpa_hip.load_ext()
-        held = self._stack
-        if held is None or not ext.watch_current(held.watch):
-            held = self._stack = None
-            seen = self._survey()
-            if seen is None:
-                return None
-            held = self._stack = _StackOperands(ext.watch(*seen))
-        key = (t_len, c_len, pos_lo, normed)
-        plan = held.plans.pop(key, None)
-        if plan is None:
-            plan = self._make_plan(held, *key)
-        held.plans[key] = plan                   # the last used one at the end
-        while len(held.plans) > held.SHAPES:
-            held.plans.popitem(last=False)
-        return plan
-
-    def _make_plan(self, held, t_len, c_len, pos_lo, normed):
-        bf16, first = torch.bfloat16, self.h[0].attn
-        if normed not in held.weights:
-            held.weights[normed] = [self._block_operands(blk, normed) for blk in self.h]
-        pos = self.positional_embedding.weight[pos_lo:pos_lo + t_len][None]
-        chan = self.channel_embedding.weight[:c_len][None]
-        blocks = []
-        for blk, weights in zip(self.h, held.weights[normed]):
-            attn = blk.attn
-            tables = (t.to(bf16) for t in attn._key_tables(pos, chan))
-            flags = ((mvpa_hip.FLAG_CONTENT if attn._content() else 0) | (mvpa_hip.FLAG_FP8_QK if attn.fp8_qk else 0))
-            blocks.append((*weights, *tables, float(blk.ln_1.eps), attn._scale(), flags, 10, attn._honours_masks))
+    def _new_plan(self, t_len, c_len):
+        """A plan without its tensors, see _set_block."""
+        first, blocks = self.h[0].attn, []
+        for blk in self.h:
+            ln, attn = blk._modules["ln_1"], blk._modules["attn"]
+            flags = (mvpa_hip.FLAG_CONTENT if attn._content() else 0) | (mvpa_hip.FLAG_FP8_QK if attn.fp8_qk else 0)
+            blocks.append((float(ln.eps), attn._scale(), flags, 10, attn._honours_masks))
         return mvpa_hip.load_ext().plan((t_len, c_len, first.num_heads, first.num_kv_heads, first.head_dim, self.embed_dim,
                                          self.h[0].mlp.down_proj.in_features),
                                         mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks)
+
+    def _set_block(self, held, plan, i, t_len, c_len, pos_lo, normed):
+        blk, behind = self.h[i], self.h[i + 1].ln_1.weight if i + 1 < len(self.h) else None
+        weights = held.weights.get((i, normed))
+        if weights is None:
+            weights = held.weights[i, normed] = self._block_operands(blk, normed)
+        tables = blk.attn._key_tables(self.positional_embedding.weight[pos_lo:pos_lo + t_len][None],
+                                      self.channel_embedding.weight[:c_len][None])
+        mvpa_hip.load_ext().set_block(plan, i, (*weights, *(t.to(torch.bfloat16) for t in tables)),
+                                      None if behind is None else mvpa_hip._as_f32_weight(behind))
 
     @staticmethod
     def _block_operands(blk, normed):
@@ -556,23 +551,43 @@ class MVPFormerModel(nn.Module):
                 head = clock.head32
             else:
                 return None
+        ext = mvpa_hip.load_ext()
+        held = self._stack
+        if held is None or not ext.watch_current(held.watch):
+            self._stack = None
+            if not self._stack_computes():
+                return None
+            held = _StackOperands()
         normed = past_key_values is None and self.h[0].norm_fused_supported(rows)
-        plan = self._native_plan(t_len, c_len, pos_lo, normed)
-        if plan is None:
-            return None
+        key = (t_len, c_len, pos_lo, normed)
+        plan = held.plans.pop(key, None)
+        fresh = plan is None
+        if fresh:
+            plan = self._new_plan(t_len, c_len)
+            self._set_block(held, plan, 0, *key)
         if past_key_values is not None:
             first = [0 if head is not None else c.next_slot() - (t_len - 1) for c in past_key_values]
             caches = ([c.k for c in past_key_values], [c.v for c in past_key_values], first)
         elif normed:
             sumsq = mvpa_hip.row_sumsq(hidden_states.reshape(rows, e))
-        ext = mvpa_hip.load_ext()
+        blocks = len(self.h)
         run = mvpa_hip._taken(ext.begin(plan, hidden_states, valid, caches, head, sumsq))
         grown = past_key_values if caches is not None and head is None else ()
         for c in grown:                     # only now: what begin() refuses leaves the caches as they were
             c.make_room()
-        out = mvpa_hip._taken(ext.enqueue(run))
+        if fresh:                           # a block runs while the next one's operands are put together
+            for i in range(1, blocks):
+                mvpa_hip._taken(ext.enqueue(run, i - 1, i))
+                self._set_block(held, plan, i, *key)
+        out = mvpa_hip._taken(ext.enqueue(run, blocks - 1 if fresh else 0, blocks))
         for c in grown:
             c.length += 1
+        held.plans[key] = plan              # whole from here on, and the one used last
+        while len(held.plans) > held.SHAPES:
+            held.plans.popitem(last=False)
+        if held.watch is None:              # last: the GPU has its work by now
+            held.watch = ext.watch(*self._survey())
+            self._stack = held
         return out
 
     def _forward(self, past_key_values, inputs_embeds, attention_mask, use_cache, position_end,

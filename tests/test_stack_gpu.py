@@ -242,8 +242,9 @@ def test_shapes_in_turn_share_weights_and_keep_their_plans(monkeypatch):
     """Shapes in turn, a stream beside them, and a stream that fills: each shape is prepared once, the weights
     once in all, results are those of a model that sees one shape only, and no more than SHAPES plans are held."""
     model, made, collected = _model(), [], []
-    make, collect = MVPFormerModel._make_plan, MVPFormerModel._block_operands
-    monkeypatch.setattr(MVPFormerModel, "_make_plan", lambda self, held, *key: made.append(key) or make(self, held, *key))
+    put, collect = MVPFormerModel._set_block, MVPFormerModel._block_operands
+    monkeypatch.setattr(MVPFormerModel, "_set_block", lambda self, held, plan, i, *key:
+                        (made.append(key) if i == 0 else None) or put(self, held, plan, i, *key))
     monkeypatch.setattr(MVPFormerModel, "_block_operands", staticmethod(lambda *a: collected.append(a) or collect(*a)))
     xs = [torch.randn(1, t, c, 128, device="cuda").bfloat16() for t, c in ((3, 8), (5, 8), (8, 64), (5, 9), (3, 8))]
     seg = torch.randn(1, 1, 8, 128, device="cuda").bfloat16()
@@ -253,8 +254,7 @@ def test_shapes_in_turn_share_weights_and_keep_their_plans(monkeypatch):
         for _ in range(2):
             model(inputs_embeds=seg, past_key_values=caches)
         made.clear(), collected.clear()
-        model._stack.plans.clear()
-        model._stack.weights.clear()
+        model._stack = None
         for _ in range(3):
             for x, want in zip(xs, alone):
                 assert torch.equal(model(inputs_embeds=x), want)
@@ -267,6 +267,35 @@ def test_shapes_in_turn_share_weights_and_keep_their_plans(monkeypatch):
             assert len(model._stack.plans) <= _StackOperands.SHAPES
             assert torch.equal(model(inputs_embeds=xs[0]), alone[0])
         assert made.count((3, 8, 0, False)) == 1
+
+
+@pytest.mark.parametrize("B,C,T", [(1, 13, 5), (2, 37, 7), (14, 128, 4), (1, 9, 0)],
+                         ids=["rows65", "rows518", "rows7168", "step"])     # ln_1 by itself, in few rows' products, in many rows'
+def test_first_pass_is_the_later_ones(monkeypatch, B, C, T):
+    """The pass that prepares the operands block by block gives bit for bit what the next one on the whole plan
+    gives, also where a pass before was cut off between two blocks: that one leaves no plan behind."""
+    model = _model(n_layer=5, n_inner=1728)
+    x = torch.randn(B, max(T, 1), C, 128, device="cuda").bfloat16()
+
+    def out():
+        with torch.no_grad():
+            if T:
+                return model(inputs_embeds=x)
+            caches = model.new_cache(B, C, max_steps=3)
+            return [model(inputs_embeds=x, past_key_values=caches)[0] for _ in range(2)][-1]
+    put = MVPFormerModel._set_block
+
+    def breaks(self, held, plan, i, *key):
+        if i == 3:
+            raise MemoryError
+        put(self, held, plan, i, *key)
+    with monkeypatch.context() as m:
+        m.setattr(MVPFormerModel, "_set_block", breaks)
+        with pytest.raises(MemoryError):
+            out()
+    assert model._stack is None
+    first = out()
+    assert model._stack.plans and torch.equal(first, out())
 
 
 def test_adapters_reach_the_stack_call():
