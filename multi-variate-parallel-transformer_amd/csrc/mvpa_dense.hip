@@ -1,6 +1,7 @@
 // Dense ops around the attention kernel: bf16 MFMA linear (y = x w^T), RMSNorm, the
 // three-way residual add and the db4 wavelet analysis of the segment encoder.
 #include "mvpa_common.h"
+#include "mvpa_tiles.h"
 
 namespace mvpa {
 
@@ -1637,13 +1638,13 @@ __global__ __launch_bounds__(256) void mean_rows_bf16_kernel(const bf16_t* __res
   }
 }
 
-// One new time step of keys and values into the slot *head of two ring buffers
-// [B,Hkv,steps,C,Dh]: k_new / v_new are [B,Hkv,C,Dh] views (element strides sb, sh, sc, unit
-// last stride) of the projection output.  One thread per 16 bytes.
-__global__ __launch_bounds__(256) void ring_append_bf16_kernel(
-    const bf16_t* __restrict__ k_new, const bf16_t* __restrict__ v_new, bf16_t* __restrict__ k_ring,
-    bf16_t* __restrict__ v_ring, const int32_t* __restrict__ head, int Hkv, int C, int Dh, int steps,
-    int64_t sb, int64_t sh, int64_t sc, int64_t total) {
+// One new time step of keys and values into slot `slot` (or *head, where given) of two caches
+// [B][Hkv][steps][C][Dh] (element strides db, dh; a slot is C * Dh): k_new / v_new are [B,Hkv,C,Dh] views
+// (element strides sb, sh, sc, unit last stride) of the projection output.  One thread per 16 bytes.
+__global__ __launch_bounds__(256) void append_bf16_kernel(
+    const bf16_t* __restrict__ k_new, const bf16_t* __restrict__ v_new, bf16_t* __restrict__ k, bf16_t* __restrict__ v,
+    const int32_t* __restrict__ head, int slot, int Hkv, int C, int Dh, int64_t sb, int64_t sh, int64_t sc, int64_t db,
+    int64_t dh, int64_t total) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (i >= total) return;
   const int d8 = Dh / 8;
@@ -1651,11 +1652,11 @@ __global__ __launch_bounds__(256) void ring_append_bf16_kernel(
   const int c = (int)((i / d8) % C);
   const int h = (int)((i / ((int64_t)d8 * C)) % Hkv);
   const int64_t b = i / ((int64_t)d8 * C * Hkv);
-  const int slot = *head;
+  if (head) slot = *head;
   const int64_t src = b * sb + h * sh + c * sc + d;
-  const int64_t dst = (((b * Hkv + h) * steps + slot) * C + c) * Dh + d;
-  *(u32x4*)(k_ring + dst) = *(const u32x4*)(k_new + src);
-  *(u32x4*)(v_ring + dst) = *(const u32x4*)(v_new + src);
+  const int64_t dst = b * db + h * dh + ((int64_t)slot * C + c) * Dh + d;
+  *(u32x4*)(k + dst) = *(const u32x4*)(k_new + src);
+  *(u32x4*)(v + dst) = *(const u32x4*)(v_new + src);
 }
 
 // -----------------------------------------------------------------------------------------
@@ -2027,6 +2028,15 @@ extern "C" int mvpa_add3_bf16(const void* a, const void* b, const void* c, void*
   return mvpa::take_launch_status();
 }
 
+int mvpa::launch_append(const bf16_t* k_new, const bf16_t* v_new, bf16_t* k, bf16_t* v, const int32_t* head, int32_t slot,
+                        int32_t B, int32_t Hkv, int32_t C, int32_t Dh, int64_t stride_b, int64_t stride_h, int64_t stride_c,
+                        int64_t cache_stride_b, int64_t cache_stride_h, hipStream_t stream) {
+  const int64_t total = (int64_t)B * Hkv * C * (Dh / 8);
+  MVPA_LAUNCH(append_bf16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, k_new, v_new, k, v, head, slot,
+              Hkv, C, Dh, stride_b, stride_h, stride_c, cache_stride_b, cache_stride_h, total);
+  return take_launch_status();
+}
+
 extern "C" int mvpa_ring_append_bf16(const void* k_new, const void* v_new, void* k_ring, void* v_ring,
                                      const int32_t* head, int32_t B, int32_t Hkv, int32_t C, int32_t Dh,
                                      int32_t steps, int64_t stride_b, int64_t stride_h, int64_t stride_c,
@@ -2036,11 +2046,9 @@ extern "C" int mvpa_ring_append_bf16(const void* k_new, const void* v_new, void*
   if (Dh % 8 != 0 || ((stride_b | stride_h | stride_c) & 7) ||
       (((uintptr_t)k_new | (uintptr_t)v_new | (uintptr_t)k_ring | (uintptr_t)v_ring) & 15))
     return MVPA_ERR_ALIGN;
-  const int64_t total = (int64_t)B * Hkv * C * (Dh / 8);
-  MVPA_LAUNCH(ring_append_bf16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0,
-                     (hipStream_t)stream, (const bf16_t*)k_new, (const bf16_t*)v_new, (bf16_t*)k_ring,
-                     (bf16_t*)v_ring, head, Hkv, C, Dh, steps, stride_b, stride_h, stride_c, total);
-  return mvpa::take_launch_status();
+  const int64_t group = (int64_t)steps * C * Dh;
+  return mvpa::launch_append((const bf16_t*)k_new, (const bf16_t*)v_new, (bf16_t*)k_ring, (bf16_t*)v_ring, head, 0, B, Hkv, C,
+                             Dh, stride_b, stride_h, stride_c, Hkv * group, group, (hipStream_t)stream);
 }
 
 extern "C" int mvpa_add3_rmsnorm_bf16(const void* a, const void* b, const void* c,

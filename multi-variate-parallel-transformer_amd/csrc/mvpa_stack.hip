@@ -10,6 +10,8 @@
 //                  that the next block wants (mvpa_tiles.hip)
 //   a step         the latter with the new keys and values written straight into the caches by the
 //                  product's epilogue, and the attention of the last time step only
+//   a step of      norm -> [q/k/v | gate/up] on 256-row tiles -> keys and values into the caches -> attention of
+//   many rows      the last time step -> tail product with residual
 #include "mvpa_mfma_tools.h"
 #include "mvpa_tiles.h"
 
@@ -20,6 +22,13 @@ namespace mvpa {
 // 1600 / 3200 / 4096 rows 105 : 68, 126 : 130, 150 : 173; of 2048 columns at 1024 / 1536 / 2048 rows
 // 258 : 203, 313 : 295, 331 : 361).
 constexpr int64_t kManyTiles = 352;
+
+// A step's products are few-row ones up to more tiles the longer the contraction (us a step of all blocks,
+// 256-row against small tiles, window 25: MVPFormer-S, 64 channels at 3072 / 3584 / 4096 / 6144 rows = 228 /
+// 266 / 304 / 456 tiles 1966 : 1925, 2211 : 2137, 2328 : 2473, 2873 : 3623; base model, 128 channels at
+// 1280 / 1536 / 2048 / 3072 rows = 300 / 360 / 480 / 720 tiles 11138 : 10066, 11519 : 10870, 12179 : 13235,
+// 18195 : 23241; 64 channels 1536 / 2048 rows 9877 : 9256, 10374 : 11535).
+static int64_t many_step_tiles(int64_t E) { return 176 + E / 8; }
 
 static int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
@@ -35,7 +44,7 @@ struct stack_ws {
 
 struct stack_plan {
   bool many, raw;                      // 256-row tiles; ln_1 inside the products
-  int64_t rows;
+  int64_t rows, ld_qkv;
   tile_split split_k;
   int runs;
   bf16_t *qkv, *both, *hidden[2], *normed;
@@ -72,14 +81,18 @@ static void stack_layout(const mvpa_stack_args* a, stack_plan& p, stack_ws& w) {
   p.raw = !a->step && a->sumsq;
   for (int i = 0; i < a->n_blocks; ++i) p.raw = p.raw && a->blocks[i].w_qkv_normed && a->blocks[i].w_gate_up_normed;
   const int64_t tiles = (p.rows + 255) / 256 * ((inner + 127) / 128 + (E + 2 * kv + 255) / 256);
-  p.many = p.raw && p.rows >= 512 && tiles >= kManyTiles && E >= 128;
-  p.qkv = (bf16_t*)w.take(p.rows * (a->step ? E : E + 2 * kv) * 2);
+  p.many = (a->step ? tiles >= many_step_tiles(E) : p.raw && tiles >= kManyTiles) && p.rows >= 512 && E >= 128;
+  p.ld_qkv = a->step && !p.many ? E : E + 2 * kv;
+  p.qkv = (bf16_t*)w.take(p.rows * p.ld_qkv * 2);
   p.both = (bf16_t*)w.take(p.rows * (E + inner) * 2);
   p.hidden[0] = (bf16_t*)w.take(p.rows * E * 2);
   p.hidden[1] = p.normed = nullptr;
   p.sumsq[0] = p.sumsq[1] = nullptr;
   p.partial = nullptr;
-  if (p.many) {
+  if (p.many && a->step) {
+    p.hidden[1] = (bf16_t*)w.take(p.rows * E * 2);
+    p.normed = (bf16_t*)w.take(p.rows * E * 2);
+  } else if (p.many) {
     p.hidden[1] = (bf16_t*)w.take(p.rows * E * 2);
     p.parts = mvpa_linear_sumsq_parts(p.rows, E);
     for (int i = 0; i < 2; ++i) p.sumsq[i] = (float*)w.take(p.rows * p.parts * 4);
@@ -157,7 +170,7 @@ extern "C" int mvpa_stack_forward_blocks(const mvpa_stack_args* a, int32_t first
     f.B = a->B; f.H = a->H; f.Hkv = a->Hkv; f.T = a->T; f.C = a->C; f.Dh = a->Dh;
     f.window = blk.window;
     f.sm_scale = blk.sm_scale;
-    const int64_t row = a->step ? E : nw;
+    const int64_t row = p.ld_qkv;
     f.q = p.qkv;
     f.q_stride_b = n * row; f.q_stride_h = a->Dh; f.q_stride_n = row;
     if (a->step) {
@@ -194,6 +207,26 @@ extern "C" int mvpa_stack_forward_blocks(const mvpa_stack_args* a, int32_t first
     return mvpa_forward(&f, stream);
   };
 
+  if (p.many && a->step) {
+    if (first == 0 && (st = mvpa_rmsnorm(a->x, a->blocks[0].ln_weight, p.normed, p.rows, (int32_t)E, E, E, a->blocks[0].ln_eps,
+                                         MVPA_BF16, MVPA_BF16, stream)) != MVPA_OK) return st;
+    for (int i = first; i < end; ++i) {
+      const mvpa_stack_block& blk = a->blocks[i];
+      const bool last = i + 1 == a->n_blocks;
+      if ((st = mvpa_linear_bf16_dual(p.normed, blk.w_qkv, p.qkv, blk.w_gate_up, p.both + E, p.rows, nw, inner, E, E, E, nw,
+                                      E, wide, stream)) != MVPA_OK) return st;
+      if ((st = launch_append(p.qkv + E, p.qkv + E + kv, (bf16_t*)blk.k_cache, (bf16_t*)blk.v_cache, a->ring_head, a->T - 1,
+                              a->B, a->Hkv, a->C, a->Dh, n * nw, a->Dh, nw, blk.cache_stride_b, blk.cache_stride_g,
+                              s)) != MVPA_OK) return st;
+      if ((st = attend(blk)) != MVPA_OK) return st;
+      if ((st = mvpa_linear_bf16_residual(p.both, blk.w_tail, i ? p.hidden[(i - 1) & 1] : a->x, p.hidden[i & 1], p.rows, E, wide,
+                                          wide, wide, E, E, stream)) != MVPA_OK) return st;
+      if ((st = mvpa_rmsnorm(p.hidden[i & 1], last ? a->lnf_weight : a->blocks[i + 1].ln_weight, last ? a->y : p.normed, p.rows,
+                             (int32_t)E, E, E, last ? a->lnf_eps : a->blocks[i + 1].ln_eps, MVPA_BF16, MVPA_BF16,
+                             stream)) != MVPA_OK) return st;
+    }
+    return MVPA_OK;
+  }
   if (p.many) {
     for (int i = first; i < end; ++i) {
       const mvpa_stack_block& blk = a->blocks[i];

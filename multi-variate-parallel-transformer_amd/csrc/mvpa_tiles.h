@@ -59,4 +59,10 @@ int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, cons
 int launch_tail_reduce(const float* P, const tile_split& split, const bf16_t* r, bf16_t* sum, bf16_t* norm, const float* w,
                        float eps, float* ss, int64_t M, int64_t N, hipStream_t s);
 
+// One new time step of keys and values, [B,Hkv,C,Dh] views (strides in elements, multiples of 8, unit last
+// stride), into slot `slot` (or *head) of caches as in tile_out.  Implemented in mvpa_dense.hip.
+int launch_append(const bf16_t* k_new, const bf16_t* v_new, bf16_t* k, bf16_t* v, const int32_t* head, int32_t slot,
+                  int32_t B, int32_t Hkv, int32_t C, int32_t Dh, int64_t stride_b, int64_t stride_h, int64_t stride_c,
+                  int64_t cache_stride_b, int64_t cache_stride_h, hipStream_t s);
+
 }  // namespace mvpa

@@ -8,6 +8,7 @@ import torch
 import torch.nn.utils.parametrize
 
 import mvpa_hip
+from layers import MvpaRingCache, MvpaRingClock
 from models.configs import MVPFORMER_S
 from models.fftencoder import WaveEncoder
 from models.mvpformer import HMVPFormer, MVPFormerConfig, MVPFormerHead, MVPFormerModel, _StackOperands
@@ -132,6 +133,34 @@ def test_validity_of_another_shape_is_refused(shape):
             model(inputs_embeds=x, channel_validity=valid)
         flash = _model()
         assert torch.equal(flash(inputs_embeds=x, channel_validity=valid), flash(inputs_embeds=x))
+
+
+@pytest.mark.parametrize("rings", [False, True])
+@pytest.mark.parametrize("B,C", [(28, 64), (32, 64), (30, 117)])      # 7, 8 and 14 tiles of 256 rows, the last with odd rows
+def test_steps_of_many_rows(B, C, rings):
+    """Steps of enough rows for the 256-row tiles, on caches and on rings, against the same steps in 64 bits:
+    the bound is that of the few-row steps beside it."""
+    model = _model(n_inner=3200)                         # 26 column tiles: 182 tiles at 7 x 256 rows, 208 at 8; the line is 192
+    steps, W = 6, 4
+    xs = torch.randn(steps, B, 1, C, 128, device="cuda").bfloat16()
+    cfg = dict(n_layer=2, n_head=2, n_head_kv=1)
+    params = {n: p.detach() for n, p in model.named_parameters()}
+    caches, out = model.new_cache(B, C, max_steps=W), []
+    clock = MvpaRingClock(W, W - 1, "cuda")
+    with torch.no_grad():
+        for i, x in enumerate(xs):
+            if rings and i == W:
+                caches = tuple(MvpaRingCache.from_cache(c, clock) for c in caches)
+            if rings and i >= W:
+                clock.advance()
+            out.append(model(inputs_embeds=x, past_key_values=caches)[0])
+    for b in (0, B - 1):
+        ref, keys, _ = O.stream_steps(xs[:, b, 0], params, cfg, W)
+        for got, want in zip(out, ref):
+            assert _rel(got[b, 0], want) <= REL
+        if not rings:
+            got = torch.stack([c.views()[0][b].permute(1, 2, 0, 3) for c in caches])
+            assert _rel(got, keys) <= REL
 
 
 def test_plan_follows_the_weights():
