@@ -934,14 +934,21 @@ int mvpa_launch_mfma(const mvpa_fwd_args* a, hipStream_t stream) {
   using namespace mvpa;
   // a decoding step cut into runs: the builds made for it, by the number of channels (us with the merge, this
   // kernel -> those: B1 H12 C64 T64 Dh64 8 runs 17.8 -> 11.2, H12 C21 16.5 -> 9.7, H16 C128 T110 Dh128 16 runs
-  // 50 -> 28, T512 108 -> 82); fp8 and the lengths they have no LDS for stay here
-  if ((a->flags & MVPA_FLAG_LAST_STEP) && a->split_ws && a->n_split > 1 && (a->flags & MVPA_FLAG_CONTENT) &&
-      (mvpa_wave_supported(a) || mvpa_step_supported(a))) {
-    const int st = mvpa_step_supported(a) ? mvpa_launch_step(a, stream) : mvpa_launch_wave(a, stream);
-    if (st != MVPA_OK) return st;
-    if (a->dtype == MVPA_F16) launch_merge<el_f16>(a, stream);
-    else launch_merge<el_bf16>(a, stream);
-    return take_launch_status();
+  // 50 -> 28, T512 108 -> 82); fp8 and the lengths they have no LDS for stay here.  Runs too long for the step
+  // kernel at 65..128 channels are mostly better off here than with the one that reads K and V once per query
+  // tile (this kernel : that one, Dh 128 C80 T1024 in 16 runs 174 : 235, B8 C80 T110 in 2 152 : 205, C128 T600
+  // in 16 135 : 130, T1024 209 : 201; Dh 64 C128 T2048 in 16 188 : 202, B4 C100 T512 in 4 179 : 190; Dh 32
+  // C128 T300 in 16 46 : 16).
+  if ((a->flags & MVPA_FLAG_LAST_STEP) && a->split_ws && a->n_split > 1 && (a->flags & MVPA_FLAG_CONTENT)) {
+    const bool step = mvpa_step_supported(a);
+    const bool wave = !step && mvpa_wave_supported(a) && (a->C <= 64 || a->Dh == 32 || (a->Dh == 128 && a->C > 96));
+    if (step || wave) {
+      const int st = step ? mvpa_launch_step(a, stream) : mvpa_launch_wave(a, stream);
+      if (st != MVPA_OK) return st;
+      if (a->dtype == MVPA_F16) launch_merge<el_f16>(a, stream);
+      else launch_merge<el_bf16>(a, stream);
+      return take_launch_status();
+    }
   }
   const int nct = a->C <= 32 ? 1 : a->C <= 64 ? 2 : 4;
   switch (a->Dh) {
