@@ -938,10 +938,13 @@ int mvpa_launch_mfma(const mvpa_fwd_args* a, hipStream_t stream) {
   // kernel at 65..128 channels are mostly better off here than with the one that reads K and V once per query
   // tile (this kernel : that one, Dh 128 C80 T1024 in 16 runs 174 : 235, B8 C80 T110 in 2 152 : 205, C128 T600
   // in 16 135 : 130, T1024 209 : 201; Dh 64 C128 T2048 in 16 188 : 202, B4 C100 T512 in 4 179 : 190; Dh 32
-  // C128 T300 in 16 46 : 16).
+  // C128 T300 in 16 46 : 16), and so are 33..64 channels at Dh 64 past one workgroup per CU, two query tiles each
+  // (B8 H12 C64 in 2 runs, T 25 / 64 / 110 19.3 : 21.1, 28.3 : 32.2, 41.2 : 42.8; B4 T110 in 2 39 : 25).
   if ((a->flags & MVPA_FLAG_LAST_STEP) && a->split_ws && a->n_split > 1 && (a->flags & MVPA_FLAG_CONTENT)) {
     const bool step = mvpa_step_supported(a);
-    const bool wave = !step && mvpa_wave_supported(a) && (a->C <= 64 || a->Dh == 32 || (a->Dh == 128 && a->C > 96));
+    const bool wave = !step && mvpa_wave_supported(a) &&
+                      (a->C <= 32 || a->Dh == 32 || (a->C <= 64 ? a->Dh == 128 || (int64_t)a->B * a->H * a->n_split <= 128
+                                                               : a->Dh == 128 && a->C > 96));
     if (step || wave) {
       const int st = step ? mvpa_launch_step(a, stream) : mvpa_launch_wave(a, stream);
       if (st != MVPA_OK) return st;

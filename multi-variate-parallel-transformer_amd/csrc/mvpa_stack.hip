@@ -66,11 +66,14 @@ static bool stack_supported(const mvpa_stack_args* a) {
 
 // Key runs of a step: a power of two, up to one workgroup per CU (the query tiles of a head are workgroups
 // of their own up to 64 channels) and no run under 4 steps (us by runs 4 / 8 / 16: H12 C64 T64 12.6 / 11.2 / 16.9,
-// H12 C21 T64 10.5 / 9.7 / 10, H16 C128 T110 Dh128 60 / 37 / 28, H16 C64 T110 Dh128 28 / 22 / 33).
+// H12 C21 T64 10.5 / 9.7 / 10, H16 C128 T110 Dh128 60 / 37 / 28, H16 C64 T110 Dh128 28 / 22 / 33); still two, of
+// 8 steps and more, while the (b, h) pairs alone leave half the CUs idle (us in one / two: B8 H16 C64 T110 Dh128
+// 216 / 87, T25 57 / 40, B8 H12 C64 T64 Dh64 40 / 28, T25 20.9 / 19.3).
 static int default_runs(const mvpa_stack_args* a) {
   const int wgs = a->B * a->H * (a->C > 64 ? 1 : (a->C + 31) / 32);
   int n = 1;
   while (2 * n * wgs <= 256 && 8 * n <= a->T) n *= 2;
+  if (n == 1 && 2 * a->B * a->H <= 256 && a->T >= 16) n = 2;
   while (n > 1 && (int64_t)(n - 1) * ((a->T + n - 1) / n) >= a->T) --n;      // no empty run
   return n;
 }

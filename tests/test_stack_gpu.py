@@ -135,6 +135,23 @@ def test_validity_of_another_shape_is_refused(shape):
         assert torch.equal(flash(inputs_embeds=x, channel_validity=valid), flash(inputs_embeds=x))
 
 
+@pytest.mark.parametrize("B,C,dims", [(1, 21, {}), (40, 40, {}), (70, 33, {}), (40, 40, dict(n_embd=256)), (2, 100, {})],
+                         ids=["B1C21", "B40C40", "B70C33", "B40C40D128", "B2C100"])
+def test_steps_in_key_runs(B, C, dims):
+    """Steps against 18 cached ones, in as many key runs as (b, h) pairs and query tiles leave room for (4, 2, 1,
+    2, 4 - on the kernels for short runs and on the tiled one), against the same steps in 64 bits."""
+    model = _model(**dims)
+    W, e = 18, model.embed_dim
+    xs = torch.randn(W + 1, B, 1, C, e, device="cuda").bfloat16()
+    caches = model.new_cache(B, C, max_steps=W)
+    with torch.no_grad():
+        out = [model(inputs_embeds=x, past_key_values=caches)[0] for x in xs]
+    for b in (0, B - 1):
+        ref, _, _ = O.stream_steps(xs[:, b, 0], {n: p.detach() for n, p in model.named_parameters()},
+                                   dict(n_layer=2, n_head=2, n_head_kv=1), W)
+        assert max(_rel(got[b, 0], want) for got, want in zip(out, ref)) <= REL
+
+
 @pytest.mark.parametrize("rings", [False, True])
 @pytest.mark.parametrize("B,C", [(28, 64), (32, 64), (30, 117)])      # 7, 8 and 14 tiles of 256 rows, the last with odd rows
 def test_steps_of_many_rows(B, C, rings):
