@@ -17,18 +17,15 @@
 
 namespace mvpa {
 
-// The 256-row tiles are the better ones once [q/k/v | gate/up] is this many of them, about a round and
-// a half of the chip (us per block, 256-row against small tiles: a model of 768 columns at
-// 1600 / 3200 / 4096 rows 105 : 68, 126 : 130, 150 : 173; of 2048 columns at 1024 / 1536 / 2048 rows
-// 258 : 203, 313 : 295, 331 : 361).
-constexpr int64_t kManyTiles = 352;
-
-// A step's products are few-row ones up to more tiles the longer the contraction (us a step of all blocks,
-// 256-row against small tiles, window 25: MVPFormer-S, 64 channels at 3072 / 3584 / 4096 / 6144 rows = 228 /
-// 266 / 304 / 456 tiles 1966 : 1925, 2211 : 2137, 2328 : 2473, 2873 : 3623; base model, 128 channels at
-// 1280 / 1536 / 2048 / 3072 rows = 300 / 360 / 480 / 720 tiles 11138 : 10066, 11519 : 10870, 12179 : 13235,
-// 18195 : 23241; 64 channels 1536 / 2048 rows 9877 : 9256, 10374 : 11535).
-static int64_t many_step_tiles(int64_t E) { return 176 + E / 8; }
+// The 256-row tiles are the better ones once [q/k/v | gate/up] is this many of them, the more the longer the
+// contraction; a step's small tiles write the caches themselves and stand a little longer.  256-row against small
+// tiles, us a pass of all blocks at so many tiles,
+//   windows of MVPFormer-S   209 1425 : 1352, 228 1364 : 1386, 247 1418 : 1536, 285 1597 : 1710, 304 1664 : 1903,
+//                            342 1726 : 2141; 266 at 37 channels 1690 : 1624
+//   of the base model        360 7849 : 7311, 420 7894 : 7989, 480 7762 : 8403, 600 9818 : 11661
+//   steps of MVPFormer-S     228 1966 : 1925, 266 2211 : 2137, 304 2328 : 2473, 456 2873 : 3623
+//   of the base model        300 11138 : 10066, 360 11519 : 10870, 480 12179 : 13235, 720 18195 : 23241
+static int64_t many_tiles(int64_t E, bool step) { return (step ? 176 : 148) + E / 8; }
 
 static int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }
 
@@ -84,7 +81,7 @@ static void stack_layout(const mvpa_stack_args* a, stack_plan& p, stack_ws& w) {
   p.raw = !a->step && a->sumsq;
   for (int i = 0; i < a->n_blocks; ++i) p.raw = p.raw && a->blocks[i].w_qkv_normed && a->blocks[i].w_gate_up_normed;
   const int64_t tiles = (p.rows + 255) / 256 * ((inner + 127) / 128 + (E + 2 * kv + 255) / 256);
-  p.many = (a->step ? tiles >= many_step_tiles(E) : p.raw && tiles >= kManyTiles) && p.rows >= 512 && E >= 128;
+  p.many = (p.raw || a->step) && tiles >= many_tiles(E, a->step) && p.rows >= 512 && E >= 128;
   p.ld_qkv = a->step && !p.many ? E : E + 2 * kv;
   p.qkv = (bf16_t*)w.take(p.rows * p.ld_qkv * 2);
   p.both = (bf16_t*)w.take(p.rows * (E + inner) * 2);

@@ -528,7 +528,8 @@ def _tables64(p, cfg, e, pos, chan):
 
 def stack_forward(embeds: torch.Tensor, params: dict, cfg: dict, chan_valid: Optional[torch.Tensor] = None):
     """mvpformer_forward without the encoder, in 64 bits: embeds [B,T,C,E], params under the names of
-    the stack alone (h.{i}.*, ln_f.weight, ...), chan_valid [B,C] -> [B,T,C,E]."""
+    the stack alone (h.{i}.*, ln_f.weight, ...), chan_valid [B,C] -> [B,T,C,E].  Products where embeds is,
+    the attention on the CPU."""
     params = {n: t.double() for n, t in params.items()}
     b, t, c, e = embeds.shape
     nh, g = cfg["n_head"], cfg["n_head_kv"]
@@ -538,9 +539,9 @@ def stack_forward(embeds: torch.Tensor, params: dict, cfg: dict, chan_valid: Opt
         tabs = _tables64(p, cfg, e, params["positional_embedding.weight"][:t], params["channel_embedding.weight"][:c])
 
         def attend(q, k, v):
-            heads = (x.view(b, t * c, n, e // nh).transpose(1, 2) for x, n in ((q, nh), (k, g), (v, g)))
-            out = mvpa_direct(*heads, *tabs, chan_valid=chan_valid)
-            return out.transpose(1, 2).reshape(b, t * c, e)
+            heads = (x.view(b, t * c, n, e // nh).transpose(1, 2).cpu() for x, n in ((q, nh), (k, g), (v, g)))
+            out = mvpa_direct(*heads, *(x.cpu() for x in tabs), chan_valid=None if chan_valid is None else chan_valid.cpu())
+            return out.transpose(1, 2).reshape(b, t * c, e).to(q.device)
         h = _block64(h, p, cfg, attend)
     return _rmsnorm64(h, params["ln_f.weight"], cfg.get("layer_norm_epsilon", 1e-5)).view(b, t, c, e)
 

@@ -54,6 +54,22 @@ def test_whole_sequence(monkeypatch, dims, B, C, T):
     assert a.shape == b.shape and _rel(a, b) <= REL
 
 
+@pytest.mark.parametrize("B,C,T", [(4, 96, 4), (4, 112, 4), (3, 117, 6)], ids=str)     # 6, 7 and 9 tiles of 256 rows
+@pytest.mark.parametrize("flash", [True, False])
+def test_windows_of_many_rows(flash, B, C, T):
+    """On either side of the line between the tile sizes, with channels absent where the class honours them,
+    against the stack in 64 bits."""
+    model = _model(flash, n_inner=3200)                  # 26 column tiles: 156 tiles at 6 x 256 rows, 182 at 7; the line is 164
+    x = torch.randn(B, T, C, 128, device="cuda").bfloat16()
+    valid = torch.rand(B, C, device="cuda") < 0.8
+    valid[:, 0] = True
+    with torch.no_grad():
+        got = model(inputs_embeds=x, channel_validity=valid)
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=2, n_head_kv=1),
+                           None if flash else valid)
+    assert _rel(got, want) <= REL
+
+
 @pytest.mark.parametrize("B,C", [(1, 5), (1, 64), (2, 100)])
 def test_steps_on_caches(monkeypatch, B, C):
     """A stream that fills its window and slides on: outputs, and every cached key and value."""
