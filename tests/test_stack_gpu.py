@@ -1,6 +1,6 @@
-"""The stack of blocks as one library call (small-tile products, caches written by their epilogue) against
-the same blocks one by one, and the one-pass encoder against its separate kernels, at the sizes where
-tiles, splits and rows end."""
+"""The stack of blocks as one library call against the stack in 64 bits and against the same blocks one by
+one, what it keeps between calls, and the one-pass encoder against its separate kernels, at the sizes where
+tiles, splits, runs and rows end."""
 import copy
 
 import pytest
@@ -16,9 +16,9 @@ from oracle import mvpa_oracle as O
 
 pytestmark = pytest.mark.gpu
 
-# Both sides multiply bf16 operands with fp32 accumulation; the library call keeps the attention and MLP
-# outputs of a block in fp32 until one rounding where the blocks one by one round three times.  Two
-# blocks, a handful of roundings of 2^-9 each: 1e-2 relative.
+# The products take bf16 operands and sum in fp32; attention output, MLP output and their sum with the residual
+# are rounded to bf16 each (in products of many rows once together), as the blocks one by one round them.  Two
+# blocks are a handful of roundings of 2^-9 each: 1e-2 relative.
 REL = 1e-2
 
 
@@ -33,7 +33,7 @@ def _model(flash=True, **kw):
 
 
 def _rel(a, b):
-    return ((a.float() - b.float()).norm() / b.float().norm()).item()
+    return ((a.double() - b.double()).norm() / b.double().norm()).item()
 
 
 @pytest.mark.parametrize("dims", [{}, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=64),      # ragged column tiles
@@ -42,8 +42,9 @@ def _rel(a, b):
 @pytest.mark.parametrize("B,C,T", [(1, 1, 1), (1, 31, 1), (1, 33, 1), (1, 64, 1), (1, 13, 5), (1, 128, 1), (3, 43, 1),
                                    (1, 64, 8), (2, 37, 7)],     # row tiles of 32, 64, 128; rows from which ln_1 is fused
                          ids=lambda v: str(v))
-def test_whole_sequence(monkeypatch, dims, B, C, T):
-    model = _model(**dims)
+@pytest.mark.parametrize("flash", [True, False], ids=["flash", "masked"])
+def test_whole_sequence(monkeypatch, flash, dims, B, C, T):
+    model = _model(flash, **dims)
     x = torch.randn(B, T, C, model.embed_dim, device="cuda").bfloat16()
     valid = torch.rand(B, C, device="cuda") < 0.8
     valid[:, 0] = True
@@ -51,7 +52,9 @@ def test_whole_sequence(monkeypatch, dims, B, C, T):
         a = model(inputs_embeds=x, channel_validity=valid)
         monkeypatch.setattr(MVPFormerModel, "_native", lambda *args: None)
         b = model(inputs_embeds=x, channel_validity=valid)
-    assert a.shape == b.shape and _rel(a, b) <= REL
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()},
+                           dict(n_layer=2, n_head=model.num_heads, n_head_kv=model.num_kv_heads), None if flash else valid)
+    assert a.shape == b.shape and _rel(a, want) <= REL and _rel(b, want) <= REL and _rel(a, b) <= REL
 
 
 @pytest.mark.parametrize("B,C,T", [(4, 96, 4), (4, 112, 4), (3, 117, 6)], ids=str)     # 6, 7 and 9 tiles of 256 rows
@@ -72,7 +75,8 @@ def test_windows_of_many_rows(flash, B, C, T):
 
 @pytest.mark.parametrize("B,C", [(1, 5), (1, 64), (2, 100)])
 def test_steps_on_caches(monkeypatch, B, C):
-    """A stream that fills its window and slides on: outputs, and every cached key and value."""
+    """A stream that fills its window and slides on: outputs, and every cached key and value, against the same
+    steps in 64 bits and between the stack call and the blocks one by one."""
     model = _model()
     xs = torch.randn(12, B, 1, C, model.embed_dim, device="cuda").bfloat16()
     runs = []
@@ -86,6 +90,14 @@ def test_steps_on_caches(monkeypatch, B, C):
             runs.append((out, [t.clone() for c in caches for t in c.views()]))
     for a, b in zip(runs[0][0] + runs[0][1], runs[1][0] + runs[1][1]):
         assert a.shape == b.shape and _rel(a, b) <= REL
+    for b in range(B):
+        ref, keys, values = O.stream_steps(xs[:, b, 0], {n: p.detach() for n, p in model.named_parameters()},
+                                           dict(n_layer=2, n_head=2, n_head_kv=1), 8)
+        for got, want in zip(runs[0][0], ref):
+            assert _rel(got[b, 0], want) <= REL
+        for i, kv in enumerate((keys, values)):
+            got = torch.stack([t[b].permute(1, 2, 0, 3) for t in runs[0][1][i::2]])
+            assert got.shape == kv.shape and _rel(got, kv) <= REL
 
 
 @pytest.mark.parametrize("C,W,steps", [(21, 14, 18), (64, 20, 21)])
