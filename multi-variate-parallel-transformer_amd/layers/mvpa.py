@@ -11,7 +11,6 @@ What differs is mechanism only:
   permute+contiguous copies of _split_heads/_merge_heads (layers/mvpa.py:161-171) vanish.
 * the score/softmax/PV chain of _rel_attn (layers/mvpa.py:173-278) is the fused kernel; no
   [B,H,N,N] tensor exists, hence `output_attentions=True` raises.
-Forward / eval only (no autograd through the kernel).
 """
 from __future__ import annotations
 
