@@ -441,7 +441,7 @@ class MVPFormerModel(nn.Module):
         def own(module):
             return isinstance(module._parameters.get("weight"), torch.Tensor)
 
-        first, inner = self.h[0].attn, self.h[0].mlp.down_proj.in_features
+        first, inner = self.h[0].attn, self.h[0].mlp.down_proj.in_features          # of their classes: _native
         shape = (first.num_heads, first.num_kv_heads, first.head_dim)
         if (_GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1] or not _plain(self.ln_f, RMSNorm)
                 or not all(map(own, (self.ln_f, self.positional_embedding, self.channel_embedding)))):
@@ -528,7 +528,11 @@ class MVPFormerModel(nn.Module):
         on caches; None where that call does not apply (an additive key bias, caches of another
         kind, shapes outside the matrix-core kernels) and the blocks go one by one."""
         bsz, t_new, c_len, e = hidden_states.shape
-        attn, inner = self.h[0].attn, self.h[0].mlp.down_proj.in_features
+        first = self.h[0]
+        if (type(first) is not MVPFormerBlock or type(first.mlp) is not GatedMLP
+                or type(first.attn) not in (MVPFormerGQAAttention, MVPFormerGQAFlashAttention)):
+            return None
+        attn, inner = first.attn, first.mlp.down_proj.in_features
         if e % 64 or inner % 64 or e > 4096 or c_len > 128 or attn.head_dim not in (32, 64, 128) or bsz == 0:
             return None
         valid = None

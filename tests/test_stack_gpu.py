@@ -297,6 +297,40 @@ def test_other_norms_are_called(C, T):
         assert _rel(got, model.ln_f(h)) <= REL
 
 
+class _Around(torch.nn.Module):
+    """A module in a block's place for attention or MLP: what it holds, called, and louder."""
+
+    def __init__(self, inner, *names):
+        super().__init__()
+        self.inner = inner
+        for n in names:
+            setattr(self, n, getattr(inner, n))
+
+    def forward(self, *args, **kw):
+        out = self.inner(*args, **kw)
+        return (out[0] * 2, *out[1:]) if isinstance(out, tuple) else out * 2
+
+
+@pytest.mark.parametrize("where", [0, 1])
+@pytest.mark.parametrize("T", [5, 0], ids=["window", "step"])
+def test_other_modules_in_a_block_are_called(where, T):
+    """Attention and MLP of other classes, with no more attributes than the blocks one by one ask for."""
+    model = _model()
+    blk = model.h[where]
+    plain = copy.deepcopy(model)
+    blk.attn, blk.mlp = _Around(blk.attn, "embed_dim"), _Around(blk.mlp, "down_proj")
+    with torch.no_grad():
+        for m in (plain.h[where].attn.c_proj, plain.h[where].mlp.down_proj):
+            m.weight.mul_(2.0)
+        x = torch.randn(1, max(T, 1), 13, 128, device="cuda").bfloat16()
+
+        def out(model):
+            if T:
+                return model(inputs_embeds=x)
+            return model(inputs_embeds=x, past_key_values=plain.new_cache(1, 13, max_steps=2))[0]
+        assert _rel(out(model), out(plain)) <= REL
+
+
 def test_weights_that_are_computed():
     """An embedding whose rows are computed on access is no operand to keep: the blocks go one by one."""
     class Twice(torch.nn.Module):
