@@ -303,6 +303,12 @@ PyObject* py_mean_rows(PyObject*, PyObject* arg) {
   END_HANDLE_TH_ERRORS
 }
 
+// as_operand, starting at a 16-byte boundary
+Tensor aligned_operand(const Tensor& t, at::ScalarType dt) {
+  Tensor r = as_operand(t, dt);
+  return (uintptr_t)r.const_data_ptr() & 15 ? r.clone() : r;
+}
+
 // ---- row operations of the training path -------------------------------------------------------
 bool f32_or_bf16(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
 
@@ -344,7 +350,7 @@ PyObject* py_silu_gate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   TORCH_CHECK(n == 1 || n == 2, "silu_gate takes gu and, for the backward, the gradient");
   at::AutoDispatchBelowADInplaceOrView guard;
-  const Tensor gu = as_operand(tensor_of(args[0]), at::kBFloat16);
+  const Tensor gu = aligned_operand(tensor_of(args[0]), at::kBFloat16);
   TORCH_CHECK(gu.dim() >= 1 && gu.size(-1) % 2 == 0 && gu.numel() > 0, "silu_gate: rows of gate and up");
   const int64_t cols = gu.size(-1) / 2, rows = gu.numel() / (2 * cols);
   std::vector<int64_t> shape(gu.sizes().begin(), gu.sizes().end());
@@ -355,7 +361,7 @@ PyObject* py_silu_gate(PyObject*, PyObject* const* args, Py_ssize_t n) {
     y = at::empty(shape, gu.options());
     st = mvpa_silu_gate_bf16(gu.data_ptr(), y.data_ptr(), rows, (int32_t)cols, current_stream());
   } else {
-    const Tensor d = as_operand(tensor_of(args[1]), at::kBFloat16);
+    const Tensor d = aligned_operand(tensor_of(args[1]), at::kBFloat16);
     TORCH_CHECK(d.sizes() == at::IntArrayRef(shape), "silu_gate: shapes differ");
     y = at::empty_like(gu);
     st = mvpa_silu_gate_backward_bf16(gu.data_ptr(), d.data_ptr(), y.data_ptr(), rows, (int32_t)cols, current_stream());

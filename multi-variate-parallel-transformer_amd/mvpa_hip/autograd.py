@@ -142,10 +142,12 @@ class _Add3RMSNormFn(torch.autograd.Function):
 
 def add3_rmsnorm(a, b, c, w, eps):
     """(a + b + c, RMSNorm(a + b + c) * w) in one pass each way, or None where the operands are not bf16
-    rows of whole 16-byte chunks on the GPU."""
+    rows of whole 16-byte chunks on the GPU, or do not start at one."""
     if (not a.is_cuda or not a.dtype == b.dtype == c.dtype == torch.bfloat16 or not a.shape == b.shape == c.shape
             or a.shape[-1] % 8 or a.shape[-1] > MAX_NORM_COLS or not a.numel()
-            or w.dtype not in (torch.bfloat16, torch.float32)):
+            or w.dtype not in (torch.bfloat16, torch.float32)
+            or any(t.is_contiguous() and t.data_ptr() % 16 for t in (a, b, c))       # others are copied to a row of their own
+            or w.dtype == torch.float32 and w.data_ptr() % 16):
         return None
     return _Add3RMSNormFn.apply(a, b, c, w, eps)
 

@@ -5,6 +5,7 @@ import torch
 
 import mvpa_hip
 from attentions.attn import FlashMVPA, FlashMVPAPacked
+from models.mvpformer import MVPFormerConfig, MVPFormerModel
 from mvpa_hip import autograd as AG
 
 pytestmark = pytest.mark.gpu
@@ -110,3 +111,45 @@ def test_packed_attention(B, C, T, H, Hkv, Dh, masked):
     for x, y in zip(got, ref):
         assert x.shape == y.shape
         assert (x.double() - y.double()).norm() <= 2.0 ** -6 * y.double().norm() + 1e-6
+
+
+def test_operands_that_start_anywhere():
+    """Rows, gradients and an fp32 norm weight at an offset of one element: the kernels that read 16 bytes at a
+    time get copies or leave the work to the general path, and values and gradients are the aligned ones'."""
+    g = torch.Generator(device="cuda").manual_seed(6)
+
+    def at_one(t):
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape).detach().requires_grad_(t.requires_grad)
+    a, b, c = ((torch.randn(6, 64, generator=g, device="cuda")).bfloat16().requires_grad_(True) for _ in range(3))
+    w = (1 + 0.1 * torch.randn(64, generator=g, device="cuda")).requires_grad_(True)
+    # a random projection as the loss: the rows of a norm have the same length whatever goes in, so the gradient of
+    # their squares is a difference of nearly equal terms, with errors above 1e-2 of what is left
+    towards = torch.randn(6, 64, generator=g, device="cuda")
+    results = []
+    for where in (lambda t: t, at_one):
+        x, weight = [where(t) for t in (a, b, c)], where(w)
+        got = AG.add3_rmsnorm(*x, weight, 1e-5)
+        if got is None:
+            total = x[0] + x[1] + x[2]
+            got = total, AG.rmsnorm(total, weight, 1e-5)
+        results.append((*got, *torch.autograd.grad((got[1].float() * towards).sum(), [*x, weight])))
+    for p, q in zip(*results):
+        _near(q, p)
+    gu, d = torch.randn(6, 64, generator=g, device="cuda").bfloat16(), torch.randn(6, 32, generator=g, device="cuda").bfloat16()
+    assert torch.equal(mvpa_hip.silu_gate(at_one(gu)), mvpa_hip.silu_gate(gu))
+    assert torch.equal(mvpa_hip.silu_gate(at_one(gu), at_one(d)), mvpa_hip.silu_gate(gu, d))
+    # a training pass on embeddings that start anywhere
+    torch.manual_seed(0)
+    dims = dict(n_positions=8, n_channels=8, n_embd=128, n_layer=2, n_head=2, n_head_kv=1, n_inner=64, resid_pdrop=0.0,
+                embd_pdrop=0.0, attn_pdrop=0.0)
+    model = MVPFormerModel(MVPFormerConfig(**dims)).to("cuda", torch.bfloat16).train()
+    x = torch.randn(1, 5, 6, 128, generator=g, device="cuda").bfloat16().requires_grad_(True)
+    towards = torch.randn(1, 5, 6, 128, generator=g, device="cuda")
+    grads = [torch.autograd.grad((model(inputs_embeds=t).float() * towards).sum(), t)[0] for t in (x, at_one(x))]
+    _near(grads[1], grads[0])
+
+
+def _near(got, ref):
+    """The general path rounds the sum of three twice: half a unit of 2^-8, 0.11 % rms of a part of the sum, and
+    the gradients, of the same size each, are rounded to bf16 on both sides: 0.4 % in all, of two blocks twice that."""
+    assert ((got.double() - ref.double()).norm() / ref.double().norm()).item() <= 1e-2
