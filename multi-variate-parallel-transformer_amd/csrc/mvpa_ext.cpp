@@ -513,6 +513,21 @@ PyObject* py_set_block(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// plan_tensors(plan): every tensor it keeps
+PyObject* py_plan_tensors(PyObject*, PyObject* o) {
+  HANDLE_TH_ERRORS
+  const Plan* p = plan_of(o);
+  if (!p) return nullptr;
+  PyObject* r = PyList_New(0);
+  for (const Tensor& t : p->keep) {
+    PyObject* w = THPVariable_Wrap(t);
+    PyList_Append(r, w);
+    Py_DECREF(w);
+  }
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
 // One pass over the blocks of a plan: its arguments, checked, and every buffer it needs.
 struct Run {
   std::vector<Tensor> keep;
@@ -638,6 +653,7 @@ PyMethodDef kMethods[] = {
     {"watch", (PyCFunction)(void*)py_watch, METH_FASTCALL, "what a model looks like now"},
     {"watch_current", (PyCFunction)py_watch_current, METH_O, "whether it still looks like that"},
     {"set_block", (PyCFunction)(void*)py_set_block, METH_FASTCALL, "operands of one block"},
+    {"plan_tensors", (PyCFunction)py_plan_tensors, METH_O, "the tensors a plan keeps"},
     {"begin", (PyCFunction)(void*)py_begin, METH_FASTCALL, "a pass over a plan's blocks, checked"},
     {"enqueue", (PyCFunction)(void*)py_enqueue, METH_FASTCALL, "launch blocks of a pass"},
     {nullptr, nullptr, 0, nullptr}};

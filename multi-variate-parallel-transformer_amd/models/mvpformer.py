@@ -14,6 +14,8 @@ from __future__ import annotations
 
 import collections
 import functools
+import itertools
+import threading
 from typing import Optional
 
 import torch
@@ -317,18 +319,66 @@ class MVPFormerBlock(nn.Module):
         return outputs, next_normed
 
 
+_PREPARING = threading.RLock()
+
+
 class _StackOperands:
     """What the library's stack call was given of a model, as long as `watch` finds the model unchanged.
 
     weights: the operands of each block that no shape enters, by (block, with ln_1 in the columns or without);
     plans: the last SHAPES shapes in use, the one used last at the end - the bias tables of each (24 blocks of
     the base model at 128 channels and 512 positions: 31 MB) beside the weights they share.  A recording's
-    shape, those of a few others and of a stream beside them stay; a stream that fills its window passes through."""
+    shape, those of a few others and of a stream beside them stay; a stream that fills its window passes through.
+    Made under _PREPARING by one thread at a time, used by any, on any stream."""
 
     SHAPES = 8
 
-    def __init__(self, watch=None):
-        self.watch, self.weights, self.plans = watch, {}, collections.OrderedDict()
+    def __init__(self):
+        self.watch, self.weights, self.plans = None, {}, collections.OrderedDict()
+        self.streams, self.made, self.waited = {}, {}, {}     # by stream: itself, its last event, {stream: event waited for}
+
+    def use(self, key):
+        """The plan of a shape, for a pass on the current stream; None: not made yet."""
+        plan = self.plans.get(key)
+        if plan is not None:
+            self.join()
+            try:
+                self.plans.move_to_end(key)
+            except KeyError:                     # given up by another thread meanwhile: its last pass
+                pass
+        return plan
+
+    def join(self):
+        """The current stream waits for the operands that passes on other streams made."""
+        raw = mvpa_hip._stream()
+        if raw in self.streams and len(self.streams) == 1 or torch.cuda.is_current_stream_capturing():
+            return                               # (a capture begins with everything done)
+        stream = self.streams.setdefault(raw, torch.cuda.current_stream())
+        waited = self.waited.setdefault(raw, {})
+        for other, event in list(self.made.items()):
+            if other != raw and waited.get(other) is not event:
+                stream.wait_event(event)
+                waited[other] = event
+
+    def add(self, key, plan, weights):
+        """A plan and the weights made for it on the current stream, whole from here on."""
+        raw = mvpa_hip._stream()
+        if not torch.cuda.is_current_stream_capturing():
+            self.streams.setdefault(raw, torch.cuda.current_stream())
+            event = torch.cuda.Event()
+            event.record()
+            self.made[raw] = event
+        self.weights.update(weights)
+        self.plans[key] = plan
+        while len(self.plans) > self.SHAPES:
+            self.retire([self.plans.popitem(last=False)[1]])
+
+    def retire(self, plans):
+        """Plans that go: their memory is free once the passes of every stream are through."""
+        if len(self.streams) > 1:
+            for t in itertools.chain.from_iterable(map(mvpa_hip.load_ext().plan_tensors, plans)):
+                for stream in list(self.streams.values()):
+                    t.record_stream(stream)
 
 
 class MVPFormerModel(nn.Module):
@@ -505,11 +555,11 @@ class MVPFormerModel(nn.Module):
                                          self.h[0].mlp.down_proj.in_features),
                                         mvpa_hip._as_f32_weight(self.ln_f.weight), float(self.ln_f.eps), blocks)
 
-    def _set_block(self, held, plan, i, t_len, c_len, pos_lo, normed):
+    def _set_block(self, known, made, plan, i, t_len, c_len, pos_lo, normed):
         blk, behind = self.h[i], self.h[i + 1].ln_1.weight if i + 1 < len(self.h) else None
-        weights = held.weights.get((i, normed))
+        weights = known.get((i, normed))
         if weights is None:
-            weights = held.weights[i, normed] = self._block_operands(blk, normed)
+            weights = made[i, normed] = self._block_operands(blk, normed)
         tables = blk.attn._key_tables(self.positional_embedding.weight[pos_lo:pos_lo + t_len][None],
                                       self.channel_embedding.weight[:c_len][None])
         mvpa_hip.load_ext().set_block(plan, i, (*weights, *(t.to(torch.bfloat16) for t in tables)),
@@ -540,7 +590,7 @@ class MVPFormerModel(nn.Module):
             valid, bias = mask.resolve(bsz, t_len, c_len)
             if bias is not None:
                 return None
-        caches = head = sumsq = None
+        caches = head = None
         rows = bsz * t_new * c_len
         if past_key_values is not None:
             kinds = {type(c) for c in past_key_values}
@@ -555,40 +605,65 @@ class MVPFormerModel(nn.Module):
                 head = clock.head32
             else:
                 return None
+        if past_key_values is not None:
+            first = [0 if head is not None else c.next_slot() - (t_len - 1) for c in past_key_values]
+            caches = ([c.k for c in past_key_values], [c.v for c in past_key_values], first)
+        grown = past_key_values if caches is not None and head is None else ()
+        normed = past_key_values is None and self.h[0].norm_fused_supported(rows)
+        key = (t_len, c_len, pos_lo, normed)
+
+        def arguments():
+            sumsq = mvpa_hip.row_sumsq(hidden_states.reshape(rows, e)) if normed else None
+            return hidden_states, valid, caches, head, sumsq
+
+        held = self._stack
+        plan = None
+        if held is not None and mvpa_hip.load_ext().watch_current(held.watch):
+            plan = held.use(key)
+        if plan is not None:
+            return self._pass(plan, arguments(), grown)
+        with _PREPARING:                    # one at a time: what is being made is nobody else's yet
+            return self._first_pass(key, arguments, grown)
+
+    def _pass(self, plan, arguments, grown, prepare=None):
+        """A pass on a plan; prepare(i): puts the operands of block i together while the one before runs."""
+        ext, blocks = mvpa_hip.load_ext(), len(self.h)
+        run = mvpa_hip._taken(ext.begin(plan, *arguments))
+        for c in grown:                     # only now: what begin() refuses leaves the caches as they were
+            c.make_room()
+        start = 0
+        if prepare is not None:
+            for i in range(1, blocks):
+                mvpa_hip._taken(ext.enqueue(run, i - 1, i))
+                prepare(i)
+            start = blocks - 1
+        out = mvpa_hip._taken(ext.enqueue(run, start, blocks))
+        for c in grown:
+            c.length += 1
+        return out
+
+    def _first_pass(self, key, arguments, grown):
+        """The pass of a model or a shape that has no plan yet, which leaves it one."""
         ext = mvpa_hip.load_ext()
         held = self._stack
         if held is None or not ext.watch_current(held.watch):
             self._stack = None
+            if held is not None:
+                held.retire(held.plans.values())
             if not self._stack_computes():
                 return None
             held = _StackOperands()
-        normed = past_key_values is None and self.h[0].norm_fused_supported(rows)
-        key = (t_len, c_len, pos_lo, normed)
-        plan = held.plans.pop(key, None)
-        fresh = plan is None
-        if fresh:
-            plan = self._new_plan(t_len, c_len)
-            self._set_block(held, plan, 0, *key)
-        if past_key_values is not None:
-            first = [0 if head is not None else c.next_slot() - (t_len - 1) for c in past_key_values]
-            caches = ([c.k for c in past_key_values], [c.v for c in past_key_values], first)
-        elif normed:
-            sumsq = mvpa_hip.row_sumsq(hidden_states.reshape(rows, e))
-        blocks = len(self.h)
-        run = mvpa_hip._taken(ext.begin(plan, hidden_states, valid, caches, head, sumsq))
-        grown = past_key_values if caches is not None and head is None else ()
-        for c in grown:                     # only now: what begin() refuses leaves the caches as they were
-            c.make_room()
-        if fresh:                           # a block runs while the next one's operands are put together
-            for i in range(1, blocks):
-                mvpa_hip._taken(ext.enqueue(run, i - 1, i))
-                self._set_block(held, plan, i, *key)
-        out = mvpa_hip._taken(ext.enqueue(run, blocks - 1 if fresh else 0, blocks))
-        for c in grown:
-            c.length += 1
-        held.plans[key] = plan              # whole from here on, and the one used last
-        while len(held.plans) > held.SHAPES:
-            held.plans.popitem(last=False)
+        plan = held.use(key)
+        if plan is not None:                # made by another thread meanwhile
+            return self._pass(plan, arguments(), grown)
+        held.join()
+        plan, weights = self._new_plan(*key[:2]), {}
+
+        def prepare(i):
+            self._set_block(held.weights, weights, plan, i, *key)
+        prepare(0)
+        out = self._pass(plan, arguments(), grown, prepare)
+        held.add(key, plan, weights)
         if held.watch is None:              # last: the GPU has its work by now
             held.watch = ext.watch(*self._survey())
             self._stack = held

@@ -2,6 +2,7 @@
 one, what it keeps between calls, and the one-pass encoder against its separate kernels, at the sizes where
 tiles, splits, runs and rows end."""
 import copy
+import threading
 
 import pytest
 import torch
@@ -351,8 +352,8 @@ def test_shapes_in_turn_share_weights_and_keep_their_plans(monkeypatch):
     once in all, results are those of a model that sees one shape only, and no more than SHAPES plans are held."""
     model, made, collected = _model(), [], []
     put, collect = MVPFormerModel._set_block, MVPFormerModel._block_operands
-    monkeypatch.setattr(MVPFormerModel, "_set_block", lambda self, held, plan, i, *key:
-                        (made.append(key) if i == 0 else None) or put(self, held, plan, i, *key))
+    monkeypatch.setattr(MVPFormerModel, "_set_block", lambda self, known, new, plan, i, *key:
+                        (made.append(key) if i == 0 else None) or put(self, known, new, plan, i, *key))
     monkeypatch.setattr(MVPFormerModel, "_block_operands", staticmethod(lambda *a: collected.append(a) or collect(*a)))
     xs = [torch.randn(1, t, c, 128, device="cuda").bfloat16() for t, c in ((3, 8), (5, 8), (8, 64), (5, 9), (3, 8))]
     seg = torch.randn(1, 1, 8, 128, device="cuda").bfloat16()
@@ -393,10 +394,10 @@ def test_first_pass_is_the_later_ones(monkeypatch, B, C, T):
             return [model(inputs_embeds=x, past_key_values=caches)[0] for _ in range(2)][-1]
     put = MVPFormerModel._set_block
 
-    def breaks(self, held, plan, i, *key):
+    def breaks(self, known, made, plan, i, *key):
         if i == 3:
             raise MemoryError
-        put(self, held, plan, i, *key)
+        put(self, known, made, plan, i, *key)
     with monkeypatch.context() as m:
         m.setattr(MVPFormerModel, "_set_block", breaks)
         with pytest.raises(MemoryError):
@@ -404,6 +405,61 @@ def test_first_pass_is_the_later_ones(monkeypatch, B, C, T):
     assert model._stack is None
     first = out()
     assert model._stack.plans and torch.equal(first, out())
+
+
+def test_passes_on_several_streams():
+    """Operands made by a pass on one stream, behind a long kernel there, used at once by passes on others; shapes
+    given up while passes on another stream still read them, with their memory taken again on the stream it came
+    from; results are those of one stream."""
+    model = _model(n_layer=3)
+    shapes = [(t, c) for t in (2, 3, 4) for c in (5, 9, 16, 33)]              # more than are kept
+    xs = [torch.randn(1, t, c, 128, device="cuda").bfloat16() for t, c in shapes]
+    with torch.no_grad():
+        want = [copy.deepcopy(model)(inputs_embeds=x) for x in xs]
+        one, two = torch.cuda.Stream(), torch.cuda.Stream()
+        torch.cuda.synchronize()
+        got = []
+        for x in xs + xs[::-1]:
+            with torch.cuda.stream(one):
+                torch.cuda._sleep(2_000_000)
+                got.append(model(inputs_embeds=x))
+            with torch.cuda.stream(two):
+                torch.cuda._sleep(1_000_000)
+                got.append(model(inputs_embeds=x))
+            with torch.cuda.stream(one):
+                dirt = [torch.full((n,), float("nan"), device="cuda") for n in (128, 1 << 10, 1 << 12) for _ in range(8)]
+        torch.cuda.synchronize()
+    del dirt
+    for i, x in enumerate(want + want[::-1]):
+        assert torch.equal(got[2 * i], x) and torch.equal(got[2 * i + 1], x)
+
+
+def test_passes_of_several_threads():
+    """First passes and later ones of four threads, each on a stream of its own."""
+    model = _model(n_layer=3)
+    xs = [torch.randn(1, t, c, 128, device="cuda").bfloat16() for t in (2, 3, 4) for c in (5, 9, 16)]
+    wrong = []
+    with torch.no_grad():
+        want = [copy.deepcopy(model)(inputs_embeds=x) for x in xs]
+        torch.cuda.synchronize()
+
+    def work(k):
+        try:
+            with torch.no_grad(), torch.cuda.stream(torch.cuda.Stream()):
+                for n in range(3 * len(xs)):
+                    i = (n * (k + 1) + k) % len(xs)
+                    out = model(inputs_embeds=xs[i])
+                    torch.cuda.current_stream().synchronize()
+                    if not torch.equal(out, want[i]):
+                        wrong.append((k, n, i))
+        except Exception as e:                               # pytest does not see another thread's
+            wrong.append(e)
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong and len(model._stack.plans) <= _StackOperands.SHAPES
 
 
 def test_adapters_reach_the_stack_call():

@@ -36,7 +36,8 @@ def _through_file(model):
                          ids=["copy", "deepcopy", "pickle", "save"])
 def test_a_model_with_a_plan_is_copied(how):
     model = _model()
-    model._stack = _StackOperands(_capsule())
+    model._stack = _StackOperands()
+    model._stack.watch = _capsule()
     other = how(model)
     assert other._stack is None and model._stack is not None
     assert all(torch.equal(a, b) for a, b in zip(model.state_dict().values(), other.state_dict().values()))
@@ -52,7 +53,8 @@ def test_a_model_saved_without_plans_loads():
 
 def test_a_replica_has_no_plan():
     model = _model()
-    model._stack = _StackOperands(_capsule())
+    model._stack = _StackOperands()
+    model._stack.watch = _capsule()
     replica = model._replicate_for_data_parallel()
     assert replica._stack is None and model._stack is not None
 
