@@ -450,6 +450,22 @@ int mvpa_rmsnorm_backward(const void* x, const void* weight, const void* dy, con
 int mvpa_silu_gate_bf16(const void* gu, void* out, int64_t rows, int32_t n, void* stream);
 int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void* dgu, int64_t rows, int32_t n, void* stream);
 
+/* Stacked projection weights with low-rank adapters (layers/mvpa.py:43-62, 86-93), all bf16 and contiguous:
+ * part i holds rows [row0, row0 + rows) of out [sum of rows, K], w + scale * b a with w [rows, K], a [r, K] and
+ * b [rows, r]; a and b both null: w as it is.  row0 is filled in by the library.  The backward writes da and db
+ * (each nullable) from the gradient of out; w is not read there.  K a multiple of 8; w, a, out and d_out at
+ * 16-byte boundaries.  Sums in fp32, one rounding. */
+#define MVPA_LORA_PARTS 8
+typedef struct mvpa_lora_part {
+  const void *w, *a, *b;
+  void *da, *db;
+  int64_t row0;
+  int32_t rows, reserved0;
+} mvpa_lora_part;
+int mvpa_lora_stack_bf16(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t r, float scale, void* out, void* stream);
+int mvpa_lora_stack_backward_bf16(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t r, float scale,
+                                  const void* d_out, void* stream);
+
 /* ---- the stack of parallel blocks as one call ---------------------------------------------------
  * models/mvpformer.py:296-381: every block x + attn(ln_1(x)) + mlp(ln_1(x)), then ln_f, on bf16 rows.
  * The launches are the library's own (mvpa_forward and the products around it); one call enqueues

@@ -641,6 +641,126 @@ PyObject* py_enqueue(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The parts of stacked projections with adapters: `mods` holds (enable, w, a | None, b | None) per module;
+// equal row slices of a module, each with its share of a and b where enabled.
+struct LoraParts {
+  std::vector<mvpa_lora_part> parts;
+  int64_t rows = 0, K = 0, r = 0;
+};
+bool lora_parts(PyObject* mods, LoraParts& l) {
+  for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
+    PyObject* mod = PyTuple_GET_ITEM(mods, m);
+    PyObject* enable = PyTuple_GET_ITEM(mod, 0);
+    const Tensor& w = tensor_of(PyTuple_GET_ITEM(mod, 1));
+    const bool has = !is_none(PyTuple_GET_ITEM(mod, 2));
+    const int64_t slices = has ? PyTuple_GET_SIZE(enable) : 1, rows = w.size(0) / slices;
+    l.K = w.size(1);
+    int64_t j = 0;
+    for (int64_t i = 0; i < slices; ++i) {
+      mvpa_lora_part p{};
+      p.w = (const char*)w.const_data_ptr() + i * rows * l.K * 2;
+      p.rows = (int32_t)rows;
+      if (has && PyTuple_GET_ITEM(enable, i) == Py_True) {
+        const Tensor &a = tensor_of(PyTuple_GET_ITEM(mod, 2)), &b = tensor_of(PyTuple_GET_ITEM(mod, 3));
+        l.r = b.size(1);
+        TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == l.K && a.size(0) >= (j + 1) * l.r && b.size(0) >= (j + 1) * rows,
+                    "lora_stack: an adapter does not fit its weight");
+        p.a = (const char*)a.const_data_ptr() + j * l.r * l.K * 2;
+        p.b = (const char*)b.const_data_ptr() + j * rows * l.r * 2;
+        ++j;
+      }
+      l.rows += rows;
+      l.parts.push_back(p);
+    }
+  }
+  return l.parts.size() <= MVPA_LORA_PARTS && l.r > 0;
+}
+
+// lora_fits(mods): whether lora_stack takes them
+PyObject* py_lora_fits(PyObject*, PyObject* mods) {
+  HANDLE_TH_ERRORS
+  int64_t K = -1, r = -1, parts = 0;
+  auto bad = [&](PyObject* o) {
+    if (!THPVariable_Check(o)) return true;
+    const Tensor& t = THPVariable_Unpack(o);
+    return !t.is_cuda() || t.scalar_type() != at::kBFloat16 || t.dim() != 2 || !t.is_contiguous() || t.numel() == 0 ||
+           ((uintptr_t)t.const_data_ptr() & 15);
+  };
+  for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
+    PyObject* mod = PyTuple_GET_ITEM(mods, m);
+    PyObject* enable = PyTuple_GET_ITEM(mod, 0);
+    if (bad(PyTuple_GET_ITEM(mod, 1))) Py_RETURN_FALSE;
+    const Tensor& w = THPVariable_Unpack(PyTuple_GET_ITEM(mod, 1));
+    if (w.size(1) % 8 || (K >= 0 && w.size(1) != K)) Py_RETURN_FALSE;
+    K = w.size(1);
+    if (is_none(PyTuple_GET_ITEM(mod, 2))) {
+      ++parts;
+      continue;
+    }
+    if (bad(PyTuple_GET_ITEM(mod, 2)) || bad(PyTuple_GET_ITEM(mod, 3))) Py_RETURN_FALSE;
+    const Tensor &a = THPVariable_Unpack(PyTuple_GET_ITEM(mod, 2)), &b = THPVariable_Unpack(PyTuple_GET_ITEM(mod, 3));
+    const int64_t slices = PyTuple_GET_SIZE(enable);
+    int64_t on = 0;
+    for (int64_t i = 0; i < slices; ++i) on += PyTuple_GET_ITEM(enable, i) == Py_True;
+    if (slices == 0 || on == 0 || w.size(0) % slices || a.size(1) != K || a.size(0) != on * b.size(1) ||
+        b.size(0) != w.size(0) / slices * on || (r >= 0 && b.size(1) != r))
+      Py_RETURN_FALSE;
+    r = b.size(1);
+    parts += slices;
+  }
+  if (r > 0 && parts <= MVPA_LORA_PARTS) Py_RETURN_TRUE;
+  Py_RETURN_FALSE;
+  END_HANDLE_TH_ERRORS
+}
+
+// lora_stack(mods, scale) -> the stacked weight;  lora_stack(mods, scale, d) -> gradients of each module's a
+// and b in turn (None without an adapter) | status
+PyObject* py_lora_stack(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK((n == 2 || n == 3) && PyTuple_Check(args[0]), "lora_stack takes the modules' weights, a scale and, for the backward, a gradient");
+  const double scale = PyFloat_AsDouble(args[1]);
+  if (PyErr_Occurred()) return nullptr;
+  at::AutoDispatchBelowADInplaceOrView guard;
+  LoraParts l;
+  if (!lora_parts(args[0], l)) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  const Tensor& first = tensor_of(PyTuple_GET_ITEM(PyTuple_GET_ITEM(args[0], 0), 1));
+  if (n == 2) {
+    Tensor out = at::empty({l.rows, l.K}, first.options());
+    const int st = mvpa_lora_stack_bf16(l.parts.data(), (int32_t)l.parts.size(), (int32_t)l.K, (int32_t)l.r, (float)scale,
+                                        out.data_ptr(), current_stream());
+    return st == MVPA_OK ? THPVariable_Wrap(out) : PyLong_FromLong(st);
+  }
+  const Tensor d = aligned_operand(tensor_of(args[2]), at::kBFloat16);
+  TORCH_CHECK(d.dim() == 2 && d.size(0) == l.rows && d.size(1) == l.K, "lora_stack: the gradient's shape differs");
+  const Py_ssize_t mods = PyTuple_GET_SIZE(args[0]);
+  std::vector<Tensor> grads(2 * mods);
+  size_t at = 0;
+  for (Py_ssize_t m = 0; m < mods; ++m) {
+    PyObject* mod = PyTuple_GET_ITEM(args[0], m);
+    if (is_none(PyTuple_GET_ITEM(mod, 2))) {
+      ++at;
+      continue;
+    }
+    grads[2 * m] = at::empty_like(tensor_of(PyTuple_GET_ITEM(mod, 2)));
+    grads[2 * m + 1] = at::empty_like(tensor_of(PyTuple_GET_ITEM(mod, 3)));
+    int64_t j = 0;
+    for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(PyTuple_GET_ITEM(mod, 0)); ++i, ++at) {
+      mvpa_lora_part& p = l.parts[at];
+      if (!p.a) continue;
+      p.da = (char*)grads[2 * m].data_ptr() + j * l.r * l.K * 2;
+      p.db = (char*)grads[2 * m + 1].data_ptr() + j * (int64_t)p.rows * l.r * 2;
+      ++j;
+    }
+  }
+  const int st = mvpa_lora_stack_backward_bf16(l.parts.data(), (int32_t)l.parts.size(), (int32_t)l.K, (int32_t)l.r, (float)scale,
+                                               d.data_ptr(), current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* res = PyTuple_New(2 * mods);
+  for (Py_ssize_t i = 0; i < 2 * mods; ++i) PyTuple_SET_ITEM(res, i, THPVariable_Wrap(grads[i]));
+  return res;
+  END_HANDLE_TH_ERRORS
+}
+
 PyMethodDef kMethods[] = {
     {"forward", (PyCFunction)(void*)py_forward, METH_FASTCALL, "fused MVPA forward"},
     {"backward", (PyCFunction)(void*)py_backward, METH_FASTCALL, "backward of the fused MVPA forward, bf16"},
@@ -649,6 +769,8 @@ PyMethodDef kMethods[] = {
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
     {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},
     {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
+    {"lora_fits", (PyCFunction)py_lora_fits, METH_O, "whether lora_stack takes these"},
+    {"lora_stack", (PyCFunction)(void*)py_lora_stack, METH_FASTCALL, "stacked weights with adapters, or the adapters' gradients"},
     {"plan", (PyCFunction)(void*)py_plan, METH_FASTCALL, "operands of a stack of blocks"},
     {"watch", (PyCFunction)(void*)py_watch, METH_FASTCALL, "what a model looks like now"},
     {"watch_current", (PyCFunction)py_watch_current, METH_O, "whether it still looks like that"},

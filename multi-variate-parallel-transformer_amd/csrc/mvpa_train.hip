@@ -152,14 +152,14 @@ __global__ __launch_bounds__(1024) void column_sum_kernel(const float* __restric
   }
 }
 
-__device__ inline void load8(const bf16_t* p, float (&v)[8]) {
-  const u32x4 x = *(const u32x4*)p;
+__device__ inline void unpack8(u32x4 x, float (&v)[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     v[2 * i] = __uint_as_float(x[i] << 16);
     v[2 * i + 1] = __uint_as_float(x[i] & 0xffff0000u);
   }
 }
+__device__ inline void load8(const bf16_t* p, float (&v)[8]) { unpack8(*(const u32x4*)p, v); }
 __device__ inline void store8(bf16_t* p, const float (&v)[8]) {
   *(u32x4*)p = u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
 }
@@ -205,6 +205,164 @@ __global__ __launch_bounds__(256) void silu_gate_backward_kernel(const bf16_t* _
     }
     store8(dgu + row * 2 * n + c, g);
     store8(dgu + row * 2 * n + n + c, u);
+  }
+}
+
+// ---- stacked projection weights with low-rank adapters (layers/mvpa.py:43-62, 86-93) ----------
+// out = [w_0 + scale b_0 a_0; w_1 + ...] over the parts of a projection and the gradients of a and b from that
+// of out.  As tensor expressions a block's pair of projections is ten launches forward and twenty-six
+// backward, none of which moves more than a megabyte: they cost a launch each.  Here one each way, sums in
+// fp32 and one rounding.  Bound by the launch and a chain of loads.  Rank 8 on
+// 1 024 of 1 280 rows of 768: 7.5 and 14 us; the training pass of twelve such blocks went from 13.8 to 11.9 ms.
+struct lora_parts {
+  mvpa_lora_part p[MVPA_LORA_PARTS];
+};
+
+constexpr int LORA_ROWS = 4;         // rows per workgroup of the stacked weight: a's columns are read once for them
+
+// eight terms k0 .. of a row of b; whole rows of 16-byte chunks where VEC, zeros past the rank
+template <bool VEC>
+__device__ inline void lora_b8(const bf16_t* row, int k0, int r, float (&v)[8]) {
+  if (VEC) {
+    load8(row + k0, v);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = k0 + i < r ? bf16_to_f32(row[k0 + i]) : 0.f;
+  }
+}
+
+// a thread takes 8 columns of LORA_ROWS rows; blockIdx.z is the part.  VEC: r a multiple of 8
+template <bool VEC>
+__global__ __launch_bounds__(128) void lora_stack_kernel(lora_parts parts, bf16_t* __restrict__ out, int K, int r, float scale) {
+  const mvpa_lora_part p = parts.p[blockIdx.z];
+  const int row0 = blockIdx.y * LORA_ROWS, c = (blockIdx.x * 128 + threadIdx.x) * 8;
+  if (row0 >= p.rows || c >= K) return;
+  const bf16_t *w = (const bf16_t*)p.w, *a = (const bf16_t*)p.a, *b = (const bf16_t*)p.b;
+  u32x4 wv[LORA_ROWS];               // requested first: the only operand that is not in a cache
+#pragma unroll
+  for (int i = 0; i < LORA_ROWS; ++i) wv[i] = *(const u32x4*)(w + (int64_t)min(row0 + i, p.rows - 1) * K + c);
+  float acc[LORA_ROWS][8];
+#pragma unroll
+  for (int i = 0; i < LORA_ROWS; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+  for (int k0 = 0; a && k0 < r; k0 += 8) {
+    float bv[LORA_ROWS][8];
+#pragma unroll
+    for (int i = 0; i < LORA_ROWS; ++i) lora_b8<VEC>(b + (int64_t)min(row0 + i, p.rows - 1) * r, k0, r, bv[i]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      float av[8];
+      load8(a + (int64_t)min(k0 + k, r - 1) * K + c, av);
+#pragma unroll
+      for (int i = 0; i < LORA_ROWS; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i][j] += bv[i][k] * av[j];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < LORA_ROWS; ++i) {
+    if (row0 + i >= p.rows) break;
+    float v[8];
+    unpack8(wv[i], v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += scale * acc[i][j];
+    store8(out + (p.row0 + row0 + i) * (int64_t)K + c, v);
+  }
+}
+
+// One launch for both gradients of every part: the first (K + 63) / 64 workgroups of a part sum
+// da[k, c] = scale sum_rows b[row, k] d[row, c] over 64 columns each (32 row shares, merged through LDS), the
+// rest take a row per wave for db[row, k] = scale sum_c d[row, c] a[k, c].  Eight of the r terms at a time.
+// b's rows go through LDS, so that what a row costs is one load of d and many of them are in flight: with b
+// read where it is used, 2 bytes at a time, the launch took 47 us.
+constexpr int LORA_B_ROWS = 1024;    // rows of b in LDS at a time
+template <bool VEC>
+__global__ __launch_bounds__(1024) void lora_stack_backward_kernel(lora_parts parts, const bf16_t* __restrict__ d, int K, int r,
+                                                                   float scale) {
+  __shared__ float red[16][8][64];
+  __shared__ __attribute__((aligned(16))) float bs[LORA_B_ROWS][8];
+  const mvpa_lora_part p = parts.p[blockIdx.y];
+  if (!p.a) return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col_groups = (K + 63) / 64;
+  const bf16_t *a = (const bf16_t*)p.a, *b = (const bf16_t*)p.b;
+  d += p.row0 * (int64_t)K;
+  if ((int)blockIdx.x < col_groups) {
+    if (!p.da) return;
+    bf16_t* da = (bf16_t*)p.da;
+    const int c = blockIdx.x * 64 + (lane & 31) * 2, share = wave * 2 + (lane >> 5);
+    for (int k0 = 0; k0 < r; k0 += 8) {
+      float acc[8][2];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) acc[i][0] = acc[i][1] = 0.f;
+      for (int first = 0; first < p.rows; first += LORA_B_ROWS) {
+        const int n = min(p.rows - first, LORA_B_ROWS);
+        __syncthreads();
+        if ((int)threadIdx.x < n) {
+          float v[8];
+          lora_b8<VEC>(b + (int64_t)(first + threadIdx.x) * r, k0, r, v);
+          store4(&bs[threadIdx.x][0], {v[0], v[1], v[2], v[3]});
+          store4(&bs[threadIdx.x][4], {v[4], v[5], v[6], v[7]});
+        }
+        __syncthreads();
+        if (c < K) {
+#pragma unroll 8
+          for (int row = share; row < n; row += 32) {
+            const uint32_t x = *(const uint32_t*)(d + (int64_t)(first + row) * K + c);
+            const float lo = __uint_as_float(x << 16), hi = __uint_as_float(x & 0xffff0000u);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+              acc[i][0] += bs[row][i] * lo;
+              acc[i][1] += bs[row][i] * hi;
+            }
+          }
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] += __shfl_xor(acc[i][j], 32);
+        if (lane < 32) {
+          red[wave][i][lane * 2] = acc[i][0];
+          red[wave][i][lane * 2 + 1] = acc[i][1];
+        }
+      }
+      __syncthreads();
+      const int i = threadIdx.x >> 6, cc = blockIdx.x * 64 + lane;
+      if (threadIdx.x < 512 && k0 + i < r && cc < K) {
+        float s = 0.f;
+#pragma unroll
+        for (int g = 0; g < 16; ++g) s += red[g][i][lane];
+        da[(int64_t)(k0 + i) * K + cc] = f32_to_bf16(scale * s);
+      }
+    }
+    return;
+  }
+  if (!p.db) return;
+  const int row = (blockIdx.x - col_groups) * 16 + wave;
+  if (row >= p.rows) return;
+  bf16_t* db = (bf16_t*)p.db;
+  for (int k0 = 0; k0 < r; k0 += 8) {
+    float acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = 0.f;
+    for (int c = lane * 8; c < K; c += 512) {
+      float x[8];
+      load8(d + (int64_t)row * K + c, x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        float av[8];
+        load8(a + (int64_t)min(k0 + i, r - 1) * K + c, av);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[i] += x[j] * av[j];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float s = wave_sum(acc[i]);
+      if (lane == 0 && k0 + i < r) db[(int64_t)row * r + k0 + i] = f32_to_bf16(scale * s);
+    }
   }
 }
 
@@ -281,5 +439,49 @@ extern "C" int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void*
   if (st != MVPA_OK) return st;
   MVPA_LAUNCH(train::silu_gate_backward_kernel, gate_grid(rows, n), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gu,
               (const bf16_t*)d, (bf16_t*)dgu, rows, n);
+  return take_launch_status();
+}
+
+// the parts' rows follow one another in the stacked weight; *rows: their sum, *most: the largest part
+static int lora_check(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t r, const void* stacked, bool backward,
+                      train::lora_parts& out, int32_t* most) {
+  if (!parts || !stacked) return MVPA_ERR_NULL;
+  if (n <= 0 || n > MVPA_LORA_PARTS || K <= 0 || r <= 0) return MVPA_ERR_SHAPE;
+  if (K % 8 != 0 || ((uintptr_t)stacked & 15)) return MVPA_ERR_ALIGN;
+  int64_t row0 = 0;
+  *most = 0;
+  for (int i = 0; i < n; ++i) {
+    mvpa_lora_part p = parts[i];
+    if (p.rows <= 0 || p.rows > (1 << 24)) return MVPA_ERR_SHAPE;
+    if ((!backward && !p.w) || !p.a != !p.b) return MVPA_ERR_NULL;
+    if ((((uintptr_t)p.a | (uintptr_t)p.b) & (r % 8 == 0 ? 15 : 1)) || ((uintptr_t)p.a & 15) || (!backward && ((uintptr_t)p.w & 15))) return MVPA_ERR_ALIGN;
+    p.row0 = row0;
+    row0 += p.rows;
+    if (p.rows > *most) *most = p.rows;
+    out.p[i] = p;
+  }
+  return MVPA_OK;
+}
+
+extern "C" int mvpa_lora_stack_bf16(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t r, float scale, void* out,
+                                    void* stream) {
+  train::lora_parts args;
+  int32_t most;
+  const int st = lora_check(parts, n, K, r, out, false, args, &most);
+  if (st != MVPA_OK) return st;
+  MVPA_LAUNCH(r % 8 == 0 ? train::lora_stack_kernel<true> : train::lora_stack_kernel<false>,
+              dim3((unsigned)((K + 1023) / 1024), (unsigned)((most + train::LORA_ROWS - 1) / train::LORA_ROWS), (unsigned)n), dim3(128),
+              0, (hipStream_t)stream, args, (bf16_t*)out, K, r, scale);
+  return take_launch_status();
+}
+
+extern "C" int mvpa_lora_stack_backward_bf16(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t r, float scale,
+                                             const void* d_out, void* stream) {
+  train::lora_parts args;
+  int32_t most;
+  const int st = lora_check(parts, n, K, r, d_out, true, args, &most);
+  if (st != MVPA_OK) return st;
+  MVPA_LAUNCH(r % 8 == 0 ? train::lora_stack_backward_kernel<true> : train::lora_stack_backward_kernel<false>, dim3((unsigned)((K + 63) / 64 + (most + 15) / 16), (unsigned)n), dim3(1024), 0,
+              (hipStream_t)stream, args, (const bf16_t*)d_out, K, r, scale);
   return take_launch_status();
 }

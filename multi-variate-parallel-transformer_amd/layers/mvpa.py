@@ -204,6 +204,20 @@ def _weight_of(mod) -> torch.Tensor:
     return mod.effective_weight() if isinstance(mod, _LoRALinear) else mod.weight
 
 
+def _stacked_weights(mods) -> torch.Tensor:
+    """The modules' weights, adapters included, stacked by rows, differentiably: one kernel each way where
+    adapters are in play (mvpa_hip.autograd.lora_stack), tensor operations for other types and classes."""
+    from mvpa_hip import autograd as AG
+    tuned = [m for m in mods if isinstance(m, _LoRALinear) and m.r > 0 and hasattr(m, "lora_A")]
+    if (tuned and all(type(m) in (_LoRALinear, torch.nn.Linear) and "effective_weight" not in m.__dict__ for m in mods)
+            and all(m.scaling == tuned[0].scaling for m in tuned) and mods[0].weight.is_cuda):
+        w = AG.lora_stack(tuple((m.enable, m.weight, m.lora_A, m.lora_B) if m in tuned else ((), m.weight, None, None)
+                                for m in mods), float(tuned[0].scaling))
+        if w is not None:
+            return w
+    return torch.cat([_weight_of(m) for m in mods], 0)
+
+
 def _linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """GPU tensors go through the library's MFMA GEMMs, bf16 or fp32."""
     if x.is_cuda and x.dtype == torch.bfloat16:
@@ -434,7 +448,7 @@ class MVPFormerGQAAttention(torch.nn.Module):
         h, hkv, dh, kv = self.num_heads, self.num_kv_heads, self.head_dim, self.embed_kv_dim
         n = t_len * c_len
         dt = hidden_states.dtype
-        w_qkv = torch.cat([_weight_of(self.q_attn), _weight_of(self.c_attn)], 0)
+        w_qkv = _stacked_weights((self.q_attn, self.c_attn))
         qkv = AG.linear(hidden_states, w_qkv).reshape(bsz, n, e + 2 * kv)
         q = qkv[:, :, :e].reshape(bsz, n, h, dh).permute(0, 2, 1, 3)
         k = qkv[:, :, e:e + kv].reshape(bsz, n, hkv, dh).permute(0, 2, 1, 3)

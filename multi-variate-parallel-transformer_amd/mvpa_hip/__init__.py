@@ -549,6 +549,13 @@ def silu_gate(gu: torch.Tensor, d: Optional[torch.Tensor] = None) -> torch.Tenso
     return _taken(ext.silu_gate(gu) if d is None else ext.silu_gate(gu, d))
 
 
+def lora_stack(mods, scale: float, d: Optional[torch.Tensor] = None):
+    """Stacked weights of modules ((enable, w, a | None, b | None), ..) with their adapters added; with d, the
+    gradients of each module's a and b (in turn) for the gradient d of that."""
+    ext = _ext or load_ext()
+    return _taken(ext.lora_stack(mods, scale) if d is None else ext.lora_stack(mods, scale, d))
+
+
 def mean_rows(x: torch.Tensor) -> torch.Tensor:
     """Mean over dim 1 of a bf16 [groups, rows, cols] tensor (unit last stride, cols a multiple of 8)
     in fp32, rounded to bf16."""

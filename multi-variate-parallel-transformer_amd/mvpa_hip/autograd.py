@@ -173,3 +173,48 @@ class _SiluGateFn(torch.autograd.Function):
 def gated_mid(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     """silu(x @ gate^T) * (x @ up^T) for w_gate_up = [gate; up]: one product, one pass over its result."""
     return _SiluGateFn.apply(linear(x, w_gate_up))
+
+
+class _LoRAStackFn(torch.autograd.Function):
+    """Weights of several modules, adapters added, stacked by rows; one launch each way.  tensors: w, a, b of
+    each module in turn, a and b None where it has no adapter."""
+
+    @staticmethod
+    def forward(ctx, scale, enables, *tensors):
+        ctx.conf = scale, enables, [w.shape[0] for w in tensors[::3]]
+        ctx.save_for_backward(*(t for i, t in enumerate(tensors) if i % 3))       # w is not needed again
+        return mvpa_hip.lora_stack(_lora_mods(enables, tensors[::3], tensors[1::3], tensors[2::3]), scale)
+
+    @staticmethod
+    def backward(ctx, d):
+        scale, enables, rows = ctx.conf
+        a, b = ctx.saved_tensors[::2], ctx.saved_tensors[1::2]
+        dw = d.split(rows)
+        needs = ctx.needs_input_grad[2:]
+        adapters = [None] * (2 * len(rows))
+        if torch.is_grad_enabled():                          # a backward that is differentiated itself
+            for m, (on, am, bm) in enumerate(zip(enables, a, b)):
+                if am is None:
+                    continue
+                n, r = rows[m] // len(on), bm.shape[1]
+                parts = [dw[m][i * n:(i + 1) * n] * scale for i, e in enumerate(on) if e]
+                adapters[2 * m] = torch.cat([bm[j * n:(j + 1) * n].t() @ x for j, x in enumerate(parts)], 0)
+                adapters[2 * m + 1] = torch.cat([x @ am[j * r:(j + 1) * r].t() for j, x in enumerate(parts)], 0)
+        elif any(needs[1::3]) or any(needs[2::3]):
+            adapters = mvpa_hip.lora_stack(_lora_mods(enables, dw, a, b), scale, d)
+        grads = []
+        for m in range(len(rows)):
+            grads += [dw[m], adapters[2 * m], adapters[2 * m + 1]]
+        return (None, None, *(g if n else None for g, n in zip(grads, needs)))
+
+
+def _lora_mods(enables, w, a, b):
+    return tuple(zip(enables, w, a, b))
+
+
+def lora_stack(mods, scale: float):
+    """cat([w + scale * b a over the enabled slices], 0) for mods = ((enable, w, a, b), ..), a and b None where a
+    module has no adapter; None where they are not contiguous bf16 matrices on the GPU at 16-byte boundaries."""
+    if not mvpa_hip.load_ext().lora_fits(mods):
+        return None
+    return _LoRAStackFn.apply(scale, tuple(m[0] for m in mods), *(t for m in mods for t in m[1:]))

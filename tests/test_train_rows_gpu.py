@@ -153,3 +153,62 @@ def _near(got, ref):
     """The general path rounds the sum of three twice: half a unit of 2^-8, 0.11 % rms of a part of the sum, and
     the gradients, of the same size each, are rounded to bf16 on both sides: 0.4 % in all, of two blocks twice that."""
     assert ((got.double() - ref.double()).norm() / ref.double().norm()).item() <= 1e-2
+
+
+# ranks around the eight that are summed together; columns around the 64 of a workgroup and the 1024 of a row's
+# threads; rows around the 8 and the 32 shares; a slice without an adapter, a module without any
+@pytest.mark.parametrize("r,cols,rows", [(1, 8, (1, 2)), (8, 768, (96, 64)), (9, 72, (33, 66)), (16, 1032, (8, 10)),
+                                         (20, 2048, (64, 4))])
+def test_stacked_weights_with_adapters(r, cols, rows):
+    g = torch.Generator(device="cuda").manual_seed(r * cols)
+
+    def rn(*s):
+        return torch.randn(s, generator=g, device="cuda").bfloat16().requires_grad_(True)
+    scale = 0.375
+    mods = [((True,), rn(rows[0], cols), rn(r, cols), rn(rows[0], r)),
+            ((False, True), rn(rows[1], cols), rn(r, cols), rn(rows[1] // 2, r)), ((), rn(3, cols), None, None),
+            ((True, False, True), rn(6, cols), rn(2 * r, cols), rn(4, r))]
+    d = torch.randn((sum(m[1].shape[0] for m in mods), cols), generator=g, device="cuda").bfloat16()
+    leaves = [t for m in mods for t in m[1:] if t is not None]
+    w = AG.lora_stack(tuple(mods), scale)
+    grads = torch.autograd.grad(w, leaves, d)
+    ref = []
+    for on, wm, a, b in mods:
+        x = wm.detach().double().requires_grad_(True)
+        y = x.clone()
+        if a is not None:
+            a, b, n = a.detach().double().requires_grad_(True), b.detach().double().requires_grad_(True), wm.shape[0] // len(on)
+            at = [i for i, e in enumerate(on) if e]
+            y = torch.cat([y[i * n:(i + 1) * n] + (scale * b[at.index(i) * n:][:n] @ a[at.index(i) * r:][:r] if i in at else 0)
+                           for i in range(len(on))], 0)
+        ref.append((y, [t for t in (x, a, b) if t is not None]))
+    whole = torch.cat([y for y, _ in ref], 0)
+    _close(w.detach(), whole.detach(), r)
+    for got, want in zip(grads, torch.autograd.grad(whole, [t for _, ts in ref for t in ts], d.double())):
+        _close(got, want, max(max(rows), cols))
+
+
+def test_stacked_weights_that_the_kernel_refuses():
+    from layers.mvpa import _LoRALinear, _stacked_weights
+    mod = _LoRALinear(20, 6, 2, 4, enable=(False, True)).to("cuda", torch.bfloat16)     # rows of 20: no whole chunks
+    with torch.no_grad():
+        mod.lora_B.normal_()
+    plain = torch.nn.Linear(20, 4, bias=False).to("cuda", torch.bfloat16)
+    assert AG.lora_stack(((mod.enable, mod.weight, mod.lora_A, mod.lora_B),), 2.0) is None
+    w = _stacked_weights((mod, plain))
+    assert torch.equal(w, torch.cat([mod.effective_weight(), plain.weight], 0))
+    w.sum().backward()
+    assert mod.lora_B.grad.abs().sum() > 0
+
+
+def test_stacked_weights_differentiate_twice():
+    torch.manual_seed(3)
+    w, a, b = (torch.randn(s, device="cuda").bfloat16().requires_grad_(True) for s in ((16, 32), (8, 32), (8, 8)))
+    y = AG.lora_stack((((False, True), w, a, b),), 0.5)
+    da, = torch.autograd.grad(y.float().pow(2).sum(), a, create_graph=True)
+    grad, = torch.autograd.grad(da.float().sum(), b)
+    wd, ad, bd = (t.detach().double().requires_grad_(True) for t in (w, a, b))
+    yd = torch.cat([wd[:8], wd[8:] + 0.5 * bd @ ad], 0)
+    dd, = torch.autograd.grad(yd.pow(2).sum(), ad, create_graph=True)
+    ref, = torch.autograd.grad(dd.sum(), bd)
+    assert ((grad.double() - ref).norm() / ref.norm()).item() <= 3e-2
