@@ -6,15 +6,18 @@
 //     d k_time[j] = sum_rows G_time[:, j] (q + v),   d k_chan likewise with z
 //     dv          = sum_rows G_time k_time = (column sums of G_time) k_time,  dz likewise,  du = sum_rows dq_content
 // As tensor operations this is some twenty passes over the largest tensors of the backward (casts, two
-// batched products each way, sums: 0.85 ms beside 1.7 ms of kernels at B4 H16 C64 T128).  Here G is read
-// twice, once by rows and once by columns, and nothing of its size is written:
-//   finish_rows     128 query rows per workgroup: products with the tables on MFMA, dq to bf16 where the
-//                   caller wants it, partial column sums of dq_content
-//   finish_tables   128 table rows per workgroup over a share of the query rows: G^T q on MFMA (both
-//                   operands by transposing LDS reads), column sums of G; fp32 partial results
+// batched products each way, sums: 0.85 ms beside 1.7 ms of kernels at B4 H16 C64 T128).  Here nothing of G's size
+// is written, and G is read
+//   once, by finish_fused (below), where the sums of all table rows fit the registers of a workgroup: up to 640
+//   columns of both tables, each rounded up to 64, at Dh 64 and 256 at Dh 128;
+//   else twice:
+//     finish_rows     128 query rows per workgroup: products with the tables on MFMA, dq to bf16 where the
+//                     caller wants it, partial column sums of dq_content
+//     finish_tables   128 table rows per workgroup over a share of the query rows: G^T q on MFMA (both
+//                     operands by transposing LDS reads), column sums of G; fp32 partial results
 //   finish_reduce   the partial results to dk_time, dk_chan; finish_biases: du, dv, dz
-// Columns of G_time that the causal mask empties (j < T-1-tq) are skipped in both.  HBM bound: 0.45 ms at that
-// size (rows 187 us, tables 189, dk and dv 60), G being 400 MB.
+// Columns of G_time that the causal mask empties (j < T-1-tq) are skipped.  HBM bound: at that size, G being
+// 400 MB of which 270 are read, 148 us in one read (3.6 TB/s with dq and q) and 187 + 189 in two; dk and dv 60.
 #include "mvpa_mfma_tools.h"
 
 namespace mvpa {
@@ -37,6 +40,7 @@ struct fin_args {
   bf16_t *du, *dvb, *dz, *dk_time, *dk_chan;
   int32_t kv_parts;                  // query heads whose partial dk, dv make one kv head's (1: summed already)
   int32_t tj_t, tj_c, n_split, split_len;   // column tiles of the two tables; row shares and their length
+  int32_t fused;                     // finish_fused: n_split workgroups a head
 };
 
 // four consecutive fp32 of a table-gradient row as bf16; zeros past the end
@@ -276,21 +280,259 @@ __global__ __launch_bounds__(256) void finish_tables_kernel(fin_args a) {
   }
 }
 
-// one workgroup per 256 / DH table rows of a kv head
+// ---- both products of G in one read ------------------------------------------------------------
+// A workgroup walks row tiles of one (b, h), `n_split` apart so that long and short rows of the causal mask are
+// dealt evenly, and keeps the fp32 table sums of ALL columns in registers over them: 16 a lane and step of 64
+// columns at Dh 64.  Per row tile and step a tile of G goes through LDS once, as bf16, and is read there twice:
+// by rows for dq^T += table^T G^T and by columns for the tables' G^T q.  The next tile of G is in flight
+// meanwhile, and a second workgroup on the CU covers the barriers.
+constexpr int FR = 128, FC = 64;     // rows of a tile, columns of a step
+
+// chunk swizzle of G rows of 128 bytes: 16 consecutive rows at one chunk (rows) and 8 rows x 4 chunks
+// (transposing reads) both spread over all banks
+__device__ inline int swz_g(int row) { return (((row >> 1) & 1) << 2) | ((row >> 2) & 3); }
+
+template <int DH, int MAXS>
+__global__ __launch_bounds__(256, DH == 64 && MAXS <= 4 ? 2 : 1) void finish_fused_kernel(fin_args a) {
+  constexpr int MT = DH / 32, NT = MT / 2, ROWB = DH * 2, CPR = DH / 8, QL = FR * CPR / 256, GB = FC * 2;
+  constexpr int C4 = DH / 4, CI = 32 * C4 / 64;      // float4 columns of a row; a lane's rows of its wave's 32
+  constexpr bool EARLY = MAXS <= 4;                  // the content is requested a tile ahead where registers allow it
+  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  // G, under the staged fp32 rows of dq; q; the rows of both tables, steps side by side
+  unsigned char *Gs = smem, *Qs = smem + FR * DH * 4, *Ts = Qs + FR * ROWB;
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int split = blockIdx.x, bh = blockIdx.y, b = bh / a.H, h = bh % a.H, g = h / (a.H / a.Hkv);
+  const int time_steps = (a.T + FC - 1) / FC, s_end = a.gc ? time_steps + (a.C + FC - 1) / FC : time_steps;
+  const int tiles = (a.N + FR - 1) / FR;
+  const int64_t rbase = (int64_t)bh * a.N;
+  const bf16_t* qbase = a.q + b * a.q_sb + h * a.q_sh;
+  const int c16 = tid & 15, gr = tid >> 4;         // this thread's four columns of a step, its rows gr + 16 i
+  // first step of a row tile: columns of G_time below T-1-tq are empty
+  auto first_step = [&](int tile) {
+    const int tq_hi = min(tile * FR + FR - 1, a.N - 1) / a.C;
+    return a.gt ? (a.T - 1 - tq_hi) / FC : time_steps;
+  };
+  float4 gv[FR / 16];
+  // the tile's part of G for step s
+  auto request = [&](int tile, int s) {
+    const bool chan = s >= time_steps;
+    const int cols = chan ? a.C : a.T, j0 = (chan ? s - time_steps : s) * FC, j = j0 + c16 * 4;
+    const float* G = (chan ? a.gc : a.gt) + (rbase + tile * FR) * cols + j0;
+    const int rows = a.N - tile * FR;
+    const uint32_t off = gr * cols + c16 * 4;
+    if ((cols & 3) == 0) {
+#pragma unroll
+      for (int i = 0; i < FR / 16; ++i) {
+        gv[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (gr + 16 * i < rows && j < cols) gv[i] = *(const float4*)(G + (int64_t)16 * i * cols + off);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < FR / 16; ++i) {
+        const float* p = G + (int64_t)16 * i * cols + off;
+        const bool on = gr + 16 * i < rows;
+        gv[i].x = on && j < cols ? p[0] : 0.f;
+        gv[i].y = on && j + 1 < cols ? p[1] : 0.f;
+        gv[i].z = on && j + 2 < cols ? p[2] : 0.f;
+        gv[i].w = on && j + 3 < cols ? p[3] : 0.f;
+      }
+    }
+  };
+  // its rows of q, straight to LDS
+  const uint32_t q_lds = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))Qs;
+  auto request_q = [&](int tile) {
+#pragma unroll
+    for (int i = 0; i < QL; ++i) {
+      const int c = i * 256 + tid, r = c / CPR, ch = (c % CPR) ^ swz_v<DH>(r);
+      load_to_lds_16(qbase + (int64_t)min(tile * FR + r, a.N - 1) * a.q_sn + ch * 8,           // G is 0 past the end
+                     __builtin_amdgcn_readfirstlane(q_lds + (i * 256 + wave * 64) * 16));
+    }
+  };
+  for (int c = tid; c < s_end * FC * CPR; c += 256) {
+    const int r = c / CPR, ch = c % CPR;
+    const bool chan = r >= time_steps * FC;
+    const int j = chan ? r - time_steps * FC : r, cols = chan ? a.C : a.T;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (j < cols) v = *(const u32x4*)((chan ? a.k_chan : a.k_time) + ((int64_t)g * cols + j) * DH + ch * 8);
+    *(u32x4*)(Ts + r * ROWB + ((ch ^ swz_v<DH>(r)) << 4)) = v;
+  }
+  f32x16 tab[MAXS][NT];
+  float cs[MAXS][4];
+  float4 dus = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+  for (int s = 0; s < MAXS; ++s) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) tab[s][t][i] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) cs[s][i] = 0.f;
+  }
+  const int jt = wave & 1, dt = (wave >> 1) * NT;    // this wave's columns of a step and rows of the table sums' transpose
+  // Addresses in LDS: every swizzle has a period of 16 rows, so that rows 16 i on are constants away.
+  // G is written with the four-column groups of 16 in the order 0 2 1 3, so that a lane's 8 operand elements of
+  // a row are together.
+  const int col_w = ((c16 & 12) | ((c16 & 1) << 1) | ((c16 >> 1) & 1)) * 4;
+  unsigned char* const g_write = Gs + gr * GB + (((col_w >> 3) ^ swz_g(gr)) << 4) + ((col_w & 4) << 1);
+  const unsigned char* const g_row = Gs + (wave * 32 + ln) * GB;
+  const int g_chunk = (hh ^ swz_g(ln)) << 4;
+  const int tr_row = 4 * hh + ((ln & 15) >> 2), tr_chunk = 4 * jt + 2 * (ln >> 4) + ((ln & 3) >> 1);
+  const unsigned char* const g_lo = Gs + tr_row * GB + ((ln & 1) << 3) + ((tr_chunk ^ swz_g(tr_row)) << 4);
+  const unsigned char* const g_hi = Gs + (tr_row + 8) * GB + ((ln & 1) << 3) + ((tr_chunk ^ swz_g(tr_row + 8)) << 4);
+  int s = 0, tile = split;
+  if (tile < tiles) {
+    s = first_step(tile);
+    request_q(tile);
+    if (s < s_end) request(tile, s);
+  }
+#pragma unroll 1
+  while (tile < tiles) {
+    // the content share of the wave's rows, a lane four columns of every 64 / C4-th of them
+    float4 cont[CI];
+    auto request_content = [&]() {
+#pragma unroll
+      for (int i = 0; i < CI; ++i) {
+        const int row = tile * FR + wave * 32 + i * (64 / C4) + lane / C4;
+        cont[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (row < a.N) cont[i] = *(const float4*)(a.dq + (rbase + row) * DH + lane % C4 * 4);
+      }
+    };
+    if (EARLY) request_content();
+    f32x16 acc[MT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mt][i] = 0.f;
+    const int next = tile + gridDim.x, next_s = next < tiles ? first_step(next) : s_end;
+    bool fresh = true;
+#pragma unroll 1
+    for (; s < s_end; ++s) {
+      __syncthreads();                               // everyone is done with the tiles before
+#pragma unroll
+      for (int i = 0; i < FR / 16; ++i)
+        *(bf16x4*)(g_write + i * 16 * GB) = bf16x4{(__bf16)gv[i].x, (__bf16)gv[i].y, (__bf16)gv[i].z, (__bf16)gv[i].w};
+#pragma unroll
+      for (int ss = 0; ss < MAXS; ++ss)
+        if (s == ss)
+#pragma unroll
+          for (int i = 0; i < FR / 16; ++i) {
+            cs[ss][0] += gv[i].x; cs[ss][1] += gv[i].y; cs[ss][2] += gv[i].z; cs[ss][3] += gv[i].w;
+          }
+      if (fresh) wait_vmcnt_imm<0>();                // q is in LDS
+      fresh = false;
+      __syncthreads();
+      {
+        const bool more = s + 1 < s_end;
+        if (more || next_s < s_end) request(more ? tile : next, more ? s + 1 : next_s);
+      }
+      const unsigned char* tab_rows = Ts + s * FC * ROWB;
+#pragma unroll
+      for (int k = 0; k < FC / 16; ++k) {
+        const bf16x8 gf = *(const bf16x8*)(g_row + (g_chunk ^ (k << 5)));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+          acc[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_tile<DH>::frag(tab_rows, k, mt, lane), gf, acc[mt], 0, 0, 0);
+      }
+#pragma unroll
+      for (int ss = 0; ss < MAXS; ++ss)
+        if (s == ss) {
+#pragma unroll
+          for (int k = 0; k < FR / 16; ++k) {
+            const bf16x4 lo = el_bf16::read_tr(g_lo + k * 16 * GB), hi = el_bf16::read_tr(g_hi + k * 16 * GB);
+            const bf16x8 gf = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+              tab[ss][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gf, tr_tile<DH>::frag(Qs, k, dt + t, lane), tab[ss][t], 0, 0, 0);
+          }
+        }
+    }
+    if (fresh && next_s < s_end) request(next, next_s);      // nothing to multiply here
+    // dq = content share + table shares: the latter go by rows through LDS, over G and q
+    if (!EARLY) request_content();
+    __syncthreads();
+    if (next < tiles) request_q(next);
+    unsigned char* st = smem + wave * 32 * ROWB * 2;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4)
+        *(float4*)(st + ln * ROWB * 2 + (((8 * mt + 2 * a4 + hh) ^ (ln & (C4 - 1))) << 4)) =
+            make_float4(acc[mt][a4 * 4], acc[mt][a4 * 4 + 1], acc[mt][a4 * 4 + 2], acc[mt][a4 * 4 + 3]);
+    wave_lds_sync();
+#pragma unroll
+    for (int i = 0; i < CI; ++i) {
+      const int r = i * (64 / C4) + lane / C4, row = tile * FR + wave * 32 + r;
+      const float4 v = *(const float4*)(st + r * ROWB * 2 + (((lane % C4) ^ (r & (C4 - 1))) << 4)), c = cont[i];
+      dus.x += c.x; dus.y += c.y; dus.z += c.z; dus.w += c.w;
+      if (row < a.N)
+        *(bf16x4*)(a.dq_out + b * a.dq_sb + h * a.dq_sh + (int64_t)row * a.dq_sn + lane % C4 * 4) =
+            bf16x4{(__bf16)(c.x + v.x), (__bf16)(c.y + v.y), (__bf16)(c.z + v.z), (__bf16)(c.w + v.w)};
+    }
+    tile = next;
+    s = next_s;
+  }
+  const int64_t part = (int64_t)bh * gridDim.x + split, rows = a.T + a.C;
+  float* P = a.p_tab + part * rows * DH;
+  float* red = (float*)smem;
+#pragma unroll
+  for (int ss = 0; ss < MAXS; ++ss) {
+    const bool chan = ss >= time_steps;
+    const int cols = chan ? a.C : a.T, j0 = (chan ? ss - time_steps : ss) * FC, row0 = chan ? a.T : 0;
+    if (j0 >= cols) continue;
+    // rows of the MFMA tile are LDS columns: undo the order of the four-column groups
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int j = j0 + jt * 32 + (i >> 3) * 16 + hh * 8 + ((i >> 2) & 1) * 4 + (i & 3);
+        if (j < cols) P[(int64_t)(row0 + j) * DH + (dt + t) * 32 + ln] = tab[ss][t][i];
+      }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[gr * FC + c16 * 4 + i] = cs[ss][i];
+    __syncthreads();
+    if (tid < FC && j0 + tid < cols) {
+      float sum = 0.f;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) sum += red[i * FC + tid];
+      a.p_col[part * rows + row0 + j0 + tid] = sum;
+    }
+  }
+  __syncthreads();
+  *(float4*)(red + (tid / C4) * DH + tid % C4 * 4) = dus;
+  __syncthreads();
+  if (tid < DH) {
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 256 / C4; ++i) sum += red[i * DH + tid];
+    a.p_du[part * DH + tid] = sum;
+  }
+}
+
+// one workgroup per table row of a kv head, its threads' 256 / DH shares of the partial results merged through LDS
+// (B4 C64 T25 H12/4, 336 parts: 14.6 -> 6 us against a share of one thread)
 template <int DH>
 __global__ __launch_bounds__(256) void finish_reduce_kernel(fin_args a) {
-  const int g = blockIdx.y, rows = a.T + a.C, j = blockIdx.x * (256 / DH) + threadIdx.x / DH, d = threadIdx.x % DH;
-  if (j >= rows) return;
-  const int grp = a.H / a.Hkv;
+  constexpr int SHARES = 256 / DH;
+  __shared__ float red[256], redc[SHARES];
+  const int g = blockIdx.y, rows = a.T + a.C, j = blockIdx.x, d = threadIdx.x % DH, share = threadIdx.x / DH;
+  const int grp = a.H / a.Hkv, np = grp * a.n_split;
   float s = 0.f, c = 0.f;
-  for (int b = 0; b < a.B; ++b) {
-    const int64_t p0 = ((int64_t)b * a.H + g * grp) * a.n_split;
-    const int np = grp * a.n_split;
-#pragma unroll 4
-    for (int p = 0; p < np; ++p) {
-      s += a.p_tab[((p0 + p) * rows + j) * DH + d];
-      c += a.p_col[(p0 + p) * rows + j];
-    }
+#pragma unroll 8
+  for (int i = share; i < a.B * np; i += SHARES) {
+    const int b = i / np, p = (b * a.H + g * grp) * a.n_split + i % np;
+    s += a.p_tab[((int64_t)p * rows + j) * DH + d];
+    c += a.p_col[(int64_t)p * rows + j];
+  }
+  red[threadIdx.x] = s;
+  if (d == 0) redc[share] = c;
+  __syncthreads();
+  if (share > 0) return;
+#pragma unroll
+  for (int i = 1; i < SHARES; ++i) {
+    s += red[i * DH + d];
+    c += redc[i];
   }
   const bool chan = j >= a.T;
   s += c * bf16_to_f32((chan ? a.bias_z : a.bias_v)[g * DH + d]);
@@ -358,6 +600,12 @@ static bool per_head(const mvpa_bwd_args* b) {
   return b->H > b->Hkv && (int64_t)b->B * b->Hkv * ((b->T + 3) / 4) < KEY_GROUPS_FULL;
 }
 
+// steps of 64 columns that finish_fused keeps sums for, 0 where they do not fit the registers
+static int fused_steps(const mvpa_bwd_args* b) {
+  const int steps = (b->T + FC - 1) / FC + (b->C + FC - 1) / FC;
+  return steps <= 4 ? 4 : steps <= 10 && b->Dh == 64 ? 10 : 0;
+}
+
 static void lay_out(const mvpa_bwd_args* b, fin_args& f, mvpa_bwd_args& w, layout& l) {
   const int64_t N = (int64_t)b->T * b->C, bhn = (int64_t)b->B * b->H * N, bgn = (int64_t)b->B * b->Hkv * N, Dh = b->Dh;
   w = *b;
@@ -371,14 +619,23 @@ static void lay_out(const mvpa_bwd_args* b, fin_args& f, mvpa_bwd_args& w, layou
   w.ws_time = l.take<float>(bhn * b->T);
   w.ws_chan = l.take<float>(bhn * ((b->C + 3) / 4 * 4));
   w.ws_qu = l.take<bf16_t>(bhn * Dh);
-  int n_split, len;
-  row_split(b, &n_split, &len);
+  const int64_t row_tiles = (N + ROWS - 1) / ROWS;
+  f.fused = fused_steps(b);
+  int n_split, len = 0;
+  if (f.fused) {
+    const int64_t s = (Dh == 64 && f.fused == 4 ? 512 : 256) / ((int64_t)b->B * b->H);    // two workgroups a CU, one at Dh 128
+    // as few as walk no more tiles each: 13 tiles take two rounds with 12 workgroups and with 7
+    const int64_t each = s < 1 ? row_tiles : (row_tiles + s - 1) / s;
+    n_split = (int)((row_tiles + each - 1) / each);
+  } else {
+    row_split(b, &n_split, &len);
+  }
   f.n_split = n_split;
   f.split_len = len;
   f.tj_t = (b->T + TJ - 1) / TJ;
   f.tj_c = (b->C + TJ - 1) / TJ;
   const int64_t parts = (int64_t)b->B * b->H * n_split, rows = b->T + b->C;
-  f.p_du = l.take<float>((int64_t)b->B * b->H * ((N + ROWS - 1) / ROWS) * Dh);
+  f.p_du = l.take<float>((int64_t)b->B * b->H * row_tiles * Dh);
   f.p_tab = l.take<float>(parts * rows * Dh);
   f.p_col = l.take<float>(parts * rows);
   f.csum = l.take<float>(b->Hkv * rows);
@@ -386,13 +643,22 @@ static void lay_out(const mvpa_bwd_args* b, fin_args& f, mvpa_bwd_args& w, layou
 
 template <int DH>
 static int launch_finish(const fin_args& f, hipStream_t s) {
-  const int row_tiles = (f.N + ROWS - 1) / ROWS;
-  MVPA_LAUNCH(finish_rows_kernel<DH>, dim3((unsigned)row_tiles, (unsigned)(f.B * f.H)), dim3(256), 0, s, f);
-  MVPA_LAUNCH(finish_tables_kernel<DH>, dim3((unsigned)(f.tj_t + f.tj_c), (unsigned)f.n_split, (unsigned)(f.B * f.H)),
-              dim3(256), 0, s, f);
+  const int row_tiles = f.fused ? f.n_split : (f.N + ROWS - 1) / ROWS;
+  if (f.fused) {
+    const size_t lds = (size_t)FR * DH * 6 +
+                       (size_t)((f.T + FC - 1) / FC + (f.C + FC - 1) / FC) * FC * DH * 2;
+    auto kern = finish_fused_kernel<DH, 4>;
+    if constexpr (DH == 64) kern = f.fused == 10 ? finish_fused_kernel<64, 10> : kern;
+    want_dynamic_lds((const void*)kern, (int)lds);
+    MVPA_LAUNCH(kern, dim3((unsigned)f.n_split, (unsigned)(f.B * f.H)), dim3(256), lds, s, f);
+  } else {
+    MVPA_LAUNCH(finish_rows_kernel<DH>, dim3((unsigned)row_tiles, (unsigned)(f.B * f.H)), dim3(256), 0, s, f);
+    MVPA_LAUNCH(finish_tables_kernel<DH>, dim3((unsigned)(f.tj_t + f.tj_c), (unsigned)f.n_split, (unsigned)(f.B * f.H)),
+                dim3(256), 0, s, f);
+  }
   const int64_t kv = 2 * (int64_t)f.B * f.Hkv * f.N * (DH / 8);
   MVPA_LAUNCH(finish_kv_kernel<DH>, dim3((unsigned)((kv + 255) / 256)), dim3(256), 0, s, f);
-  MVPA_LAUNCH(finish_reduce_kernel<DH>, dim3((unsigned)((f.T + f.C + 256 / DH - 1) / (256 / DH)), (unsigned)f.Hkv), dim3(256), 0, s, f);
+  MVPA_LAUNCH(finish_reduce_kernel<DH>, dim3((unsigned)(f.T + f.C), (unsigned)f.Hkv), dim3(256), 0, s, f);
   MVPA_LAUNCH(finish_biases_kernel<DH>, dim3((unsigned)f.Hkv, 3), dim3(1024), 0, s, f, row_tiles);
   return take_launch_status();
 }

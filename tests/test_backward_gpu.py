@@ -318,3 +318,54 @@ def test_long_walks_against_the_fp32_kernels(T, C, Dh, window, masked):
         return torch.autograd.grad(out, leaves, d.to(dtype))
     for n, x, y in zip(NAMES, grads(torch.bfloat16), grads(torch.float32)):
         assert (x.double() - y.double()).norm() <= 2e-2 * y.double().norm(), n      # the bf16 bound of this file
+
+
+@pytest.mark.parametrize("cfg,flags", [
+    (dict(B=1, C=1, T=1, H=2, Hkv=1, Dh=64), {}),                   # one row
+    (dict(B=1, C=64, T=64, H=3, Hkv=3, Dh=64), {}),                 # whole steps of 64 columns, whole tiles of 128 rows
+    (dict(B=2, C=63, T=67, H=16, Hkv=4, Dh=64), {}),                # more row tiles than workgroups, ragged everything
+    (dict(B=1, C=65, T=128, H=2, Hkv=2, Dh=64), {}),                # four steps, the last of one column
+    (dict(B=1, C=65, T=129, H=2, Hkv=2, Dh=64), {}),                # five: the build of up to ten
+    (dict(B=1, C=2, T=512, H=2, Hkv=1, Dh=64), {}),                 # nine
+    (dict(B=1, C=1, T=640, H=1, Hkv=1, Dh=64), {}),                 # eleven: a pass by rows and one by columns
+    (dict(B=2, C=32, T=70, H=4, Hkv=2, Dh=128), {}),                # three steps at Dh 128
+    (dict(B=1, C=128, T=128, H=2, Hkv=1, Dh=128), {}),              # four
+    (dict(B=1, C=5, T=257, H=2, Hkv=1, Dh=128), {}),                # six: the two passes
+    (dict(B=1, C=40, T=37, H=2, Hkv=1, Dh=64), dict(time_bias=False)),
+    (dict(B=1, C=40, T=37, H=2, Hkv=1, Dh=64), dict(chan_bias=False)),
+    (dict(B=1, C=40, T=37, H=2, Hkv=1, Dh=128), dict(time_bias=False, chan_bias=False)),
+], ids=lambda c: "-".join(f"{k}{int(v)}" for k, v in c.items()) or "both")
+def test_backward_finish_against_table_products(cfg, flags):
+    """mvpa_backward_full against mvpa_backward's fp32 results and the products of the table gradients in 64 bits.
+    G is rounded to bf16 once (2^-8 of each term) and so is the result; the fp32 sums of up to 2^17 terms add less
+    than 2^-10 of the sum of their magnitudes."""
+    import mvpa_hip
+    inp = make_mvpa_inputs(seed=23, qkv_unit=True, **cfg).to("cuda", torch.bfloat16)
+    tabs = (inp.u, inp.vb, inp.z, inp.k_time, inp.k_chan)
+    out, lse = mvpa_hip.mvpa_forward(inp.q, inp.k, inp.v, *tabs, return_lse=True, **flags)
+    d_o = torch.randn(out.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).bfloat16()
+    scale = cfg["Dh"] ** -0.5
+    got = mvpa_hip.mvpa_backward_full(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=scale, **flags)
+    dq_c, dk, dv, dbt, dbc = (t.double() for t in mvpa_hip.mvpa_backward(inp.q, inp.k, inp.v, out, d_o, lse, *tabs,
+                                                                         sm_scale=scale, **flags))
+    B, H, N, Dh = inp.q.shape
+    Hkv = cfg["Hkv"]
+
+    def rows(t):
+        return t.reshape(B, Hkv, -1, t.shape[-1])
+    q, dq, size_q = rows(inp.q).double(), rows(dq_c), rows(dq_c).abs()
+    want, size = {"u": dq.sum((0, 2))}, {"u": size_q.sum((0, 2))}
+    for on, G, tab, bias, name, tname in ((flags.get("time_bias", True), dbt, inp.k_time, inp.vb, "vb", "k_time"),
+                                          (flags.get("chan_bias", True), dbc, inp.k_chan, inp.z, "z", "k_chan")):
+        G, tab, qb = rows(G) * int(on), tab.double(), q + bias.double()[None, :, None]
+        dq, size_q = dq + G @ tab, size_q + G.abs() @ tab.abs()
+        want[name], size[name] = (G @ tab).sum((0, 2)), (G.abs() @ tab.abs()).sum((0, 2))
+        want[tname] = (G.transpose(2, 3).contiguous() @ qb).sum(0)
+        size[tname] = (G.abs().transpose(2, 3).contiguous() @ (q.abs() + bias.double().abs()[None, :, None])).sum(0)
+    want.update(q=dq.reshape(B, H, N, Dh), k=dk, v=dv)
+    # dk, dv: the query heads of a kv head may come as parts that are added afterwards, another order of fp32 sums
+    # whose terms are at least as large as a typical element
+    size.update(q=size_q.reshape(B, H, N, Dh), k=dk.abs() + dk.pow(2).mean().sqrt(), v=dv.abs() + dv.pow(2).mean().sqrt())
+    for n, g in zip(NAMES, got):
+        bound = 1.02 * 2.0 ** -8 * (want[n].abs() + size[n]) + 2.0 ** -10 * size[n]
+        assert ((g.double() - want[n]).abs() <= bound).all(), n
