@@ -450,6 +450,12 @@ int mvpa_rmsnorm_backward(const void* x, const void* weight, const void* dy, con
 int mvpa_silu_gate_bf16(const void* gu, void* out, int64_t rows, int32_t n, void* stream);
 int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void* dgu, int64_t rows, int32_t n, void* stream);
 
+/* dw[N,K] = dy[M,N]^T x[M,K]: the weight gradient of y = x w^T, bf16 in and out, fp32 sums.  N, K and the row
+ * strides (in elements) multiples of 8, 16-byte aligned pointers; ws: mvpa_linear_wgrad_ws_bytes(M, N, K) bytes. */
+size_t mvpa_linear_wgrad_ws_bytes(int64_t M, int64_t N, int64_t K);
+int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, int64_t M, int64_t N, int64_t K, int64_t lddy, int64_t ldx,
+                           int64_t lddw, void* ws, size_t ws_bytes, void* stream);
+
 /* Stacked projection weights with low-rank adapters (layers/mvpa.py:43-62, 86-93), all bf16 and contiguous:
  * part i holds rows [row0, row0 + rows) of out [sum of rows, K], w + scale * b a with w [rows, K], a [r, K] and
  * b [rows, r]; a and b both null: w as it is.  row0 is filled in by the library.  The backward writes da and db

@@ -272,6 +272,28 @@ PyObject* py_linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linear_wgrad(dy [M, N], x [M, K]) -> dy^T x | status
+PyObject* py_linear_wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 2, "linear_wgrad takes dy and x");
+  const Tensor &dy = tensor_of(args[0]), &x = tensor_of(args[1]);
+  on_gpu(dy);
+  on_gpu(x);
+  TORCH_CHECK(dy.dim() == 2 && x.dim() == 2 && dy.size(0) == x.size(0) && dy.scalar_type() == at::kBFloat16 &&
+                  x.scalar_type() == at::kBFloat16,
+              "linear_wgrad: bf16 rows");
+  const int64_t M = dy.size(0), N = dy.size(1), K = x.size(1);
+  if (dy.stride(1) != 1 || x.stride(1) != 1 || M == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor dw = at::empty({N, K}, x.options()), ws;
+  const size_t bytes = mvpa_linear_wgrad_ws_bytes(M, N, K);
+  if (bytes) ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
+  const int st = mvpa_linear_wgrad_bf16(dy.data_ptr(), x.data_ptr(), dw.data_ptr(), M, N, K, dy.stride(0), x.stride(0), K,
+                                        bytes ? ws.data_ptr() : nullptr, bytes, current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(dw) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
 // encode(x [M, L] fp32, norm weight fp32, levels, dwt_size, pitch, eps) -> [M, pitch] bf16 | status
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -765,6 +787,7 @@ PyMethodDef kMethods[] = {
     {"forward", (PyCFunction)(void*)py_forward, METH_FASTCALL, "fused MVPA forward"},
     {"backward", (PyCFunction)(void*)py_backward, METH_FASTCALL, "backward of the fused MVPA forward, bf16"},
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
+    {"linear_wgrad", (PyCFunction)(void*)py_linear_wgrad, METH_FASTCALL, "dy^T @ x in bf16"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
     {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},

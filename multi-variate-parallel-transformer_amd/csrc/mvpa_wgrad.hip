@@ -1,0 +1,243 @@
+// Weight gradients: dW[N,K] = dY[M,N]^T X[M,K] in bf16 with fp32 sums (the backward of layers/mvpa.py:354-359, 400
+// and of the MLP's projections, models/mvpformer.py:146).
+//
+// The output is small and the contraction long (MVPFormer-S, 6400 rows: 36 .. 162 tiles of 128 x 128 over 100
+// blocks of 64 rows), so the tiles alone do not fill 256 CUs: the rows are dealt over `splits` workgroups per
+// tile, fp32 partial tiles meet in a second kernel, or over two groups of waves of a workgroup that meet in LDS.  Both operands are contracted over their slow index: they go
+// straight from memory to LDS as they lie, [64 rows][128 columns], and both MFMA operands come out of transposing
+// LDS reads.  A group is 4 waves of 64 x 64 outputs (64 accumulator registers) on two 32 KiB stages, so that
+// two share a CU.  Per block of 64 rows one barrier, in front of its last quarter: that quarter's fragments
+// are in registers, the barrier publishes the next block and frees this one's stage for the block after next.
+// Bound by the fragment reads (one per product) and the tile requests: 960 TFLOP/s on [4096,2048] over 6400 rows, 710
+// on [3456,768] with its partial tiles (13 of 48 us).
+#include "mvpa_mfma_tools.h"
+
+namespace mvpa {
+namespace wgrad {
+
+constexpr int TILE = 128, KB = 64;               // outputs of a tile each way, rows of a block
+constexpr int ROWB = TILE * 2, STAGE = 2 * KB * ROWB;
+constexpr int LOADS = STAGE / 1024 / 4;          // 1 KiB requests per wave and block
+
+struct args {
+  const bf16_t *dy, *x;
+  void* out;                                     // dW, or the partial tiles [splits][N][K]
+  int64_t ldy, ldx, ldo;
+  int32_t M, N, K, tiles_k, splits, blocks;      // blocks of rows in all
+};
+
+// fragment of a [64][128] tile contracted over its rows: column 32 c + lane's, rows 16 s + 8 rd + 4 hh + e
+__device__ inline bf16x8 frag(const unsigned char* p, int s) {
+  const bf16x4 lo = el_bf16::read_tr(p + 16 * s * ROWB), hi = el_bf16::read_tr(p + (16 * s + 8) * ROWB);
+  return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+template <int GROUPS, bool PARTIAL>
+__global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char all_stages[];
+  const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, group = __builtin_amdgcn_readfirstlane(tid >> 8);
+  unsigned char* const smem = all_stages + group * 2 * STAGE;
+  // ids equal mod 8 run on one XCD: it gets neighbouring tiles of one share of the rows, which read the same
+  // rows at about the same time
+  const int total = gridDim.x, per = total / 8, more = total % 8, xcd = blockIdx.x & 7;
+  const int id = xcd * per + min(xcd, more) + (int)(blockIdx.x >> 3);
+  const int tiles = total / a.splits, split = id / tiles, tile = id % tiles;
+  const int n0 = tile / a.tiles_k * TILE, k0 = tile % a.tiles_k * TILE;
+  const int first = (int)((int64_t)a.blocks * split / a.splits), last = (int)((int64_t)a.blocks * (split + 1) / a.splits);
+  const int count = (last - first + GROUPS - 1) / GROUPS;       // blocks of a group: first + group, + GROUPS ..
+  const int64_t m_end = min((int64_t)last * KB, (int64_t)a.M);
+  auto row_of = [&](int kb) { return (int64_t)(first + group + kb * GROUPS) * KB; };
+
+  // request i of a wave: rows 4 (wave + 4 (i & 3)) .. of dY (i < 4) or X; lane: row lane / 16, chunk lane % 16
+  const int row_l = lane >> 4, chunk = ((lane & 15) ^ swz_v<TILE>(row_l)) * 8;
+  const bf16_t* dy = a.dy + min(n0 + chunk, a.N - 8);           // columns past the end: any, their outputs are not stored
+  const bf16_t* x = a.x + min(k0 + chunk, a.K - 8);
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
+  auto request = [&](int kb, int stage) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int r = 4 * (wave + 4 * (i & 3));
+      const int64_t m = min(row_of(kb) + r + row_l, m_end - 1);
+      load_to_lds_16(i < LOADS / 2 ? dy + m * a.ldy : x + m * a.ldx, lds0 + stage * STAGE + (i < LOADS / 2 ? 0 : STAGE / 2) + r * ROWB);
+    }
+  };
+  // a block that reaches past the last row: zeros there, in what this wave has requested itself
+  auto cut = [&](int kb, int stage) {
+    if (row_of(kb) + KB <= m_end) return;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int r = 4 * (wave + 4 * (i & 3)) + row_l;
+      if (row_of(kb) + r >= m_end)
+        *(u32x4*)(smem + stage * STAGE + (i < LOADS / 2 ? 0 : STAGE / 2) + r * ROWB + (lane & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+
+  const int wn = wave >> 1, wk = wave & 1, row0 = 4 * hh + ((ln & 15) >> 2);
+  const unsigned char *pa[2], *pb[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    const int sub = 2 * (ln >> 4) + ((ln & 3) >> 1), base = row0 * ROWB + ((ln & 1) << 3);
+    pa[c] = smem + base + (((4 * (2 * wn + c) + sub) ^ swz_v<TILE>(row0)) << 4);
+    pb[c] = smem + STAGE / 2 + base + (((4 * (2 * wk + c) + sub) ^ swz_v<TILE>(row0)) << 4);
+  }
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+  request(0, 0);
+  if (count > 1) {
+    request(1, 1);
+    wait_vmcnt_imm<LOADS>();
+  } else {
+    wait_vmcnt_imm<0>();
+  }
+  cut(0, 0);
+  lds_barrier();
+  bf16x8 fa[2], fb[2];
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    fa[c] = frag(pa[c], 0);
+    fb[c] = frag(pb[c], 0);
+  }
+#pragma unroll 1
+  for (int kb = 0; kb < count; ++kb) {
+    const int st = (kb & 1) * STAGE;
+#pragma unroll
+    for (int s = 0; s < KB / 16; ++s) {
+      bf16x8 na[2], nb[2];
+      if (s + 1 < KB / 16) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          na[c] = frag(pa[c] + st, s + 1);
+          nb[c] = frag(pb[c] + st, s + 1);
+        }
+      } else {
+        wait_vmcnt_imm<0>();                     // block kb + 1, requested a block ago
+        if (kb + 1 < count) cut(kb + 1, (kb + 1) & 1);
+        lds_barrier();
+        if (kb + 2 < count) request(kb + 2, kb & 1);
+        const int next = STAGE - st;             // past the end: what lies there, for nobody
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          na[c] = frag(pa[c] + next, 0);
+          nb[c] = frag(pb[c] + next, 0);
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        fa[c] = na[c];
+        fb[c] = nb[c];
+      }
+    }
+  }
+  if (GROUPS == 2) {                             // the second group's sums to the first, 64 KiB over the first's stages
+    __syncthreads();
+    float* merge = (float*)all_stages + wave * 64 * 64 + lane;
+    if (group == 1) {
+#pragma unroll
+      for (int i = 0; i < 64; ++i) merge[i * 64] = acc[i >> 5][(i >> 4) & 1][i & 15];
+    }
+    __syncthreads();
+    if (group == 1) return;
+#pragma unroll
+    for (int i = 0; i < 64; ++i) acc[i >> 5][(i >> 4) & 1][i & 15] += merge[i * 64];
+  }
+  // lane: column k0 + 64 wk + 32 j + ln of 16 rows
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int k = k0 + 64 * wk + 32 * j + ln;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int n = n0 + 64 * wn + 32 * i + (e >> 2) * 8 + hh * 4 + (e & 3);
+        if (n < a.N && k < a.K) {
+          if (PARTIAL) ((float*)a.out)[((int64_t)split * a.N + n) * a.K + k] = acc[i][j][e];
+          else ((bf16_t*)a.out)[n * a.ldo + k] = f32_to_bf16(acc[i][j][e]);
+        }
+      }
+    }
+}
+
+// dW = the sum of the partial tiles, a thread 8 columns of a row
+__global__ __launch_bounds__(256) void linear_wgrad_reduce_kernel(const float* __restrict__ part, bf16_t* __restrict__ dw, int N, int K,
+                                                                  int64_t ldo, int splits) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8, size = (int64_t)N * K;
+  if (i >= size) return;
+  float v[8] = {};
+#pragma unroll 4
+  for (int s = 0; s < splits; ++s) {
+    const float4 lo = *(const float4*)(part + s * size + i), hi = *(const float4*)(part + s * size + i + 4);
+    v[0] += lo.x; v[1] += lo.y; v[2] += lo.z; v[3] += lo.w;
+    v[4] += hi.x; v[5] += hi.y; v[6] += hi.z; v[7] += hi.w;
+  }
+  *(bf16x8*)(dw + i / K * ldo + i % K) = bf16x8{(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3],
+                                                (__bf16)v[4], (__bf16)v[5], (__bf16)v[6], (__bf16)v[7]};
+}
+
+static int tiles_of(int64_t N, int64_t K) { return (int)((N + TILE - 1) / TILE * ((K + TILE - 1) / TILE)); }
+
+// How the rows are dealt, by what a launch was seen to take: a group of 4 waves 1.27 us a block where two share a
+// CU, partial results 2 x 4 bytes an output and share at 4.8 TB/s.  6400 rows, us (vendor library): [3456,768]
+// 52 (65), [768,1728] 34 -> 28 with pairs of groups (50), [1280,768] 28 -> 22 (42), [768,768] 24 -> 16 (39).
+struct plan {
+  int groups, splits;
+};
+static plan plan_of(int64_t M, int64_t N, int64_t K) {
+  const int64_t blocks = (M + KB - 1) / KB, tiles = tiles_of(N, K);
+  plan best{1, 1};
+  double best_us = 1e30;
+  for (int groups = 1; groups <= 2; ++groups)
+    for (int s = 1; s <= 32 && (s == 1 || (int64_t)s * groups <= blocks); ++s) {
+      const int64_t slots = 512 / groups, rounds = (tiles * s + slots - 1) / slots, each = (blocks + s * groups - 1) / (s * groups);
+      const double us = rounds * each * 1.27 + (s > 1 ? 3.0 + 8e-6 * s * N * K / 4.8 : 0.0);
+      if (us < best_us) {
+        best_us = us;
+        best = {groups, s};
+      }
+    }
+  return best;
+}
+
+}  // namespace wgrad
+}  // namespace mvpa
+
+using namespace mvpa;
+
+extern "C" size_t mvpa_linear_wgrad_ws_bytes(int64_t M, int64_t N, int64_t K) {
+  if (M <= 0 || N <= 0 || K <= 0 || N > (1 << 20) || K > (1 << 20)) return 0;
+  const int s = wgrad::plan_of(M, N, K).splits;
+  return s == 1 ? 0 : (size_t)s * N * K * sizeof(float);
+}
+
+extern "C" int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, int64_t M, int64_t N, int64_t K, int64_t lddy,
+                                      int64_t ldx, int64_t lddw, void* ws, size_t ws_bytes, void* stream) {
+  if (!dy || !x || !dw) return MVPA_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || N > (1 << 20) || K > (1 << 20) || M > ((int64_t)1 << 30) || lddy < N || ldx < K || lddw < K)
+    return MVPA_ERR_SHAPE;
+  if ((N | K | lddy | ldx | lddw) % 8 != 0 || (((uintptr_t)dy | (uintptr_t)x | (uintptr_t)dw | (uintptr_t)ws) & 15)) return MVPA_ERR_ALIGN;
+  const wgrad::plan p = wgrad::plan_of(M, N, K);
+  const size_t need = p.splits == 1 ? 0 : (size_t)p.splits * N * K * sizeof(float);
+  if (need > ws_bytes || (need && !ws)) return MVPA_ERR_WS_SIZE;
+  wgrad::args a{(const bf16_t*)dy, (const bf16_t*)x, p.splits > 1 ? ws : dw, lddy, ldx, lddw, (int32_t)M, (int32_t)N, (int32_t)K,
+                (int32_t)((K + wgrad::TILE - 1) / wgrad::TILE), p.splits, (int32_t)((M + wgrad::KB - 1) / wgrad::KB)};
+  hipStream_t s = (hipStream_t)stream;
+  auto kern = p.groups == 2 ? p.splits > 1 ? wgrad::linear_wgrad_kernel<2, true> : wgrad::linear_wgrad_kernel<2, false>
+                            : p.splits > 1 ? wgrad::linear_wgrad_kernel<1, true> : wgrad::linear_wgrad_kernel<1, false>;
+  const int lds = 2 * wgrad::STAGE * p.groups;
+  want_dynamic_lds((const void*)kern, lds);
+  MVPA_LAUNCH(kern, dim3((unsigned)(wgrad::tiles_of(N, K) * p.splits)), dim3(256 * p.groups), lds, s, a);
+  if (p.splits > 1)
+    MVPA_LAUNCH(wgrad::linear_wgrad_reduce_kernel, dim3((unsigned)((N * K / 8 + 255) / 256)), dim3(256), 0, s, (const float*)ws,
+                (bf16_t*)dw, (int)N, (int)K, lddw, p.splits);
+  return take_launch_status();
+}

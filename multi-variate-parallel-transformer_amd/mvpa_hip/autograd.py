@@ -1,10 +1,9 @@
 """Differentiable wrappers of the library's dense ops, for gradients through the layer and stack
 modules (the reference trains through layers/mvpa.py:280-337 and models/mvpformer.py:132-147).
 
-Forward passes are the library's kernels.  The backward passes of the bf16 products are the two
-plain products dX = dY W and dW = dY^T X on the vendor library through torch.matmul: it reads
-the transposed operand in place and splits the long contraction of a weight gradient (a small
-[N,K] output over all rows), which this library's GEMM would run on a few dozen tiles.  Norm,
+Forward passes are the library's kernels.  Of the backward passes of the bf16 products dX = dY W is
+on the vendor library through torch.matmul, which reads the transposed operand in place, and dW = dY^T X
+on a kernel of the library where that is the faster one (_weight_gradient).  Norm,
 gated activation and residual sums run on kernels of the library both ways (csrc/mvpa_train.hip).  The attention operator itself is
 `attentions.attn.FlashMVPA` (mvpa_backward kernels).
 """
@@ -19,8 +18,23 @@ def wants_grad(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+def _weight_gradient(dy, x):
+    """dy^T x of bf16 rows.  The library's kernel (csrc/mvpa_wgrad.hip) where its row shares pay: from 2560 rows and
+    below 256 tiles of 128 x 128, us against the vendor library: [768,768] 3000 rows 20 / 28, 6400 22 / 39, 16384
+    34 / 91; [3456,768] 33 / 39, 48 / 61, 102 / 148.  Below it the second launch costs more than is gained (2048 rows
+    16.5 / 16, 1024 14.7 / 11), and with 256 tiles the vendor's larger ones fill the chip too ([2048,2048] 65 / 64 at
+    6400 rows, [11264,2048] 321 / 260)."""
+    (m, n), k = dy.shape, x.shape[-1]
+    if m >= 2560 and -(-n // 128) * -(-k // 128) < 256 and not torch.is_grad_enabled():
+        dw = mvpa_hip.load_ext().linear_wgrad(dy, x)
+        if type(dw) is not int:                              # a status: rows that do not start at 16-byte boundaries
+            return dw
+    return torch.matmul(dy.t(), x)
+
+
 class _LinearFn(torch.autograd.Function):
-    """y = x @ w^T, bf16, any leading shape of x: forward on the GPU library, backward on the vendor GEMM."""
+    """y = x @ w^T, bf16, any leading shape of x: forward on the GPU library, backward dX on the vendor GEMM and
+    dW as above."""
 
     @staticmethod
     def forward(ctx, x, w):
@@ -36,7 +50,7 @@ class _LinearFn(torch.autograd.Function):
         if ctx.needs_input_grad[0]:
             dx = torch.matmul(dy2, w).view(x.shape)                               # [M,N] @ [N,K]
         if ctx.needs_input_grad[1]:
-            dw = torch.matmul(dy2.t(), x.reshape(-1, k))                          # [N,M] @ [M,K]
+            dw = _weight_gradient(dy2, x.reshape(-1, k))                          # [N,M] @ [M,K]
         return dx, dw
 
 

@@ -16,7 +16,7 @@ EXT = os.path.join(HERE, "_mvpa_ext.so")
 
 SOURCES = ["mvpa_api.hip", "mvpa_generic.hip", "mvpa_mfma.hip", "mvpa_wave.hip", "mvpa_step.hip", "mvpa_mfma64.hip", "mvpa_mfma128.hip", "mvpa_dense.hip", "mvpa_backward.hip",
            "mvpa_backward_mfma.hip", "mvpa_static_ws.hip", "mvpa_fp8.hip", "mvpa_tiles.hip", "mvpa_stack.hip", "mvpa_bwd_finish.hip",
-           "mvpa_train.hip"]
+           "mvpa_train.hip", "mvpa_wgrad.hip"]
 
 # -packed-fp32-ops: keep the compiler from forming packed fp32 VALU instructions.
 FLAGS = [

@@ -212,3 +212,27 @@ def test_stacked_weights_differentiate_twice():
     dd, = torch.autograd.grad(yd.pow(2).sum(), ad, create_graph=True)
     ref, = torch.autograd.grad(dd.sum(), bd)
     assert ((grad.double() - ref).norm() / ref.norm()).item() <= 3e-2
+
+
+# rows around the 64 of a block and the shares; outputs around tiles of 128, the smallest ones, operands with a row
+# pitch; one share, several, one and two groups of waves
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (63, 128, 128), (64, 136, 120), (65, 8, 264), (129, 256, 1024), (700, 1280, 768),
+                                   (6400, 768, 1728), (2561, 3456, 768), (1000, 2048, 2056), (20000, 8, 16)])
+def test_weight_gradient(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    dy, x = (torch.randn((m, c + 8), generator=g, device="cuda").bfloat16()[:, :c] for c in (n, k))
+    dw = mvpa_hip.load_ext().linear_wgrad(dy, x)
+    _close(dw, dy.double().t() @ x.double(), m)
+    dw = mvpa_hip.load_ext().linear_wgrad(dy.contiguous(), x.contiguous())
+    _close(dw, dy.double().t() @ x.double(), m)
+
+
+def test_weight_gradient_refuses_rows_off_16_bytes():
+    x = torch.randn(64, 24, device="cuda").bfloat16()
+    for dy in (x[:, 1:9], x[:, :12], x.t()):
+        assert type(mvpa_hip.load_ext().linear_wgrad(dy, x[:dy.shape[0]])) is int
+    w = torch.randn(24, 8, device="cuda").bfloat16().requires_grad_(True)
+    x = torch.randn(3000, 8, device="cuda").bfloat16()                            # through the autograd function: any rows
+    dy = torch.randn(3000 * 24 + 1, device="cuda").bfloat16()[1:].view(3000, 24)
+    dw, = torch.autograd.grad(AG.linear(x, w), w, dy)
+    _close(dw, dy.double().t() @ x.double(), 3000)
