@@ -6,32 +6,39 @@
 // time of such a product is the latency of its chain of k-blocks, so the operands come through a ring
 // of STAGES direct-to-LDS blocks of 64: STAGES - 1 blocks are in flight at any time.
 //   4 waves.  WM = 4: a wave owns 32 rows of x and all 64 columns.  WM = 2 / 1: two / four waves share
-//   the rows and take 32 / 16 of every 64 k each; their sums meet in LDS at the end, so that a wave
-//   always holds two 32 x 32 tiles (for the gated product: the gate and the up columns of an output).
+//   the rows and take 32 / 16 of every 64 k each, so that a wave always holds two 32 x 32 tiles (for the gated
+//   product: the gate and the up columns of an output).
+//   The sums go through LDS by rows and every thread finishes and stores 16 bytes of a row: stored as the
+//   products leave them, 8 or 16 bytes of each of 32 rows per instruction, the partial sums of 525 rows of 768
+//   alone took 3 us.
 //   Rows are 128 bytes with the 16-byte chunks XOR-swizzled as in mvpa_dense.hip.
 #include "mvpa_tiles.h"
 
 #include "mvpa_mfma_tools.h"
 
+#include <type_traits>
+
 namespace mvpa {
 
 constexpr int TL_BN = 64, TL_BK = 64, TL_ROWB = TL_BK * 2;
+constexpr int TL_SUM = TL_BN * 4;                   // bytes of a row of sums: 16 chunks, XOR-swizzled by the row
 
 template <int WM, int STAGES>
 struct tile_cfg {
   static constexpr int BM = 32 * WM, KH = 4 / WM, LPW = WM + 2;      // 1 KiB loads per wave and block
   static constexpr int STAGE = (BM + TL_BN) * TL_ROWB;
   static constexpr int LDS = STAGES * STAGE;
-  static_assert((KH - 1) * WM * 8192 <= LDS, "the sums of the k-parts fit the ring");
+  static_assert(4 * 32 * TL_SUM <= LDS, "the sums of all waves fit the ring");
 };
 
-// acc[j] = rows 32j.. of the w tile times the wave's 32 rows of x, k-blocks [kb0, kb1); complete in the
-// waves of k-part 0 only.  wrow(r): which row of W feeds row r of the tile.
+// The tile's products over k-blocks [kb0, kb1), left in LDS for tile_sum.  wrow(r): which row of W feeds row r of
+// the tile.
 template <int WM, int STAGES, typename WRow>
 __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* __restrict__ X, int64_t ldx, int64_t m0,
                                              int64_t M, const bf16_t* __restrict__ W, int64_t ldw, WRow wrow,
-                                             int kb0, int kb1, f32x16 (&acc)[2]) {
+                                             int kb0, int kb1) {
   using G = tile_cfg<WM, STAGES>;
+  f32x16 acc[2];
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, kh = wave / WM;
@@ -104,30 +111,29 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
       for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s], acc[j], 0, 0, 0);
     st = st + G::STAGE == lds + G::LDS ? lds : st + G::STAGE;
   }
-  if (G::KH > 1) {
-    lds_barrier();
-    float* red = (float*)lds + lane;
-    if (kh > 0) {
+  // every wave's sums by rows of x, [k part][BM rows][64 columns] over the ring
+  lds_barrier();
+  unsigned char* sums = lds + (kh * G::BM + wm * 32 + ln) * TL_SUM;
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) red[((((kh - 1) * WM + wm) * 2 + j) * 16 + r) * 64] = acc[j][r];
-    }
-    lds_barrier();
-    if (kh == 0) {
-#pragma unroll
-      for (int p = 0; p < G::KH - 1; ++p)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) acc[j][r] += red[(((p * WM + wm) * 2 + j) * 16 + r) * 64];
-    }
-  }
+    for (int a4 = 0; a4 < 4; ++a4)
+      *(float4*)(sums + (((8 * j + 2 * a4 + hh) ^ (ln & 15)) << 4)) =
+          make_float4(acc[j][a4 * 4], acc[j][a4 * 4 + 1], acc[j][a4 * 4 + 2], acc[j][a4 * 4 + 3]);
+  lds_barrier();
 }
 
-__device__ inline void store_quad(bf16_t* p, float a, float b, float c, float d) {
-  bf16x4 o = {(__bf16)a, (__bf16)b, (__bf16)c, (__bf16)d};
-  *(bf16x4*)p = o;
+// four columns 4 c .. of row r of the tile, summed over the k parts
+template <typename G>
+__device__ __forceinline__ float4 tile_sum(const unsigned char* lds, int r, int c) {
+  const unsigned char* p = lds + r * TL_SUM + ((c ^ (r & 15)) << 4);
+  float4 v = *(const float4*)p;
+#pragma unroll
+  for (int k = 1; k < G::KH; ++k) {
+    const float4 o = *(const float4*)(p + k * G::BM * TL_SUM);
+    v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w;
+  }
+  return v;
 }
 
 // Workgroup id -> (column tile, row tile): ids equal mod 8 share an XCD and its L2; the row tiles of a
@@ -139,6 +145,92 @@ __device__ inline bool tile_coords(int id, int ct, int mt, int& col, int& row) {
   return col < ct;
 }
 
+// What a row tile of WM * 32 rows does: the last one of many where few rows are left takes a smaller one, in
+// whose blocks x is less (525 rows: 13 of them are left to a fifth tile of 128)
+template <int WM, int STAGES, typename F>
+__device__ __forceinline__ void for_rows_left(int64_t rows, F f) {
+  if constexpr (WM == 4 && STAGES == 3) {
+    if (rows <= 32) f(std::integral_constant<int, 1>(), std::integral_constant<int, 6>());
+    else if (rows <= 64) f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+    else f(std::integral_constant<int, 4>(), std::integral_constant<int, 3>());
+    static_assert(tile_cfg<1, 6>::LDS <= tile_cfg<4, 3>::LDS && tile_cfg<2, 4>::LDS <= tile_cfg<4, 3>::LDS, "LDS of the launch");
+  } else {
+    f(std::integral_constant<int, WM>(), std::integral_constant<int, STAGES>());
+  }
+}
+
+template <int WM, int STAGES>
+__device__ __forceinline__ void tile_dual(unsigned char* tl_lds, const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+                                          const bf16_t* __restrict__ W0, int N0, int64_t ldw0, const tile_out& out,
+                                          const tile_gated& gt, const tile_norm& nrm, int gated_ct, int col, int64_t m0) {
+  using G = tile_cfg<WM, STAGES>;
+  const int tid = threadIdx.x;
+  const bool gated = col < gated_ct;
+  const int n0 = gated ? col * 32 : (col - gated_ct) * TL_BN, N = gated ? gt.N : N0;
+  // sums of squares of the rows this thread will finish: requested in front of the product, used behind it
+  constexpr int ROWS = G::BM / 32;                  // every 64th row of the gated product, every 32nd of the plain one
+  const int r0 = gated ? tid >> 2 : tid >> 3, dr = gated ? 64 : 32;
+  float ss[ROWS];
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) ss[i] = nrm.ss ? nrm.ss[min(m0 + r0 + i * dr, M - 1) * nrm.parts] : 0.f;
+  if (gated)
+    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, gt.w, gt.ldw,
+                             [&](int r) { return (int64_t)((r >> 5) * N + min(n0 + (r & 31), N - 1)); }, 0, K / TL_BK);
+  else
+    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W0, ldw0, [&](int r) { return (int64_t)min(n0 + r, N0 - 1); }, 0, K / TL_BK);
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) asm volatile("" : "+v"(ss[i]));       // not before the product
+  auto factor = [&](int i, int64_t m) {
+    if (!nrm.ss) return 1.f;
+    float s = ss[i];
+    for (int p = 1; p < nrm.parts; ++p) s += nrm.ss[m * nrm.parts + p];
+    return rsqrtf(s / (float)K + nrm.eps);
+  };
+  if (gated) {                                      // 8 outputs of a row per thread
+    const int c = tid & 3, n = n0 + c * 8;
+#pragma unroll
+    for (int i = 0; i < (G::BM + 63) / 64; ++i) {
+      const int r = r0 + i * 64;
+      const int64_t m = m0 + r;
+      if (r >= G::BM || m >= M || n >= N) continue;
+      const float rn = factor(i, m);
+      bf16x8 o;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const float4 g4 = tile_sum<G>(tl_lds, r, 2 * c + q), u4 = tile_sum<G>(tl_lds, r, 8 + 2 * c + q);
+        const float g[4] = {g4.x, g4.y, g4.z, g4.w}, u[4] = {u4.x, u4.y, u4.z, u4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float x = g[e] * rn;
+          o[4 * q + e] = (__bf16)(x / (1.f + __expf(-x)) * (u[e] * rn));
+        }
+      }
+      *(bf16x8*)(gt.y + m * gt.ldy + n) = o;
+    }
+    return;
+  }
+  const int slot = out.k ? (out.head ? *out.head : out.slot) : 0, c = tid & 7, n = n0 + c * 8;
+#pragma unroll
+  for (int i = 0; i < ROWS; ++i) {
+    const int r = r0 + i * 32;
+    const int64_t m = m0 + r;
+    if (m >= M || n >= N0) continue;
+    bf16_t* dst;
+    if (n < out.n_y) {
+      dst = out.y + m * out.ldy + n;
+    } else {
+      const int o = n - out.n_y, is_v = o >= out.n_kv, e = is_v ? o - out.n_kv : o;
+      const int g = e / out.Dh, d = e - g * out.Dh;
+      const int b = (int)m / out.C, ch = (int)m - b * out.C;
+      dst = (is_v ? out.v : out.k) + b * out.stride_b + g * out.stride_g + ((int64_t)slot * out.C + ch) * out.Dh + d;
+    }
+    const float rn = factor(i, m);
+    const float4 lo = tile_sum<G>(tl_lds, r, 2 * c), hi = tile_sum<G>(tl_lds, r, 2 * c + 1);
+    *(bf16x8*)dst = bf16x8{(__bf16)(lo.x * rn), (__bf16)(lo.y * rn), (__bf16)(lo.z * rn), (__bf16)(lo.w * rn),
+                           (__bf16)(hi.x * rn), (__bf16)(hi.y * rn), (__bf16)(hi.z * rn), (__bf16)(hi.w * rn)};
+  }
+}
+
 template <int WM, int STAGES>
 __global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
                                                         const bf16_t* __restrict__ W0, int N0, int64_t ldw0,
@@ -147,59 +239,10 @@ __global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict
   extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
   int col, row;
   if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
-  const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t m0 = (int64_t)row * 32 * WM;
-  const int64_t m = m0 + (wave % WM) * 32 + ln;
-  f32x16 acc[2];
-  float rn = 1.f;                                   // this lane's row factor
-  if (nrm.ss) {
-    const float* pp = nrm.ss + min(m, M - 1) * nrm.parts;
-    float ss = 0.f;
-    for (int p = 0; p < nrm.parts; ++p) ss += pp[p];
-    rn = rsqrtf(ss / (float)K + nrm.eps);
-  }
-  if (col < gated_ct) {
-    const int n0 = col * 32, N = gt.N;
-    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, gt.w, gt.ldw,
-                             [&](int r) { return (int64_t)((r >> 5) * N + min(n0 + (r & 31), N - 1)); }, 0, K / TL_BK, acc);
-    if (wave >= WM || m >= M) return;
-#pragma unroll
-    for (int a4 = 0; a4 < 4; ++a4) {
-      const int n = n0 + a4 * 8 + hh * 4;
-      if (n >= N) continue;
-      float o[4];
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const float g = acc[0][a4 * 4 + r] * rn;
-        o[r] = g / (1.f + __expf(-g)) * (acc[1][a4 * 4 + r] * rn);
-      }
-      store_quad(gt.y + m * gt.ldy + n, o[0], o[1], o[2], o[3]);
-    }
-    return;
-  }
-  const int n0 = (col - gated_ct) * TL_BN;
-  tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W0, ldw0, [&](int r) { return (int64_t)min(n0 + r, N0 - 1); }, 0,
-                           K / TL_BK, acc);
-  if (wave >= WM || m >= M) return;
-  const int slot = out.k ? (out.head ? *out.head : out.slot) : 0;
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int a4 = 0; a4 < 4; ++a4) {
-      const int n = n0 + j * 32 + a4 * 8 + hh * 4;
-      if (n >= N0) continue;
-      bf16_t* dst;
-      if (n < out.n_y) {
-        dst = out.y + m * out.ldy + n;
-      } else {
-        const int i = n - out.n_y, is_v = i >= out.n_kv, e = is_v ? i - out.n_kv : i;
-        const int g = e / out.Dh, d = e - g * out.Dh;
-        const int b = (int)m / out.C, c = (int)m - b * out.C;
-        dst = (is_v ? out.v : out.k) + b * out.stride_b + g * out.stride_g + ((int64_t)slot * out.C + c) * out.Dh + d;
-      }
-      store_quad(dst, acc[j][a4 * 4] * rn, acc[j][a4 * 4 + 1] * rn, acc[j][a4 * 4 + 2] * rn, acc[j][a4 * 4 + 3] * rn);
-    }
+  for_rows_left<WM, STAGES>(M - m0, [&](auto wm, auto stages) {
+    tile_dual<wm(), stages()>(tl_lds, X, M, K, ldx, W0, N0, ldw0, out, gt, nrm, gated_ct, col, m0);
+  });
 }
 
 template <int WM, int STAGES>
@@ -207,30 +250,22 @@ __global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restr
                                                            const bf16_t* __restrict__ W, int N, int64_t ldw,
                                                            float* __restrict__ P, tile_split sp, int ct, int mt) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
-  int cz, row;
-  const int splits = sp.a + sp.b;
-  if (!tile_coords(blockIdx.x, ct * splits, mt, cz, row)) return;
-  const int col = cz / splits, z = cz - col * splits;
+  // an XCD (ids equal mod 8) takes neighbours of one part, row tiles fastest: it reads that part's columns of x, not
+  // all of them, and its panel of w once
+  const int total = ct * (sp.a + sp.b) * mt, per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (id >= total) return;
+  const int cz = id / mt, row = id - cz * mt, z = cz / ct, col = cz - z * ct;
   const int kb0 = z < sp.a ? z * sp.per_a : sp.nkb_a + (z - sp.a) * sp.per_b;
   const int kb1 = z < sp.a ? min(kb0 + sp.per_a, sp.nkb_a) : min(kb0 + sp.per_b, K / TL_BK);
-  const int lane = threadIdx.x & 63, ln = lane & 31, hh = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t m0 = (int64_t)row * 32 * WM;
-  const int64_t m = m0 + (wave % WM) * 32 + ln;
-  const int n0 = col * TL_BN;
-  f32x16 acc[2];
-  tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0,
-                           kb1, acc);
-  if (wave >= WM || m >= M) return;
-  float* prow = P + ((int64_t)z * M + m) * N;
+  const int n0 = col * TL_BN, c = threadIdx.x & 15, n = n0 + c * 4;
+  for_rows_left<WM, STAGES>(M - m0, [&](auto wm, auto stages) {
+    using G = tile_cfg<wm(), stages()>;
+    tile_product<wm(), stages()>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0, kb1);
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int a4 = 0; a4 < 4; ++a4) {
-      const int n = n0 + j * 32 + a4 * 8 + hh * 4;
-      if (n < N)
-        *(float4*)(prow + n) = make_float4(acc[j][a4 * 4], acc[j][a4 * 4 + 1], acc[j][a4 * 4 + 2], acc[j][a4 * 4 + 3]);
-    }
+    for (int r = threadIdx.x >> 4; r < G::BM; r += 16)
+      if (m0 + r < M && n < N) *(float4*)(P + ((int64_t)z * M + m0 + r) * N + n) = tile_sum<G>(tl_lds, r, c);
+  });
 }
 
 // One workgroup per row: the partial sums of a split-K tail product, the residual, one rounding, and
@@ -320,22 +355,26 @@ int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const b
 }
 
 // Partial sums per output element: enough workgroups for every CU, about 4 k-blocks each or more, at most
-// 8 or 9 (every one of them is 4 bytes written and read again per output element).
+// 8 or 9 (every one of them is 4 bytes written and read again per output element).  Never a little more than one
+// workgroup a CU: a CU takes blocks at a fixed rate, and the 288 workgroups of the base model's 3 + 6 parts took as
+// long as 512 (128 rows: 19.5 us, in 2 + 6 parts 14.5; 64 rows 14.4 and 10.1).
 tile_split make_tile_split(int64_t M, int64_t N, int64_t K, int64_t Ka) {
   const int64_t wgs = ((N + TL_BN - 1) / TL_BN) * ((M + 127) / 128), nkb = K / TL_BK, na = Ka / TL_BK, nb = nkb - na;
   int64_t z = (256 + wgs / 2) / wgs;
   if (z > nkb / 4) z = nkb / 4;
   if (z > 8) z = 8;
   if (z < 1) z = 1;
-  const int64_t per = (nkb + z - 1) / z;
+  auto parts_of = [](int64_t n, int64_t per) { return (n + per - 1) / per; };
+  int64_t per = parts_of(nkb, z);                   // blocks of the longest part
+  while ((parts_of(na, per) + parts_of(nb, per)) * wgs > 256 && z > 2 && z * wgs <= 256 && per < nkb) ++per;
   tile_split sp;
   sp.nkb_a = (int32_t)na;
-  sp.a = (int32_t)((na + per - 1) / per);
-  sp.per_a = sp.a ? (int32_t)((na + sp.a - 1) / sp.a) : 0;
-  sp.b = (int32_t)((nb + per - 1) / per);
-  sp.per_b = sp.b ? (int32_t)((nb + sp.b - 1) / sp.b) : 0;
-  if (sp.a) sp.a = (int32_t)((na + sp.per_a - 1) / sp.per_a);
-  if (sp.b) sp.b = (int32_t)((nb + sp.per_b - 1) / sp.per_b);
+  sp.a = (int32_t)parts_of(na, per);
+  sp.per_a = sp.a ? (int32_t)parts_of(na, sp.a) : 0;
+  sp.b = (int32_t)parts_of(nb, per);
+  sp.per_b = sp.b ? (int32_t)parts_of(nb, sp.b) : 0;
+  if (sp.a) sp.a = (int32_t)parts_of(na, sp.per_a);
+  if (sp.b) sp.b = (int32_t)parts_of(nb, sp.per_b);
   return sp;
 }
 
@@ -346,7 +385,7 @@ static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, 
   auto kern = tile_partial_kernel<WM, STAGES>;
   want_dynamic_lds((const void*)kern, G::LDS);
   const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
-  MVPA_LAUNCH(kern, dim3((unsigned)((ct * sp.total() + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w,
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct * sp.total() * mt + 7) / 8 * 8)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w,
               (int)N, ldw, P, sp, ct, mt);
   return take_launch_status();
 }

@@ -74,6 +74,17 @@ def test_windows_of_many_rows(flash, B, C, T):
     assert _rel(got, want) <= REL
 
 
+@pytest.mark.parametrize("B,C,T", [(5, 32, 1), (7, 23, 1), (3, 32, 2), (193, 1, 1), (41, 64, 1)], ids=str)    # 32, 33, 64 and 65 left
+def test_rows_left_to_a_last_tile(B, C, T):
+    """The last of several row tiles by how many rows are left to it, against the stack in 64 bits."""
+    model = _model(n_inner=448)
+    x = torch.randn(B, T, C, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = model(inputs_embeds=x)
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=2, n_head_kv=1), None)
+    assert _rel(got, want) <= REL
+
+
 @pytest.mark.parametrize("B,C", [(1, 5), (1, 64), (2, 100)])
 def test_steps_on_caches(monkeypatch, B, C):
     """A stream that fills its window and slides on: outputs, and every cached key and value, against the same
