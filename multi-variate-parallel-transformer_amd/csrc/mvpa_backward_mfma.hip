@@ -116,7 +116,11 @@ __device__ inline bf16x8 pack8(const f32x16& v, int base) {
   return out.f;
 }
 
-__device__ inline float xhalf_sum(float x) { return x + __shfl_xor(x, 32); }
+// sum over a lane and its partner in the other half-wave, without a trip through the LDS crossbar
+__device__ inline float xhalf_sum(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
 
 // chunk swizzles of a row of 2 DH bytes: row fragments / transposing reads (as in the forward)
 template <int DH> __device__ inline int swz_row(int row) { return DH == 64 ? ((row >> 1) & 7) : (row & 15); }
@@ -125,10 +129,10 @@ template <int DH> __device__ inline int swz_tr(int row) { return DH == 64 ? (((r
 // ONE: the whole walk.  FAR, WIN: the steps before a wave's content window and those from it on, as a launch
 // each, FAR first.  At Dh 128 a wave of the whole walk takes 475 registers and has its SIMD to itself: the far steps'
 // LDS reads, products, reductions and table slabs simply add up (0.89 us a step of 2 x 64 queries at T 512, 0.25 of
-// them products).  FAR alone fits in 256, and two waves cover each other's waits (1.3 us a step of 4 x 64 queries).
+// them products).  FAR alone fits in 256, and two waves cover each other's waits (1.2 us a step of 4 x 64 queries).
 enum query_phase { ONE, FAR, WIN };
 template <int DH, int NCT, int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : QUERY_WAVES<DH, NCT>;
-template <int DH, int NCT, int PHASE> constexpr int PHASE_STAGES = PHASE == FAR ? 5 : QSTAGES<DH, NCT>;
+template <int DH, int NCT, int PHASE> constexpr int PHASE_STAGES = PHASE == FAR ? 4 : QSTAGES<DH, NCT>;
 
 template <int DH, int NCT, int PHASE>
 __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
@@ -241,7 +245,7 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
     }
   };
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
+  for (int s = 0; s < (PHASE == FAR ? 2 : STAGES - 1); ++s)
     if (tk_lo + s <= tk_hi) issue_tile(tk_lo + s, s, PHASE != FAR && tk_lo + s >= tk_near);
 
   // ---- set-up: operand fragments, delta, channel-bias tile
@@ -508,7 +512,7 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
       }
     esum += et;
     const float gt = et * (xhalf_sum((dot[0] + dot[1]) + (dot[2] + dot[3])) - delta * sumEc);
-    if (hh == 0) Gtb[(tkp & 31) * GP + ln] = gt;
+    Gtb[(tkp & 31) * GP + ln] = gt;               // both halves hold it: no branch
   };
   // one far step: products of tile tk into cur, reduction of step tk-1 (in prev) alongside
   auto far_step = [&](int tk, int& tkp, f32x16 (&cur)[NCT], const f32x16 (&prev)[NCT]) {
@@ -593,27 +597,42 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
       }
     }
     gt = xhalf_sum(gt);
-    if (hh == 0) Gtb[((tk - tk_first) & 31) * GP + ln] = gt;
+    Gtb[((tk - tk_first) & 31) * GP + ln] = gt;
   };
 
   // far steps first, then the steps inside the window; waves that are done keep the ring and the barriers going
   int tk = tk_lo;
   if constexpr (PHASE == FAR) {
-    f32x16 dP[NCT];
-    for (; tk < far_end; ++tk) {
-      const unsigned char* Vrow = ring_step(tk);
-      time_slab(tk);
+    // Two steps per barrier, the tiles of the next two requested behind it.  With a barrier a step the two waves of a
+    // SIMD read, multiply and reduce at the same time, and the three add up (T 512 and 128 channels: 2.80 ms a launch,
+    // 2.47 .. 2.56 with half the barriers).
+    auto pair_step = [&](int t0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      lds_barrier();
 #pragma unroll
-      for (int t = 0; t < NCT; ++t) {
+      for (int d = 2; d < 4; ++d)
+        if (t0 + d <= tk_hi) issue_tile(t0 + d, (t0 + d) & 3, false);
+    };
+    for (; tk < far_end; tk += 2) {
+      pair_step(tk);
+      if ((tk & 31) == 0) time_slab(tk);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) dP[t][i] = 0.f;
+      for (int d = 0; d < 2; ++d) {
+        if (tk + d >= far_end) break;
+        const unsigned char* Vrow = smem + ((tk + d) & 3) * STAGE_BYTES;
+        f32x16 dP[NCT];
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks)
-          dP[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB), dOf[ks], dP[t], 0, 0, 0);
+        for (int t = 0; t < NCT; ++t) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) dP[t][i] = 0.f;
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks)
+            dP[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB), dOf[ks], dP[t], 0, 0, 0);
+        }
+        far_reduce(dP, tk + d);
       }
-      far_reduce(dP, tk);
     }
-    for (; tk <= tk_hi; ++tk) (void)ring_step(tk);
+    for (; tk <= tk_hi; tk += 2) pair_step(tk);
   } else if constexpr (PHASE == ONE) {
     f32x16 dPa[NCT], dPb[NCT];
     int tkp = -1;
