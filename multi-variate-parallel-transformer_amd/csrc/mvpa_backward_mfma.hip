@@ -14,9 +14,8 @@
 // Outputs are those of mvpa_backward (include/mvpa_hip.h): the content share of dq and the two
 // bias-table gradients.  For the key pass the workspace receives, in base-2 score units, -delta,
 // the channel-table rows, (time bias - L) laid out [b,h,tq,tk,cq] and (q+u) * scale in bf16.
-// K and V tiles come through a ring of LDS stages filled by direct-to-LDS loads two key steps
-// ahead, K in two copies (row fragments for K Q^T, transposed fragments for K^T dS^T); far key
-// steps fetch V only.
+// K and V tiles come through a ring of LDS stages filled by direct-to-LDS loads, K in two copies (row fragments
+// for K Q^T, transposed fragments for K^T dS^T); far key steps fetch V only.
 #include "mvpa_common.h"
 
 #include <type_traits>
@@ -28,6 +27,7 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
@@ -36,14 +36,10 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 // Head dim DH is 64 or 128: KS = DH / 16 contraction blocks per product, MT = DH / 32 output tiles
 // of the gradients, rows of ROWB = 2 DH bytes (CPR = DH / 8 chunks of 16 bytes) in the LDS tiles.
 constexpr int KSTAGES = 3;                        // ring depth of the key pass
-// ring depth of the query pass: three stages, two where three would not fit the LDS
-template <int DH, int NCT> constexpr int QSTAGES = (DH == 128 && NCT == 2) ? 2 : 3;
-// waves per workgroup of the query pass: with two channel tiles of Dh 64 8 waves (4 query time
-// steps) share the K/V ring and each SIMD holds two waves
-template <int DH, int NCT> constexpr int QUERY_WAVES = (NCT == 2 && DH == 64) ? 8 : 4;
-// floats of per-wave scratch in the query pass: the two time-bias slabs [32][32] + [32][33]; the
-// channel tables of the set-up ([32 NCT][32]) and of the epilogue ([32][32 NCT + 1]) overlay them
-constexpr int WAVE_SCRATCH = 1024 + 32 * 33;
+// floats of per-wave scratch in the query pass: a slab of 32 key steps' time-bias exponents [step][query] and of their
+// gradients [query][step].  The channel table of the set-up ([64][32]) overlays them.
+constexpr int WAVE_SCRATCH = 2048;
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));        // four floats at any float's address
 
 __device__ inline void wave_sync_lds() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -95,8 +91,7 @@ __device__ inline bf16x8 as_frag(u32x4 v) {
 }
 
 // 8 bf16 of a q row + bias, scaled, as an MFMA fragment
-__device__ inline bf16x8 qfrag(u32x4 raw, const bf16_t* __restrict__ bias, float scale) {
-  const u32x4 braw = *(const u32x4*)bias;
+__device__ inline bf16x8 qfrag(u32x4 raw, u32x4 braw, float scale) {
   bf16x8 out;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -121,6 +116,10 @@ __device__ inline float xhalf_sum(float x) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
+__device__ inline float xhalf_max(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
 
 // chunk swizzles of a row of 2 DH bytes: row fragments / transposing reads (as in the forward)
 template <int DH> __device__ inline int swz_row(int row) { return DH == 64 ? ((row >> 1) & 7) : (row & 15); }
@@ -130,30 +129,41 @@ template <int DH> __device__ inline int swz_tr(int row) { return DH == 64 ? (((r
 // each, FAR first.  At Dh 128 a wave of the whole walk takes 475 registers and has its SIMD to itself: the far steps'
 // LDS reads, products, reductions and table slabs simply add up (0.89 us a step of 2 x 64 queries at T 512, 0.25 of
 // them products).  FAR alone fits in 256, and two waves cover each other's waits (1.2 us a step of 4 x 64 queries).
+//
+// At Dh 64 a workgroup is 4 waves and two of them share a CU (80 KB and 256 registers): a third of a workgroup's life
+// at T 128 is set-up, slabs and epilogue, chains of waits that leave the CU idle if all its waves are in them at
+// once.  B4 H16 C64, T 128 / 256 / 512, one workgroup of 8 waves with a barrier a step against this: 920 / 1243 /
+// 2043 -> 714 / 1030 / 1720 us; B4 H12 C21 T25 53 -> 34 us.  The clock is what is left: the waits of a far step have
+// gone from 1040 to 570 of 1770 -> 1350 cycles, and it falls from 2.25 to 1.9 GHz as they go.
 enum query_phase { ONE, FAR, WIN };
-template <int DH, int NCT, int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : QUERY_WAVES<DH, NCT>;
-template <int DH, int NCT, int PHASE> constexpr int PHASE_STAGES = PHASE == FAR ? 4 : QSTAGES<DH, NCT>;
+template <int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : 4;
+// waves per SIMD: at Dh 64 two workgroups share a CU
+template <int DH, int PHASE> constexpr int PHASE_OCC = PHASE == FAR || DH == 64 ? 2 : 1;
+// The ring holds six tiles: three units of far steps, V of two steps each, or two units of a step with content,
+// V | K | K (transposing).
+template <int DH, int NCT> constexpr int TILE_BYTES = NCT * 32 * 2 * DH;
+template <int DH, int NCT, int PHASE> constexpr int QUERY_LDS = 6 * TILE_BYTES<DH, NCT> + PHASE_WAVES<PHASE> * WAVE_SCRATCH * 4;
 
 template <int DH, int NCT, int PHASE>
-__global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
+__global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
-  constexpr int NW = PHASE_WAVES<DH, NCT, PHASE>;
-  constexpr bool SOLO = NW == 4;                  // one wave per SIMD
-  constexpr int CP = NCT * 32, TQW = NW / NCT, TILE = CP * ROWB;
-  static_assert(64 * 32 <= WAVE_SCRATCH && 32 * (CP + 1) <= WAVE_SCRATCH, "channel tables overlay the slabs");
-  // stage: V | K | K (transposing); FAR reads V only
-  constexpr int STAGES = PHASE_STAGES<DH, NCT, PHASE>, STAGE_BYTES = PHASE == FAR ? TILE : 3 * TILE;
+  constexpr int NW = PHASE_WAVES<PHASE>;
+  constexpr bool SOLO = PHASE_OCC<DH, PHASE> == 1;                // one wave per SIMD
+  constexpr int CP = NCT * 32, TQW = NW / NCT, TILE = TILE_BYTES<DH, NCT>;
+  static_assert(64 * 32 <= WAVE_SCRATCH && (1 + 32 * (CP + 1)) * 4 <= QUERY_LDS<DH, NCT, PHASE> / NW, "channel tables overlay the rest");
   constexpr int LPW = TILE / 1024 / NW;           // 1 KiB wave loads per wave and tile copy
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
-  float* wave_base = (float*)(smem + STAGES * STAGE_BYTES);
+  float* wave_base = (float*)(smem + 6 * TILE);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
-  constexpr int GP = 33, PC = CP + 1;             // padded pitches: the transposed reads spread over the banks
-  float* Stb = wave_base + wave * WAVE_SCRATCH;           // [32][32] time-bias scores of a slab
-  float* Gtb = Stb + 1024;                                // [32][GP] their gradients
-  float* scr = Stb;       // before the first slab [CP][32] channel table, after the last one [32][PC]
+  constexpr int PC = CP + 1;                      // padded pitch of the epilogue's table
+  float* Stb = wave_base + wave * WAVE_SCRATCH;           // [32 steps][32 queries] time-bias exponents of a slab
+  float* Gtb = Stb + 1024;                                // [32 queries][32 steps] their gradients, in swizzled fours
+  float* scr = Stb;                                       // before the first slab [64][32] channel table
+  float* g_lane = Gtb + ln * 32;                          // step j of the slab at 4 ((j >> 2) ^ (ln & 7)) + (j & 3)
+  const int g_swz = (ln & 7) << 2;
 
   const int T_ = a.T, C_ = a.C, W = a.window, N = a.T * a.C;
   const int CW = (C_ + 3) & ~3;                   // row pitch of the Ec tiles in the workspace
@@ -229,40 +239,64 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
   const int tk_lo = PHASE == WIN ? tk_near : 0;
   const int tk_hi = PHASE == FAR ? (far_top < tq0 ? -1 : far_top - W - 1) : tq_hi;
   const int tk_first = PHASE == WIN ? far_end : 0;                // slabs of 32 steps count from here
+  const int far_lim = PHASE == FAR ? tk_hi + 1 : PHASE == WIN ? 0 : tk_near;       // steps before it are walked in pairs
   const uint32_t ring_lds = (uint32_t)(uintptr_t)(BWD_LDS_PTR(unsigned char))smem;
-  auto issue_tile = [&](int tk, int stage_idx, bool with_k) {
-    const uint32_t st = ring_lds + stage_idx * STAGE_BYTES;
+  auto issue_v = [&](int tk, uint32_t dst) {
     const bf16_t* vsrc = vbase + (int64_t)tk * C_ * a.v_stride_n;
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) dma16(vsrc + v_off[i], st + (wave + NW * i) * 1024);
-    if (with_k) {
-      const bf16_t* ksrc = kbase + (int64_t)tk * C_ * a.k_stride_n;
+    for (int i = 0; i < LPW; ++i) dma16(vsrc + v_off[i], dst + (wave + NW * i) * 1024);
+  };
+  auto issue_far = [&](int tk, int slot) {
+    issue_v(tk, ring_lds + slot * 2 * TILE);
+    if (tk + 1 < far_lim) issue_v(tk + 1, ring_lds + (slot * 2 + 1) * TILE);
+  };
+  auto issue_near = [&](int tk, int half) {
+    if (PHASE == FAR || tk > tk_hi) return;
+    const uint32_t st = ring_lds + half * 3 * TILE;
+    issue_v(tk, st);
+    const bf16_t* ksrc = kbase + (int64_t)tk * C_ * a.k_stride_n;
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) {
-        dma16(ksrc + k_off_r[i], st + TILE + (wave + NW * i) * 1024);
-        dma16(ksrc + k_off_t[i], st + 2 * TILE + (wave + NW * i) * 1024);
-      }
+    for (int i = 0; i < LPW; ++i) {
+      dma16(ksrc + k_off_r[i], st + TILE + (wave + NW * i) * 1024);
+      dma16(ksrc + k_off_t[i], st + 2 * TILE + (wave + NW * i) * 1024);
     }
   };
-#pragma unroll
-  for (int s = 0; s < (PHASE == FAR ? 2 : STAGES - 1); ++s)
-    if (tk_lo + s <= tk_hi) issue_tile(tk_lo + s, s, PHASE != FAR && tk_lo + s >= tk_near);
+  // The last far unit takes slot 0, so that the first content unit can be on its way to the ring's second half
+  const int far_units = (far_lim + 1) >> 1;
+  int slot = far_units ? 2 - (far_units + 1) % 3 : 0;
+  if (far_units) {
+    issue_far(0, slot);
+    if (far_units > 1) issue_far(2, slot == 2 ? 0 : slot + 1);
+  } else {
+    issue_near(tk_lo, 1);
+  }
 
   // ---- set-up: operand fragments, delta, channel-bias tile
   bf16x8 dOf[KS];            // (q+u), (q+v) fragments are re-formed where needed, not kept
   f32x16 Ec[NCT];            // exp2(channel bias - mc): the far steps' probabilities up to a scalar
   float delta = 0.f, mc = -INFINITY, sumEc = 0.f;
-  uint32_t kbits[NCT];
   // every global load of the set-up goes out before the first use: one round trip, not one per
   // fragment.  The log-sum-exp is among them so that its wait does not fall into the loops, where
   // it would drain the whole ring (vmcnt 0) at every key step.
-  u32x4 raw_[KS], draw_[KS], oraw_[KS];
+  u32x4 raw_[KS], draw_[KS], oraw_[KS], bz_[KS], bu_[KS];
+  u32x4 er[KS][2];
+  auto window_row = [&](int t) { return max(C_ - 1 - max(cqw0 + 31 - k0 - t * 32, k0 + t * 32 + 31 - cqw0), 0); };
+  auto load_window = [&](int t) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt)
+        er[ks][tt] = *(const u32x4*)(kchan + (int64_t)min(window_row(t) + tt * 32 + ln, C_ - 1) * DH + ks * 16 + hh * 8);
+  };
+  load_window(0);
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
     const int d0 = ks * 16 + hh * 8;
     raw_[ks] = *(const u32x4*)(qrow + d0);
     draw_[ks] = *(const u32x4*)(drow + d0);
     oraw_[ks] = *(const u32x4*)(orow + d0);
+    bz_[ks] = *(const u32x4*)(bz + d0);
+    if (DH == 64) bu_[ks] = *(const u32x4*)(bu + d0);
   }
   const float lse = a.lse[row];
   uint64_t kmask;                                 // the (up to 64) key channels of this launch
@@ -277,10 +311,8 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
     bf16x8 qz[KS];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-      const int d0 = ks * 16 + hh * 8;
       const u32x4 raw = raw_[ks], draw = draw_[ks], oraw = oraw_[ks];
-      if (PHASE != WIN && qok) *(bf16x8*)((bf16_t*)a.ws_qu + row * DH + d0) = qfrag(raw, bu + d0, sc2);   // for the key pass
-      qz[ks] = qfrag(raw, bz + d0, sc2);
+      qz[ks] = qfrag(raw, bz_[ks], sc2);
       dOf[ks] = as_frag(draw);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -289,8 +321,6 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
       }
     }
     delta = xhalf_sum(delta);
-#pragma unroll
-    for (int t = 0; t < NCT; ++t) kbits[t] = (uint32_t)(kmask >> (t * 32 + 4 * hh));
     // Channel-bias tile, one key tile at a time: the 32 queries of this wave and the 32 keys of
     // tile t are at most 63 channels apart in either direction, so the rows C-1-d of the table
     // (q+z).k_chan^T they need lie in a window of 64 rows starting at jlo.  That window goes
@@ -298,53 +328,45 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
     // gathered from it; -inf where the key channel is padding or absent.
 #pragma unroll
     for (int t = 0; t < NCT; ++t) {
-      const int ck0 = k0 + t * 32;
-      const int dmax = max(cqw0 + 31 - ck0, ck0 + 31 - cqw0);       // > 0
-      const int jlo = max(C_ - 1 - dmax, 0);
+      const int ck0 = k0 + t * 32, jlo = window_row(t);
       f32x16 sct[2];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) sct[tt][i] = 0.f;
-      u32x4 er[KS][2];
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-          er[ks][tt] = *(const u32x4*)(kchan + (int64_t)min(jlo + tt * 32 + ln, C_ - 1) * DH + ks * 16 + hh * 8);
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
           sct[tt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(er[ks][tt]), qz[ks], sct[tt], 0, 0, 0);
+      if (t + 1 < NCT) load_window(t + 1);        // on their way while this tile is gathered
+      if (!has_chan)
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) sct[tt][i] = 0.f;
       wave_sync_lds();                            // the previous tile's gather is done with the scratch
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int j = tt * 32 + (i >> 2) * 8 + hh * 4 + (i & 3);
-          scr[j * 32 + ln] = has_chan ? sct[tt][i] : 0.f;
-        }
+        for (int i = 0; i < 16; ++i) scr[(tt * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)) * 32 + ln] = sct[tt][i];
       wave_sync_lds();
-      // row of the window for key ck = c_i + 4hh: (C-1-jlo) - |cq - ck|, clamped into the window
-      // for padded queries / keys (their values are never used)
-      const uint32_t cq4 = (uint32_t)(cq - 4 * hh + 4);
-      const int top = C_ - 1 - jlo;
+      // Row of the window for key ck = ck0 + c_i + 4hh: (C-1-jlo) - |cq - ck|, at most 62.  In floats, where the
+      // absolute value is free; rows below 0 belong to padded queries and keys, for which any value does.
+      const float top = (float)((C_ - 1 - jlo) * 32 + ln), dc = (float)(32 * (cq - ck0 - 4 * hh));
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const uint32_t ci4 = (uint32_t)(ck0 + (i >> 2) * 8 + (i & 3) + 4);
-        const int dist = (int)(max(cq4, ci4) - min(cq4, ci4));
-        const int jr = min(max(top - dist, 0), 63);
-        const float val = scr[jr * 32 + ln];
-        const bool kv = (kbits[t] >> ((i >> 2) * 8 + (i & 3))) & 1u;
-        Ec[t][i] = kv ? val : -INFINITY;
+      for (int i = 0; i < 16; ++i) Ec[t][i] = scr[(int)fmaxf(top - fabsf(dc - (float)(32 * ((i >> 2) * 8 + (i & 3)))), 0.f)];
+      if ((uint32_t)(kmask >> (t * 32)) != 0xffffffffu) {
+        const uint32_t kbits = (uint32_t)(kmask >> (t * 32 + 4 * hh));
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Ec[t][i] = ((kbits >> ((i >> 2) * 8 + (i & 3))) & 1u) ? Ec[t][i] : -INFINITY;
       }
     }
 #pragma unroll
     for (int t = 0; t < NCT; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) mc = fmaxf(mc, Ec[t][i]);
-    mc = fmaxf(mc, __shfl_xor(mc, 32));
+    mc = xhalf_max(mc);
     if (mc == -INFINITY) mc = 0.f;                // no valid key channel at all
 #pragma unroll
     for (int t = 0; t < NCT; ++t)
@@ -354,6 +376,14 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
         sumEc += Ec[t][i];
       }
     sumEc = xhalf_sum(sumEc);
+    bf16x8 qu[KS];
+    if constexpr (PHASE != WIN) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        const int d0 = ks * 16 + hh * 8;
+        qu[ks] = DH == 64 ? qfrag(raw_[ks], bu_[ks], sc2) : qfrag(*(const u32x4*)(qrow + d0), *(const u32x4*)(bu + d0), sc2);
+      }
+    }
     // for the key pass: (q+u) * scale, delta, and the tile exp2(channel bias - mc) by
     // [query][key channel]; and the rows of dbias_time that no key step reaches
     if (PHASE != WIN && qok) {
@@ -367,7 +397,12 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
             *(float4*)(wc + ci) = make_float4(Ec[t][a4 * 4], Ec[t][a4 * 4 + 1], Ec[t][a4 * 4 + 2], Ec[t][a4 * 4 + 3]);
         }
     }
-    if (PHASE != WIN && qok && hh == 0) a.ws_delta[row] = -delta;
+    // the stores last: loads return behind the stores before them
+    if (PHASE != WIN && qok) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) *(bf16x8*)((bf16_t*)a.ws_qu + row * DH + ks * 16 + hh * 8) = qu[ks];
+      if (hh == 0) a.ws_delta[row] = -delta;
+    }
   }
 
   f32x16 dq[MT], dSc[NCT];
@@ -388,8 +423,14 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
 
   // the columns of dbias_time that no key step reaches (once: by the launch that does not add)
   if (PHASE != WIN && !accum)
-    for (int q = hh; q < nq_live; q += 2)
-      for (int j = ln; j < T_ - 1 - tq; j += 32) a.dbias_time[(wrow0 + q) * T_ + j] = 0.f;
+    for (int q = lane >> 3; q < nq_live; q += 8) {
+      float* dst = a.dbias_time + (wrow0 + q) * T_;
+      const int n = T_ - 1 - tq;
+      if (n >= 4)
+        for (int j = 4 * (lane & 7); j < n; j += 32) *(f32x4u*)(dst + min(j, n - 4)) = f32x4u{0.f, 0.f, 0.f, 0.f};
+      else if ((lane & 7) < n)
+        dst[lane & 7] = 0.f;
+    }
 
   // ---- loop-invariant fragment offsets
   int r_lane[KS], t_lane[MT];
@@ -409,82 +450,81 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
+  // the first n floats of each of the first rows rows of a slab: eight lanes a row, four floats a lane; the last four
+  // of a row overlap the ones before them with the same values
+  auto store_rows = [&](int rows, int n, auto at, auto value) __attribute__((always_inline)) {
+    int l = lane;
+    asm volatile("" : "+v"(l));                    // the addresses are formed here, not kept in registers over the walk
+    if (n >= 4) {
+      const int c = min(4 * (l & 7), n - 4);
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int r = it * 8 + (l >> 3);
+        f32x4u v;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) v[x] = value(r, c + x);
+        if (r < rows && 4 * (l & 7) < n) *(f32x4u*)(at(r) + c) = v;
+      }
+    } else {
+#pragma unroll 1
+      for (int r = l >> 2; r < rows; r += 16)
+        if ((l & 3) < n) at(r)[l & 3] = value(r, l & 3);
+    }
+  };
+
   // writes the gradients of the slab that started at key step tks, and its per-pair scalars for
   // the key pass (the exponent e = time bias - L + mc for pairs inside the window, else exp2(e))
-  auto flush_slab = [&](int tks) {
+  auto flush_slab = [&](int tks) __attribute__((always_inline)) {
     const int nj = min(32, (PHASE == FAR ? far_end : tq + 1) - tks);
-    // fixed trip counts with predicates: the LDS reads of several iterations go out together
-#pragma unroll 8
-    for (int it = 0; it < 16; ++it) {
-      const int jj = 2 * it + hh, tkk = tks + jj;
-      const float e = Stb[jj * 32 + ln] - lse + mc;
-      const bool near_pair = has_content && (W <= 0 || tq - tkk <= W || tq == T_ - 1);
-      const float val = near_pair ? e : __builtin_amdgcn_exp2f(e);
-      if (qok && jj < nj) a.ws_time[(((int64_t)bh * T_ + tq) * T_ + tkk) * C_ + cq] = val;
-    }
+    store_rows(nj, min(32, C_ - cqw0), [&](int jj) { return a.ws_time + (((int64_t)bh * T_ + tq) * T_ + tks + jj) * C_ + cqw0; },
+               [&](int jj, int q) {
+                 const float e = Stb[jj * 32 + q];
+                 const bool near_pair = has_content && (W <= 0 || tq - tks - jj <= W || tq == T_ - 1);
+                 return near_pair ? e : __builtin_amdgcn_exp2f(e);
+               });
     const int j0 = time_row(tq, tks, T_);
-#pragma unroll 8
-    for (int it = 0; it < 16; ++it) {
-      const int q = 2 * it + hh;
-      const float g = Gtb[ln * GP + q] * a.sm_scale;
-      if (q < nq_live && ln < nj) {
-        float* dst = a.dbias_time + (wrow0 + q) * T_ + j0 + ln;
-        // launches of one stream: the key parts add up.  An atomic add without a return value,
-        // not a load and a store: nothing waits for the old value (every address has one writer)
-        if (accum) atomicAdd(dst, g);
-        else *dst = g;
-      }
-    }
-  };
-
-  int stage = 0;
-  // advances the ring to key step tk and returns the stage that holds its tiles
-  auto ring_step = [&](int tk) -> const unsigned char* {
-    // tile tk has landed once at most the loads of the younger tiles are in flight (a count that
-    // is too small only waits longer)
-    constexpr int WITH_K = PHASE == FAR ? 1 : 3;  // tiles of a step from tk_near on
-    if ((PHASE == FAR || tk + 1 >= tk_near) && tk + STAGES - 2 <= tk_hi) {
-      wait_vmcnt_imm<(STAGES - 2) * WITH_K * LPW>();
+    if (!accum) {
+      store_rows(nq_live, nj, [&](int q) { return a.dbias_time + (wrow0 + q) * T_ + j0; },
+                 [&](int q, int jj) { return Gtb[q * 32 + (jj ^ ((q & 7) << 2))] * a.sm_scale; });
     } else {
-      int younger = 0;
-#pragma unroll
-      for (int d = 1; d <= STAGES - 2; ++d)
-        if (tk + d <= tk_hi) younger += LPW * (tk + d >= tk_near ? WITH_K : 1);
-      wait_vmcnt(younger);
+      // launches of one stream: the key parts add up.  An atomic add without a return value, not a load and a
+      // store: nothing waits for the old value (every address has one writer)
+#pragma unroll 8
+      for (int it = 0; it < 16; ++it) {
+        const int q = 2 * it + hh;
+        const float g = Gtb[q * 32 + (ln ^ ((q & 7) << 2))] * a.sm_scale;
+        if (q < nq_live && ln < nj) atomicAdd(a.dbias_time + (wrow0 + q) * T_ + j0 + ln, g);
+      }
     }
-    lds_barrier();            // tile tk visible to all; everyone is done with tile tk-1's stage
-    if (tk + STAGES - 1 <= tk_hi)
-      issue_tile(tk + STAGES - 1, stage == 0 ? STAGES - 1 : stage - 1, PHASE != FAR && tk + STAGES - 1 >= tk_near);
-    const unsigned char* Vrow = smem + stage * STAGE_BYTES;
-    stage = stage + 1 == STAGES ? 0 : stage + 1;
-    return Vrow;
   };
 
-  // every 32 key steps: write the finished slab, form the next slab of time-bias scores
-  auto time_slab = [&](int tk) {
+  // Every 32 key steps: form the next slab of time-bias scores, write the finished one.  In this order: loads return
+  // behind the stores before them.
+  auto time_slab = [&](int tk) __attribute__((always_inline)) {
     if (((tk - tk_first) & 31) == 0) {
-      if (tk > tk_first) {
-        wave_sync_lds();
-        flush_slab(tk - 32);
-        wave_sync_lds();
-      }
       f32x16 stc;
 #pragma unroll
       for (int i = 0; i < 16; ++i) stc[i] = 0.f;
       if (has_time) {
         const int j = min(time_row(tq, tk, T_) + ln, T_ - 1);
-        u32x4 rr[KS], qr[KS];
+        u32x4 rr[KS], qr[KS], br[KS];
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {         // every load before the first use
           rr[ks] = *(const u32x4*)(ktime + (int64_t)j * DH + ks * 16 + hh * 8);
           qr[ks] = *(const u32x4*)(qrow + ks * 16 + hh * 8);
+          br[ks] = *(const u32x4*)(bv + ks * 16 + hh * 8);
         }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-          stc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(rr[ks]), qfrag(qr[ks], bv + ks * 16 + hh * 8, sc2), stc, 0, 0, 0);
+          stc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(rr[ks]), qfrag(qr[ks], br[ks], sc2), stc, 0, 0, 0);
+      }
+      if (tk > tk_first) {
+        wave_sync_lds();
+        flush_slab(tk - 32);
+        wave_sync_lds();
       }
 #pragma unroll
-      for (int i = 0; i < 16; ++i) Stb[((i >> 2) * 8 + hh * 4 + (i & 3)) * 32 + ln] = stc[i];
+      for (int i = 0; i < 16; ++i) Stb[((i >> 2) * 8 + hh * 4 + (i & 3)) * 32 + ln] = stc[i] - lse + mc;
       wave_sync_lds();
     }
   };
@@ -495,13 +535,26 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
   //     dbias_chan share   = Ec (sum_tk et dP - delta sum_tk et)   (formed after the loop)
   // (all of them, like dS below, times the score scale where they are written)
   // costs two FMAs per element and no exponential per element.
-  // The loop is software-pipelined: the products of step tk are issued to the matrix cores, and
-  // the vector work on the products of step tk-1 runs meanwhile.
   float esum = 0.f;
-  // reduces the products of far step tkp (none if tkp < 0)
-  auto far_reduce = [&](const f32x16 (&dP)[NCT], int tkp) {
-    if (tkp < 0) return;
-    const float et = __builtin_amdgcn_exp2f(Stb[(tkp & 31) * 32 + ln] - lse + mc);
+  // Every fragment is read before the first product: read where they are used, each waits out the LDS latency.
+  auto far_read = [&](const unsigned char* Vrow, bf16x8 (&vf)[KS][NCT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) vf[ks][t] = *(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB);
+  };
+  auto far_products = [&](const bf16x8 (&vf)[KS][NCT], f32x16 (&dP)[NCT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < NCT; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) dP[t][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int t = 0; t < NCT; ++t) dP[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks][t], dOf[ks], dP[t], 0, 0, 0);
+  };
+  auto far_reduce = [&](const f32x16 (&dP)[NCT], float st, int tk) __attribute__((always_inline)) {
+    const float et = __builtin_amdgcn_exp2f(st);
     float dot[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < NCT; ++t)
@@ -512,48 +565,32 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
       }
     esum += et;
     const float gt = et * (xhalf_sum((dot[0] + dot[1]) + (dot[2] + dot[3])) - delta * sumEc);
-    Gtb[(tkp & 31) * GP + ln] = gt;               // both halves hold it: no branch
+    g_lane[(tk & 31) ^ g_swz] = gt;               // both halves hold it: no branch
   };
-  // one far step: products of tile tk into cur, reduction of step tk-1 (in prev) alongside
-  auto far_step = [&](int tk, int& tkp, f32x16 (&cur)[NCT], const f32x16 (&prev)[NCT]) {
-    const unsigned char* Vrow = ring_step(tk);
-    if ((tk & 31) == 0) {                         // the slab about to be written must be complete
-      far_reduce(prev, tkp);
-      tkp = -1;
-      time_slab(tk);
-    }
+  auto far_one = [&](const unsigned char* Vrow, int tk) __attribute__((always_inline)) {
     bf16x8 vf[KS][NCT];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int t = 0; t < NCT; ++t) vf[ks][t] = *(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB);
-#pragma unroll
-    for (int t = 0; t < NCT; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) cur[t][i] = 0.f;
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-#pragma unroll
-      for (int t = 0; t < NCT; ++t)
-        cur[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[ks][t], dOf[ks], cur[t], 0, 0, 0);
-    far_reduce(prev, tkp);
-    tkp = tk;
+    f32x16 dP[NCT];
+    far_read(Vrow, vf);
+    const float st = Stb[(tk & 31) * 32 + ln];
+    __builtin_amdgcn_sched_barrier(0);
+    far_products(vf, dP);
+    far_reduce(dP, st, tk);
   };
 
   // A key step inside the content window
   f32x16 Bc[NCT];
   bf16x8 Qu[KS];
-  auto near_step = [&](const unsigned char* Vrow, int tk) {
+  auto near_step = [&](const unsigned char* Vrow, int tk) __attribute__((always_inline)) {
     const unsigned char* Krow = Vrow + TILE;
     const unsigned char* Ktr = Vrow + 2 * TILE;
-    const float off2 = Stb[((tk - tk_first) & 31) * 32 + ln] - lse;
+    const float off2 = Stb[((tk - tk_first) & 31) * 32 + ln];
     float gt = 0.f;
 #pragma unroll
     for (int t = 0; t < NCT; ++t) {               // one key-channel tile at a time: fewer live tiles
       // A wave that has its SIMD to itself sends out every LDS read of a phase before the first product or
       // exponential of it: read where they are used, each pair of fragments waits out the LDS latency (last time
       // step of 512: 512 such steps, the longest chain of the launch; 4.92 -> 4.64 ms at B1 H16 C64 of 128 Dh128).
-      // Two waves cover each other's waits, and 256 registers do not hold the fragments (78 spilled, 0.90 -> 1.23 ms).
+      // Two waves cover each other's waits (read ahead at Dh 64: 786 us and 16 registers spilled against 785).
       const unsigned char *Kt = Krow + t * 32 * ROWB, *Vt = Vrow + t * 32 * ROWB;
       bf16x8 kf[KS], vf[KS], kt[2][MT];
       if constexpr (SOLO) {
@@ -597,74 +634,78 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
       }
     }
     gt = xhalf_sum(gt);
-    Gtb[((tk - tk_first) & 31) * GP + ln] = gt;
+    g_lane[((tk - tk_first) & 31) ^ g_swz] = gt;
   };
 
   // far steps first, then the steps inside the window; waves that are done keep the ring and the barriers going
   int tk = tk_lo;
-  if constexpr (PHASE == FAR) {
-    // Two steps per barrier, the tiles of the next two requested behind it.  With a barrier a step the two waves of a
-    // SIMD read, multiply and reduce at the same time, and the three add up (T 512 and 128 channels: 2.80 ms a launch,
-    // 2.47 .. 2.56 with half the barriers).
-    auto pair_step = [&](int t0) {
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      lds_barrier();
-#pragma unroll
-      for (int d = 2; d < 4; ++d)
-        if (t0 + d <= tk_hi) issue_tile(t0 + d, (t0 + d) & 3, false);
-    };
-    for (; tk < far_end; tk += 2) {
-      pair_step(tk);
+  if constexpr (PHASE != WIN) {
+    // Two steps per barrier, two units on their way.  With a barrier a step the two waves of a SIMD read, multiply and
+    // reduce at the same time, and the three add up (T 512, 128 channels of Dh 128: 2.80 ms a launch, 2.47 .. 2.56
+    // with half the barriers).
+    for (; tk < far_lim; tk += 2) {
+      if (tk + 3 < far_lim) wait_vmcnt_imm<2 * LPW>();            // the unit behind this one may be under way
+      else if (tk + 2 < far_lim) wait_vmcnt_imm<LPW>();
+      else wait_vmcnt_imm<0>();
+      lds_barrier();                              // the unit is visible to all; everyone is done with the one before
+      if (tk + 4 < far_lim) issue_far(tk + 4, slot == 0 ? 2 : slot - 1);
+      else if (tk + 2 >= far_lim) issue_near(far_lim, 1);
+      const unsigned char* Vrow = smem + slot * 2 * TILE;
+      slot = slot == 2 ? 0 : slot + 1;
+      if (tk >= far_end) continue;
       if ((tk & 31) == 0) time_slab(tk);
-#pragma unroll
-      for (int d = 0; d < 2; ++d) {
-        if (tk + d >= far_end) break;
-        const unsigned char* Vrow = smem + ((tk + d) & 3) * STAGE_BYTES;
-        f32x16 dP[NCT];
-#pragma unroll
-        for (int t = 0; t < NCT; ++t) {
-#pragma unroll
-          for (int i = 0; i < 16; ++i) dP[t][i] = 0.f;
-#pragma unroll
-          for (int ks = 0; ks < KS; ++ks)
-            dP[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*(const bf16x8*)(Vrow + r_lane[ks] + t * 32 * ROWB), dOf[ks], dP[t], 0, 0, 0);
-        }
-        far_reduce(dP, tk + d);
+      if (PHASE == FAR || tk + 1 >= min(far_lim, far_end)) {
+        far_one(Vrow, tk);
+        if (tk + 1 < min(far_lim, far_end)) far_one(Vrow + TILE, tk + 1);
+      } else {
+        // the second step's products run while the first one's are reduced
+        bf16x8 vf[KS][NCT];
+        f32x16 dPa[NCT], dPb[NCT];
+        far_read(Vrow, vf);
+        const float sa = Stb[(tk & 31) * 32 + ln], sb = Stb[((tk & 31) + 1) * 32 + ln];
+        __builtin_amdgcn_sched_barrier(0);
+        far_products(vf, dPa);
+        far_read(Vrow + TILE, vf);
+        __builtin_amdgcn_sched_barrier(0);
+        far_products(vf, dPb);
+        far_reduce(dPa, sa, tk);
+        far_reduce(dPb, sb, tk + 1);
       }
     }
-    for (; tk <= tk_hi; tk += 2) pair_step(tk);
-  } else if constexpr (PHASE == ONE) {
-    f32x16 dPa[NCT], dPb[NCT];
-    int tkp = -1;
-    for (; tk + 1 < far_end; tk += 2) {
-      far_step(tk, tkp, dPa, dPb);
-      far_step(tk + 1, tkp, dPb, dPa);
-    }
-    if (tk < far_end) {
-      far_step(tk, tkp, dPa, dPb);
-      ++tk;
-      far_reduce(dPa, tkp);
-    } else {
-      far_reduce(dPb, tkp);
-    }
+    tk = far_lim;
   }
+  int half = 1;
+  auto near_unit = [&](int tk) __attribute__((always_inline)) -> const unsigned char* {
+    wait_vmcnt_imm<0>();
+    lds_barrier();
+    issue_near(tk + 1, half ^ 1);
+    const unsigned char* p = smem + half * 3 * TILE;
+    half ^= 1;
+    return p;
+  };
+  if constexpr (PHASE == ONE)
+    for (; tk < far_end; ++tk) {                  // far for this wave, not for the workgroup
+      const unsigned char* Vrow = near_unit(tk);
+      time_slab(tk);
+      far_one(Vrow, tk);
+    }
   // the far steps' share of the channel-table gradient; from here on the tile holds the bias
 #pragma unroll
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) dSc[t][i] = Ec[t][i] * (dSc[t][i] - delta * esum);
   if constexpr (PHASE != FAR) {
-  // Bc = mc + log2(Ec): the table it was gathered from lies under the slabs by now (-inf where
+  // Bc = log2(Ec): the table it was gathered from lies under the slabs by now (-inf where
   // Ec = 0: masked keys, and biases more than 126 octaves below the row's largest)
 #pragma unroll
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) Bc[t][i] = mc + __builtin_amdgcn_logf(Ec[t][i]);
+    for (int i = 0; i < 16; ++i) Bc[t][i] = __builtin_amdgcn_logf(Ec[t][i]);
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
-    Qu[ks] = qfrag(*(const u32x4*)(qrow + ks * 16 + hh * 8), bu + ks * 16 + hh * 8, sc2);
+    Qu[ks] = qfrag(*(const u32x4*)(qrow + ks * 16 + hh * 8), *(const u32x4*)(bu + ks * 16 + hh * 8), sc2);
   for (; tk <= tq_hi; ++tk) {
-    const unsigned char* Vrow = ring_step(tk);
+    const unsigned char* Vrow = near_unit(tk);
     if (active && tk >= far_end && tk <= tq) {
       time_slab(tk);
       near_step(Vrow, tk);
@@ -672,10 +713,11 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
   }
   }
 
-  if (!active) return;
   wave_sync_lds();
   const int tk_end = PHASE == FAR ? far_end : tq + 1;
-  if (tk_end > tk_first) flush_slab(tk_first + ((tk_end - 1 - tk_first) & ~31));
+  if (active && tk_end > tk_first) flush_slab(tk_first + ((tk_end - 1 - tk_first) & ~31));
+  lds_barrier();                                  // from here on the waves share out the whole of the LDS
+  if (!active) return;
 
   // dq^T[d][q]: this lane's query, d = 32mt + 8a4 + 4hh + 0..3
   if (PHASE != FAR && qok) {
@@ -700,26 +742,29 @@ __global__ __launch_bounds__((PHASE_WAVES<DH, NCT, PHASE> * 64)) void mvpa_bwd_q
   // C-1-d collects the two key channels cq-d and cq+d (those of them that this launch holds).
   // The tile goes to a per-wave table [32 queries][PC] by local key channel, and each output row
   // is gathered from it (LDS float atomics for the scatter form were measured at ~0.3 us apiece).
-  wave_sync_lds();
+  // The column behind the last channel, and the one before the first, is zero: key channels that this launch does
+  // not hold.
+  float* tab = (float*)(smem + wave * (QUERY_LDS<DH, NCT, PHASE> / NW)) + 1;
 #pragma unroll
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) scr[ln * PC + t * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i] * a.sm_scale;
+    for (int i = 0; i < 16; ++i) tab[ln * PC + t * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i] * a.sm_scale;
+  tab[ln * PC + CP] = 0.f;
+  if (lane == 0) tab[-1] = 0.f;
   wave_sync_lds();
   for (int c0 = 0; c0 < C_; c0 += 64) {
     const int col = c0 + lane;
     const int d = C_ - 1 - col;                   // this lane's column holds distance d
+    const int lo = cqw0 - k0 - d, hi = d > 0 ? cqw0 - k0 + d : CP;           // local key channels of query 0 (d = 0: one)
+    float* dst = a.dbias_chan + wrow0 * C_ + col;
+    if (col < C_) {
 #pragma unroll 8
-    for (int q = 0; q < 32; ++q) {
-      const int lo = cq0 + q - d - k0, hi = cq0 + q + d - k0;      // local key channels
-      float g = scr[q * PC + max(0, min(lo, CP - 1))];
-      const float g2 = scr[q * PC + max(0, min(hi, CP - 1))];
-      if (lo < 0 || lo >= CP || d < 0) g = 0.f;
-      if (d > 0 && hi >= 0 && hi < CP) g += g2;
-      if (q < nq_live && col < C_) {
-        float* dst = a.dbias_chan + (wrow0 + q) * C_ + col;
-        if (accum || PHASE == WIN) atomicAdd(dst, g);
-        else *dst = g;
+      for (int q = 0; q < 32; ++q) {
+        const float g = tab[q * PC + min(max(lo + q, -1), CP)] + tab[q * PC + min(max(hi + q, -1), CP)];
+        if (q < nq_live) {
+          if (accum || PHASE == WIN) atomicAdd(dst + q * C_, g);
+          else dst[q * C_] = g;
+        }
       }
     }
   }
@@ -754,11 +799,10 @@ int mvpa_bwd_query_mfma_supported(const mvpa_bwd_args* a) {
 template <int DH, int NCT, int PHASE>
 static void launch_query(const mvpa_bwd_args* a, hipStream_t stream, int q0, int k0, int accum) {
   using namespace mvpa::bwdq;
-  constexpr int nw = PHASE_WAVES<DH, NCT, PHASE>, tqw = nw / NCT, cp = NCT * 32, ROWB = 2 * DH;
+  constexpr int nw = PHASE_WAVES<PHASE>, tqw = nw / NCT;
   const int nt = (a->T + tqw - 1) / tqw;
-  constexpr size_t lds = (size_t)PHASE_STAGES<DH, NCT, PHASE> * (PHASE == FAR ? 1 : 3) * cp * ROWB +
-                         (size_t)nw * WAVE_SCRATCH * sizeof(float);
-  static_assert(lds <= 160 * 1024, "query-pass ring exceeds the LDS");
+  constexpr size_t lds = QUERY_LDS<DH, NCT, PHASE>;
+  static_assert(lds <= 160 * 1024 / (DH == 64 ? 2 : 1), "query-pass ring exceeds the LDS");
   dim3 grid((unsigned)(nt * a->B * a->H));
   auto kern = mvpa_bwd_query_mfma_kernel<DH, NCT, PHASE>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);

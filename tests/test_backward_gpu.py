@@ -320,6 +320,27 @@ def test_long_walks_against_the_fp32_kernels(T, C, Dh, window, masked):
         assert (x.double() - y.double()).norm() <= 2e-2 * y.double().norm(), n      # the bf16 bound of this file
 
 
+@pytest.mark.parametrize("C,Dh,T,window", [
+    *[(33, 64, T, 2) for T in range(4, 16)],      # 0 .. 6 units of far steps, whole and half; T even and odd
+    (35, 64, 37, 31), (66, 64, 36, 3), (3, 64, 35, 2), (2, 64, 67, 30), (34, 64, 99, 1),      # rows and slabs of 1 .. 3
+    (33, 128, 9, 2), (2, 128, 34, 1), (67, 128, 267, 3),
+])
+def test_query_pass_units_and_short_rows(C, Dh, T, window):
+    """The query pass walks far steps in units of two and writes rows in fours: every remainder of both, against the
+    fp32 kernels on the same (bf16) inputs."""
+    inp = make_mvpa_inputs(seed=T + C, qkv_unit=True, B=1, C=C, T=T, H=2, Hkv=1, Dh=Dh).round_to(torch.bfloat16)
+    d_out = torch.randn(inp.q.shape, generator=torch.Generator().manual_seed(T)).bfloat16().float()
+    valid = None
+    if T % 3 == 0 and C > 2:
+        valid = torch.ones(1, C, dtype=torch.bool)
+        valid[:, [0, C - 2]] = False
+    _, ref = _gpu_grads(inp, d_out, window, torch.float32, chan_valid=valid)
+    _, got = _gpu_grads(inp, d_out, window, torch.bfloat16, chan_valid=valid)
+    for n in NAMES:
+        a, b = got[n].double(), ref[n].double()
+        assert torch.isfinite(a).all() and (a - b).norm() <= 2e-2 * b.norm(), n             # the bf16 bound of this file
+
+
 @pytest.mark.parametrize("cfg,flags", [
     (dict(B=1, C=1, T=1, H=2, Hkv=1, Dh=64), {}),                   # one row
     (dict(B=1, C=64, T=64, H=3, Hkv=3, Dh=64), {}),                 # whole steps of 64 columns, whole tiles of 128 rows
