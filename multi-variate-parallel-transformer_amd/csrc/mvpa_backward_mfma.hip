@@ -14,8 +14,8 @@
 // Outputs are those of mvpa_backward (include/mvpa_hip.h): the content share of dq and the two
 // bias-table gradients.  For the key pass the workspace receives, in base-2 score units, -delta,
 // the channel-table rows, (time bias - L) laid out [b,h,tq,tk,cq] and (q+u) * scale in bf16.
-// K and V tiles come through a ring of LDS stages filled by direct-to-LDS loads, K in two copies (row fragments
-// for K Q^T, transposed fragments for K^T dS^T); far key steps fetch V only.
+// K and V tiles come through a ring of LDS stages filled by direct-to-LDS loads; one copy of K serves the row
+// fragments of K Q^T and the transposed ones of K^T dS^T; far key steps fetch V only.
 #include "mvpa_common.h"
 
 #include <type_traits>
@@ -35,7 +35,6 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 // Head dim DH is 64 or 128: KS = DH / 16 contraction blocks per product, MT = DH / 32 output tiles
 // of the gradients, rows of ROWB = 2 DH bytes (CPR = DH / 8 chunks of 16 bytes) in the LDS tiles.
-constexpr int KSTAGES = 3;                        // ring depth of the key pass
 // floats of per-wave scratch in the query pass: a slab of 32 key steps' time-bias exponents [step][query] and of their
 // gradients [query][step].  The channel table of the set-up ([64][32]) overlays them.
 constexpr int WAVE_SCRATCH = 2048;
@@ -121,9 +120,12 @@ __device__ inline float xhalf_max(float x) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 
-// chunk swizzles of a row of 2 DH bytes: row fragments / transposing reads (as in the forward)
-template <int DH> __device__ inline int swz_row(int row) { return DH == 64 ? ((row >> 1) & 7) : (row & 15); }
-template <int DH> __device__ inline int swz_tr(int row) { return DH == 64 ? (((row >> 1) & 1) << 2) : ((row & 3) << 2); }
+// The 16-byte chunks of a row of 2 DH bytes are swizzled so that both kinds of reads of one copy are free of bank
+// conflicts: a row fragment takes one chunk of 16 rows (256 bytes of banks: all its chunks at Dh 128, two rows' at Dh
+// 64, differ), a transposing read four chunks of four rows (differ in bits 2, 3; at Dh 64 rows of one parity in bit 2).
+template <int DH> __device__ inline int swz(int row) {
+  return DH == 64 ? ((row >> 1) & 1) << 2 | ((row >> 2) & 3) : (row & 3) << 2 | ((row >> 2) & 3);
+}
 
 // ONE: the whole walk.  FAR, WIN: the steps before a wave's content window and those from it on, as a launch
 // each, FAR first.  At Dh 128 a wave of the whole walk takes 475 registers and has its SIMD to itself: the far steps'
@@ -139,8 +141,7 @@ enum query_phase { ONE, FAR, WIN };
 template <int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : 4;
 // waves per SIMD: at Dh 64 two workgroups share a CU
 template <int DH, int PHASE> constexpr int PHASE_OCC = PHASE == FAR || DH == 64 ? 2 : 1;
-// The ring holds six tiles: three units of far steps, V of two steps each, or two units of a step with content,
-// V | K | K (transposing).
+// The ring holds three units of two tiles: V of two far steps, or V and K of a step with content.
 template <int DH, int NCT> constexpr int TILE_BYTES = NCT * 32 * 2 * DH;
 template <int DH, int NCT, int PHASE> constexpr int QUERY_LDS = 6 * TILE_BYTES<DH, NCT> + PHASE_WAVES<PHASE> * WAVE_SCRATCH * 4;
 
@@ -220,15 +221,14 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   const float sc2 = a.sm_scale * kLog2e;          // scores live in the base-2 domain
 
   // ---- the ring: per-wave source offsets (the swizzle is applied on the source side), prologue
-  int k_off_r[LPW], k_off_t[LPW], v_off[LPW];
+  int k_off[LPW], v_off[LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
     const int pc = (wave + NW * i) * 64 + lane;
     const int r = pc / CPR, phys = pc % CPR;
     const int rc = min(k0 + r, C_ - 1);           // key channels k0 .. of this launch
-    k_off_r[i] = rc * (int)a.k_stride_n + ((phys ^ swz_row<DH>(r)) << 3);
-    k_off_t[i] = rc * (int)a.k_stride_n + ((phys ^ swz_tr<DH>(r)) << 3);
-    v_off[i] = rc * (int)a.v_stride_n + ((phys ^ swz_row<DH>(r)) << 3);
+    k_off[i] = rc * (int)a.k_stride_n + ((phys ^ swz<DH>(r)) << 3);
+    v_off[i] = rc * (int)a.v_stride_n + ((phys ^ swz<DH>(r)) << 3);
   }
   // first key step whose K is needed: the band of the earliest query step of the workgroup
   const int tk_near = !has_content ? tq_hi + 1 : (W <= 0 || tq_hi == T_ - 1) ? 0 : max(0, tq0 - W);
@@ -246,30 +246,43 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
 #pragma unroll
     for (int i = 0; i < LPW; ++i) dma16(vsrc + v_off[i], dst + (wave + NW * i) * 1024);
   };
-  auto issue_far = [&](int tk, int slot) {
-    issue_v(tk, ring_lds + slot * 2 * TILE);
-    if (tk + 1 < far_lim) issue_v(tk + 1, ring_lds + (slot * 2 + 1) * TILE);
-  };
-  auto issue_near = [&](int tk, int half) {
-    if (PHASE == FAR || tk > tk_hi) return;
-    const uint32_t st = ring_lds + half * 3 * TILE;
+  auto next_unit = [&](int tk) { return PHASE != WIN && tk < far_lim ? min(tk + 2, far_lim) : tk + 1; };
+  auto unit_loads = [&](int tk) { return tk > tk_hi ? 0 : PHASE != WIN && tk + 1 == far_lim ? LPW : 2 * LPW; };
+  auto issue_unit = [&](int tk, int slot) {
+    if (tk > tk_hi) return;
+    const uint32_t st = ring_lds + slot * 2 * TILE;
     issue_v(tk, st);
-    const bf16_t* ksrc = kbase + (int64_t)tk * C_ * a.k_stride_n;
+    if (PHASE != WIN && tk < far_lim) {
+      if (tk + 1 < far_lim) issue_v(tk + 1, st + TILE);
+    } else {
+      const bf16_t* ksrc = kbase + (int64_t)tk * C_ * a.k_stride_n;
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) {
-      dma16(ksrc + k_off_r[i], st + TILE + (wave + NW * i) * 1024);
-      dma16(ksrc + k_off_t[i], st + 2 * TILE + (wave + NW * i) * 1024);
+      for (int i = 0; i < LPW; ++i) dma16(ksrc + k_off[i], st + TILE + (wave + NW * i) * 1024);
     }
   };
-  // The last far unit takes slot 0, so that the first content unit can be on its way to the ring's second half
-  const int far_units = (far_lim + 1) >> 1;
-  int slot = far_units ? 2 - (far_units + 1) % 3 : 0;
-  if (far_units) {
-    issue_far(0, slot);
-    if (far_units > 1) issue_far(2, slot == 2 ? 0 : slot + 1);
-  } else {
-    issue_near(tk_lo, 1);
-  }
+  issue_unit(tk_lo, 0);
+  issue_unit(next_unit(tk_lo), 1);
+  int slot = 0;
+  // the stage of the unit of key step tk; requests the unit after the next one
+  auto begin_unit = [&](int tk) __attribute__((always_inline)) -> const unsigned char* {
+    const int before = slot == 0 ? 2 : slot - 1;
+    if (PHASE != WIN && tk + 5 < far_lim) {       // far steps all around
+      wait_vmcnt_imm<2 * LPW>();
+      lds_barrier();                              // the unit is visible to all; everyone is done with the one before
+      issue_v(tk + 4, ring_lds + before * 2 * TILE);
+      issue_v(tk + 5, ring_lds + (before * 2 + 1) * TILE);
+    } else {
+      const int next = next_unit(tk), loads = unit_loads(next);   // these may be under way
+      if (loads == 2 * LPW) wait_vmcnt_imm<2 * LPW>();
+      else if (loads == LPW) wait_vmcnt_imm<LPW>();
+      else wait_vmcnt_imm<0>();
+      lds_barrier();
+      issue_unit(next_unit(next), before);
+    }
+    const unsigned char* p = smem + slot * 2 * TILE;
+    slot = slot == 2 ? 0 : slot + 1;
+    return p;
+  };
 
   // ---- set-up: operand fragments, delta, channel-bias tile
   bf16x8 dOf[KS];            // (q+u), (q+v) fragments are re-formed where needed, not kept
@@ -438,15 +451,15 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     const int e = (ln & 15) >> 2, aa = ln & 3, grp = ln >> 4;
     const int row0 = 4 * hh + e;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) r_lane[ks] = ln * ROWB + (((2 * ks + hh) ^ swz_row<DH>(ln)) << 4);
+    for (int ks = 0; ks < KS; ++ks) r_lane[ks] = ln * ROWB + (((2 * ks + hh) ^ swz<DH>(ln)) << 4);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp + (aa >> 1)) ^ swz_tr<DH>(row0)) << 4) + ((aa & 1) << 3);
+      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp + (aa >> 1)) ^ swz<DH>(row0)) << 4) + ((aa & 1) << 3);
   }
   auto tr_frag = [&](const unsigned char* tile_p, int t, int s, int mt) -> bf16x8 {
-    const unsigned char* p = tile_p + t_lane[mt] + (32 * t + 16 * s) * ROWB;
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))p);
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB));
+    const unsigned char* p = tile_p + (32 * t + 16 * s) * ROWB;   // eight rows on, bit 1 of the swizzle is the other
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + t_lane[mt]));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB + (t_lane[mt] ^ 32)));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
@@ -582,7 +595,6 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   bf16x8 Qu[KS];
   auto near_step = [&](const unsigned char* Vrow, int tk) __attribute__((always_inline)) {
     const unsigned char* Krow = Vrow + TILE;
-    const unsigned char* Ktr = Vrow + 2 * TILE;
     const float off2 = Stb[((tk - tk_first) & 31) * 32 + ln];
     float gt = 0.f;
 #pragma unroll
@@ -614,7 +626,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) kt[s][mt] = tr_frag(Ktr, t, s, mt);
+          for (int mt = 0; mt < MT; ++mt) kt[s][mt] = tr_frag(Krow, t, s, mt);
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -630,7 +642,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
         const bf16x8 dsf = pack8(S, 8 * s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          dq[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(SOLO ? kt[s][mt] : tr_frag(Ktr, t, s, mt), dsf, dq[mt], 0, 0, 0);
+          dq[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(SOLO ? kt[s][mt] : tr_frag(Krow, t, s, mt), dsf, dq[mt], 0, 0, 0);
       }
     }
     gt = xhalf_sum(gt);
@@ -644,14 +656,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     // reduce at the same time, and the three add up (T 512, 128 channels of Dh 128: 2.80 ms a launch, 2.47 .. 2.56
     // with half the barriers).
     for (; tk < far_lim; tk += 2) {
-      if (tk + 3 < far_lim) wait_vmcnt_imm<2 * LPW>();            // the unit behind this one may be under way
-      else if (tk + 2 < far_lim) wait_vmcnt_imm<LPW>();
-      else wait_vmcnt_imm<0>();
-      lds_barrier();                              // the unit is visible to all; everyone is done with the one before
-      if (tk + 4 < far_lim) issue_far(tk + 4, slot == 0 ? 2 : slot - 1);
-      else if (tk + 2 >= far_lim) issue_near(far_lim, 1);
-      const unsigned char* Vrow = smem + slot * 2 * TILE;
-      slot = slot == 2 ? 0 : slot + 1;
+      const unsigned char* Vrow = begin_unit(tk);
       if (tk >= far_end) continue;
       if ((tk & 31) == 0) time_slab(tk);
       if (PHASE == FAR || tk + 1 >= min(far_lim, far_end)) {
@@ -674,18 +679,9 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     }
     tk = far_lim;
   }
-  int half = 1;
-  auto near_unit = [&](int tk) __attribute__((always_inline)) -> const unsigned char* {
-    wait_vmcnt_imm<0>();
-    lds_barrier();
-    issue_near(tk + 1, half ^ 1);
-    const unsigned char* p = smem + half * 3 * TILE;
-    half ^= 1;
-    return p;
-  };
   if constexpr (PHASE == ONE)
     for (; tk < far_end; ++tk) {                  // far for this wave, not for the workgroup
-      const unsigned char* Vrow = near_unit(tk);
+      const unsigned char* Vrow = begin_unit(tk);
       time_slab(tk);
       far_one(Vrow, tk);
     }
@@ -705,7 +701,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   for (int ks = 0; ks < KS; ++ks)
     Qu[ks] = qfrag(*(const u32x4*)(qrow + ks * 16 + hh * 8), *(const u32x4*)(bu + ks * 16 + hh * 8), sc2);
   for (; tk <= tq_hi; ++tk) {
-    const unsigned char* Vrow = near_unit(tk);
+    const unsigned char* Vrow = begin_unit(tk);
     if (active && tk >= far_end && tk <= tq) {
       time_slab(tk);
       near_step(Vrow, tk);
@@ -821,36 +817,35 @@ static void launch_query(const mvpa_bwd_args* a, hipStream_t stream, int q0, int
 //     inside :  P = exp2((q+u) K^T + e) o Ec,  dP = dO V^T,  dS = P o (dP - delta[q])
 //               dv^T[d][key] += dO^T[d][q] P[q][key],   dk^T[d][key] += (q+u)^T[d][q] dS[q][key]
 //     outside:  P = exp2(e) Ec,                dv^T += dO^T P           (dk gets nothing)
-// Per (head, tq) one ring stage holds dO in the transposing-read swizzle, the Ec tile and the
-// scalars, and for steps that are inside the window for some wave also dO in the row-fragment
-// swizzle, (q+u) * scale in both swizzles and delta; direct-to-LDS loads fetch it two steps
-// ahead.  The query steps are walked from the last one down and the workgroups of one
-// (b, kv head) sit on one XCD: they then read the same stage data at about the same time and
-// share it in L2.  MASKED: the query part holds fewer channels than its tiles, padded query rows are cut.
+// Per (head, tq) one ring stage holds dO, the Ec tile and the scalars, and for steps that are inside the window for
+// some wave also (q+u) * scale and delta; direct-to-LDS loads fetch it one or two steps ahead.  The query steps are
+// walked from the last one down and the workgroups of one (b, kv head) sit on one XCD: they then read the same stage
+// data at about the same time and share it in L2.  MASKED: the query part holds fewer channels than its tiles, padded query rows are cut.
 // ==========================================================================================
 namespace mvpa {
 namespace bwdq {
 
-// waves per workgroup of the key pass: every wave of a workgroup reads the same stage (only the
-// per-key-step scalars differ), so with two channel tiles 8 waves (4 key steps) share it and each
-// SIMD holds two waves
-template <int NCT> constexpr int KEY_WAVES = NCT == 2 ? 8 : 4;
+// Every wave of a workgroup reads the same stage (only the per-key-step scalars differ), and no wave has work on all of
+// its steps: with a window of 10 a workgroup of two key steps walks 13 for 12, one of four 15.  At Dh 64 two
+// workgroups share a CU, which one copy of dO and (q+u) a stage makes room for (67 KB; with copies for each kind of read
+// 8 waves had the CU to themselves): B4 H16 C64 T128 404 -> 340 us, 315 with dv read at the start and not at the end;
+// Dh 128, T 512, 32 of 128 channels 279 -> 240 us.  (dk read at the start as well: 250.)
+constexpr int KEY_WAVES = 4;
+template <int NCT> constexpr int KSTAGES = NCT == 2 ? 2 : 3;      // ring depth
 
 // NEAR: the far steps are left to mvpa_bwd_far_kernel, which has written dv before.
 template <int DH, int NCT, bool MASKED, bool NEAR>
-__global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum, int per_head) {
+__global__ __launch_bounds__(KEY_WAVES * 64, DH == 64 ? 2 : 1) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum, int per_head) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
-  constexpr int NW = KEY_WAVES<NCT>;
+  constexpr int NW = KEY_WAVES;
   constexpr int CP = NCT * 32, KT = NW / NCT, TILE = CP * ROWB;
   constexpr int CS_BYTES = CP * CP * 4, SC_BYTES = (KT + 1) * 256;
-  constexpr int STAGES = KSTAGES, STAGE_BYTES = 4 * TILE + CS_BYTES + SC_BYTES;
-  static_assert(STAGES == 3, "the wait below counts the loads of exactly one younger step");
+  constexpr int STAGES = KSTAGES<NCT>, STAGE_BYTES = 2 * TILE + CS_BYTES + SC_BYTES;
   constexpr int LPW = TILE / 1024 / NW, CS_LPW = CS_BYTES / 1024 / NW;
   // direct-to-LDS loads per wave and step
-  constexpr int LPS_FAR = LPW + CS_LPW + 1, LPS_NEAR = 4 * LPW + CS_LPW + 2;
-  // stage layout: dO (transposing) | Ec | scalars | dO (rows) | (q+u) (rows) | (q+u) (transposing)
-  constexpr int OFF_DTR = 0, OFF_EC = TILE, OFF_SC = TILE + CS_BYTES, OFF_DROW = OFF_SC + SC_BYTES,
-                OFF_QROW = OFF_DROW + TILE, OFF_QTR = OFF_QROW + TILE;
+  constexpr int LPS_FAR = LPW + CS_LPW + 1, LPS_NEAR = 2 * LPW + CS_LPW + 2;
+  // stage layout: dO | Ec | scalars | (q+u)
+  constexpr int OFF_DO = 0, OFF_EC = TILE, OFF_SC = TILE + CS_BYTES, OFF_QU = OFF_SC + SC_BYTES;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -916,16 +911,14 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   }
 
   // ---- the ring: per-wave source offsets (swizzles applied on the source side)
-  int q_off_r[LPW], q_off_t[LPW], d_off_r[LPW], d_off_t[LPW], cs_off[CS_LPW];
+  int q_off[LPW], d_off[LPW], cs_off[CS_LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
     const int pc = (wave + NW * i) * 64 + lane;
     const int r = pc / CPR, phys = pc % CPR;
     const int rc = min(q0 + r, C_ - 1);
-    q_off_r[i] = rc * DH + ((phys ^ swz_row<DH>(r)) << 3);
-    q_off_t[i] = rc * DH + ((phys ^ swz_tr<DH>(r)) << 3);
-    d_off_r[i] = rc * (int)a.do_stride_n + ((phys ^ swz_row<DH>(r)) << 3);
-    d_off_t[i] = rc * (int)a.do_stride_n + ((phys ^ swz_tr<DH>(r)) << 3);
+    q_off[i] = rc * DH + ((phys ^ swz<DH>(r)) << 3);
+    d_off[i] = rc * (int)a.do_stride_n + ((phys ^ swz<DH>(r)) << 3);
   }
   // the Ec tile [C][C] lands with a row pitch of CP floats
 #pragma unroll
@@ -963,19 +956,14 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   auto issue_step = [&](int tq, int stage_idx) {
     const uint32_t st = ring_lds + stage_idx * STAGE_BYTES;
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) dma16(p_do + d_off_t[i], st + OFF_DTR + (wave + NW * i) * 1024);
+    for (int i = 0; i < LPW; ++i) dma16(p_do + d_off[i], st + OFF_DO + (wave + NW * i) * 1024);
 #pragma unroll
     for (int i = 0; i < CS_LPW; ++i) dma16(p_ec + cs_off[i], st + OFF_EC + (wave + NW * i) * 1024);
     // per-query scalar of this wave's key step
     dma4(p_sc + sc_lane, st + OFF_SC + ktw * 256);
     if (wg_near(tq)) {
 #pragma unroll
-      for (int i = 0; i < LPW; ++i) {
-        const uint32_t dst = st + (wave + NW * i) * 1024;
-        dma16(p_do + d_off_r[i], dst + OFF_DROW);
-        dma16(p_qu + q_off_r[i], dst + OFF_QROW);
-        dma16(p_qu + q_off_t[i], dst + OFF_QTR);
-      }
+      for (int i = 0; i < LPW; ++i) dma16(p_qu + q_off[i], st + OFF_QU + (wave + NW * i) * 1024);
       dma4(p_de + sc_lane, st + OFF_SC + KT * 256);
     }
   };
@@ -985,21 +973,31 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) { dK[mt][i] = 0.f; dV[mt][i] = 0.f; }
+  const int64_t out_row = ((int64_t)bg * N + (int64_t)tkc * C_ + ck) * DH;
+  const bool stores = wave_on && ck < C_;
+  if ((NEAR || accum) && stores)                  // launches of one stream: dv goes on from what is there
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4) {
+        const float4 v = *(const float4*)(a.dv + out_row + mt * 32 + a4 * 8 + hh * 4);
+        dV[mt][a4 * 4] = v.x; dV[mt][a4 * 4 + 1] = v.y; dV[mt][a4 * 4 + 2] = v.z; dV[mt][a4 * 4 + 3] = v.w;
+      }
 
   int r_lane[KS], t_lane[MT];
   {
     const int e = (ln & 15) >> 2, aa = ln & 3, grp16 = ln >> 4;
     const int row0 = 4 * hh + e;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) r_lane[ks] = ln * ROWB + (((2 * ks + hh) ^ swz_row<DH>(ln)) << 4);
+    for (int ks = 0; ks < KS; ++ks) r_lane[ks] = ln * ROWB + (((2 * ks + hh) ^ swz<DH>(ln)) << 4);
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp16 + (aa >> 1)) ^ swz_tr<DH>(row0)) << 4) + ((aa & 1) << 3);
+      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp16 + (aa >> 1)) ^ swz<DH>(row0)) << 4) + ((aa & 1) << 3);
   }
   auto tr_frag = [&](const unsigned char* tile_p, int qt, int s, int mt) -> bf16x8 {
-    const unsigned char* p = tile_p + t_lane[mt] + (32 * qt + 16 * s) * ROWB;
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))p);
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB));
+    const unsigned char* p = tile_p + (32 * qt + 16 * s) * ROWB;  // eight rows on, bit 1 of the swizzle is the other
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + t_lane[mt]));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB + (t_lane[mt] ^ 32)));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
 
@@ -1039,7 +1037,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
   auto ring_step = [&]() -> const unsigned char* {
     // the step has landed once only the loads of the one younger step are in flight
     const int next_tq = ring_tq - 1 < tk0 ? T_ - 1 : ring_tq == T_ - 1 ? top : ring_tq - 1;
-    if (it + 1 >= nsteps) wait_vmcnt_imm<0>();
+    if (STAGES == 2 || it + 1 >= nsteps) wait_vmcnt_imm<0>();
     else if (wg_near(next_tq)) wait_vmcnt_imm<LPS_NEAR>();
     else wait_vmcnt_imm<LPS_FAR>();
     lds_barrier();            // this step's stage visible to all; the previous one is free
@@ -1053,7 +1051,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
 
   // ---- a query step outside the content window: P = Ec * exp2(e), dv only
   auto far_step = [&](const unsigned char* base) {
-    const unsigned char* Dtr = base + OFF_DTR;
+    const unsigned char* Do = base + OFF_DO;
     const float* Ecs = (const float*)(base + OFF_EC) + ckl;
     const float* ET = (const float*)(base + OFF_SC) + ktw * 64;
 #pragma unroll
@@ -1074,17 +1072,15 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
         const bf16x8 pf = cut(pack8(P, 8 * s), qt, s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
-          dV[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Dtr, qt, s, mt), pf, dV[mt], 0, 0, 0);
+          dV[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Do, qt, s, mt), pf, dV[mt], 0, 0, 0);
       }
     }
   };
 
   // ---- a query step inside the content window
   auto near_step = [&](const unsigned char* base) {
-    const unsigned char* Dtr = base + OFF_DTR;
-    const unsigned char* Drow = base + OFF_DROW;
-    const unsigned char* Qrow = base + OFF_QROW;
-    const unsigned char* Qtr = base + OFF_QTR;
+    const unsigned char* Do = base + OFF_DO;
+    const unsigned char* Qu = base + OFF_QU;
     const float* Ecs = (const float*)(base + OFF_EC) + ckl;
     const float* TL = (const float*)(base + OFF_SC) + ktw * 64;
     const float* De = (const float*)(base + OFF_SC) + KT * 64;
@@ -1103,8 +1099,8 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
       bf16x8 qf[KS], df[KS];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        qf[ks] = *(const bf16x8*)(Qrow + r_lane[ks] + qt * 32 * ROWB);
-        df[ks] = *(const bf16x8*)(Drow + r_lane[ks] + qt * 32 * ROWB);
+        qf[ks] = *(const bf16x8*)(Qu + r_lane[ks] + qt * 32 * ROWB);
+        df[ks] = *(const bf16x8*)(Do + r_lane[ks] + qt * 32 * ROWB);
       }
       __builtin_amdgcn_sched_barrier(0);          // every read out before the first product
 #pragma unroll
@@ -1128,8 +1124,8 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
         const bf16x8 sf = cut(pack8(dS, 8 * s), qt, s);
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-          dV[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Dtr, qt, s, mt), pf, dV[mt], 0, 0, 0);
-          dK[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Qtr, qt, s, mt), sf, dK[mt], 0, 0, 0);
+          dV[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Do, qt, s, mt), pf, dV[mt], 0, 0, 0);
+          dK[mt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(tr_frag(Qu, qt, s, mt), sf, dK[mt], 0, 0, 0);
         }
       }
     }
@@ -1162,8 +1158,7 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
     for (int n = n_idle; n > 0; --n) (void)ring_step();
   }
 
-  if (wave_on && ck < C_) {
-    const int64_t o = (((int64_t)bg * N) + (int64_t)tk * C_ + ck) * DH;
+  if (stores) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
@@ -1171,17 +1166,13 @@ __global__ __launch_bounds__(KEY_WAVES<NCT> * 64) void mvpa_bwd_key_mfma_kernel(
         const int d = mt * 32 + a4 * 8 + hh * 4;
         constexpr float f = 1.f / kLog2e;
         float4 vk = make_float4(dK[mt][a4 * 4] * f, dK[mt][a4 * 4 + 1] * f, dK[mt][a4 * 4 + 2] * f, dK[mt][a4 * 4 + 3] * f);
-        float4 vv = make_float4(dV[mt][a4 * 4], dV[mt][a4 * 4 + 1], dV[mt][a4 * 4 + 2], dV[mt][a4 * 4 + 3]);
+        const float4 vv = make_float4(dV[mt][a4 * 4], dV[mt][a4 * 4 + 1], dV[mt][a4 * 4 + 2], dV[mt][a4 * 4 + 3]);
         if (accum) {                              // launches of one stream: the query parts add up
-          const float4 ok = *(const float4*)(a.dk + o + d);
+          const float4 ok = *(const float4*)(a.dk + out_row + d);
           vk = make_float4(vk.x + ok.x, vk.y + ok.y, vk.z + ok.z, vk.w + ok.w);
         }
-        if (NEAR || accum) {
-          const float4 ov = *(const float4*)(a.dv + o + d);
-          vv = make_float4(vv.x + ov.x, vv.y + ov.y, vv.z + ov.z, vv.w + ov.w);
-        }
-        *(float4*)(a.dk + o + d) = vk;
-        *(float4*)(a.dv + o + d) = vv;
+        *(float4*)(a.dk + out_row + d) = vk;
+        *(float4*)(a.dv + out_row + d) = vv;
       }
   }
 }
@@ -1238,7 +1229,7 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
     const int pc = (wave + NW * i) * 64 + lane, r = pc / CPR, phys = pc % CPR;
-    d_off[i] = min(q0 + r, C_ - 1) * (int)a.do_stride_n + ((phys ^ swz_tr<DH>(r)) << 3);
+    d_off[i] = min(q0 + r, C_ - 1) * (int)a.do_stride_n + ((phys ^ swz<DH>(r)) << 3);
   }
 #pragma unroll
   for (int i = 0; i < CS_LPW; ++i) {
@@ -1292,12 +1283,12 @@ __global__ __launch_bounds__(FAR_WAVES<DH> * 64) void mvpa_bwd_far_kernel(mvpa_b
     const int e = (ln & 15) >> 2, aa = ln & 3, grp16 = ln >> 4, row0 = 4 * hh + e;
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
-      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp16 + (aa >> 1)) ^ swz_tr<DH>(row0)) << 4) + ((aa & 1) << 3);
+      t_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp16 + (aa >> 1)) ^ swz<DH>(row0)) << 4) + ((aa & 1) << 3);
   }
   auto tr_frag = [&](const unsigned char* tile_p, int qt, int s, int mt) -> bf16x8 {
-    const unsigned char* p = tile_p + t_lane[mt] + (32 * qt + 16 * s) * ROWB;
-    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))p);
-    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB));
+    const unsigned char* p = tile_p + (32 * qt + 16 * s) * ROWB;  // eight rows on, bit 1 of the swizzle is the other
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + t_lane[mt]));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4bf16((BWD_LDS_PTR(bf16x4))(p + 8 * ROWB + (t_lane[mt] ^ 32)));
     return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
   };
   // the query whose scalar this lane holds: register n = lane & 15 of the product layout
@@ -1393,9 +1384,9 @@ static void launch_far(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 template <int DH, int NCT, bool MASKED, bool NEAR>
 static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum, int per_head) {
   using namespace mvpa::bwdq;
-  constexpr int nw = KEY_WAVES<NCT>, cp = NCT * 32, kt = nw / NCT, ROWB = 2 * DH;
-  static_assert((size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256) <= 160 * 1024, "key-pass ring exceeds the LDS");
-  const size_t lds = (size_t)KSTAGES * (4 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256);
+  constexpr int nw = KEY_WAVES, cp = NCT * 32, kt = nw / NCT, ROWB = 2 * DH;
+  static_assert((size_t)KSTAGES<NCT> * (2 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256) <= 160 * 1024 / (DH == 64 ? 2 : 1), "key-pass ring exceeds the LDS");
+  const size_t lds = (size_t)KSTAGES<NCT> * (2 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256);
   dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * (per_head ? a->H : a->Hkv)));
   auto kern = mvpa_bwd_key_mfma_kernel<DH, NCT, MASKED, NEAR>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
