@@ -139,19 +139,29 @@ template <int DH> __device__ inline int swz(int row) {
 // gone from 1040 to 570 of 1770 -> 1350 cycles, and it falls from 2.25 to 1.9 GHz as they go.
 enum query_phase { ONE, FAR, WIN };
 template <int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : 4;
+// The last time step keeps the content term at every key step, T steps where the others have window + 1.  At Dh 128
+// with two key tiles it has a workgroup to itself, in which two waves share a query tile and take a key tile each (window
+// launch at T 512, 128 channels, most of which was this chain: 1.15 -> 0.99 ms).  At Dh 64 the chain hides behind the
+// rest, and the longer code takes what it gives (T 25: 70 -> 73 us, T 128 730, T 512 1690 either way).
+template <int DH, int NCT, int PHASE> constexpr bool LAST_APART = DH == 128 && NCT == 2 && PHASE != FAR;
+template <int DH, int NCT, int PHASE> __host__ __device__ inline int query_tiles(int T, bool content) {
+  constexpr int TQW = PHASE_WAVES<PHASE> / NCT;
+  return LAST_APART<DH, NCT, PHASE> && content ? (T - 1 + TQW - 1) / TQW + 1 : (T + TQW - 1) / TQW;
+}
 // waves per SIMD: at Dh 64 two workgroups share a CU
 template <int DH, int PHASE> constexpr int PHASE_OCC = PHASE == FAR || DH == 64 ? 2 : 1;
 // The ring holds three units of two tiles: V of two far steps, or V and K of a step with content.
 template <int DH, int NCT> constexpr int TILE_BYTES = NCT * 32 * 2 * DH;
 template <int DH, int NCT, int PHASE> constexpr int QUERY_LDS = 6 * TILE_BYTES<DH, NCT> + PHASE_WAVES<PHASE> * WAVE_SCRATCH * 4;
 
-template <int DH, int NCT, int PHASE>
-__global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
+// One tile of query time steps of one (b, h).  LAST: the last time step alone.
+template <int DH, int NCT, int PHASE, bool LAST>
+__device__ __forceinline__ void query_walk(const mvpa_bwd_args& a, int q0, int k0, int accum, int bh, int tile) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
   constexpr int NW = PHASE_WAVES<PHASE>;
   constexpr bool SOLO = PHASE_OCC<DH, PHASE> == 1;                // one wave per SIMD
   constexpr int CP = NCT * 32, TQW = NW / NCT, TILE = TILE_BYTES<DH, NCT>;
-  static_assert(64 * 32 <= WAVE_SCRATCH && (1 + 32 * (CP + 1)) * 4 <= QUERY_LDS<DH, NCT, PHASE> / NW, "channel tables overlay the rest");
+  static_assert(64 * 32 <= WAVE_SCRATCH && (1 + 32 * (CP + 1)) * 4 <= QUERY_LDS<DH, NCT, PHASE> / NW && MT * 4096 <= QUERY_LDS<DH, NCT, PHASE> / NW, "channel tables overlay the rest");
   constexpr int LPW = TILE / 1024 / NW;           // 1 KiB wave loads per wave and tile copy
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
   float* wave_base = (float*)(smem + 6 * TILE);
@@ -171,36 +181,14 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   const bool has_content = a.flags & MVPA_FLAG_CONTENT;
   const bool has_time = a.flags & MVPA_FLAG_TIME_BIAS;
   const bool has_chan = a.flags & MVPA_FLAG_CHAN_BIAS;
-  const int nt = (T_ + TQW - 1) / TQW;
-  // blocks go round-robin over the 8 XCDs: keep the tiles of one (b,h) on one XCD (they walk the
-  // same K and V in step, so its L2 serves all but the first), long tiles first.  The tile with
-  // the last time step keeps the content term at every key step and runs about twice as long as
-  // the next one: all of those go first, or the last of them would end the launch alone.
-  const int nbh = a.B * a.H;
-  int bh, tile;
-  {
-    const int L = blockIdx.x;
-    if (nt == 1) {
-      bh = L;
-      tile = 0;
-    } else if (L < nbh) {
-      bh = L;
-      tile = nt - 1;
-    } else if ((nbh & 7) == 0) {
-      const int s = (L - nbh) >> 3;
-      bh = ((L - nbh) & 7) + 8 * (s / (nt - 1));
-      tile = nt - 2 - s % (nt - 1);
-    } else {
-      bh = (L - nbh) / (nt - 1);
-      tile = nt - 2 - (L - nbh) % (nt - 1);
-    }
-  }
   const int b = bh / a.H, h = bh % a.H;
   const int g = h / (a.H / a.Hkv);
-  const int tq0 = tile * TQW;
-  const int tq_hi = min(T_ - 1, tq0 + TQW - 1);
-  const int tq = tq0 + wave / NCT;
-  const bool active = tq < T_;
+  const int tq_end = LAST_APART<DH, NCT, PHASE> && has_content ? T_ - 2 : T_ - 1;    // the last step of these tiles
+  const int tq0 = LAST ? T_ - 1 : tile * TQW;
+  const int tq_hi = LAST ? T_ - 1 : min(tq_end, tq0 + TQW - 1);
+  const int tq = LAST ? T_ - 1 : tq0 + wave / NCT;
+  const bool second = LAST && wave >= NCT;        // wave w and wave w + NCT take a key tile each
+  const bool active = LAST || tq <= tq_hi;
   const int cqw0 = q0 + (wave % NCT) * 32;        // first query channel of this wave
   const int cq = cqw0 + ln;
   const bool qok = active && cq < C_;
@@ -231,10 +219,10 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     v_off[i] = rc * (int)a.v_stride_n + ((phys ^ swz<DH>(r)) << 3);
   }
   // first key step whose K is needed: the band of the earliest query step of the workgroup
-  const int tk_near = !has_content ? tq_hi + 1 : (W <= 0 || tq_hi == T_ - 1) ? 0 : max(0, tq0 - W);
+  const int tk_near = LAST ? 0 : !has_content ? tq_hi + 1 : (W <= 0 || tq_hi == T_ - 1) ? 0 : max(0, tq0 - W);
   // this wave's far steps are those before far_end (none for the last time step, whose queries keep the content
   // term everywhere); the workgroup walks the key steps tk_lo .. tk_hi
-  const int far_end = !active ? 0 : !has_content ? tq + 1 : (W <= 0 || tq == T_ - 1) ? 0 : max(0, tq - W);
+  const int far_end = !active || LAST ? 0 : !has_content ? tq + 1 : (W <= 0 || tq == T_ - 1) ? 0 : max(0, tq - W);
   const int far_top = tq_hi == T_ - 1 ? T_ - 2 : tq_hi;           // FAR: the latest query step with far steps
   const int tk_lo = PHASE == WIN ? tk_near : 0;
   const int tk_hi = PHASE == FAR ? (far_top < tq0 ? -1 : far_top - W - 1) : tq_hi;
@@ -399,7 +387,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     }
     // for the key pass: (q+u) * scale, delta, and the tile exp2(channel bias - mc) by
     // [query][key channel]; and the rows of dbias_time that no key step reaches
-    if (PHASE != WIN && qok) {
+    if (PHASE != WIN && qok && !second) {
       float* wc = a.ws_chan + row * CW + k0;      // rows of CW floats: 16-byte aligned for any C
 #pragma unroll
       for (int t = 0; t < NCT; ++t)
@@ -411,7 +399,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
         }
     }
     // the stores last: loads return behind the stores before them
-    if (PHASE != WIN && qok) {
+    if (PHASE != WIN && qok && !second) {
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) *(bf16x8*)((bf16_t*)a.ws_qu + row * DH + ks * 16 + hh * 8) = qu[ks];
       if (hh == 0) a.ws_delta[row] = -delta;
@@ -489,23 +477,28 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   // the key pass (the exponent e = time bias - L + mc for pairs inside the window, else exp2(e))
   auto flush_slab = [&](int tks) __attribute__((always_inline)) {
     const int nj = min(32, (PHASE == FAR ? far_end : tq + 1) - tks);
+    if (!second)
     store_rows(nj, min(32, C_ - cqw0), [&](int jj) { return a.ws_time + (((int64_t)bh * T_ + tq) * T_ + tks + jj) * C_ + cqw0; },
                [&](int jj, int q) {
                  const float e = Stb[jj * 32 + q];
                  const bool near_pair = has_content && (W <= 0 || tq - tks - jj <= W || tq == T_ - 1);
                  return near_pair ? e : __builtin_amdgcn_exp2f(e);
                });
+    if (LAST && !second) return;                // the second wave adds up both waves' gradients
     const int j0 = time_row(tq, tks, T_);
+    auto gradient = [&](int q, int jj) __attribute__((always_inline)) {
+      const float* g = Gtb + q * 32 + (jj ^ ((q & 7) << 2));
+      return (second ? g[0] + g[-NCT * WAVE_SCRATCH] : g[0]) * a.sm_scale;
+    };
     if (!accum) {
-      store_rows(nq_live, nj, [&](int q) { return a.dbias_time + (wrow0 + q) * T_ + j0; },
-                 [&](int q, int jj) { return Gtb[q * 32 + (jj ^ ((q & 7) << 2))] * a.sm_scale; });
+      store_rows(nq_live, nj, [&](int q) { return a.dbias_time + (wrow0 + q) * T_ + j0; }, gradient);
     } else {
       // launches of one stream: the key parts add up.  An atomic add without a return value, not a load and a
       // store: nothing waits for the old value (every address has one writer)
 #pragma unroll 8
       for (int it = 0; it < 16; ++it) {
         const int q = 2 * it + hh;
-        const float g = Gtb[q * 32 + (ln ^ ((q & 7) << 2))] * a.sm_scale;
+        const float g = gradient(q, ln);
         if (q < nq_live && ln < nj) atomicAdd(a.dbias_time + (wrow0 + q) * T_ + j0 + ln, g);
       }
     }
@@ -532,9 +525,11 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
           stc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_frag(rr[ks]), qfrag(qr[ks], br[ks], sc2), stc, 0, 0, 0);
       }
       if (tk > tk_first) {
-        wave_sync_lds();
+        if constexpr (LAST) lds_barrier();
+        else wave_sync_lds();
         flush_slab(tk - 32);
-        wave_sync_lds();
+        if constexpr (LAST) lds_barrier();
+        else wave_sync_lds();
       }
 #pragma unroll
       for (int i = 0; i < 16; ++i) Stb[((i >> 2) * 8 + hh * 4 + (i & 3)) * 32 + ln] = stc[i] - lse + mc;
@@ -594,11 +589,18 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   f32x16 Bc[NCT];
   bf16x8 Qu[KS];
   auto near_step = [&](const unsigned char* Vrow, int tk) __attribute__((always_inline)) {
+    Vrow += second ? 32 * ROWB : 0;
     const unsigned char* Krow = Vrow + TILE;
     const float off2 = Stb[((tk - tk_first) & 31) * 32 + ln];
     float gt = 0.f;
+    // A branch between the tiles where a wave has 512 registers: without it the two are mixed, which takes 36 registers
+    // more and their copies from the accumulation half (window launch at Dh 128, T 512, 128 channels: 1045 against 990 us).
+    int tiles = NCT;
+    if constexpr (SOLO) asm volatile("" : "+s"(tiles));
 #pragma unroll
     for (int t = 0; t < NCT; ++t) {               // one key-channel tile at a time: fewer live tiles
+      if (t > 0 && LAST) break;                   // tile 0 is this wave's
+      if (t >= tiles) break;
       // A wave that has its SIMD to itself sends out every LDS read of a phase before the first product or
       // exponential of it: read where they are used, each pair of fragments waits out the LDS latency (last time
       // step of 512: 512 such steps, the longest chain of the launch; 4.92 -> 4.64 ms at B1 H16 C64 of 128 Dh128).
@@ -651,7 +653,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
 
   // far steps first, then the steps inside the window; waves that are done keep the ring and the barriers going
   int tk = tk_lo;
-  if constexpr (PHASE != WIN) {
+  if constexpr (PHASE != WIN && !LAST) {
     // Two steps per barrier, two units on their way.  With a barrier a step the two waves of a SIMD read, multiply and
     // reduce at the same time, and the three add up (T 512, 128 channels of Dh 128: 2.80 ms a launch, 2.47 .. 2.56
     // with half the barriers).
@@ -679,7 +681,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     }
     tk = far_lim;
   }
-  if constexpr (PHASE == ONE)
+  if constexpr (PHASE == ONE && !LAST)
     for (; tk < far_end; ++tk) {                  // far for this wave, not for the workgroup
       const unsigned char* Vrow = begin_unit(tk);
       time_slab(tk);
@@ -697,6 +699,7 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   for (int t = 0; t < NCT; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) Bc[t][i] = __builtin_amdgcn_logf(Ec[t][i]);
+  if (second) Bc[0] = Bc[NCT - 1];
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks)
     Qu[ks] = qfrag(*(const u32x4*)(qrow + ks * 16 + hh * 8), *(const u32x4*)(bu + ks * 16 + hh * 8), sc2);
@@ -709,30 +712,12 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   }
   }
 
-  wave_sync_lds();
+  if constexpr (LAST) lds_barrier();
+  else wave_sync_lds();
   const int tk_end = PHASE == FAR ? far_end : tq + 1;
   if (active && tk_end > tk_first) flush_slab(tk_first + ((tk_end - 1 - tk_first) & ~31));
   lds_barrier();                                  // from here on the waves share out the whole of the LDS
   if (!active) return;
-
-  // dq^T[d][q]: this lane's query, d = 32mt + 8a4 + 4hh + 0..3
-  if (PHASE != FAR && qok) {
-    float* dqo = a.dq + row * DH;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int a4 = 0; a4 < 4; ++a4)
-      {
-        float4* dst = (float4*)(dqo + mt * 32 + a4 * 8 + hh * 4);
-        float4 val = make_float4(dq[mt][a4 * 4] * a.sm_scale, dq[mt][a4 * 4 + 1] * a.sm_scale,
-                                 dq[mt][a4 * 4 + 2] * a.sm_scale, dq[mt][a4 * 4 + 3] * a.sm_scale);
-        if (accum) {
-          const float4 old = *dst;
-          val = make_float4(val.x + old.x, val.y + old.y, val.z + old.z, val.w + old.w);
-        }
-        *dst = val;
-      }
-  }
 
   // channel-table gradient: element (ck) of query cq goes to column C-1-|cq-ck|, so column
   // C-1-d collects the two key channels cq-d and cq+d (those of them that this launch holds).
@@ -740,14 +725,55 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
   // is gathered from it (LDS float atomics for the scatter form were measured at ~0.3 us apiece).
   // The column behind the last channel, and the one before the first, is zero: key channels that this launch does
   // not hold.
-  float* tab = (float*)(smem + wave * (QUERY_LDS<DH, NCT, PHASE> / NW)) + 1;
+  constexpr int SHARE = QUERY_LDS<DH, NCT, PHASE> / NW / 4;
+  float* share = (float*)smem + wave * SHARE;
+  float* tab = share - (second ? NCT * SHARE : 0) + 1;
 #pragma unroll
-  for (int t = 0; t < NCT; ++t)
+  for (int t = 0; t < NCT; ++t) {
+    if (t > 0 && LAST) break;
+    const int col = second ? 32 : t * 32;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) tab[ln * PC + t * 32 + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i] * a.sm_scale;
-  tab[ln * PC + CP] = 0.f;
-  if (lane == 0) tab[-1] = 0.f;
-  wave_sync_lds();
+    for (int i = 0; i < 16; ++i) tab[ln * PC + col + (i >> 2) * 8 + hh * 4 + (i & 3)] = dSc[t][i] * a.sm_scale;
+  }
+  if (!second) {
+    tab[ln * PC + CP] = 0.f;
+    if (lane == 0) tab[-1] = 0.f;
+  }
+  // two waves of one query tile: the first stores the sum of their dq, the second the table of both
+  if (second) {
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) share[(mt * 16 + i) * 64 + lane] = dq[mt][i];
+  }
+  if constexpr (LAST) lds_barrier();
+  else wave_sync_lds();
+  // dq^T[d][q]: this lane's query, d = 32mt + 8a4 + 4hh + 0..3
+  if (PHASE != FAR && qok && !second) {
+    const float* other = share + NCT * SHARE + lane;
+    float* dqo = a.dq + row * DH;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int a4 = 0; a4 < 4; ++a4)
+      {
+        float4* dst = (float4*)(dqo + mt * 32 + a4 * 8 + hh * 4);
+        float v[4];
+#pragma unroll
+        for (int x = 0; x < 4; ++x) {
+          v[x] = dq[mt][a4 * 4 + x];
+          if (LAST) v[x] += other[(mt * 16 + a4 * 4 + x) * 64];
+          v[x] *= a.sm_scale;
+        }
+        float4 val = make_float4(v[0], v[1], v[2], v[3]);
+        if (accum) {
+          const float4 old = *dst;
+          val = make_float4(val.x + old.x, val.y + old.y, val.z + old.z, val.w + old.w);
+        }
+        *dst = val;
+      }
+  }
+  if (LAST && !second) return;
   for (int c0 = 0; c0 < C_; c0 += 64) {
     const int col = c0 + lane;
     const int d = C_ - 1 - col;                   // this lane's column holds distance d
@@ -764,6 +790,40 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
       }
     }
   }
+}
+
+template <int DH, int NCT, int PHASE>
+__global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) void mvpa_bwd_query_mfma_kernel(mvpa_bwd_args a, int q0, int k0, int accum) {
+  const bool has_content = a.flags & MVPA_FLAG_CONTENT;
+  const int nt = query_tiles<DH, NCT, PHASE>(a.T, has_content);
+  // blocks go round-robin over the 8 XCDs: keep the tiles of one (b,h) on one XCD (they walk the
+  // same K and V in step, so its L2 serves all but the first), long tiles first.  The tile with
+  // the last time step runs longest: all of those go first, or the last of them would end the launch alone.
+  const int nbh = a.B * a.H;
+  int bh, tile;
+  {
+    const int L = blockIdx.x;
+    if (nt == 1) {
+      bh = L;
+      tile = 0;
+    } else if (L < nbh) {
+      bh = L;
+      tile = nt - 1;
+    } else if ((nbh & 7) == 0) {
+      const int s = (L - nbh) >> 3;
+      bh = ((L - nbh) & 7) + 8 * (s / (nt - 1));
+      tile = nt - 2 - s % (nt - 1);
+    } else {
+      bh = (L - nbh) / (nt - 1);
+      tile = nt - 2 - (L - nbh) % (nt - 1);
+    }
+  }
+  if constexpr (LAST_APART<DH, NCT, PHASE>)
+    if (has_content && tile == nt - 1) {
+      query_walk<DH, NCT, PHASE, true>(a, q0, k0, accum, bh, tile);
+      return;
+    }
+  query_walk<DH, NCT, PHASE, false>(a, q0, k0, accum, bh, tile);
 }
 
 }  // namespace bwdq
@@ -795,8 +855,8 @@ int mvpa_bwd_query_mfma_supported(const mvpa_bwd_args* a) {
 template <int DH, int NCT, int PHASE>
 static void launch_query(const mvpa_bwd_args* a, hipStream_t stream, int q0, int k0, int accum) {
   using namespace mvpa::bwdq;
-  constexpr int nw = PHASE_WAVES<PHASE>, tqw = nw / NCT;
-  const int nt = (a->T + tqw - 1) / tqw;
+  constexpr int nw = PHASE_WAVES<PHASE>;
+  const int nt = query_tiles<DH, NCT, PHASE>(a->T, a->flags & MVPA_FLAG_CONTENT);
   constexpr size_t lds = QUERY_LDS<DH, NCT, PHASE>;
   static_assert(lds <= 160 * 1024 / (DH == 64 ? 2 : 1), "query-pass ring exceeds the LDS");
   dim3 grid((unsigned)(nt * a->B * a->H));
