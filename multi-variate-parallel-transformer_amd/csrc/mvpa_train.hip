@@ -23,13 +23,14 @@ __device__ inline float wave_sum(float x) {
   return x;
 }
 
-__device__ inline void load4(const float* p, float (&v)[4]) {
-  const f32x4 x = *(const f32x4*)p;
+// four values as they lie in memory
+__device__ inline f32x4 raw4(const float* p) { return *(const f32x4*)p; }
+__device__ inline u32x2 raw4(const bf16_t* p) { return *(const u32x2*)p; }
+__device__ inline void widen(f32x4 x, float (&v)[4]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = x[i];
 }
-__device__ inline void load4(const bf16_t* p, float (&v)[4]) {
-  const u32x2 x = *(const u32x2*)p;
+__device__ inline void widen(u32x2 x, float (&v)[4]) {
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     v[2 * i] = __uint_as_float(x[i] << 16);
@@ -46,7 +47,7 @@ __device__ inline void get4(const T* row, int c, int cols, float (&v)[4]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = 0.f;
   if (VEC) {
-    if (c < cols) load4(row + c, v);
+    if (c < cols) widen(raw4(row + c), v);
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -67,7 +68,10 @@ __device__ inline void put4(T* row, int c, int cols, const float (&v)[4]) {
 // y = x r w with r = rsqrt(mean(x^2) + eps):   dx = r w dy - x r^3 mean(x w dy) (+ res),   dw = sum_rows dy x r
 // A wave owns whole rows, a lane the same columns of each of them: the row is in registers between its
 // two sums and its result, and the lane's share of dw stays there over all rows.  HBM bound.  512 workgroups:
-// with one per four rows the partial sums of dw are as many bytes as a row operand.
+// with one per four rows the partial sums of dw are as many bytes as a row operand.  The next row is requested
+// before the sums of this one, without a branch per chunk, behind which each load would be waited for by itself: with
+// the sums of dw 18.6 -> 13.8 us for 6400 rows of 768 in bf16, 144 -> 79 for 65536.  Wider rows do not fit the registers
+// twice (2560 in fp32: 69 -> 174 us) and are read as they come.
 template <typename TX, typename TW, int NCH, bool VEC>
 __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restrict__ x, const TW* __restrict__ w,
                                                                const bf16_t* __restrict__ dy, const TX* __restrict__ res,
@@ -83,14 +87,46 @@ __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restr
     for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
   }
   const float rcols = 1.f / (float)cols;
-  for (int64_t row = (int64_t)blockIdx.x * 4 + wave; row < rows; row += (int64_t)gridDim.x * 4) {
-    float xv[NCH][4], gv[NCH][4];
+  // chunks beyond the row read its last four columns and count as zero
+  constexpr bool AHEAD = VEC && NCH <= (sizeof(TX) == 2 ? 8 : 4);
+  constexpr int NR = AHEAD ? NCH : 1;
+  decltype(raw4(x)) x_raw[NR], r_raw[NR];
+  u32x2 g_raw[NR];
+  const TX* res_or_x = res ? res : x;
+  auto request = [&](int64_t row) {
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) {
+        const int64_t at = row * cols + min((i * 64 + lane) * 4, cols - 4);
+        x_raw[i] = raw4(x + at);
+        g_raw[i] = raw4(dy + at);
+        r_raw[i] = raw4(res_or_x + at);
+      }
+    }
+  };
+  const int64_t first = (int64_t)blockIdx.x * 4 + wave, stride = (int64_t)gridDim.x * 4;
+  if (first < rows) request(first);
+  for (int64_t row = first; row < rows; row += stride) {
+    float xv[NCH][4], gv[NCH][4], add[NR][4];
     float ss = 0.f, dot = 0.f;
 #pragma unroll
     for (int i = 0; i < NCH; ++i) {
-      get4<VEC>(x + row * cols, (i * 64 + lane) * 4, cols, xv[i]);
-      get4<VEC>(dy + row * cols, (i * 64 + lane) * 4, cols, gv[i]);
+      const int c = (i * 64 + lane) * 4;
+      if constexpr (AHEAD) {
+        widen(x_raw[i], xv[i]);
+        widen(g_raw[i], gv[i]);
+        widen(r_raw[i], add[i]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (c >= cols) xv[i][j] = gv[i][j] = 0.f;
+          if (!res) add[i][j] = 0.f;
+        }
+      } else {
+        get4<VEC>(x + row * cols, c, cols, xv[i]);
+        get4<VEC>(dy + row * cols, c, cols, gv[i]);
+      }
     }
+    request(min(row + stride, rows - 1));
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
@@ -105,10 +141,10 @@ __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restr
     for (int i = 0; i < NCH; ++i) {
       const int c = (i * 64 + lane) * 4;
       if (dx) {
-        float o[4], add[4] = {0.f, 0.f, 0.f, 0.f};
-        if (res) get4<VEC>(res + row * cols, c, cols, add);
+        float o[4], late[4] = {0.f, 0.f, 0.f, 0.f};
+        if (!AHEAD && res) get4<VEC>(res + row * cols, c, cols, late);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) o[j] = r * (gv[i][j] * wv[i][j]) - xv[i][j] * k + add[j];
+        for (int j = 0; j < 4; ++j) o[j] = r * (gv[i][j] * wv[i][j]) - xv[i][j] * k + (AHEAD ? add[AHEAD ? i : 0][j] : late[j]);
         put4<VEC>(dx + row * cols, c, cols, o);
       }
 #pragma unroll
