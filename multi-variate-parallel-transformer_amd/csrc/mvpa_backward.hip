@@ -308,7 +308,7 @@ static int launch_bwd_dh(const mvpa_bwd_args* a, hipStream_t stream, bool query_
 
 }  // namespace mvpa
 
-int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_head) {
+int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out) {
   if (!a) return MVPA_ERR_NULL;
   if (a->struct_size != sizeof(mvpa_bwd_args)) return MVPA_ERR_STRUCT;
   if (!a->q || !a->k || !a->v || !a->o || !a->d_o || !a->lse || !a->dq || !a->dk || !a->dv ||
@@ -324,10 +324,10 @@ int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_he
   if (a->dtype == MVPA_F32) return mvpa::launch_bwd_dh<float>(a, stream, true);
   if (a->dtype == MVPA_BF16) {
     // bf16, Dh = 64 or 128, C <= 128: both passes run on MFMA
-    if (mvpa_bwd_query_mfma_supported(a)) return mvpa_launch_bwd_mfma(a, stream, per_head);
+    if (mvpa_bwd_query_mfma_supported(a)) return mvpa_launch_bwd_mfma(a, stream, per_head, out);
     return mvpa::launch_bwd_dh<mvpa::bf16_t>(a, stream, true);
   }
   return MVPA_ERR_DTYPE;
 }
 
-extern "C" int mvpa_backward(const mvpa_bwd_args* a, void* stream) { return mvpa_backward_checked(a, (hipStream_t)stream, 0); }
+extern "C" int mvpa_backward(const mvpa_bwd_args* a, void* stream) { return mvpa_backward_checked(a, (hipStream_t)stream, 0, nullptr); }

@@ -895,7 +895,7 @@ template <int NCT> constexpr int KSTAGES = NCT == 2 ? 2 : 3;      // ring depth
 
 // NEAR: the far steps are left to mvpa_bwd_far_kernel, which has written dv before.
 template <int DH, int NCT, bool MASKED, bool NEAR>
-__global__ __launch_bounds__(KEY_WAVES * 64, DH == 64 ? 2 : 1) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, int k0, int q0, int accum, int per_head) {
+__global__ __launch_bounds__(KEY_WAVES * 64, DH == 64 ? 2 : 1) void mvpa_bwd_key_mfma_kernel(mvpa_bwd_args a, mvpa_kv_out out, int k0, int q0, int accum, int per_head) {
   constexpr int KS = DH / 16, MT = DH / 32, ROWB = 2 * DH, CPR = DH / 8;
   constexpr int NW = KEY_WAVES;
   constexpr int CP = NCT * 32, KT = NW / NCT, TILE = CP * ROWB;
@@ -1218,21 +1218,53 @@ __global__ __launch_bounds__(KEY_WAVES * 64, DH == 64 ? 2 : 1) void mvpa_bwd_key
     for (int n = n_idle; n > 0; --n) (void)ring_step();
   }
 
+  // The last of the launches that add to these rows rounds them to the caller's dk and dv where there are such: a
+  // lane swaps half of two runs of four columns with its partner and stores eight (a pass over the fp32 results took
+  // 61 us at B4 H16 C64 T128).
   if (stores) {
+    constexpr float f = 1.f / kLog2e;
+    const int64_t n_out = (int64_t)tk * C_ + ck;
+    bf16_t* dk_out = (bf16_t*)out.dk + b * out.dk_sb + g * out.dk_sh + n_out * out.dk_sn;
+    bf16_t* dv_out = (bf16_t*)out.dv + b * out.dv_sb + g * out.dv_sh + n_out * out.dv_sn;
+    auto store8 = [&](bf16_t* dst, const float (&x)[2][4]) {
+      union { bf16x2 h[2]; uint32_t w[2]; } p[2];
+#pragma unroll
+      for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) p[r].h[e] = __builtin_convertvector(f32x2{x[r][2 * e], x[r][2 * e + 1]}, bf16x2);
+      const auto w0 = __builtin_amdgcn_permlane32_swap(p[0].w[0], p[1].w[0], false, false);
+      const auto w1 = __builtin_amdgcn_permlane32_swap(p[0].w[1], p[1].w[1], false, false);
+      *(u32x4*)dst = u32x4{w0[0], w1[0], w0[1], w1[1]};
+    };
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int a4 = 0; a4 < 4; ++a4) {
-        const int d = mt * 32 + a4 * 8 + hh * 4;
-        constexpr float f = 1.f / kLog2e;
-        float4 vk = make_float4(dK[mt][a4 * 4] * f, dK[mt][a4 * 4 + 1] * f, dK[mt][a4 * 4 + 2] * f, dK[mt][a4 * 4 + 3] * f);
-        const float4 vv = make_float4(dV[mt][a4 * 4], dV[mt][a4 * 4 + 1], dV[mt][a4 * 4 + 2], dV[mt][a4 * 4 + 3]);
-        if (accum) {                              // launches of one stream: the query parts add up
-          const float4 ok = *(const float4*)(a.dk + out_row + d);
-          vk = make_float4(vk.x + ok.x, vk.y + ok.y, vk.z + ok.z, vk.w + ok.w);
+      for (int a2 = 0; a2 < 2; ++a2) {
+        float vk[2][4], vv[2][4];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            vk[r][x] = dK[mt][(2 * a2 + r) * 4 + x] * f;
+            vv[r][x] = dV[mt][(2 * a2 + r) * 4 + x];
+          }
+        const int64_t d = out_row + mt * 32 + a2 * 16 + hh * 4;
+        if (accum)                                // launches of one stream: the query parts add up
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            const float4 ok = *(const float4*)(a.dk + d + 8 * r);
+            vk[r][0] += ok.x; vk[r][1] += ok.y; vk[r][2] += ok.z; vk[r][3] += ok.w;
+          }
+        if (out.dk) {
+          store8(dk_out + mt * 32 + a2 * 16 + hh * 8, vk);
+          store8(dv_out + mt * 32 + a2 * 16 + hh * 8, vv);
+        } else {
+#pragma unroll
+          for (int r = 0; r < 2; ++r) {
+            *(float4*)(a.dk + d + 8 * r) = make_float4(vk[r][0], vk[r][1], vk[r][2], vk[r][3]);
+            *(float4*)(a.dv + d + 8 * r) = make_float4(vv[r][0], vv[r][1], vv[r][2], vv[r][3]);
+          }
         }
-        *(float4*)(a.dk + out_row + d) = vk;
-        *(float4*)(a.dv + out_row + d) = vv;
       }
   }
 }
@@ -1442,7 +1474,7 @@ static void launch_far(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 }
 
 template <int DH, int NCT, bool MASKED, bool NEAR>
-static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q0, int accum, int per_head) {
+static void launch_key(const mvpa_bwd_args* a, const mvpa_kv_out& out, hipStream_t stream, int k0, int q0, int accum, int per_head) {
   using namespace mvpa::bwdq;
   constexpr int nw = KEY_WAVES, cp = NCT * 32, kt = nw / NCT, ROWB = 2 * DH;
   static_assert((size_t)KSTAGES<NCT> * (2 * cp * ROWB + cp * cp * 4 + (kt + 1) * 256) <= 160 * 1024 / (DH == 64 ? 2 : 1), "key-pass ring exceeds the LDS");
@@ -1450,7 +1482,7 @@ static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
   dim3 grid((unsigned)(((a->T + kt - 1) / kt) * a->B * (per_head ? a->H : a->Hkv)));
   auto kern = mvpa_bwd_key_mfma_kernel<DH, NCT, MASKED, NEAR>;
   mvpa::want_dynamic_lds((const void*)kern, (int)lds);
-  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, k0, q0, accum, per_head);
+  MVPA_LAUNCH(kern, grid, dim3(nw * 64), lds, stream, *a, out, k0, q0, accum, per_head);
 }
 
 // Both passes.  Up to 32 channels: one launch each with one channel tile per wave; up to 64: one
@@ -1467,7 +1499,7 @@ static void launch_key(const mvpa_bwd_args* a, hipStream_t stream, int k0, int q
 // T 512 40.8 / 39.3 (query pass 18.5 / 16.3).
 constexpr int SPLIT_STEPS = 256;
 template <int DH>
-static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per_head) {
+static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out) {
   using namespace mvpa::bwdq;
   const int C = a->C, T = a->T;
   constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
@@ -1482,9 +1514,10 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
   const bool split_query = DH == 128 && (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && T - 2 - a->window >= SPLIT_STEPS;
   auto key_launch = [&](auto near, int kk, int qq, int accum) {
     constexpr bool NEAR = decltype(near)::value;
+    const mvpa_kv_out to = out && qq + KEY_CP >= C ? *out : mvpa_kv_out{};        // the last query part rounds
     const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
-    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, stream, kk, qq, accum, per_head);
-    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, stream, kk, qq, accum, per_head);
+    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, to, stream, kk, qq, accum, per_head);
+    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, to, stream, kk, qq, accum, per_head);
   };
   auto key_launches = [&](int q0, int k0, int span, bool first_q) {
     if (far) launch_far<DH>(a, stream, k0, q0, !first_q, per_head);
@@ -1497,8 +1530,9 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
   };
   if (C <= 32) {
     launch_query<DH, 1, ONE>(a, stream, 0, 0, 0);
-    if (C == 32) launch_key<DH, 1, false, false>(a, stream, 0, 0, 0, per_head);
-    else launch_key<DH, 1, true, false>(a, stream, 0, 0, 0, per_head);
+    const mvpa_kv_out to = out ? *out : mvpa_kv_out{};
+    if (C == 32) launch_key<DH, 1, false, false>(a, to, stream, 0, 0, 0, per_head);
+    else launch_key<DH, 1, true, false>(a, to, stream, 0, 0, 0, per_head);
   } else {
     const int parts = (C + 63) / 64;
     for (int kp = 0; kp < parts; ++kp)
@@ -1515,8 +1549,8 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
   }
 }
 
-int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head) {
-  if (a->Dh == 64) launch_bwd_parts<64>(a, stream, per_head);
-  else launch_bwd_parts<128>(a, stream, per_head);
+int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out) {
+  if (a->Dh == 64) launch_bwd_parts<64>(a, stream, per_head, out);
+  else launch_bwd_parts<128>(a, stream, per_head, out);
   return mvpa::take_launch_status();
 }

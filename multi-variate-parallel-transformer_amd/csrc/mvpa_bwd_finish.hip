@@ -28,7 +28,7 @@ constexpr int JB = 64;               // table rows per step of finish_rows
 constexpr int TJ = 128, TN = 64;     // table rows per workgroup, query rows per step of finish_tables
 
 struct fin_args {
-  int32_t B, H, Hkv, T, C, N;
+  int32_t B, H, Hkv, T, C, N, kv_done;
   const bf16_t* q;
   int64_t q_sb, q_sh, q_sn;
   const bf16_t *bias_v, *bias_z, *k_time, *k_chan;
@@ -591,13 +591,39 @@ static void row_split(const mvpa_bwd_args* b, int* n_split, int* len) {
   *n_split = (int)((N + *len - 1) / *len);
 }
 
-// A workgroup of the key pass walks the query heads of a kv head one after the other.  Where its workgroups (of four
-// key steps) are less than two rounds of the chip, each query head gets its own, and finish_kv adds up their dk, dv.
+// A workgroup of the key pass walks the query heads of a kv head one after the other.  Where its workgroups (counted
+// as four key steps each) are less than two rounds of the chip, each query head gets its own, and finish_kv adds up their dk, dv.
 // Forward and backward without / with, us: B4 C64 T25 H12/4 (112 workgroups) 342 / 293, B1 C64 T64 (64) 468 / 329,
 // B2 C64 T128 (256) 1091 / 1022, B1 C128 T128 H16/8 Dh128 (256) 5810 / 5350, B4 C128 T64 H16/8 Dh128 (512) 7430 / 7870.
 constexpr int64_t KEY_GROUPS_FULL = 512;
 static bool per_head(const mvpa_bwd_args* b) {
   return b->H > b->Hkv && (int64_t)b->B * b->Hkv * ((b->T + 3) / 4) < KEY_GROUPS_FULL;
+}
+
+// dk and dv share no memory with what the passes read
+static bool apart(const mvpa_bwd_args* a, const mvpa_bwd_grads* o) {
+  struct span { uintptr_t lo, hi; };
+  const int64_t N = (int64_t)a->T * a->C;
+  auto rows = [&](const void* p, int heads, int64_t sb, int64_t sh, int64_t sn) {
+    int64_t lo = 0, hi = a->Dh;
+    for (const int64_t reach : {(a->B - 1) * sb, (heads - 1) * sh, (N - 1) * sn}) (reach < 0 ? lo : hi) += reach;
+    return span{(uintptr_t)p + 2 * lo, (uintptr_t)p + 2 * hi};
+  };
+  auto flat = [](const void* p, int64_t bytes) { return span{(uintptr_t)p, (uintptr_t)p + (p ? bytes : 0)}; };
+  const span outs[] = {rows(o->dk, a->Hkv, o->dk_stride_b, o->dk_stride_h, o->dk_stride_n),
+                       rows(o->dv, a->Hkv, o->dv_stride_b, o->dv_stride_h, o->dv_stride_n)};
+  const span ins[] = {rows(a->q, a->H, a->q_stride_b, a->q_stride_h, a->q_stride_n),
+                      rows(a->k, a->Hkv, a->k_stride_b, a->k_stride_h, a->k_stride_n),
+                      rows(a->v, a->Hkv, a->v_stride_b, a->v_stride_h, a->v_stride_n),
+                      rows(a->o, a->H, a->o_stride_b, a->o_stride_h, a->o_stride_n),
+                      rows(a->d_o, a->H, a->do_stride_b, a->do_stride_h, a->do_stride_n),
+                      flat(a->lse, 4 * a->B * a->H * N), flat(a->bias_u, 2 * a->Hkv * a->Dh), flat(a->bias_v, 2 * a->Hkv * a->Dh),
+                      flat(a->bias_z, 2 * a->Hkv * a->Dh), flat(a->k_time, 2ll * a->Hkv * a->T * a->Dh),
+                      flat(a->k_chan, 2ll * a->Hkv * a->C * a->Dh), flat(a->chan_valid, (int64_t)a->B * a->C)};
+  for (const span& x : outs)
+    for (const span& y : ins)
+      if (x.lo < y.hi && y.lo < x.hi) return false;
+  return true;
 }
 
 // steps of 64 columns that finish_fused keeps sums for, 0 where they do not fit the registers
@@ -657,7 +683,9 @@ static int launch_finish(const fin_args& f, hipStream_t s) {
                 dim3(256), 0, s, f);
   }
   const int64_t kv = 2 * (int64_t)f.B * f.Hkv * f.N * (DH / 8);
-  MVPA_LAUNCH(finish_kv_kernel<DH>, dim3((unsigned)((kv + 255) / 256)), dim3(256), 0, s, f);
+  if (!f.kv_done) {
+    MVPA_LAUNCH(finish_kv_kernel<DH>, dim3((unsigned)((kv + 255) / 256)), dim3(256), 0, s, f);
+  }
   MVPA_LAUNCH(finish_reduce_kernel<DH>, dim3((unsigned)(f.T + f.C), (unsigned)f.Hkv), dim3(256), 0, s, f);
   MVPA_LAUNCH(finish_biases_kernel<DH>, dim3((unsigned)f.Hkv, 3), dim3(1024), 0, s, f, row_tiles);
   return take_launch_status();
@@ -692,7 +720,10 @@ extern "C" int mvpa_backward_full(const mvpa_bwd_args* a, const mvpa_bwd_grads* 
   fin::lay_out(a, f, w, l);
   if ((size_t)l.used > ws_bytes) return MVPA_ERR_WS_SIZE;
   if (!mvpa_bwd_query_mfma_supported(&w)) return MVPA_ERR_UNSUPPORTED;
-  const int st = mvpa_backward_checked(&w, (hipStream_t)stream, f.kv_parts > 1);
+  // dk and dv from the key pass itself, unless parts of them are to be added or they lie where inputs are still read
+  const mvpa_kv_out out{o->dk, o->dv, o->dk_stride_b, o->dk_stride_h, o->dk_stride_n, o->dv_stride_b, o->dv_stride_h, o->dv_stride_n};
+  f.kv_done = f.kv_parts == 1 && fin::apart(a, o);
+  const int st = mvpa_backward_checked(&w, (hipStream_t)stream, f.kv_parts > 1, f.kv_done ? &out : nullptr);
   if (st != MVPA_OK) return st;
   f.B = a->B; f.H = a->H; f.Hkv = a->Hkv; f.T = a->T; f.C = a->C; f.N = a->T * a->C;
   f.q = (const bf16_t*)a->q;

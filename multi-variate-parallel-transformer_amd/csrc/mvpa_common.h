@@ -154,5 +154,10 @@ int mvpa_launch_mfma128(const mvpa_fwd_args* a, hipStream_t stream);
 // backward, query pass on MFMA (bf16, Dh = 64, C <= 64)
 int mvpa_bwd_query_mfma_supported(const mvpa_bwd_args* a);
 // per_head: dk and dv come per query head ([B,H,N,Dh]), for the caller to add up
-int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head);
-int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_head);
+// bf16 [B,Hkv,N,Dh] at element strides, in place of the fp32 results a->dk, a->dv (which then are workspace)
+struct mvpa_kv_out {
+  void *dk, *dv;
+  int64_t dk_sb, dk_sh, dk_sn, dv_sb, dv_sh, dv_sn;
+};
+int mvpa_launch_bwd_mfma(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out);
+int mvpa_backward_checked(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out);

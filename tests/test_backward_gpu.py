@@ -390,3 +390,23 @@ def test_backward_finish_against_table_products(cfg, flags):
     for n, g in zip(NAMES, got):
         bound = 1.02 * 2.0 ** -8 * (want[n].abs() + size[n]) + 2.0 ** -10 * size[n]
         assert ((g.double() - want[n]).abs() <= bound).all(), n
+
+
+@pytest.mark.parametrize("C,T,Dh,H,Hkv", [
+    (5, 9, 64, 2, 2), (32, 20, 64, 2, 2), (33, 45, 64, 3, 3), (64, 130, 64, 16, 16), (65, 14, 64, 2, 2), (128, 33, 64, 2, 2),
+    (20, 15, 128, 2, 2), (40, 13, 128, 2, 2), (100, 30, 128, 2, 2),
+    (64, 160, 64, 32, 16),                        # two query heads walked by one workgroup
+])
+def test_key_gradients_rounded_where_they_are_summed(C, T, Dh, H, Hkv):
+    """dk and dv of mvpa_backward_full are the fp32 results of mvpa_backward, rounded once: bit for bit."""
+    import mvpa_hip
+    inp = make_mvpa_inputs(seed=29, qkv_unit=True, B=1, C=C, T=T, H=H, Hkv=Hkv, Dh=Dh).to("cuda", torch.bfloat16)
+    tabs = (inp.u, inp.vb, inp.z, inp.k_time, inp.k_chan)
+    if H > Hkv:
+        assert Hkv * ((T + 3) // 4) >= 512                         # fewer: a workgroup per query head, sums of parts
+    out, lse = mvpa_hip.mvpa_forward(inp.q, inp.k, inp.v, *tabs, return_lse=True)
+    d_o = torch.randn(out.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(3)).bfloat16()
+    scale = Dh ** -0.5
+    got = dict(zip(NAMES, mvpa_hip.mvpa_backward_full(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=scale)))
+    _, dk, dv, _, _ = mvpa_hip.mvpa_backward(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=scale)
+    assert torch.equal(got["k"], dk.bfloat16()) and torch.equal(got["v"], dv.bfloat16())
