@@ -395,7 +395,7 @@ def test_backward_finish_against_table_products(cfg, flags):
 @pytest.mark.parametrize("C,T,Dh,H,Hkv", [
     (5, 9, 64, 2, 2), (32, 20, 64, 2, 2), (33, 45, 64, 3, 3), (64, 130, 64, 16, 16), (65, 14, 64, 2, 2), (128, 33, 64, 2, 2),
     (20, 15, 128, 2, 2), (40, 13, 128, 2, 2), (100, 30, 128, 2, 2),
-    (64, 160, 64, 32, 16),                        # two query heads walked by one workgroup
+    (32, 160, 64, 32, 16),                        # two query heads walked by one workgroup
 ])
 def test_key_gradients_rounded_where_they_are_summed(C, T, Dh, H, Hkv):
     """dk and dv of mvpa_backward_full are the fp32 results of mvpa_backward, rounded once: bit for bit."""
@@ -403,10 +403,27 @@ def test_key_gradients_rounded_where_they_are_summed(C, T, Dh, H, Hkv):
     inp = make_mvpa_inputs(seed=29, qkv_unit=True, B=1, C=C, T=T, H=H, Hkv=Hkv, Dh=Dh).to("cuda", torch.bfloat16)
     tabs = (inp.u, inp.vb, inp.z, inp.k_time, inp.k_chan)
     if H > Hkv:
-        assert Hkv * ((T + 3) // 4) >= 512                         # fewer: a workgroup per query head, sums of parts
+        assert C <= 32 and Hkv * ((T + 3) // 4) >= 512             # fewer: a workgroup per query head, sums of parts
     out, lse = mvpa_hip.mvpa_forward(inp.q, inp.k, inp.v, *tabs, return_lse=True)
     d_o = torch.randn(out.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(3)).bfloat16()
     scale = Dh ** -0.5
     got = dict(zip(NAMES, mvpa_hip.mvpa_backward_full(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=scale)))
     _, dk, dv, _, _ = mvpa_hip.mvpa_backward(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=scale)
     assert torch.equal(got["k"], dk.bfloat16()) and torch.equal(got["v"], dv.bfloat16())
+
+
+@pytest.mark.parametrize("B,C,T,H,Hkv", [(2, 40, 256, 12, 4), (5, 64, 252, 4, 2), (10, 33, 508, 2, 1), (10, 33, 509, 2, 1), (3, 40, 63, 8, 4)])
+def test_workgroups_per_query_head(B, C, T, H, Hkv):
+    """Both sides of the lines where each query head gets its own workgroups in the key pass (and the far kernel with
+    them): dk and dv against those of mvpa_backward, which never does.  Parts of fp32 sums in another order, one rounding."""
+    import mvpa_hip
+    inp = make_mvpa_inputs(seed=31, qkv_unit=True, B=B, C=C, T=T, H=H, Hkv=Hkv, Dh=64).to("cuda", torch.bfloat16)
+    tabs = (inp.u, inp.vb, inp.z, inp.k_time, inp.k_chan)
+    out, lse = mvpa_hip.mvpa_forward(inp.q, inp.k, inp.v, *tabs, return_lse=True)
+    d_o = torch.randn(out.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(5)).bfloat16()
+    got = dict(zip(NAMES, mvpa_hip.mvpa_backward_full(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=0.125)))
+    _, dk, dv, _, _ = mvpa_hip.mvpa_backward(inp.q, inp.k, inp.v, out, d_o, lse, *tabs, sm_scale=0.125)
+    for n, want in (("k", dk.double()), ("v", dv.double())):
+        # terms of the sums are at least as large as a typical element; 2^-10 of them for the order, as above
+        bound = 1.01 * 2.0 ** -8 * want.abs() + 2.0 ** -10 * (want.abs() + want.pow(2).mean().sqrt())
+        assert ((got[n].double() - want).abs() <= bound).all(), n
