@@ -1505,12 +1505,13 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
   constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
   // Far query steps (outside the content window and not the last step) in a kernel of their own where its
   // workgroups, of four times as many key steps, still fill the chip.  Forward and backward, far kernel / without:
-  // Dh 64, C 64, T 128: 384 workgroups 1794 / 1825 us, 256: 1265 / 1220, 128: 811 / 707;
-  // Dh 128, C 128: T 128, 128 workgroups 5.77 / 6.15 ms, T 512, 512 workgroups 40.9 / 50.7.
+  // Dh 64, C 64, T 128: 384 workgroups 1327 / 1495 us, 256: 962 / 1022, 192: 793 / 850, 128: 667 / 589; T 256 of 256:
+  // 1480 / 1648; T 64, C 40 of 192: 495 / 495; T 64 of 48: 315 / 272;
+  // Dh 128, H16/8: B1 C64 T128, 256 workgroups, 1259 / 1453; C 128: T 128, 128 workgroups 5.77 / 6.15 ms.
   constexpr int FAR_KT = FR * FAR_WAVES<DH> / 2;
   const int64_t far_groups = (int64_t)a->B * (per_head ? a->H : a->Hkv) * ((T + FAR_KT - 1) / FAR_KT);
   const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= FAR_KT &&
-                   far_groups >= (DH == 64 ? 384 : 128);
+                   far_groups >= (DH == 64 ? 192 : 128);
   const bool split_query = DH == 128 && (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && T - 2 - a->window >= SPLIT_STEPS;
   auto key_launch = [&](auto near, int kk, int qq, int accum) {
     constexpr bool NEAR = decltype(near)::value;
