@@ -128,14 +128,14 @@ template <int DH> __device__ inline int swz(int row) {
 }
 
 // ONE: the whole walk.  FAR, WIN: the steps before a wave's content window and those from it on, as a launch
-// each, FAR first.  At Dh 128 a wave of the whole walk takes 475 registers and has its SIMD to itself: the far steps'
+// each, FAR first.  At Dh 128 a wave of the whole walk takes 420 registers and has its SIMD to itself: the far steps'
 // LDS reads, products, reductions and table slabs simply add up (0.89 us a step of 2 x 64 queries at T 512, 0.25 of
 // them products).  FAR alone fits in 256, and two waves cover each other's waits (1.2 us a step of 4 x 64 queries).
 //
 // At Dh 64 a workgroup is 4 waves and two of them share a CU (80 KB and 256 registers): a third of a workgroup's life
 // at T 128 is set-up, slabs and epilogue, chains of waits that leave the CU idle if all its waves are in them at
 // once.  B4 H16 C64, T 128 / 256 / 512, one workgroup of 8 waves with a barrier a step against this: 920 / 1243 /
-// 2043 -> 714 / 1030 / 1720 us; B4 H12 C21 T25 53 -> 34 us.  The clock is what is left: the waits of a far step have
+// 2043 -> 735 / 1040 / 1730 us; B4 H12 C21 T25 53 -> 34 us.  The clock is what is left: the waits of a far step have
 // gone from 1040 to 570 of 1770 -> 1350 cycles, and it falls from 2.25 to 1.9 GHz as they go.
 enum query_phase { ONE, FAR, WIN };
 template <int PHASE> constexpr int PHASE_WAVES = PHASE == FAR ? 8 : 4;
@@ -1495,8 +1495,8 @@ static void launch_key(const mvpa_bwd_args* a, const mvpa_kv_out& out, hipStream
 // takes the (query part, key part) pair of a query-pass launch in quarters of 32 x 32 channels
 // (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).
 // far steps of the longest walk from which the two phases of the query pass are a launch each (Dh 128): the
-// set-up of a workgroup is paid twice.  Forward and backward, one launch / two: T 128 5.77 / 5.95 ms (C 128, B 1),
-// T 512 40.8 / 39.3 (query pass 18.5 / 16.3).
+// set-up of a workgroup is paid twice.  Forward and backward, one launch / two, H16/8: B2 C128 T128 8.39 / 8.82 ms, B1
+// C128 T200 9.01 / 9.10, B2 C64 T256 6.40 / 6.37, B1 C128 T300 17.1 / 17.0, T 512 36.4 / 35.8.
 constexpr int SPLIT_STEPS = 256;
 template <int DH>
 static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out) {
