@@ -25,7 +25,7 @@ FLAG_LAST_STEP = 32
 FLAG_RING = 64
 FLAG_CAUSAL, FLAG_CONTENT, FLAG_TIME_BIAS, FLAG_CHAN_BIAS, FLAG_FP8_QK = 1, 2, 4, 8, 16
 
-ERR_HEAD_DIM, ERR_HEAD_RATIO, ERR_CTX, ERR_SHAPE, ERR_UNSUPPORTED = -2, -3, -4, -5, -8
+ERR_HEAD_DIM, ERR_HEAD_RATIO, ERR_CTX, ERR_SHAPE, ERR_ALIGN, ERR_UNSUPPORTED = -2, -3, -4, -5, -7, -8
 
 
 class MvpaFwdArgs(ctypes.Structure):

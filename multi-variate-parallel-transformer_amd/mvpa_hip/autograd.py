@@ -27,8 +27,9 @@ def _weight_gradient(dy, x):
     (m, n), k = dy.shape, x.shape[-1]
     if m >= 2560 and -(-n // 128) * -(-k // 128) < 256 and not torch.is_grad_enabled():
         dw = mvpa_hip.load_ext().linear_wgrad(dy, x)
-        if type(dw) is not int:                              # a status: rows that do not start at 16-byte boundaries
-            return dw
+        # rows that do not start at 16-byte boundaries or overlap are the vendor library's; any other status is an error
+        if type(dw) is not int or dw not in (mvpa_hip.ERR_ALIGN, mvpa_hip.ERR_SHAPE, mvpa_hip.ERR_UNSUPPORTED):
+            return mvpa_hip._taken(dw)
     return torch.matmul(dy.t(), x)
 
 

@@ -229,6 +229,26 @@ def test_python_operator_errors():
         flashmvpa(q, b, b, b, kv, torch.zeros(1, 4, 4, 32), torch.zeros(1, 4, 3, 32), kv, True, 0.1)
 
 
+@pytest.mark.parametrize("status,falls_back", [(-5, True), (-7, True), (-8, True), (-1, False), (-10, False), (-12, False)])
+def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_back):
+    """Operands the kernel does not take go to the general product; a launch that failed or a workspace that is too
+    small does not."""
+    from mvpa_hip import autograd as AG
+
+    class Refusing:
+        @staticmethod
+        def linear_wgrad(dy, x):
+            return status
+    monkeypatch.setattr(mvpa_hip, "load_ext", lambda: Refusing)
+    dy, x = torch.ones(2560, 8, dtype=torch.bfloat16), torch.ones(2560, 16, dtype=torch.bfloat16)
+    with torch.no_grad():
+        if falls_back:
+            assert torch.equal(AG._weight_gradient(dy, x), dy.t() @ x)
+        else:
+            with pytest.raises(mvpa_hip.MvpaError):
+                AG._weight_gradient(dy, x)
+
+
 def test_layer_state_dict_names():
     from types import SimpleNamespace
     from layers import MVPFormerGQAAttention, MVPFormerGQAFlashAttention

@@ -236,3 +236,20 @@ def test_weight_gradient_refuses_rows_off_16_bytes():
     dy = torch.randn(3000 * 24 + 1, device="cuda").bfloat16()[1:].view(3000, 24)
     dw, = torch.autograd.grad(AG.linear(x, w), w, dy)
     _close(dw, dy.double().t() @ x.double(), 3000)
+
+
+def test_weight_gradient_of_aligned_rows_is_the_kernels(monkeypatch):
+    """Through the autograd function, from 2560 rows on: what it returns is what the kernel returned."""
+    ext, seen = mvpa_hip.load_ext(), []
+    kernel = ext.linear_wgrad
+
+    def record(dy, x):
+        seen.append(kernel(dy, x))
+        return seen[-1]
+    monkeypatch.setattr(ext, "linear_wgrad", record)
+    for m in (2559, 2560):
+        x, dy = torch.randn(m, 72, device="cuda").bfloat16(), torch.randn(m, 136, device="cuda").bfloat16()
+        w = torch.randn(136, 72, device="cuda").bfloat16().requires_grad_(True)
+        dw, = torch.autograd.grad(AG.linear(x, w), w, dy)
+        _close(dw, dy.double().t() @ x.double(), m)
+    assert len(seen) == 1 and isinstance(seen[0], torch.Tensor) and torch.equal(seen[0], dw)
