@@ -663,30 +663,53 @@ PyObject* py_enqueue(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// The parts of stacked projections with adapters: `mods` holds (enable, w, a | None, b | None) per module;
-// equal row slices of a module, each with its share of a and b where enabled.
+// `mods`: a tuple of (enable, w, a | None, b | None) per module, enable a tuple of truth values
+bool lora_modules(PyObject* mods) {
+  if (!PyTuple_Check(mods) || PyTuple_GET_SIZE(mods) == 0) return false;
+  for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
+    PyObject* mod = PyTuple_GET_ITEM(mods, m);
+    if (!PyTuple_Check(mod) || PyTuple_GET_SIZE(mod) != 4 || !PyTuple_Check(PyTuple_GET_ITEM(mod, 0))) return false;
+  }
+  return true;
+}
+
+// The parts of stacked projections with adapters: equal row slices of a module, each with its share of a and b
+// where enabled.  Operands as the kernels read them; the backward's come out of autograd's hands (a saved-tensor hook
+// may return them in another layout).  Of w the backward takes the shape.
 struct LoraParts {
   std::vector<mvpa_lora_part> parts;
+  std::vector<Tensor> keep;
   int64_t rows = 0, K = 0, r = 0;
 };
-bool lora_parts(PyObject* mods, LoraParts& l) {
+bool lora_parts(PyObject* mods, bool backward, LoraParts& l) {
+  TORCH_CHECK(lora_modules(mods), "lora_stack: (enable, w, a, b) per module");
+  auto held = [&](const Tensor& t) -> Tensor { return l.keep.emplace_back(aligned_operand(t, at::kBFloat16)); };
   for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
     PyObject* mod = PyTuple_GET_ITEM(mods, m);
     PyObject* enable = PyTuple_GET_ITEM(mod, 0);
-    const Tensor& w = tensor_of(PyTuple_GET_ITEM(mod, 1));
+    const Tensor& shape = tensor_of(PyTuple_GET_ITEM(mod, 1));
     const bool has = !is_none(PyTuple_GET_ITEM(mod, 2));
-    const int64_t slices = has ? PyTuple_GET_SIZE(enable) : 1, rows = w.size(0) / slices;
-    l.K = w.size(1);
+    const int64_t slices = has ? PyTuple_GET_SIZE(enable) : 1;
+    TORCH_CHECK(shape.dim() == 2 && slices > 0 && shape.size(0) % slices == 0 && (l.K == 0 || shape.size(1) == l.K),
+                "lora_stack: weights of one width, in equal slices");
+    const int64_t rows = shape.size(0) / slices;
+    l.K = shape.size(1);
+    const Tensor w = backward ? Tensor() : held(shape);
+    Tensor a, b;
+    if (has) {
+      a = held(tensor_of(PyTuple_GET_ITEM(mod, 2)));
+      b = held(tensor_of(PyTuple_GET_ITEM(mod, 3)));
+      TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == l.K && (l.r == 0 || b.size(1) == l.r),
+                  "lora_stack: an adapter does not fit its weight");
+      l.r = b.size(1);
+    }
     int64_t j = 0;
     for (int64_t i = 0; i < slices; ++i) {
       mvpa_lora_part p{};
-      p.w = (const char*)w.const_data_ptr() + i * rows * l.K * 2;
+      if (!backward) p.w = (const char*)w.const_data_ptr() + i * rows * l.K * 2;
       p.rows = (int32_t)rows;
       if (has && PyTuple_GET_ITEM(enable, i) == Py_True) {
-        const Tensor &a = tensor_of(PyTuple_GET_ITEM(mod, 2)), &b = tensor_of(PyTuple_GET_ITEM(mod, 3));
-        l.r = b.size(1);
-        TORCH_CHECK(a.dim() == 2 && b.dim() == 2 && a.size(1) == l.K && a.size(0) >= (j + 1) * l.r && b.size(0) >= (j + 1) * rows,
-                    "lora_stack: an adapter does not fit its weight");
+        TORCH_CHECK(a.size(0) >= (j + 1) * l.r && b.size(0) >= (j + 1) * rows, "lora_stack: an adapter does not fit its weight");
         p.a = (const char*)a.const_data_ptr() + j * l.r * l.K * 2;
         p.b = (const char*)b.const_data_ptr() + j * rows * l.r * 2;
         ++j;
@@ -708,6 +731,7 @@ PyObject* py_lora_fits(PyObject*, PyObject* mods) {
     return !t.is_cuda() || t.scalar_type() != at::kBFloat16 || t.dim() != 2 || !t.is_contiguous() || t.numel() == 0 ||
            ((uintptr_t)t.const_data_ptr() & 15);
   };
+  if (!lora_modules(mods)) Py_RETURN_FALSE;
   for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
     PyObject* mod = PyTuple_GET_ITEM(mods, m);
     PyObject* enable = PyTuple_GET_ITEM(mod, 0);
@@ -739,12 +763,12 @@ PyObject* py_lora_fits(PyObject*, PyObject* mods) {
 // and b in turn (None without an adapter) | status
 PyObject* py_lora_stack(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  TORCH_CHECK((n == 2 || n == 3) && PyTuple_Check(args[0]), "lora_stack takes the modules' weights, a scale and, for the backward, a gradient");
+  TORCH_CHECK(n == 2 || n == 3, "lora_stack takes the modules' weights, a scale and, for the backward, a gradient");
   const double scale = PyFloat_AsDouble(args[1]);
   if (PyErr_Occurred()) return nullptr;
   at::AutoDispatchBelowADInplaceOrView guard;
   LoraParts l;
-  if (!lora_parts(args[0], l)) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  if (!lora_parts(args[0], n == 3, l)) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
   const Tensor& first = tensor_of(PyTuple_GET_ITEM(PyTuple_GET_ITEM(args[0], 0), 1));
   if (n == 2) {
     Tensor out = at::empty({l.rows, l.K}, first.options());
@@ -763,8 +787,7 @@ PyObject* py_lora_stack(PyObject*, PyObject* const* args, Py_ssize_t n) {
       ++at;
       continue;
     }
-    grads[2 * m] = at::empty_like(tensor_of(PyTuple_GET_ITEM(mod, 2)));
-    grads[2 * m + 1] = at::empty_like(tensor_of(PyTuple_GET_ITEM(mod, 3)));
+    for (int i = 0; i < 2; ++i) grads[2 * m + i] = at::empty(tensor_of(PyTuple_GET_ITEM(mod, 2 + i)).sizes(), d.options());
     int64_t j = 0;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(PyTuple_GET_ITEM(mod, 0)); ++i, ++at) {
       mvpa_lora_part& p = l.parts[at];

@@ -211,8 +211,8 @@ def _stacked_weights(mods) -> torch.Tensor:
     tuned = [m for m in mods if isinstance(m, _LoRALinear) and m.r > 0 and hasattr(m, "lora_A")]
     if (tuned and all(type(m) in (_LoRALinear, torch.nn.Linear) and "effective_weight" not in m.__dict__ for m in mods)
             and all(m.scaling == tuned[0].scaling for m in tuned) and mods[0].weight.is_cuda):
-        w = AG.lora_stack(tuple((m.enable, m.weight, m.lora_A, m.lora_B) if m in tuned else ((), m.weight, None, None)
-                                for m in mods), float(tuned[0].scaling))
+        w = AG.lora_stack(tuple((tuple(map(bool, m.enable)), m.weight, m.lora_A, m.lora_B) if m in tuned
+                                else ((), m.weight, None, None) for m in mods), float(tuned[0].scaling))
         if w is not None:
             return w
     return torch.cat([_weight_of(m) for m in mods], 0)

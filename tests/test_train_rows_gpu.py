@@ -201,6 +201,40 @@ def test_stacked_weights_that_the_kernel_refuses():
     assert mod.lora_B.grad.abs().sum() > 0
 
 
+def test_stacked_weights_by_a_list_of_slices():
+    """`enable` as any sequence of truth values, as effective_weight() takes it; the binding itself refuses what is no tuple."""
+    from layers.mvpa import _LoRALinear, _stacked_weights
+    mod = _LoRALinear(16, 6, 2, 4, enable=(False, True)).to("cuda", torch.bfloat16)
+    with torch.no_grad():
+        mod.lora_B.normal_()
+    want = _stacked_weights((mod,))
+    for enable in ([False, True], [0, 1], (0, 1)):
+        mod.enable = enable
+        assert torch.equal(_stacked_weights((mod,)), want)
+    bad = (([False, True], mod.weight, mod.lora_A, mod.lora_B),)
+    assert AG.lora_stack(bad, 2.0) is None and AG.lora_stack([bad[0]], 2.0) is None
+    with pytest.raises(RuntimeError):
+        mvpa_hip.lora_stack(bad, 2.0)
+
+
+@pytest.mark.parametrize("unpack", [lambda t: t.t().contiguous().t(), lambda t: torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape),
+                                    lambda t: t.cpu()], ids=["columns", "offset", "host"])
+def test_stacked_weights_with_hooks_on_what_is_saved(unpack):
+    """A hook may hand the adapters back in another layout; on the host they are an error, not an address."""
+    torch.manual_seed(4)
+    w, a, b = (torch.randn(s, device="cuda").bfloat16().requires_grad_(True) for s in ((16, 32), (8, 32), (16, 8)))
+    mods, d = (((True,), w, a, b),), torch.randn(16, 32, device="cuda").bfloat16()
+    want = torch.autograd.grad(AG.lora_stack(mods, 0.5), (a, b), d)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+        y = AG.lora_stack(mods, 0.5)
+        if not unpack(a).is_cuda:
+            with pytest.raises(RuntimeError):
+                torch.autograd.grad(y, (a, b), d)
+            return
+        got = torch.autograd.grad(y, (a, b), d)
+    assert all(torch.equal(x, z) and x.shape == z.shape for x, z in zip(got, want))
+
+
 def test_stacked_weights_differentiate_twice():
     torch.manual_seed(3)
     w, a, b = (torch.randn(s, device="cuda").bfloat16().requires_grad_(True) for s in ((16, 32), (8, 32), (8, 8)))
