@@ -18,6 +18,13 @@ def wants_grad(*tensors) -> bool:
     return torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors)
 
 
+def _mapped(*tensors) -> bool:
+    """Whether a vmap runs over one of them (autograd.grad with is_grads_batched, torch.func): such a tensor has no
+    memory of its own that a kernel of the library could read."""
+    f = torch._C._functorch
+    return any(t is not None and (f.is_functorch_wrapped_tensor(t) or f.is_legacy_batchedtensor(t)) for t in tensors)
+
+
 def _weight_gradient(dy, x):
     """dy^T x of bf16 rows.  The library's kernel (csrc/mvpa_wgrad.hip) where its row shares pay: from 2560 rows and
     below 256 tiles of 128 x 128, us against the vendor library: [768,768] 3000 rows 20 / 28, 6400 22 / 39, 16384
@@ -25,6 +32,8 @@ def _weight_gradient(dy, x):
     16.5 / 16, 1024 14.7 / 11), and with 256 tiles the vendor's larger ones fill the chip too ([2048,2048] 65 / 64 at
     6400 rows, [11264,2048] 321 / 260)."""
     (m, n), k = dy.shape, x.shape[-1]
+    if _mapped(dy, x):                                       # rows of several gradients: one product, no batched one
+        return torch.matmul(dy.t().contiguous(), x)
     if m >= 2560 and -(-n // 128) * -(-k // 128) < 256 and not torch.is_grad_enabled():
         dw = mvpa_hip.load_ext().linear_wgrad(dy, x)
         # rows that do not start at 16-byte boundaries or overlap are the vendor library's; any other status is an error
@@ -207,13 +216,13 @@ class _LoRAStackFn(torch.autograd.Function):
         dw = d.split(rows)
         needs = ctx.needs_input_grad[2:]
         adapters = [None] * (2 * len(rows))
-        if torch.is_grad_enabled():                          # a backward that is differentiated itself
+        if torch.is_grad_enabled() or _mapped(d, *a, *b):     # a backward that is differentiated itself, or mapped over
             for m, (on, am, bm) in enumerate(zip(enables, a, b)):
                 if am is None:
                     continue
                 n, r = rows[m] // len(on), bm.shape[1]
                 parts = [dw[m][i * n:(i + 1) * n] * scale for i, e in enumerate(on) if e]
-                adapters[2 * m] = torch.cat([bm[j * n:(j + 1) * n].t() @ x for j, x in enumerate(parts)], 0)
+                adapters[2 * m] = torch.cat([(x.t().contiguous() @ bm[j * n:(j + 1) * n]).t() for j, x in enumerate(parts)], 0)
                 adapters[2 * m + 1] = torch.cat([x @ am[j * r:(j + 1) * r].t() for j, x in enumerate(parts)], 0)
         elif any(needs[1::3]) or any(needs[2::3]):
             adapters = mvpa_hip.lora_stack(_lora_mods(enables, dw, a, b), scale, d)

@@ -249,6 +249,32 @@ def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_bac
                 AG._weight_gradient(dy, x)
 
 
+def test_weight_gradients_under_vmap_are_no_kernel_call(monkeypatch):
+    """Gradients of several losses at once (is_grads_batched) come as tensors without memory of their own."""
+    from mvpa_hip import autograd as AG
+
+    def refuse():
+        raise AssertionError("the kernel was called")
+    monkeypatch.setattr(mvpa_hip, "load_ext", refuse)
+    g = torch.Generator().manual_seed(0)
+    dy, x = (torch.randn(s, generator=g) for s in ((3, 2560, 8), (2560, 16)))
+    want = dy.transpose(1, 2).contiguous() @ x
+    with torch.no_grad():
+        assert torch.allclose(torch.func.vmap(lambda d: AG._weight_gradient(d, x))(dy), want, atol=1e-3)
+
+    class Product(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, w):
+            return x @ w.t()
+
+        @staticmethod
+        def backward(ctx, d):
+            return AG._weight_gradient(d, x)
+    w = torch.randn(8, 16, generator=g).requires_grad_(True)
+    got, = torch.autograd.grad(Product.apply(w), w, dy, is_grads_batched=True)
+    assert torch.allclose(got, want, atol=1e-3)
+
+
 def test_layer_state_dict_names():
     from types import SimpleNamespace
     from layers import MVPFormerGQAAttention, MVPFormerGQAFlashAttention

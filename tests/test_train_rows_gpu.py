@@ -287,3 +287,17 @@ def test_weight_gradient_of_aligned_rows_is_the_kernels(monkeypatch):
         dw, = torch.autograd.grad(AG.linear(x, w), w, dy)
         _close(dw, dy.double().t() @ x.double(), m)
     assert len(seen) == 1 and isinstance(seen[0], torch.Tensor) and torch.equal(seen[0], dw)
+
+
+def test_gradients_of_several_losses_at_once():
+    """is_grads_batched through a projection of 2560 rows and more and through stacked weights with adapters."""
+    torch.manual_seed(5)
+    mods = tuple((on, *(torch.randn(s, device="cuda").bfloat16().requires_grad_(True) for s in ((rows, 64), (8, 64), (16, 8))))
+                 for on, rows in (((True,), 16), ((False, True), 32)))
+    leaves = [t for m in mods for t in m[1:]]
+    y = AG.linear(torch.randn(2560, 64, device="cuda").bfloat16(), AG.lora_stack(mods, 0.5))
+    d = torch.randn(3, *y.shape, device="cuda").bfloat16()
+    got = torch.autograd.grad(y, leaves, d, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for whole, one in zip(got, torch.autograd.grad(y, leaves, d[i], retain_graph=True)):
+            _near(whole[i], one)
