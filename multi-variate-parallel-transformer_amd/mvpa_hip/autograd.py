@@ -25,16 +25,26 @@ def _mapped(*tensors) -> bool:
     return any(t is not None and (f.is_functorch_wrapped_tensor(t) or f.is_legacy_batchedtensor(t)) for t in tensors)
 
 
+def _wgrad_on_kernel(m, n, k) -> bool:
+    """Whether the kernel of csrc/mvpa_wgrad.hip (both launches) is the faster one for dY^T X of [m, n] and [m, k],
+    us against the vendor library.  From 2560 rows: [768,768] 19 / 23, 6400 rows 23 / 46, 131072 241 / 588; [3456,768]
+    31 / 37, 51 / 70.  Below it the second launch costs more than is gained (2048 rows of [768,768] 16.5 / 16, 1024
+    14.7 / 11).  With 256 tiles of 128 x 128 the vendor's larger ones fill the chip too ([2048,2048] 65 / 64 at 6400 rows,
+    [11264,2048] 321 / 260), and so they do where many tiles meet many rows (in millions of rows times tiles:
+    [3456,768] 10.6 415 / 544, [3072,1024] 6.3 310 / 308, 12.6 588 / 452, [1536,2048] 25 1252 / 1029), earlier where rows
+    do not start at lines of 128 bytes ([640,4000] 5.2 211 / 318, 10.5 622 / 427).  Fewer than 64 tiles gain at any
+    number of rows.  Long thin outputs are padding for the most part (25600 rows of [8,16000] 169 / 154; [8,8192] of 65536 221 / 265)."""
+    tiles = -(-n // 128) * -(-k // 128)
+    if m < 2560 or tiles >= 256 or (min(n, k) < 64 and tiles > 96):
+        return False
+    return tiles < 64 or m * tiles < (12 << 20 if n % 64 == 0 and k % 64 == 0 else 8 << 20)
+
+
 def _weight_gradient(dy, x):
-    """dy^T x of bf16 rows.  The library's kernel (csrc/mvpa_wgrad.hip) where its row shares pay: from 2560 rows and
-    below 256 tiles of 128 x 128, us against the vendor library: [768,768] 3000 rows 20 / 28, 6400 22 / 39, 16384
-    34 / 91; [3456,768] 33 / 39, 48 / 61, 102 / 148.  Below it the second launch costs more than is gained (2048 rows
-    16.5 / 16, 1024 14.7 / 11), and with 256 tiles the vendor's larger ones fill the chip too ([2048,2048] 65 / 64 at
-    6400 rows, [11264,2048] 321 / 260)."""
-    (m, n), k = dy.shape, x.shape[-1]
+    """dy^T x of bf16 rows, on the library's kernel where that is the faster one."""
     if _mapped(dy, x):                                       # rows of several gradients: one product, no batched one
         return torch.matmul(dy.t().contiguous(), x)
-    if m >= 2560 and -(-n // 128) * -(-k // 128) < 256 and not torch.is_grad_enabled():
+    if _wgrad_on_kernel(*dy.shape, x.shape[-1]) and not torch.is_grad_enabled():
         dw = mvpa_hip.load_ext().linear_wgrad(dy, x)
         # rows that do not start at 16-byte boundaries or overlap are the vendor library's; any other status is an error
         if type(dw) is not int or dw not in (mvpa_hip.ERR_ALIGN, mvpa_hip.ERR_SHAPE, mvpa_hip.ERR_UNSUPPORTED):

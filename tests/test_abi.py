@@ -249,6 +249,18 @@ def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_bac
                 AG._weight_gradient(dy, x)
 
 
+@pytest.mark.parametrize("m,n,k,kernel", [
+    (2559, 768, 768, False), (2560, 768, 768, True), (1 << 20, 768, 768, True),     # rows, few tiles at any number of them
+    (6400, 2048, 1920, True), (6400, 2048, 2048, False),                            # 240 and 256 tiles
+    (65536, 3456, 768, True), (65535, 3072, 1024, True), (65536, 3072, 1024, False), (131072, 3456, 768, False),
+    (32768, 640, 4000, True), (65536, 640, 4000, False),                            # rows of 8000 bytes
+    (25600, 8, 12288, True), (25600, 8, 16000, False), (25600, 16000, 8, False), (25600, 64, 16000, True),
+])
+def test_which_weight_gradients_the_kernel_takes(m, n, k, kernel):
+    from mvpa_hip import autograd as AG
+    assert AG._wgrad_on_kernel(m, n, k) is kernel
+
+
 def test_weight_gradients_under_vmap_are_no_kernel_call(monkeypatch):
     """Gradients of several losses at once (is_grads_batched) come as tensors without memory of their own."""
     from mvpa_hip import autograd as AG
