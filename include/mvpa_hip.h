@@ -462,6 +462,7 @@ int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, int64_t M, i
  * (each nullable) from the gradient of out; w is not read there.  K a multiple of 8; w, a, out and d_out at
  * 16-byte boundaries.  Sums in fp32, one rounding. */
 #define MVPA_LORA_PARTS 8
+#define MVPA_LORA_ROWS (1 << 24)     /* the most rows of a part */
 typedef struct mvpa_lora_part {
   const void *w, *a, *b;
   void *da, *db;

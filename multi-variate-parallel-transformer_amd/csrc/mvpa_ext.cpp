@@ -740,6 +740,7 @@ PyObject* py_lora_fits(PyObject*, PyObject* mods) {
     if (w.size(1) % 8 || (K >= 0 && w.size(1) != K)) Py_RETURN_FALSE;
     K = w.size(1);
     if (is_none(PyTuple_GET_ITEM(mod, 2))) {
+      if (w.size(0) > MVPA_LORA_ROWS) Py_RETURN_FALSE;
       ++parts;
       continue;
     }
@@ -749,7 +750,7 @@ PyObject* py_lora_fits(PyObject*, PyObject* mods) {
     int64_t on = 0;
     for (int64_t i = 0; i < slices; ++i) on += PyTuple_GET_ITEM(enable, i) == Py_True;
     if (slices == 0 || on == 0 || w.size(0) % slices || a.size(1) != K || a.size(0) != on * b.size(1) ||
-        b.size(0) != w.size(0) / slices * on || (r >= 0 && b.size(1) != r))
+        b.size(0) != w.size(0) / slices * on || w.size(0) / slices > MVPA_LORA_ROWS || (r >= 0 && b.size(1) != r))
       Py_RETURN_FALSE;
     r = b.size(1);
     parts += slices;

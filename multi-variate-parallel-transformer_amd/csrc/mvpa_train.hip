@@ -267,11 +267,12 @@ __device__ inline void lora_b8(const bf16_t* row, int k0, int r, float (&v)[8]) 
   }
 }
 
-// a thread takes 8 columns of LORA_ROWS rows; blockIdx.z is the part.  VEC: r a multiple of 8
+// a thread takes 8 columns of LORA_ROWS rows (groups of them along x, whose grid takes any number of them); blockIdx.z is
+// the part.  VEC: r a multiple of 8
 template <bool VEC>
 __global__ __launch_bounds__(128) void lora_stack_kernel(lora_parts parts, bf16_t* __restrict__ out, int K, int r, float scale) {
   const mvpa_lora_part p = parts.p[blockIdx.z];
-  const int row0 = blockIdx.y * LORA_ROWS, c = (blockIdx.x * 128 + threadIdx.x) * 8;
+  const int row0 = blockIdx.x * LORA_ROWS, c = (blockIdx.y * 128 + threadIdx.x) * 8;
   if (row0 >= p.rows || c >= K) return;
   const bf16_t *w = (const bf16_t*)p.w, *a = (const bf16_t*)p.a, *b = (const bf16_t*)p.b;
   u32x4 wv[LORA_ROWS];               // requested first: the only operand that is not in a cache
@@ -488,7 +489,7 @@ static int lora_check(const mvpa_lora_part* parts, int32_t n, int32_t K, int32_t
   *most = 0;
   for (int i = 0; i < n; ++i) {
     mvpa_lora_part p = parts[i];
-    if (p.rows <= 0 || p.rows > (1 << 24)) return MVPA_ERR_SHAPE;
+    if (p.rows <= 0 || p.rows > MVPA_LORA_ROWS) return MVPA_ERR_SHAPE;
     if ((!backward && !p.w) || !p.a != !p.b) return MVPA_ERR_NULL;
     if ((((uintptr_t)p.a | (uintptr_t)p.b) & (r % 8 == 0 ? 15 : 1)) || ((uintptr_t)p.a & 15) || (!backward && ((uintptr_t)p.w & 15))) return MVPA_ERR_ALIGN;
     p.row0 = row0;
@@ -506,7 +507,7 @@ extern "C" int mvpa_lora_stack_bf16(const mvpa_lora_part* parts, int32_t n, int3
   const int st = lora_check(parts, n, K, r, out, false, args, &most);
   if (st != MVPA_OK) return st;
   MVPA_LAUNCH(r % 8 == 0 ? train::lora_stack_kernel<true> : train::lora_stack_kernel<false>,
-              dim3((unsigned)((K + 1023) / 1024), (unsigned)((most + train::LORA_ROWS - 1) / train::LORA_ROWS), (unsigned)n), dim3(128),
+              dim3((unsigned)((most + train::LORA_ROWS - 1) / train::LORA_ROWS), (unsigned)((K + 1023) / 1024), (unsigned)n), dim3(128),
               0, (hipStream_t)stream, args, (bf16_t*)out, K, r, scale);
   return take_launch_status();
 }

@@ -158,7 +158,8 @@ def _near(got, ref):
 # ranks around the eight that are summed together; columns around the 64 of a workgroup and the 1024 of a row's
 # threads; rows around the 8 and the 32 shares; a slice without an adapter, a module without any
 @pytest.mark.parametrize("r,cols,rows", [(1, 8, (1, 2)), (8, 768, (96, 64)), (9, 72, (33, 66)), (16, 1032, (8, 10)),
-                                         (20, 2048, (64, 4))])
+                                         (20, 2048, (64, 4)),
+                                         (8, 16, (262148, 64))])      # more row groups than a grid takes along y
 def test_stacked_weights_with_adapters(r, cols, rows):
     g = torch.Generator(device="cuda").manual_seed(r * cols)
 
