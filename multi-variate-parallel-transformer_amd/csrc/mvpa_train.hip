@@ -68,11 +68,11 @@ __device__ inline void put4(T* row, int c, int cols, const float (&v)[4]) {
 // y = x r w with r = rsqrt(mean(x^2) + eps):   dx = r w dy - x r^3 mean(x w dy) (+ res),   dw = sum_rows dy x r
 // A wave owns whole rows, a lane the same columns of each of them: the row is in registers between its
 // two sums and its result, and the lane's share of dw stays there over all rows.  HBM bound.  512 workgroups:
-// with one per four rows the partial sums of dw are as many bytes as a row operand.  The next row is requested
-// before the sums of this one, without a branch per chunk, behind which each load would be waited for by itself: with
-// the sums of dw 18.6 -> 13.8 us for 6400 rows of 768 in bf16, 144 -> 79 for 65536.  Wider rows do not fit the registers
-// twice (2560 in fp32: 69 -> 174 us) and are read as they come.
-template <typename TX, typename TW, int NCH, bool VEC>
+// with one per four rows the partial sums of dw are as many bytes as a row operand.  AHEAD: the wave's next row, where
+// there is one, is requested before the sums of this one, without a branch per chunk, behind which each load would be
+// waited for by itself: with the sums of dw 18.6 -> 13.8 us for 6400 rows of 768 in bf16, 144 -> 79 for 65536.  Where that
+// pays: launch_norm.
+template <typename TX, typename TW, int NCH, bool VEC, bool AHEAD>
 __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restrict__ x, const TW* __restrict__ w,
                                                                const bf16_t* __restrict__ dy, const TX* __restrict__ res,
                                                                TX* __restrict__ dx, float* __restrict__ part,
@@ -88,11 +88,10 @@ __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restr
   }
   const float rcols = 1.f / (float)cols;
   // chunks beyond the row read its last four columns and count as zero
-  constexpr bool AHEAD = VEC && NCH <= (sizeof(TX) == 2 ? 8 : 4);
+  static_assert(VEC || !AHEAD, "whole chunks");
   constexpr int NR = AHEAD ? NCH : 1;
-  decltype(raw4(x)) x_raw[NR], r_raw[NR];
+  decltype(raw4(x)) x_raw[NR], r_raw[NR] = {};
   u32x2 g_raw[NR];
-  const TX* res_or_x = res ? res : x;
   auto request = [&](int64_t row) {
     if constexpr (AHEAD) {
 #pragma unroll
@@ -100,8 +99,10 @@ __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restr
         const int64_t at = row * cols + min((i * 64 + lane) * 4, cols - 4);
         x_raw[i] = raw4(x + at);
         g_raw[i] = raw4(dy + at);
-        r_raw[i] = raw4(res_or_x + at);
       }
+      if (res)
+#pragma unroll
+        for (int i = 0; i < NCH; ++i) r_raw[i] = raw4(res + row * cols + min((i * 64 + lane) * 4, cols - 4));
     }
   };
   const int64_t first = (int64_t)blockIdx.x * 4 + wave, stride = (int64_t)gridDim.x * 4;
@@ -117,16 +118,14 @@ __global__ __launch_bounds__(256) void rmsnorm_backward_kernel(const TX* __restr
         widen(g_raw[i], gv[i]);
         widen(r_raw[i], add[i]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
+        for (int j = 0; j < 4; ++j)
           if (c >= cols) xv[i][j] = gv[i][j] = 0.f;
-          if (!res) add[i][j] = 0.f;
-        }
       } else {
         get4<VEC>(x + row * cols, c, cols, xv[i]);
         get4<VEC>(dy + row * cols, c, cols, gv[i]);
       }
     }
-    request(min(row + stride, rows - 1));
+    if (row + stride < rows) request(row + stride);
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
@@ -412,13 +411,20 @@ static void launch_norm(const void* x, const void* w, const void* dy, const void
     MVPA_LAUNCH(kern, dim3((unsigned)row_groups(rows)), dim3(256), 0, s, (const TX*)x, (const TW*)w, (const bf16_t*)dy,
                 (const TX*)res, (TX*)dx, part, rows, cols, eps);
   };
+  // The next row ahead: up to 1024 columns.  Up to 2048 in bf16 it takes the registers of a second row, and the waves of a
+  // launch whose operands the caches hold wait less for memory than for each other.  us, rows as they come / ahead, dx
+  // and dw, and with res: 1600 x 2048 13.3 / 19.6, 14.1 / 19.6; 6400 x 2048 28.9 / 33.6, 33.0 / 33.6; 16384 x 2048 50 / 57,
+  // 61 / 57; 30000 x 2048 119 / 97, 157 / 97; 30000 x 1280 60 / 74, 74 / 74; 65536 x 1280 163 / 170, 218 / 170; 30000 x 1536
+  // 87 / 86, 105 / 86.  In fp32, and wider, two rows do not fit the registers (2560 in fp32: 69 / 174).
+  const bool far = sizeof(TX) == 2 && rows * cols >= (res ? 40000000 : 45000000) && (res || cols > 1408);
   if (!vec) {
-    if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, false>);
-    else go(rmsnorm_backward_kernel<TX, TW, 16, false>);
-  } else if (cols <= 768) go(rmsnorm_backward_kernel<TX, TW, 3, true>);
-  else if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, true>);
-  else if (cols <= 2048) go(rmsnorm_backward_kernel<TX, TW, 8, true>);
-  else go(rmsnorm_backward_kernel<TX, TW, 16, true>);
+    if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, false, false>);
+    else go(rmsnorm_backward_kernel<TX, TW, 16, false, false>);
+  } else if (cols <= 768) go(rmsnorm_backward_kernel<TX, TW, 3, true, true>);
+  else if (cols <= 1024) go(rmsnorm_backward_kernel<TX, TW, 4, true, true>);
+  else if (cols <= 2048 && far) go(rmsnorm_backward_kernel<TX, TW, 8, true, sizeof(TX) == 2>);
+  else if (cols <= 2048) go(rmsnorm_backward_kernel<TX, TW, 8, true, false>);
+  else go(rmsnorm_backward_kernel<TX, TW, 16, true, false>);
 }
 
 }  // namespace train

@@ -49,6 +49,13 @@ def test_norm_backward(cols, rows, xt, wt, res):
     assert none is None and torch.equal(only_w, dw)
 
 
+@pytest.mark.parametrize("cols,rows,res", [(1156, 34602, True), (1156, 34603, True), (2048, 21973, False), (1408, 31961, False),
+                                           (1412, 31870, False)])
+def test_norm_backward_of_many_rows(cols, rows, res):
+    """Either side of the lines from which rows of more than 1024 columns are requested one ahead."""
+    test_norm_backward(cols, rows, torch.bfloat16, torch.float32, res)
+
+
 @pytest.mark.parametrize("rows,n", [(1, 8), (3, 2040), (4, 2048), (5, 2056), (33, 344), (130, 5632)])
 def test_silu_gate(rows, n):
     g = torch.Generator(device="cuda").manual_seed(rows * n)
