@@ -145,13 +145,16 @@ __device__ inline bool tile_coords(int id, int ct, int mt, int& col, int& row) {
   return col < ct;
 }
 
-// What a row tile of WM * 32 rows does: the last one of many where few rows are left takes a smaller one, in
-// whose blocks x is less (525 rows: 13 of them are left to a fifth tile of 128)
+// What a row tile of WM * 32 rows does: the last one of `mt` where few rows are left takes a smaller one, in whose blocks x
+// is less (525 rows: 13 of them are left to a fifth tile of 128).  33 .. 64 rows from five tiles on: with fewer, all tiles run
+// at about the same time and the smaller one, which splits the contraction over its waves, is the last to end (windows of
+// MVPFormer-S, as a tile of 128 / of 64, us: 192 rows 442 / 451, 320 359 / 367; 8 blocks of the base model: 448 rows 882 /
+// 907, 576 1136 / 1119, 704 1233 / 1204).
 template <int WM, int STAGES, typename F>
-__device__ __forceinline__ void for_rows_left(int64_t rows, F f) {
+__device__ __forceinline__ void for_rows_left(int64_t rows, int mt, F f) {
   if constexpr (WM == 4 && STAGES == 3) {
     if (rows <= 32) f(std::integral_constant<int, 1>(), std::integral_constant<int, 6>());
-    else if (rows <= 64) f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
+    else if (rows <= 64 && mt > 4) f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
     else f(std::integral_constant<int, 4>(), std::integral_constant<int, 3>());
     static_assert(tile_cfg<1, 6>::LDS <= tile_cfg<4, 3>::LDS && tile_cfg<2, 4>::LDS <= tile_cfg<4, 3>::LDS, "LDS of the launch");
   } else {
@@ -240,7 +243,7 @@ __global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict
   int col, row;
   if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
   const int64_t m0 = (int64_t)row * 32 * WM;
-  for_rows_left<WM, STAGES>(M - m0, [&](auto wm, auto stages) {
+  for_rows_left<WM, STAGES>(M - m0, mt, [&](auto wm, auto stages) {
     tile_dual<wm(), stages()>(tl_lds, X, M, K, ldx, W0, N0, ldw0, out, gt, nrm, gated_ct, col, m0);
   });
 }
@@ -248,18 +251,29 @@ __global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict
 template <int WM, int STAGES>
 __global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
                                                            const bf16_t* __restrict__ W, int N, int64_t ldw,
-                                                           float* __restrict__ P, tile_split sp, int ct, int mt) {
+                                                           float* __restrict__ P, tile_split sp, int ct, int mt, bool spread) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
   // an XCD (ids equal mod 8) takes neighbours of one part, row tiles fastest: it reads that part's columns of x, not
-  // all of them, and its panel of w once
-  const int total = ct * (sp.a + sp.b) * mt, per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-  if (id >= total) return;
-  const int cz = id / mt, row = id - cz * mt, z = cz / ct, col = cz - z * ct;
+  // all of them, and its panel of w once.  spread: parts of a column side by side, dealt over the XCDs
+  const int splits = sp.a + sp.b, total = ct * splits * mt, per = (total + 7) / 8;
+  int row, z, col;
+  if (spread) {
+    int cz;
+    if (!tile_coords(blockIdx.x, ct * splits, mt, cz, row)) return;
+    col = cz / splits;
+    z = cz - col * splits;
+  } else {
+    const int id = (blockIdx.x & 7) * per + (blockIdx.x >> 3), cz = id / mt;
+    if (id >= total) return;
+    row = id - cz * mt;
+    z = cz / ct;
+    col = cz - z * ct;
+  }
   const int kb0 = z < sp.a ? z * sp.per_a : sp.nkb_a + (z - sp.a) * sp.per_b;
   const int kb1 = z < sp.a ? min(kb0 + sp.per_a, sp.nkb_a) : min(kb0 + sp.per_b, K / TL_BK);
   const int64_t m0 = (int64_t)row * 32 * WM;
   const int n0 = col * TL_BN, c = threadIdx.x & 15, n = n0 + c * 4;
-  for_rows_left<WM, STAGES>(M - m0, [&](auto wm, auto stages) {
+  for_rows_left<WM, STAGES>(M - m0, mt, [&](auto wm, auto stages) {
     using G = tile_cfg<wm(), stages()>;
     tile_product<wm(), stages()>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0, kb1);
 #pragma unroll
@@ -385,8 +399,12 @@ static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, 
   auto kern = tile_partial_kernel<WM, STAGES>;
   want_dynamic_lds((const void*)kern, G::LDS);
   const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
-  MVPA_LAUNCH(kern, dim3((unsigned)((ct * sp.total() * mt + 7) / 8 * 8)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w,
-              (int)N, ldw, P, sp, ct, mt);
+  // A part's columns of x to an XCD, but for three row tiles and more of an x that the L2 of each (4 MB) holds as a whole.
+  // Windows of MVPFormer-S (2816 columns), part to an XCD / spread, us: 130 rows 418 / 427, 270 354 / 360, 320 362 / 359, 448
+  // 390 / 380, 512 405 / 391, 525 443 / 447; eight blocks of the base model (7680), 406 rows 859 / 871, 448 887 / 899.
+  const bool spread = mt > 2 && M * K * 2 <= (4 << 20);
+  const int ids = spread ? (ct * sp.total() + 7) / 8 * 8 * mt : (ct * sp.total() * mt + 7) / 8 * 8;
+  MVPA_LAUNCH(kern, dim3((unsigned)ids), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, P, sp, ct, mt, spread);
   return take_launch_status();
 }
 

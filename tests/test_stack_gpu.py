@@ -74,7 +74,9 @@ def test_windows_of_many_rows(flash, B, C, T):
     assert _rel(got, want) <= REL
 
 
-@pytest.mark.parametrize("B,C,T", [(5, 32, 1), (7, 23, 1), (3, 32, 2), (193, 1, 1), (41, 64, 1)], ids=str)    # 32, 33, 64 and 65 left
+@pytest.mark.parametrize("B,C,T", [(5, 32, 1), (7, 23, 1), (3, 32, 2), (193, 1, 1), (41, 64, 1),               # 32, 33, 64 and 65 left
+                                   (1, 64, 7), (9, 61, 1), (1, 96, 6),              # 64 to a fourth tile, 37 and 64 to a fifth
+                                   (65, 56, 1), (331, 11, 1)], ids=str)             # x of the last product up to and over 4 MB
 def test_rows_left_to_a_last_tile(B, C, T):
     """The last of several row tiles by how many rows are left to it, against the stack in 64 bits."""
     model = _model(n_inner=448)
