@@ -721,10 +721,10 @@ bool lora_parts(PyObject* mods, bool backward, LoraParts& l) {
   return l.parts.size() <= MVPA_LORA_PARTS && l.r > 0;
 }
 
-// lora_fits(mods): whether lora_stack takes them
+// lora_fits(mods): whether lora_stack takes them and is the faster way
 PyObject* py_lora_fits(PyObject*, PyObject* mods) {
   HANDLE_TH_ERRORS
-  int64_t K = -1, r = -1, parts = 0;
+  int64_t K = -1, r = -1, parts = 0, most = 0;
   auto bad = [&](PyObject* o) {
     if (!THPVariable_Check(o)) return true;
     const Tensor& t = THPVariable_Unpack(o);
@@ -750,12 +750,17 @@ PyObject* py_lora_fits(PyObject*, PyObject* mods) {
     int64_t on = 0;
     for (int64_t i = 0; i < slices; ++i) on += PyTuple_GET_ITEM(enable, i) == Py_True;
     if (slices == 0 || on == 0 || w.size(0) % slices || a.size(1) != K || a.size(0) != on * b.size(1) ||
-        b.size(0) != w.size(0) / slices * on || w.size(0) / slices > MVPA_LORA_ROWS || (r >= 0 && b.size(1) != r))
+        b.size(0) != w.size(0) / slices * on || (r >= 0 && b.size(1) != r))
       Py_RETURN_FALSE;
     r = b.size(1);
     parts += slices;
+    most = std::max(most, w.size(0) / slices);
   }
-  if (r > 0 && parts <= MVPA_LORA_PARTS) Py_RETURN_TRUE;
+  // The kernel walks all rows of a part for every eight of its r terms, 64 columns a workgroup: beyond this tensor
+  // operations are faster.  Both ways on the GPU, us, kernels / tensor operations, q and two slices of kv rows: 2048 +
+  // 2 x 1024 rows of 2048 r 64 203 / 281, r 96 293 / 281; 4096 + 2 x 1024 of 4096 r 32 259 / 403, r 48 381 / 436, r 64
+  // 506 / 434; 1024 + 2 x 512 of 1024 r 128 160 / 205; 768 + 2 x 256 of 768 r 8 18 / 164.
+  if (r > 0 && parts <= MVPA_LORA_PARTS && r * most <= 160 * 1024) Py_RETURN_TRUE;
   Py_RETURN_FALSE;
   END_HANDLE_TH_ERRORS
 }

@@ -178,7 +178,10 @@ def test_stacked_weights_with_adapters(r, cols, rows):
             ((True, False, True), rn(6, cols), rn(2 * r, cols), rn(4, r))]
     d = torch.randn((sum(m[1].shape[0] for m in mods), cols), generator=g, device="cuda").bfloat16()
     leaves = [t for m in mods for t in m[1:] if t is not None]
-    w = AG.lora_stack(tuple(mods), scale)
+    if rows[0] > 4 * 65535:                              # more than lora_stack hands to the kernel
+        w = AG._LoRAStackFn.apply(scale, tuple(m[0] for m in mods), *(t for m in mods for t in m[1:]))
+    else:
+        w = AG.lora_stack(tuple(mods), scale)
     grads = torch.autograd.grad(w, leaves, d)
     ref = []
     for on, wm, a, b in mods:
@@ -207,6 +210,17 @@ def test_stacked_weights_that_the_kernel_refuses():
     assert torch.equal(w, torch.cat([mod.effective_weight(), plain.weight], 0))
     w.sum().backward()
     assert mod.lora_B.grad.abs().sum() > 0
+
+
+@pytest.mark.parametrize("rows,kernel", [(1280, True), (1281, False)])
+def test_stacked_weights_of_large_rank(rows, kernel):
+    """Rank times rows of the largest part up to 160 * 1024 on the kernel."""
+    from layers.mvpa import _LoRALinear, _stacked_weights
+    mod = _LoRALinear(16, 2 * rows, 128, 4, enable=(False, True)).to("cuda", torch.bfloat16)
+    with torch.no_grad():
+        mod.lora_B.normal_()
+    assert (AG.lora_stack(((mod.enable, mod.weight, mod.lora_A, mod.lora_B),), mod.scaling) is None) is not kernel
+    _near(_stacked_weights((mod,)).detach(), mod.effective_weight().detach())
 
 
 def test_stacked_weights_by_a_list_of_slices():
