@@ -262,7 +262,9 @@ int mvpa_backward(const mvpa_bwd_args* args, void* stream);
  * 128, C <= 128, causal, no key bias; MVPA_ERR_UNSUPPORTED otherwise).  Of `args` the input fields are read
  * (through lse); its gradient and workspace fields are taken from `ws`
  * (mvpa_backward_full_ws_bytes(args), 256-byte aligned).  dq, dk, dv at element strides that are multiples
- * of 8; the rest contiguous. */
+ * of 8; the rest contiguous.  dk and dv may lie over the inputs.  The workspace depends on the launches that the
+ * shape takes, not on its size alone: with H > Hkv and few key workgroups it holds fp32 dk and dv per query head, H / Hkv
+ * times as much. */
 typedef struct mvpa_bwd_grads {
   uint32_t struct_size;      /* = sizeof(mvpa_bwd_grads)                                      */
   uint32_t reserved0;

@@ -53,7 +53,7 @@ __device__ inline void lds_barrier() {
 
 // direct-to-LDS loads: lane L's 16 (4) bytes land at lds_base + 16 L (4 L).  Inline assembly so
 // that the compiler does not drain the ring in front of later LDS reads; completion is awaited
-// with wait_vmcnt() before the barrier that publishes a stage.
+// with wait_vmcnt_imm before the barrier that publishes a stage.
 __device__ inline void dma16(const void* gptr, uint32_t lds_base) {
   lds_base = __builtin_amdgcn_readfirstlane(lds_base);    // uniform by construction; pins it to an SGPR
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
@@ -68,19 +68,6 @@ __device__ inline void dma4(const void* gptr, uint32_t lds_base) {
 template <int N>
 __device__ inline void wait_vmcnt_imm() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// wait until at most n (0..6) of this wave's vector-memory operations are outstanding
-__device__ inline void wait_vmcnt(int n) {
-  switch (n) {
-    case 0: wait_vmcnt_imm<0>(); break;
-    case 1: wait_vmcnt_imm<1>(); break;
-    case 2: wait_vmcnt_imm<2>(); break;
-    case 3: wait_vmcnt_imm<3>(); break;
-    case 4: wait_vmcnt_imm<4>(); break;
-    case 5: wait_vmcnt_imm<5>(); break;
-    default: wait_vmcnt_imm<6>(); break;
-  }
 }
 
 __device__ inline bf16x8 as_frag(u32x4 v) {
@@ -866,8 +853,8 @@ static void launch_query(const mvpa_bwd_args* a, hipStream_t stream, int q0, int
 }
 
 // ==========================================================================================
-// The KEY pass: dk, dv.  A workgroup owns 4 consecutive key time steps of one kv head; a
-// wave owns 32 key channels of one of them (its K and V rows stay in registers as MFMA B
+// The KEY pass: dk, dv.  A workgroup of 4 waves owns consecutive key time steps of one kv head, 2 with two
+// channel tiles and 4 with one; a wave owns 32 key channels of one of them (its K and V rows stay in registers as MFMA B
 // operands) and walks every query time step tq >= tk of every query head of the group, both
 // query-channel tiles in turn.  Products are formed NON-transposed here, S[q][key] = (q+u) K^T,
 // so that a lane owns one key and the contraction index of dv^T = dO^T P and dk^T = (q+u)^T dS
@@ -1491,9 +1478,10 @@ static void launch_key(const mvpa_bwd_args* a, const mvpa_kv_out& out, hipStream
 // gradients) and of disjoint query channels (to dk, dv) simply add up, so every (query part, key
 // part) pair is one query-pass launch followed by the key-pass launch that consumes its
 // workspace; later launches add to what earlier ones wrote (one stream, hence ordered).
-// At Dh 128 a key-pass stage of 64 channels does not fit the LDS three times: the key pass then
-// takes the (query part, key part) pair of a query-pass launch in quarters of 32 x 32 channels
-// (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).
+// At Dh 128 the key pass takes the (query part, key part) pair of a query-pass launch in quarters of 32 x 32
+// channels (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).  That
+// was forced while a stage held two copies of each tile; with one, two channel tiles would fit as well (two stages 99 840
+// bytes, 195 .. 215 + 160 registers against 175 .. 181 + 160), which has not been measured.
 // far steps of the longest walk from which the two phases of the query pass are a launch each (Dh 128): the
 // set-up of a workgroup is paid twice.  Forward and backward, one launch / two, H16/8: B2 C128 T128 8.39 / 8.82 ms, B1
 // C128 T200 9.01 / 9.10, B2 C64 T256 6.40 / 6.37, B1 C128 T300 17.1 / 17.0, T 512 36.4 / 35.8.
@@ -1504,7 +1492,7 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
   const int C = a->C, T = a->T;
   constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
   // Far query steps (outside the content window and not the last step) in a kernel of their own where its
-  // workgroups, of four times as many key steps, still fill the chip.  Forward and backward, far kernel / without:
+  // workgroups, of FAR_KT key steps (16 at Dh 64, 8 at Dh 128; 2 and 4 in the key pass), still fill the chip.  Forward and backward, far kernel / without:
   // Dh 64, C 64, T 128: 384 workgroups 1327 / 1495 us, 256: 962 / 1022, 192: 793 / 850, 128: 667 / 589; T 256 of 256:
   // 1480 / 1648; T 64, C 40 of 192: 495 / 495; T 64 of 48: 315 / 272;
   // Dh 128, H16/8: B1 C64 T128, 256 workgroups, 1259 / 1453; C 128: T 128, 128 workgroups 5.77 / 6.15 ms.

@@ -17,7 +17,9 @@
 //                     operands by transposing LDS reads), column sums of G; fp32 partial results
 //   finish_reduce   the partial results to dk_time, dk_chan; finish_biases: du, dv, dz
 // Columns of G_time that the causal mask empties (j < T-1-tq) are skipped.  HBM bound: at that size, G being
-// 400 MB of which 270 are read, 148 us in one read (3.6 TB/s with dq and q) and 187 + 189 in two; dk and dv 60.
+// 400 MB of which 270 are read, 148 us in one read (3.6 TB/s with dq and q) and 187 + 189 in two.  dk and dv come rounded from
+// the key pass; finish_kv rounds and adds them (60 us at that size) where each query head has parts of its own or
+// the results lie over what the passes read.
 #include "mvpa_mfma_tools.h"
 
 namespace mvpa {
