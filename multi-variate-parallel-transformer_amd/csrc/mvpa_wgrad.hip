@@ -8,8 +8,8 @@
 // LDS reads.  A group is 4 waves of 64 x 64 outputs (64 accumulator registers) on two 32 KiB stages, so that
 // two share a CU.  Per block of 64 rows one barrier, in front of its last quarter: that quarter's fragments
 // are in registers, the barrier publishes the next block and frees this one's stage for the block after next.
-// Bound by the fragment reads (one per product) and the tile requests: 960 TFLOP/s on [4096,2048] over 6400 rows, 710
-// on [3456,768] with its partial tiles (13 of 48 us).
+// Bound by the fragment reads (one per product) and the tile requests: 44 us for [3456,768] over 6400 rows, 780 TFLOP/s, 55
+// with the partial tiles added up.
 #include "mvpa_mfma_tools.h"
 
 namespace mvpa {
@@ -187,8 +187,9 @@ __global__ __launch_bounds__(256) void linear_wgrad_reduce_kernel(const float* _
 static int tiles_of(int64_t N, int64_t K) { return (int)((N + TILE - 1) / TILE * ((K + TILE - 1) / TILE)); }
 
 // How the rows are dealt, by what a launch was seen to take: a group of 4 waves 1.27 us a block where two share a
-// CU, partial results 2 x 4 bytes an output and share at 4.8 TB/s.  6400 rows, us (vendor library): [3456,768]
-// 52 (65), [768,1728] 34 -> 28 with pairs of groups (50), [1280,768] 28 -> 22 (42), [768,768] 24 -> 16 (39).
+// CU, partial results 2 x 4 bytes an output and share at 4.8 TB/s.  Both launches over 6400 rows, eight sets of them in
+// turn, us (vendor library): [3456,768] 55 (69), [768,1728] 36 (50), [1280,768] 27 (41), [768,768] 22 (39).  Pairs of groups
+// took 6 to 8 us off the last three.
 struct plan {
   int groups, splits;
 };

@@ -26,18 +26,25 @@ def _mapped(*tensors) -> bool:
 
 
 def _wgrad_on_kernel(m, n, k) -> bool:
-    """Whether the kernel of csrc/mvpa_wgrad.hip (both launches) is the faster one for dY^T X of [m, n] and [m, k],
-    us against the vendor library.  From 2560 rows: [768,768] 19 / 23, 6400 rows 23 / 46, 131072 241 / 588; [3456,768]
-    31 / 37, 51 / 70.  Below it the second launch costs more than is gained (2048 rows of [768,768] 16.5 / 16, 1024
-    14.7 / 11).  With 256 tiles of 128 x 128 the vendor's larger ones fill the chip too ([2048,2048] 65 / 64 at 6400 rows,
-    [11264,2048] 321 / 260), and so they do where many tiles meet many rows (in millions of rows times tiles:
-    [3456,768] 10.6 415 / 544, [3072,1024] 6.3 310 / 308, 12.6 588 / 452, [1536,2048] 25 1252 / 1029), earlier where rows
-    do not start at lines of 128 bytes ([640,4000] 5.2 211 / 318, 10.5 622 / 427).  Fewer than 64 tiles gain at any
-    number of rows.  Long thin outputs are padding for the most part (25600 rows of [8,16000] 169 / 154; [8,8192] of 65536 221 / 265)."""
+    """Whether the kernel of csrc/mvpa_wgrad.hip is the faster one for dY^T X of [m, n] and [m, k], by the tiles of 128 x 128
+    in its output.  us, both launches of it / the vendor library, eight sets of rows in turn:
+        25 tiles  [640,640]    2560 rows 16 / 19, 6400 21 / 39, 25600 42 / 147
+        36        [768,768]    2816 21 / 20, 3072 20 / 22, 6400 22 / 39, 25600 49 / 155
+        60        [1280,768]   2560 23 / 19, 3072 23 / 22, 3584 23 / 25, 6400 27 / 41, 25600 68 / 163
+        84        [768,1728]   2560 21 / 23, 6400 36 / 50, 25600 104 / 285
+        162       [3456,768]   2560 30 / 30, 6400 55 / 69, 25600 181 / 279
+        169       [1664,1664]  5120 59 / 56, 6400 55 / 72
+        180       [2560,1152]  2560 30 / 30, 6400 79 / 70, 16384 171 / 146
+        225       [1920,1920]  2560 34 / 32, 6400 80 / 73, 25600 314 / 258
+    Fewer rows do not pay for the second launch, and with more tiles the vendor's larger ones fill the chip too.  So they do
+    where many tiles meet many rows (the same rows again, in millions of rows times tiles: [3456,768] 10.6 415 / 544,
+    [1536,2048] 25 1252 / 1029), earlier where rows do not start at lines of 128 bytes ([640,4000] 5.2 211 / 318, 10.5 622 /
+    427).  Long thin outputs are padding for the most part (25600 rows of [8,16000] 169 / 154)."""
     tiles = -(-n // 128) * -(-k // 128)
-    if m < 2560 or tiles >= 256 or (min(n, k) < 64 and tiles > 96):
+    if tiles > 170 or (min(n, k) < 64 and tiles > 96):
         return False
-    return tiles < 64 or m * tiles < (12 << 20 if n % 64 == 0 and k % 64 == 0 else 8 << 20)
+    least = 2560 if tiles <= 30 else 3072 if tiles <= 50 else 3584 if tiles <= 64 else 2560 if tiles <= 162 else 6400
+    return m >= least and (tiles < 64 or m * tiles < (12 << 20 if n % 64 == 0 and k % 64 == 0 else 8 << 20))
 
 
 def _weight_gradient(dy, x):

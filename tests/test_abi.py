@@ -250,9 +250,10 @@ def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_bac
 
 
 @pytest.mark.parametrize("m,n,k,kernel", [
-    (2559, 768, 768, False), (2560, 768, 768, True), (1 << 20, 768, 768, True),     # rows, few tiles at any number of them
-    (6400, 2048, 1920, True), (6400, 2048, 2048, False),                            # 240 and 256 tiles
-    (65536, 3456, 768, True), (65535, 3072, 1024, True), (65536, 3072, 1024, False), (131072, 3456, 768, False),
+    (2559, 640, 640, False), (2560, 640, 640, True), (3071, 768, 768, False), (3072, 768, 768, True),      # rows by tiles
+    (3583, 1280, 768, False), (3584, 1280, 768, True), (2559, 768, 1728, False), (2560, 768, 1728, True),
+    (6399, 1664, 1664, False), (6400, 1664, 1664, True), (6400, 2048, 1408, False),                          # 169, 176
+    (1 << 20, 768, 768, True), (65536, 3456, 768, True), (131072, 3456, 768, False),                        # few tiles, many
     (32768, 640, 4000, True), (65536, 640, 4000, False),                            # rows of 8000 bytes
     (25600, 8, 12288, True), (25600, 8, 16000, False), (25600, 16000, 8, False), (25600, 64, 16000, True),
 ])
