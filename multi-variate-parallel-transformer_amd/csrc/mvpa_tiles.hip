@@ -399,10 +399,11 @@ static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, 
   auto kern = tile_partial_kernel<WM, STAGES>;
   want_dynamic_lds((const void*)kern, G::LDS);
   const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
-  // A part's columns of x to an XCD, but for three row tiles and more of an x that the L2 of each (4 MB) holds as a whole.
-  // Windows of MVPFormer-S (2816 columns), part to an XCD / spread, us: 130 rows 418 / 427, 270 354 / 360, 320 362 / 359, 448
-  // 390 / 380, 512 405 / 391, 525 443 / 447; eight blocks of the base model (7680), 406 rows 859 / 871, 448 887 / 899.
-  const bool spread = mt > 2 && M * K * 2 <= (4 << 20);
+  // A part's columns of x to an XCD, but for four row tiles of an x that the L2 of each (4 MB) holds as a whole.  Windows of
+  // MVPFormer-S (2496 columns), part to an XCD / spread, us: 130 rows 418 / 427, 256 356 / 357, 288 362 / 367, 384 369 / 366,
+  // 406 383 / 380, 448 390 / 380, 512 405 / 391, 525 443 / 447; eight blocks of the base model (7680), 406 rows 859 / 871, 448
+  // 887 / 899.
+  const bool spread = mt == 4 && M * K * 2 <= (4 << 20);
   const int ids = spread ? (ct * sp.total() + 7) / 8 * 8 * mt : (ct * sp.total() * mt + 7) / 8 * 8;
   MVPA_LAUNCH(kern, dim3((unsigned)ids), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, P, sp, ct, mt, spread);
   return take_launch_status();

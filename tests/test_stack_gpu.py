@@ -75,12 +75,22 @@ def test_windows_of_many_rows(flash, B, C, T):
 
 
 @pytest.mark.parametrize("B,C,T", [(5, 32, 1), (7, 23, 1), (3, 32, 2), (193, 1, 1), (41, 64, 1),               # 32, 33, 64 and 65 left
-                                   (1, 64, 7), (9, 61, 1), (1, 96, 6),              # 64 to a fourth tile, 37 and 64 to a fifth
-                                   (65, 56, 1), (331, 11, 1)], ids=str)             # x of the last product up to and over 4 MB
+                                   (1, 64, 7), (9, 61, 1), (1, 96, 6)], ids=str)    # 64 to a fourth tile, 37 and 64 to a fifth
 def test_rows_left_to_a_last_tile(B, C, T):
     """The last of several row tiles by how many rows are left to it, against the stack in 64 bits."""
     model = _model(n_inner=448)
     x = torch.randn(B, T, C, 128, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = model(inputs_embeds=x)
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=2, n_head_kv=1), None)
+    assert _rel(got, want) <= REL
+
+
+@pytest.mark.parametrize("C,T,inner", [(125, 4, 4032), (128, 4, 4032), (96, 4, 448), (77, 5, 448), (103, 5, 448)])
+def test_parts_of_the_tail_product_by_xcd(C, T, inner):
+    """Four row tiles with x of the tail product up to and over 4 MB; three, four and five row tiles."""
+    model = _model(n_inner=inner)
+    x = torch.randn(1, T, C, 128, device="cuda").bfloat16()
     with torch.no_grad():
         got = model(inputs_embeds=x)
     want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=2, n_head_kv=1), None)
