@@ -288,8 +288,9 @@ __global__ __launch_bounds__(128) void lora_stack_kernel(lora_parts parts, bf16_
     for (int i = 0; i < LORA_ROWS; ++i) lora_b8<VEC>(b + (int64_t)min(row0 + i, p.rows - 1) * r, k0, r, bv[i]);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
+      if (!VEC && k0 + k >= r) break;            // no zero times a row of a, which may be infinite
       float av[8];
-      load8(a + (int64_t)min(k0 + k, r - 1) * K + c, av);
+      load8(a + (int64_t)(k0 + k) * K + c, av);
 #pragma unroll
       for (int i = 0; i < LORA_ROWS; ++i)
 #pragma unroll

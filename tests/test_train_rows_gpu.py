@@ -212,6 +212,19 @@ def test_stacked_weights_that_the_kernel_refuses():
     assert mod.lora_B.grad.abs().sum() > 0
 
 
+@pytest.mark.parametrize("r", [1, 8, 13])
+def test_stacked_weights_with_infinite_adapters(r):
+    """An infinity in the last row of a stays one: nothing past the rank is multiplied with it."""
+    w, a, b = torch.zeros(6, 16), torch.zeros(r, 16), torch.ones(6, r)
+    a[-1, 3], a[0, 5] = float("inf"), -float("inf")
+    b[1] = -1
+    got = AG.lora_stack((((True,), *(t.cuda().bfloat16() for t in (w, a, b))),), 0.5).float().cpu()
+    want = torch.zeros(6, 16)
+    for c, sign in ((3, 1), (5, -1)):
+        want[:, c] = sign * b[:, 0] * float("inf")
+    assert torch.equal(got, want)
+
+
 @pytest.mark.parametrize("rows,kernel", [(1280, True), (1281, False)])
 def test_stacked_weights_of_large_rank(rows, kernel):
     """Rank times rows of the largest part up to 160 * 1024 on the kernel."""
