@@ -282,6 +282,7 @@ PyObject* py_linear_wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
   TORCH_CHECK(dy.dim() == 2 && x.dim() == 2 && dy.size(0) == x.size(0) && dy.scalar_type() == at::kBFloat16 &&
                   x.scalar_type() == at::kBFloat16,
               "linear_wgrad: bf16 rows");
+  TORCH_CHECK(dy.device() == x.device(), "linear_wgrad: dy and x on one GPU");
   const int64_t M = dy.size(0), N = dy.size(1), K = x.size(1);
   if (dy.stride(1) != 1 || x.stride(1) != 1 || M == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
   at::AutoDispatchBelowADInplaceOrView guard;
@@ -683,7 +684,11 @@ struct LoraParts {
 };
 bool lora_parts(PyObject* mods, bool backward, LoraParts& l) {
   TORCH_CHECK(lora_modules(mods), "lora_stack: (enable, w, a, b) per module");
-  auto held = [&](const Tensor& t) -> Tensor { return l.keep.emplace_back(aligned_operand(t, at::kBFloat16)); };
+  auto held = [&](const Tensor& t) -> Tensor {
+    l.keep.emplace_back(aligned_operand(t, at::kBFloat16));
+    TORCH_CHECK(l.keep.back().device() == l.keep.front().device(), "lora_stack: operands on one GPU");
+    return l.keep.back();
+  };
   for (Py_ssize_t m = 0; m < PyTuple_GET_SIZE(mods); ++m) {
     PyObject* mod = PyTuple_GET_ITEM(mods, m);
     PyObject* enable = PyTuple_GET_ITEM(mod, 0);
@@ -725,10 +730,12 @@ bool lora_parts(PyObject* mods, bool backward, LoraParts& l) {
 PyObject* py_lora_fits(PyObject*, PyObject* mods) {
   HANDLE_TH_ERRORS
   int64_t K = -1, r = -1, parts = 0, most = 0;
+  const Tensor* first = nullptr;
   auto bad = [&](PyObject* o) {
     if (!THPVariable_Check(o)) return true;
     const Tensor& t = THPVariable_Unpack(o);
-    return !t.is_cuda() || t.scalar_type() != at::kBFloat16 || t.dim() != 2 || !t.is_contiguous() || t.numel() == 0 ||
+    if (!first) first = &t;
+    return !t.is_cuda() || t.device() != first->device() || t.scalar_type() != at::kBFloat16 || t.dim() != 2 || !t.is_contiguous() || t.numel() == 0 ||
            ((uintptr_t)t.const_data_ptr() & 15);
   };
   if (!lora_modules(mods)) Py_RETURN_FALSE;
@@ -784,6 +791,7 @@ PyObject* py_lora_stack(PyObject*, PyObject* const* args, Py_ssize_t n) {
   }
   const Tensor d = aligned_operand(tensor_of(args[2]), at::kBFloat16);
   TORCH_CHECK(d.dim() == 2 && d.size(0) == l.rows && d.size(1) == l.K, "lora_stack: the gradient's shape differs");
+  TORCH_CHECK(l.keep.empty() || d.device() == l.keep.front().device(), "lora_stack: operands on one GPU");
   const Py_ssize_t mods = PyTuple_GET_SIZE(args[0]);
   std::vector<Tensor> grads(2 * mods);
   size_t at = 0;

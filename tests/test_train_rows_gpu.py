@@ -336,3 +336,17 @@ def test_gradients_of_several_losses_at_once():
     for i in range(3):
         for whole, one in zip(got, torch.autograd.grad(y, leaves, d[i], retain_graph=True)):
             _near(whole[i], one)
+
+
+@pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two GPUs")
+def test_operands_on_two_gpus_are_refused():
+    """As tensor operations refuse them: no kernel reads another GPU's memory."""
+    here, there = (torch.ones(16, 16, dtype=torch.bfloat16, device=f"cuda:{i}") for i in range(2))
+    for mods in (((True,), here, there, here),), (((True,), here, here, here), ((), there, None, None)):
+        assert AG.lora_stack(mods, 1.0) is None
+        with pytest.raises(RuntimeError):
+            mvpa_hip.lora_stack(mods, 1.0)
+    with pytest.raises(RuntimeError):
+        mvpa_hip.lora_stack((((True,), here, here, here),), 1.0, there)
+    with pytest.raises(RuntimeError):
+        mvpa_hip.load_ext().linear_wgrad(here, there)
