@@ -116,14 +116,21 @@ extern "C" int mvpa_forward(const mvpa_fwd_args* a, void* stream) {
     if (a->kernel == MVPA_KERNEL_MFMA_SPLIT) return mvpa_launch_mfma128(a, st);
     if (a->kernel == MVPA_KERNEL_MFMA) return mvpa_launch_mfma(a, st);
     // AUTO: the specialised builds where they are the faster ones.
-    // Launches that leave the chip idle: the build whose waves split the keys of a query tile, up to two
-    // workgroups per CU, and further with one query tile per step, where the other kernel's time is one
-    // chain over the steps whatever the batch (us, general -> this: H12 C21 T25 24 -> 13 at B1, 24.5 -> 20
-    // at B2, 25 -> 35 at B4; C21 T50 35 -> 23; C32 T64 54 -> 28; C21 T110 84 -> 58; C64 T12 17.5 -> 13,
-    // C64 T25 24.4 -> 25; H4 C8 T32 Dh32 22 -> 8; H16 Dh128 C21 T25 35 -> 25).
+    // Launches that leave the chip idle: the build whose waves split the keys of a query tile.  Its time follows the
+    // number of its workgroups (B H T and the query tiles of a step), the other kernels' is one chain over the steps
+    // until they fill the chip, so the line lies where the two meet (us, general : this).  Up to 32 channels,
+    // T 25 by B H 12 / 24 / 48 / 64: 23.5 : 10.0, 23.7 : 12.8, 24.1 : 21.6, 24.2 : 26.9; T 32 at 48 / 64 27.9 : 24.0, 28.1 :
+    // 32.2; T 64 at 24 / 48 51.5 : 33.1, 51.8 : 58.1; T 110 at 16 / 24 81.6 : 67.9, 82.4 : 97.9; T 200 at 12 / 16 149 : 124,
+    // 150 : 165.  33..64 channels, by workgroups, T 12 at 576 / 1152 17.3 : 13.5, 19.1 : 22.3; T 16 at 768 19.1 : 16.3; T 25
+    // at 600 / 800 / 1200 23.2 : 16.9, 23.6 : 21.6, 25.9 : 26.7; T 40 at 960 29.5 : 35.4; Dh 32 at 768 / 1600 18.1 : 13.5,
+    // 24.8 : 26.8.  Head size 128 has one workgroup per CU (C21 T25 H16 35 : 25).
     if (!(a->flags & MVPA_FLAG_LAST_STEP) && a->C <= (a->Dh == 128 ? 32 : 64) && mvpa_wave_supported(a)) {
-      const int64_t wgs = (int64_t)a->B * a->H * ((a->C + 31) / 32) * a->T;
-      if (wgs <= 512 || (a->C <= 32 && a->T <= 128 && wgs <= 24 * (int64_t)a->T)) return mvpa_launch_wave(a, st);
+      const int64_t wgs = (int64_t)a->B * a->H * ((a->C + 31) / 32) * a->T, T = a->T;
+      int64_t most = 512;
+      if (a->Dh == 128) most = T <= 128 && 24 * T > most ? 24 * T : most;
+      else if (a->C > 32) most = T <= 32 ? 768 : most;
+      else if (48 * T > most) most = 48 * T < 2048 ? 48 * T : 2048;
+      if (wgs <= most) return mvpa_launch_wave(a, st);
     }
     // 65..128 channels at head size 64 or 128: the build of csrc/mvpa_mfma128.hip wins at every
     // length and channel count measured (Dh 128, B1 H16: C128 T 16 .. 1024 13 .. 20 % less time than

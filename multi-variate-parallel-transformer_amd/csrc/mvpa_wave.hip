@@ -11,7 +11,11 @@
 // load straight from global memory touches 32 lines for one KiB, at about two cycles each (q, bias and
 // table rows loaded that way took 8 us of a launch).  Arithmetic, roundings and operand layouts are
 // those of mvpa_mfma.hip; steps outside the content window skip K and the product with it.
-// Bound: the latency of set-up, of one or a few tiles per wave, and of the merge.
+// Bound: the latency of set-up, of one or a few tiles per wave, and of the merge.  What hides it is a second
+// workgroup on the CU, so head sizes up to 64 keep to 128 registers and 80 KB (tables of up to 64 rows): (q + u),
+// (q + v), (q + z) are formed once for all waves and stay in LDS, table rows go there directly, and addresses of a
+// tile are one register each.  With 165 registers, one workgroup a CU, B1 H12 Hkv4 C21 T25 Dh64 took two rounds of
+// an XCD's 32 CUs: 12.1 -> 9.9 us; C21 T64 23 -> 20.
 #include "mvpa_mfma_tools.h"
 
 namespace mvpa {
@@ -22,12 +26,12 @@ template <int DH>
 struct wave_cfg {
   static constexpr int KS = DH / 16, MT = DH / 32, ROWB = DH * 2, CHUNKS = DH / 8;
   static constexpr int TILE = 32 * ROWB, KV = 2 * TILE;           // one wave's K tile, then its V tile
-  static constexpr int Q_BYTES = 35 * ROWB;                       // 32 q rows, then u, v, z
+  static constexpr int Q_BYTES = 32 * ROWB;                       // (q + u) * scale
   static constexpr int MERGE = WV_WAVES * (64 + DH * 33) * 4;     // m, l and accumulators of every wave
 };
 
 template <int DH, typename E>
-__global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_args a, step_geom geo) {
+__global__ __launch_bounds__(WV_WAVES * 64, DH == 128 ? 2 : 4) void mvpa_wave_kernel(mvpa_fwd_args a, step_geom geo) {
   using x8 = typename E::x8;
   using x4 = typename E::x4;
   using x2 = typename E::x2;
@@ -78,23 +82,23 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
   constexpr int NL = DH / 16;
   const auto row_of = [&](int i) { return (i * 64 + lane) / CHUNKS; };
   const auto chunk_of = [&](int i) { return (i * 64 + lane) % CHUNKS; };
-  int koff[NL], voff[NL];
-#pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int c = min(ct * 32 + row_of(i), C_ - 1);
-    koff[i] = c * (int)a.k_stride_n + chunk_of(i) * 8;
-    voff[i] = c * (int)a.v_stride_n + chunk_of(i) * 8;
-  }
+  // bytes from the step's first row to this lane's chunk 0, and to the last row's; the NL chunks lie RPL rows apart
+  constexpr int RPL = 64 / CHUNKS;
+  uint32_t koff = (uint32_t)((ct * 32 + row_of(0)) * (int)a.k_stride_n + chunk_of(0) * 8) * 2u;
+  uint32_t voff = (uint32_t)((ct * 32 + row_of(0)) * (int)a.v_stride_n + chunk_of(0) * 8) * 2u;
+  uint32_t kend = (uint32_t)((C_ - 1) * (int)a.k_stride_n + chunk_of(0) * 8) * 2u;
+  uint32_t vend = (uint32_t)((C_ - 1) * (int)a.v_stride_n + chunk_of(0) * 8) * 2u;
   u32x4 kr[NL], vr[NL];
   auto request = [&](int s) {
+    asm volatile("" : "+v"(koff), "+v"(voff), "+v"(kend), "+v"(vend));   // (no 64-bit addresses held over the loop)
     if (s >= near0) {
-      const bf16_t* ks = kbase + (int64_t)s * C_ * a.k_stride_n;
+      const char* ks = (const char*)(kbase + (int64_t)s * C_ * a.k_stride_n);
 #pragma unroll
-      for (int i = 0; i < NL; ++i) kr[i] = *(const u32x4*)(ks + koff[i]);
+      for (int i = 0; i < NL; ++i) kr[i] = *(const u32x4*)(ks + min(koff + i * RPL * 2u * (uint32_t)a.k_stride_n, kend));
     }
-    const bf16_t* vs = vbase + (int64_t)s * C_ * a.v_stride_n;
+    const char* vs = (const char*)(vbase + (int64_t)s * C_ * a.v_stride_n);
 #pragma unroll
-    for (int i = 0; i < NL; ++i) vr[i] = *(const u32x4*)(vs + voff[i]);
+    for (int i = 0; i < NL; ++i) vr[i] = *(const u32x4*)(vs + min(voff + i * RPL * 2u * (uint32_t)a.v_stride_n, vend));
   };
   unsigned char* kl = wv_lds + wave * G::KV;
   unsigned char* vl = kl + G::TILE;
@@ -102,79 +106,75 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
 #pragma unroll
     for (int i = 0; i < NL; ++i) *(u32x4*)(kl + row_of(i) * ROWB + ((chunk_of(i) ^ swz_k<DH>(row_of(i))) << 4)) = r[i];
   };
-  int k_lane[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) k_lane[ks] = ln * ROWB + (((2 * ks + hh) ^ swz_k<DH>(ln)) << 4);
+  // fragment ks of row ln: the chunk's bits lie above the row's, so one address serves all (k_frag ^ ks << 5)
+  int k_frag = ln * ROWB + ((hh ^ swz_k<DH>(ln)) << 4);
 
-  // ---- set-up.  Requests, in the order of their use: the tile's q rows and the three bias vectors (a chunk
-  // or two per thread), the table rows of the wave's first 32-row tile, the wave's first K and V tiles.
-  constexpr int QN = (35 * CHUNKS + WV_WAVES * 64 - 1) / (WV_WAVES * 64);
-  u32x4 qr[QN];
-#pragma unroll
-  for (int i = 0; i < QN; ++i) {
-    const int pc = min(i * WV_WAVES * 64 + tid, 35 * CHUNKS - 1), row = pc / CHUNKS, c = pc % CHUNKS;
-    const bf16_t* src = row < 32 ? qbase + (int64_t)min(tile * 32 + row, C_ - 1) * a.q_stride_n
-                                 : (const bf16_t*)(row == 32 ? a.bias_u : row == 33 ? a.bias_v : a.bias_z) + g * DH;
-    qr[i] = *(const u32x4*)(src + c * 8);
-  }
+  // ---- set-up.  Requests, in the order of their use: a chunk of the tile's q rows and of the three bias vectors
+  // per thread, the table rows of the wave's first 32-row tile, the wave's first K and V tiles.
+  constexpr int QCH = 32 * CHUNKS, QN = (QCH + WV_WAVES * 64 - 1) / (WV_WAVES * 64);
+  static_assert(QN == 1, "a chunk of q per thread");
+  const int q_row = min(tid / CHUNKS, 31), q_chunk = tid % CHUNKS;
+  const u32x4 q_raw = *(const u32x4*)(qbase + (int64_t)min(tile * 32 + q_row, C_ - 1) * a.q_stride_n + q_chunk * 8);
+  const u32x4 u_raw = *(const u32x4*)((const bf16_t*)a.bias_u + g * DH + q_chunk * 8);
+  const u32x4 v_raw = *(const u32x4*)((const bf16_t*)a.bias_v + g * DH + q_chunk * 8);
+  const u32x4 z_raw = *(const u32x4*)((const bf16_t*)a.bias_z + g * DH + q_chunk * 8);
   const int ch_rows = qt * 32, n_tasks = qt + (steps + 31) / 32;
-  u32x4 er[NL];
-  auto request_rows = [&](int t) {                  // 32 table rows: channel tiles first, then time tiles
+  const uint32_t kl0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))wv_lds + wave * G::KV;
+  auto request_rows = [&](int t) {                  // 32 table rows into the wave's K tile: channel tiles first, then time tiles
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
+      const int tr = row_of(i);
       const bf16_t* row;
       if (t < qt) {
-        row = kchan + (int64_t)min(t * 32 + row_of(i), C_ - 1) * DH;
+        row = kchan + (int64_t)min(t * 32 + tr, C_ - 1) * DH;
       } else {
-        const int r = (t - qt) * 32 + row_of(i);
+        const int r = (t - qt) * 32 + tr;
         int j = last_only ? t_lo + r : time_row(tq, r, a.T);
-        if (ring) j = (j + ring_rot) % a.T;
+        j += ring_rot;
+        if (ring && j >= a.T) j -= a.T;
         row = ktime + (int64_t)min(j, a.T - 1) * DH;              // rows past the run: never used
       }
-      er[i] = *(const u32x4*)(row + chunk_of(i) * 8);
+      load_to_lds_16(row + (chunk_of(i) ^ swz_k<DH>(tr)) * 8, kl0 + i * 1024);
     }
   };
   if (wave < n_tasks) request_rows(wave);
   int s = wave / qt2;
   if (s < n_units) request(s);
   __builtin_amdgcn_sched_barrier(0);
+  // (q + bias) * scale of the tile, once for all waves: u for the key tiles; v and z, which the tables alone
+  // need, where the first two waves will keep their V tiles
   unsigned char* ql = wv_lds + WV_WAVES * G::KV;
-#pragma unroll
-  for (int i = 0; i < QN; ++i) {
-    const int pc = min(i * WV_WAVES * 64 + tid, 35 * CHUNKS - 1), row = pc / CHUNKS, c = pc % CHUNKS;
-    *(u32x4*)(ql + row * ROWB + ((row < 32 ? c ^ swz_k<DH>(row) : c) << 4)) = qr[i];
+  unsigned char* qv = wv_lds + G::TILE;
+  unsigned char* qz = qv + G::KV;
+  if (QCH == WV_WAVES * 64 || tid < QCH) {
+    const int at = q_row * ROWB + ((q_chunk ^ swz_k<DH>(q_row)) << 4);
+    float f[8];
+    E::unpack(q_raw, f);
+    *(x8*)(ql + at) = qfrag_fma<E>(f, u_raw, sc2);
+    *(x8*)(qv + at) = qfrag_fma<E>(f, v_raw, sc2);
+    *(x8*)(qz + at) = qfrag_fma<E>(f, z_raw, sc2);
   }
   lds_barrier();
   float* Sc = (float*)(ql + G::Q_BYTES);
   float* St = Sc + ch_rows * 32;
-  u32x4 raw[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) raw[ks] = *(const u32x4*)(ql + k_lane[ks]);
-  auto biased = [&](int ks, int row) {              // (q + bias) * scale; rows 32, 33, 34 hold u, v, z
-    float f[8];
-    E::unpack(raw[ks], f);
-    return qfrag_fma<E>(f, *(const u32x4*)(ql + row * ROWB + ((2 * ks + hh) << 4)), sc2);
-  };
   for (int t = wave; t < n_tasks; t += WV_WAVES) {
     const bool chan = t < qt;
     if (t != wave) request_rows(t);
-    put_k(er);
+    wait_vmcnt_imm<0>();
     wave_lds_sync();
     f32x16 acc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[i] = 0.f;
     if (chan ? has_chan : has_time) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) acc = E::mfma(*(const x8*)(kl + k_lane[ks]), biased(ks, chan ? 34 : 33), acc, 0, 0, 0);
+      for (int ks = 0; ks < KS; ++ks)
+        acc = E::mfma(*(const x8*)(kl + (k_frag ^ (ks << 5))), *(const x8*)((chan ? qz : qv) + (k_frag ^ (ks << 5))), acc, 0, 0, 0);
     }
     wave_lds_sync();
     float* dst = (chan ? Sc : St) + (chan ? t : t - qt) * 1024 + ln;
 #pragma unroll
     for (int i = 0; i < 16; ++i) dst[((i >> 2) * 8 + hh * 4 + (i & 3)) * 32] = acc[i];
   }
-  x8 Qu[KS];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) Qu[ks] = biased(ks, 32);
   uint32_t kbits;                                   // bit 8(i/4) + i%4: this lane's key i exists and is present
   {
     const int ck = ct * 32 + ln;
@@ -193,12 +193,10 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
   }
 
   // ---- the wave's key tiles
-  int v_lane[MT];
+  int v_frag;                                       // of output tile mt: v_frag ^ mt << 6
   {
     const int e = (ln & 15) >> 2, aa = ln & 3, grp = ln >> 4, row0 = 4 * hh + e;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-      v_lane[mt] = row0 * ROWB + (((4 * mt + 2 * grp + (aa >> 1)) ^ swz_v<DH>(row0)) << 4) + ((aa & 1) << 3);
+    v_frag = row0 * ROWB + (((2 * grp + (aa >> 1)) ^ swz_v<DH>(row0)) << 4) + ((aa & 1) << 3);
   }
   float m_run = kMFloor, l_run = 0.f;
   f32x16 acc[MT];
@@ -209,6 +207,7 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
 
   for (; s < n_units; s += spr) {
     const bool near = s >= near0;
+    asm volatile("" : "+v"(k_frag), "+v"(v_frag));   // (addresses formed where they are used: 128 registers)
     if (near) put_k(kr);
 #pragma unroll
     for (int i = 0; i < NL; ++i) *(u32x4*)(vl + row_of(i) * ROWB + ((chunk_of(i) ^ swz_v<DH>(row_of(i))) << 4)) = vr[i];
@@ -217,7 +216,7 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
     f32x16 S = Bc;
     if (near) {
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) S = E::mfma(*(const x8*)(kl + k_lane[ks]), Qu[ks], S, 0, 0, 0);
+      for (int ks = 0; ks < KS; ++ks) S = E::mfma(*(const x8*)(kl + (k_frag ^ (ks << 5))), *(const x8*)(ql + (k_frag ^ (ks << 5))), S, 0, 0, 0);
     }
     const float st = St[s * 32 + ln];
     float rmax = -INFINITY;
@@ -248,7 +247,7 @@ __global__ __launch_bounds__(WV_WAVES * 64, 2) void mvpa_wave_kernel(mvpa_fwd_ar
     for (int p = 0; p < 2; ++p)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const unsigned char* vp = vl + v_lane[mt] + 16 * p * ROWB;
+        const unsigned char* vp = vl + (v_frag ^ (mt << 6)) + 16 * p * ROWB;
         const x4 lo = E::read_tr(vp), hi = E::read_tr(vp + 8 * ROWB);
         acc[mt] = E::mfma(__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7), P[p], acc[mt], 0, 0, 0);
       }
@@ -318,7 +317,7 @@ static int launch_wave_t(const mvpa_fwd_args* a, int lds, hipStream_t stream) {
 static int wave_lds_bytes(const mvpa_fwd_args* a) {
   const int steps = (a->flags & MVPA_FLAG_LAST_STEP) && a->n_split > 1 ? (a->T + a->n_split - 1) / a->n_split : a->T;
   const int rows = (a->C + 31) / 32 * 32 + (steps + 31) / 32 * 32;
-  const int run = (WV_WAVES * 64 + 35) * a->Dh * 2 + rows * 128, merge = WV_WAVES * (64 + a->Dh * 33) * 4;
+  const int run = (WV_WAVES * 64 + 32) * a->Dh * 2 + rows * 128, merge = WV_WAVES * (64 + a->Dh * 33) * 4;
   return run > merge ? run : merge;
 }
 
@@ -326,7 +325,9 @@ static int wave_lds_bytes(const mvpa_fwd_args* a) {
 
 // Shapes: those of the tiled kernel, without the fp8 content term, as long as the tables fit the LDS.
 int mvpa_wave_supported(const mvpa_fwd_args* a) {
-  return mvpa_mfma_supported(a) && !(a->flags & MVPA_FLAG_FP8_QK) && mvpa::wave_lds_bytes(a) <= 160 * 1024;
+  const int64_t row = a->k_stride_n > a->v_stride_n ? a->k_stride_n : a->v_stride_n;
+  return mvpa_mfma_supported(a) && !(a->flags & MVPA_FLAG_FP8_QK) && mvpa::wave_lds_bytes(a) <= 160 * 1024 &&
+         row < ((int64_t)1 << 24);                 // 128 rows of a step, padded ones too, in 32 bits of bytes
 }
 
 int mvpa_launch_wave(const mvpa_fwd_args* a, hipStream_t stream) {

@@ -255,6 +255,39 @@ def test_fp16_mfma_shapes(cfg):
     assert (lse.cpu().double() - ref_lse).abs().max().item() <= FP16_LSE
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("cfg", [
+    dict(B=1, C=1, T=1, H=1, Dh=64),
+    dict(B=2, C=21, T=25, H=12, Hkv=4, Dh=64, validity=True),      # two workgroups a CU
+    dict(B=1, C=32, T=33, H=6, Hkv=2, Dh=64),                      # two tiles of the time table
+    dict(B=1, C=33, T=12, H=3, Dh=64),                             # a second query tile of one row
+    dict(B=1, C=64, T=12, H=32, Hkv=4, Dh=64),                     # 768 workgroups
+    dict(B=1, C=5, T=300, H=1, Dh=64),                             # more table tiles than waves
+    dict(B=1, C=31, T=290, H=1, Dh=32, validity=True),
+    dict(B=1, C=30, T=40, H=2, Dh=128),
+], ids=lambda c: "B{B}C{C}T{T}H{H}D{Dh}".format(**c))
+def test_small_launches_of_the_default_selector(cfg, dtype):
+    """The launches that the build with the keys of a query tile split over the waves serves, q, k and v as
+    views of one projection's rows (each with strides of its own)."""
+    inp = make_mvpa_inputs(seed=23, table_std=0.3, qkv_unit=True, **cfg).round_to(dtype)
+    d = inp.to("cuda", dtype)
+
+    def rows(x, pad):          # [B,H,N,Dh] as a view of [B,N,H*Dh+pad]
+        B, H, N, Dh = x.shape
+        m = torch.zeros((B, N, H * Dh + pad), dtype=dtype, device="cuda")
+        m[:, :, :H * Dh] = x.permute(0, 2, 1, 3).reshape(B, N, H * Dh)
+        return m[:, :, :H * Dh].view(B, N, H, Dh).permute(0, 2, 1, 3)
+    out, lse = mvpa_hip.mvpa_forward(rows(d.q, 0), rows(d.k, 8), rows(d.v, 24), d.u, d.vb, d.z, d.k_time, d.k_chan,
+                                     chan_valid=d.chan_valid, return_lse=True)
+    ref, ref_lse = _oracle(inp, return_lse=True)
+    if dtype == torch.bfloat16:
+        _check_bf16(out, ref)
+    else:
+        o = out.float().cpu()
+        assert (o - ref.float()).abs().max().item() <= FP16_MAX_ABS and _rel_l2(o, ref.float()) <= FP16_REL_L2
+    assert (lse.cpu().double() - ref_lse).abs().max().item() <= (3e-2 if dtype == torch.bfloat16 else FP16_LSE)
+
+
 def test_fp16_dispatch_and_what_it_refuses():
     """fp16 under the default selector takes the matrix-core kernel (bit for bit the forced
     launch); the specialised bf16 builds and the fp8 content term refuse fp16 tensors."""
