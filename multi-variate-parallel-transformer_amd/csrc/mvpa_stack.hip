@@ -271,7 +271,7 @@ extern "C" int mvpa_stack_forward_blocks(const mvpa_stack_args* a, int32_t first
     if ((st = attend(blk)) != MVPA_OK) return st;
     if ((st = launch_tile_partial(p.both, p.rows, wide, wide, (const bf16_t*)blk.w_tail, E, wide, p.partial, p.split_k, s)) != MVPA_OK) return st;
     const bool last = i + 1 == a->n_blocks;
-    if ((st = launch_tail_reduce(p.partial, p.split_k, x, p.hidden[0], last ? (bf16_t*)a->y : p.normed,
+    if ((st = launch_tail_reduce(p.partial, p.split_k, x, p.hidden[0], last ? (bf16_t*)a->y : p.raw ? nullptr : p.normed,
                                  last ? a->lnf_weight : a->blocks[i + 1].ln_weight, last ? a->lnf_eps : a->blocks[i + 1].ln_eps,
                                  p.raw && !last ? p.sumsq[0] : nullptr, p.rows, E, s)) != MVPA_OK) return st;
   }

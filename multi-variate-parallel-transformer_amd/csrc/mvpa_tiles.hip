@@ -20,6 +20,8 @@
 
 namespace mvpa {
 
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+
 constexpr int TL_BN = 64, TL_BK = 64, TL_ROWB = TL_BK * 2;
 constexpr int TL_SUM = TL_BN * 4;                   // bytes of a row of sums: 16 chunks, XOR-swizzled by the row
 
@@ -284,46 +286,60 @@ __global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restr
 
 // One workgroup per row: the partial sums of a split-K tail product, the residual, one rounding, and
 // the RMSNorm that the next product wants, while the row is in registers (8 columns per lane and chunk).
-template <int CHUNKS>
+// Bound by the trip to the sums, which other XCDs have just written: all PARTS (the next of 4, 6, 8, 9 from their number; past
+// the last, the last once more, not added), the residual and the norm's weight are requested together.  With one part after the
+// other and the weight behind the sums of squares a stream's step (64 rows of 768, 9 parts, 12 launches) took 414 us and takes
+// 396, a step of the base model (128 rows of 2048, 8 parts, 24 launches) 1803 and 1792; 525 rows (4 parts) 517 and 518.
+template <int CHUNKS, int PARTS>
 __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restrict__ P, int split_a, int split_b,
                                                           const bf16_t* __restrict__ R, bf16_t* __restrict__ S,
                                                           bf16_t* __restrict__ Y, const float* __restrict__ w,
                                                           float eps, float* __restrict__ ss_out, int64_t M, int N) {
   __shared__ float red[4];
   const int64_t m = blockIdx.x;
+  const int parts = split_a + split_b;
   float v[CHUNKS][8], ss = 0.f;
+  f32x4 p[CHUNKS][PARTS][2], wr[CHUNKS][2];
+  u32x4 rr[CHUNKS];
+#pragma unroll
+  for (int c = 0; c < CHUNKS; ++c) {                // lanes past the row: its last columns, for nobody
+    const int n = min((c * 256 + (int)threadIdx.x) * 8, N - 8);
+    rr[c] = *(const u32x4*)(R + m * N + n);
+#pragma unroll
+    for (int z = 0; z < PARTS; ++z) {
+      const float* at = P + ((int64_t)min(z, parts - 1) * M + m) * N + n;
+      p[c][z][0] = *(const f32x4*)at;
+      p[c][z][1] = *(const f32x4*)(at + 4);
+    }
+    const float* at = (Y ? w : P) + n;              // without a norm: anything
+    wr[c][0] = *(const f32x4*)at;
+    wr[c][1] = *(const f32x4*)(at + 4);
+  }
+  __builtin_amdgcn_sched_barrier(0);                // every request first
+  // without branches, behind which the loads would be put and waited for one by one
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
     const int n = (c * 256 + threadIdx.x) * 8;
-    if (n < N) {
-      const u32x4 rr = *(const u32x4*)(R + m * N + n);
+    float a[8] = {}, b[8] = {};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[c][2 * i] = __uint_as_float(rr[i] << 16);
-        v[c][2 * i + 1] = __uint_as_float(rr[i] & 0xffff0000u);
-      }
-      auto add_part = [&](int z0, int z1) {
-        float s[8] = {};
-        for (int z = z0; z < z1; ++z) {
-          const float* p = P + ((int64_t)z * M + m) * N + n;
-          const float4 a = *(const float4*)p, b = *(const float4*)(p + 4);
-          s[0] += a.x; s[1] += a.y; s[2] += a.z; s[3] += a.w;
-          s[4] += b.x; s[5] += b.y; s[6] += b.z; s[7] += b.w;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[c][i] += (float)(__bf16)s[i];
-      };
-      add_part(split_a, split_a + split_b);
-      if (split_a) add_part(0, split_a);
-      bf16x8 o;
+    for (int z = 0; z < PARTS; ++z)
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        o[i] = (__bf16)v[c][i];
-        v[c][i] = (float)o[i];
-        ss += v[c][i] * v[c][i];
+        const float x = p[c][z][i >> 2][i & 3];
+        a[i] += z < split_a ? x : 0.f;
+        b[i] += z >= split_a && z < parts ? x : 0.f;
       }
-      *(bf16x8*)(S + m * N + n) = o;
+    bf16x8 o;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[c][i] = __uint_as_float(i & 1 ? rr[c][i >> 1] & 0xffff0000u : rr[c][i >> 1] << 16);
+      v[c][i] += (float)(__bf16)b[i];
+      v[c][i] += (float)(__bf16)a[i];               // 0 where there is no first run
+      o[i] = (__bf16)v[c][i];
+      v[c][i] = (float)o[i];
+      ss += n < N ? v[c][i] * v[c][i] : 0.f;
     }
+    if (n < N) *(bf16x8*)(S + m * N + n) = o;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
@@ -337,11 +353,9 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
   for (int c = 0; c < CHUNKS; ++c) {
     const int n = (c * 256 + threadIdx.x) * 8;
     if (n < N) {
-      const float4 a = *(const float4*)(w + n), b = *(const float4*)(w + n + 4);
-      const float g[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
       bf16x8 o;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = (__bf16)(v[c][i] * inv * g[i]);
+      for (int i = 0; i < 8; ++i) o[i] = (__bf16)(v[c][i] * inv * wr[c][i >> 2][i & 3]);
       *(bf16x8*)(Y + m * N + n) = o;
     }
   }
@@ -419,8 +433,14 @@ int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, cons
 
 int launch_tail_reduce(const float* P, const tile_split& split, const bf16_t* r, bf16_t* sum, bf16_t* norm, const float* w,
                        float eps, float* ss, int64_t M, int64_t N, hipStream_t s) {
-  if (N <= 2048) MVPA_LAUNCH(tail_reduce_kernel<1>, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
-  else MVPA_LAUNCH(tail_reduce_kernel<2>, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
+  auto pick = [&](auto chunks) {
+    constexpr int CH = decltype(chunks)::value;
+    const int parts = split.total();                // at most 9: make_tile_split
+    return parts <= 4 ? tail_reduce_kernel<CH, 4> : parts <= 6 ? tail_reduce_kernel<CH, 6> : parts <= 8 ? tail_reduce_kernel<CH, 8>
+                                                                                                      : tail_reduce_kernel<CH, 9>;
+  };
+  auto kern = N <= 2048 ? pick(std::integral_constant<int, 1>()) : pick(std::integral_constant<int, 2>());
+  MVPA_LAUNCH(kern, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
   return take_launch_status();
 }
 
