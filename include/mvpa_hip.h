@@ -432,6 +432,22 @@ int mvpa_ring_append_bf16(const void* k_new, const void* v_new, void* k_ring, vo
 int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64_t M, int32_t L, int32_t levels,
                              int32_t dwt_size, int64_t ldy, float eps, void* stream);
 
+/* 1 where mvpa_wavedec_db4_rmsnorm takes rows of L samples, 0 where it does not. */
+int mvpa_wavedec_db4_rmsnorm_fits(int32_t L, int32_t levels, int32_t dwt_size);
+
+/* The same, and what the gradient of the norm's weight needs: the coefficients in fp32, coeffs[M,ldy] (16-byte
+ * aligned, zeros past them), and the factor 1 / sqrt(mean square + eps) of every row, inv[M]. */
+int mvpa_wavedec_db4_rmsnorm_saved(const float* x, const float* weight, void* y, float* coeffs, float* inv, int64_t M, int32_t L,
+                                   int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream);
+
+/* dw[c] = sum over the rows of dy[r,c] x[r,c] inv[r]: the weight's share of the backward of y = x inv weight with
+ * fp32 rows x (row pitch ldx), bf16 dy (lddy) and the row factors inv, pitches multiples of 4 that reach over
+ * whole groups of 4 columns, x 16-byte and dy 8-byte aligned.  dw is fp32 with w_f32 and bf16 otherwise; ws takes
+ * mvpa_norm_dw_ws_bytes(rows, cols) bytes, 16-byte aligned. */
+size_t mvpa_norm_dw_ws_bytes(int64_t rows, int32_t cols);
+int mvpa_norm_dw(const float* x, const float* inv, const void* dy, void* dw, void* ws, int64_t rows, int32_t cols, int64_t ldx,
+                 int64_t lddy, int32_t w_f32, void* stream);
+
 /* out[g] = mean over its `rows` rows of a group of bf16 rows (fp32 sum, one rounding): the mean over
  * the channels of the last segment's hidden state (models/mvpformer.py:947-953).  Group g starts at
  * x + g * group_stride (elements), rows are ldx elements apart; cols a multiple of 8. */

@@ -1531,15 +1531,23 @@ __global__ __launch_bounds__(256) void wavedec_db4_kernel(const float* __restric
 // sample and 2 bytes out per coefficient (as three launches through fp32 coefficients: 98 us for
 // 16384 rows of 512, of which the row-per-workgroup analysis with a barrier per level took 72).
 // G threads own a row: one wave for short rows (no workgroup barrier at all), a workgroup for long
-// ones.  Periodic wrap by copies of 8 samples on either side of an approximation, so that the taps of
-// output k are the 8 consecutive samples 2k-6 .. 2k+1 without an index modulo n.
+// ones.  Even and odd samples lie in arrays of their own, with copies of 8 samples around them for the periodic wrap: a thread
+// takes outputs 2 t and 2 t + 1, whose taps are the six pairs E, O[2 t - 4 .. 2 t + 1], without an index modulo n and
+// without bank conflicts, and of a row that a workgroup owns the last levels are one wave's (taps read one by one with a stride
+// of two floats, every level with two barriers: 6400 rows of 2560 60 -> 46 us, 16384 of 512 34.0 -> 29.7, 64 of 512 7.5 -> 8.0).
+// With coef_out (row pitch ldy) and inv_out the coefficients and the factor of every row leave as well: a
+// training pass wants them for the gradient of the norm's weight (norm_dw_kernel).
 // -----------------------------------------------------------------------------------------
+// floats of the even (or odd) samples of n, four in front and behind for the wrap
+__host__ __device__ constexpr int wavedec_half(int n) { return (4 + (n + 1) / 2 + 4 + 3) & ~3; }
+
 template <int G>
 __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* __restrict__ x,
                                                                   const float* __restrict__ w,
-                                                                  bf16_t* __restrict__ y, int64_t M, int L,
+                                                                  bf16_t* __restrict__ y, float* __restrict__ coef_out,
+                                                                  float* __restrict__ inv_out, int64_t M, int L,
                                                                   int levels, int dwt_size, int64_t ldy, float eps,
-                                                                  int row_floats) {
+                                                                  int row_floats, bool vec) {
   extern __shared__ __attribute__((aligned(16))) float wd_lds[];
   __shared__ float red[4];
   const int sub = threadIdx.x / G, t = threadIdx.x % G;
@@ -1554,44 +1562,107 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
   };
-  constexpr int PAD = 8;
-  const int half = (L + 7) / 2;
-  float* cur = wd_lds + sub * row_floats + PAD;     // [PAD | L | PAD]
-  float* nxt = cur + ((L + 2 * PAD + 3) & ~3);      // [PAD | half | PAD]
-  float* coef = nxt + ((half + 2 * PAD + 3) & ~3) - PAD;
+  const int first = wavedec_half(L), later = wavedec_half((L + 7) / 2);
+  float* even = wd_lds + sub * row_floats + 4;      // sample 2 i; then the odd ones, 2 i + 1
+  float* odd = even + first;
+  float* next_even = odd + first;
+  float* next_odd = next_even + later;
+  float* coef = next_odd + later - 4;
   const float* xr = x + row * L;
-  for (int i = t; i < L; i += G) cur[i] = xr[i];
-  int n = L, tail = dwt_size;
-  float ss = 0.f;
-  for (int lv = 1; lv <= levels; ++lv) {
-    sync();
-    if (t < PAD) {
-      cur[t - PAD] = cur[n + t - PAD];
-      cur[n + t] = cur[t];
-    }
-    sync();
-    const int m = (n + 7) >> 1;
-    tail -= m;
-    for (int k = t; k < m; k += G) {
-      float lo = 0.f, hi = 0.f;
+  // sample k of n, and its copies in front of and behind them for the periodic wrap: a wave by itself makes those in one go
+  // instead (wrap), which takes it less time than the branches; a workgroup would need one more barrier
+  auto put = [](float* e, float* o, int k, int n, float v) {
+    (k & 1 ? o : e)[k >> 1] = v;
+    if (G == 64) return;
+    if (k < 8) ((n + k) & 1 ? o : e)[(n + k) >> 1] = v;
+    if (k >= n - 8) ((k - n) & 1 ? o : e)[(k - n) >> 1] = v;
+  };
+  if (vec) {
+    for (int i = t; i < L / 4; i += G) {
+      const float4 v = *(const float4*)(xr + 4 * i);
+      *(float2*)(even + 2 * i) = make_float2(v.x, v.z);
+      *(float2*)(odd + 2 * i) = make_float2(v.y, v.w);
+      if (G == 256 && (i < 2 || i >= L / 4 - 2)) {
+        const float q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float v = cur[2 * k + 1 - j];
-        lo += kDb4Lo[j] * v;
-        hi += ((j & 1) ? kDb4Lo[7 - j] : -kDb4Lo[7 - j]) * v;
+        for (int j = 0; j < 4; ++j) put(even, odd, 4 * i + j, L, q[j]);
       }
-      nxt[k] = lo;
-      coef[tail + k] = hi;
-      ss += hi * hi;
     }
-    float* sw = cur;
-    cur = nxt;
-    nxt = sw;
-    n = m;
+  } else {
+    for (int i = t; i < L; i += G) put(even, odd, i, L, xr[i]);
+  }
+  int n = L, tail = dwt_size;
+  auto level = [&](int threads) {
+    const int m = (n + 7) >> 1;
+    const int at = tail - m;
+    for (int k = 2 * t; k < m; k += 2 * threads) {
+      float e[6], o[6];
+#pragma unroll
+      for (int i = 0; i < 6; i += 2) {
+        const float2 a = *(const float2*)(even + k - 4 + i), b = *(const float2*)(odd + k - 4 + i);
+        e[i] = a.x; e[i + 1] = a.y;
+        o[i] = b.x; o[i + 1] = b.y;
+      }
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        float lo = 0.f, hi = 0.f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {               // tap j of output k + q: sample 2 (k + q) + 1 - j
+          const float v = j & 1 ? e[4 + q - (j >> 1)] : o[4 + q - (j >> 1)];
+          lo += kDb4Lo[j] * v;
+          hi += ((j & 1) ? kDb4Lo[7 - j] : -kDb4Lo[7 - j]) * v;
+        }
+        if (k + q < m) {
+          put(next_even, next_odd, k + q, m, lo);
+          coef[at + k + q] = hi;
+        }
+      }
+    }
+  };
+  auto advance = [&]() {
+    n = (n + 7) >> 1;
+    tail -= n;
+    float* sw = even; even = next_even; next_even = sw;
+    sw = odd; odd = next_odd; next_odd = sw;
+  };
+  auto wrap = [&]() {                               // samples -8 .. -1 and n .. n + 7 (n is at least 8)
+    if (t < 16) {
+      const int to = t < 8 ? t - 8 : n + t - 8, from = t < 8 ? n + t - 8 : t - 8;
+      (to & 1 ? odd : even)[to >> 1] = (from & 1 ? odd : even)[from >> 1];
+    }
+  };
+  int lv = 0;
+  for (; lv < levels && (G == 64 || n > 256); ++lv) {
+    sync();
+    if (G == 64) {
+      wrap();
+      sync();
+    }
+    level(G);
+    advance();
+  }
+  if (G == 256) {                                   // what is left is a wave's work, without barriers of the workgroup
+    sync();
+    for (; lv < levels; ++lv) {
+      if (t < 64) {
+        level(64);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      advance();
+    }
   }
   sync();
+  // the sum of squares level by level, as their outputs are dealt to the threads one by one
+  float ss = 0.f;
+  for (int lev = 0, of = L, at = dwt_size; lev < levels; ++lev) {
+    of = (of + 7) >> 1;
+    at -= of;
+    for (int k = t; k < of; k += G) ss += coef[at + k] * coef[at + k];
+  }
   for (int k = t; k < n; k += G) {
-    const float v = cur[k];
+    const float v = (k & 1 ? odd : even)[k >> 1];
     coef[k] = v;
     ss += v * v;
   }
@@ -1604,11 +1675,24 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
     sync();
   }
   const float inv = rsqrtf(ss / (float)dwt_size + eps);
+  if (inv_out && t == 0) inv_out[row] = inv;
   for (int c = t * 8; c < ldy; c += G * 8) {
-    float v[8];
+    float v[8] = {}, f[8] = {}, g[8] = {};
+    if (c < dwt_size) vec8<float>::load(coef + c, f);          // (a row's coefficients take whole groups of 8)
+    if (vec && c + 8 <= dwt_size) {
+      vec8<float>::load(w + c, g);
+    } else {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = c + i < dwt_size ? coef[c + i] * inv * w[c + i] : 0.f;
+      for (int i = 0; i < 8; ++i)
+        if (c + i < dwt_size) g[i] = w[c + i];
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f[i] = c + i < dwt_size ? f[i] : 0.f;
+      v[i] = f[i] * inv * g[i];
+    }
     vec8<bf16_t>::store(y + row * ldy + c, v);
+    if (coef_out) vec8<float>::store(coef_out + row * ldy + c, f);
   }
 }
 
@@ -2083,29 +2167,55 @@ extern "C" int mvpa_wavedec_db4(const float* x, float* coeffs, int64_t M, int32_
   return mvpa::take_launch_status();
 }
 
-extern "C" int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64_t M, int32_t L,
-                                        int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream) {
-  if (!x || !weight || !y) return MVPA_ERR_NULL;
-  if (M <= 0 || L < 8 || levels < 1 || ldy < dwt_size) return MVPA_ERR_SHAPE;
-  if ((ldy & 7) || ((uintptr_t)y & 15)) return MVPA_ERR_ALIGN;
-  int n = L, total = 0;
+// floats of a row of L samples: samples and first approximation with their wrap copies, coefficients
+static int wavedec_row_floats(int32_t L, int32_t dwt_size) {
+  return 2 * wavedec_half(L) + 2 * wavedec_half((L + 7) / 2) + ((dwt_size + 7) & ~7);
+}
+
+static int wavedec_rmsnorm_check(int32_t L, int32_t levels, int32_t dwt_size) {
+  if (L < 8 || levels < 1) return MVPA_ERR_SHAPE;
+  int64_t n = L, total = 0;
   for (int lv = 0; lv < levels; ++lv) {
     if (n < 8) return MVPA_ERR_UNSUPPORTED;
     n = (n + 7) >> 1;
     total += n;
   }
   if (total + n != dwt_size) return MVPA_ERR_SHAPE;
-  // per row: samples and first approximation with their wrap copies, coefficients
-  const int row_floats = ((L + 16 + 3) & ~3) + (((L + 7) / 2 + 16 + 3) & ~3) + ((dwt_size + 3) & ~3);
+  return L > 1 << 20 || wavedec_row_floats(L, dwt_size) * 4 > 157 * 1024 ? MVPA_ERR_UNSUPPORTED : MVPA_OK;
+}
+
+extern "C" int mvpa_wavedec_db4_rmsnorm_fits(int32_t L, int32_t levels, int32_t dwt_size) {
+  return wavedec_rmsnorm_check(L, levels, dwt_size) == MVPA_OK;
+}
+
+static int launch_wavedec_rmsnorm(const float* x, const float* weight, void* y, float* coeffs, float* inv, int64_t M, int32_t L,
+                                  int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream) {
+  if (!x || !weight || !y) return MVPA_ERR_NULL;
+  if (M <= 0 || L < 8 || levels < 1 || ldy < dwt_size) return MVPA_ERR_SHAPE;
+  if ((ldy & 7) || (((uintptr_t)y | (uintptr_t)coeffs) & 15)) return MVPA_ERR_ALIGN;
+  const int st = wavedec_rmsnorm_check(L, levels, dwt_size);
+  if (st != MVPA_OK) return st;
+  const int row_floats = wavedec_row_floats(L, dwt_size);
   // one wave per row while four rows leave room for two workgroups per CU
   const bool wave = row_floats * 4 * 4 <= 80 * 1024;
   const int lds = row_floats * 4 * (wave ? 4 : 1);
-  if (lds > 156 * 1024) return MVPA_ERR_UNSUPPORTED;
   auto kern = wave ? wavedec_db4_rmsnorm_kernel<64> : wavedec_db4_rmsnorm_kernel<256>;
   if (lds > 64 * 1024) mvpa::want_dynamic_lds((const void*)kern, lds);
   MVPA_LAUNCH(kern, dim3((unsigned)(wave ? (M + 3) / 4 : M)), dim3(256), lds, (hipStream_t)stream, x, weight, (bf16_t*)y,
-              M, L, levels, dwt_size, ldy, eps, row_floats);
+              coeffs, inv, M, L, levels, dwt_size, ldy, eps, row_floats,
+              L % 4 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0);
   return mvpa::take_launch_status();
+}
+
+extern "C" int mvpa_wavedec_db4_rmsnorm(const float* x, const float* weight, void* y, int64_t M, int32_t L,
+                                        int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream) {
+  return launch_wavedec_rmsnorm(x, weight, y, nullptr, nullptr, M, L, levels, dwt_size, ldy, eps, stream);
+}
+
+extern "C" int mvpa_wavedec_db4_rmsnorm_saved(const float* x, const float* weight, void* y, float* coeffs, float* inv, int64_t M,
+                                              int32_t L, int32_t levels, int32_t dwt_size, int64_t ldy, float eps, void* stream) {
+  if (!coeffs || !inv) return MVPA_ERR_NULL;
+  return launch_wavedec_rmsnorm(x, weight, y, coeffs, inv, M, L, levels, dwt_size, ldy, eps, stream);
 }
 
 extern "C" int mvpa_mean_rows_bf16(const void* x, void* out, int64_t groups, int64_t rows, int32_t cols, int64_t ldx,

@@ -295,6 +295,14 @@ PyObject* py_linear_wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// as_operand, starting at a 16-byte boundary
+Tensor aligned_operand(const Tensor& t, at::ScalarType dt) {
+  Tensor r = as_operand(t, dt);
+  return (uintptr_t)r.const_data_ptr() & 15 ? r.clone() : r;
+}
+
+bool f32_or_bf16(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
+
 // encode(x [M, L] fp32, norm weight fp32, levels, dwt_size, pitch, eps) -> [M, pitch] bf16 | status
 PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -312,6 +320,51 @@ PyObject* py_encode(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// encode_saved(as encode) -> ([M, pitch] bf16, the coefficients [M, pitch] fp32, the row factors [M]) | status
+PyObject* py_encode_saved(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 6, "encode_saved takes 6 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor x = as_operand(tensor_of(args[0]), at::kFloat), w = as_operand(tensor_of(args[1]), at::kFloat);
+  const long levels = PyLong_AsLong(args[2]), dwt = PyLong_AsLong(args[3]), pitch = PyLong_AsLong(args[4]);
+  const double eps = PyFloat_AsDouble(args[5]);
+  if (PyErr_Occurred()) return nullptr;
+  TORCH_CHECK(x.dim() == 2 && w.numel() == dwt && w.device() == x.device(), "encode_saved: rows of samples, a weight per coefficient on their GPU");
+  Tensor y = at::empty({x.size(0), pitch}, x.options().dtype(at::kBFloat16));
+  Tensor coeffs = at::empty({x.size(0), pitch}, x.options()), inv = at::empty({x.size(0)}, x.options());
+  const int st = mvpa_wavedec_db4_rmsnorm_saved((const float*)x.data_ptr(), (const float*)w.data_ptr(), y.data_ptr(),
+                                                (float*)coeffs.data_ptr(), (float*)inv.data_ptr(), x.size(0), (int32_t)x.size(1),
+                                                (int32_t)levels, (int32_t)dwt, pitch, (float)eps, current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* r = PyTuple_New(3);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(y));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(coeffs));
+  PyTuple_SET_ITEM(r, 2, THPVariable_Wrap(inv));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// norm_dw(x [M, pitch] fp32, inv [M] fp32, dy [M, pitch] bf16, weight) -> the weight's gradient | status
+PyObject* py_norm_dw(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 4, "norm_dw takes 4 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor x = aligned_operand(tensor_of(args[0]), at::kFloat), inv = as_operand(tensor_of(args[1]), at::kFloat);
+  const Tensor dy = aligned_operand(tensor_of(args[2]), at::kBFloat16);
+  const Tensor& w = tensor_of(args[3]);
+  TORCH_CHECK_TYPE(f32_or_bf16(w), "norm_dw: fp32 or bf16");
+  TORCH_CHECK(x.dim() == 2 && dy.sizes() == x.sizes() && inv.numel() == x.size(0) && w.numel() <= x.size(1) &&
+              dy.device() == x.device() && inv.device() == x.device() && w.device() == x.device(), "norm_dw: operands differ");
+  const int64_t rows = x.size(0);
+  const int32_t cols = (int32_t)w.numel();
+  Tensor dw = at::empty(w.sizes(), w.options());
+  Tensor ws = at::empty({(int64_t)mvpa_norm_dw_ws_bytes(rows, cols)}, x.options().dtype(at::kByte));
+  const int st = mvpa_norm_dw((const float*)x.data_ptr(), (const float*)inv.data_ptr(), dy.data_ptr(), dw.data_ptr(), ws.data_ptr(),
+                              rows, cols, x.stride(0), dy.stride(0), w.scalar_type() == at::kFloat, current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(dw) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
 // mean_rows(x [G, R, E] bf16, unit last stride) -> [G, E] | status
 PyObject* py_mean_rows(PyObject*, PyObject* arg) {
   HANDLE_TH_ERRORS
@@ -326,15 +379,7 @@ PyObject* py_mean_rows(PyObject*, PyObject* arg) {
   END_HANDLE_TH_ERRORS
 }
 
-// as_operand, starting at a 16-byte boundary
-Tensor aligned_operand(const Tensor& t, at::ScalarType dt) {
-  Tensor r = as_operand(t, dt);
-  return (uintptr_t)r.const_data_ptr() & 15 ? r.clone() : r;
-}
-
 // ---- row operations of the training path -------------------------------------------------------
-bool f32_or_bf16(const Tensor& t) { return t.scalar_type() == at::kFloat || t.scalar_type() == at::kBFloat16; }
-
 // norm_backward(x, weight, dy, res | None, eps, need_dx, need_dw) -> (dx | None, dw | None) | status
 PyObject* py_norm_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
@@ -827,6 +872,8 @@ PyMethodDef kMethods[] = {
     {"linear_wgrad", (PyCFunction)(void*)py_linear_wgrad, METH_FASTCALL, "dy^T @ x in bf16"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
+    {"encode_saved", (PyCFunction)(void*)py_encode_saved, METH_FASTCALL, "encode, with what its backward needs"},
+    {"norm_dw", (PyCFunction)(void*)py_norm_dw, METH_FASTCALL, "gradient of a norm's weight from saved row factors"},
     {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},
     {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
     {"lora_fits", (PyCFunction)py_lora_fits, METH_O, "whether lora_stack takes these"},

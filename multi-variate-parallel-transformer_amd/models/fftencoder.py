@@ -74,10 +74,12 @@ class WaveEncoder(BrainEncoder):
 
     def _forward_autograd(self, x: Tensor) -> Tensor:
         pad = self._padded_k() - self.dwt_size
-        coeffs = self.block(x)                                                  # fp32, no gradient
-        normed = AG.rmsnorm(coeffs, self.ln.weight, 1e-5, out_dtype=torch.bfloat16)
         # whole 64-element k-blocks, as on the inference path: the zero columns contribute nothing
-        return AG.linear(torch.nn.functional.pad(normed, (0, pad)),
+        normed = AG.encoder_norm(x, self.ln.weight, self._padded_k(), 1e-5)
+        if normed is None:
+            coeffs = self.block(x)                                              # fp32, no gradient
+            normed = torch.nn.functional.pad(AG.rmsnorm(coeffs, self.ln.weight, 1e-5, out_dtype=torch.bfloat16), (0, pad))
+        return AG.linear(normed,
                          torch.nn.functional.pad(self.proj.weight.to(torch.bfloat16), (0, pad)))
 
     def _forward_fused(self, x: Tensor) -> Tensor:

@@ -147,6 +147,8 @@ def load_library() -> ctypes.CDLL:
     lib.mvpa_add3_rmsnorm_bf16.argtypes = [vp, vp, vp, vp, vp, vp, i64, i32, f32, vp]
     lib.mvpa_wavedec_db4.restype = ctypes.c_int
     lib.mvpa_wavedec_db4.argtypes = [vp, vp, i64, i32, i32, i32, i64, vp]
+    lib.mvpa_wavedec_db4_rmsnorm_fits.restype = ctypes.c_int
+    lib.mvpa_wavedec_db4_rmsnorm_fits.argtypes = [i32, i32, i32]
     if lib.mvpa_version() != 3:
         raise RuntimeError("libmvpa_hip ABI version mismatch")
     _lib = lib
@@ -575,6 +577,30 @@ def wavedec_db4_rmsnorm(x: torch.Tensor, weight: torch.Tensor, pitch: int, eps: 
         y[:, total:].zero_()
         rmsnorm(coeffs, weight, eps, out=y[:, :total])
     return _taken(y)
+
+
+@functools.lru_cache(maxsize=64)
+def _wavedec_row_fits(length: int) -> bool:
+    return load_library().mvpa_wavedec_db4_rmsnorm_fits(length, *_dwt_shape(length)) == 1
+
+
+def wavedec_fits(x: torch.Tensor) -> bool:
+    """Whether wavedec_db4_rmsnorm takes the rows x in one pass."""
+    return x.dim() == 2 and x.shape[0] > 0 and _wavedec_row_fits(x.shape[1])
+
+
+def wavedec_db4_rmsnorm_saved(x: torch.Tensor, weight: torch.Tensor, pitch: int, eps: float = 1e-5):
+    """(wavedec_db4_rmsnorm, the coefficients in fp32 [M, pitch], the factor of every row [M]) of rows that fit the one
+    pass (wavedec_fits)."""
+    levels, total = _dwt_shape(x.shape[1])
+    assert weight.numel() == total, "wavedec_db4_rmsnorm: one weight per coefficient"
+    return _taken((_ext or load_ext()).encode_saved(x, _as_f32_weight(weight), levels, total, pitch, eps))
+
+
+def norm_dw(x: torch.Tensor, inv: torch.Tensor, dy: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """The gradient of `weight` in y = x inv weight from that of y: fp32 rows x [M, pitch], bf16 dy [M, pitch], row
+    factors inv [M]; columns past the weight's are not looked at."""
+    return _taken((_ext or load_ext()).norm_dw(x, inv, dy, weight))
 
 
 def linear_norm_fused_supported(M: int, K: int, N: int) -> bool:

@@ -160,6 +160,35 @@ def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype=None) -> tor
     return mvpa_hip.rmsnorm(x, w, eps, out_dtype=out_dtype)
 
 
+class _EncoderNormFn(torch.autograd.Function):
+    """RMSNorm of the wavelet coefficients of signal rows, zeros past them up to whole blocks of the projection.  The transform has
+    no parameters and carries no gradient (models/fftencoder.py:80: no_grad)."""
+
+    @staticmethod
+    def forward(ctx, x, w, pitch, eps):
+        y, coeffs, inv = mvpa_hip.wavedec_db4_rmsnorm_saved(x, w, pitch, eps)
+        ctx.save_for_backward(coeffs, inv, w)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        coeffs, inv, w = ctx.saved_tensors
+        if not ctx.needs_input_grad[1]:
+            return None, None, None, None
+        if not torch.is_grad_enabled() and not _mapped(dy) and dy.dtype == torch.bfloat16:
+            return None, mvpa_hip.norm_dw(coeffs, inv, dy, w), None, None
+        n = w.shape[0]                                       # a backward that is differentiated itself, or mapped over
+        return None, (dy[:, :n].float() * coeffs[:, :n] * inv[:, None]).sum(0).to(w.dtype), None, None
+
+
+def encoder_norm(x: torch.Tensor, w: torch.Tensor, pitch: int, eps: float):
+    """[M, L] signal rows -> bf16 [M, pitch]: wavelet analysis, norm and zeros in one pass, or None where the rows are
+    too long for it, are none, or the weight is of another type."""
+    if not x.is_cuda or w.dtype not in (torch.float32, torch.bfloat16) or not mvpa_hip.wavedec_fits(x):
+        return None
+    return _EncoderNormFn.apply(x.detach().float(), w, pitch, eps)
+
+
 class _Add3RMSNormFn(torch.autograd.Function):
     """(s, RMSNorm(s) w) with s = a + b + c: the residual update of a block and the norm behind it."""
 

@@ -350,3 +350,36 @@ def test_operands_on_two_gpus_are_refused():
         mvpa_hip.lora_stack((((True,), here, here, here),), 1.0, there)
     with pytest.raises(RuntimeError):
         mvpa_hip.load_ext().linear_wgrad(here, there)
+
+
+# one wave a row and a workgroup a row, odd sizes of every level, rows at odd boundaries of 16 bytes (odd L); rows: one, fewer
+# than a wave's share, every group of rows and a remainder
+@pytest.mark.parametrize("L,M,wt", [(97, 1, torch.float32), (512, 131, torch.bfloat16), (1001, 33, torch.float32),
+                                    (2560, 2051, torch.bfloat16), (4095, 65, torch.bfloat16)])
+def test_encoder_norm(L, M, wt):
+    """Analysis and norm of a training pass against the two kernels, the weight's gradient against 64 bits."""
+    g = torch.Generator(device="cuda").manual_seed(L + M)
+    total = sum(mvpa_hip.dwt_sizes(L)[1])
+    pitch = (total + 63) // 64 * 64
+    x = torch.randn((M, L), generator=g, device="cuda")
+    w = (1 + 0.1 * torch.randn(total, generator=g, device="cuda")).to(wt).requires_grad_()
+    y = AG.encoder_norm(x, w, pitch, 1e-5)
+    coeffs = mvpa_hip.wavedec_db4(x)
+    ref = mvpa_hip.rmsnorm(coeffs, w.detach().float(), 1e-5, out=torch.empty(M, total, device="cuda"))
+    assert (y[:, total:] == 0).all()
+    assert ((y[:, :total].float() - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
+    dy = torch.randn((M, pitch), generator=g, device="cuda").bfloat16()
+    dw, = torch.autograd.grad(y, w, dy, retain_graph=True)
+    c = coeffs.double()
+    inv = (c.pow(2).mean(-1, keepdim=True) + 1e-5).rsqrt()
+    assert dw.dtype == wt
+    _close(dw, (dy[:, :total].double() * c * inv).sum(0), M * 4)
+    again, = torch.autograd.grad(y, w, dy.clone().requires_grad_(), create_graph=True)      # the general expression
+    assert ((again.double() - dw.double()).abs() <= 2.0 ** -7 * dw.double().abs() + 1e-3 * M ** 0.5).all()
+    both, = torch.autograd.grad(y, w, torch.stack([dy, 2 * dy]), is_grads_batched=True)
+    assert ((both[1].double() - 2 * again.double()).abs() <= 2.0 ** -7 * both[1].double().abs() + 1e-3 * M ** 0.5).all()
+
+
+def test_encoder_norm_of_rows_beyond_the_one_pass():
+    assert AG.encoder_norm(torch.zeros(2, 40000, device="cuda"), torch.ones(sum(mvpa_hip.dwt_sizes(40000)[1]), device="cuda"), 40960, 1e-5) is None
+    assert AG.encoder_norm(torch.zeros(0, 512, device="cuda"), torch.ones(550, device="cuda"), 576, 1e-5) is None
