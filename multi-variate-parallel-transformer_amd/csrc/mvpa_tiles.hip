@@ -4,7 +4,9 @@
 // columns: 18 of them on 256 CUs, 50 us for 2 GFLOP).  Here a workgroup is 32 * WM rows of x by 64 rows
 // of w, and a product with a long contraction and a narrow output is split over K as well.  The
 // time of such a product is the latency of its chain of k-blocks, so the operands come through a ring
-// of STAGES direct-to-LDS blocks of 64: STAGES - 1 blocks are in flight at any time.
+// of STAGES direct-to-LDS blocks of 64: STAGES - 1 blocks are in flight at any time, and the fragments of the next block are on
+// their way from LDS while this one is multiplied (with a block's fragments read where its products stand, a few
+// at a time: 32 rows of x, [768,2624] weights 9.8 -> 6.0 us, [2048,2048] 8.7 -> 5.8; 128 x 64 tiles 16.1 -> 13.6).
 //   4 waves.  WM = 4: a wave owns 32 rows of x and all 64 columns.  WM = 2 / 1: two / four waves share
 //   the rows and take 32 / 16 of every 64 k each, so that a wave always holds two 32 x 32 tiles (for the gated
 //   product: the gate and the up columns of an output).
@@ -80,38 +82,72 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
     for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
   const int nkb = kb1 - kb0;
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s)
+  for (int s = 0; s < STAGES; ++s)
     if (s < nkb) issue();
 
   constexpr int SL = 4 / G::KH;                     // 16-wide k-slices of a block per wave
+  struct frags { bf16x8 x[SL], w[SL][2]; };
   int frag[SL];
 #pragma unroll
   for (int s = 0; s < SL; ++s) frag[s] = ln * TL_ROWB + (((2 * (kh * SL + s) + hh) ^ ((ln >> 1) & 7)) << 4);
-  const unsigned char* st = lds;
-  for (int kb = 0; kb < nkb; ++kb) {
-    // block kb has landed once only the loads of the younger blocks are still out
-    const int younger = min(STAGES - 2, nkb - 1 - kb);
-    if (younger == STAGES - 2) wait_vmcnt_imm<(STAGES - 2) * G::LPW>();
-    else if (STAGES > 3 && younger == STAGES - 3) wait_vmcnt_imm<(STAGES > 3 ? STAGES - 3 : 0) * G::LPW>();
-    else if (STAGES > 4 && younger == STAGES - 4) wait_vmcnt_imm<(STAGES > 4 ? STAGES - 4 : 0) * G::LPW>();
-    else if (STAGES > 5 && younger == STAGES - 5) wait_vmcnt_imm<(STAGES > 5 ? STAGES - 5 : 0) * G::LPW>();
-    else wait_vmcnt_imm<0>();
-    lds_barrier();                                  // ... for every wave; and block kb - 1 is read by all
-    if (kb + STAGES - 1 < nkb) issue();
+  const unsigned char* st = lds;                    // the stage whose fragments are read next
+  auto read = [&](frags& f) {
     const unsigned char* xb = st + wm * 32 * TL_ROWB;
     const unsigned char* wb = st + G::BM * TL_ROWB;
-    bf16x8 xf[SL], wf[SL][2];
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
-      xf[s] = *(const bf16x8*)(xb + frag[s]);
+      f.x[s] = *(const bf16x8*)(xb + frag[s]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) wf[s][j] = *(const bf16x8*)(wb + j * 32 * TL_ROWB + frag[s]);
+      for (int j = 0; j < 2; ++j) f.w[s][j] = *(const bf16x8*)(wb + j * 32 * TL_ROWB + frag[s]);
     }
+    st = st + G::STAGE == lds + G::LDS ? lds : st + G::STAGE;
+  };
+  auto multiply = [&](const frags& f) {
 #pragma unroll
     for (int s = 0; s < SL; ++s)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[s][j], xf[s], acc[j], 0, 0, 0);
-    st = st + G::STAGE == lds + G::LDS ? lds : st + G::STAGE;
+      for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[s][j], f.x[s], acc[j], 0, 0, 0);
+  };
+  // One step: block kb's fragments are in registers.  Behind the barrier block kb + 1 has landed (only the loads of
+  // younger blocks are still out), and block kb is read by all: its stage takes block kb + STAGES.
+  auto step = [&](const frags& now, frags& next) {
+    wait_vmcnt_imm<(STAGES - 2) * G::LPW>();
+    lds_barrier();
+    issue();
+    read(next);
+    multiply(now);
+  };
+  frags fa, fb;
+  const int steady = max(nkb - STAGES, 0), last = min(STAGES, nkb) - 1;
+  if (last == STAGES - 1) wait_vmcnt_imm<(STAGES - 1) * G::LPW>();
+  else wait_vmcnt_imm<0>();
+  lds_barrier();
+  read(fa);
+  int kb = 0;
+  for (; kb + 1 < steady; kb += 2) {
+    step(fa, fb);
+    step(fb, fa);
+  }
+  if (kb < steady) {
+    step(fa, fb);
+    fa = fb;
+  }
+  if (last & 1) fb = fa;                            // what is left: an even number of blocks behind this one from fa, an odd from fb
+#pragma unroll
+  for (int r = STAGES - 1; r >= 0; --r) {
+    if (r > last) continue;
+    if (r > 0) {
+      // (r is a constant of every copy of the loop's body)
+      static_assert(STAGES <= 6, "waits below");
+      if (r == 5) wait_vmcnt_imm<4 * G::LPW>();
+      else if (r == 4) wait_vmcnt_imm<3 * G::LPW>();
+      else if (r == 3) wait_vmcnt_imm<2 * G::LPW>();
+      else if (r == 2) wait_vmcnt_imm<G::LPW>();
+      else wait_vmcnt_imm<0>();
+      lds_barrier();
+      read(r & 1 ? fa : fb);
+    }
+    multiply(r & 1 ? fb : fa);
   }
   // every wave's sums by rows of x, [k part][BM rows][64 columns] over the ring
   lds_barrier();
@@ -374,10 +410,21 @@ static int launch_dual_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, con
   return take_launch_status();
 }
 
+// The smallest tile that gives at most one workgroup a CU: what a product of few rows takes is its chain of blocks, and a
+// block of 32 rows of x is 12 KB, of 64 16, of 128 24.  With more workgroups than CUs the panels of w are read again instead.
+// [q/k/v | gate/up] of MVPFormer-S (74 columns of tiles), tiles of 32 / 64 / 128 rows, us: 32 rows 4.8 / 5.1 / 7.0, 64 4.8 /
+// 5.4 / 7.1, 100 6.1 / 5.4 / 7.9, 192 6.7 / 5.5 / 7.8, 256 8.7 / 7.7 / 7.6, 400 11.8 / 10.0 / 9.3; of the base model (240): 32
+// 15.0 / 14.8 / 16.2, 64 20.9 / 17.9 / 17.8, 100 26.6 / 22.7 / 19.2, 128 29.8 / 24.4 / 20.8.
+static int tile_rows(int64_t M, int64_t per_row_tile) {
+  if ((M + 31) / 32 * per_row_tile <= 256) return 32;
+  return (M + 63) / 64 * per_row_tile <= 256 ? 64 : 128;
+}
+
 int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,
                      const tile_out& out, const tile_gated& gated, const tile_norm& norm, hipStream_t s) {
-  if (M <= 32) return launch_dual_t<1, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
-  if (M <= 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  const int rows = tile_rows(M, (gated.w ? (gated.N + 31) / 32 : 0) + (w0 ? (N0 + TL_BN - 1) / TL_BN : 0));
+  if (rows == 32) return launch_dual_t<1, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  if (rows == 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (M <= 128) return launch_dual_t<4, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   return launch_dual_t<4, 3>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
 }
@@ -425,8 +472,11 @@ static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, 
 
 int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw,
                         float* P, const tile_split& splits, hipStream_t s) {
+  // As above, but that tiles of 32 rows are for 32 rows alone: the chains are a part's few blocks.  Tail of MVPFormer-S (12
+  // columns of tiles in up to 9 parts), tiles of 32 / 64 / 128 rows, us: 64 rows 4.3 / 4.3 / 5.3, 128 5.2 / 4.4 / 6.1, 192 7.2 / 5.8 /
+  // 5.7; of the base model (32 in 8): 64 12.9 / 10.4 / 10.5, 100 16.7 / 13.0 / 11.8, 128 18.3 / 14.2 / 12.8.
   if (M <= 32) return launch_partial_t<1, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
-  if (M <= 64) return launch_partial_t<2, 5>(x, M, K, ldx, w, N, ldw, P, splits, s);
+  if (tile_rows(M, (N + TL_BN - 1) / TL_BN * splits.total()) <= 64) return launch_partial_t<2, 5>(x, M, K, ldx, w, N, ldw, P, splits, s);
   if (M <= 128) return launch_partial_t<4, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
   return launch_partial_t<4, 3>(x, M, K, ldx, w, N, ldw, P, splits, s);
 }

@@ -86,6 +86,20 @@ def test_rows_left_to_a_last_tile(B, C, T):
     assert _rel(got, want) <= REL
 
 
+# tiles of 32 rows up to 96 of them, of 64 up to 192, of 128 beyond, with 2 and 5 blocks in the projections' chains
+@pytest.mark.parametrize("C,T", [(96, 1), (97, 1), (96, 2), (193, 1), (65, 3)], ids=str)
+@pytest.mark.parametrize("dims", [{}, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=1536)], ids=["D128", "D320"])
+def test_rows_either_side_of_a_tile_size(C, T, dims):
+    """The tile that [q/k/v | gate/up] and the tail product take by their rows, against the stack in 64 bits."""
+    model = _model(**{"n_inner": 2048, **dims})
+    x = torch.randn(1, T, C, model.embed_dim, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = model(inputs_embeds=x)
+    heads = dict(n_layer=2, n_head=dims.get("n_head", 2), n_head_kv=dims.get("n_head_kv", 1))
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, heads, None)
+    assert _rel(got, want) <= REL
+
+
 @pytest.mark.parametrize("C,T,inner", [(125, 4, 4032), (128, 4, 4032), (96, 4, 448), (77, 5, 448), (103, 5, 448)])
 def test_parts_of_the_tail_product_by_xcd(C, T, inner):
     """Four row tiles with x of the tail product up to and over 4 MB; three, four and five row tiles."""
