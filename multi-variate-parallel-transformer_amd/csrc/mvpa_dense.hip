@@ -1850,6 +1850,7 @@ extern "C" int mvpa_linear_bf16(const void* x, const void* w, void* y, int64_t M
   hipStream_t s = (hipStream_t)stream;
   const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
   bf16_t* yp = (bf16_t*)y;
+  if (epilogue == 0 && mvpa::tile_linear_pays(M, N, K, ldx, ldw, ldy, y)) return mvpa::launch_tile_linear(xp, M, K, ldx, wp, N, ldw, yp, ldy, s);
   // large tiles when there is enough work and rows can be fetched in whole 16-byte chunks;
   // the tile width is the one that needs the fewest (workgroup rounds x width) on 256 CUs
   if (M >= 512 && (K & 7) == 0 && (ldy & 3) == 0 && ((uintptr_t)y & 7) == 0) {

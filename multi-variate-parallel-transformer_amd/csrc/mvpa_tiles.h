@@ -41,6 +41,11 @@ struct tile_norm {
 int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,
                      const tile_out& out, const tile_gated& gated, const tile_norm& norm, hipStream_t s);
 
+// y = x w^T where the tiles are the faster ones (tile_linear_pays; operands 16-byte aligned): few enough of them.
+bool tile_linear_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, const void* y);
+int launch_tile_linear(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw, bf16_t* y,
+                       int64_t ldy, hipStream_t s);
+
 // How a contraction is cut: columns [0, Ka) of x into `a` runs of per_a k-blocks, the rest (all of it where
 // Ka is 0) into `b` runs of per_b.
 struct tile_split {

@@ -27,25 +27,25 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int TL_BN = 64, TL_BK = 64, TL_ROWB = TL_BK * 2;
 constexpr int TL_SUM = TL_BN * 4;                   // bytes of a row of sums: 16 chunks, XOR-swizzled by the row
 
-template <int WM, int STAGES>
+template <int WM, int STAGES, int CT = 2>           // CT: tiles of 32 columns of a wave
 struct tile_cfg {
-  static constexpr int BM = 32 * WM, KH = 4 / WM, LPW = WM + 2;      // 1 KiB loads per wave and block
+  static constexpr int BM = 32 * WM, CW = 2 / CT, KH = 4 / (WM * CW), LPW = WM + 2;      // LPW: 1 KiB loads per wave and block
   static constexpr int STAGE = (BM + TL_BN) * TL_ROWB;
   static constexpr int LDS = STAGES * STAGE;
-  static_assert(4 * 32 * TL_SUM <= LDS, "the sums of all waves fit the ring");
+  static_assert(WM * CW * KH == 4 && KH * BM * TL_SUM <= LDS, "four waves, and their sums fit the ring");
 };
 
 // The tile's products over k-blocks [kb0, kb1), left in LDS for tile_sum.  wrow(r): which row of W feeds row r of
 // the tile.
-template <int WM, int STAGES, typename WRow>
+template <int WM, int STAGES, int CT = 2, typename WRow>
 __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* __restrict__ X, int64_t ldx, int64_t m0,
                                              int64_t M, const bf16_t* __restrict__ W, int64_t ldw, WRow wrow,
                                              int kb0, int kb1) {
-  using G = tile_cfg<WM, STAGES>;
-  f32x16 acc[2];
+  using G = tile_cfg<WM, STAGES, CT>;
+  f32x16 acc[CT];
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave % WM, kh = wave / WM;
+  const int wm = wave % WM, wc = wave / WM % G::CW, kh = wave / (WM * G::CW);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))lds;
 
   // load i of a wave: rows (wave + 4i) * 8 .. + 7 of the block, x rows first (i < WM), then w rows
@@ -77,7 +77,7 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
   };
 
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < CT; ++j)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[j][r] = 0.f;
   const int nkb = kb1 - kb0;
@@ -86,19 +86,19 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
     if (s < nkb) issue();
 
   constexpr int SL = 4 / G::KH;                     // 16-wide k-slices of a block per wave
-  struct frags { bf16x8 x[SL], w[SL][2]; };
+  struct frags { bf16x8 x[SL], w[SL][CT]; };
   int frag[SL];
 #pragma unroll
   for (int s = 0; s < SL; ++s) frag[s] = ln * TL_ROWB + (((2 * (kh * SL + s) + hh) ^ ((ln >> 1) & 7)) << 4);
   const unsigned char* st = lds;                    // the stage whose fragments are read next
   auto read = [&](frags& f) {
     const unsigned char* xb = st + wm * 32 * TL_ROWB;
-    const unsigned char* wb = st + G::BM * TL_ROWB;
+    const unsigned char* wb = st + (G::BM + wc * 32) * TL_ROWB;
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
       f.x[s] = *(const bf16x8*)(xb + frag[s]);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) f.w[s][j] = *(const bf16x8*)(wb + j * 32 * TL_ROWB + frag[s]);
+      for (int j = 0; j < CT; ++j) f.w[s][j] = *(const bf16x8*)(wb + j * 32 * TL_ROWB + frag[s]);
     }
     st = st + G::STAGE == lds + G::LDS ? lds : st + G::STAGE;
   };
@@ -106,7 +106,7 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
 #pragma unroll
     for (int s = 0; s < SL; ++s)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[s][j], f.x[s], acc[j], 0, 0, 0);
+      for (int j = 0; j < CT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f.w[s][j], f.x[s], acc[j], 0, 0, 0);
   };
   // One step: block kb's fragments are in registers.  Behind the barrier block kb + 1 has landed (only the loads of
   // younger blocks are still out), and block kb is read by all: its stage takes block kb + STAGES.
@@ -153,10 +153,10 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
   lds_barrier();
   unsigned char* sums = lds + (kh * G::BM + wm * 32 + ln) * TL_SUM;
 #pragma unroll
-  for (int j = 0; j < 2; ++j)
+  for (int j = 0; j < CT; ++j)
 #pragma unroll
     for (int a4 = 0; a4 < 4; ++a4)
-      *(float4*)(sums + (((8 * j + 2 * a4 + hh) ^ (ln & 15)) << 4)) =
+      *(float4*)(sums + (((8 * (wc * CT + j) + 2 * a4 + hh) ^ (ln & 15)) << 4)) =
           make_float4(acc[j][a4 * 4], acc[j][a4 * 4 + 1], acc[j][a4 * 4 + 2], acc[j][a4 * 4 + 3]);
   lds_barrier();
 }
@@ -320,6 +320,29 @@ __global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restr
   });
 }
 
+// A product by itself: every output's sum is one chain over K, as in the large tiles (and the same bits)
+template <int WM, int STAGES, int CT>
+__global__ __launch_bounds__(256) void tile_linear_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+                                                          const bf16_t* __restrict__ W, int N, int64_t ldw, bf16_t* __restrict__ Y,
+                                                          int64_t ldy, int ct, int mt) {
+  using G = tile_cfg<WM, STAGES, CT>;
+  static_assert(G::KH == 1, "one chain");
+  extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
+  int col, row;
+  if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
+  const int64_t m0 = (int64_t)row * G::BM;
+  const int n0 = col * TL_BN, c = threadIdx.x & 7, n = n0 + c * 8;
+  tile_product<WM, STAGES, CT>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, 0, K / TL_BK);
+#pragma unroll
+  for (int i = 0; i < G::BM / 32; ++i) {
+    const int r = (threadIdx.x >> 3) + i * 32;
+    if (m0 + r >= M || n >= N) continue;
+    const float4 lo = tile_sum<G>(tl_lds, r, 2 * c), hi = tile_sum<G>(tl_lds, r, 2 * c + 1);
+    *(bf16x8*)(Y + (m0 + r) * ldy + n) = bf16x8{(__bf16)lo.x, (__bf16)lo.y, (__bf16)lo.z, (__bf16)lo.w,
+                                                (__bf16)hi.x, (__bf16)hi.y, (__bf16)hi.z, (__bf16)hi.w};
+  }
+}
+
 // One workgroup per row: the partial sums of a split-K tail product, the residual, one rounding, and
 // the RMSNorm that the next product wants, while the row is in registers (8 columns per lane and chunk).
 // Bound by the trip to the sums, which other XCDs have just written: all PARTS (the next of 4, 6, 8, 9 from their number; past
@@ -427,6 +450,33 @@ int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const b
   if (rows == 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (M <= 128) return launch_dual_t<4, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   return launch_dual_t<4, 3>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+}
+
+template <int WM, int STAGES, int CT>
+static int launch_linear_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw, bf16_t* y,
+                           int64_t ldy, hipStream_t s) {
+  using G = tile_cfg<WM, STAGES, CT>;
+  auto kern = tile_linear_kernel<WM, STAGES, CT>;
+  want_dynamic_lds((const void*)kern, G::LDS);
+  const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, y, ldy, ct, mt);
+  return take_launch_status();
+}
+
+// Where 256-row tiles leave most CUs without work, and below 512 rows, where they are not used.  us, large tiles (below 512 rows
+// the 128 x 128 ones) / these: [768,768] 130 rows 19.8 / 4.4, 525 13.7 / 5.2, 1600 14.0 / 7.4, 3000 (288 tiles) 14.3 / 12.0, 4096
+// (384) 14.6 / 14.9; [768,2624] 525 35.5 / 10.0, 3000 36.9 / 31.0, 4096 37.4 / 42.6; [2048,2048] 130 40.5 / 8.1, 1152 (288)
+// 28.2 / 18.0, 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1; [2048,576] 1152 11.3 / 8.2, 2048 11.4 / 12.0.
+bool tile_linear_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, const void* y) {
+  const int64_t ct = (N + TL_BN - 1) / TL_BN;
+  return M > 128 && K % TL_BK == 0 && N % 8 == 0 && ldy % 8 == 0 && ((uintptr_t)y & 15) == 0 && M < (1 << 20) && N < (1 << 20) &&
+         K < (1 << 30) && 128 * ldx < (1 << 30) && N * ldw < ((int64_t)1 << 31) && (M + 127) / 128 * ct <= 288;
+}
+
+int launch_tile_linear(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw, bf16_t* y,
+                       int64_t ldy, hipStream_t s) {
+  if ((M + 63) / 64 * ((N + TL_BN - 1) / TL_BN) <= 256) return launch_linear_t<2, 5, 1>(x, M, K, ldx, w, N, ldw, y, ldy, s);
+  return launch_linear_t<4, 3, 2>(x, M, K, ldx, w, N, ldw, y, ldy, s);
 }
 
 // Partial sums per output element: enough workgroups for every CU, about 4 k-blocks each or more, at most

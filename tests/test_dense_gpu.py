@@ -48,6 +48,24 @@ def test_linear_gated(M, N, K):
     assert (y.double() - ref).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 1e-5
 
 
+# one block, fewer blocks than the ring holds, as many, a few more and many; rows and columns either side of a tile; tiles of 64 rows
+# (525 x 768, 512 x 2048) and of 128 (576 x 2048, 1024 x 2048); N short of a whole tile
+@pytest.mark.parametrize("M,N,K", [(129, 8, 64), (192, 72, 128), (193, 64, 320), (525, 768, 384), (512, 2048, 192), (576, 2048, 64),
+                                   (577, 2040, 192), (1024, 2048, 256), (525, 768, 2624)])
+def test_linear_on_small_tiles(M, N, K):
+    """Few tiles of 256 rows: the product on smaller ones, into rows of an x with another pitch, against float64, and the same bits
+    as on large tiles (every sum is one chain over K there too)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    xw = torch.randn(M, K + 64, generator=g).bfloat16().cuda()
+    w = (torch.randn(N, K, generator=g) * 0.05).bfloat16().cuda()
+    x = xw[:, 32:32 + K]
+    y = mvpa_hip.linear(x, w)
+    ref = x.double() @ w.double().T
+    assert (y.double() - ref).abs().max().item() <= 2 ** -8 * ref.abs().max().item() + 1e-6
+    many = torch.cat([x, torch.zeros(289 * 128 // -(-N // 64), K, device="cuda", dtype=torch.bfloat16)])
+    assert K < 128 or torch.equal(mvpa_hip.linear(many, w)[:M], y)
+
+
 @pytest.mark.parametrize("M,N,K", [(1024, 768, 2496), (16384, 768, 2496), (600, 130, 96), (4096, 2048, 7680),
                                    (2000, 200, 160), (8192, 520, 256)])
 def test_linear_with_residual_in_the_epilogue(M, N, K):
