@@ -1,22 +1,23 @@
 // Weight gradients: dW[N,K] = dY[M,N]^T X[M,K] in bf16 with fp32 sums (the backward of layers/mvpa.py:354-359, 400
 // and of the MLP's projections, models/mvpformer.py:146).
 //
-// The output is small and the contraction long (MVPFormer-S, 6400 rows: 36 .. 162 tiles of 128 x 128 over 100
-// blocks of 64 rows), so the tiles alone do not fill 256 CUs: the rows are dealt over `splits` workgroups per
+// The output is small and the contraction long (MVPFormer-S, 6400 rows: 36 .. 162 tiles of 128 x 128 over 200
+// blocks of 32 rows), so the tiles alone do not fill 256 CUs: the rows are dealt over `splits` workgroups per
 // tile, fp32 partial tiles meet in a second kernel, or over two groups of waves of a workgroup that meet in LDS.  Both operands are contracted over their slow index: they go
-// straight from memory to LDS as they lie, [64 rows][128 columns], and both MFMA operands come out of transposing
-// LDS reads.  A group is 4 waves of 64 x 64 outputs (64 accumulator registers) on two 32 KiB stages, so that
-// two share a CU.  Per block of 64 rows one barrier, in front of its last quarter: that quarter's fragments
-// are in registers, the barrier publishes the next block and frees this one's stage for the block after next.
-// Bound by the fragment reads (one per product) and the tile requests: 44 us for [3456,768] over 6400 rows, 780 TFLOP/s, 55
-// with the partial tiles added up.
+// straight from memory to LDS as they lie, [32 rows][128 columns], and both MFMA operands come out of transposing
+// LDS reads.  A group is 4 waves of 64 x 64 outputs (64 accumulator registers) on five 16 KiB stages of 32 rows, so
+// that two share a CU and four blocks of each are on their way.  Per block one barrier, in front of its last half: that half's
+// fragments are in registers, the barrier publishes the next block and frees this one's stage for the block five further on.
+// Bound by the fragment reads (one per product).  With two stages of 64 rows, one block on its way, and an address formed by
+// every lane for every request, both launches / now, us: [3456,768] over 6400 rows 56.1 / 53.5, 25600 175 / 165; [768,2624] 52.1 /
+// 45.7, 161 / 129; [768,768] 21.9 / 21.8, 60 / 49.
 #include "mvpa_mfma_tools.h"
 
 namespace mvpa {
 namespace wgrad {
 
-constexpr int TILE = 128, KB = 64;               // outputs of a tile each way, rows of a block
-constexpr int ROWB = TILE * 2, STAGE = 2 * KB * ROWB;
+constexpr int TILE = 128, KB = 32;               // outputs of a tile each way, rows of a block
+constexpr int ROWB = TILE * 2, STAGE = 2 * KB * ROWB, STAGES = 5;
 constexpr int LOADS = STAGE / 1024 / 4;          // 1 KiB requests per wave and block
 
 struct args {
@@ -26,7 +27,7 @@ struct args {
   int32_t M, N, K, tiles_k, splits, blocks;      // blocks of rows in all
 };
 
-// fragment of a [64][128] tile contracted over its rows: column 32 c + lane's, rows 16 s + 8 rd + 4 hh + e
+// fragment of a [32][128] tile contracted over its rows: column 32 c + lane's, rows 16 s + 8 rd + 4 hh + e
 __device__ inline bf16x8 frag(const unsigned char* p, int s) {
   const bf16x4 lo = el_bf16::read_tr(p + 16 * s * ROWB), hi = el_bf16::read_tr(p + (16 * s + 8) * ROWB);
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
@@ -37,7 +38,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char all_stages[];
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3, group = __builtin_amdgcn_readfirstlane(tid >> 8);
-  unsigned char* const smem = all_stages + group * 2 * STAGE;
+  unsigned char* const smem = all_stages + group * STAGES * STAGE;
   // ids equal mod 8 run on one XCD: it gets neighbouring tiles of one share of the rows, which read the same
   // rows at about the same time
   const int total = gridDim.x, per = total / 8, more = total % 8, xcd = blockIdx.x & 7;
@@ -49,17 +50,33 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
   const int64_t m_end = min((int64_t)last * KB, (int64_t)a.M);
   auto row_of = [&](int kb) { return (int64_t)(first + group + kb * GROUPS) * KB; };
 
-  // request i of a wave: rows 4 (wave + 4 (i & 3)) .. of dY (i < 4) or X; lane: row lane / 16, chunk lane % 16
+  // requests of a wave: rows 4 wave + 16 i .. of dY and of X; lane: row lane / 16, chunk lane % 16
   const int row_l = lane >> 4, chunk = ((lane & 15) ^ swz_v<TILE>(row_l)) * 8;
-  const bf16_t* dy = a.dy + min(n0 + chunk, a.N - 8);           // columns past the end: any, their outputs are not stored
-  const bf16_t* x = a.x + min(k0 + chunk, a.K - 8);
+  // columns past the end: any, their outputs are not stored
+  const uint32_t col_y = (uint32_t)min(n0 + chunk, a.N - 8), col_x = (uint32_t)min(k0 + chunk, a.K - 8);
+  const uint32_t off_y = (uint32_t)(row_l * (int)a.ldy + col_y) * 2, off_x = (uint32_t)(row_l * (int)a.ldx + col_x) * 2;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))smem;
+  // rows of a block that is whole: a uniform base and the lane's own offset, which does not change (addresses formed per
+  // lane cost as many vector cycles as the products)
   auto request = [&](int kb, int stage) {
+    const int64_t m0 = row_of(kb) + 4 * wave;
+    const uint32_t dst = lds0 + stage * STAGE + 4 * wave * ROWB;
+    if (row_of(kb) + KB <= m_end) {
+      const bf16_t *y = a.dy + m0 * a.ldy, *x = a.x + m0 * a.ldx;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-      const int r = 4 * (wave + 4 * (i & 3));
-      const int64_t m = min(row_of(kb) + r + row_l, m_end - 1);
-      load_to_lds_16(i < LOADS / 2 ? dy + m * a.ldy : x + m * a.ldx, lds0 + stage * STAGE + (i < LOADS / 2 ? 0 : STAGE / 2) + r * ROWB);
+      for (int i = 0; i < LOADS / 2; ++i) {
+        load_to_lds_16(y + (int64_t)(16 * i) * a.ldy, off_y, dst + 16 * i * ROWB);
+        load_to_lds_16(x + (int64_t)(16 * i) * a.ldx, off_x, dst + STAGE / 2 + 16 * i * ROWB);
+      }
+    } else {                                     // the last row again where there are no more
+      const int64_t m1 = min(m0, m_end - 1);
+      const bf16_t *y = a.dy + m1 * a.ldy, *x = a.x + m1 * a.ldx;
+#pragma unroll
+      for (int i = 0; i < LOADS / 2; ++i) {
+        const int r = (int)(min(m0 + 16 * i + row_l, m_end - 1) - m1);
+        load_to_lds_16(y, (uint32_t)(r * (int)a.ldy + col_y) * 2, dst + 16 * i * ROWB);
+        load_to_lds_16(x, (uint32_t)(r * (int)a.ldx + col_x) * 2, dst + STAGE / 2 + 16 * i * ROWB);
+      }
     }
   };
   // a block that reaches past the last row: zeros there, in what this wave has requested itself
@@ -67,7 +84,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
     if (row_of(kb) + KB <= m_end) return;
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
-      const int r = 4 * (wave + 4 * (i & 3)) + row_l;
+      const int r = 4 * wave + 16 * (i % (LOADS / 2)) + row_l;
       if (row_of(kb) + r >= m_end)
         *(u32x4*)(smem + stage * STAGE + (i < LOADS / 2 ? 0 : STAGE / 2) + r * ROWB + (lane & 15) * 16) = u32x4{0u, 0u, 0u, 0u};
     }
@@ -89,13 +106,11 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
 #pragma unroll
       for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
-  request(0, 0);
-  if (count > 1) {
-    request(1, 1);
-    wait_vmcnt_imm<LOADS>();
-  } else {
-    wait_vmcnt_imm<0>();
-  }
+#pragma unroll
+  for (int b = 0; b < STAGES; ++b)
+    if (b < count) request(b, b);
+  if (count >= STAGES) wait_vmcnt_imm<(STAGES - 1) * LOADS>();
+  else wait_vmcnt_imm<0>();
   cut(0, 0);
   lds_barrier();
   bf16x8 fa[2], fb[2];
@@ -104,9 +119,10 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
     fa[c] = frag(pa[c], 0);
     fb[c] = frag(pb[c], 0);
   }
+  int stage = 0;
 #pragma unroll 1
   for (int kb = 0; kb < count; ++kb) {
-    const int st = (kb & 1) * STAGE;
+    const int st = stage * STAGE, next = stage + 1 == STAGES ? 0 : stage + 1;
 #pragma unroll
     for (int s = 0; s < KB / 16; ++s) {
       bf16x8 na[2], nb[2];
@@ -117,15 +133,16 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
           nb[c] = frag(pb[c] + st, s + 1);
         }
       } else {
-        wait_vmcnt_imm<0>();                     // block kb + 1, requested a block ago
-        if (kb + 1 < count) cut(kb + 1, (kb + 1) & 1);
+        // block kb + 1, requested STAGES - 1 blocks ago: younger ones stay out while there are STAGES - 2 of them
+        if (kb + STAGES <= count) wait_vmcnt_imm<(STAGES - 2) * LOADS>();
+        else wait_vmcnt_imm<0>();
+        if (kb + 1 < count) cut(kb + 1, next);
         lds_barrier();
-        if (kb + 2 < count) request(kb + 2, kb & 1);
-        const int next = STAGE - st;             // past the end: what lies there, for nobody
+        if (kb + STAGES < count) request(kb + STAGES, stage);
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          na[c] = frag(pa[c] + next, 0);
-          nb[c] = frag(pb[c] + next, 0);
+        for (int c = 0; c < 2; ++c) {            // past the end: what lies there, for nobody
+          na[c] = frag(pa[c] + next * STAGE, 0);
+          nb[c] = frag(pb[c] + next * STAGE, 0);
         }
       }
 #pragma unroll
@@ -138,6 +155,7 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
         fb[c] = nb[c];
       }
     }
+    stage = next;
   }
   if (GROUPS == 2) {                             // the second group's sums to the first, 64 KiB over the first's stages
     __syncthreads();
@@ -186,9 +204,9 @@ __global__ __launch_bounds__(256) void linear_wgrad_reduce_kernel(const float* _
 
 static int tiles_of(int64_t N, int64_t K) { return (int)((N + TILE - 1) / TILE * ((K + TILE - 1) / TILE)); }
 
-// How the rows are dealt, by what a launch was seen to take: a group of 4 waves 1.27 us a block where two share a
+// How the rows are dealt, by what a launch was seen to take: a group of 4 waves 0.6 us a block where two share a
 // CU, partial results 2 x 4 bytes an output and share at 4.8 TB/s.  Both launches over 6400 rows, eight sets of them in
-// turn, us (vendor library): [3456,768] 55 (69), [768,1728] 36 (50), [1280,768] 27 (41), [768,768] 22 (39).  Pairs of groups
+// turn, us (vendor library): [3456,768] 53 (73), [768,1728] 32 (49), [1280,768] 26 (42), [768,768] 22 (39).  Pairs of groups
 // took 6 to 8 us off the last three.
 struct plan {
   int groups, splits;
@@ -200,7 +218,7 @@ static plan plan_of(int64_t M, int64_t N, int64_t K) {
   for (int groups = 1; groups <= 2; ++groups)
     for (int s = 1; s <= 32 && (s == 1 || (int64_t)s * groups <= blocks); ++s) {
       const int64_t slots = 512 / groups, rounds = (tiles * s + slots - 1) / slots, each = (blocks + s * groups - 1) / (s * groups);
-      const double us = rounds * each * 1.27 + (s > 1 ? 3.0 + 8e-6 * s * N * K / 4.8 : 0.0);
+      const double us = rounds * each * 0.6 + (s > 1 ? 3.0 + 8e-6 * s * N * K / 4.8 : 0.0);
       if (us < best_us) {
         best_us = us;
         best = {groups, s};
@@ -225,6 +243,7 @@ extern "C" int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, i
   if (!dy || !x || !dw) return MVPA_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || N > (1 << 20) || K > (1 << 20) || M > ((int64_t)1 << 30) || lddy < N || ldx < K || lddw < K)
     return MVPA_ERR_SHAPE;
+  if (lddy > (1 << 26) || ldx > (1 << 26)) return MVPA_ERR_UNSUPPORTED;      // 32-bit offsets from a block's first row
   if ((N | K | lddy | ldx | lddw) % 8 != 0 || (((uintptr_t)dy | (uintptr_t)x | (uintptr_t)dw | (uintptr_t)ws) & 15)) return MVPA_ERR_ALIGN;
   const wgrad::plan p = wgrad::plan_of(M, N, K);
   const size_t need = p.splits == 1 ? 0 : (size_t)p.splits * N * K * sizeof(float);
@@ -234,7 +253,7 @@ extern "C" int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, i
   hipStream_t s = (hipStream_t)stream;
   auto kern = p.groups == 2 ? p.splits > 1 ? wgrad::linear_wgrad_kernel<2, true> : wgrad::linear_wgrad_kernel<2, false>
                             : p.splits > 1 ? wgrad::linear_wgrad_kernel<1, true> : wgrad::linear_wgrad_kernel<1, false>;
-  const int lds = 2 * wgrad::STAGE * p.groups;
+  const int lds = wgrad::STAGES * wgrad::STAGE * p.groups;
   want_dynamic_lds((const void*)kern, lds);
   MVPA_LAUNCH(kern, dim3((unsigned)(wgrad::tiles_of(N, K) * p.splits)), dim3(256 * p.groups), lds, s, a);
   if (p.splits > 1)

@@ -283,9 +283,9 @@ def test_stacked_weights_differentiate_twice():
     assert ((grad.double() - ref).norm() / ref.norm()).item() <= 3e-2
 
 
-# rows around the 64 of a block and the shares; outputs around tiles of 128, the smallest ones, operands with a row
+# rows around the 32 of a block, the five blocks of the ring and the shares; outputs around tiles of 128, the smallest ones, operands with a row
 # pitch; one share, several, one and two groups of waves
-@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (63, 128, 128), (64, 136, 120), (65, 8, 264), (129, 256, 1024), (700, 1280, 768),
+@pytest.mark.parametrize("m,n,k", [(1, 8, 8), (31, 8, 8), (63, 128, 128), (64, 136, 120), (65, 8, 264), (160, 8, 8), (161, 1664, 1664), (193, 136, 8), (129, 256, 1024), (700, 1280, 768),
                                    (6400, 768, 1728), (2561, 3456, 768), (1000, 2048, 2056), (20000, 8, 16)])
 def test_weight_gradient(m, n, k):
     g = torch.Generator(device="cuda").manual_seed(m + n)
