@@ -118,17 +118,22 @@ extern "C" int mvpa_forward(const mvpa_fwd_args* a, void* stream) {
     // AUTO: the specialised builds where they are the faster ones.
     // Launches that leave the chip idle: the build whose waves split the keys of a query tile.  Its time follows the
     // number of its workgroups (B H T and the query tiles of a step), the other kernels' is one chain over the steps
-    // until they fill the chip, so the line lies where the two meet (us, general : this).  Up to 32 channels,
-    // T 25 by B H 12 / 24 / 48 / 64: 23.5 : 10.0, 23.7 : 12.8, 24.1 : 21.6, 24.2 : 26.9; T 32 at 48 / 64 27.9 : 24.0, 28.1 :
-    // 32.2; T 64 at 24 / 48 51.5 : 33.1, 51.8 : 58.1; T 110 at 16 / 24 81.6 : 67.9, 82.4 : 97.9; T 200 at 12 / 16 149 : 124,
-    // 150 : 165.  33..64 channels, by workgroups, T 12 at 576 / 1152 17.3 : 13.5, 19.1 : 22.3; T 16 at 768 19.1 : 16.3; T 25
+    // until they fill the chip, so the line lies where the two meet (us, general : this).  Up to 32 channels and 64, by B H:
+    // T 25 at 12 / 24 / 48 / 64 23.5 : 10.0, 23.7 : 12.8, 24.1 : 21.6, 24.2 : 26.9; T 32 at 48 / 64 27.9 : 24.0, 28.1 :
+    // 32.2; T 64 at 12 / 24 / 48 50.1 : 19.1, 50.5 : 33.8, 51.8 : 58.1.  From T 80 on the general kernel's last step is no chain of
+    // one wave, and tables of more than 64 rows leave this one a workgroup a CU: T 80 at 12 / 24 41.4 : 33.7, 42.5 : 64.7; T 96 at
+    // 12 45.8 : 43.0; T 110 at 16 51.9 : 68.4; T 160 at 12 67.4 : 87.2; T 200 at 8 80.6 : 85.6; T 300 at 4 114 : 83.9; T 500
+    // at 4 181 : 197; head size 32 T 100 at 16 35.0 : 32.9, T 200 at 8 57 : 47, T 250 at 8 68.4 : 66.6, T 500 at 4 122 : 160.
+    // 33..64 channels, by workgroups, T 12 at 576 / 1152 17.3 : 13.5, 19.1 : 22.3; T 16 at 768 19.1 : 16.3; T 25
     // at 600 / 800 / 1200 23.2 : 16.9, 23.6 : 21.6, 25.9 : 26.7; T 40 at 960 29.5 : 35.4; Dh 32 at 768 / 1600 18.1 : 13.5,
-    // 24.8 : 26.8.  Head size 128 has one workgroup per CU (C21 T25 H16 35 : 25).
+    // 24.8 : 26.8.  Head size 128 has one workgroup per CU, the general kernel two from T 32: C21 H16 T 25 36 : 20, T 48 45 : 36,
+    // T 64 51 : 50, T 96 74 : 84, T 128 89 : 123; H24 T 32 37 : 30, T 64 61 : 70.
     if (!(a->flags & MVPA_FLAG_LAST_STEP) && a->C <= (a->Dh == 128 ? 32 : 64) && mvpa_wave_supported(a)) {
       const int64_t wgs = (int64_t)a->B * a->H * ((a->C + 31) / 32) * a->T, T = a->T;
       int64_t most = 512;
-      if (a->Dh == 128) most = T <= 128 && 24 * T > most ? 24 * T : most;
+      if (a->Dh == 128) most = T >= 32 ? 1024 : 24 * T > most ? 24 * T : most;
       else if (a->C > 32) most = T <= 32 ? 768 : most;
+      else if (T >= (a->Dh == 32 ? 257 : 80)) most = 1200;
       else if (48 * T > most) most = 48 * T < 2048 ? 48 * T : 2048;
       if (wgs <= most) return mvpa_launch_wave(a, st);
     }

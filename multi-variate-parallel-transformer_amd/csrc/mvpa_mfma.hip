@@ -56,7 +56,19 @@ struct Cfg {
   static constexpr int STAGE_BYTES = 2 * TILE_BYTES;         // K tile then V tile
   static constexpr int RING_BYTES = STAGES * STAGE_BYTES;
   static constexpr int STB_BYTES = NW * 32 * 32 * 4;
-  static constexpr int MAIN_BYTES = RING_BYTES + STB_BYTES;
+  // who takes the last time step, which keeps the content term for every key step: two pairs of waves in turn (SPLIT), or
+  // every wave by itself on a stage of its own (SOLO); see the kernel
+  static constexpr bool SPLIT = TQW == 2 && STAGES == 4 && KH == 1;
+  static constexpr bool SOLO = WPT == 1 && TQW > 2 && STAGES == 4;
+  static constexpr int STB_AT = SOLO && NW > STAGES ? NW * STAGE_BYTES : RING_BYTES;   // the slabs lie behind all stages
+  static constexpr int MAIN_BYTES = STB_AT + STB_BYTES;
+  // (of short sequences the last step is hardly longer than the others, and its own workgroup is one more: B8 H16 C30 T16 Dh128
+  // 52 -> 59 us, B4 T24 43 -> 50, B6 C25 T32 92 -> 87; B4 H12 C21 T64 Dh64 53 -> 55)
+  static constexpr int SOLO_T = DH == 128 ? 32 : 80;
+  __host__ __device__ static constexpr bool solo(int T) { return SOLO && T >= SOLO_T; }
+  __host__ __device__ static constexpr int time_tiles(int T) {
+    return SPLIT ? 1 + T / 2 : solo(T) ? 1 + (T - 1 + TQW - 1) / TQW : (T + TQW - 1) / TQW;
+  }
   static constexpr int SETUP_BYTES = NW * CP * 32 * 4;
   static constexpr int LDS_BYTES = MAIN_BYTES > SETUP_BYTES ? MAIN_BYTES : SETUP_BYTES;
   // the set-up scratch fits behind the stages of the prologue tiles
@@ -74,7 +86,7 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
   using G = Cfg<DH, NCT, NW, STAGES, KH>;
   constexpr int CP = G::CP, KS = G::KS, MT = G::MT, ROWB = G::ROWB, CHUNKS = G::CHUNKS;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
-  float* Stb_all = (float*)(smem_raw + G::RING_BYTES);          // [NW][32][32]
+  float* Stb_all = (float*)(smem_raw + G::STB_AT);              // [NW][32][32]
   // [NW][CP][32] set-up scratch; aliases the ring (and the slabs), see EARLY
   float* setup_all = (float*)(smem_raw + (G::EARLY ? (STAGES - 1) * G::STAGE_BYTES : 0));
 
@@ -110,8 +122,13 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
   // barrier, one pair of waves takes the even and the other the odd one at the same time, and the
   // two partial soft-max states are merged through LDS at the end.  That workgroup is the critical
   // path of a launch (content term at every key step), and this halves it.
-  constexpr bool SPLIT = G::TQW == 2 && STAGES == 4 && KH == 1;
-  const int nt = SPLIT ? 1 + T_ / 2 : (T_ + G::TQW - 1) / G::TQW;
+  // SOLO (a wave per query time step): the last time step has a workgroup of its own as well, whose waves take every NW-th
+  // key step each, load them into a stage of their own and meet in the merge alone.  As one wave's chain it was what a launch
+  // waited for: B1 H4 C5 T256 Dh32 137 -> 36 us, B1 H16 C19 T239 Dh64 174 -> 119, C21 T200 Dh128 280 -> 254 (-> 168 with two
+  // workgroups a CU), B8 H16 C30 T100 Dh64 266 -> 248.
+  constexpr bool SPLIT = G::SPLIT;
+  const bool solo = G::solo(T_);
+  const int nt = G::time_tiles(T_);
   const int nbh = a.B * a.H;
   // MVPA_FLAG_LAST_STEP: only the workgroup of the last time step runs, one per (b, h); q, o and
   // lse are indexed by channel alone
@@ -129,13 +146,15 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
   const int b = bh / a.H, h = bh % a.H;
   const int g = h / (a.H / a.Hkv);
   const bool split_last = SPLIT && tile == nt - 1;
+  const bool alone = (SPLIT || solo) && tile == nt - 1;            // the last time step's own workgroup
+  const bool solo_last = G::SOLO && solo && alone && has_content;             // (far steps all of them without the content term)
   const int par = wave / G::WPT;                   // split_last: parity of this wave's key steps
   const int kh = KH > 1 ? (wave / G::QT) % KH : 0; // the part of the keys this wave works on
   const int key0 = kh * (NCT * 32);                // its first key channel
   const int key_off = key0 * G::ROWB;              // ... as a byte offset into a K or V tile
-  const int tq0 = split_last ? T_ - 1 : tile * G::TQW;
-  const int tq_hi = split_last ? T_ - 1 : min(T_ - 1 - (SPLIT ? 1 : 0), tq0 + G::TQW - 1);
-  const int tq = split_last ? T_ - 1 : tq0 + wave / G::WPT;
+  const int tq0 = alone ? T_ - 1 : tile * G::TQW;
+  const int tq_hi = alone ? T_ - 1 : min(T_ - 1 - (SPLIT || solo ? 1 : 0), tq0 + G::TQW - 1);
+  const int tq = split_last || solo_last ? T_ - 1 : tq0 + wave / G::WPT;
   const bool active = tq <= tq_hi && (!last_only || tq == T_ - 1);
   const int cq = (wave % G::QT) * 32 + ln;         // this lane's query channel
   const bool qok = active && cq < C_;
@@ -225,7 +244,7 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
   // prologue leaves alone (the last stage and the time-bias slabs, both first written after the
   // first barrier of the key loop) the tiles are requested right away, so that their round trip
   // overlaps the set-up instead of following it.
-  if (G::EARLY) {
+  if (G::EARLY && !solo_last) {
     if (SLAB_LDS && slab_lds) issue_rows(0);
 #pragma unroll
     for (int s = 0; s < STAGES - 1; ++s)
@@ -367,7 +386,7 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[mt][i] = 0.f;
 
-  if (!G::EARLY) {
+  if (!G::EARLY && !solo_last) {
     lds_barrier();           // the set-up scratch aliases the stages the prologue fills
     if (SLAB_LDS && slab_lds) issue_rows(0);
 #pragma unroll
@@ -632,6 +651,34 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
     l_run += ls;
   };
 
+  // =========================== last time step, a wave by itself ==============================
+  if (solo_last) {
+    unsigned char* own = smem_raw + wave * G::STAGE_BYTES;
+    auto issue_own = [&](int tk) {
+      const bf16_t* ksrc = kbase + (int64_t)tk * C_ * a.k_stride_n;
+      const bf16_t* vsrc = vbase + (int64_t)tk * C_ * a.v_stride_n;
+      const uint32_t dst = ring_lds + wave * G::STAGE_BYTES;
+#pragma unroll
+      for (int li = 0; li < G::WLOADS; ++li) {
+        const int pc = li * 64 + lane, row = pc / CHUNKS, phys = pc % CHUNKS, rowc = min(row, C_ - 1);
+        load_to_lds_16(ksrc, (uint32_t)(rowc * (int)a.k_stride_n + ((phys ^ swz_k<DH>(row)) << 3)) * 2u, dst + li * 1024);
+        load_to_lds_16(vsrc, (uint32_t)(rowc * (int)a.v_stride_n + ((phys ^ swz_v<DH>(row)) << 3)) * 2u, dst + G::TILE_BYTES + li * 1024);
+      }
+    };
+    lds_barrier();                                 // everybody is done with the set-up scratch
+    int slab = -1;
+    if (wave < T_) issue_own(wave);
+    for (int tk = wave; tk < T_; tk += NW) {
+      if (tk >> 5 != slab) {
+        slab = tk >> 5;
+        time_slab(slab << 5, false);
+      }
+      wait_vmcnt_imm<0>();
+      near_step(own, tk);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");           // the stage is read
+      if (tk + NW < T_) issue_own(tk + NW);
+    }
+  } else
   // =========================== split last time step: two key steps per barrier ===============
   // Tile t lives in stage t % 4.  The prologue has tiles 0..2 in flight; at the barrier of pair k
   // the stages of pair k-1 are free and receive pair k+1 (tile 3 alone at k = 0), which then has
@@ -756,7 +803,33 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
   }   // !split_last
 
   // =========================== epilogue ===========================
-  if (split_last || KH > 1) {
+  if (solo_last) {
+    lds_barrier();                                 // every wave is done with its stage and slab
+    constexpr int SLOT = (2 + MT * 16) * 64;
+    static_assert(!G::SOLO || (NW - 1) * SLOT * 4 <= G::LDS_BYTES, "merge buffer");
+    float* mb = (float*)smem_raw + lane;
+    if (wave > 0) {
+      float* w = mb + (wave - 1) * SLOT;
+      w[0] = m_run;
+      w[64] = l_run;
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) w[(2 + mt * 16 + i) * 64] = acc[mt][i];
+    }
+    lds_barrier();
+    if (wave > 0) return;
+    for (int p = 0; p < NW - 1; ++p) {
+      const float* w = mb + p * SLOT;
+      const float m = fmaxf(m_run, w[0]), a0 = fast_exp2(m_run - m), a1 = fast_exp2(w[0] - m);
+      m_run = m;
+      l_run = a0 * l_run + a1 * w[64];
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[mt][i] = a0 * acc[mt][i] + a1 * w[(2 + mt * 16 + i) * 64];
+    }
+  } else if (split_last || KH > 1) {
     // two waves hold partial soft-max states of the same queries (split last time step: even and
     // odd key steps; KH = 2: the two parts of the key channels): the second one's m, l and
     // accumulator tiles go through LDS into the first one's
@@ -891,7 +964,7 @@ static int launch_one(const mvpa_fwd_args* a, hipStream_t stream) {
   auto kern = (n_split > 1 || ring) ? mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, true, E>
                           : mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, false, E>;
   mvpa::want_dynamic_lds((const void*)kern, (int)G::LDS_BYTES);
-  const int nt = (G::TQW == 2 && STAGES == 4 && KH == 1) ? 1 + a->T / 2 : (a->T + G::TQW - 1) / G::TQW;   // as in the kernel
+  const int nt = G::time_tiles(a->T);
   dim3 grid((unsigned)((last ? n_split : nt) * a->B * a->H));
   MVPA_LAUNCH(kern, grid, dim3(G::THREADS), G::LDS_BYTES, stream, *a);
   if (n_split > 1) launch_merge<E>(a, stream);
@@ -966,6 +1039,10 @@ int mvpa_launch_mfma(const mvpa_fwd_args* a, hipStream_t stream) {
       // (4 query tiles x 2 key parts), two waves per SIMD
       return launch_cfg<64, 2, 8, 3, 1, 2>(a, stream);
     case 128:
+      // two workgroups per CU (2 x 80 KiB, 50 to 80 registers spilled in the slabs) where the far steps are many: B3 H16 C19 T511
+      // 3931 -> 2065 us, B8 C32 T128 966 -> 643, B8 C25 T64 329 -> 237, T32 127 -> 107, but B4 C30 T24 43 -> 74 and
+      // B8 T16 52 -> 66
+      if (nct == 1 && a->T >= 32) return launch_cfg<128, 1, 4, 4, 2>(a, stream);
       if (nct == 1) return launch_cfg<128, 1, 4, 4>(a, stream);
       if (nct == 2) return launch_cfg<128, 2, 4, 3>(a, stream);
       // key-run (decoding) launches of 97..128 channels: the keys of a step in two parts, 8 waves,

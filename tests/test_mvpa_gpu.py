@@ -1,5 +1,5 @@
 """GPU parity of the fused MVPA forward (through the C ABI) against the CPU oracle."""
-import math
+import copy
 
 import pytest
 import torch
@@ -286,6 +286,47 @@ def test_small_launches_of_the_default_selector(cfg, dtype):
         o = out.float().cpu()
         assert (o - ref.float()).abs().max().item() <= FP16_MAX_ABS and _rel_l2(o, ref.float()) <= FP16_REL_L2
     assert (lse.cpu().double() - ref_lse).abs().max().item() <= (3e-2 if dtype == torch.bfloat16 else FP16_LSE)
+
+
+# either side of the lengths from which the last time step has a workgroup of its own (32 at head size 128, 80 below), fewer and
+# more steps than a wave's share, the slab's 32 steps, a last tile of one query step, every channel but one absent
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("cfg", [
+    dict(B=1, C=32, T=31, H=2, Dh=128), dict(B=1, C=1, T=32, H=2, Hkv=1, Dh=128), dict(B=2, C=21, T=33, H=2, Dh=128, validity=True),
+    dict(B=1, C=17, T=100, H=2, Dh=128), dict(B=1, C=32, T=79, H=2, Dh=64), dict(B=2, C=19, T=80, H=2, Hkv=1, Dh=64, validity=True),
+    dict(B=1, C=32, T=89, H=2, Dh=64), dict(B=1, C=5, T=129, H=2, Dh=64), dict(B=1, C=30, T=97, H=2, Dh=32, validity=True),
+], ids=lambda c: "C{C}T{T}D{Dh}".format(**c))
+def test_last_step_on_a_workgroup_of_its_own(cfg, dtype):
+    """Up to 32 channels on the tiled kernel: every row and lse against the oracle."""
+    inp = make_mvpa_inputs(seed=29, table_std=0.3, qkv_unit=True, **cfg).round_to(dtype)
+    out, lse = _gpu(inp, dtype, kernel=mvpa_hip.KERNEL_MFMA, return_lse=True)
+    ref, ref_lse = _oracle(inp, return_lse=True)
+    if dtype == torch.bfloat16:
+        _check_bf16(out, ref)
+    else:
+        o = out.float().cpu()
+        assert (o - ref.float()).abs().max().item() <= FP16_MAX_ABS and _rel_l2(o, ref.float()) <= FP16_REL_L2
+    assert (lse.cpu().double() - ref_lse).abs().max().item() <= (3e-2 if dtype == torch.bfloat16 else FP16_LSE)
+
+
+@pytest.mark.parametrize("kw", [dict(content=False), dict(time_bias=False), dict(chan_bias=False), dict(window=0), dict(window=200),
+                                dict(fp8_qk=True)], ids=lambda k: "-".join("%s%s" % i for i in k.items()))
+@pytest.mark.parametrize("dh", [64, 128])
+def test_last_step_on_a_workgroup_of_its_own_flags(kw, dh):
+    inp = make_mvpa_inputs(seed=31, B=1, C=13, T=90, H=2, Dh=dh, table_std=0.3, qkv_unit=True).round_to(torch.bfloat16)
+    out = _gpu(inp, torch.bfloat16, kernel=mvpa_hip.KERNEL_MFMA, **kw)
+    ref_in = copy.copy(inp)
+    if not kw.get("time_bias", True):
+        ref_in.k_time = torch.zeros_like(inp.k_time)
+    if not kw.get("chan_bias", True):
+        ref_in.k_chan = torch.zeros_like(inp.k_chan)
+    okw = {"window": kw["window"]} if "window" in kw else {"global_att": False} if "content" in kw else {}
+    ref = _oracle(ref_in, **okw)
+    if "fp8_qk" in kw:
+        assert (out.float().cpu() - ref.float()).abs().max().item() <= FP8_TOL[True]["max_abs"]
+        assert _rel_l2(out.float().cpu(), ref.float()) <= FP8_TOL[True]["rel_l2"]
+    else:
+        _check_bf16(out, ref)
 
 
 def test_fp16_dispatch_and_what_it_refuses():
