@@ -355,7 +355,8 @@ def test_operands_on_two_gpus_are_refused():
 # one wave a row and a workgroup a row, odd sizes of every level, rows at odd boundaries of 16 bytes (odd L); rows: one, fewer
 # than a wave's share, every group of rows and a remainder
 @pytest.mark.parametrize("L,M,wt", [(97, 1, torch.float32), (512, 131, torch.bfloat16), (1001, 33, torch.float32),
-                                    (2560, 2051, torch.bfloat16), (4095, 65, torch.bfloat16)])
+                                    (2560, 2051, torch.bfloat16), (4095, 65, torch.bfloat16),
+                                    (16032, 3, torch.float32)])                  # (the longest in one pass)
 def test_encoder_norm(L, M, wt):
     """Analysis and norm of a training pass against the two kernels, the weight's gradient against 64 bits."""
     g = torch.Generator(device="cuda").manual_seed(L + M)
@@ -381,5 +382,6 @@ def test_encoder_norm(L, M, wt):
 
 
 def test_encoder_norm_of_rows_beyond_the_one_pass():
-    assert AG.encoder_norm(torch.zeros(2, 40000, device="cuda"), torch.ones(sum(mvpa_hip.dwt_sizes(40000)[1]), device="cuda"), 40960, 1e-5) is None
+    for L in (16033, 40000):
+        assert AG.encoder_norm(torch.zeros(2, L, device="cuda"), torch.ones(sum(mvpa_hip.dwt_sizes(L)[1]), device="cuda"), 40960, 1e-5) is None
     assert AG.encoder_norm(torch.zeros(0, 512, device="cuda"), torch.ones(550, device="cuda"), 576, 1e-5) is None
