@@ -9,7 +9,7 @@
 // at a time: 32 rows of x, [768,2624] weights 9.8 -> 6.0 us, [2048,2048] 8.7 -> 5.8; 128 x 64 tiles 16.1 -> 13.6).
 //   4 waves.  WM = 4: a wave owns 32 rows of x and all 64 columns.  WM = 2 / 1: two / four waves share
 //   the rows and take 32 / 16 of every 64 k each, so that a wave always holds two 32 x 32 tiles (for the gated
-//   product: the gate and the up columns of an output).
+//   product: the gate and the up columns of an output).  128 columns: twice the waves.
 //   The sums go through LDS by rows and every thread finishes and stores 16 bytes of a row: stored as the
 //   products leave them, 8 or 16 bytes of each of 32 rows per instruction, the partial sums of 525 rows of 768
 //   alone took 3 us.
@@ -27,36 +27,38 @@ typedef __attribute__((ext_vector_type(4))) float f32x4;
 constexpr int TL_BN = 64, TL_BK = 64, TL_ROWB = TL_BK * 2;
 constexpr int TL_SUM = TL_BN * 4;                   // bytes of a row of sums: 16 chunks, XOR-swizzled by the row
 
-template <int WM, int STAGES, int CT = 2>           // CT: tiles of 32 columns of a wave
+template <int WM, int STAGES, int CT = 2, int BN = TL_BN>           // CT: tiles of 32 columns of a wave
 struct tile_cfg {
-  static constexpr int BM = 32 * WM, CW = 2 / CT, KH = 4 / (WM * CW), LPW = WM + 2;      // LPW: 1 KiB loads per wave and block
-  static constexpr int STAGE = (BM + TL_BN) * TL_ROWB;
-  static constexpr int LDS = STAGES * STAGE;
-  static_assert(WM * CW * KH == 4 && KH * BM * TL_SUM <= LDS, "four waves, and their sums fit the ring");
+  static constexpr int BM = 32 * WM, CW = BN / 32 / CT, NW = BN / 16, KH = NW / (WM * CW);
+  static constexpr int XL = BM / 8 / NW, LPW = (BM + BN) / 8 / NW;          // 1 KiB loads per wave and block: of x, in all
+  static constexpr int STAGE = (BM + BN) * TL_ROWB;
+  static constexpr int LDS = STAGES * STAGE, SUMS = KH * BM * TL_SUM;       // SUMS: of 64 columns
+  static_assert(WM * CW * KH == NW && XL * 8 * NW == BM && LPW * 8 * NW == BM + BN && BN / TL_BN * SUMS <= LDS,
+                "four waves for every 64 columns, and their sums fit the ring");
 };
 
 // The tile's products over k-blocks [kb0, kb1), left in LDS for tile_sum.  wrow(r): which row of W feeds row r of
 // the tile.
-template <int WM, int STAGES, int CT = 2, typename WRow>
+template <int WM, int STAGES, int CT = 2, int BN = TL_BN, typename WRow>
 __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* __restrict__ X, int64_t ldx, int64_t m0,
                                              int64_t M, const bf16_t* __restrict__ W, int64_t ldw, WRow wrow,
                                              int kb0, int kb1) {
-  using G = tile_cfg<WM, STAGES, CT>;
+  using G = tile_cfg<WM, STAGES, CT, BN>;
   f32x16 acc[CT];
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % WM, wc = wave / WM % G::CW, kh = wave / (WM * G::CW);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(LDS_PTR(unsigned char))lds;
 
-  // load i of a wave: rows (wave + 4i) * 8 .. + 7 of the block, x rows first (i < WM), then w rows
+  // load i of a wave: rows (wave + NW i) * 8 .. + 7 of the block, x rows first (i < XL), then w rows
   uint32_t off[G::LPW];
   {
     const int rsub = lane >> 3, phys = lane & 7;
 #pragma unroll
     for (int i = 0; i < G::LPW; ++i) {
-      const int row = (wave + 4 * i) * 8 + rsub;
+      const int row = (wave + G::NW * i) * 8 + rsub;
       const int chunk = (phys ^ ((row >> 1) & 7)) << 3;
-      if (i < WM) {
+      if (i < G::XL) {
         const int64_t m = m0 + row;
         off[i] = (uint32_t)((((m < M ? m : M - 1) - m0) * ldx + chunk) * 2);
       } else {
@@ -70,7 +72,7 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
   auto issue = [&]() {
 #pragma unroll
     for (int i = 0; i < G::LPW; ++i)
-      load_to_lds_16(i < WM ? (const void*)xs : (const void*)ws, off[i], dst + (wave + 4 * i) * 1024);
+      load_to_lds_16(i < G::XL ? (const void*)xs : (const void*)ws, off[i], dst + (wave + G::NW * i) * 1024);
     xs += TL_BK;
     ws += TL_BK;
     dst = dst + G::STAGE == lds0 + G::LDS ? lds0 : dst + G::STAGE;
@@ -93,7 +95,7 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
   const unsigned char* st = lds;                    // the stage whose fragments are read next
   auto read = [&](frags& f) {
     const unsigned char* xb = st + wm * 32 * TL_ROWB;
-    const unsigned char* wb = st + (G::BM + wc * 32) * TL_ROWB;
+    const unsigned char* wb = st + (G::BM + wc * CT * 32) * TL_ROWB;
 #pragma unroll
     for (int s = 0; s < SL; ++s) {
       f.x[s] = *(const bf16x8*)(xb + frag[s]);
@@ -149,14 +151,14 @@ __device__ __forceinline__ void tile_product(unsigned char* lds, const bf16_t* _
     }
     multiply(r & 1 ? fb : fa);
   }
-  // every wave's sums by rows of x, [k part][BM rows][64 columns] over the ring
+  // every wave's sums by rows of x, [64 columns of the tile][k part][BM rows] over the ring
   lds_barrier();
   unsigned char* sums = lds + (kh * G::BM + wm * 32 + ln) * TL_SUM;
 #pragma unroll
   for (int j = 0; j < CT; ++j)
 #pragma unroll
     for (int a4 = 0; a4 < 4; ++a4)
-      *(float4*)(sums + (((8 * (wc * CT + j) + 2 * a4 + hh) ^ (ln & 15)) << 4)) =
+      *(float4*)(sums + (wc * CT + j) / 2 * G::SUMS + (((8 * ((wc * CT + j) & 1) + 2 * a4 + hh) ^ (ln & 15)) << 4)) =
           make_float4(acc[j][a4 * 4], acc[j][a4 * 4 + 1], acc[j][a4 * 4 + 2], acc[j][a4 * 4 + 3]);
   lds_barrier();
 }
@@ -200,14 +202,16 @@ __device__ __forceinline__ void for_rows_left(int64_t rows, int mt, F f) {
   }
 }
 
-template <int WM, int STAGES>
+template <int WM, int STAGES, int BN>
 __device__ __forceinline__ void tile_dual(unsigned char* tl_lds, const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
                                           const bf16_t* __restrict__ W0, int N0, int64_t ldw0, const tile_out& out,
                                           const tile_gated& gt, const tile_norm& nrm, int gated_ct, int col, int64_t m0) {
-  using G = tile_cfg<WM, STAGES>;
-  const int tid = threadIdx.x;
+  using G = tile_cfg<WM, STAGES, 2, BN>;
+  constexpr int PER = BN / TL_BN;                   // 256 threads finish 64 columns
+  const int tid = threadIdx.x & 255, part = PER > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
   const bool gated = col < gated_ct;
-  const int n0 = gated ? col * 32 : (col - gated_ct) * TL_BN, N = gated ? gt.N : N0;
+  const int first = gated ? col * PER * 32 : (col - gated_ct) * BN, N = gated ? gt.N : N0;
+  const int n0 = first + part * (gated ? 32 : TL_BN);
   // sums of squares of the rows this thread will finish: requested in front of the product, used behind it
   constexpr int ROWS = G::BM / 32;                  // every 64th row of the gated product, every 32nd of the plain one
   const int r0 = gated ? tid >> 2 : tid >> 3, dr = gated ? 64 : 32;
@@ -215,10 +219,11 @@ __device__ __forceinline__ void tile_dual(unsigned char* tl_lds, const bf16_t* _
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) ss[i] = nrm.ss ? nrm.ss[min(m0 + r0 + i * dr, M - 1) * nrm.parts] : 0.f;
   if (gated)
-    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, gt.w, gt.ldw,
-                             [&](int r) { return (int64_t)((r >> 5) * N + min(n0 + (r & 31), N - 1)); }, 0, K / TL_BK);
+    tile_product<WM, STAGES, 2, BN>(tl_lds, X, ldx, m0, M, gt.w, gt.ldw, [&](int r) {
+      return (int64_t)((r >> 5 & 1) * N + min(first + (r >> 6) * 32 + (r & 31), N - 1)); }, 0, K / TL_BK);
   else
-    tile_product<WM, STAGES>(tl_lds, X, ldx, m0, M, W0, ldw0, [&](int r) { return (int64_t)min(n0 + r, N0 - 1); }, 0, K / TL_BK);
+    tile_product<WM, STAGES, 2, BN>(tl_lds, X, ldx, m0, M, W0, ldw0, [&](int r) { return (int64_t)min(first + r, N0 - 1); }, 0, K / TL_BK);
+  tl_lds += part * G::SUMS;
 #pragma unroll
   for (int i = 0; i < ROWS; ++i) asm volatile("" : "+v"(ss[i]));       // not before the product
   auto factor = [&](int i, int64_t m) {
@@ -272,8 +277,8 @@ __device__ __forceinline__ void tile_dual(unsigned char* tl_lds, const bf16_t* _
   }
 }
 
-template <int WM, int STAGES>
-__global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+template <int WM, int STAGES, int BN>
+__global__ __launch_bounds__(BN * 4) void tile_dual_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
                                                         const bf16_t* __restrict__ W0, int N0, int64_t ldw0,
                                                         tile_out out, tile_gated gt, tile_norm nrm, int gated_ct,
                                                         int ct, int mt) {
@@ -282,7 +287,7 @@ __global__ __launch_bounds__(256) void tile_dual_kernel(const bf16_t* __restrict
   if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
   const int64_t m0 = (int64_t)row * 32 * WM;
   for_rows_left<WM, STAGES>(M - m0, mt, [&](auto wm, auto stages) {
-    tile_dual<wm(), stages()>(tl_lds, X, M, K, ldx, W0, N0, ldw0, out, gt, nrm, gated_ct, col, m0);
+    tile_dual<wm(), stages(), BN>(tl_lds, X, M, K, ldx, W0, N0, ldw0, out, gt, nrm, gated_ct, col, m0);
   });
 }
 
@@ -420,15 +425,15 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
   }
 }
 
-template <int WM, int STAGES>
+template <int WM, int STAGES, int BN = TL_BN>
 static int launch_dual_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,
                          const tile_out& out, const tile_gated& gated, const tile_norm& norm, hipStream_t s) {
-  using G = tile_cfg<WM, STAGES>;
-  auto kern = tile_dual_kernel<WM, STAGES>;
+  using G = tile_cfg<WM, STAGES, 2, BN>;
+  auto kern = tile_dual_kernel<WM, STAGES, BN>;
   want_dynamic_lds((const void*)kern, G::LDS);
-  const int gct = gated.w ? (gated.N + 31) / 32 : 0;
-  const int ct = gct + (w0 ? (int)((N0 + TL_BN - 1) / TL_BN) : 0), mt = (int)((M + G::BM - 1) / G::BM);
-  MVPA_LAUNCH(kern, dim3((unsigned)((ct + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w0, (int)N0, ldw0,
+  const int gct = gated.w ? (gated.N + BN / 2 - 1) / (BN / 2) : 0;
+  const int ct = gct + (w0 ? (int)((N0 + BN - 1) / BN) : 0), mt = (int)((M + G::BM - 1) / G::BM);
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct + 7) / 8 * 8 * mt)), dim3(G::NW * 64), G::LDS, s, x, M, (int)K, ldx, w0, (int)N0, ldw0,
               out, gated, norm, gct, ct, mt);
   return take_launch_status();
 }
@@ -449,6 +454,13 @@ int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const b
   if (rows == 32) return launch_dual_t<1, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (rows == 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (M <= 128) return launch_dual_t<4, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
+  // Where most CUs would hold two tiles of 128 x 64 that read the same x twice: one of 128 x 128 on eight waves instead.  Passes,
+  // 64 / 128 columns, us: base model (two boxes) 192 rows (360 tiles' worth) 1424 / 1364 .. 1421, 209 1463 / 1394 .. 1446, 256 1594 / 1485 ..
+  // 1522; MVPFormer-S 640 (370) 417 / 410, 768 (444) 457 / 451, but 396 (229) 404 / 407, 414 (239) 381 / 383, 525 (304) 459 / 461.
+  const int64_t cols = (gated.w ? (gated.N + 31) / 32 : 0) + (w0 ? (N0 + TL_BN - 1) / TL_BN : 0);
+  const int64_t wide = (gated.w ? (gated.N + 63) / 64 : 0) + (w0 ? (N0 + 127) / 128 : 0);
+  if (M * cols > 128 * 352 && (M + 127) / 128 * wide <= 256)
+    return launch_dual_t<4, 4, 128>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   return launch_dual_t<4, 3>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
 }
 

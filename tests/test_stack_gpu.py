@@ -100,6 +100,22 @@ def test_rows_either_side_of_a_tile_size(C, T, dims):
     assert _rel(got, want) <= REL
 
 
+# 129 columns of tiles (an odd number of the gated ones): narrow, wide with 94 and 128 rows left to the last tile, narrow again;
+# an odd number in both products, the last gated one of 8 columns: wide with 62 and 128 rows left
+@pytest.mark.parametrize("C,T,dims", [(87, 4, dict(n_inner=4000)), (70, 5, dict(n_inner=4000)), (96, 4, dict(n_inner=4000)),
+                                      (77, 5, dict(n_inner=4000)), (82, 7, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=2024)),
+                                      (128, 5, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=2024))])
+def test_tiles_of_twice_the_columns(C, T, dims):
+    """Tiles of 128 rows and 128 columns of [q/k/v | gate/up] on either side of their range, against the stack in 64 bits."""
+    model = _model(**dims)
+    x = torch.randn(1, T, C, model.embed_dim, device="cuda").bfloat16()
+    with torch.no_grad():
+        got = model(inputs_embeds=x)
+    heads = dict(n_layer=2, n_head=dims.get("n_head", 2), n_head_kv=dims.get("n_head_kv", 1))
+    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, heads, None)
+    assert _rel(got, want) <= REL
+
+
 @pytest.mark.parametrize("C,T,inner", [(125, 4, 4032), (128, 4, 4032), (96, 4, 448), (77, 5, 448), (103, 5, 448)])
 def test_parts_of_the_tail_product_by_xcd(C, T, inner):
     """Four row tiles with x of the tail product up to and over 4 MB; three, four and five row tiles."""
