@@ -1682,7 +1682,7 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       f[i] = c + i < dwt_size ? f[i] : 0.f;
-      v[i] = f[i] * inv * g[i];
+      v[i] = c + i < dwt_size ? f[i] * inv * g[i] : 0.f;      // (inv is NaN where a sample is: 0 x NaN would not do)
     }
     vec8<bf16_t>::store(y + row * ldy + c, v);
     if (coef_out) vec8<float>::store(coef_out + row * ldy + c, f);

@@ -381,6 +381,21 @@ def test_encoder_norm(L, M, wt):
     assert ((both[1].double() - 2 * again.double()).abs() <= 2.0 ** -7 * both[1].double().abs() + 1e-3 * M ** 0.5).all()
 
 
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38], ids=str)
+@pytest.mark.parametrize("L", [97, 512, 2560])             # one wave a row, a workgroup a row
+def test_columns_past_the_coefficients_are_zero_whatever_a_row_holds(L, bad):
+    total = sum(mvpa_hip.dwt_sizes(L)[1])
+    pitch = (total + 63) // 64 * 64 + 64
+    x = torch.randn(9, L, device="cuda")
+    good = mvpa_hip.wavedec_db4_rmsnorm(x, torch.ones(total, device="cuda"), pitch)
+    x[4, L // 3] = bad
+    w = torch.ones(total, device="cuda", requires_grad=True)
+    for y in (mvpa_hip.wavedec_db4_rmsnorm(x, w.detach(), pitch), AG.encoder_norm(x, w, pitch, 1e-5)):
+        assert (y[:, total:] == 0).all()
+        rows = torch.arange(9, device="cuda") != 4
+        assert torch.equal(y[rows], good[rows])
+
+
 def test_encoder_norm_of_rows_beyond_the_one_pass():
     for L in (16033, 40000):
         assert AG.encoder_norm(torch.zeros(2, L, device="cuda"), torch.ones(sum(mvpa_hip.dwt_sizes(L)[1]), device="cuda"), 40960, 1e-5) is None
