@@ -1524,10 +1524,13 @@ __global__ __launch_bounds__(256) void wavedec_db4_kernel(const float* __restric
 // sample and 2 bytes out per coefficient (as three launches through fp32 coefficients: 98 us for
 // 16384 rows of 512, of which the row-per-workgroup analysis with a barrier per level took 72).
 // G threads own a row: one wave for short rows (no workgroup barrier at all), a workgroup for long
-// ones.  Even and odd samples lie in arrays of their own, with copies of 8 samples around them for the periodic wrap: a thread
-// takes outputs 2 t and 2 t + 1, whose taps are the six pairs E, O[2 t - 4 .. 2 t + 1], without an index modulo n and
-// without bank conflicts, and of a row that a workgroup owns the last levels are one wave's (taps read one by one with a stride
-// of two floats, every level with two barriers: 6400 rows of 2560 60 -> 46 us, 16384 of 512 34.0 -> 29.7, 64 of 512 7.5 -> 8.0).
+// ones.  Even and odd samples lie in arrays of their own, with copies of 8 samples around them for the periodic wrap: output k's
+// taps are the four pairs E, O[k - 3 .. k], without an index modulo n and without bank conflicts.  A workgroup meets once a level, and
+// the levels of at most 64 outputs are its first wave's.  What is bound by latency (few rows) or by instructions (many short ones)
+// is: trips to memory, so the samples come in groups and the norm's weight ahead of the levels.  us, taps with a stride of two floats and
+// two barriers a level / pairs of outputs a thread, samples one by one, weight and sum of squares at the end / now: 64 rows of 512 7.9 /
+// 8.2 / 7.3, 16384 of 512 34.0 / 29.9 / 26.7, 64 of 2560 8.5 / 9.7 / 8.2, 6400 of 2560 60 / 51 / 45, 64 of 4095 11.0 / 15.4 / 10.9, 6400 of
+// 1001 44 / 47 / 29, but 16384 of 64 11.3 / 14.2 / 13.3.
 // With coef_out (row pitch ldy) and inv_out the coefficients and the factor of every row leave as well: a
 // training pass wants them for the gradient of the norm's weight (norm_dw_kernel).
 // -----------------------------------------------------------------------------------------
@@ -1540,7 +1543,7 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
                                                                   bf16_t* __restrict__ y, float* __restrict__ coef_out,
                                                                   float* __restrict__ inv_out, int64_t M, int L,
                                                                   int levels, int dwt_size, int64_t ldy, float eps,
-                                                                  int row_floats, bool vec) {
+                                                                  int row_floats, bool vec_x, bool vec_w) {
   extern __shared__ __attribute__((aligned(16))) float wd_lds[];
   __shared__ float red[4];
   const int sub = threadIdx.x / G, t = threadIdx.x % G;
@@ -1562,102 +1565,132 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
   float* next_odd = next_even + later;
   float* coef = next_odd + later - 4;
   const float* xr = x + row * L;
-  // sample k of n, and its copies in front of and behind them for the periodic wrap: a wave by itself makes those in one go
-  // instead (wrap), which takes it less time than the branches; a workgroup would need one more barrier
-  auto put = [](float* e, float* o, int k, int n, float v) {
-    (k & 1 ? o : e)[k >> 1] = v;
-    if (G == 64) return;
-    if (k < 8) ((n + k) & 1 ? o : e)[(n + k) >> 1] = v;
-    if (k >= n - 8) ((k - n) & 1 ? o : e)[(k - n) >> 1] = v;
-  };
-  if (vec) {
-    for (int i = t; i < L / 4; i += G) {
-      const float4 v = *(const float4*)(xr + 4 * i);
-      *(float2*)(even + 2 * i) = make_float2(v.x, v.z);
-      *(float2*)(odd + 2 * i) = make_float2(v.y, v.w);
-      if (G == 256 && (i < 2 || i >= L / 4 - 2)) {
-        const float q[4] = {v.x, v.y, v.z, v.w};
+  // requested together: the copies around the row, the norm's weight for the first two groups of columns, the first samples.  No branch a
+  // lane takes by itself: its loads would be waited for where it ends
+  const float around = xr[t < 8 ? L - 8 + t : t < 16 ? t - 8 : 0];
+  auto weights = [&](int c, float (&g)[8]) { vec8<float>::load(w + min(c, (dwt_size - 8) & ~7), g); };
+  float g0[8] = {}, g1[8] = {};                     // (of whole groups; the last one's lie a column a lane)
+  if (vec_w) {
+    weights(t * 8, g0);
+    if (ldy > G * 8) weights((t + G) * 8, g1);
+  }
+  const float last_w = w[min((dwt_size & ~7) + (t & 7), dwt_size - 1)];
+  if (vec_x) {
+    constexpr int U = G == 64 ? 2 : 4;
+    for (int i0 = 0; i0 < L / 4; i0 += U * G) {
+      float4 v[U];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) put(even, odd, 4 * i + j, L, q[j]);
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * G < L / 4) v[u] = *(const float4*)(xr + 4 * min(i0 + u * G + t, L / 4 - 1));
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int i = i0 + u * G + t;
+        if (i0 + u * G >= L / 4 || i >= L / 4) continue;
+        *(float2*)(even + 2 * i) = make_float2(v[u].x, v[u].z);
+        *(float2*)(odd + 2 * i) = make_float2(v[u].y, v[u].w);
       }
     }
   } else {
-    for (int i = t; i < L; i += G) put(even, odd, i, L, xr[i]);
-  }
-  int n = L, tail = dwt_size;
-  auto level = [&](int threads) {
-    const int m = (n + 7) >> 1;
-    const int at = tail - m;
-    for (int k = 2 * t; k < m; k += 2 * threads) {
-      float e[6], o[6];
+    constexpr int U = G == 64 ? 4 : 8;
+    float* mine = (t & 1 ? odd : even) + (t >> 1);
+    for (int i0 = 0; i0 < L; i0 += U * G) {
+      float v[U];
 #pragma unroll
-      for (int i = 0; i < 6; i += 2) {
-        const float2 a = *(const float2*)(even + k - 4 + i), b = *(const float2*)(odd + k - 4 + i);
-        e[i] = a.x; e[i + 1] = a.y;
-        o[i] = b.x; o[i + 1] = b.y;
-      }
+      for (int u = 0; u < U; ++u)
+        if (i0 + u * G < L) v[u] = xr[min(i0 + u * G + t, L - 1)];
 #pragma unroll
-      for (int q = 0; q < 2; ++q) {
-        float lo = 0.f, hi = 0.f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {               // tap j of output k + q: sample 2 (k + q) + 1 - j
-          const float v = j & 1 ? e[4 + q - (j >> 1)] : o[4 + q - (j >> 1)];
-          lo += kDb4Lo[j] * v;
-          hi += ((j & 1) ? kDb4Lo[7 - j] : -kDb4Lo[7 - j]) * v;
-        }
-        if (k + q < m) {
-          put(next_even, next_odd, k + q, m, lo);
-          coef[at + k + q] = hi;
-        }
+      for (int u = 0; u < U; ++u) {
+        if (i0 + u * G < L && i0 + u * G + t < L) mine[(i0 + u * G) / 2] = v[u];
       }
     }
-  };
-  auto advance = [&]() {
-    n = (n + 7) >> 1;
-    tail -= n;
+  }
+  if (t < 16) {
+    const int to = t < 8 ? t - 8 : L + t - 8;
+    (to & 1 ? odd : even)[to >> 1] = around;
+  }
+  int n = L, tail = dwt_size;
+  float ss = 0.f;
+  // output k of a level and the one `threads` further on, whose loads and chains run side by side; the sum of squares takes them in
+  // their order
+  auto level = [&](int threads) {
+    const int m = (n + 7) >> 1, at = tail - m;
+    float* mine = (t & 1 ? next_odd : next_even) + (t >> 1);
+    auto taps = [&](int k, float& lo, float& hi) {
+      float e[4], o[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        e[i] = even[k - 3 + i];
+        o[i] = odd[k - 3 + i];
+      }
+      lo = hi = 0.f;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {                 // tap j: sample 2 k + 1 - j
+        const float v = j & 1 ? e[3 - (j >> 1)] : o[3 - (j >> 1)];
+        lo += kDb4Lo[j] * v;
+        hi += ((j & 1) ? kDb4Lo[7 - j] : -kDb4Lo[7 - j]) * v;
+      }
+    };
+    // and its copies in front of and behind the level's m for the periodic wrap
+    auto put = [&](int k, float lo, float hi) {
+      mine[(k - t) >> 1] = lo;
+      if (G == 256 && k < 8) ((m + k) & 1 ? next_odd : next_even)[(m + k) >> 1] = lo;
+      if (G == 256 && k >= m - 8) ((k - m) & 1 ? next_odd : next_even)[(k - m) >> 1] = lo;
+      coef[at + k] = hi;
+      ss = fmaf(hi, hi, ss);
+    };
+    for (int k0 = 0; k0 < m; k0 += 2 * threads) {
+      float lo, hi, lo2, hi2;
+      const int k = k0 + t;
+      taps(min(k, m - 1), lo, hi);
+      if (k0 + threads < m) {
+        taps(min(k + threads, m - 1), lo2, hi2);
+        put(k, lo, hi);
+        if (k + threads < m) put(k + threads, lo2, hi2);
+      } else if (k < m) {
+        put(k, lo, hi);
+      }
+    }
+    n = m;
+    tail = at;
     float* sw = even; even = next_even; next_even = sw;
     sw = odd; odd = next_odd; next_odd = sw;
   };
-  auto wrap = [&]() {                               // samples -8 .. -1 and n .. n + 7 (n is at least 8)
+  auto wrap = [&]() {                               // the copies of a wave's own level
     if (t < 16) {
       const int to = t < 8 ? t - 8 : n + t - 8, from = t < 8 ? n + t - 8 : t - 8;
       (to & 1 ? odd : even)[to >> 1] = (from & 1 ? odd : even)[from >> 1];
     }
   };
   int lv = 0;
-  for (; lv < levels && (G == 64 || n > 256); ++lv) {
+  for (; lv < levels && (G == 64 || n > 121); ++lv) {
     sync();
-    if (G == 64) {
+    if (G == 64 && lv > 0) {
       wrap();
       sync();
     }
     level(G);
-    advance();
   }
-  if (G == 256) {                                   // what is left is a wave's work, without barriers of the workgroup
-    sync();
-    for (; lv < levels; ++lv) {
-      if (t < 64) {
+  sync();
+  if (G == 256 && lv < levels) {                    // outputs of one wave and fewer: without barriers of the workgroup
+    if (t < 64) {
+      for (; lv < levels; ++lv) {
         level(64);
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
       }
-      advance();
+      for (int k = t; k < n; k += 64) {
+        const float v = (k & 1 ? odd : even)[k >> 1];
+        coef[k] = v;
+        ss = fmaf(v, v, ss);
+      }
     }
-  }
-  sync();
-  // the sum of squares level by level, as their outputs are dealt to the threads one by one
-  float ss = 0.f;
-  for (int lev = 0, of = L, at = dwt_size; lev < levels; ++lev) {
-    of = (of + 7) >> 1;
-    at -= of;
-    for (int k = t; k < of; k += G) ss += coef[at + k] * coef[at + k];
-  }
-  for (int k = t; k < n; k += G) {
-    const float v = (k & 1 ? odd : even)[k >> 1];
-    coef[k] = v;
-    ss += v * v;
+  } else {
+    for (int k = t; k < n; k += G) {
+      const float v = (k & 1 ? odd : even)[k >> 1];
+      coef[k] = v;
+      ss = fmaf(v, v, ss);
+    }
   }
   ss = wave_sum(ss);
   if (G == 256) {
@@ -1669,23 +1702,26 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
   }
   const float inv = rsqrtf(ss / (float)dwt_size + eps);
   if (inv_out && t == 0) inv_out[row] = inv;
-  for (int c = t * 8; c < ldy; c += G * 8) {
-    float v[8] = {}, f[8] = {}, g[8] = {};
-    if (c < dwt_size) vec8<float>::load(coef + c, f);          // (a row's coefficients take whole groups of 8)
-    if (vec && c + 8 <= dwt_size) {
-      vec8<float>::load(w + c, g);
-    } else {
+  for (int c0 = 0; c0 < ldy; c0 += G * 8) {
+    const int c = c0 + t * 8;
+    float v[8], f[8];
+    vec8<float>::load(coef + min(c, (dwt_size - 1) & ~7), f);        // (a row's coefficients take whole groups of 8)
+    if (!vec_w) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (c + i < dwt_size) g[i] = w[c + i];
+      for (int i = 0; i < 8; ++i) g0[i] = w[min(c + i, dwt_size - 1)];
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      const float g = c + 8 <= dwt_size ? g0[i] : __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(last_w), i));
       f[i] = c + i < dwt_size ? f[i] : 0.f;
-      v[i] = c + i < dwt_size ? f[i] * inv * g[i] : 0.f;      // (inv is NaN where a sample is: 0 x NaN would not do)
+      v[i] = c + i < dwt_size ? f[i] * inv * g : 0.f;          // (inv is NaN where a sample is: 0 x NaN would not do)
+      g0[i] = g1[i];
     }
-    vec8<bf16_t>::store(y + row * ldy + c, v);
-    if (coef_out) vec8<float>::store(coef_out + row * ldy + c, f);
+    if (vec_w && c0 + 2 * G * 8 < dwt_size) weights(c + 2 * G * 8, g1);
+    if (c < ldy) {
+      vec8<bf16_t>::store(y + row * ldy + c, v);
+      if (coef_out) vec8<float>::store(coef_out + row * ldy + c, f);
+    }
   }
 }
 
@@ -2197,7 +2233,7 @@ static int launch_wavedec_rmsnorm(const float* x, const float* weight, void* y, 
   if (lds > 64 * 1024) mvpa::want_dynamic_lds((const void*)kern, lds);
   MVPA_LAUNCH(kern, dim3((unsigned)(wave ? (M + 3) / 4 : M)), dim3(256), lds, (hipStream_t)stream, x, weight, (bf16_t*)y,
               coeffs, inv, M, L, levels, dwt_size, ldy, eps, row_floats,
-              L % 4 == 0 && (((uintptr_t)x | (uintptr_t)weight) & 15) == 0);
+              L % 4 == 0 && ((uintptr_t)x & 15) == 0, ((uintptr_t)weight & 15) == 0);
   return mvpa::take_launch_status();
 }
 

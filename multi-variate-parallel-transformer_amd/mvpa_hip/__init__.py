@@ -566,7 +566,7 @@ def mean_rows(x: torch.Tensor) -> torch.Tensor:
 
 def wavedec_db4_rmsnorm(x: torch.Tensor, weight: torch.Tensor, pitch: int, eps: float = 1e-5) -> torch.Tensor:
     """RMSNorm of the db4 coefficients of x [M, L] in bf16, [M, pitch] with zeros past the coefficients:
-    wavedec_db4 and rmsnorm, in one pass where a row fits the LDS (up to about 15 900 samples)."""
+    wavedec_db4 and rmsnorm, in one pass where a row fits the LDS (up to 16 032 samples)."""
     _, length = x.shape
     levels, total = _dwt_shape(length)
     assert weight.numel() == total, "wavedec_db4_rmsnorm: one weight per coefficient"

@@ -576,7 +576,7 @@ def test_a_used_model_is_copied():
         assert not torch.equal(other(inputs_embeds=x), first) and torch.equal(model(inputs_embeds=x), first)
 
 
-@pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560, 15930, 15931, 16384])    # the longest in one pass, and beyond
+@pytest.mark.parametrize("L", [97, 333, 512, 1001, 2560, 15930, 15931, 16032, 16033, 16384])   # the longest in one pass is 16032
 @pytest.mark.parametrize("M", [1, 5])
 def test_encoder_in_one_pass(L, M):
     """Analysis, norm and rounding in one kernel against the two kernels: the same fp32 formula, summed
@@ -590,6 +590,22 @@ def test_encoder_in_one_pass(L, M):
     ref = mvpa_hip.rmsnorm(mvpa_hip.wavedec_db4(x), w, 1e-5, out=torch.empty(M, total, device="cuda"))
     assert (got[:, total:] == 0).all()
     assert ((got[:, :total] - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
+
+
+# the shortest; whole groups of eight coefficients; 504, 512 and 513 of them (a wave's groups of columns); the longest row that a
+# wave owns and the next; the levels that one wave finishes from the first, the second, .. on
+@pytest.mark.parametrize("L", [14, 17, 61, 121, 122, 463, 471, 473, 2010, 2011, 2012, 3000, 4095, 4100])
+def test_encoder_in_one_pass_at_any_boundary(L):
+    """Rows and norm weights that start at any element, either side of every group and level."""
+    total = sum(mvpa_hip.dwt_sizes(L)[1])
+    pitch = (total + 63) // 64 * 64
+    x, w = torch.randn(7 * L + 1, device="cuda"), 1.0 + 0.1 * torch.randn(total + 1, device="cuda")
+    for at in (0, 1):
+        rows, weight = x[at:at + 7 * L].view(7, L), w[at:at + total]
+        got = mvpa_hip.wavedec_db4_rmsnorm(rows, weight, pitch).float()
+        ref = mvpa_hip.rmsnorm(mvpa_hip.wavedec_db4(rows), weight.clone(), 1e-5, out=torch.empty(7, total, device="cuda"))
+        assert (got[:, total:] == 0).all()
+        assert ((got[:, :total] - ref).abs() <= ref.abs() * 2.0 ** -8 + 1e-6).all()
 
 
 def test_encoder_refuses_other_shapes():
