@@ -360,7 +360,7 @@ PyObject* py_norm_dw(PyObject*, PyObject* const* args, Py_ssize_t n) {
   Tensor dw = at::empty(w.sizes(), w.options());
   Tensor ws = at::empty({(int64_t)mvpa_norm_dw_ws_bytes(rows, cols)}, x.options().dtype(at::kByte));
   const int st = mvpa_norm_dw((const float*)x.data_ptr(), (const float*)inv.data_ptr(), dy.data_ptr(), dw.data_ptr(), ws.data_ptr(),
-                              rows, cols, x.stride(0), dy.stride(0), w.scalar_type() == at::kFloat, current_stream());
+                              rows, cols, x.size(1), x.size(1), w.scalar_type() == at::kFloat, current_stream());   // (one row may have any stride)
   return st == MVPA_OK ? THPVariable_Wrap(dw) : PyLong_FromLong(st);
   END_HANDLE_TH_ERRORS
 }

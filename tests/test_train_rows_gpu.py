@@ -381,6 +381,15 @@ def test_encoder_norm(L, M, wt):
     assert ((both[1].double() - 2 * again.double()).abs() <= 2.0 ** -7 * both[1].double().abs() + 1e-3 * M ** 0.5).all()
 
 
+def test_weight_gradient_of_the_encoder_norm_takes_one_row_of_any_stride():
+    total, pitch = 550, 576
+    x, w = torch.randn(1, 512, device="cuda"), torch.ones(total, device="cuda", requires_grad=True)
+    dy = torch.randn(pitch, 1, device="cuda").bfloat16()
+    got, = torch.autograd.grad(AG.encoder_norm(x, w, pitch, 1e-5), w, dy.t())
+    want, = torch.autograd.grad(AG.encoder_norm(x, w, pitch, 1e-5), w, dy.t().clone(memory_format=torch.contiguous_format).view(1, pitch))
+    assert dy.t().stride(0) == 1 and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38], ids=str)
 @pytest.mark.parametrize("L", [97, 512, 2560])             # one wave a row, a workgroup a row
 def test_columns_past_the_coefficients_are_zero_whatever_a_row_holds(L, bad):
