@@ -75,7 +75,9 @@ class WaveEncoder(BrainEncoder):
     def _forward_autograd(self, x: Tensor) -> Tensor:
         pad = self._padded_k() - self.dwt_size
         # whole 64-element k-blocks, as on the inference path: the zero columns contribute nothing
-        normed = AG.encoder_norm(x, self.ln.weight, self._padded_k(), 1e-5)
+        normed = None
+        if type(self).block is _ANALYSIS and "block" not in self.__dict__:      # another analysis is asked for its coefficients
+            normed = AG.encoder_norm(x, self.ln.weight, self._padded_k(), 1e-5)
         if normed is None:
             coeffs = self.block(x)                                              # fp32, no gradient
             normed = torch.nn.functional.pad(AG.rmsnorm(coeffs, self.ln.weight, 1e-5, out_dtype=torch.bfloat16), (0, pad))
@@ -88,3 +90,6 @@ class WaveEncoder(BrainEncoder):
 
     def encode(self, x: Tensor) -> Tensor:
         return self.forward(x)
+
+
+_ANALYSIS = WaveEncoder.block

@@ -5,6 +5,7 @@ import torch
 
 import mvpa_hip
 from attentions.attn import FlashMVPA, FlashMVPAPacked
+from models.fftencoder import WaveEncoder
 from models.mvpformer import MVPFormerConfig, MVPFormerModel
 from mvpa_hip import autograd as AG
 
@@ -388,6 +389,22 @@ def test_weight_gradient_of_the_encoder_norm_takes_one_row_of_any_stride():
     got, = torch.autograd.grad(AG.encoder_norm(x, w, pitch, 1e-5), w, dy.t())
     want, = torch.autograd.grad(AG.encoder_norm(x, w, pitch, 1e-5), w, dy.t().clone(memory_format=torch.contiguous_format).view(1, pitch))
     assert dy.t().stride(0) == 1 and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("how", ["subclass", "object", "class"])
+def test_an_analysis_of_its_own_is_heard_in_training(monkeypatch, how):
+    def block(self, x):
+        return 2.0 + mvpa_hip.wavedec_db4(x.float())
+    kind = type("Own", (WaveEncoder,), dict(block=block)) if how == "subclass" else WaveEncoder
+    enc = kind(512, 64).to("cuda", torch.bfloat16).train()
+    if how == "object":
+        enc.block = lambda x: block(enc, x)
+    elif how == "class":
+        monkeypatch.setattr(WaveEncoder, "block", block)
+    x = torch.randn(9, 512, device="cuda")
+    normed = mvpa_hip.rmsnorm(2.0 + mvpa_hip.wavedec_db4(x), enc.ln.weight.detach(), 1e-5, out_dtype=torch.bfloat16)
+    want = normed.double() @ enc.proj.weight.detach().double().T
+    assert ((enc(x).double() - want).norm() / want.norm()).item() <= 1e-2          # one bf16 rounding of the product
 
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf"), 3e38], ids=str)
