@@ -186,6 +186,8 @@ def encoder_norm(x: torch.Tensor, w: torch.Tensor, pitch: int, eps: float):
     too long for it, are none, or the weight is of another type."""
     if not x.is_cuda or w.dtype not in (torch.float32, torch.bfloat16) or not mvpa_hip.wavedec_fits(x):
         return None
+    if not wants_grad(w):                                    # a frozen norm: nothing is kept
+        return mvpa_hip.wavedec_db4_rmsnorm(x, w, pitch, eps)
     return _EncoderNormFn.apply(x.detach().float(), w, pitch, eps)
 
 

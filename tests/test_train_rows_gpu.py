@@ -391,6 +391,16 @@ def test_weight_gradient_of_the_encoder_norm_takes_one_row_of_any_stride():
     assert dy.t().stride(0) == 1 and torch.equal(got, want)
 
 
+def test_a_frozen_encoder_norm_keeps_no_coefficients(monkeypatch):
+    x, w = torch.randn(33, 512, device="cuda"), (1 + 0.1 * torch.randn(550, device="cuda")).requires_grad_()
+    kept = AG.encoder_norm(x, w, 576, 1e-5)
+    with torch.no_grad():
+        assert torch.equal(AG.encoder_norm(x, w, 576, 1e-5), kept)
+    monkeypatch.setattr(mvpa_hip, "wavedec_db4_rmsnorm_saved", None)
+    got = AG.encoder_norm(x, w.detach(), 576, 1e-5)
+    assert got.grad_fn is None and torch.equal(got, kept)
+
+
 @pytest.mark.parametrize("how", ["subclass", "object", "class"])
 def test_an_analysis_of_its_own_is_heard_in_training(monkeypatch, how):
     def block(self, x):
