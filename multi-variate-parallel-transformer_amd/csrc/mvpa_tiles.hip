@@ -442,10 +442,11 @@ static int launch_dual_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, con
 // block of 32 rows of x is 12 KB, of 64 16, of 128 24.  With more workgroups than CUs the panels of w are read again instead.
 // [q/k/v | gate/up] of MVPFormer-S (74 columns of tiles), tiles of 32 / 64 / 128 rows, us: 32 rows 4.8 / 5.1 / 7.0, 64 4.8 /
 // 5.4 / 7.1, 100 6.1 / 5.4 / 7.9, 192 6.7 / 5.5 / 7.8, 256 8.7 / 7.7 / 7.6, 400 11.8 / 10.0 / 9.3; of the base model (240): 32
-// 15.0 / 14.8 / 16.2, 64 20.9 / 17.9 / 17.8, 100 26.6 / 22.7 / 19.2, 128 29.8 / 24.4 / 20.8.
+// 15.0 / 14.8 / 16.2, 64 20.9 / 17.9 / 17.8, 100 26.6 / 22.7 / 19.2, 128 29.8 / 24.4 / 20.8.  Never more rows than there are: the
+// workgroups would be as many (width 3072, 336 columns of tiles, 21 rows 24 / . / 31, 64 rows . / 27 / 32).
 static int tile_rows(int64_t M, int64_t per_row_tile) {
-  if ((M + 31) / 32 * per_row_tile <= 256) return 32;
-  return (M + 63) / 64 * per_row_tile <= 256 ? 64 : 128;
+  if (M <= 32 || (M + 31) / 32 * per_row_tile <= 256) return 32;
+  return M <= 64 || (M + 63) / 64 * per_row_tile <= 256 ? 64 : 128;
 }
 
 int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w0, int64_t N0, int64_t ldw0,

@@ -100,6 +100,23 @@ def test_rows_either_side_of_a_tile_size(C, T, dims):
     assert _rel(got, want) <= REL
 
 
+@pytest.mark.parametrize("C", [1, 21, 32, 33, 64, 65, 128])
+@pytest.mark.parametrize("step", [False, True])
+def test_few_rows_of_many_columns(C, step):
+    """260 columns of tiles, more than there are CUs: the tile follows the rows, against the stack in 64 bits."""
+    model = _model(n_inner=8192)
+    x = torch.randn(1, 2 if step else 1, C, 128, device="cuda").bfloat16()
+    params, heads = {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=2, n_head_kv=1)
+    with torch.no_grad():
+        if step:
+            caches = model.new_cache(1, C, max_steps=2)
+            got = torch.stack([model(inputs_embeds=x[:, t:t + 1], past_key_values=caches)[0][0, 0] for t in (0, 1)])
+            want = O.stream_steps(x[0], params, heads, 2)[0]
+        else:
+            got, want = model(inputs_embeds=x), O.stack_forward(x, params, heads, None)
+    assert _rel(got, want) <= REL
+
+
 # 129 columns of tiles (an odd number of the gated ones): narrow, wide with 94 and 128 rows left to the last tile, narrow again;
 # an odd number in both products, the last gated one of 8 columns: wide with 62 and 128 rows left
 @pytest.mark.parametrize("C,T,dims", [(87, 4, dict(n_inner=4000)), (70, 5, dict(n_inner=4000)), (96, 4, dict(n_inner=4000)),
