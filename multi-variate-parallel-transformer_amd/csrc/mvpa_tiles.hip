@@ -348,30 +348,31 @@ __global__ __launch_bounds__(256) void tile_linear_kernel(const bf16_t* __restri
   }
 }
 
-// One workgroup per row: the partial sums of a split-K tail product, the residual, one rounding, and
+// One workgroup per row, a wave per 512 columns: the partial sums of a split-K tail product, the residual, one rounding, and
 // the RMSNorm that the next product wants, while the row is in registers (8 columns per lane and chunk).
-// Bound by the trip to the sums, which other XCDs have just written: all PARTS (the next of 4, 6, 8, 9 from their number; past
-// the last, the last once more, not added), the residual and the norm's weight are requested together.  With one part after the
-// other and the weight behind the sums of squares a stream's step (64 rows of 768, 9 parts, 12 launches) took 414 us and takes
-// 396, a step of the base model (128 rows of 2048, 8 parts, 24 launches) 1803 and 1792; 525 rows (4 parts) 517 and 518.
-template <int CHUNKS, int PARTS>
-__global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restrict__ P, int split_a, int split_b,
-                                                          const bf16_t* __restrict__ R, bf16_t* __restrict__ S,
-                                                          bf16_t* __restrict__ Y, const float* __restrict__ w,
+// Bound by the trip to the sums, which other XCDs have just written, and with hundreds of rows by what is requested: all parts, the
+// residual and the norm's weight are requested together, and nothing beside them.  TWO: the first split_a parts are a product
+// of their own.  us, one part after the other and the weight behind the sums of squares / everything together for the next of 4, 6,
+// 8, 9 parts in four waves a row / now: 64 rows of 768, 9 parts 3.6 / 3.6 / 3.2; 525, 4 parts 3.3 / 3.9 / 3.3; 1200, 2 parts 3.6 / 5.0 / 3.7; 128
+// rows of 2048, 8 parts 3.65 / 3.6 / 3.6; 768 rows of 3072, 1 part 4.9 / 6.7 / 5.1.
+template <int CHUNKS, int PARTS, bool TWO>
+__global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restrict__ P, int split_a, const bf16_t* __restrict__ R,
+                                                          bf16_t* __restrict__ S, bf16_t* __restrict__ Y, const float* __restrict__ w,
                                                           float eps, float* __restrict__ ss_out, int64_t M, int N) {
   __shared__ float red[4];
   const int64_t m = blockIdx.x;
-  const int parts = split_a + split_b;
+  const int wave0 = __builtin_amdgcn_readfirstlane(threadIdx.x & ~63) * 8;
   float v[CHUNKS][8], ss = 0.f;
   f32x4 p[CHUNKS][PARTS][2], wr[CHUNKS][2];
   u32x4 rr[CHUNKS];
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {                // lanes past the row: its last columns, for nobody
+    if (c > 0 && wave0 + c * 2048 >= N) continue;   // (a whole wave: nothing)
     const int n = min((c * 256 + (int)threadIdx.x) * 8, N - 8);
     rr[c] = *(const u32x4*)(R + m * N + n);
 #pragma unroll
     for (int z = 0; z < PARTS; ++z) {
-      const float* at = P + ((int64_t)min(z, parts - 1) * M + m) * N + n;
+      const float* at = P + ((int64_t)z * M + m) * N + n;
       p[c][z][0] = *(const f32x4*)at;
       p[c][z][1] = *(const f32x4*)(at + 4);
     }
@@ -383,6 +384,7 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
   // without branches, behind which the loads would be put and waited for one by one
 #pragma unroll
   for (int c = 0; c < CHUNKS; ++c) {
+    if (c > 0 && wave0 + c * 2048 >= N) continue;
     const int n = (c * 256 + threadIdx.x) * 8;
     float a[8] = {}, b[8] = {};
 #pragma unroll
@@ -390,15 +392,15 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const float x = p[c][z][i >> 2][i & 3];
-        a[i] += z < split_a ? x : 0.f;
-        b[i] += z >= split_a && z < parts ? x : 0.f;
+        if (TWO) a[i] += z < split_a ? x : 0.f;
+        b[i] += !TWO || z >= split_a ? x : 0.f;
       }
     bf16x8 o;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       v[c][i] = __uint_as_float(i & 1 ? rr[c][i >> 1] & 0xffff0000u : rr[c][i >> 1] << 16);
       v[c][i] += (float)(__bf16)b[i];
-      v[c][i] += (float)(__bf16)a[i];               // 0 where there is no first run
+      if (TWO) v[c][i] += (float)(__bf16)a[i];
       o[i] = (__bf16)v[c][i];
       v[c][i] = (float)o[i];
       ss += n < N ? v[c][i] * v[c][i] : 0.f;
@@ -409,7 +411,8 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
   for (int off = 32; off > 0; off >>= 1) ss += __shfl_xor(ss, off);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
   __syncthreads();
-  const float tot = red[0] + red[1] + red[2] + red[3];
+  float tot = red[0];
+  for (int k = 1; k < (int)blockDim.x / 64; ++k) tot += red[k];
   if (ss_out && threadIdx.x == 0) ss_out[m] = tot;
   if (!Y) return;
   const float inv = rsqrtf(tot / (float)N + eps);
@@ -423,6 +426,13 @@ __global__ __launch_bounds__(256) void tail_reduce_kernel(const float* __restric
       *(bf16x8*)(Y + m * N + n) = o;
     }
   }
+}
+
+template <int CHUNKS, int PARTS = 9>                // at most 9 parts: make_tile_split
+static auto tail_reduce_for(const tile_split& split) {
+  if constexpr (PARTS > 1)
+    if (split.total() < PARTS) return tail_reduce_for<CHUNKS, PARTS - 1>(split);
+  return split.a ? tail_reduce_kernel<CHUNKS, PARTS, true> : tail_reduce_kernel<CHUNKS, PARTS, false>;
 }
 
 template <int WM, int STAGES, int BN = TL_BN>
@@ -546,14 +556,9 @@ int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, cons
 
 int launch_tail_reduce(const float* P, const tile_split& split, const bf16_t* r, bf16_t* sum, bf16_t* norm, const float* w,
                        float eps, float* ss, int64_t M, int64_t N, hipStream_t s) {
-  auto pick = [&](auto chunks) {
-    constexpr int CH = decltype(chunks)::value;
-    const int parts = split.total();                // at most 9: make_tile_split
-    return parts <= 4 ? tail_reduce_kernel<CH, 4> : parts <= 6 ? tail_reduce_kernel<CH, 6> : parts <= 8 ? tail_reduce_kernel<CH, 8>
-                                                                                                      : tail_reduce_kernel<CH, 9>;
-  };
-  auto kern = N <= 2048 ? pick(std::integral_constant<int, 1>()) : pick(std::integral_constant<int, 2>());
-  MVPA_LAUNCH(kern, dim3((unsigned)M), dim3(256), 0, s, P, split.a, split.b, r, sum, norm, w, eps, ss, M, (int)N);
+  auto kern = N <= 2048 ? tail_reduce_for<1>(split) : tail_reduce_for<2>(split);
+  const unsigned waves = N <= 2048 ? (unsigned)(N + 511) / 512 : 4;
+  MVPA_LAUNCH(kern, dim3((unsigned)M), dim3(waves * 64), 0, s, P, split.a, r, sum, norm, w, eps, ss, M, (int)N);
   return take_launch_status();
 }
 

@@ -100,6 +100,24 @@ def test_rows_either_side_of_a_tile_size(C, T, dims):
     assert _rel(got, want) <= REL
 
 
+# rows of one wave, of one and a little more, of all four, of two rounds with one wave left; 1 .. 9 parts by rows and contraction
+@pytest.mark.parametrize("e,inner", [(64, 64), (512, 192), (576, 192), (768, 1728), (2048, 512), (2112, 64), (4096, 64)])
+@pytest.mark.parametrize("C,T", [(5, 1), (33, 2), (67, 5)], ids=str)
+def test_rows_of_the_tail(e, inner, C, T):
+    """Sum of the parts, residual and norm by the width of a row, whole windows and steps, against the stack in 64 bits."""
+    model = _model(n_embd=e, n_head=e // 64, n_head_kv=1, n_inner=inner)
+    for n, p in model.named_parameters():
+        if "ln" not in n:                                # scores as wide as at 128 columns: REL is for those, and sharper ones magnify roundings
+            p.data.mul_((128 / max(e, 128)) ** 0.5)
+    x = torch.randn(1, T, C, e, device="cuda").bfloat16()
+    params, heads = {n: p.detach() for n, p in model.named_parameters()}, dict(n_layer=2, n_head=e // 64, n_head_kv=1)
+    caches = model.new_cache(1, C, max_steps=T)
+    with torch.no_grad():
+        assert _rel(model(inputs_embeds=x), O.stack_forward(x, params, heads, None)) <= REL
+        steps = torch.stack([model(inputs_embeds=x[:, t:t + 1], past_key_values=caches)[0][0, 0] for t in range(T)])
+    assert _rel(steps, O.stream_steps(x[0], params, heads, T)[0]) <= REL
+
+
 @pytest.mark.parametrize("C", [1, 21, 32, 33, 64, 65, 128])
 @pytest.mark.parametrize("step", [False, True])
 def test_few_rows_of_many_columns(C, step):
