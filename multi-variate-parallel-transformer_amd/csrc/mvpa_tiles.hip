@@ -333,9 +333,11 @@ __global__ __launch_bounds__(256) void tile_linear_kernel(const bf16_t* __restri
   using G = tile_cfg<WM, STAGES, CT>;
   static_assert(G::KH == 1, "one chain");
   extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
-  int col, row;
-  if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
-  const int64_t m0 = (int64_t)row * G::BM;
+  // An eighth of the tiles to an XCD, row tiles fastest.  (A column of tiles to an XCD left seven of them idle where there is one:
+  // [8,768] 9999 rows 15.8 -> 5.2 us, [64,4096] 16384 108 -> 22, and [768,2624] 1152 14.8 -> 11.4.)
+  const int total = ct * mt, per = (total + 7) / 8, id = (blockIdx.x & 7) * per + (blockIdx.x >> 3), col = id / mt;
+  if (id >= total) return;
+  const int64_t m0 = (int64_t)(id - col * mt) * G::BM;
   const int n0 = col * TL_BN, c = threadIdx.x & 7, n = n0 + c * 8;
   tile_product<WM, STAGES, CT>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, 0, K / TL_BK);
 #pragma unroll
@@ -482,14 +484,15 @@ static int launch_linear_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, c
   auto kern = tile_linear_kernel<WM, STAGES, CT>;
   want_dynamic_lds((const void*)kern, G::LDS);
   const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
-  MVPA_LAUNCH(kern, dim3((unsigned)((ct + 7) / 8 * 8 * mt)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, y, ldy, ct, mt);
+  MVPA_LAUNCH(kern, dim3((unsigned)((ct * mt + 7) / 8 * 8)), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, y, ldy, ct, mt);
   return take_launch_status();
 }
 
 // Where 256-row tiles leave most CUs without work, and below 512 rows, where they are not used.  us, large tiles (below 512 rows
-// the 128 x 128 ones) / these: [768,768] 130 rows 19.8 / 4.4, 525 13.7 / 5.2, 1600 14.0 / 7.4, 3000 (288 tiles) 14.3 / 12.0, 4096
-// (384) 14.6 / 14.9; [768,2624] 525 35.5 / 10.0, 3000 36.9 / 31.0, 4096 37.4 / 42.6; [2048,2048] 130 40.5 / 8.1, 1152 (288)
-// 28.2 / 18.0, 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1; [2048,576] 1152 11.3 / 8.2, 2048 11.4 / 12.0.
+// the 128 x 128 ones) / these: [768,768] 129 rows 20.4 / 5.1, 525 11.9 / 5.2, 1600 12.2 / 6.8, 3000 (288 tiles) 14.2 / 11.3; [768,2624] 525
+// 35.2 / 10.3, 3000 38.0 / 28.9; [2048,2048] 129 40.7 / 8.3, 1152 (288) 28.9 / 19.2; [2048,576] 1152 10.5 / 8.3; [8,768] 16384 (128) 13.7 /
+// 5.3; [256,8192] 4096 (128) 97.5 / 40.6.  Past the line, before the XCDs shared the tiles: [768,768] 4096 rows (384) 14.6 / 14.9, [768,2624]
+// 37.4 / 42.6, [2048,2048] 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1, [2048,576] 2048 11.4 / 12.0.
 bool tile_linear_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, const void* y) {
   const int64_t ct = (N + TL_BN - 1) / TL_BN;
   return M > 128 && K % TL_BK == 0 && N % 8 == 0 && ldy % 8 == 0 && ((uintptr_t)y & 15) == 0 && M < (1 << 20) && N < (1 << 20) &&

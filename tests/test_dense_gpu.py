@@ -51,7 +51,8 @@ def test_linear_gated(M, N, K):
 # one block, fewer blocks than the ring holds, as many, a few more and many; rows and columns either side of a tile; tiles of 64 rows
 # (525 x 768, 512 x 2048) and of 128 (576 x 2048, 1024 x 2048); N short of a whole tile
 @pytest.mark.parametrize("M,N,K", [(129, 8, 64), (192, 72, 128), (193, 64, 320), (525, 768, 384), (512, 2048, 192), (576, 2048, 64),
-                                   (577, 2040, 192), (1024, 2048, 256), (525, 768, 2624)])
+                                   (577, 2040, 192), (1024, 2048, 256), (525, 768, 2624),
+                                   (16385, 8, 64), (9999, 104, 192), (16400, 72, 128), (12288, 192, 64)])     # fewer columns of tiles than XCDs
 def test_linear_on_small_tiles(M, N, K):
     """Few tiles of 256 rows: the product on smaller ones, into rows of an x with another pitch, against float64, and the same bits
     as on large tiles (every sum is one chain over K there too)."""
