@@ -431,15 +431,26 @@ __device__ inline void dma_to_lds_16(const void* gptr, uint32_t lds_base) {
 // XCD is given an eighth of that walk: the 32 workgroups that it runs side by side cover GM rows x 32/GM
 // columns of tiles and read GM + 32/GM operand panels between them instead of one panel per workgroup and more.
 // (Tile rows that are no multiple of 32 went row by row over all XCDs: [7000,768]·[3456,768]ᵀ 45.3 -> 40.3 us, 12000 rows
-// 86 -> 75, [5000,7680]·[2048,7680]ᵀ 172 -> 161, 6400 rows 42.5 -> 39.7.)
-__device__ inline void tile_of_workgroup(int64_t L, int64_t mt64, int64_t nt64, int64_t* tm, int64_t* tn) {
+// 86 -> 75, [5000,7680]·[2048,7680]ᵀ 172 -> 161, 6400 rows 42.5 -> 39.7.)  They still do where the contraction is a block or
+// two: panels cost nothing there, and y goes out in the order of memory (row by row / in groups, us: [1600,64]·[4096,64]ᵀ 5.4 / 5.9,
+// [3000,64]·[8192,64]ᵀ 13.2 / 14.0, [12800,64]·[3456,64]ᵀ 21.8 / 24.7; from 128 columns on either is the faster one by turns).
+__device__ inline void tile_of_workgroup(int64_t L, int64_t mt64, int64_t nt64, int64_t K, int64_t* tm, int64_t* tn) {
   constexpr int GM = 4;
-  const int mt = (int)mt64, nt = (int)nt64, xcd = (int)(L & 7), total = mt * nt, per = total / 8;
-  const int id = xcd * per + min(xcd, total - per * 8) + (int)(L >> 3);
-  const int g = id / (GM * nt), r = id - g * (GM * nt), rows = min(GM, mt - g * GM);
+  const int mt = (int)mt64, nt = (int)nt64;
+  int m, n;
+  if (K < 128 && mt % (8 * GM) != 0) {
+    m = (int)L / nt;
+    n = (int)L - m * nt;
+  } else {
+    const int xcd = (int)(L & 7), total = mt * nt, per = total / 8;
+    const int id = xcd * per + min(xcd, total - per * 8) + (int)(L >> 3);
+    const int g = id / (GM * nt), r = id - g * (GM * nt), rows = min(GM, mt - g * GM);
+    n = r / rows;
+    m = g * GM + r - n * rows;
+  }
   // (wave-uniform by construction; said so to the compiler, which keeps them in scalar registers)
-  *tn = __builtin_amdgcn_readfirstlane(r / rows);
-  *tm = __builtin_amdgcn_readfirstlane(g * GM + r % rows);
+  *tn = __builtin_amdgcn_readfirstlane(n);
+  *tm = __builtin_amdgcn_readfirstlane(m);
 }
 
 // ---- epilogue of the large-tile kernels, through LDS (LDS_BYTES of it, idle by now).
@@ -609,7 +620,7 @@ __global__ __launch_bounds__(512) void linear_bf16_big_kernel(const bf16_t* __re
   // per-lane source rows of this wave's loads (row clamped into range: such rows are never stored)
   auto set_tile = [&](int64_t L) {
     int64_t tile_m, tile_n;
-    tile_of_workgroup(L, mt, nt, &tile_m, &tile_n);
+    tile_of_workgroup(L, mt, nt, K, &tile_m, &tile_n);
     m0 = tile_m * BM;
     n0 = tile_n * OUT_COLS;
     const int rsub = lane >> 3, phys = lane & 7;
@@ -761,7 +772,7 @@ __global__ __launch_bounds__(512) void linear_bf16_ring_kernel(const bf16_t* __r
   const int wm = wave >> 1, wc = wave & 1;
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;    // output columns per workgroup
   int64_t tile_m, tile_n;
-  tile_of_workgroup(blockIdx.x, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, &tile_m, &tile_n);
+  tile_of_workgroup(blockIdx.x, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, K, &tile_m, &tile_n);
   const int64_t m0 = tile_m * BM, n0 = tile_n * OUT_COLS;
   const int nkb = (int)(K / BK);
 
@@ -944,7 +955,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   const int wm = wave >> 1, wc = wave & 1;
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;    // output columns per workgroup
   int64_t tile_m, tile_n;
-  tile_of_workgroup(tile, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, &tile_m, &tile_n);
+  tile_of_workgroup(tile, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, K, &tile_m, &tile_n);
   const int64_t m0 = tile_m * BM, n0 = tile_n * OUT_COLS;
   const int nkb = (int)(K / BK);
 
