@@ -8,8 +8,9 @@
 // their way from LDS while this one is multiplied (with a block's fragments read where its products stand, a few
 // at a time: 32 rows of x, [768,2624] weights 9.8 -> 6.0 us, [2048,2048] 8.7 -> 5.8; 128 x 64 tiles 16.1 -> 13.6).
 //   4 waves.  WM = 4: a wave owns 32 rows of x and all 64 columns.  WM = 2 / 1: two / four waves share
-//   the rows and take 32 / 16 of every 64 k each, so that a wave always holds two 32 x 32 tiles (for the gated
-//   product: the gate and the up columns of an output).  128 columns: twice the waves.
+//   the rows and take 32 / 16 of every 64 k each, so that a wave holds two 32 x 32 tiles (for the gated
+//   product: the gate and the up columns of an output); a product by itself on 64 rows, whose sums stay one chain, one a
+//   wave.  128 columns: twice the waves.
 //   The sums go through LDS by rows and every thread finishes and stores 16 bytes of a row: stored as the
 //   products leave them, 8 or 16 bytes of each of 32 rows per instruction, the partial sums of 525 rows of 768
 //   alone took 3 us.
@@ -186,14 +187,14 @@ __device__ inline bool tile_coords(int id, int ct, int mt, int& col, int& row) {
 }
 
 // What a row tile of WM * 32 rows does: the last one of `mt` where few rows are left takes a smaller one, in whose blocks x
-// is less (525 rows: 13 of them are left to a fifth tile of 128).  33 .. 64 rows from five tiles on: with fewer, all tiles run
-// at about the same time and the smaller one, which splits the contraction over its waves, is the last to end (windows of
-// MVPFormer-S, as a tile of 128 / of 64, us: 192 rows 442 / 451, 320 359 / 367; 8 blocks of the base model: 448 rows 882 /
-// 907, 576 1136 / 1119, 704 1233 / 1204).
+// is less (525 rows: 13 of them are left to a fifth tile of 128).  Up to 32 rows from `least` tiles on: of two, the smaller one, whose
+// waves split every block, is the last to end ([q/k/v | gate/up] of width 4096, 129 rows 90 us, 192 rows without it 78).  33 .. 64 rows
+// from five tiles on; with fragments a block ahead it takes as long as a whole one there (us, [q/k/v | gate/up] of MVPFormer-S, as a tile of
+// 128 / of 64: 560 rows 9.7 / 9.7, 832 14.1 / 13.9; the base model 832 70.7 / 74.3, 704 59.4 / 59.0; tail products 1 % either way).
 template <int WM, int STAGES, typename F>
-__device__ __forceinline__ void for_rows_left(int64_t rows, int mt, F f) {
+__device__ __forceinline__ void for_rows_left(int64_t rows, int mt, int least, F f) {
   if constexpr (WM == 4 && STAGES == 3) {
-    if (rows <= 32) f(std::integral_constant<int, 1>(), std::integral_constant<int, 6>());
+    if (rows <= 32 && mt >= least) f(std::integral_constant<int, 1>(), std::integral_constant<int, 6>());
     else if (rows <= 64 && mt > 4) f(std::integral_constant<int, 2>(), std::integral_constant<int, 4>());
     else f(std::integral_constant<int, 4>(), std::integral_constant<int, 3>());
     static_assert(tile_cfg<1, 6>::LDS <= tile_cfg<4, 3>::LDS && tile_cfg<2, 4>::LDS <= tile_cfg<4, 3>::LDS, "LDS of the launch");
@@ -286,13 +287,13 @@ __global__ __launch_bounds__(BN * 4) void tile_dual_kernel(const bf16_t* __restr
   int col, row;
   if (!tile_coords(blockIdx.x, ct, mt, col, row)) return;
   const int64_t m0 = (int64_t)row * 32 * WM;
-  for_rows_left<WM, STAGES>(M - m0, mt, [&](auto wm, auto stages) {
+  for_rows_left<WM, STAGES>(M - m0, mt, 3, [&](auto wm, auto stages) {
     tile_dual<wm(), stages(), BN>(tl_lds, X, M, K, ldx, W0, N0, ldw0, out, gt, nrm, gated_ct, col, m0);
   });
 }
 
-template <int WM, int STAGES>
-__global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
+template <int WM, int STAGES, int BN>
+__global__ __launch_bounds__(BN * 4) void tile_partial_kernel(const bf16_t* __restrict__ X, int64_t M, int K, int64_t ldx,
                                                            const bf16_t* __restrict__ W, int N, int64_t ldw,
                                                            float* __restrict__ P, tile_split sp, int ct, int mt, bool spread) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char tl_lds[];
@@ -315,13 +316,15 @@ __global__ __launch_bounds__(256) void tile_partial_kernel(const bf16_t* __restr
   const int kb0 = z < sp.a ? z * sp.per_a : sp.nkb_a + (z - sp.a) * sp.per_b;
   const int kb1 = z < sp.a ? min(kb0 + sp.per_a, sp.nkb_a) : min(kb0 + sp.per_b, K / TL_BK);
   const int64_t m0 = (int64_t)row * 32 * WM;
-  const int n0 = col * TL_BN, c = threadIdx.x & 15, n = n0 + c * 4;
-  for_rows_left<WM, STAGES>(M - m0, mt, [&](auto wm, auto stages) {
-    using G = tile_cfg<wm(), stages()>;
-    tile_product<wm(), stages()>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0, kb1);
+  // 256 threads finish 64 columns
+  const int n0 = col * BN, part = BN > TL_BN ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, c = threadIdx.x & 15;
+  const int n = n0 + part * TL_BN + c * 4;
+  for_rows_left<WM, STAGES>(M - m0, mt, 2, [&](auto wm, auto stages) {
+    using G = tile_cfg<wm(), stages(), 2, BN>;
+    tile_product<wm(), stages(), 2, BN>(tl_lds, X, ldx, m0, M, W, ldw, [&](int r) { return (int64_t)min(n0 + r, N - 1); }, kb0, kb1);
 #pragma unroll
-    for (int r = threadIdx.x >> 4; r < G::BM; r += 16)
-      if (m0 + r < M && n < N) *(float4*)(P + ((int64_t)z * M + m0 + r) * N + n) = tile_sum<G>(tl_lds, r, c);
+    for (int r = (threadIdx.x & 255) >> 4; r < G::BM; r += 16)
+      if (m0 + r < M && n < N) *(float4*)(P + ((int64_t)z * M + m0 + r) * N + n) = tile_sum<G>(tl_lds + part * G::SUMS, r, c);
   });
 }
 
@@ -467,12 +470,15 @@ int launch_tile_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const b
   if (rows == 32) return launch_dual_t<1, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (rows == 64) return launch_dual_t<2, 5>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   if (M <= 128) return launch_dual_t<4, 6>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
-  // Where most CUs would hold two tiles of 128 x 64 that read the same x twice: one of 128 x 128 on eight waves instead.  Passes,
-  // 64 / 128 columns, us: base model (two boxes) 192 rows (360 tiles' worth) 1424 / 1364 .. 1421, 209 1463 / 1394 .. 1446, 256 1594 / 1485 ..
-  // 1522; MVPFormer-S 640 (370) 417 / 410, 768 (444) 457 / 451, but 396 (229) 404 / 407, 414 (239) 381 / 383, 525 (304) 459 / 461.
+  // Where a CU would hold two tiles of 128 x 64, which read the same x twice and share its LDS unevenly with CUs that hold one: one of
+  // 128 x 128 on eight waves instead, as long as they are one a CU.  us, 64 / 128 columns: base model, 129 rows 24.4 / 20.4, 192 22.1 / 20.3, 256
+  // 23.5 / 21.5; MVPFormer-S 385 9.8 / 9.6, 525 10.0 / 9.8, 768 10.9 / 10.5; one of 64 columns a CU: S 300 7.3 / 9.4.  Chains of a few
+  // blocks keep the narrow ones (256 columns, 1200 rows 6.7 / 6.9).  More than one a CU: long chains whose last round is more than half
+  // full, or of many rounds (base 300 rows, 1.4 rounds, 31.4 / 34.7, 512, 1.9, 41.8 / 39.7; width 4096 129, 1.7, 90 / 66, 640, 4.3, 184 / 174; S
+  // 800, 1.0, 14.1 / 17.4, 1600, 1.9, 21.4 / 26.7).
   const int64_t cols = (gated.w ? (gated.N + 31) / 32 : 0) + (w0 ? (N0 + TL_BN - 1) / TL_BN : 0);
-  const int64_t wide = (gated.w ? (gated.N + 63) / 64 : 0) + (w0 ? (N0 + 127) / 128 : 0);
-  if (M * cols > 128 * 352 && (M + 127) / 128 * wide <= 256)
+  const int64_t mt = (M + 127) / 128, wide = mt * ((gated.w ? (gated.N + 63) / 64 : 0) + (w0 ? (N0 + 127) / 128 : 0));
+  if (mt * cols > 256 && K >= 8 * TL_BK && (wide <= 256 || (K >= 24 * TL_BK && ((wide - 1) % 256 >= 128 || wide > 5 * 256))))
     return launch_dual_t<4, 4, 128>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
   return launch_dual_t<4, 3>(x, M, K, ldx, w0, N0, ldw0, out, gated, norm, s);
 }
@@ -529,20 +535,19 @@ tile_split make_tile_split(int64_t M, int64_t N, int64_t K, int64_t Ka) {
   return sp;
 }
 
-template <int WM, int STAGES>
+template <int WM, int STAGES, int BN = TL_BN>
 static int launch_partial_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw,
                             float* P, const tile_split& sp, hipStream_t s) {
-  using G = tile_cfg<WM, STAGES>;
-  auto kern = tile_partial_kernel<WM, STAGES>;
+  using G = tile_cfg<WM, STAGES, 2, BN>;
+  auto kern = tile_partial_kernel<WM, STAGES, BN>;
   want_dynamic_lds((const void*)kern, G::LDS);
-  const int ct = (int)((N + TL_BN - 1) / TL_BN), mt = (int)((M + G::BM - 1) / G::BM);
+  const int ct = (int)((N + BN - 1) / BN), mt = (int)((M + G::BM - 1) / G::BM);
   // A part's columns of x to an XCD, but for four row tiles of an x that the L2 of each (4 MB) holds as a whole.  Windows of
-  // MVPFormer-S (2496 columns), part to an XCD / spread, us: 130 rows 418 / 427, 256 356 / 357, 288 362 / 367, 384 369 / 366,
-  // 406 383 / 380, 448 390 / 380, 512 405 / 391, 525 443 / 447; eight blocks of the base model (7680), 406 rows 859 / 871, 448
-  // 887 / 899.
+  // MVPFormer-S (2496 columns), part to an XCD / spread, us: 384 rows (three tiles) 343 / 351, 392 368 / 366, 416 370 / 369, 448 373 / 370, 480
+  // 377 / 372, 512 375 / 367; four blocks of the base model (7680), 448 rows 412 / 411.
   const bool spread = mt == 4 && M * K * 2 <= (4 << 20);
   const int ids = spread ? (ct * sp.total() + 7) / 8 * 8 * mt : (ct * sp.total() * mt + 7) / 8 * 8;
-  MVPA_LAUNCH(kern, dim3((unsigned)ids), dim3(256), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, P, sp, ct, mt, spread);
+  MVPA_LAUNCH(kern, dim3((unsigned)ids), dim3(G::NW * 64), G::LDS, s, x, M, (int)K, ldx, w, (int)N, ldw, P, sp, ct, mt, spread);
   return take_launch_status();
 }
 
@@ -554,6 +559,12 @@ int launch_tile_partial(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, cons
   if (M <= 32) return launch_partial_t<1, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
   if (tile_rows(M, (N + TL_BN - 1) / TL_BN * splits.total()) <= 64) return launch_partial_t<2, 5>(x, M, K, ldx, w, N, ldw, P, splits, s);
   if (M <= 128) return launch_partial_t<4, 6>(x, M, K, ldx, w, N, ldw, P, splits, s);
+  // As in launch_tile_dual.  us, 64 / 128 columns: base model, 300 rows in 3 parts 24.6 / 21.4, 525 in 2 35.1 / 29.5, 1200 76.7 / 54.7; width 3072,
+  // 192 in 3 33.1 / 28.2, 768 99.6 / 71.8 (64 columns, fragments read where their products stand: 23.8, 32.8, 65.2, 30.5, 84.5);
+  // MVPFormer-S, 641 in 4 9.0 / 8.5, but one a CU: 600 6.8 / 8.4, 1024 rows of the base model 42.7 / 51.9.
+  const int64_t row_tiles = (M + 127) / 128 * splits.total();
+  if (row_tiles * ((N + TL_BN - 1) / TL_BN) > 256 && row_tiles * ((N + 127) / 128) <= 256 && splits.per_b >= 8)
+    return launch_partial_t<4, 4, 128>(x, M, K, ldx, w, N, ldw, P, splits, s);
   return launch_partial_t<4, 3>(x, M, K, ldx, w, N, ldw, P, splits, s);
 }
 

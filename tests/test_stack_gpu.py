@@ -135,20 +135,65 @@ def test_few_rows_of_many_columns(C, step):
     assert _rel(got, want) <= REL
 
 
-# 129 columns of tiles (an odd number of the gated ones): narrow, wide with 94 and 128 rows left to the last tile, narrow again;
-# an odd number in both products, the last gated one of 8 columns: wide with 62 and 128 rows left
-@pytest.mark.parametrize("C,T,dims", [(87, 4, dict(n_inner=4000)), (70, 5, dict(n_inner=4000)), (96, 4, dict(n_inner=4000)),
-                                      (77, 5, dict(n_inner=4000)), (82, 7, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=2024)),
-                                      (128, 5, dict(n_embd=320, n_head=5, n_head_kv=5, n_inner=2024))])
-def test_tiles_of_twice_the_columns(C, T, dims):
-    """Tiles of 128 rows and 128 columns of [q/k/v | gate/up] on either side of their range, against the stack in 64 bits."""
-    model = _model(**dims)
+def _wide(monkeypatch, **dims):
+    """A model whose scores are as wide as those of 128 columns (REL is for those), and a check that the stack call took it."""
+    model, native, taken = _model(**dims), MVPFormerModel._native, []
+    for n, p in model.named_parameters():
+        if "ln" not in n:
+            p.data.mul_((128 / model.embed_dim) ** 0.5)
+
+    def spy(self, *args):
+        out = native(self, *args)
+        taken.append(out is not None)
+        return out
+    monkeypatch.setattr(MVPFormerModel, "_native", spy)
+    heads = dict(n_layer=2, n_head=dims["n_head"], n_head_kv=dims["n_head_kv"])
+    return model, {n: p.detach() for n, p in model.named_parameters()}, heads, taken
+
+
+# [q/k/v | gate/up] of 130 columns of tiles an eight-wave tile takes two of: 1, 94 and 128 rows in the second of two tiles, one tile, more of the
+# wide ones than CUs; an odd number of columns; long chains past one a CU (1.5 and 1.4 rounds); the tail product: 780 rows in parts, an odd number
+# of columns with 20 rows left
+W512 = dict(n_embd=512, n_head=16, n_head_kv=1, n_inner=3840)
+W576 = dict(n_embd=576, n_head=18, n_head_kv=2, n_inner=3840)
+W1536 = dict(n_embd=1536, n_head=24, n_head_kv=1, n_inner=11520)
+
+
+@pytest.mark.parametrize("C,T,dims", [(43, 3, W512), (74, 3, W512), (64, 4, W512), (64, 2, W512), (103, 5, W512), (43, 3, W576), (51, 5, W576),
+                                      (74, 3, W1536), (43, 3, dict(W1536, n_inner=10240)), (111, 7, W512), (110, 6, W576)],
+                         ids=lambda v: str(v["n_embd"]) if isinstance(v, dict) else str(v))
+def test_tiles_of_twice_the_columns(monkeypatch, C, T, dims):
+    """Tiles of 128 rows and 128 columns on either side of their range, against the stack in 64 bits."""
+    model, params, heads, taken = _wide(monkeypatch, **dims)
     x = torch.randn(1, T, C, model.embed_dim, device="cuda").bfloat16()
     with torch.no_grad():
         got = model(inputs_embeds=x)
-    heads = dict(n_layer=2, n_head=dims.get("n_head", 2), n_head_kv=dims.get("n_head_kv", 1))
-    want = O.stack_forward(x, {n: p.detach() for n, p in model.named_parameters()}, heads, None)
-    assert _rel(got, want) <= REL
+    assert taken == [True] and _rel(got, O.stack_forward(x, params, heads, None)) <= REL
+
+
+@pytest.mark.parametrize("rings", [False, True])
+@pytest.mark.parametrize("B,C,dims", [(2, 74, W512), (3, 43, W576), (7, 111, W512)], ids=["148", "129", "777"])
+def test_steps_on_tiles_of_twice_the_columns(monkeypatch, B, C, dims, rings):
+    """The same tiles with keys and values that go to caches and rings, against the same steps in 64 bits."""
+    model, params, heads, taken = _wide(monkeypatch, **dims)
+    steps, W = 5, 3
+    xs = torch.randn(steps, B, 1, C, model.embed_dim, device="cuda").bfloat16()
+    caches, out = model.new_cache(B, C, max_steps=W), []
+    clock = MvpaRingClock(W, W - 1, "cuda")
+    with torch.no_grad():
+        for i, x in enumerate(xs):
+            if rings and i == W:
+                caches = tuple(MvpaRingCache.from_cache(c, clock) for c in caches)
+            if rings and i >= W:
+                clock.advance()
+            out.append(model(inputs_embeds=x, past_key_values=caches)[0])
+    assert taken == [True] * steps
+    for b in (0, B - 1):
+        ref, keys, _ = O.stream_steps(xs[:, b, 0], params, heads, W)
+        for got, want in zip(out, ref):
+            assert _rel(got[b, 0], want) <= REL
+        if not rings:
+            assert _rel(torch.stack([c.views()[0][b].permute(1, 2, 0, 3) for c in caches]), keys) <= REL
 
 
 @pytest.mark.parametrize("C,T,inner", [(125, 4, 4032), (128, 4, 4032), (96, 4, 448), (77, 5, 448), (103, 5, 448)])
