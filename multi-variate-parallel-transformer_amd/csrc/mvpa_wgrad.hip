@@ -33,7 +33,7 @@ __device__ inline bf16x8 frag(const unsigned char* p, int s) {
   return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-template <int GROUPS, bool PARTIAL>
+template <int GROUPS, bool PARTIAL, bool FAR = false>
 __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char all_stages[];
   const int tid = threadIdx.x, lane = tid & 63, ln = lane & 31, hh = lane >> 5;
@@ -61,12 +61,19 @@ __global__ __launch_bounds__(256 * GROUPS, 2) void linear_wgrad_kernel(args a) {
   auto request = [&](int kb, int stage) {
     const int64_t m0 = row_of(kb) + 4 * wave;
     const uint32_t dst = lds0 + stage * STAGE + 4 * wave * ROWB;
-    if (row_of(kb) + KB <= m_end) {
+    if (!FAR && row_of(kb) + KB <= m_end) {
       const bf16_t *y = a.dy + m0 * a.ldy, *x = a.x + m0 * a.ldx;
 #pragma unroll
       for (int i = 0; i < LOADS / 2; ++i) {
         load_to_lds_16(y + (int64_t)(16 * i) * a.ldy, off_y, dst + 16 * i * ROWB);
         load_to_lds_16(x + (int64_t)(16 * i) * a.ldx, off_x, dst + STAGE / 2 + 16 * i * ROWB);
+      }
+    } else if (FAR) {                            // rows farther apart than 32 bits of a block's bytes
+#pragma unroll
+      for (int i = 0; i < LOADS / 2; ++i) {
+        const int64_t m = min(m0 + 16 * i + row_l, m_end - 1);
+        load_to_lds_16(a.dy + m * a.ldy + col_y, dst + 16 * i * ROWB);
+        load_to_lds_16(a.x + m * a.ldx + col_x, dst + STAGE / 2 + 16 * i * ROWB);
       }
     } else {                                     // the last row again where there are no more
       const int64_t m1 = min(m0, m_end - 1);
@@ -243,7 +250,6 @@ extern "C" int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, i
   if (!dy || !x || !dw) return MVPA_ERR_NULL;
   if (M <= 0 || N <= 0 || K <= 0 || N > (1 << 20) || K > (1 << 20) || M > ((int64_t)1 << 30) || lddy < N || ldx < K || lddw < K)
     return MVPA_ERR_SHAPE;
-  if (lddy > (1 << 26) || ldx > (1 << 26)) return MVPA_ERR_UNSUPPORTED;      // 32-bit offsets from a block's first row
   if ((N | K | lddy | ldx | lddw) % 8 != 0 || (((uintptr_t)dy | (uintptr_t)x | (uintptr_t)dw | (uintptr_t)ws) & 15)) return MVPA_ERR_ALIGN;
   const wgrad::plan p = wgrad::plan_of(M, N, K);
   const size_t need = p.splits == 1 ? 0 : (size_t)p.splits * N * K * sizeof(float);
@@ -251,11 +257,15 @@ extern "C" int mvpa_linear_wgrad_bf16(const void* dy, const void* x, void* dw, i
   wgrad::args a{(const bf16_t*)dy, (const bf16_t*)x, p.splits > 1 ? ws : dw, lddy, ldx, lddw, (int32_t)M, (int32_t)N, (int32_t)K,
                 (int32_t)((K + wgrad::TILE - 1) / wgrad::TILE), p.splits, (int32_t)((M + wgrad::KB - 1) / wgrad::KB)};
   hipStream_t s = (hipStream_t)stream;
-  auto kern = p.groups == 2 ? p.splits > 1 ? wgrad::linear_wgrad_kernel<2, true> : wgrad::linear_wgrad_kernel<2, false>
+  // rows farther apart than 32 bits of a block's bytes: a handful of them fills the memory, any plan will do
+  const bool far = lddy > (1 << 26) || ldx > (1 << 26);
+  const int groups = far ? 1 : p.groups;
+  auto kern = far ? p.splits > 1 ? wgrad::linear_wgrad_kernel<1, true, true> : wgrad::linear_wgrad_kernel<1, false, true>
+            : groups == 2 ? p.splits > 1 ? wgrad::linear_wgrad_kernel<2, true> : wgrad::linear_wgrad_kernel<2, false>
                             : p.splits > 1 ? wgrad::linear_wgrad_kernel<1, true> : wgrad::linear_wgrad_kernel<1, false>;
-  const int lds = wgrad::STAGES * wgrad::STAGE * p.groups;
+  const int lds = wgrad::STAGES * wgrad::STAGE * groups;
   want_dynamic_lds((const void*)kern, lds);
-  MVPA_LAUNCH(kern, dim3((unsigned)(wgrad::tiles_of(N, K) * p.splits)), dim3(256 * p.groups), lds, s, a);
+  MVPA_LAUNCH(kern, dim3((unsigned)(wgrad::tiles_of(N, K) * p.splits)), dim3(256 * groups), lds, s, a);
   if (p.splits > 1)
     MVPA_LAUNCH(wgrad::linear_wgrad_reduce_kernel, dim3((unsigned)((N * K / 8 + 255) / 256)), dim3(256), 0, s, (const float*)ws,
                 (bf16_t*)dw, (int)N, (int)K, lddw, p.splits);

@@ -339,6 +339,17 @@ def test_gradients_of_several_losses_at_once():
             _near(whole[i], one)
 
 
+def test_weight_gradient_of_rows_far_apart():
+    """Row pitches past 32 bits of a block's bytes: 40 rows of a view into 5.4 GB, either operand."""
+    pitch = (1 << 26) + 8
+    far = torch.empty(40 * pitch, dtype=torch.bfloat16, device="cuda").view(40, pitch)[:, :136]
+    near = torch.randn(40, 264, device="cuda").bfloat16()
+    far.copy_(torch.randn(40, 136, device="cuda").bfloat16())
+    for dy, x in ((far, near), (near, far)):
+        got = mvpa_hip.load_ext().linear_wgrad(dy, x)
+        _close(got, dy.double().T @ x.double(), 40)
+
+
 @pytest.mark.skipif(torch.cuda.device_count() < 2, reason="two GPUs")
 def test_operands_on_two_gpus_are_refused():
     """As tensor operations refuse them: no kernel reads another GPU's memory."""
