@@ -211,10 +211,13 @@ __global__ __launch_bounds__(256) void linear_wgrad_reduce_kernel(const float* _
 
 static int tiles_of(int64_t N, int64_t K) { return (int)((N + TILE - 1) / TILE * ((K + TILE - 1) / TILE)); }
 
-// How the rows are dealt, by what a launch was seen to take: a group of 4 waves 0.6 us a block where two share a
-// CU, partial results 2 x 4 bytes an output and share at 4.8 TB/s.  Both launches over 6400 rows, eight sets of them in
+// How the rows are dealt, by what launches were seen to take (every plan of 132 shapes: the one chosen here is 0.5 % behind the best on
+// average, 4 % with 0.6 us a block, 3 for a second launch and no more for a second group): a group of 4 waves 0.45 us a block
+// where two share a CU and 0.4 alone, the second group's sums 2.5, partial results one launch, 0.15 a share and 2 x 4 bytes an
+// output and share at 6 TB/s.  Both launches over 6400 rows, eight sets of them in
 // turn, us (vendor library): [3456,768] 53 (73), [768,1728] 32 (49), [1280,768] 26 (42), [768,768] 22 (39).  Pairs of groups
-// took 6 to 8 us off the last three.
+// took 6 to 8 us off the last three.  ([3456,768] over 5120 rows 42.7 -> 46.5 us when blocks became 32 rows, 43.1 with these costs; 64 rows of
+// [768,768] 7.65 -> 8.8 -> 7.75.)
 struct plan {
   int groups, splits;
 };
@@ -225,7 +228,9 @@ static plan plan_of(int64_t M, int64_t N, int64_t K) {
   for (int groups = 1; groups <= 2; ++groups)
     for (int s = 1; s <= 32 && (s == 1 || (int64_t)s * groups <= blocks); ++s) {
       const int64_t slots = 512 / groups, rounds = (tiles * s + slots - 1) / slots, each = (blocks + s * groups - 1) / (s * groups);
-      const double us = rounds * each * 0.6 + (s > 1 ? 3.0 + 8e-6 * s * N * K / 4.8 : 0.0);
+      const int64_t last = (tiles * s - (rounds - 1) * slots) * groups;          // groups of the last round
+      const double us = each * ((rounds - 1) * 0.45 + (last <= 256 ? 0.4 : 0.45)) + (groups - 1) * 2.5 +
+                        (s > 1 ? 1.0 + 0.15 * s + 8e-6 * s * N * K / 6.0 : 0.0);
       if (us < best_us) {
         best_us = us;
         best = {groups, s};
