@@ -39,7 +39,8 @@ namespace mvpa {
 // NCT = key-channel tiles a WAVE handles per key step; KH = parts the keys of a step are split
 // into (each part has its own waves, which keep a partial soft-max state over their keys and merge
 // at the end).  Queries and keys cover the same QT = NCT * KH tiles of 32 channels.
-template <int DH, int NCT, int NW, int STAGES, int KH = 1>
+// ALONE: whether the build has the last time step's own loop (SOLO below).
+template <int DH, int NCT, int NW, int STAGES, int KH = 1, bool ALONE = true>
 struct Cfg {
   static constexpr int QT = NCT * KH;          // 32-channel tiles per time step
   static constexpr int CP = QT * 32;           // padded channels per time step (rows of a K/V tile)
@@ -59,7 +60,7 @@ struct Cfg {
   // who takes the last time step, which keeps the content term for every key step: two pairs of waves in turn (SPLIT), or
   // every wave by itself on a stage of its own (SOLO); see the kernel
   static constexpr bool SPLIT = TQW == 2 && STAGES == 4 && KH == 1;
-  static constexpr bool SOLO = WPT == 1 && TQW > 2 && STAGES == 4;
+  static constexpr bool SOLO = ALONE && WPT == 1 && TQW > 2 && STAGES == 4;
   static constexpr int STB_AT = SOLO && NW > STAGES ? NW * STAGE_BYTES : RING_BYTES;   // the slabs lie behind all stages
   static constexpr int MAIN_BYTES = STB_AT + STB_BYTES;
   // (of short sequences the last step is hardly longer than the others, and its own workgroup is one more: B8 H16 C30 T16 Dh128
@@ -78,12 +79,12 @@ struct Cfg {
   static_assert(WLOADS % NW == 0 || WLOADS < NW, "every loading wave issues the same number of loads");
 };
 
-template <int DH, int NCT, int NW, int STAGES, int MINB, bool FP8, int KH, bool RUNS, typename E>
+template <int DH, int NCT, int NW, int STAGES, int MINB, bool FP8, int KH, bool RUNS, bool ALONE, typename E>
 __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args a) {
   using x8 = typename E::x8;                     // fragments of the element type (bf16 or fp16)
   using x4 = typename E::x4;
   using x2 = typename E::x2;
-  using G = Cfg<DH, NCT, NW, STAGES, KH>;
+  using G = Cfg<DH, NCT, NW, STAGES, KH, ALONE>;
   constexpr int CP = G::CP, KS = G::KS, MT = G::MT, ROWB = G::ROWB, CHUNKS = G::CHUNKS;
   extern __shared__ __attribute__((aligned(1024))) unsigned char smem_raw[];
   float* Stb_all = (float*)(smem_raw + G::STB_AT);              // [NW][32][32]
@@ -961,12 +962,27 @@ static int launch_one(const mvpa_fwd_args* a, hipStream_t stream) {
   const bool content = a->flags & MVPA_FLAG_CONTENT;
   if (ring && !content) return MVPA_ERR_UNSUPPORTED;      // the run build has no far path
   if (!content) n_split = 1;
-  auto kern = (n_split > 1 || ring) ? mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, true, E>
-                          : mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, false, E>;
-  mvpa::want_dynamic_lds((const void*)kern, (int)G::LDS_BYTES);
-  const int nt = G::time_tiles(a->T);
-  dim3 grid((unsigned)((last ? n_split : nt) * a->B * a->H));
-  MVPA_LAUNCH(kern, grid, dim3(G::THREADS), G::LDS_BYTES, stream, *a);
+  const bool runs = n_split > 1 || ring;
+  auto go = [&](auto cfg, auto kern) {
+    using L = decltype(cfg);
+    mvpa::want_dynamic_lds((const void*)kern, (int)L::LDS_BYTES);
+    dim3 grid((unsigned)((last ? n_split : L::time_tiles(a->T)) * a->B * a->H));
+    MVPA_LAUNCH(kern, grid, dim3(L::THREADS), L::LDS_BYTES, stream, *a);
+  };
+  // Too short for the last step's own loop: builds without it where only such launches come (head size 128, one workgroup a CU), and
+  // runs at head size 64 in fp8, where it lets two workgroups share a CU (122 registers and 64 KB, with it 159 and 96 KB; C21, 64
+  // steps in 4 runs, 512 / 2048 (b, h) and runs 41 / 112 us, with it 55 / 169)
+  using Short = Cfg<DH, NCT, NW, STAGES, KH, false>;
+  constexpr bool ONLY_SHORT = DH == 128 && MINB == 1, TWO_A_CU = FP8 && DH == 64 && G::SOLO;
+  if constexpr (ONLY_SHORT) {
+    if (runs) go(Short(), mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, true, false, E>);
+    else go(Short(), mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, false, false, E>);
+  } else {
+    if (TWO_A_CU && runs && !G::solo((a->T + n_split - 1) / n_split))
+      go(Short(), mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, true, !TWO_A_CU, E>);
+    else if (runs) go(G(), mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, true, true, E>);
+    else go(G(), mvpa_mfma_kernel<DH, NCT, NW, STAGES, MINB, FP8, KH, false, true, E>);
+  }
   if (n_split > 1) launch_merge<E>(a, stream);
   return mvpa::take_launch_status();
 }
@@ -1039,9 +1055,10 @@ int mvpa_launch_mfma(const mvpa_fwd_args* a, hipStream_t stream) {
       // (4 query tiles x 2 key parts), two waves per SIMD
       return launch_cfg<64, 2, 8, 3, 1, 2>(a, stream);
     case 128:
-      // two workgroups per CU (2 x 80 KiB, 50 to 80 registers spilled in the slabs) where the far steps are many: B3 H16 C19 T511
-      // 3931 -> 2065 us, B8 C32 T128 966 -> 643, B8 C25 T64 329 -> 237, T32 127 -> 107, but B4 C30 T24 43 -> 74 and
-      // B8 T16 52 -> 66
+      // two workgroups per CU (2 x 80 KiB, 50 to 80 registers spilled in the slabs) from 32 steps on, on few workgroups as well: one / two, us: B3
+      // H16 C19 T511 3931 / 2065, B8 C32 T128 966 / 643, B8 C25 T32 127 / 107, but B4 C30 T24 43 / 74 and B8 T16 52 / 66; grids of up to 256
+      // workgroups 0.95 of the time (fp8 0.85), B1 H4 C21 T150 98.6 / 88 down to H12 T80 63.6 / 64.5; last steps alone T64 of 128 (b, h) 30.2 /
+      // 31.9, of 300 62 / 50 (fp8 59 / 60, 105 / 84)
       if (nct == 1 && a->T >= 32) return launch_cfg<128, 1, 4, 4, 2>(a, stream);
       if (nct == 1) return launch_cfg<128, 1, 4, 4>(a, stream);
       if (nct == 2) return launch_cfg<128, 2, 4, 3>(a, stream);

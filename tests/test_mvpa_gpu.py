@@ -945,6 +945,10 @@ LAST_STEP_SHAPES = [
     dict(B=2, C=20, T=40, H=2, Hkv=1, Dh=64),      # 8 waves = 8 time steps per workgroup: 7 of them idle
     dict(B=1, C=64, T=9, H=2, Hkv=2, Dh=128),
     dict(B=3, C=8, T=1, H=1, Hkv=1, Dh=32),        # nothing cached yet
+    dict(B=1, C=20, T=31, H=2, Hkv=1, Dh=128),     # either side of the last step's own workgroup
+    dict(B=1, C=20, T=40, H=2, Hkv=1, Dh=128),
+    dict(B=1, C=21, T=90, H=2, Hkv=2, Dh=64),
+    dict(B=1, C=30, T=81, H=2, Hkv=1, Dh=32),
 ]
 
 
@@ -979,6 +983,12 @@ SPLIT_CASES = [
     (dict(B=1, C=97, T=66, H=2, Hkv=1, Dh=128), 2),
     (dict(B=1, C=70, T=200, H=2, Hkv=1, Dh=64), 2),
     (dict(B=1, C=128, T=72, H=2, Hkv=2, Dh=32), 2),
+    (dict(B=2, C=20, T=158, H=2, Hkv=1, Dh=64), 2),     # runs of 79 and of 80 steps, of 80 with 79 left, on one build and the other
+    (dict(B=2, C=20, T=160, H=2, Hkv=1, Dh=64), 2),
+    (dict(B=1, C=32, T=239, H=2, Hkv=2, Dh=64), 3),
+    (dict(B=1, C=21, T=24, H=2, Hkv=1, Dh=128), 2),
+    (dict(B=1, C=21, T=40, H=2, Hkv=1, Dh=128), 3),
+    (dict(B=1, C=21, T=99, H=2, Hkv=1, Dh=128), 3),
 ]
 
 
