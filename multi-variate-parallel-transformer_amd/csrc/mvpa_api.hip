@@ -126,12 +126,13 @@ extern "C" int mvpa_forward(const mvpa_fwd_args* a, void* stream) {
     // at 4 181 : 197; head size 32 T 100 at 16 35.0 : 32.9, T 200 at 8 57 : 47, T 250 at 8 68.4 : 66.6, T 500 at 4 122 : 160.
     // 33..64 channels, by workgroups, T 12 at 576 / 1152 17.3 : 13.5, 19.1 : 22.3; T 16 at 768 19.1 : 16.3; T 25
     // at 600 / 800 / 1200 23.2 : 16.9, 23.6 : 21.6, 25.9 : 26.7; T 40 at 960 29.5 : 35.4; Dh 32 at 768 / 1600 18.1 : 13.5,
-    // 24.8 : 26.8.  Head size 128 has one workgroup per CU, the general kernel two from T 32: C21 H16 T 25 36 : 20, T 48 45 : 36,
-    // T 64 51 : 50, T 96 74 : 84, T 128 89 : 123; H24 T 32 37 : 30, T 64 61 : 70.
+    // 24.8 : 26.8.  Head size 128 has one workgroup per CU, the general kernel two from T 32, C21 by workgroups: T 32 at 1024 / 1280
+    // 37.3 : 38.5, 48.2 : 48.1; T 48 at 1152 / 1536 51.4 : 50.5, 55.0 : 63.0; T 64 at 1024 / 1536 52.0 : 48.3, 63.3 : 69.5; T 100 at 1200 / 1600
+    // 83 : 66, 79 : 86; T 128 at 1024 78 : 66; T 25 at 400 36 : 20.
     if (!(a->flags & MVPA_FLAG_LAST_STEP) && a->C <= (a->Dh == 128 ? 32 : 64) && mvpa_wave_supported(a)) {
       const int64_t wgs = (int64_t)a->B * a->H * ((a->C + 31) / 32) * a->T, T = a->T;
       int64_t most = 512;
-      if (a->Dh == 128) most = T >= 32 ? 1024 : 24 * T > most ? 24 * T : most;
+      if (a->Dh == 128) most = T >= 32 ? 1200 : 24 * T > most ? 24 * T : most;
       else if (a->C > 32) most = T <= 32 ? 768 : most;
       else if (T >= (a->Dh == 32 ? 257 : 80)) most = 1200;
       else if (48 * T > most) most = 48 * T < 2048 ? 48 * T : 2048;
