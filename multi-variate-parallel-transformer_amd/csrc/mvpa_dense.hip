@@ -432,25 +432,27 @@ __device__ inline void dma_to_lds_16(const void* gptr, uint32_t lds_base) {
 // columns of tiles and read GM + 32/GM operand panels between them instead of one panel per workgroup and more.
 // (Tile rows that are no multiple of 32 went row by row over all XCDs: [7000,768]·[3456,768]ᵀ 45.3 -> 40.3 us, 12000 rows
 // 86 -> 75, [5000,7680]·[2048,7680]ᵀ 172 -> 161, 6400 rows 42.5 -> 39.7.)  They still do where the contraction is a block or
-// two: panels cost nothing there, and y goes out in the order of memory (row by row / in groups, us: [1600,64]·[4096,64]ᵀ 5.4 / 5.9,
-// [3000,64]·[8192,64]ᵀ 13.2 / 14.0, [12800,64]·[3456,64]ᵀ 21.8 / 24.7; from 128 columns on either is the faster one by turns).
+// two, panels cost nothing and y goes out in the order of memory, and up to 511 columns where many columns of tiles are a multiple
+// of 8, so that each belongs to one XCD as it is (row by row / in groups, us: [1600,64]·[4096,64]ᵀ 5.4 / 5.9, [3000,64]·[8192,64]ᵀ 13.2 /
+// 14.0, [12800,64]·[3456,64]ᵀ 21.8 / 24.7; [1600,192]·[4096,192]ᵀ 7.7 / 8.4, [5000,256]·[8192,256]ᵀ 34.5 / 37, [3000,256]·[16384,256]ᵀ 0.92 of the
+// time, but [12800,192]·[4096,192]ᵀ 44 / 40; from 768 columns on level).
 __device__ inline void tile_of_workgroup(int64_t L, int64_t mt64, int64_t nt64, int64_t K, int64_t* tm, int64_t* tn) {
-  constexpr int GM = 4;
-  const int mt = (int)mt64, nt = (int)nt64;
-  int m, n;
-  if (K < 128 && mt % (8 * GM) != 0) {
-    m = (int)L / nt;
-    n = (int)L - m * nt;
+  constexpr uint32_t GM = 4;
+  const uint32_t mt = (uint32_t)mt64, nt = (uint32_t)nt64, id0 = (uint32_t)L;
+  uint32_t m, n;
+  if (mt % (8 * GM) != 0 && (K < 128 || (K < 512 && nt >= 32 && nt % 8 == 0))) {
+    m = id0 / nt;
+    n = id0 - m * nt;
   } else {
-    const int xcd = (int)(L & 7), total = mt * nt, per = total / 8;
-    const int id = xcd * per + min(xcd, total - per * 8) + (int)(L >> 3);
-    const int g = id / (GM * nt), r = id - g * (GM * nt), rows = min(GM, mt - g * GM);
+    const uint32_t xcd = id0 & 7, total = mt * nt, per = total / 8, group = GM * nt;
+    const uint32_t id = xcd * per + min(xcd, total - per * 8) + (id0 >> 3), g = id / group, r = id - g * group;
+    const uint32_t rows = min(GM, mt - g * GM);
     n = r / rows;
     m = g * GM + r - n * rows;
   }
   // (wave-uniform by construction; said so to the compiler, which keeps them in scalar registers)
-  *tn = __builtin_amdgcn_readfirstlane(n);
-  *tm = __builtin_amdgcn_readfirstlane(m);
+  *tn = __builtin_amdgcn_readfirstlane((int)n);
+  *tm = __builtin_amdgcn_readfirstlane((int)m);
 }
 
 // ---- epilogue of the large-tile kernels, through LDS (LDS_BYTES of it, idle by now).

@@ -17,6 +17,8 @@ pytestmark = pytest.mark.gpu
                                    (600, 130, 128), (1000, 200, 192), (5000, 333, 256), (513, 257, 1024),
                                    # fewer than 128 columns: tiles row by row, 20 and 64 rows of them, one column
                                    (5000, 2056, 64), (16384, 1000, 96), (40000, 130, 120), (5000, 777, 127),
+                                   # 32 and 64 columns of tiles, the last one ragged
+                                   (1100, 4090, 128), (2900, 8185, 448),
                                    # at most 128 rows: the K-split kernel of a decoding step
                                    (64, 1280, 768), (64, 768, 1728), (33, 130, 550), (1, 768, 768), (20, 100, 72),
                                    (32, 2048, 5632), (128, 2048, 2048), (100, 3072, 2048), (65, 96, 24)])
