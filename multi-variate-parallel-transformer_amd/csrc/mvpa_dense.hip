@@ -1543,14 +1543,15 @@ __global__ __launch_bounds__(256) void wavedec_db4_kernel(const float* __restric
 // is: trips to memory, so the samples come in groups and the norm's weight ahead of the levels.  us, taps with a stride of two floats and
 // two barriers a level / pairs of outputs a thread, samples one by one, weight and sum of squares at the end / now: 64 rows of 512 7.9 /
 // 8.2 / 7.3, 16384 of 512 34.0 / 29.9 / 26.7, 64 of 2560 8.5 / 9.7 / 8.2, 6400 of 2560 60 / 51 / 45, 64 of 4095 11.0 / 15.4 / 10.9, 6400 of
-// 1001 44 / 47 / 29, but 16384 of 64 11.3 / 14.2 / 13.3.
+// 1001 44 / 47 / 29, 6400 of 97 7.1 / 8.3 / 7.1, but 16384 of 64 11.3 / 14.2 / 12.1.  SHORT (levels of at most 64 outputs, rows of up to 121
+// samples): one output a thread and level, the loops of longer rows left out (without this build 13.3).
 // With coef_out (row pitch ldy) and inv_out the coefficients and the factor of every row leave as well: a
 // training pass wants them for the gradient of the norm's weight (norm_dw_kernel).
 // -----------------------------------------------------------------------------------------
 // floats of the even (or odd) samples of n, four in front and behind for the wrap
 __host__ __device__ constexpr int wavedec_half(int n) { return (4 + (n + 1) / 2 + 4 + 3) & ~3; }
 
-template <int G>
+template <int G, bool SHORT>
 __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* __restrict__ x,
                                                                   const float* __restrict__ w,
                                                                   bf16_t* __restrict__ y, float* __restrict__ coef_out,
@@ -1585,11 +1586,11 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
   float g0[8] = {}, g1[8] = {};                     // (of whole groups; the last one's lie a column a lane)
   if (vec_w) {
     weights(t * 8, g0);
-    if (ldy > G * 8) weights((t + G) * 8, g1);
+    if (!SHORT && ldy > G * 8) weights((t + G) * 8, g1);
   }
   const float last_w = w[min((dwt_size & ~7) + (t & 7), dwt_size - 1)];
   if (vec_x) {
-    constexpr int U = G == 64 ? 2 : 4;
+    constexpr int U = SHORT ? 1 : G == 64 ? 2 : 4;
     for (int i0 = 0; i0 < L / 4; i0 += U * G) {
       float4 v[U];
 #pragma unroll
@@ -1604,7 +1605,7 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
       }
     }
   } else {
-    constexpr int U = G == 64 ? 4 : 8;
+    constexpr int U = SHORT ? 2 : G == 64 ? 4 : 8;
     float* mine = (t & 1 ? odd : even) + (t >> 1);
     for (int i0 = 0; i0 < L; i0 += U * G) {
       float v[U];
@@ -1651,11 +1652,11 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
       coef[at + k] = hi;
       ss = fmaf(hi, hi, ss);
     };
-    for (int k0 = 0; k0 < m; k0 += 2 * threads) {
+    for (int k0 = 0; SHORT ? k0 == 0 : k0 < m; k0 += 2 * threads) {
       float lo, hi, lo2, hi2;
       const int k = k0 + t;
       taps(min(k, m - 1), lo, hi);
-      if (k0 + threads < m) {
+      if (!SHORT && k0 + threads < m) {
         taps(min(k + threads, m - 1), lo2, hi2);
         put(k, lo, hi);
         if (k + threads < m) put(k + threads, lo2, hi2);
@@ -1730,7 +1731,7 @@ __global__ __launch_bounds__(256) void wavedec_db4_rmsnorm_kernel(const float* _
       v[i] = c + i < dwt_size ? f[i] * inv * g : 0.f;          // (inv is NaN where a sample is: 0 x NaN would not do)
       g0[i] = g1[i];
     }
-    if (vec_w && c0 + 2 * G * 8 < dwt_size) weights(c + 2 * G * 8, g1);
+    if (!SHORT && vec_w && c0 + 2 * G * 8 < dwt_size) weights(c + 2 * G * 8, g1);
     if (c < ldy) {
       vec8<bf16_t>::store(y + row * ldy + c, v);
       if (coef_out) vec8<float>::store(coef_out + row * ldy + c, f);
@@ -2242,7 +2243,7 @@ static int launch_wavedec_rmsnorm(const float* x, const float* weight, void* y, 
   // one wave per row while four rows leave room for two workgroups per CU
   const bool wave = row_floats * 4 * 4 <= 80 * 1024;
   const int lds = row_floats * 4 * (wave ? 4 : 1);
-  auto kern = wave ? wavedec_db4_rmsnorm_kernel<64> : wavedec_db4_rmsnorm_kernel<256>;
+  auto kern = L <= 121 ? wavedec_db4_rmsnorm_kernel<64, true> : wave ? wavedec_db4_rmsnorm_kernel<64, false> : wavedec_db4_rmsnorm_kernel<256, false>;
   if (lds > 64 * 1024) mvpa::want_dynamic_lds((const void*)kern, lds);
   MVPA_LAUNCH(kern, dim3((unsigned)(wave ? (M + 3) / 4 : M)), dim3(256), lds, (hipStream_t)stream, x, weight, (bf16_t*)y,
               coeffs, inv, M, L, levels, dwt_size, ldy, eps, row_floats,
