@@ -19,12 +19,13 @@ namespace mvpa {
 
 // The 256-row tiles are the better ones once [q/k/v | gate/up] is this many of them, the more the longer the
 // contraction; a step's small tiles write the caches themselves and stand a little longer.  256-row against small
-// tiles, us a pass of all blocks at so many tiles,
-//   windows of MVPFormer-S   209 1425 : 1352, 228 1364 : 1386, 247 1418 : 1536, 285 1597 : 1710, 304 1664 : 1903,
-//                            342 1726 : 2141; 266 at 37 channels 1690 : 1624
-//   of the base model        360 7849 : 7311, 420 7894 : 7989, 480 7762 : 8403, 600 9818 : 11661
-//   steps of MVPFormer-S     228 1966 : 1925, 266 2211 : 2137, 304 2328 : 2473, 456 2873 : 3623
-//   of the base model        300 11138 : 10066, 360 11519 : 10870, 480 12179 : 13235, 720 18195 : 23241
+// tiles, us a pass of all blocks (four of the base model's) at so many tiles,
+//   windows of MVPFormer-S   228 1454 : 1306, 247 1486 : 1418, 266 1718 : 1552, 285 1717 : 1658, 304 1751 : 1777,
+//                            342 1874 : 2029; 266 at 37 channels 2077 : 1882
+//   of the base model        360 1244 : 1009, 420 1264 : 1096, 480 1315 : 1261, 600 1575 : 1690, 720 1659 : 2045
+//   steps of MVPFormer-S     228 2002 : 2005, 266 2218 : 2243, 304 2288 : 2552, 456 2804 : 3781
+//   of the base model        300 1597 : 1376, 360 1616 : 1509, 420 1636 : 1694, 480 1676 : 1883
+// (The lines were drawn when small tiles took up to a fifth more; those of windows lie early by as much.)
 static int64_t many_tiles(int64_t E, bool step) { return (step ? 176 : 148) + E / 8; }
 
 static int64_t up256(int64_t n) { return (n + 255) & ~(int64_t)255; }

@@ -498,7 +498,9 @@ static int launch_linear_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, c
 // the 128 x 128 ones) / these: [768,768] 129 rows 20.4 / 5.1, 525 11.9 / 5.2, 1600 12.2 / 6.8, 3000 (288 tiles) 14.2 / 11.3; [768,2624] 525
 // 35.2 / 10.3, 3000 38.0 / 28.9; [2048,2048] 129 40.7 / 8.3, 1152 (288) 28.9 / 19.2; [2048,576] 1152 10.5 / 8.3; [8,768] 16384 (128) 13.7 /
 // 5.3; [256,8192] 4096 (128) 97.5 / 40.6.  Past the line, before the XCDs shared the tiles: [768,768] 4096 rows (384) 14.6 / 14.9, [768,2624]
-// 37.4 / 42.6, [2048,2048] 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1, [2048,576] 2048 11.4 / 12.0.
+// 37.4 / 42.6, [2048,2048] 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1, [2048,576] 2048 11.4 / 12.0.  Up to 128 rows keep the kernels of a
+// step, whose sums are in another order, and not for their speed: [768,576] 64 rows 7.7 / 4.1, [768,2624] 11.8 / 9.2, [2048,2048] 128 14.4 /
+// 7.9, 1 8.9 / 7.6; [1024,4096] 32 12.9 / 12.9, 1 11.1 / 12.7.
 bool tile_linear_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, const void* y) {
   const int64_t ct = (N + TL_BN - 1) / TL_BN;
   return M > 128 && K % TL_BK == 0 && N % 8 == 0 && ldy % 8 == 0 && ((uintptr_t)y & 15) == 0 && M < (1 << 20) && N < (1 << 20) &&

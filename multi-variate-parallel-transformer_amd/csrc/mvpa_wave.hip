@@ -12,7 +12,8 @@
 // table rows loaded that way took 8 us of a launch).  Arithmetic, roundings and operand layouts are
 // those of mvpa_mfma.hip; steps outside the content window skip K and the product with it.
 // Bound: the latency of set-up, of one or a few tiles per wave, and of the merge.  What hides it is a second
-// workgroup on the CU, so head sizes up to 64 keep to 128 registers and 80 KB (tables of up to 64 rows): (q + u),
+// workgroup on the CU, so head sizes up to 64 keep to 128 registers (at 64 one of them spills: 8 bytes of scratch a
+// lane) and 80 KB (tables of up to 64 rows): (q + u),
 // (q + v), (q + z) are formed once for all waves and stay in LDS, table rows go there directly, and addresses of a
 // tile are one register each.  With 165 registers, one workgroup a CU, B1 H12 Hkv4 C21 T25 Dh64 took two rounds of
 // an XCD's 32 CUs: 12.1 -> 9.9 us; C21 T64 23 -> 20.

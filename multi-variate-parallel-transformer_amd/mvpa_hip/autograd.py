@@ -28,18 +28,20 @@ def _mapped(*tensors) -> bool:
 def _wgrad_on_kernel(m, n, k) -> bool:
     """Whether the kernel of csrc/mvpa_wgrad.hip is the faster one for dY^T X of [m, n] and [m, k], by the tiles of 128 x 128
     in its output.  us, both launches of it / the vendor library, eight sets of rows in turn:
-        25 tiles  [640,640]    2560 rows 16 / 19, 6400 21 / 39, 25600 42 / 147
-        36        [768,768]    2816 21 / 20, 3072 20 / 22, 6400 22 / 39, 25600 49 / 155
-        60        [1280,768]   2560 23 / 19, 3072 23 / 22, 3584 23 / 25, 6400 27 / 41, 25600 68 / 163
-        84        [768,1728]   2560 21 / 23, 6400 36 / 50, 25600 104 / 285
-        162       [3456,768]   2560 30 / 30, 6400 55 / 69, 25600 181 / 279
-        169       [1664,1664]  5120 59 / 56, 6400 55 / 72
-        180       [2560,1152]  2560 30 / 30, 6400 79 / 70, 16384 171 / 146
-        225       [1920,1920]  2560 34 / 32, 6400 80 / 73, 25600 314 / 258
-    Fewer rows do not pay for the second launch, and with more tiles the vendor's larger ones fill the chip too.  So they do
-    where many tiles meet many rows (the same rows again, in millions of rows times tiles: [3456,768] 10.6 415 / 544,
-    [1536,2048] 25 1252 / 1029), earlier where rows do not start at lines of 128 bytes ([640,4000] 5.2 211 / 318, 10.5 622 /
-    427).  Long thin outputs are padding for the most part (25600 rows of [8,16000] 169 / 154)."""
+        25 tiles  [640,640]    2560 rows 16 / 19, 6400 22 / 38, 25600 38 / 156
+        36        [768,768]    2816 19 / 20, 3072 19 / 22, 6400 22 / 39, 25600 48 / 157
+        60        [1280,768]   2560 23 / 19, 3072 23 / 22, 3584 23 / 25, 6400 26 / 42, 25600 70 / 172
+        84        [768,1728]   2560 21 / 24, 6400 32 / 51, 25600 93 / 283
+        162       [3456,768]   2560 26 / 29, 6400 52 / 72, 25600 171 / 280, 65536 410 / 541
+        169       [1664,1664]  2560 27 / 29, 5120 46 / 55, 6400 53 / 72
+        180       [2560,1152]  2560 27 / 29, 6400 65 / 72, 16384 144 / 174
+        225       [1920,1920]  2560 29 / 31, 6400 64 / 74, 25600 232 / 259
+        432       [2048,3456]  2560 49 / 49, 6400 116 / 108, 25600 484 / 437
+    Fewer rows do not pay for the second launch, and with many tiles the vendor's larger ones fill the chip too; so they do
+    where many tiles meet many rows, earlier where rows do not start at lines of 128 bytes (rows times tiles in millions: [3456,768]
+    10.6 410 / 541, [1536,2048] 25 1008 / 1024; [640,4000] 5.2 241 / 312, 10.5 478 / 428).  Long thin outputs are padding for the most
+    part (25600 rows of [8,16000] 144 / 139).  The limits of tiles and of rows from 162 tiles on were drawn with a kernel that took up to a
+    fifth more (180 tiles 79 / 70, 225 80 / 73 over 6400 rows): they lie on the safe side."""
     tiles = -(-n // 128) * -(-k // 128)
     if tiles > 170 or (min(n, k) < 64 and tiles > 96):
         return False
