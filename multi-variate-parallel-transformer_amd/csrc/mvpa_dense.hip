@@ -925,7 +925,7 @@ static int launch_ring(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 }
 
 // -----------------------------------------------------------------------------------------
-// The large-tile kernel on two stages of 64-wide k-blocks (K a multiple of 64).
+// The large-tile kernel on two or three stages of 64-wide k-blocks (K a multiple of 64).
 // A request of the 32-wide ring covers 64 bytes of a row - half a cache line, whose other half
 // the next k-block asks for again, one k-block's worth of other lines (32 KiB per CU) later.  Here
 // a wave load covers 8 rows x 128 bytes, whole lines, and LDS holds two blocks of 64.  The order of a
@@ -934,9 +934,16 @@ static int launch_ring(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 // publishes the next block, whose first fragments are read under that last quarter's products, and
 // frees this block's stage, into which the block after next is requested at once - a full block's
 // time ahead of the barrier that will wait for it.  One request per block without a branch (past
-// the end the last block again, into a stage nobody reads), so the wait is a fixed vmcnt(0).
+// the end the last block again, into a stage nobody reads), so the wait is a fixed vmcnt.
+// A block of 256 x 128 outputs is 0.5 us of products, less than the trip to the L2 at its busiest, and its 48 KB leave room for a
+// third stage, so that two blocks are on their way: us, two / three stages, [768,768] over 6400 rows 14.0 / 12.7, [768,1728] 25.2 /
+// 22.3, [768,3456] 46.0 / 39.8, [2048,2048] over 3000 29.5 / 27.3; level where 192 or 256 columns are the better tile.
 // Same tile order, roles, row mapping and epilogues as the other large-tile kernels.
 // -----------------------------------------------------------------------------------------
+constexpr int pair_stages(int BN) { return BN == 128 ? 3 : 2; }
+constexpr int pair_lds(int BN) { return pair_stages(BN) * (256 + BN) * 128; }
+constexpr int pair_lds(int BN0, int BN1) { return pair_lds(BN0) > pair_lds(BN1) ? pair_lds(BN0) : pair_lds(BN1); }
+
 template <int BN, int EPI, int STATS = 0>
 __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gsm,
                                                  const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
@@ -944,7 +951,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
                                                  int64_t ldx, int64_t ldw, int64_t ldy,
                                                  const bf16_t* __restrict__ R, int64_t ldr,
                                                  const row_stats* rs = nullptr) {
-  constexpr int BM = 256, BK = 64, ROWB = BK * 2, STAGES = 2;
+  constexpr int BM = 256, BK = 64, ROWB = BK * 2, STAGES = pair_stages(BN);
   constexpr int WN = BN / 2, NB = WN / 32;            // per-wave extent over w rows
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
   constexpr int A_LOADS = A_BYTES / 1024 / 8, B_LOADS = B_BYTES / 1024 / 8;   // 1 KiB wave loads per wave and block
@@ -1004,7 +1011,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     for (int i = 0; i < B_LOADS; ++i)
       asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
                    :: "v"(boff[i]), "s"(ws), "s"(iss_lds + A_BYTES + (wave + 8 * i) * 1024) : "memory", "m0");
-    iss_lds = iss_lds == lds0 ? lds0 + STAGE : lds0;
+    iss_lds = iss_lds == lds0 + (STAGES - 1) * STAGE ? lds0 : iss_lds + STAGE;
     if (iss_kb + 1 < nkb) {
       ++iss_kb;
       xs += BK;
@@ -1043,9 +1050,9 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
       }
     }
   }
-  issue_block();
-  issue_block();
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(A_LOADS + B_LOADS) : "memory");
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s) issue_block();
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (A_LOADS + B_LOADS)) : "memory");
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   bf16x8 xf0[2], wf0[NB];
 #pragma unroll
@@ -1064,7 +1071,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
 
   for (int kb = 0; kb < nkb; ++kb) {
     const unsigned char* st = gsm + cur * STAGE;
-    cur ^= 1;
+    cur = STAGES == 2 ? cur ^ 1 : cur == STAGES - 1 ? 0 : cur + 1;
     const unsigned char* sn = gsm + cur * STAGE;
     bf16x8 xf1[2], wf1[NB];
     // slices 0 .. 2: the fragments of slice s+1 are requested before the products of slice s
@@ -1099,7 +1106,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
       for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf0[i], xf0[j], acc[i][j], 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
     // the next block has landed, and every fragment of this one is in registers: publish / free
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * (A_LOADS + B_LOADS)) : "memory");
     if (STATS == 1 && kb == 0) {
       // (every load of this wave is back here, the partial sums among them: no wait of their own;
       // the factors are published by the barriers of the blocks that follow)
@@ -1215,7 +1222,7 @@ template <int BN>
 static int launch_pair_sumsq(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K,
                              int64_t ldx, int64_t ldw, int64_t ldy, hipStream_t s, const bf16_t* r, int64_t ldr,
                              float* ss_out, int32_t parts) {
-  constexpr int LDS = 2 * (256 + BN) * 128;
+  constexpr int LDS = pair_lds(BN);
   auto kern = linear_bf16_pair_sumsq_kernel<BN>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   dim3 grid((unsigned)(((N + BN - 1) / BN) * ((M + 255) / 256)));
@@ -1228,7 +1235,7 @@ template <int BN0>
 static int launch_pair_dual_normed(const bf16_t* x, int64_t M, int64_t K, int64_t ldx,
                                    const mvpa::linear_pair_problem& plain, const mvpa::linear_pair_problem& gated,
                                    const mvpa::row_stats& rs, hipStream_t s) {
-  constexpr int LDS = 2 * (256 + 256) * 128 + 1024;     // ring + the tile's 256 norm factors
+  constexpr int LDS = pair_lds(BN0, 256) + 1024;     // ring + the tile's 256 norm factors
   auto kern = linear_bf16_pair_dual_normed_kernel<BN0>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   const int64_t mt = (M + 255) / 256;
@@ -1242,7 +1249,7 @@ template <int BN, int EPI>
 static int launch_pair(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K,
                        int64_t ldx, int64_t ldw, int64_t ldy, hipStream_t s,
                        const bf16_t* r = nullptr, int64_t ldr = 0) {
-  constexpr int LDS = 2 * (256 + BN) * 128;
+  constexpr int LDS = pair_lds(BN);
   auto kern = linear_bf16_pair_kernel<BN, EPI>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;
@@ -1254,7 +1261,7 @@ static int launch_pair(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 template <int BN0>
 static int launch_pair_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const mvpa::linear_pair_problem& plain,
                             const mvpa::linear_pair_problem& gated, hipStream_t s) {
-  constexpr int LDS = 2 * (256 + 256) * 128;
+  constexpr int LDS = pair_lds(BN0, 256);
   auto kern = linear_bf16_pair_dual_kernel<BN0>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   const int64_t mt = (M + 255) / 256;

@@ -15,6 +15,8 @@ pytestmark = pytest.mark.gpu
                                    (8192, 1000, 200), (16384, 520, 72),
                                    # K a multiple of 64: the 64-wide two-stage kernel, ragged rows and columns, two k-blocks only
                                    (600, 130, 128), (1000, 200, 192), (5000, 333, 256), (513, 257, 1024),
+                                   # 128 columns a tile on three stages: fewer blocks than stages, as many, one more, many
+                                   (600, 1000, 128), (5000, 520, 192), (700, 1290, 256), (4097, 776, 1728),
                                    # fewer than 128 columns: tiles row by row, 20 and 64 rows of them, one column
                                    (5000, 2056, 64), (16384, 1000, 96), (40000, 130, 120), (5000, 777, 127),
                                    # 32 and 64 columns of tiles, the last one ragged
