@@ -468,6 +468,12 @@ int mvpa_rmsnorm_backward(const void* x, const void* weight, const void* dy, con
 int mvpa_silu_gate_bf16(const void* gu, void* out, int64_t rows, int32_t n, void* stream);
 int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void* dgu, int64_t rows, int32_t n, void* stream);
 
+/* Gradients of the generative score (models/mvpformer.py:749-764), s[b,t,c] = cosine similarity of nxt[b,t+1,c] and pred[b,t,c]
+ * over cols, for the gradient d [B,T-1,C] of s: d_nxt and d_pred [B,T,C,cols] (one may be null), zeros in the step that has no
+ * partner.  Contiguous bf16 rows, d fp32; T > 1, cols a multiple of 8, 16-byte aligned pointers. */
+int mvpa_cosine_steps_backward_bf16(const void* nxt, const void* pred, const float* d, void* d_nxt, void* d_pred, int64_t B,
+                                    int64_t T, int64_t C, int32_t cols, float eps, void* stream);
+
 /* dw[N,K] = dy[M,N]^T x[M,K]: the weight gradient of y = x w^T, bf16 in and out, fp32 sums.  N, K and the row
  * strides (in elements) multiples of 8, 16-byte aligned pointers; ws: mvpa_linear_wgrad_ws_bytes(M, N, K) bytes. */
 size_t mvpa_linear_wgrad_ws_bytes(int64_t M, int64_t N, int64_t K);

@@ -438,6 +438,31 @@ PyObject* py_silu_gate(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// cosine_steps_backward(nxt [B,T,C,E], pred, d [B,T-1,C], eps, need_nxt, need_pred) -> (d_nxt | None, d_pred | None) | status
+PyObject* py_cosine_steps_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 6, "cosine_steps_backward takes 6 arguments");
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor a = aligned_operand(tensor_of(args[0]), at::kBFloat16), b = aligned_operand(tensor_of(args[1]), at::kBFloat16);
+  const Tensor d = as_operand(tensor_of(args[2]), at::kFloat);
+  const double eps = PyFloat_AsDouble(args[3]);
+  if (PyErr_Occurred()) return nullptr;
+  TORCH_CHECK(a.dim() == 4 && b.sizes() == a.sizes() && d.dim() == 3 && d.size(0) == a.size(0) && d.size(1) == a.size(1) - 1 &&
+              d.size(2) == a.size(2) && b.device() == a.device() && d.device() == a.device(), "cosine_steps_backward: operands differ");
+  Tensor da, db;
+  if (args[4] == Py_True) da = at::empty_like(a);
+  if (args[5] == Py_True) db = at::empty_like(b);
+  const int st = mvpa_cosine_steps_backward_bf16(a.data_ptr(), b.data_ptr(), (const float*)d.data_ptr(), da.defined() ? da.data_ptr() : nullptr,
+                                                 db.defined() ? db.data_ptr() : nullptr, a.size(0), a.size(1), a.size(2),
+                                                 (int32_t)a.size(3), (float)eps, current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* r = PyTuple_New(2);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(da));           // an undefined tensor comes out as None
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(db));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
 // ---- the stack of blocks ----------------------------------------------------------------------
 // What a model looked like when a plan was made from it: entries of modules' parameter and sub-module tables
 // (identity), the storages and versions of the tensors found there, and the sizes of the tables that grow
@@ -875,6 +900,7 @@ PyMethodDef kMethods[] = {
     {"encode_saved", (PyCFunction)(void*)py_encode_saved, METH_FASTCALL, "encode, with what its backward needs"},
     {"norm_dw", (PyCFunction)(void*)py_norm_dw, METH_FASTCALL, "gradient of a norm's weight from saved row factors"},
     {"norm_backward", (PyCFunction)(void*)py_norm_backward, METH_FASTCALL, "backward of RMSNorm"},
+    {"cosine_steps_backward", (PyCFunction)(void*)py_cosine_steps_backward, METH_FASTCALL, "gradients of the generative score"},
     {"silu_gate", (PyCFunction)(void*)py_silu_gate, METH_FASTCALL, "silu(gate) * up, or its backward"},
     {"lora_fits", (PyCFunction)py_lora_fits, METH_O, "whether lora_stack takes these"},
     {"lora_stack", (PyCFunction)(void*)py_lora_stack, METH_FASTCALL, "stacked weights with adapters, or the adapters' gradients"},

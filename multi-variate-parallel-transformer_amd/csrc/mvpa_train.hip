@@ -243,6 +243,66 @@ __device__ inline void store8(bf16_t* p, const float (&v)[8]) {
   *(u32x4*)p = u32x4{pack2(v[0], v[1]), pack2(v[2], v[3]), pack2(v[4], v[5]), pack2(v[6], v[7])};
 }
 
+// The generative score's backward (models/mvpformer.py:749-764): step t + 1 of a against step t of b.
+//   s = a.b / (|a|' |b|'),  |x|' = max(|x|, eps):   da = d (b / (|a|' |b|') - a s / (|a|' |a|)), db likewise,
+// the norms not held at eps in the derivative, as torch.cosine_similarity has it; zeros for the step without a partner.  A wave
+// owns a pair of rows and reads them twice, the second time from the caches.  HBM bound; as tensor operations on fp32
+// copies the score and its backward were 45 launches, 330 us at B4 C64 T25 E768, of which this one takes 9 and the forward 5.
+__global__ __launch_bounds__(256) void cosine_steps_backward_kernel(const bf16_t* __restrict__ a, const bf16_t* __restrict__ b,
+                                                                    const float* __restrict__ d, bf16_t* __restrict__ da,
+                                                                    bf16_t* __restrict__ db, int64_t rows, int64_t T, int64_t C,
+                                                                    int cols, float eps) {
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const int lane = threadIdx.x & 63;
+  const int64_t bt = row / C, n = bt / T, t = bt - n * T;
+  const bf16_t* ar = a + row * cols;
+  bf16_t* dar = da ? da + row * cols : nullptr;
+  if (t == 0) {                      // a's first step and b's last one
+    bf16_t* dbr = db ? db + (row + (T - 1) * C) * cols : nullptr;
+    for (int c = lane * 8; c < cols; c += 512) {
+      if (dar) *(u32x4*)(dar + c) = u32x4{0u, 0u, 0u, 0u};
+      if (dbr) *(u32x4*)(dbr + c) = u32x4{0u, 0u, 0u, 0u};
+    }
+    return;
+  }
+  const bf16_t* br = b + (row - C) * cols;
+  bf16_t* dbr = db ? db + (row - C) * cols : nullptr;
+  const float g = d[row - (n + 1) * C];
+  float dot = 0.f, na = 0.f, nb = 0.f;
+  for (int c = lane * 8; c < cols; c += 512) {
+    float x[8], y[8];
+    load8(ar + c, x);
+    load8(br + c, y);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      dot += x[i] * y[i];
+      na += x[i] * x[i];
+      nb += y[i] * y[i];
+    }
+  }
+  dot = wave_sum(dot);
+  na = sqrtf(wave_sum(na));
+  nb = sqrtf(wave_sum(nb));
+  const float ia = 1.f / fmaxf(na, eps), ib = 1.f / fmaxf(nb, eps), s = dot * ia * ib;
+  const float cross = g * ia * ib, ca = na > 0.f ? g * s * ia / na : 0.f, cb = nb > 0.f ? g * s * ib / nb : 0.f;
+  for (int c = lane * 8; c < cols; c += 512) {
+    float x[8], y[8], o[8];
+    load8(ar + c, x);
+    load8(br + c, y);
+    if (dar) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = cross * y[i] - ca * x[i];
+      store8(dar + c, o);
+    }
+    if (dbr) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) o[i] = cross * x[i] - cb * y[i];
+      store8(dbr + c, o);
+    }
+  }
+}
+
 constexpr int GATE_ROWS = 4;         // rows per thread: their loads go out together
 
 // out = silu(gate) up for rows [gate | up] of 2 n columns; a thread takes 8 columns of GATE_ROWS rows
@@ -547,6 +607,17 @@ extern "C" int mvpa_silu_gate_backward_bf16(const void* gu, const void* d, void*
   if (st != MVPA_OK) return st;
   MVPA_LAUNCH(train::silu_gate_backward_kernel, gate_grid(rows, n), dim3(256), 0, (hipStream_t)stream, (const bf16_t*)gu,
               (const bf16_t*)d, (bf16_t*)dgu, rows, n);
+  return take_launch_status();
+}
+
+extern "C" int mvpa_cosine_steps_backward_bf16(const void* nxt, const void* pred, const float* d, void* d_nxt, void* d_pred, int64_t B,
+                                               int64_t T, int64_t C, int32_t cols, float eps, void* stream) {
+  if (!nxt || !pred || !d || (!d_nxt && !d_pred)) return MVPA_ERR_NULL;
+  if (B <= 0 || T <= 1 || C <= 0 || cols <= 0 || T > ((int64_t)1 << 31) / C || B > ((int64_t)1 << 31) / (T * C)) return MVPA_ERR_SHAPE;
+  if (cols % 8 != 0 || (((uintptr_t)nxt | (uintptr_t)pred | (uintptr_t)d_nxt | (uintptr_t)d_pred) & 15)) return MVPA_ERR_ALIGN;
+  const int64_t rows = B * T * C;
+  MVPA_LAUNCH(train::cosine_steps_backward_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, (hipStream_t)stream,
+              (const bf16_t*)nxt, (const bf16_t*)pred, d, (bf16_t*)d_nxt, (bf16_t*)d_pred, rows, T, C, cols, eps);
   return take_launch_status();
 }
 

@@ -932,7 +932,8 @@ class HMVPFormer(BrainModel):
         out, enc = self._common_forward(batch)
         out = self.head(out)
         if torch.is_grad_enabled():
-            return torch.cosine_similarity(enc[:, 1:].float(), out[:, :-1].float(), dim=-1)
+            score = AG.cosine_steps(enc, out)
+            return torch.cosine_similarity(enc[:, 1:].float(), out[:, :-1].float(), dim=-1) if score is None else score
         if enc.is_cuda and enc.dtype == torch.bfloat16 and out.dtype == torch.bfloat16 and enc.shape[-1] % 8 == 0:
             return mvpa_hip.cosine_similarity_steps(enc, out)
         return torch.cosine_similarity(enc[:, 1:].float(), out[:, :-1].float(), dim=-1)

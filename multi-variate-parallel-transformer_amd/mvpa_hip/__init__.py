@@ -551,6 +551,11 @@ def silu_gate(gu: torch.Tensor, d: Optional[torch.Tensor] = None) -> torch.Tenso
     return _taken(ext.silu_gate(gu) if d is None else ext.silu_gate(gu, d))
 
 
+def cosine_steps_backward(nxt, pred, d, eps: float, need_nxt: bool, need_pred: bool):
+    """Gradients (d_nxt, d_pred) of cosine_similarity_steps for the gradient d of its result."""
+    return _taken((_ext or load_ext()).cosine_steps_backward(nxt, pred, d, float(eps), bool(need_nxt), bool(need_pred)))
+
+
 def lora_stack(mods, scale: float, d: Optional[torch.Tensor] = None):
     """Stacked weights of modules ((enable, w, a | None, b | None), ..) with their adapters added; with d, the
     gradients of each module's a and b (in turn) for the gradient d of that."""

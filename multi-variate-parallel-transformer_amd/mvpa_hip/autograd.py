@@ -249,6 +249,41 @@ def gated_mid(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     return _SiluGateFn.apply(linear(x, w_gate_up))
 
 
+class _CosineStepsFn(torch.autograd.Function):
+    """Cosine similarity of step t + 1 of nxt and step t of pred [B, T, C, E], one pass each way."""
+
+    @staticmethod
+    def forward(ctx, nxt, pred, eps):
+        ctx.save_for_backward(nxt, pred)
+        ctx.eps = eps
+        return mvpa_hip.cosine_similarity_steps(nxt, pred, eps)
+
+    @staticmethod
+    def backward(ctx, d):
+        nxt, pred = ctx.saved_tensors
+        if not torch.is_grad_enabled() and not _mapped(d):
+            return (*mvpa_hip.cosine_steps_backward(nxt, pred, d, ctx.eps, *ctx.needs_input_grad[:2]), None)
+        # a backward that is differentiated itself, or mapped over
+        a, b, d = nxt[:, 1:].float(), pred[:, :-1].float(), d[..., None]
+        na, nb = a.norm(dim=-1, keepdim=True), b.norm(dim=-1, keepdim=True)
+        ia, ib = 1 / na.clamp_min(ctx.eps), 1 / nb.clamp_min(ctx.eps)
+        s, tiny = (a * b).sum(-1, keepdim=True) * ia * ib, torch.finfo(torch.float32).tiny
+        da = d * (b * ia * ib - a * s * ia / na.clamp_min(tiny))
+        db = d * (a * ia * ib - b * s * ib / nb.clamp_min(tiny))
+        pad = torch.nn.functional.pad
+        return pad(da, (0, 0, 0, 0, 1, 0)).to(nxt.dtype), pad(db, (0, 0, 0, 0, 0, 1)).to(pred.dtype), None
+
+
+def cosine_steps(nxt: torch.Tensor, pred: torch.Tensor, eps: float = 1e-8):
+    """torch.cosine_similarity(nxt[:, 1:], pred[:, :-1], dim=-1) in fp32 with gradients, or None where the two are not bf16
+    rows of whole 16-byte chunks on the GPU, or there is no pair of steps."""
+    if (not nxt.is_cuda or not nxt.dtype == pred.dtype == torch.bfloat16 or nxt.shape != pred.shape or nxt.dim() != 4
+            or nxt.shape[-1] % 8 or nxt.shape[1] < 2 or not nxt.numel() or nxt.device != pred.device or _mapped(nxt, pred)
+            or any(t.is_contiguous() and t.data_ptr() % 16 for t in (nxt, pred))):     # others are copied to rows of their own
+        return None
+    return _CosineStepsFn.apply(nxt, pred, eps)
+
+
 class _LoRAStackFn(torch.autograd.Function):
     """Weights of several modules, adapters added, stacked by rows; one launch each way.  tensors: w, a, b of
     each module in turn, a and b None where it has no adapter."""

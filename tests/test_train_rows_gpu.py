@@ -71,6 +71,32 @@ def test_silu_gate(rows, n):
     _close(dup, d.double() * gate * s)
 
 
+# one pair of steps, rows of less than a wave, of a chunk more, of several; one channel; a row of zeros, one shorter than eps
+@pytest.mark.parametrize("B,T,C,E", [(1, 2, 1, 8), (2, 5, 7, 520), (3, 4, 5, 1032), (1, 25, 64, 768)])
+def test_generative_score_gradients(B, T, C, E):
+    g = torch.Generator(device="cuda").manual_seed(B * T * C + E)
+    a, b = (torch.randn((B, T, C, E), generator=g, device="cuda").bfloat16().requires_grad_() for _ in range(2))
+    with torch.no_grad():
+        if T > 2:
+            a[0, 1, 0], b[0, 2, -1] = 0, 1e-9 / E
+    d = torch.randn((B, T - 1, C), generator=g, device="cuda")
+    s = AG.cosine_steps(a, b)
+    ad, bd = a.detach().double().requires_grad_(), b.detach().double().requires_grad_()
+    ref = torch.cosine_similarity(ad[:, 1:], bd[:, :-1], dim=-1)
+    _close(s, ref, E)
+    want = torch.autograd.grad(ref, (ad, bd), d.double())
+    for x, w in zip(torch.autograd.grad(s, (a, b), d, retain_graph=True), want):
+        # a difference of two terms of about the result's size
+        assert ((x.double() - w).abs() <= 2.0 ** -8 * 1.01 * w.abs() + 2.0 ** -18 * (w.abs() + w.norm(dim=-1, keepdim=True))).all()
+        assert x.shape == a.shape and (w != 0).logical_or(x == 0).all()
+    both = torch.autograd.grad(s, (a, b), torch.stack([d, 2 * d]), is_grads_batched=True, retain_graph=True)
+    for x, y, w in zip(both, torch.autograd.grad(s, (a, b), d, create_graph=True), want):
+        assert (x[0] - y).norm() <= 1e-2 * w.norm() and (y.double() - w).norm() <= 1e-2 * w.norm() and y.requires_grad
+    only, = torch.autograd.grad(AG.cosine_steps(a.detach(), b), b, d)
+    assert (only.double() - want[1]).norm() <= 1e-2 * want[1].norm()
+    assert AG.cosine_steps(a[..., 4:], b[..., 4:]) is None and AG.cosine_steps(a[:, :1], b[:, :1]) is None
+
+
 @pytest.mark.parametrize("cols", [8, 768])
 def test_add3_norm_gradients(cols):
     """Gradients through both results, through one of them, and of a gradient (the tensor expressions)."""
