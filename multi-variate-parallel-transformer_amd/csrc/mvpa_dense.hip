@@ -481,7 +481,7 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN / 64][2], unsigned
                                        int64_t m0, int64_t n0, int64_t M, int64_t N,
                                        bf16_t* __restrict__ Y, int64_t ldy,
                                        const bf16_t* __restrict__ R, int64_t ldr,
-                                       const row_stats* rs = nullptr, int64_t tile_n = 0) {
+                                       const row_stats* rs = nullptr, int64_t tile_n = 0, float factor = 1.f) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
   constexpr int WN = BN / 2, NB = WN / 32;
   const int ln = lane & 31, hh = lane >> 5;
@@ -497,8 +497,11 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN / 64][2], unsigned
                      (EPI != 2 || ((ldr & 7) == 0 && ((uintptr_t)R & 15) == 0));
   const int64_t ncol0 = n0 + wc * WC;
   float rnorm[2] = {1.f, 1.f};
-  if (STATS == 1) {        // the tile's 256 factors were put behind the ring when the tile began
-    const float* rstat = (const float*)(gsm + LDS_BYTES);
+  if (STATS == 1) {        // the tile's 256 factors, a row's with its two threads, to the lanes that hold its sums
+    float* rstat = (float*)(gsm + LDS_BYTES - 1024);
+    static_assert(STATS != 1 || 8 * 32 * PITCH <= LDS_BYTES - 1024, "the factors lie behind the staging area");
+    if ((lane & 1) == 0) rstat[wave * 32 + (lane >> 1)] = factor;
+    __syncthreads();
 #pragma unroll
     for (int j = 0; j < 2; ++j) rnorm[j] = rstat[wm * 64 + j * 32 + ln];
   }
@@ -925,23 +928,27 @@ static int launch_ring(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 }
 
 // -----------------------------------------------------------------------------------------
-// The large-tile kernel on two or three stages of 64-wide k-blocks (K a multiple of 64).
+// The large-tile kernel on rings of 64-wide k-blocks (K a multiple of 64).
 // A request of the 32-wide ring covers 64 bytes of a row - half a cache line, whose other half
 // the next k-block asks for again, one k-block's worth of other lines (32 KiB per CU) later.  Here
-// a wave load covers 8 rows x 128 bytes, whole lines, and LDS holds two blocks of 64.  The order of a
-// block keeps what the ring gained: the barrier sits in front of the block's LAST quarter, whose
-// fragments are in registers by then (lgkmcnt 0 before it: nobody still reads the block); it
-// publishes the next block, whose first fragments are read under that last quarter's products, and
-// frees this block's stage, into which the block after next is requested at once - a full block's
-// time ahead of the barrier that will wait for it.  One request per block without a branch (past
-// the end the last block again, into a stage nobody reads), so the wait is a fixed vmcnt.
-// A block of 256 x 128 outputs is 0.5 us of products, less than the trip to the L2 at its busiest, and its 48 KB leave room for a
-// third stage, so that two blocks are on their way: us, two / three stages, [768,768] over 6400 rows 14.0 / 12.7, [768,1728] 25.2 /
-// 22.3, [768,3456] 46.0 / 39.8, [2048,2048] over 3000 29.5 / 27.3; level where 192 or 256 columns are the better tile.
+// a wave load covers 8 rows x 128 bytes, whole lines.  The order of a block keeps what the ring gained: the barrier sits
+// in front of the block's LAST quarter, whose fragments are in registers by then (lgkmcnt 0 before it: nobody still reads the
+// block); it publishes the next block, whose first fragments are read under that last quarter's products, and
+// frees this block's stages, into which later blocks are requested at once.  Past the end the last block is requested again, into a
+// stage nobody reads, so that the wait is a fixed vmcnt.  x and w have rings of their own: three stages of x, whose rows come from
+// farther away, and as many of w as the 160 KB leave (two of 256 or 192 columns, three of 128).
+// What bounds a block is the requests: a wave stands while its request waits for the one address unit of the CU (1 KiB in 16
+// cycles, 64 of them a block of 256 x 256 = 1024 cycles beside 2048 of products), and with all requests of a block sent together behind
+// the barrier every wave stood there at once.  So they go out one behind a product, over half a block, and only waves 0 .. 3 send
+// them, one of the two on each SIMD: the other has products for the matrix unit meanwhile (128 columns, half the products: all
+// waves send).  us, two stages and requests together / spread / by four waves / three stages of x: [3456,768] over 16384
+// rows 99 / 95 / 92 / 89, [768,2496] 62 / 62 / 59 / 52, [2048,2048] over 65536 486 / 470 / 446 / 433, [2048,7680] 1650 / 1605 / 1518 /
+// 1480, 8192^3 850 / 820 / 780 / 785; 128 columns, over 6400 rows [768,768] 14.3 / 12.0, [768,1728] 26.2 / 22.2, [768,3456] 46.3 / 36.
 // Same tile order, roles, row mapping and epilogues as the other large-tile kernels.
 // -----------------------------------------------------------------------------------------
-constexpr int pair_stages(int BN) { return BN == 128 ? 3 : 2; }
-constexpr int pair_lds(int BN) { return pair_stages(BN) * (256 + BN) * 128; }
+constexpr int pair_x_stages(int) { return 3; }
+constexpr int pair_w_stages(int BN) { return BN == 128 ? 3 : 2; }
+constexpr int pair_lds(int BN) { return (pair_x_stages(BN) * 256 + pair_w_stages(BN) * BN) * 128; }
 constexpr int pair_lds(int BN0, int BN1) { return pair_lds(BN0) > pair_lds(BN1) ? pair_lds(BN0) : pair_lds(BN1); }
 
 template <int BN, int EPI, int STATS = 0>
@@ -951,10 +958,11 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
                                                  int64_t ldx, int64_t ldw, int64_t ldy,
                                                  const bf16_t* __restrict__ R, int64_t ldr,
                                                  const row_stats* rs = nullptr) {
-  constexpr int BM = 256, BK = 64, ROWB = BK * 2, STAGES = pair_stages(BN);
+  constexpr int BM = 256, BK = 64, ROWB = BK * 2, X_STAGES = pair_x_stages(BN), W_STAGES = pair_w_stages(BN);
   constexpr int WN = BN / 2, NB = WN / 32;            // per-wave extent over w rows
-  constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, STAGE = A_BYTES + B_BYTES;
-  constexpr int A_LOADS = A_BYTES / 1024 / 8, B_LOADS = B_BYTES / 1024 / 8;   // 1 KiB wave loads per wave and block
+  constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, W_RING = X_STAGES * A_BYTES;
+  constexpr int LOADERS = BN == 128 ? 8 : 4;          // waves that request
+  constexpr int A_LOADS = A_BYTES / 1024 / LOADERS, B_LOADS = B_BYTES / 1024 / LOADERS;   // 1 KiB requests of such a wave per block
   static_assert(B_BYTES % (8 * 1024) == 0, "every wave issues the same number of loads");
   static_assert(EPI != 1 || NB % 2 == 0, "gate/up pairs need an even number of sub-blocks");
 
@@ -982,8 +990,9 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   // chunk L%8; per-lane byte offsets from wave-uniform bases (rows clamped into range: such rows
   // are never stored).
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)gsm;
-  int iss_kb = 0;
-  uint32_t iss_lds = lds0;
+  const int lw = wave % LOADERS;
+  int x_kb = 0, w_kb = 0;
+  uint32_t x_lds = lds0 + lw * 1024, w_lds = lds0 + W_RING + lw * 1024;
   const int64_t wrow0 = w_row(0);
   const bf16_t* xs = X + m0 * ldx;
   const bf16_t* ws = W + wrow0 * ldw;
@@ -992,74 +1001,86 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     const int rsub = lane >> 3, phys = lane & 7;
 #pragma unroll
     for (int i = 0; i < A_LOADS; ++i) {
-      const int row = (wave + 8 * i) * 8 + rsub;
+      const int row = (lw + LOADERS * i) * 8 + rsub;
       const int64_t m = m0 + row;
       aoff[i] = (uint32_t)((((m < M ? m : M - 1) - m0) * ldx + ((phys ^ ((row >> 1) & 7)) << 3)) * 2);
     }
 #pragma unroll
     for (int i = 0; i < B_LOADS; ++i) {
-      const int row = (wave + 8 * i) * 8 + rsub;
+      const int row = (lw + LOADERS * i) * 8 + rsub;
       boff[i] = (uint32_t)(((w_row(row) - wrow0) * ldw + ((phys ^ ((row >> 1) & 7)) << 3)) * 2);
     }
   }
-  auto issue_block = [&]() {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i)
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :: "v"(aoff[i]), "s"(xs), "s"(iss_lds + (wave + 8 * i) * 1024) : "memory", "m0");
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i)
-      asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                   :: "v"(boff[i]), "s"(ws), "s"(iss_lds + A_BYTES + (wave + 8 * i) * 1024) : "memory", "m0");
-    iss_lds = iss_lds == lds0 + (STAGES - 1) * STAGE ? lds0 : iss_lds + STAGE;
-    if (iss_kb + 1 < nkb) {
-      ++iss_kb;
+  auto request_x = [&](int i) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(aoff[i]), "s"(xs), "s"(x_lds + LOADERS * i * 1024) : "memory", "m0");
+  };
+  auto request_w = [&](int i) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+                 :: "v"(boff[i]), "s"(ws), "s"(w_lds + LOADERS * i * 1024) : "memory", "m0");
+  };
+  auto next_x = [&]() {                               // past the end the last block once more, into a stage nobody reads
+    x_lds = x_lds >= lds0 + (X_STAGES - 1) * A_BYTES ? x_lds - (X_STAGES - 1) * A_BYTES : x_lds + A_BYTES;
+    if (x_kb + 1 < nkb) {
+      ++x_kb;
       xs += BK;
+    }
+  };
+  auto next_w = [&]() {
+    w_lds = w_lds >= lds0 + W_RING + (W_STAGES - 1) * B_BYTES ? w_lds - (W_STAGES - 1) * B_BYTES : w_lds + B_BYTES;
+    if (w_kb + 1 < nkb) {
+      ++w_kb;
       ws += BK;
     }
   };
+  const bool loader = wave < LOADERS;
 
   // fragment offsets: row ln of a 32-row block, chunk (2s+hh) ^ swizzle(ln) for the four 16-wide slices
   int frag_off[4];
 #pragma unroll
   for (int sl = 0; sl < 4; ++sl) frag_off[sl] = ln * ROWB + (((2 * sl + hh) ^ ((ln >> 1) & 7)) << 4);
-  const int a_lane = (wm * 64) * ROWB, b_lane = A_BYTES + (wc * WN) * ROWB;
+  const int a_lane = (wm * 64) * ROWB;
+  auto x_frag = [&](const unsigned char* st, int j, int sl) { return *(const bf16x8*)(st + a_lane + j * 32 * ROWB + frag_off[sl]); };
+  auto w_frag = [&](const unsigned char* st, int i, int sl) { return *(const bf16x8*)(st + (wc * WN + i * 32) * ROWB + frag_off[sl]); };
 
   // STATS 1: the norm factors of the tile's 256 rows, r = rsqrt(sum of the row's partial sums of
   // squares / K + eps).  Two threads share a row and half of its partial sums each; the loads go
-  // out in front of the first blocks and are long back when those have landed.  The factors wait
-  // in LDS behind the ring for the epilogue.
-  float rpart = 0.f;
+  // out in front of the first blocks and are added up behind the last.
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  f32x4 rraw[2] = {};
   if (STATS == 1) {
-    const int row = tid >> 1, half = tid & 1;
-    const int64_t m = m0 + row;
-    const int parts = rs->parts_in;
+    const int64_t m = m0 + (tid >> 1), parts = rs->parts_in;
     if (m < M) {
       const float* pp = rs->ss_in + m * parts;
-      if ((parts & 7) == 0 && parts <= 16) {
-        typedef __attribute__((ext_vector_type(4))) float f32x4;
-        const f32x4* q4 = (const f32x4*)(pp + half * (parts >> 1));
-        const f32x4 a = q4[0];
-        rpart = (a.x + a.y) + (a.z + a.w);
-        if (parts == 16) {
-          const f32x4 b4 = q4[1];
-          rpart += (b4.x + b4.y) + (b4.z + b4.w);
-        }
-      } else if (half == 0) {
-        for (int p2 = 0; p2 < parts; ++p2) rpart += pp[p2];
+      if (parts == 8 || parts == 16) {
+        const f32x4* q4 = (const f32x4*)(pp + (tid & 1) * (parts >> 1));
+        rraw[0] = q4[0];
+        if (parts == 16) rraw[1] = q4[1];
+      } else if ((tid & 1) == 0) {
+        for (int p2 = 0; p2 < parts; ++p2) rraw[0].x += pp[p2];
       }
     }
   }
 #pragma unroll
-  for (int s = 0; s < STAGES; ++s) issue_block();
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((STAGES - 1) * (A_LOADS + B_LOADS)) : "memory");
+  for (int s = 0; s < X_STAGES; ++s) {
+    if (s < W_STAGES) {
+#pragma unroll
+      for (int i = 0; i < B_LOADS; ++i)
+        if (loader) request_w(i);
+      next_w();
+    }
+#pragma unroll
+    for (int i = 0; i < A_LOADS; ++i)
+      if (loader) request_x(i);
+    next_x();
+  }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((X_STAGES - 1) * A_LOADS + (W_STAGES - 1) * B_LOADS) : "memory");
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  bf16x8 xf0[2], wf0[NB];
+  bf16x8 xf[2][2], wf[2][NB];                         // two slices' fragments
 #pragma unroll
-  for (int j = 0; j < 2; ++j) xf0[j] = *(const bf16x8*)(gsm + a_lane + j * 32 * ROWB + frag_off[0]);
+  for (int j = 0; j < 2; ++j) xf[0][j] = x_frag(gsm, j, 0);
 #pragma unroll
-  for (int i = 0; i < NB; ++i) wf0[i] = *(const bf16x8*)(gsm + b_lane + i * 32 * ROWB + frag_off[0]);
-  int cur = 0;                                        // stage of the block being multiplied
+  for (int i = 0; i < NB; ++i) wf[0][i] = w_frag(gsm + W_RING, i, 0);
 
   f32x16 acc[NB][2];
 #pragma unroll
@@ -1069,68 +1090,54 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
+  const unsigned char *xst = gsm, *wst = gsm + W_RING;          // the stages whose fragments are read next
   for (int kb = 0; kb < nkb; ++kb) {
-    const unsigned char* st = gsm + cur * STAGE;
-    cur = STAGES == 2 ? cur ^ 1 : cur == STAGES - 1 ? 0 : cur + 1;
-    const unsigned char* sn = gsm + cur * STAGE;
-    bf16x8 xf1[2], wf1[NB];
-    // slices 0 .. 2: the fragments of slice s+1 are requested before the products of slice s
+    // products of the fragments in f; between them the next slice's fragments are read and, for `turn` 0 .. 3 (the block's last
+    // slice, then three of the block behind it), the requests of a block sent
+    static_assert(NB >= 2, "a product for every fragment read");
+    auto products = [&](int f, int turn, int next_slice) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) xf1[j] = *(const bf16x8*)(st + a_lane + j * 32 * ROWB + frag_off[1]);
+      for (int q = 0; q < 2 * NB; ++q) {
+        const int i = q / 2, j = q % 2;
+        __builtin_amdgcn_sched_barrier(0);
+        if (q < 2) xf[f ^ 1][q] = x_frag(xst, q, next_slice);
+        else if (q < 2 + NB) wf[f ^ 1][q - 2] = w_frag(wst, q - 2, next_slice);
+        __builtin_amdgcn_sched_barrier(0);
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[f][i], xf[f][j], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        constexpr int L = A_LOADS + B_LOADS, SPAN = (BN == 128 ? 6 : 4) * NB;
+        const int p = turn * 2 * NB + q, r0 = p * L / SPAN, r1 = (p + 1) * L / SPAN;
+        if (p < SPAN && (kb > 0 || turn == 0)) {
+          if (r0 < r1 && loader)
 #pragma unroll
-    for (int i = 0; i < NB; ++i) wf1[i] = *(const bf16x8*)(st + b_lane + i * 32 * ROWB + frag_off[1]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf0[i], xf0[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) xf0[j] = *(const bf16x8*)(st + a_lane + j * 32 * ROWB + frag_off[2]);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) wf0[i] = *(const bf16x8*)(st + b_lane + i * 32 * ROWB + frag_off[2]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf1[i], xf1[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < 2; ++j) xf1[j] = *(const bf16x8*)(st + a_lane + j * 32 * ROWB + frag_off[3]);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) wf1[i] = *(const bf16x8*)(st + b_lane + i * 32 * ROWB + frag_off[3]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf0[i], xf0[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    // the next block has landed, and every fragment of this one is in registers: publish / free
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((STAGES - 2) * (A_LOADS + B_LOADS)) : "memory");
-    if (STATS == 1 && kb == 0) {
-      // (every load of this wave is back here, the partial sums among them: no wait of their own;
-      // the factors are published by the barriers of the blocks that follow)
-      rpart += __shfl_xor(rpart, 1);
-      if ((tid & 1) == 0) ((float*)(gsm + STAGES * STAGE))[tid >> 1] = rsqrtf(rpart * rs->inv_cols + rs->eps);
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) xf0[j] = *(const bf16x8*)(sn + a_lane + j * 32 * ROWB + frag_off[0]);
-#pragma unroll
-    for (int i = 0; i < NB; ++i) wf0[i] = *(const bf16x8*)(sn + b_lane + i * 32 * ROWB + frag_off[0]);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf1[i], xf1[j], acc[i][j], 0, 0, 0);
-        if (i == 0 && j == 0) {
-          __builtin_amdgcn_sched_barrier(0);
-          issue_block();                              // the block after next, into the stage just freed
+            for (int r = r0; r < r1; ++r) {
+              if (r < B_LOADS) request_w(r);
+              else request_x(r - B_LOADS);
+            }
+          if (p == SPAN - 1) {
+            next_w();
+            next_x();
+          }
         }
       }
-    __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    products(0, 1, 1);
+    products(1, 2, 2);
+    products(0, 3, 3);
+    // the next block has landed, and every fragment of this one is in registers: publish / free
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((X_STAGES - 2) * A_LOADS + (W_STAGES - 2) * B_LOADS) : "memory");
+    xst = xst == gsm + (X_STAGES - 1) * A_BYTES ? gsm : xst + A_BYTES;
+    wst = wst == gsm + W_RING + (W_STAGES - 1) * B_BYTES ? gsm + W_RING : wst + B_BYTES;
+    products(1, 0, 0);
   }
-  staged_epilogue<BN, EPI, STAGES * STAGE, STATS>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n);
+  float factor = 1.f;
+  if (STATS == 1) {
+    const f32x4 r = rraw[0], r2 = rraw[1];
+    const float half = ((r.x + r.y) + (r.z + r.w)) + ((r2.x + r2.y) + (r2.z + r2.w));
+    factor = rsqrtf((half + __shfl_xor(half, 1)) * rs->inv_cols + rs->eps);
+  }
+  staged_epilogue<BN, EPI, pair_lds(BN), STATS>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n, factor);
 }
 
 template <int BN, int EPI>
@@ -1235,7 +1242,7 @@ template <int BN0>
 static int launch_pair_dual_normed(const bf16_t* x, int64_t M, int64_t K, int64_t ldx,
                                    const mvpa::linear_pair_problem& plain, const mvpa::linear_pair_problem& gated,
                                    const mvpa::row_stats& rs, hipStream_t s) {
-  constexpr int LDS = pair_lds(BN0, 256) + 1024;     // ring + the tile's 256 norm factors
+  constexpr int LDS = pair_lds(BN0, 256);
   auto kern = linear_bf16_pair_dual_normed_kernel<BN0>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   const int64_t mt = (M + 255) / 256;
