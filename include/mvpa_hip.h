@@ -316,6 +316,12 @@ int mvpa_debug_maps(int32_t T, int32_t C, int32_t window, uint32_t flags,
 int mvpa_linear_bf16(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K,
                      int64_t ldx, int64_t ldw, int64_t ldy, int32_t epilogue, void* stream);
 
+/* y[M,N] = x[M,K] @ w[K,N]: the gradient dX = dY W of a product's input, w as the product itself reads it.  Large shapes
+ * only: M >= 512, K a multiple of 64 and at least 128; MVPA_ERR_UNSUPPORTED otherwise.  N and the row strides (in elements)
+ * multiples of 8, 16-byte aligned pointers. */
+int mvpa_linear_bf16_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                        int64_t ldy, void* stream);
+
 /* y[M,N] = x[M,K] @ w[N,K]^T + r[M,N]: the product with the residual rows added in its epilogue
  * (the sum is rounded to bf16 once more after the add).  With x = [attention output | MLP
  * activations] side by side and w = [c_proj | down_proj] it is the whole tail of the parallel

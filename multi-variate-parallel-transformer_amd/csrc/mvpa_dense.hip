@@ -1,6 +1,7 @@
 // Dense ops around the attention kernel: bf16 MFMA linear (y = x w^T), RMSNorm, the
 // three-way residual add and the db4 wavelet analysis of the segment encoder.
 #include "mvpa_common.h"
+#include "mvpa_mfma_tools.h"
 #include "mvpa_tiles.h"
 
 namespace mvpa {
@@ -951,7 +952,15 @@ constexpr int pair_w_stages(int BN) { return BN == 128 ? 3 : 2; }
 constexpr int pair_lds(int BN) { return (pair_x_stages(BN) * 256 + pair_w_stages(BN) * BN) * 128; }
 constexpr int pair_lds(int BN0, int BN1) { return pair_lds(BN0) > pair_lds(BN1) ? pair_lds(BN0) : pair_lds(BN1); }
 
-template <int BN, int EPI, int STATS = 0>
+// WT: y = x w with w [K, N], the gradient of a product's input (dX = dY W).  A block of w is 64 of its rows by BN columns,
+// requested as it lies; fragments come out of transposing reads, eight rows of which are 64 bytes each: the 16-byte chunks of a
+// row are XORed so that four rows in a row cover all banks.
+template <int BN>
+__device__ inline int swz_wt(int row) {
+  return BN == 192 ? (row & 2) << 1 : (row & 3) << 2;  // (six times 64 bytes a row: the pitch itself tells odd rows from even ones)
+}
+
+template <int BN, int EPI, int STATS = 0, bool WT = false>
 __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gsm,
                                                  const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                  bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
@@ -993,9 +1002,10 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   const int lw = wave % LOADERS;
   int x_kb = 0, w_kb = 0;
   uint32_t x_lds = lds0 + lw * 1024, w_lds = lds0 + W_RING + lw * 1024;
-  const int64_t wrow0 = w_row(0);
+  const int64_t wrow0 = WT ? 0 : w_row(0);
   const bf16_t* xs = X + m0 * ldx;
   const bf16_t* ws = W + wrow0 * ldw;
+  const int64_t ws_step = WT ? BK * ldw : BK;
   uint32_t aoff[A_LOADS], boff[B_LOADS];
   {
     const int rsub = lane >> 3, phys = lane & 7;
@@ -1007,8 +1017,14 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     }
 #pragma unroll
     for (int i = 0; i < B_LOADS; ++i) {
-      const int row = (lw + LOADERS * i) * 8 + rsub;
-      boff[i] = (uint32_t)(((w_row(row) - wrow0) * ldw + ((phys ^ ((row >> 1) & 7)) << 3)) * 2);
+      if (WT) {                                       // columns past the end: its last eight, whose products are not stored
+        const int at = (lw + LOADERS * i) * 64 + lane, row = at / (BN / 8);
+        const int64_t n = n0 + ((at % (BN / 8)) ^ swz_wt<BN>(row)) * 8;
+        boff[i] = (uint32_t)((row * ldw + (n < N ? n : N - 8)) * 2);
+      } else {
+        const int row = (lw + LOADERS * i) * 8 + rsub;
+        boff[i] = (uint32_t)(((w_row(row) - wrow0) * ldw + ((phys ^ ((row >> 1) & 7)) << 3)) * 2);
+      }
     }
   }
   auto request_x = [&](int i) {
@@ -1030,7 +1046,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     w_lds = w_lds >= lds0 + W_RING + (W_STAGES - 1) * B_BYTES ? w_lds - (W_STAGES - 1) * B_BYTES : w_lds + B_BYTES;
     if (w_kb + 1 < nkb) {
       ++w_kb;
-      ws += BK;
+      ws += ws_step;
     }
   };
   const bool loader = wave < LOADERS;
@@ -1040,8 +1056,23 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
 #pragma unroll
   for (int sl = 0; sl < 4; ++sl) frag_off[sl] = ln * ROWB + (((2 * sl + hh) ^ ((ln >> 1) & 7)) << 4);
   const int a_lane = (wm * 64) * ROWB;
+  int w_lane[WT ? NB : 1];                            // WT: rows 8 hh + (ln & 15) / 4, the lane's 4 of 32 columns
+  if (WT) {
+    const int row = 8 * hh + ((ln & 15) >> 2);
+#pragma unroll
+    for (int i = 0; i < NB; ++i)
+      w_lane[WT ? i : 0] = row * (BN * 2) + ((((wc * WN + i * 32) / 8 + 2 * (ln >> 4) + ((ln & 3) >> 1)) ^ swz_wt<BN>(row)) << 4) + ((ln & 1) << 3);
+  }
   auto x_frag = [&](const unsigned char* st, int j, int sl) { return *(const bf16x8*)(st + a_lane + j * 32 * ROWB + frag_off[sl]); };
-  auto w_frag = [&](const unsigned char* st, int i, int sl) { return *(const bf16x8*)(st + (wc * WN + i * 32) * ROWB + frag_off[sl]); };
+  auto w_frag = [&](const unsigned char* st, int i, int sl) {
+    if constexpr (WT) {
+      const unsigned char* p = st + w_lane[i] + 16 * sl * (BN * 2);
+      const bf16x4 lo = el_bf16::read_tr(p), hi = el_bf16::read_tr(p + 4 * (BN * 2));
+      return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      return *(const bf16x8*)(st + (wc * WN + i * 32) * ROWB + frag_off[sl]);
+    }
+  };
 
   // STATS 1: the norm factors of the tile's 256 rows, r = rsqrt(sum of the row's partial sums of
   // squares / K + eps).  Two threads share a row and half of its partial sums each; the loads go
@@ -1149,6 +1180,15 @@ __global__ __launch_bounds__(512) void linear_bf16_pair_kernel(const bf16_t* __r
                                                                const bf16_t* __restrict__ R, int64_t ldr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
   linear_pair_tile<BN, EPI>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, R, ldr);
+}
+
+// y = x w, w [K, N]
+template <int BN>
+__global__ __launch_bounds__(512) void linear_bf16_pair_nn_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
+                                                                  bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
+                                                                  int64_t ldx, int64_t ldw, int64_t ldy) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
+  linear_pair_tile<BN, 0, 0, true>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, nullptr, 0);
 }
 
 // Two products of one launch: y0 = x w0^T (tiles 256 x BN0) and y1 = silu(x wg^T) * (x wu^T)
@@ -1262,6 +1302,16 @@ static int launch_pair(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;
   dim3 grid((unsigned)(((N + OUT_COLS - 1) / OUT_COLS) * ((M + 255) / 256)));
   MVPA_LAUNCH(kern, grid, dim3(512), LDS, s, x, w, y, M, N, K, ldx, ldw, ldy, r, ldr);
+  return mvpa::take_launch_status();
+}
+
+template <int BN>
+static int launch_pair_nn(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                          int64_t ldy, hipStream_t s) {
+  constexpr int LDS = pair_lds(BN);
+  auto kern = linear_bf16_pair_nn_kernel<BN>;
+  mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
+  MVPA_LAUNCH(kern, dim3((unsigned)(((N + BN - 1) / BN) * ((M + 255) / 256))), dim3(512), LDS, s, x, w, y, M, N, K, ldx, ldw, ldy);
   return mvpa::take_launch_status();
 }
 
@@ -2034,6 +2084,20 @@ static int residual_tile_width(int64_t M, int64_t N) {
   auto cost = [&](int bn) -> int64_t { return ((mt * ((N + bn - 1) / bn) + 255) / 256) * bn; };
   const int64_t c256 = cost(256), c192 = cost(192), c128 = cost(128);
   return (c256 <= c192 && c256 <= c128) ? 256 : c192 <= c128 ? 192 : 128;
+}
+
+extern "C" int mvpa_linear_bf16_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                   int64_t ldy, void* stream) {
+  if (!x || !w || !y) return MVPA_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldw < N || ldy < N) return MVPA_ERR_SHAPE;
+  if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) || ((ldx | ldw | ldy | N) & 7)) return MVPA_ERR_ALIGN;
+  if (M < 512 || (K & 63) || K < 128 || 256 * ldx >= ((int64_t)1 << 30) || 64 * ldw >= ((int64_t)1 << 30)) return MVPA_ERR_UNSUPPORTED;
+  hipStream_t s = (hipStream_t)stream;
+  const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
+  const int bn = residual_tile_width(M, N);
+  if (bn == 256) return mvpa::launch_pair_nn<256>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
+  if (bn == 192) return mvpa::launch_pair_nn<192>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
+  return mvpa::launch_pair_nn<128>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
 }
 
 extern "C" int32_t mvpa_linear_sumsq_parts(int64_t M, int64_t N) {

@@ -295,6 +295,26 @@ PyObject* py_linear_wgrad(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linear_nn(dy [M, K], w [K, N]) -> dy w | status
+PyObject* py_linear_nn(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 2, "linear_nn takes dy and w");
+  const Tensor &dy = tensor_of(args[0]), &w = tensor_of(args[1]);
+  on_gpu(dy);
+  on_gpu(w);
+  TORCH_CHECK(dy.dim() == 2 && w.dim() == 2 && dy.size(1) == w.size(0) && dy.scalar_type() == at::kBFloat16 &&
+                  w.scalar_type() == at::kBFloat16,
+              "linear_nn: bf16 matrices");
+  TORCH_CHECK(dy.device() == w.device(), "linear_nn: dy and w on one GPU");
+  const int64_t M = dy.size(0), K = dy.size(1), N = w.size(1);
+  if (dy.stride(1) != 1 || w.stride(1) != 1 || M == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor dx = at::empty({M, N}, dy.options());
+  const int st = mvpa_linear_bf16_nn(dy.data_ptr(), w.data_ptr(), dx.data_ptr(), M, N, K, dy.stride(0), w.stride(0), N, current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(dx) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
 // as_operand, starting at a 16-byte boundary
 Tensor aligned_operand(const Tensor& t, at::ScalarType dt) {
   Tensor r = as_operand(t, dt);
@@ -895,6 +915,7 @@ PyMethodDef kMethods[] = {
     {"backward", (PyCFunction)(void*)py_backward, METH_FASTCALL, "backward of the fused MVPA forward, bf16"},
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
     {"linear_wgrad", (PyCFunction)(void*)py_linear_wgrad, METH_FASTCALL, "dy^T @ x in bf16"},
+    {"linear_nn", (PyCFunction)(void*)py_linear_nn, METH_FASTCALL, "dy @ w in bf16"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
     {"encode_saved", (PyCFunction)(void*)py_encode_saved, METH_FASTCALL, "encode, with what its backward needs"},

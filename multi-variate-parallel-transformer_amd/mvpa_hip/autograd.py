@@ -1,9 +1,9 @@
 """Differentiable wrappers of the library's dense ops, for gradients through the layer and stack
 modules (the reference trains through layers/mvpa.py:280-337 and models/mvpformer.py:132-147).
 
-Forward passes are the library's kernels.  Of the backward passes of the bf16 products dX = dY W is
-on the vendor library through torch.matmul, which reads the transposed operand in place, and dW = dY^T X
-on a kernel of the library where that is the faster one (_weight_gradient).  Norm,
+Forward passes are the library's kernels.  Of the backward passes of the bf16 products dX = dY W and dW = dY^T X
+run on kernels of the library where those are the faster ones (_input_gradient, _weight_gradient), elsewhere on the
+vendor library through torch.matmul, which reads transposed operands in place too.  Norm,
 gated activation and residual sums run on kernels of the library both ways (csrc/mvpa_train.hip).  The attention operator itself is
 `attentions.attn.FlashMVPA` (mvpa_backward kernels).
 """
@@ -61,9 +61,33 @@ def _weight_gradient(dy, x):
     return torch.matmul(dy.t(), x)
 
 
+def _dx_on_kernel(m, n, k) -> bool:
+    """Whether the library's product dY W of [m, k] and [k, n] is the faster one, by its tiles of 256 x 128 (a CU each) and the
+    length of a tile's chain.  us, it / the vendor library, four sets of operands in turn:
+        k 768   [768,.]    2800 rows (66 tiles) 11.7 / 11.3, 4096 (96) 11.7 / 14.0, 6400 12.9 / 20.0, 12800 19.9 / 21.4
+                [1728,.]   1024 rows (56) 12.6 / 10.3, 1600 (98) 12.9 / 14.2, 6400 22.2 / 26.1, 20000 61 / 75
+                [2624,.]   600 rows (63) 12.6 / 11.6, 1024 (84) 12.8 / 13.7, 6400 37 / 45
+        k 1280  [768,.]    3500 rows (84) 16.4 / 15.6, 4096 (96) 16.5 / 18.3, 6400 18.2 / 26.8
+        k 2048  [2048,.]   1600 rows (112) 24.7 / 23.5, 2048 (128) 23.9 / 24.9, 2800 (176) 26 / 37, 20000 160 / 157
+                [5632,.]   600 rows (132) 23.9 / 23.7, 1600 (308) 40.7 / 38.5, 6400 127 / 154
+        k 3456  [768,.]    4096 rows (96) 35.9 / 40.1, 5120 (120) 36.0 / 35.7, 6400 (150) 41.5 / 41.3, 20000 93 / 94
+        k 4096  [1024,.]   4096 rows (128) 43.6 / 41.3, 5120 (160) 49.2 / 49.8, 9000 81 / 77, 12800 96 / 100
+        k 11264 [2048,.]   2048 rows (128) 137 / 115, 2800 (176) 142 / 158, 6400 244 / 363"""
+    return m >= 512 and -(-m // 256) * -(-n // 128) >= (96 if k <= 1536 else 144)
+
+
+def _input_gradient(dy, w):
+    """dy w of bf16 rows, on the library's kernel where that is the faster one."""
+    if _dx_on_kernel(dy.shape[0], w.shape[1], w.shape[0]) and not torch.is_grad_enabled() and not _mapped(dy, w):
+        dx = mvpa_hip.load_ext().linear_nn(dy, w)
+        # contractions that are not whole blocks and rows that do not start at 16-byte boundaries are the vendor library's
+        if type(dx) is not int or dx not in (mvpa_hip.ERR_ALIGN, mvpa_hip.ERR_SHAPE, mvpa_hip.ERR_UNSUPPORTED):
+            return mvpa_hip._taken(dx)
+    return torch.matmul(dy, w)
+
+
 class _LinearFn(torch.autograd.Function):
-    """y = x @ w^T, bf16, any leading shape of x: forward on the GPU library, backward dX on the vendor GEMM and
-    dW as above."""
+    """y = x @ w^T, bf16, any leading shape of x: forward on the GPU library, backward dX and dW as above."""
 
     @staticmethod
     def forward(ctx, x, w):
@@ -77,7 +101,7 @@ class _LinearFn(torch.autograd.Function):
         dy2 = dy.reshape(-1, dy.shape[-1]).contiguous()
         dx = dw = None
         if ctx.needs_input_grad[0]:
-            dx = torch.matmul(dy2, w).view(x.shape)                               # [M,N] @ [N,K]
+            dx = _input_gradient(dy2, w).view(x.shape)                            # [M,N] @ [N,K]
         if ctx.needs_input_grad[1]:
             dw = _weight_gradient(dy2, x.reshape(-1, k))                          # [N,M] @ [M,K]
         return dx, dw

@@ -54,6 +54,32 @@ def test_linear_gated(M, N, K):
     assert (y.double() - ref).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 1e-5
 
 
+# tiles of 128, 192 and 256 columns, whole and ragged; fewer blocks of the contraction than stages, as many and more; rows that
+# lie farther apart than they are long
+@pytest.mark.parametrize("M,N,K,pad", [(512, 8, 128, 0), (600, 136, 192, 8), (700, 776, 256, 0), (12800, 768, 192, 64), (6400, 1720, 320, 8),
+                                       (16384, 1000, 256, 0), (5120, 2624, 768, 0), (4100, 768, 3456, 16)])
+def test_product_with_rows_of_w_contracted(M, N, K, pad):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn((M, K + pad), generator=g, device="cuda").bfloat16()[:, :K]
+    w = (torch.randn((K, N + pad), generator=g, device="cuda") * 0.05).bfloat16()[:, :N]
+    y = mvpa_hip.load_ext().linear_nn(x, w)
+    ref = x.double() @ w.double()
+    assert (y.double() - ref).abs().max().item() <= 2 ** -8 * ref.abs().max().item() + 1e-6
+    # the same chain of sums as the product with w transposed
+    if not pad and N % 64 == 0:
+        assert torch.equal(y, mvpa_hip.linear(x, w.t().contiguous()))
+
+
+def test_product_with_rows_of_w_contracted_refuses():
+    x, w = torch.zeros(512, 128, device="cuda").bfloat16(), torch.zeros(128, 64, device="cuda").bfloat16()
+    nn = mvpa_hip.load_ext().linear_nn
+    for a, b in [(x[:511], w), (x[:, :64], w[:64]), (x[:, :96], w[:96])]:
+        assert nn(a, b) == mvpa_hip.ERR_UNSUPPORTED
+    assert nn(x, w[:, :60]) == mvpa_hip.ERR_ALIGN and nn(x[:, 4:68], w[:64]) == mvpa_hip.ERR_ALIGN
+    with pytest.raises(RuntimeError):
+        nn(x, w[:64])
+
+
 # one block, fewer blocks than the ring holds, as many, a few more and many; rows and columns either side of a tile; tiles of 64 rows
 # (525 x 768, 512 x 2048) and of 128 (576 x 2048, 1024 x 2048); N short of a whole tile
 @pytest.mark.parametrize("M,N,K", [(129, 8, 64), (192, 72, 128), (193, 64, 320), (525, 768, 384), (512, 2048, 192), (576, 2048, 64),
