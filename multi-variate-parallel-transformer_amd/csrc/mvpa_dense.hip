@@ -477,16 +477,17 @@ struct row_stats {
   int32_t parts_out;
 };
 
-template <int BN, int EPI, int LDS_BYTES, int STATS = 0>
-__device__ inline void staged_epilogue(const f32x16 (&acc)[BN / 64][2], unsigned char* gsm, int wave, int lane,
+template <int BN, int EPI, int LDS_BYTES, int STATS = 0, int XJ = 2, int XW = 4>      // XJ, XW: blocks of 32 rows of a wave, waves along the rows
+__device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], unsigned char* gsm, int wave, int lane,
                                        int64_t m0, int64_t n0, int64_t M, int64_t N,
                                        bf16_t* __restrict__ Y, int64_t ldy,
                                        const bf16_t* __restrict__ R, int64_t ldr,
                                        const row_stats* rs = nullptr, int64_t tile_n = 0, float factor = 1.f) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
-  constexpr int WN = BN / 2, NB = WN / 32;
+  constexpr int WW = 8 / XW, WN = BN / WW, NB = WN / 32;
+  static_assert((EPI != 1 && STATS == 0) || (XJ == 2 && XW == 4), "gates and statistics on 256 rows");
   const int ln = lane & 31, hh = lane >> 5;
-  const int wm = wave >> 1, wc = wave & 1;
+  const int wm = wave / WW, wc = wave % WW;
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // requests past the end; last reads
   constexpr int WC = EPI == 1 ? WN / 2 : WN;          // output columns of a wave
   constexpr int PITCH = WC * 2 + 16;                  // bytes per staged row (+16: rows spread over the banks)
@@ -497,17 +498,19 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN / 64][2], unsigned
   const bool vec16 = (ldy & 7) == 0 && ((uintptr_t)Y & 15) == 0 &&
                      (EPI != 2 || ((ldr & 7) == 0 && ((uintptr_t)R & 15) == 0));
   const int64_t ncol0 = n0 + wc * WC;
-  float rnorm[2] = {1.f, 1.f};
+  float rnorm[XJ];
+#pragma unroll
+  for (int j = 0; j < XJ; ++j) rnorm[j] = 1.f;
   if (STATS == 1) {        // the tile's 256 factors, a row's with its two threads, to the lanes that hold its sums
     float* rstat = (float*)(gsm + LDS_BYTES - 1024);
     static_assert(STATS != 1 || 8 * 32 * PITCH <= LDS_BYTES - 1024, "the factors lie behind the staging area");
     if ((lane & 1) == 0) rstat[wave * 32 + (lane >> 1)] = factor;
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 2; ++j) rnorm[j] = rstat[wm * 64 + j * 32 + ln];
+    for (int j = 0; j < XJ; ++j) rnorm[j] = rstat[wm * 64 + j * 32 + ln];
   }
 #pragma unroll
-  for (int j = 0; j < 2; ++j) {
+  for (int j = 0; j < XJ; ++j) {
     if (EPI == 1) {
 #pragma unroll
       for (int p2 = 0; p2 < NB / 2; ++p2)
@@ -541,7 +544,7 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN / 64][2], unsigned
       const int row = it * RPI + rr;
       if (rr >= RPI || row >= 32) continue;         // (CPR = 12: 60 lanes carry 5 rows)
       u32x4 v = *(const u32x4*)(stg + row * PITCH + cc * 16);
-      const int64_t m = m0 + wm * 64 + j * 32 + row;
+      const int64_t m = m0 + wm * (32 * XJ) + j * 32 + row;
       const int64_t n = ncol0 + cc * 8;
       float sq = 0.f;
       if (m < M) {
@@ -946,11 +949,19 @@ static int launch_ring(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 // rows 99 / 95 / 92 / 89, [768,2496] 62 / 62 / 59 / 52, [2048,2048] over 65536 486 / 470 / 446 / 433, [2048,7680] 1650 / 1605 / 1518 /
 // 1480, 8192^3 850 / 820 / 780 / 785; 128 columns, over 6400 rows [768,768] 14.3 / 12.0, [768,1728] 26.2 / 22.2, [768,3456] 46.3 / 36.
 // Same tile order, roles, row mapping and epilogues as the other large-tile kernels.
+// Tiles of 128 columns have 256 rows or fewer (pair_tile_rows): waves of 64 x 64 outputs four by two, of 96 x 32 or 64 x 32 two by four.
 // -----------------------------------------------------------------------------------------
-constexpr int pair_x_stages(int) { return 3; }
-constexpr int pair_w_stages(int BN) { return BN == 128 ? 3 : 2; }
-constexpr int pair_lds(int BN) { return (pair_x_stages(BN) * 256 + pair_w_stages(BN) * BN) * 128; }
-constexpr int pair_lds(int BN0, int BN1) { return pair_lds(BN0) > pair_lds(BN1) ? pair_lds(BN0) : pair_lds(BN1); }
+template <int BN, int XJ = 2, int XW = 4>            // blocks of 32 rows of a wave, waves along the rows
+struct pair_cfg {
+  static constexpr int BM = 32 * XJ * XW, X_STAGES = BM == 256 ? 3 : 4, W_STAGES = BM == 256 && BN != 128 ? 2 : X_STAGES;
+  static constexpr int LOADERS = BN == 128 ? 8 : 4;   // waves that request
+  static constexpr int LDS = (X_STAGES * BM + W_STAGES * BN) * 128;
+  static_assert(LDS <= 160 * 1024, "of a CU");
+};
+template <int BN>
+constexpr int pair_lds = pair_cfg<BN>::LDS;
+template <int BN0>                                    // of a launch whose other tiles have 256 columns
+constexpr int pair_dual_lds = pair_lds<BN0> > pair_lds<256> ? pair_lds<BN0> : pair_lds<256>;
 
 // WT: y = x w with w [K, N], the gradient of a product's input (dX = dY W).  A block of w is 64 of its rows by BN columns,
 // requested as it lies; fragments come out of transposing reads, eight rows of which are 64 bytes each: the 16-byte chunks of a
@@ -960,17 +971,17 @@ __device__ inline int swz_wt(int row) {
   return BN == 192 ? (row & 2) << 1 : (row & 3) << 2;  // (six times 64 bytes a row: the pitch itself tells odd rows from even ones)
 }
 
-template <int BN, int EPI, int STATS = 0, bool WT = false>
+template <int BN, int EPI, int STATS = 0, bool WT = false, int XJ = 2, int XW = 4>
 __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gsm,
                                                  const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                  bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
                                                  int64_t ldx, int64_t ldw, int64_t ldy,
                                                  const bf16_t* __restrict__ R, int64_t ldr,
                                                  const row_stats* rs = nullptr) {
-  constexpr int BM = 256, BK = 64, ROWB = BK * 2, X_STAGES = pair_x_stages(BN), W_STAGES = pair_w_stages(BN);
-  constexpr int WN = BN / 2, NB = WN / 32;            // per-wave extent over w rows
+  using G = pair_cfg<BN, XJ, XW>;
+  constexpr int BM = G::BM, BK = 64, ROWB = BK * 2, X_STAGES = G::X_STAGES, W_STAGES = G::W_STAGES, LOADERS = G::LOADERS;
+  constexpr int WW = 8 / XW, WN = BN / WW, NB = WN / 32;        // per-wave extent over w rows
   constexpr int A_BYTES = BM * ROWB, B_BYTES = BN * ROWB, W_RING = X_STAGES * A_BYTES;
-  constexpr int LOADERS = BN == 128 ? 8 : 4;          // waves that request
   constexpr int A_LOADS = A_BYTES / 1024 / LOADERS, B_LOADS = B_BYTES / 1024 / LOADERS;   // 1 KiB requests of such a wave per block
   static_assert(B_BYTES % (8 * 1024) == 0, "every wave issues the same number of loads");
   static_assert(EPI != 1 || NB % 2 == 0, "gate/up pairs need an even number of sub-blocks");
@@ -978,7 +989,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
-  const int wm = wave >> 1, wc = wave & 1;
+  const int wm = wave / WW, wc = wave % WW;
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;    // output columns per workgroup
   int64_t tile_m, tile_n;
   tile_of_workgroup(tile, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, K, &tile_m, &tile_n);
@@ -1055,7 +1066,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   int frag_off[4];
 #pragma unroll
   for (int sl = 0; sl < 4; ++sl) frag_off[sl] = ln * ROWB + (((2 * sl + hh) ^ ((ln >> 1) & 7)) << 4);
-  const int a_lane = (wm * 64) * ROWB;
+  const int a_lane = wm * (32 * XJ) * ROWB;
   int w_lane[WT ? NB : 1];                            // WT: rows 8 hh + (ln & 15) / 4, the lane's 4 of 32 columns
   if (WT) {
     const int row = 8 * hh + ((ln & 15) >> 2);
@@ -1107,17 +1118,17 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   }
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"((X_STAGES - 1) * A_LOADS + (W_STAGES - 1) * B_LOADS) : "memory");
   asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-  bf16x8 xf[2][2], wf[2][NB];                         // two slices' fragments
+  bf16x8 xf[2][XJ], wf[2][NB];                         // two slices' fragments
 #pragma unroll
-  for (int j = 0; j < 2; ++j) xf[0][j] = x_frag(gsm, j, 0);
+  for (int j = 0; j < XJ; ++j) xf[0][j] = x_frag(gsm, j, 0);
 #pragma unroll
   for (int i = 0; i < NB; ++i) wf[0][i] = w_frag(gsm + W_RING, i, 0);
 
-  f32x16 acc[NB][2];
+  f32x16 acc[NB][XJ];
 #pragma unroll
   for (int i = 0; i < NB; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int j = 0; j < XJ; ++j)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
@@ -1125,19 +1136,22 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   for (int kb = 0; kb < nkb; ++kb) {
     // products of the fragments in f; between them the next slice's fragments are read and, for `turn` 0 .. 3 (the block's last
     // slice, then three of the block behind it), the requests of a block sent
-    static_assert(NB >= 2, "a product for every fragment read");
     auto products = [&](int f, int turn, int next_slice) {
+      constexpr int P = NB * XJ, R = XJ + NB, EACH = R <= P ? P : R;       // products, fragments to read
 #pragma unroll
-      for (int q = 0; q < 2 * NB; ++q) {
-        const int i = q / 2, j = q % 2;
+      for (int q = 0; q < P; ++q) {
+        const int i = q / XJ, j = q % XJ;
         __builtin_amdgcn_sched_barrier(0);
-        if (q < 2) xf[f ^ 1][q] = x_frag(xst, q, next_slice);
-        else if (q < 2 + NB) wf[f ^ 1][q - 2] = w_frag(wst, q - 2, next_slice);
+#pragma unroll
+        for (int z = q * EACH / P; z < (q + 1) * EACH / P; ++z) {
+          if (z < XJ) xf[f ^ 1][z] = x_frag(xst, z, next_slice);
+          else if (z < R) wf[f ^ 1][z - XJ] = w_frag(wst, z - XJ, next_slice);
+        }
         __builtin_amdgcn_sched_barrier(0);
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[f][i], xf[f][j], acc[i][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        constexpr int L = A_LOADS + B_LOADS, SPAN = (BN == 128 ? 6 : 4) * NB;
-        const int p = turn * 2 * NB + q, r0 = p * L / SPAN, r1 = (p + 1) * L / SPAN;
+        constexpr int L = A_LOADS + B_LOADS, SPAN = (BN == 128 ? 3 : 2) * P;
+        const int p = turn * P + q, r0 = p * L / SPAN, r1 = (p + 1) * L / SPAN;
         if (p < SPAN && (kb > 0 || turn == 0)) {
           if (r0 < r1 && loader)
 #pragma unroll
@@ -1168,10 +1182,10 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     const float half = ((r.x + r.y) + (r.z + r.w)) + ((r2.x + r2.y) + (r2.z + r2.w));
     factor = rsqrtf((half + __shfl_xor(half, 1)) * rs->inv_cols + rs->eps);
   }
-  staged_epilogue<BN, EPI, pair_lds(BN), STATS>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n, factor);
+  staged_epilogue<BN, EPI, G::LDS, STATS, XJ, XW>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n, factor);
 }
 
-template <int BN, int EPI>
+template <int BN, int EPI, int XJ = 2, int XW = 4>
 __global__ __launch_bounds__(512) void linear_bf16_pair_kernel(const bf16_t* __restrict__ X,
                                                                const bf16_t* __restrict__ W,
                                                                bf16_t* __restrict__ Y, int64_t M,
@@ -1179,16 +1193,16 @@ __global__ __launch_bounds__(512) void linear_bf16_pair_kernel(const bf16_t* __r
                                                                int64_t ldw, int64_t ldy,
                                                                const bf16_t* __restrict__ R, int64_t ldr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
-  linear_pair_tile<BN, EPI>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, R, ldr);
+  linear_pair_tile<BN, EPI, 0, false, XJ, XW>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, R, ldr);
 }
 
 // y = x w, w [K, N]
-template <int BN>
+template <int BN, int XJ = 2, int XW = 4>
 __global__ __launch_bounds__(512) void linear_bf16_pair_nn_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
                                                                   bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
                                                                   int64_t ldx, int64_t ldw, int64_t ldy) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
-  linear_pair_tile<BN, 0, 0, true>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, nullptr, 0);
+  linear_pair_tile<BN, 0, 0, true, XJ, XW>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, nullptr, 0);
 }
 
 // Two products of one launch: y0 = x w0^T (tiles 256 x BN0) and y1 = silu(x wg^T) * (x wu^T)
@@ -1269,7 +1283,7 @@ template <int BN>
 static int launch_pair_sumsq(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K,
                              int64_t ldx, int64_t ldw, int64_t ldy, hipStream_t s, const bf16_t* r, int64_t ldr,
                              float* ss_out, int32_t parts) {
-  constexpr int LDS = pair_lds(BN);
+  constexpr int LDS = pair_lds<BN>;
   auto kern = linear_bf16_pair_sumsq_kernel<BN>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   dim3 grid((unsigned)(((N + BN - 1) / BN) * ((M + 255) / 256)));
@@ -1282,7 +1296,7 @@ template <int BN0>
 static int launch_pair_dual_normed(const bf16_t* x, int64_t M, int64_t K, int64_t ldx,
                                    const mvpa::linear_pair_problem& plain, const mvpa::linear_pair_problem& gated,
                                    const mvpa::row_stats& rs, hipStream_t s) {
-  constexpr int LDS = pair_lds(BN0, 256);
+  constexpr int LDS = pair_dual_lds<BN0>;
   auto kern = linear_bf16_pair_dual_normed_kernel<BN0>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   const int64_t mt = (M + 255) / 256;
@@ -1292,33 +1306,42 @@ static int launch_pair_dual_normed(const bf16_t* x, int64_t M, int64_t K, int64_
   return mvpa::take_launch_status();
 }
 
-template <int BN, int EPI>
+// Rows of a tile of 128 columns: the fewest that give a CU no second tile.  What such a launch takes is the chain of one tile's
+// blocks, and a block of 128 / 192 / 256 rows is 0.4 / 0.5 / 0.65 us.  us, tiles of 256 / 192 / 128 rows: [768,768] over 4096 rows
+// 11.3 / 10.3 / 8.6, 6400 (300 tiles of 128) 12.8 / 11.8 / 16.6; [768,1728] 4096 19.9 / 18.7 / 14.8, 6400 23.0 / 20.6 / 30.8; [1280,768] 3200
+// 12.5 / 11.1 / 9.9, 6400 (340 of 192) 15.3 / 22.8 / 18.3; dX of [3456,768] 512 35.0 / 29.3 / 23.5, 6400 41.6 / 39.5 / 52.9.
+static int pair_tile_rows(int64_t M, int64_t N) {
+  const int64_t nt = (N + 127) / 128;
+  return (M + 127) / 128 * nt <= 256 ? 128 : (M + 191) / 192 * nt <= 256 ? 192 : 256;
+}
+
+template <int BN, int EPI, int XJ = 2, int XW = 4>
 static int launch_pair(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K,
                        int64_t ldx, int64_t ldw, int64_t ldy, hipStream_t s,
                        const bf16_t* r = nullptr, int64_t ldr = 0) {
-  constexpr int LDS = pair_lds(BN);
-  auto kern = linear_bf16_pair_kernel<BN, EPI>;
-  mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
+  using G = mvpa::pair_cfg<BN, XJ, XW>;
+  auto kern = linear_bf16_pair_kernel<BN, EPI, XJ, XW>;
+  mvpa::want_dynamic_lds((const void*)kern, G::LDS);
   constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;
-  dim3 grid((unsigned)(((N + OUT_COLS - 1) / OUT_COLS) * ((M + 255) / 256)));
-  MVPA_LAUNCH(kern, grid, dim3(512), LDS, s, x, w, y, M, N, K, ldx, ldw, ldy, r, ldr);
+  dim3 grid((unsigned)(((N + OUT_COLS - 1) / OUT_COLS) * ((M + G::BM - 1) / G::BM)));
+  MVPA_LAUNCH(kern, grid, dim3(512), G::LDS, s, x, w, y, M, N, K, ldx, ldw, ldy, r, ldr);
   return mvpa::take_launch_status();
 }
 
-template <int BN>
+template <int BN, int XJ = 2, int XW = 4>
 static int launch_pair_nn(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                           int64_t ldy, hipStream_t s) {
-  constexpr int LDS = pair_lds(BN);
-  auto kern = linear_bf16_pair_nn_kernel<BN>;
-  mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
-  MVPA_LAUNCH(kern, dim3((unsigned)(((N + BN - 1) / BN) * ((M + 255) / 256))), dim3(512), LDS, s, x, w, y, M, N, K, ldx, ldw, ldy);
+  using G = mvpa::pair_cfg<BN, XJ, XW>;
+  auto kern = linear_bf16_pair_nn_kernel<BN, XJ, XW>;
+  mvpa::want_dynamic_lds((const void*)kern, G::LDS);
+  MVPA_LAUNCH(kern, dim3((unsigned)(((N + BN - 1) / BN) * ((M + G::BM - 1) / G::BM))), dim3(512), G::LDS, s, x, w, y, M, N, K, ldx, ldw, ldy);
   return mvpa::take_launch_status();
 }
 
 template <int BN0>
 static int launch_pair_dual(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const mvpa::linear_pair_problem& plain,
                             const mvpa::linear_pair_problem& gated, hipStream_t s) {
-  constexpr int LDS = pair_lds(BN0, 256);
+  constexpr int LDS = pair_dual_lds<BN0>;
   auto kern = linear_bf16_pair_dual_kernel<BN0>;
   mvpa::want_dynamic_lds((const void*)kern, (int)LDS);
   const int64_t mt = (M + 255) / 256;
@@ -1997,6 +2020,9 @@ extern "C" int mvpa_linear_bf16(const void* x, const void* w, void* y, int64_t M
       return pair ? launch_pair<192, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s)
            : ring ? launch_ring<192, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s)
                   : launch_big<192, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s);
+    const int rows = pair ? pair_tile_rows(M, N) : 256;
+    if (rows == 128) return launch_pair<128, 0, 2, 2>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s);
+    if (rows == 192) return launch_pair<128, 0, 3, 2>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s);
     return pair ? launch_pair<128, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s)
            : ring ? launch_ring<128, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s)
                 : launch_big<128, 0>(xp, wp, yp, M, N, K, ldx, ldw, ldy, s);
@@ -2097,6 +2123,9 @@ extern "C" int mvpa_linear_bf16_nn(const void* x, const void* w, void* y, int64_
   const int bn = residual_tile_width(M, N);
   if (bn == 256) return mvpa::launch_pair_nn<256>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
   if (bn == 192) return mvpa::launch_pair_nn<192>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
+  const int rows = mvpa::pair_tile_rows(M, N);
+  if (rows == 128) return mvpa::launch_pair_nn<128, 2, 2>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
+  if (rows == 192) return mvpa::launch_pair_nn<128, 3, 2>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
   return mvpa::launch_pair_nn<128>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
 }
 

@@ -494,17 +494,17 @@ static int launch_linear_t(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, c
   return take_launch_status();
 }
 
-// Where 256-row tiles leave most CUs without work, and below 512 rows, where they are not used.  us, large tiles (below 512 rows
-// the 128 x 128 ones) / these: [768,768] 129 rows 20.4 / 5.1, 525 11.9 / 5.2, 1600 12.2 / 6.8, 3000 (288 tiles) 14.2 / 11.3; [768,2624] 525
-// 35.2 / 10.3, 3000 38.0 / 28.9; [2048,2048] 129 40.7 / 8.3, 1152 (288) 28.9 / 19.2; [2048,576] 1152 10.5 / 8.3; [8,768] 16384 (128) 13.7 /
-// 5.3; [256,8192] 4096 (128) 97.5 / 40.6.  Past the line, before the XCDs shared the tiles: [768,768] 4096 rows (384) 14.6 / 14.9, [768,2624]
-// 37.4 / 42.6, [2048,2048] 2048 (512) 28.8 / 25.8, 3000 (768) 30.4 / 46.1, [2048,576] 2048 11.4 / 12.0.  Up to 128 rows keep the kernels of a
+// Where large tiles leave most CUs without work: up to one of these a CU, and below 512 rows, where large ones are not used, up to 288.
+// us, large tiles (below 512 rows the 128 x 128 ones without a ring, from there the ones of pair_tile_rows) / these: [768,768] 129 rows 20.4 /
+// 5.1, 525 8.0 / 7.2, 1600 8.1 / 7.2, 2500 8.2 / 8.4, 3000 (288 tiles) 8.2 / 11.1; [768,2624] 525 17.9 / 9.7, 2500 18.5 / 18.3, 3000 18.6 / 28;
+// [2048,2048] 129 40.7 / 8.3, 800 15.7 / 12.1, 1152 (288) 17.1 / 19.0; [1280,768] 1600 (260) 8.5 / 9.7; [256,8192] 6000 (188) 70 / 61; [64,4096] 6000
+// 26.5 / 13.5: of 64 columns and fewer they stay, half of a large tile would be empty.  Up to 128 rows keep the kernels of a
 // step, whose sums are in another order, and not for their speed: [768,576] 64 rows 7.7 / 4.1, [768,2624] 11.8 / 9.2, [2048,2048] 128 14.4 /
 // 7.9, 1 8.9 / 7.6; [1024,4096] 32 12.9 / 12.9, 1 11.1 / 12.7.
 bool tile_linear_pays(int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw, int64_t ldy, const void* y) {
-  const int64_t ct = (N + TL_BN - 1) / TL_BN;
+  const int64_t ct = (N + TL_BN - 1) / TL_BN, most = M >= 512 && N > TL_BN && K >= 128 ? 256 : 288;
   return M > 128 && K % TL_BK == 0 && N % 8 == 0 && ldy % 8 == 0 && ((uintptr_t)y & 15) == 0 && M < (1 << 20) && N < (1 << 20) &&
-         K < (1 << 30) && 128 * ldx < (1 << 30) && N * ldw < ((int64_t)1 << 31) && (M + 127) / 128 * ct <= 288;
+         K < (1 << 30) && 128 * ldx < (1 << 30) && N * ldw < ((int64_t)1 << 31) && (M + 127) / 128 * ct <= most;
 }
 
 int launch_tile_linear(const bf16_t* x, int64_t M, int64_t K, int64_t ldx, const bf16_t* w, int64_t N, int64_t ldw, bf16_t* y,

@@ -62,18 +62,20 @@ def _weight_gradient(dy, x):
 
 
 def _dx_on_kernel(m, n, k) -> bool:
-    """Whether the library's product dY W of [m, k] and [k, n] is the faster one, by its tiles of 256 x 128 (a CU each) and the
-    length of a tile's chain.  us, it / the vendor library, four sets of operands in turn:
-        k 768   [768,.]    2800 rows (66 tiles) 11.7 / 11.3, 4096 (96) 11.7 / 14.0, 6400 12.9 / 20.0, 12800 19.9 / 21.4
-                [1728,.]   1024 rows (56) 12.6 / 10.3, 1600 (98) 12.9 / 14.2, 6400 22.2 / 26.1, 20000 61 / 75
-                [2624,.]   600 rows (63) 12.6 / 11.6, 1024 (84) 12.8 / 13.7, 6400 37 / 45
-        k 1280  [768,.]    3500 rows (84) 16.4 / 15.6, 4096 (96) 16.5 / 18.3, 6400 18.2 / 26.8
-        k 2048  [2048,.]   1600 rows (112) 24.7 / 23.5, 2048 (128) 23.9 / 24.9, 2800 (176) 26 / 37, 20000 160 / 157
-                [5632,.]   600 rows (132) 23.9 / 23.7, 1600 (308) 40.7 / 38.5, 6400 127 / 154
-        k 3456  [768,.]    4096 rows (96) 35.9 / 40.1, 5120 (120) 36.0 / 35.7, 6400 (150) 41.5 / 41.3, 20000 93 / 94
-        k 4096  [1024,.]   4096 rows (128) 43.6 / 41.3, 5120 (160) 49.2 / 49.8, 9000 81 / 77, 12800 96 / 100
-        k 11264 [2048,.]   2048 rows (128) 137 / 115, 2800 (176) 142 / 158, 6400 244 / 363"""
-    return m >= 512 and -(-m // 256) * -(-n // 128) >= (96 if k <= 1536 else 144)
+    """Whether the library's product dY W of [m, k] and [k, n] is the faster one, by its tiles of 128 x 128.  us, it / the vendor
+    library, four sets of operands in turn:
+        k 192   [640,.]    600 rows (25 tiles) 4.6 / 4.9, 6400 5.4 / 7.9
+        k 512   [512,.]    600 rows (20) 6.4 / 6.9, 6400 7.6 / 11.5
+        k 768   [576,.]    1600 rows (65) 9.0 / 8.6, 2048 (80) 8.9 / 10.8
+                [768,.]    1024 rows (48) 8.5 / 8.4, 1600 (78) 8.7 / 11.1, 6400 12.5 / 20.7, 20000 28.0 / 28.5
+                [1728,.]   600 rows (70) 8.9 / 9.4, 6400 21.3 / 26.0, 20000 62 / 75
+        k 1280  [768,.]    1024 rows (48) 11.5 / 11.2, 1600 (78) 11.7 / 12.3, 6400 18.8 / 27.2
+        k 2048  [2048,.]   600 rows (80) 16.5 / 17.1, 2800 27 / 39, 5120 44.7 / 43.8, 20000 162 / 159
+                [5632,.]   600 rows (220) 20.4 / 24.6, 1600 41.2 / 39.7, 6400 129 / 158
+        k 3456  [768,.]    1024 rows (48) 23.7 / 19.9, 1600 (78) 23.8 / 23.6, 4096 29 / 41, 6400 39.9 / 40.7
+        k 4096  [1024,.]   1024 rows (64) 27.4 / 23.3, 1600 (104) 27.7 / 32.0, 6400 57 / 61, 9000 83 / 80, 20000 166 / 156
+        k 11264 [2048,.]   600 rows (80) 79 / 90, 1024 (128) 91 / 87, 6400 250 / 361"""
+    return m >= 512 and (k <= 512 or -(-m // 128) * -(-n // 128) >= 72)
 
 
 def _input_gradient(dy, w):

@@ -15,8 +15,10 @@ pytestmark = pytest.mark.gpu
                                    (8192, 1000, 200), (16384, 520, 72),
                                    # K a multiple of 64: the 64-wide two-stage kernel, ragged rows and columns, two k-blocks only
                                    (600, 130, 128), (1000, 200, 192), (5000, 333, 256), (513, 257, 1024),
-                                   # 128 columns a tile on three stages: fewer blocks than stages, as many, one more, many
+                                   # tiles of 128 columns and 128 rows: fewer blocks than stages, as many, one more, many
                                    (600, 1000, 128), (5000, 520, 192), (700, 1290, 256), (4097, 776, 1728),
+                                   # of 192 rows, of 256
+                                   (5000, 776, 192), (6400, 768, 256), (6400, 768, 2624), (6400, 1280, 192), (6001, 1290, 320),
                                    # fewer than 128 columns: tiles row by row, 20 and 64 rows of them, one column
                                    (5000, 2056, 64), (16384, 1000, 96), (40000, 130, 120), (5000, 777, 127),
                                    # 32 and 64 columns of tiles, the last one ragged
@@ -54,10 +56,10 @@ def test_linear_gated(M, N, K):
     assert (y.double() - ref).abs().max().item() <= 2 ** -7 * ref.abs().max().item() + 1e-5
 
 
-# tiles of 128, 192 and 256 columns, whole and ragged; fewer blocks of the contraction than stages, as many and more; rows that
+# tiles of 128 (of 128, 192 and 256 rows), 192 and 256 columns, whole and ragged; fewer blocks of the contraction than stages, as many and more; rows that
 # lie farther apart than they are long
 @pytest.mark.parametrize("M,N,K,pad", [(512, 8, 128, 0), (600, 136, 192, 8), (700, 776, 256, 0), (12800, 768, 192, 64), (6400, 1720, 320, 8),
-                                       (16384, 1000, 256, 0), (5120, 2624, 768, 0), (4100, 768, 3456, 16)])
+                                       (16384, 1000, 256, 0), (6400, 768, 320, 0), (6001, 1288, 192, 8), (5120, 2624, 768, 0), (4100, 768, 3456, 16)])
 def test_product_with_rows_of_w_contracted(M, N, K, pad):
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn((M, K + pad), generator=g, device="cuda").bfloat16()[:, :K]
