@@ -322,6 +322,18 @@ int mvpa_linear_bf16(const void* x, const void* w, void* y, int64_t M, int64_t N
 int mvpa_linear_bf16_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                         int64_t ldy, void* stream);
 
+/* The same with the rows of w in two matrices [K0,N] and [K1,N] of one row pitch, K0 and K1 multiples of 64. */
+int mvpa_linear_bf16_nn2(const void* x, const void* w0, const void* w1, void* y, int64_t M, int64_t N, int64_t K0, int64_t K1,
+                         int64_t ldx, int64_t ldw, int64_t ldy, void* stream);
+
+/* The gated MLP of a training pass (models/mvpformer.py:114): gu = [x @ wg^T | x @ wu^T] (contiguous rows of 2 N) and mid =
+ * silu(gate) * up of the rounded rows (contiguous rows of N), in one launch; and dgu = [dgate | dup] for the gradient dy of
+ * y = mid @ wd^T, wd [K,N], from gu as the forward left it.  Shapes as mvpa_linear_bf16_nn, gu, mid and dgu contiguous. */
+int mvpa_gated_rows_bf16(const void* x, const void* wg, const void* wu, void* gu, void* mid, int64_t M, int64_t N, int64_t K,
+                         int64_t ldx, int64_t ldw, void* stream);
+int mvpa_gated_rows_backward_bf16(const void* dy, const void* wd, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K,
+                                  int64_t lddy, int64_t ldw, void* stream);
+
 /* y[M,N] = x[M,K] @ w[N,K]^T + r[M,N]: the product with the residual rows added in its epilogue
  * (the sum is rounded to bf16 once more after the add).  With x = [attention output | MLP
  * activations] side by side and w = [c_proj | down_proj] it is the whole tail of the parallel

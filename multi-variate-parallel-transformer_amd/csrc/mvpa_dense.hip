@@ -469,6 +469,19 @@ __device__ inline void tile_of_workgroup(int64_t L, int64_t mt64, int64_t nt64, 
 //            is converted (the norm's weight is folded into w's columns by the caller);
 //   STATS 2  the partial sums of squares of the rows this product writes (final bf16 values, this
 //            wave's columns) go to ss_out[m][2 * column tile + column half].
+// The MLP of a training pass (models/mvpformer.py:114), EPI 3 and 4:
+//   EPI 3  the tile's columns are BN/2 of the gate and BN/2 of the up product: both are stored side by side (their rows are the
+//          backward's operands) and silu(gate) * up beside them.  A row's gate lies with one wave, its up columns with
+//          another: they meet where the staged rows are read back, each wave taking every other group of rows;
+//   EPI 4  the product is the gradient of silu(gate) * up: the rows of gate and up that the forward stored are requested in front of
+//          the staging, and their gradients leave in its place.
+// The values are those of the passes by themselves (silu_gate_kernel, silu_gate_backward_kernel), which would read again what was just
+// written.
+struct gated_rows {
+  const bf16_t* gu;        // [M][2 N], gate then up; what EPI 3 stores is y
+  bf16_t* mid;             // [M][N]
+};
+
 struct row_stats {
   const float* ss_in;      // [M][parts_in]
   int32_t parts_in;
@@ -477,15 +490,19 @@ struct row_stats {
   int32_t parts_out;
 };
 
+// to 3 ulp: one wave of the two on a SIMD has nobody to hide the forty instructions of expf and a division behind
+__device__ inline float fast_sigmoid(float g) { return __builtin_amdgcn_rcpf(1.f + __builtin_amdgcn_exp2f(-g * 1.44269504f)); }
+
 template <int BN, int EPI, int LDS_BYTES, int STATS = 0, int XJ = 2, int XW = 4>      // XJ, XW: blocks of 32 rows of a wave, waves along the rows
 __device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], unsigned char* gsm, int wave, int lane,
                                        int64_t m0, int64_t n0, int64_t M, int64_t N,
                                        bf16_t* __restrict__ Y, int64_t ldy,
                                        const bf16_t* __restrict__ R, int64_t ldr,
-                                       const row_stats* rs = nullptr, int64_t tile_n = 0, float factor = 1.f) {
+                                       const row_stats* rs = nullptr, int64_t tile_n = 0, float factor = 1.f,
+                                       const gated_rows& gr = {}) {
   typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
   constexpr int WW = 8 / XW, WN = BN / WW, NB = WN / 32;
-  static_assert((EPI != 1 && STATS == 0) || (XJ == 2 && XW == 4), "gates and statistics on 256 rows");
+  static_assert((EPI != 1 && STATS == 0) || (XJ == 2 && XW == 4), "interleaved gates and statistics on 256 rows");
   const int ln = lane & 31, hh = lane >> 5;
   const int wm = wave / WW, wc = wave % WW;
   asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");   // requests past the end; last reads
@@ -497,7 +514,7 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], u
   unsigned char* stg = gsm + wave * (32 * PITCH);
   const bool vec16 = (ldy & 7) == 0 && ((uintptr_t)Y & 15) == 0 &&
                      (EPI != 2 || ((ldr & 7) == 0 && ((uintptr_t)R & 15) == 0));
-  const int64_t ncol0 = n0 + wc * WC;
+  const int64_t ncol0 = n0 + (EPI == 3 ? wc % (WW / 2) : wc) * WC;
   float rnorm[XJ];
 #pragma unroll
   for (int j = 0; j < XJ; ++j) rnorm[j] = 1.f;
@@ -509,6 +526,18 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], u
 #pragma unroll
     for (int j = 0; j < XJ; ++j) rnorm[j] = rstat[wm * 64 + j * 32 + ln];
   }
+  constexpr int ITS = (32 + RPI - 1) / RPI;
+  u32x4 gate[2][EPI == 4 ? ITS : 1], up[2][EPI == 4 ? ITS : 1];
+  auto request_gates = [&](int j) {                   // (past the end: the last row and columns, for nobody)
+#pragma unroll
+    for (int it = 0; it < ITS; ++it) {
+      const int64_t m = m0 + wm * (32 * XJ) + j * 32 + it * RPI + lane / CPR, n = ncol0 + lane % CPR * 8;
+      const bf16_t* at = gr.gu + (m < M ? m : M - 1) * (2 * N) + (n < N ? n : N - 8);
+      gate[j & 1][EPI == 4 ? it : 0] = *(const u32x4*)at;
+      up[j & 1][EPI == 4 ? it : 0] = *(const u32x4*)(at + N);
+    }
+  };
+  if (EPI == 4) request_gates(0);
 #pragma unroll
   for (int j = 0; j < XJ; ++j) {
     if (EPI == 1) {
@@ -538,12 +567,47 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], u
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (EPI == 3) __syncthreads();
+    if (EPI == 4 && j + 1 < XJ) request_gates(j + 1);
     const int rr = lane / CPR, cc = lane % CPR;
 #pragma unroll
-    for (int it = 0; it < (32 + RPI - 1) / RPI; ++it) {
+    for (int it = 0; it < ITS; ++it) {
       const int row = it * RPI + rr;
       if (rr >= RPI || row >= 32) continue;         // (CPR = 12: 60 lanes carry 5 rows)
       u32x4 v = *(const u32x4*)(stg + row * PITCH + cc * 16);
+      if (EPI == 3 || EPI == 4) {                     // whole chunks: N is a multiple of 8
+        const int64_t m = m0 + wm * (32 * XJ) + j * 32 + row, n = ncol0 + cc * 8;
+        if (m >= M || n >= N) continue;
+        const bool is_up = EPI == 3 && wc >= WW / 2;
+        bf16_t* dst = Y + m * ldy + n;
+        if (EPI == 4) {
+          bf16x8 dg, du;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            auto wide = [&](u32x4 x) { return __uint_as_float(e & 1 ? x[e >> 1] & 0xffff0000u : x[e >> 1] << 16); };
+            const float g = wide(gate[j & 1][EPI == 4 ? it : 0]), u = wide(up[j & 1][EPI == 4 ? it : 0]), d = wide(v), s = fast_sigmoid(g);
+            dg[e] = (__bf16)(d * u * (s * (1.f + g * (1.f - s))));
+            du[e] = (__bf16)(d * g * s);
+          }
+          __builtin_nontemporal_store(dg, (bf16x8*)dst);
+          __builtin_nontemporal_store(du, (bf16x8*)(dst + N));
+          continue;
+        }
+        __builtin_nontemporal_store(v, (u32x4*)(dst + (is_up ? N : 0)));
+        if ((it & 1) == (is_up ? 1 : 0)) {
+          const int other = wm * WW + (wc + WW / 2) % WW;
+          const u32x4 w = *(const u32x4*)(gsm + other * (32 * PITCH) + row * PITCH + cc * 16);
+          bf16x8 o;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            auto wide = [&](u32x4 x) { return __uint_as_float(e & 1 ? x[e >> 1] & 0xffff0000u : x[e >> 1] << 16); };
+            const float g = wide(is_up ? w : v), u = wide(is_up ? v : w);
+            o[e] = (__bf16)(g * fast_sigmoid(g) * u);
+          }
+          __builtin_nontemporal_store(o, (bf16x8*)(gr.mid + m * N + n));
+        }
+        continue;
+      }
       const int64_t m = m0 + wm * (32 * XJ) + j * 32 + row;
       const int64_t n = ncol0 + cc * 8;
       float sq = 0.f;
@@ -588,6 +652,7 @@ __device__ inline void staged_epilogue(const f32x16 (&acc)[BN * XW / 256][XJ], u
         if (cc == 0 && m < M) rs->ss_out[m * rs->parts_out + tile_n * 2 + wc] = sq;
       }
     }
+    if (EPI == 3 && j + 1 < XJ) __syncthreads();
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -977,7 +1042,8 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
                                                  bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
                                                  int64_t ldx, int64_t ldw, int64_t ldy,
                                                  const bf16_t* __restrict__ R, int64_t ldr,
-                                                 const row_stats* rs = nullptr) {
+                                                 const row_stats* rs = nullptr, const bf16_t* __restrict__ W2 = nullptr,
+                                                 int split = 0, const gated_rows& gr = {}) {
   using G = pair_cfg<BN, XJ, XW>;
   constexpr int BM = G::BM, BK = 64, ROWB = BK * 2, X_STAGES = G::X_STAGES, W_STAGES = G::W_STAGES, LOADERS = G::LOADERS;
   constexpr int WW = 8 / XW, WN = BN / WW, NB = WN / 32;        // per-wave extent over w rows
@@ -990,7 +1056,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ln = lane & 31, hh = lane >> 5;
   const int wm = wave / WW, wc = wave % WW;
-  constexpr int OUT_COLS = EPI == 1 ? BN / 2 : BN;    // output columns per workgroup
+  constexpr int OUT_COLS = EPI == 1 || EPI == 3 ? BN / 2 : BN;  // output columns per workgroup
   int64_t tile_m, tile_n;
   tile_of_workgroup(tile, (M + BM - 1) / BM, (N + OUT_COLS - 1) / OUT_COLS, K, &tile_m, &tile_n);
   const int64_t m0 = tile_m * BM, n0 = tile_n * OUT_COLS;
@@ -1002,7 +1068,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
       const int64_t col = n0 + wcol * (WN / 2) + (nb >> 1) * 32 + i;
       return ((nb & 1) ? N : 0) + (col < N ? col : N - 1);
     }
-    const int64_t n = n0 + r;
+    const int64_t n = n0 + (EPI == 3 ? r % (BN / 2) : r);         // EPI 3: rows of w, then of w2
     return n < N ? n : N - 1;
   };
 
@@ -1015,7 +1081,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
   uint32_t x_lds = lds0 + lw * 1024, w_lds = lds0 + W_RING + lw * 1024;
   const int64_t wrow0 = WT ? 0 : w_row(0);
   const bf16_t* xs = X + m0 * ldx;
-  const bf16_t* ws = W + wrow0 * ldw;
+  const bf16_t *ws = W + wrow0 * ldw, *ws2 = EPI == 3 ? W2 + wrow0 * ldw : W2;
   const int64_t ws_step = WT ? BK * ldw : BK;
   uint32_t aoff[A_LOADS], boff[B_LOADS];
   {
@@ -1043,8 +1109,9 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
                  :: "v"(aoff[i]), "s"(xs), "s"(x_lds + LOADERS * i * 1024) : "memory", "m0");
   };
   auto request_w = [&](int i) {
+    static_assert(EPI != 3 || B_LOADS % 2 == 0, "requests of either weight");
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-                 :: "v"(boff[i]), "s"(ws), "s"(w_lds + LOADERS * i * 1024) : "memory", "m0");
+                 :: "v"(boff[i]), "s"(EPI == 3 && i >= B_LOADS / 2 ? ws2 : ws), "s"(w_lds + LOADERS * i * 1024) : "memory", "m0");
   };
   auto next_x = [&]() {                               // past the end the last block once more, into a stage nobody reads
     x_lds = x_lds >= lds0 + (X_STAGES - 1) * A_BYTES ? x_lds - (X_STAGES - 1) * A_BYTES : x_lds + A_BYTES;
@@ -1057,7 +1124,8 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     w_lds = w_lds >= lds0 + W_RING + (W_STAGES - 1) * B_BYTES ? w_lds - (W_STAGES - 1) * B_BYTES : w_lds + B_BYTES;
     if (w_kb + 1 < nkb) {
       ++w_kb;
-      ws += ws_step;
+      ws = WT && w_kb == split ? ws2 : ws + ws_step;          // (split 0: never)
+      if (EPI == 3) ws2 += ws_step;
     }
   };
   const bool loader = wave < LOADERS;
@@ -1182,7 +1250,7 @@ __device__ __forceinline__ void linear_pair_tile(int64_t tile, unsigned char* gs
     const float half = ((r.x + r.y) + (r.z + r.w)) + ((r2.x + r2.y) + (r2.z + r2.w));
     factor = rsqrtf((half + __shfl_xor(half, 1)) * rs->inv_cols + rs->eps);
   }
-  staged_epilogue<BN, EPI, G::LDS, STATS, XJ, XW>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n, factor);
+  staged_epilogue<BN, EPI, G::LDS, STATS, XJ, XW>(acc, gsm, wave, lane, m0, n0, M, N, Y, ldy, R, ldr, rs, tile_n, factor, gr);
 }
 
 template <int BN, int EPI, int XJ = 2, int XW = 4>
@@ -1196,13 +1264,24 @@ __global__ __launch_bounds__(512) void linear_bf16_pair_kernel(const bf16_t* __r
   linear_pair_tile<BN, EPI, 0, false, XJ, XW>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, R, ldr);
 }
 
-// y = x w, w [K, N]
-template <int BN, int XJ = 2, int XW = 4>
+// y = x w, w [K, N]; with split, blocks from there on are rows of w2.  EPI 4: gr
+template <int BN, int EPI, int XJ = 2, int XW = 4>
 __global__ __launch_bounds__(512) void linear_bf16_pair_nn_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ W,
-                                                                  bf16_t* __restrict__ Y, int64_t M, int64_t N, int64_t K,
-                                                                  int64_t ldx, int64_t ldw, int64_t ldy) {
+                                                                  const bf16_t* __restrict__ W2, int split, bf16_t* __restrict__ Y,
+                                                                  int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                                                  int64_t ldy, gated_rows gr) {
   extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
-  linear_pair_tile<BN, 0, 0, true, XJ, XW>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, nullptr, 0);
+  linear_pair_tile<BN, EPI, 0, true, XJ, XW>(blockIdx.x, gsm, X, W, Y, M, N, K, ldx, ldw, ldy, nullptr, 0, nullptr, W2, split, gr);
+}
+
+// gate and up rows of x with silu(gate) * up beside them
+template <int BN, int XJ = 2, int XW = 4>
+__global__ __launch_bounds__(512) void linear_bf16_pair_gates_kernel(const bf16_t* __restrict__ X, const bf16_t* __restrict__ WG,
+                                                                     const bf16_t* __restrict__ WU, bf16_t* __restrict__ Y,
+                                                                     int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
+                                                                     gated_rows gr) {
+  extern __shared__ __attribute__((aligned(1024))) unsigned char gsm[];
+  linear_pair_tile<BN, 3, 0, false, XJ, XW>(blockIdx.x, gsm, X, WG, Y, M, N, K, ldx, ldw, 2 * N, nullptr, 0, nullptr, WU, 0, gr);
 }
 
 // Two products of one launch: y0 = x w0^T (tiles 256 x BN0) and y1 = silu(x wg^T) * (x wu^T)
@@ -1328,13 +1407,32 @@ static int launch_pair(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
   return mvpa::take_launch_status();
 }
 
-template <int BN, int XJ = 2, int XW = 4>
-static int launch_pair_nn(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
-                          int64_t ldy, hipStream_t s) {
+struct pair_nn_args {
+  const bf16_t *x, *w, *w2;
+  bf16_t* y;
+  int64_t M, N, K, ldx, ldw, ldy;
+  int split;
+  mvpa::gated_rows gr;
+};
+
+template <int BN, int EPI, int XJ = 2, int XW = 4>
+static int launch_pair_nn_t(const pair_nn_args& a, hipStream_t s) {
   using G = mvpa::pair_cfg<BN, XJ, XW>;
-  auto kern = linear_bf16_pair_nn_kernel<BN, XJ, XW>;
+  auto kern = linear_bf16_pair_nn_kernel<BN, EPI, XJ, XW>;
   mvpa::want_dynamic_lds((const void*)kern, G::LDS);
-  MVPA_LAUNCH(kern, dim3((unsigned)(((N + BN - 1) / BN) * ((M + G::BM - 1) / G::BM))), dim3(512), G::LDS, s, x, w, y, M, N, K, ldx, ldw, ldy);
+  MVPA_LAUNCH(kern, dim3((unsigned)(((a.N + BN - 1) / BN) * ((a.M + G::BM - 1) / G::BM))), dim3(512), G::LDS, s, a.x, a.w, a.w2, a.split,
+              a.y, a.M, a.N, a.K, a.ldx, a.ldw, a.ldy, a.gr);
+  return mvpa::take_launch_status();
+}
+
+template <int BN, int XJ = 2, int XW = 4>
+static int launch_pair_gates(const bf16_t* x, const bf16_t* wg, const bf16_t* wu, bf16_t* gu, bf16_t* mid, int64_t M, int64_t N,
+                             int64_t K, int64_t ldx, int64_t ldw, hipStream_t s) {
+  using G = mvpa::pair_cfg<BN, XJ, XW>;
+  auto kern = linear_bf16_pair_gates_kernel<BN, XJ, XW>;
+  mvpa::want_dynamic_lds((const void*)kern, G::LDS);
+  MVPA_LAUNCH(kern, dim3((unsigned)(((N + BN / 2 - 1) / (BN / 2)) * ((M + G::BM - 1) / G::BM))), dim3(512), G::LDS, s, x, wg, wu, gu, M, N, K,
+              ldx, ldw, mvpa::gated_rows{nullptr, mid});
   return mvpa::take_launch_status();
 }
 
@@ -2112,21 +2210,69 @@ static int residual_tile_width(int64_t M, int64_t N) {
   return (c256 <= c192 && c256 <= c128) ? 256 : c192 <= c128 ? 192 : 128;
 }
 
+template <int EPI>
+static int launch_pair_nn(const mvpa::pair_nn_args& a, hipStream_t s) {
+  const int bn = residual_tile_width(a.M, a.N);
+  if (bn == 256) return mvpa::launch_pair_nn_t<256, EPI>(a, s);
+  if (bn == 192) return mvpa::launch_pair_nn_t<192, EPI>(a, s);
+  const int rows = mvpa::pair_tile_rows(a.M, a.N);
+  if (rows == 128) return mvpa::launch_pair_nn_t<128, EPI, 2, 2>(a, s);
+  if (rows == 192) return mvpa::launch_pair_nn_t<128, EPI, 3, 2>(a, s);
+  return mvpa::launch_pair_nn_t<128, EPI>(a, s);
+}
+
+static int pair_nn_check(const mvpa::pair_nn_args& a) {
+  if (!a.x || !a.w || !a.y) return MVPA_ERR_NULL;
+  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.ldx < a.K || a.ldw < a.N || a.ldy < a.N) return MVPA_ERR_SHAPE;
+  if ((((uintptr_t)a.x | (uintptr_t)a.w | (uintptr_t)a.w2 | (uintptr_t)a.y | (uintptr_t)a.gr.gu) & 15) || ((a.ldx | a.ldw | a.ldy | a.N) & 7))
+    return MVPA_ERR_ALIGN;
+  if (a.M < 512 || (a.K & 63) || a.K < 128 || a.K > ((int64_t)1 << 30) || 256 * a.ldx >= ((int64_t)1 << 30) || 64 * a.ldw >= ((int64_t)1 << 30))
+    return MVPA_ERR_UNSUPPORTED;
+  return MVPA_OK;
+}
+
 extern "C" int mvpa_linear_bf16_nn(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, int64_t ldx, int64_t ldw,
                                    int64_t ldy, void* stream) {
-  if (!x || !w || !y) return MVPA_ERR_NULL;
-  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldw < N || ldy < N) return MVPA_ERR_SHAPE;
-  if ((((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) & 15) || ((ldx | ldw | ldy | N) & 7)) return MVPA_ERR_ALIGN;
-  if (M < 512 || (K & 63) || K < 128 || 256 * ldx >= ((int64_t)1 << 30) || 64 * ldw >= ((int64_t)1 << 30)) return MVPA_ERR_UNSUPPORTED;
+  const mvpa::pair_nn_args a{(const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)y, M, N, K, ldx, ldw, ldy, 0, {}};
+  const int st = pair_nn_check(a);
+  return st == MVPA_OK ? launch_pair_nn<0>(a, (hipStream_t)stream) : st;
+}
+
+extern "C" int mvpa_linear_bf16_nn2(const void* x, const void* w0, const void* w1, void* y, int64_t M, int64_t N, int64_t K0,
+                                    int64_t K1, int64_t ldx, int64_t ldw, int64_t ldy, void* stream) {
+  if (!w1) return MVPA_ERR_NULL;
+  if (K0 <= 0 || K1 <= 0) return MVPA_ERR_SHAPE;
+  const mvpa::pair_nn_args a{(const bf16_t*)x, (const bf16_t*)w0, (const bf16_t*)w1, (bf16_t*)y, M, N, K0 + K1, ldx, ldw, ldy, (int)(K0 / 64), {}};
+  const int st = pair_nn_check(a);
+  if (st != MVPA_OK) return st;
+  return K0 & 63 ? MVPA_ERR_UNSUPPORTED : launch_pair_nn<0>(a, (hipStream_t)stream);
+}
+
+extern "C" int mvpa_gated_rows_bf16(const void* x, const void* wg, const void* wu, void* gu, void* mid, int64_t M, int64_t N, int64_t K,
+                                    int64_t ldx, int64_t ldw, void* stream) {
+  if (!x || !wg || !wu || !gu || !mid) return MVPA_ERR_NULL;
+  if (M <= 0 || N <= 0 || K <= 0 || ldx < K || ldw < K) return MVPA_ERR_SHAPE;
+  if ((((uintptr_t)x | (uintptr_t)wg | (uintptr_t)wu | (uintptr_t)gu | (uintptr_t)mid) & 15) || ((ldx | ldw | N) & 7)) return MVPA_ERR_ALIGN;
+  if (M < 512 || (K & 63) || K < 128 || 256 * ldx >= ((int64_t)1 << 30) || 256 * ldw >= ((int64_t)1 << 30)) return MVPA_ERR_UNSUPPORTED;
   hipStream_t s = (hipStream_t)stream;
-  const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
-  const int bn = residual_tile_width(M, N);
-  if (bn == 256) return mvpa::launch_pair_nn<256>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
-  if (bn == 192) return mvpa::launch_pair_nn<192>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
-  const int rows = mvpa::pair_tile_rows(M, N);
-  if (rows == 128) return mvpa::launch_pair_nn<128, 2, 2>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
-  if (rows == 192) return mvpa::launch_pair_nn<128, 3, 2>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
-  return mvpa::launch_pair_nn<128>(xp, wp, (bf16_t*)y, M, N, K, ldx, ldw, ldy, s);
+  const bf16_t *xp = (const bf16_t*)x, *g = (const bf16_t*)wg, *u = (const bf16_t*)wu;
+  // half of a tile's columns to either weight: the widths as for a product of twice the columns
+  const int64_t cols = 2 * N;
+  const int bn = residual_tile_width(M, cols);
+  if (bn == 256) return mvpa::launch_pair_gates<256>(xp, g, u, (bf16_t*)gu, (bf16_t*)mid, M, N, K, ldx, ldw, s);
+  if (bn == 192) return mvpa::launch_pair_gates<192>(xp, g, u, (bf16_t*)gu, (bf16_t*)mid, M, N, K, ldx, ldw, s);
+  const int rows = mvpa::pair_tile_rows(M, cols);
+  if (rows == 128) return mvpa::launch_pair_gates<128, 2, 2>(xp, g, u, (bf16_t*)gu, (bf16_t*)mid, M, N, K, ldx, ldw, s);
+  if (rows == 192) return mvpa::launch_pair_gates<128, 3, 2>(xp, g, u, (bf16_t*)gu, (bf16_t*)mid, M, N, K, ldx, ldw, s);
+  return mvpa::launch_pair_gates<128>(xp, g, u, (bf16_t*)gu, (bf16_t*)mid, M, N, K, ldx, ldw, s);
+}
+
+extern "C" int mvpa_gated_rows_backward_bf16(const void* dy, const void* wd, const void* gu, void* dgu, int64_t M, int64_t N, int64_t K,
+                                             int64_t lddy, int64_t ldw, void* stream) {
+  if (!gu) return MVPA_ERR_NULL;
+  const mvpa::pair_nn_args a{(const bf16_t*)dy, (const bf16_t*)wd, nullptr, (bf16_t*)dgu, M, N, K, lddy, ldw, 2 * N, 0, {(const bf16_t*)gu, nullptr}};
+  const int st = pair_nn_check(a);
+  return st == MVPA_OK ? launch_pair_nn<4>(a, (hipStream_t)stream) : st;
 }
 
 extern "C" int32_t mvpa_linear_sumsq_parts(int64_t M, int64_t N) {

@@ -315,6 +315,70 @@ PyObject* py_linear_nn(PyObject*, PyObject* const* args, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// linear_nn2(dy [M, K0 + K1], w0 [K0, N], w1 [K1, N]) -> dy [w0; w1] | status
+PyObject* py_linear_nn2(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 3, "linear_nn2 takes dy and the two halves of w");
+  const Tensor &dy = tensor_of(args[0]), &w0 = tensor_of(args[1]), &w1 = tensor_of(args[2]);
+  on_gpu(dy);
+  TORCH_CHECK(dy.dim() == 2 && w0.dim() == 2 && w1.dim() == 2 && w0.size(1) == w1.size(1) && dy.size(1) == w0.size(0) + w1.size(0) &&
+                  dy.scalar_type() == at::kBFloat16 && w0.scalar_type() == at::kBFloat16 && w1.scalar_type() == at::kBFloat16,
+              "linear_nn2: bf16 matrices");
+  TORCH_CHECK(dy.device() == w0.device() && dy.device() == w1.device(), "linear_nn2: operands on one GPU");
+  const int64_t M = dy.size(0), N = w0.size(1);
+  if (dy.stride(1) != 1 || w0.stride(1) != 1 || w1.stride(1) != 1 || w0.stride(0) != w1.stride(0) || M == 0)
+    return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor dx = at::empty({M, N}, dy.options());
+  const int st = mvpa_linear_bf16_nn2(dy.data_ptr(), w0.data_ptr(), w1.data_ptr(), dx.data_ptr(), M, N, w0.size(0), w1.size(0),
+                                      dy.stride(0), w0.stride(0), N, current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(dx) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
+// gated_rows(x [M, K], gate [N, K], up [N, K]) -> (x [gate; up]^T, silu(gate) up) | status
+PyObject* py_gated_rows(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 3, "gated_rows takes x and two weights");
+  const Tensor &x = tensor_of(args[0]), &g = tensor_of(args[1]), &u = tensor_of(args[2]);
+  on_gpu(x);
+  TORCH_CHECK(x.dim() == 2 && g.dim() == 2 && g.sizes() == u.sizes() && g.size(1) == x.size(1) && x.scalar_type() == at::kBFloat16 &&
+                  g.scalar_type() == at::kBFloat16 && u.scalar_type() == at::kBFloat16 && x.device() == g.device() && x.device() == u.device(),
+              "gated_rows: bf16 matrices on one GPU");
+  const int64_t M = x.size(0), N = g.size(0);
+  if (x.stride(1) != 1 || g.stride(1) != 1 || u.stride(1) != 1 || g.stride(0) != u.stride(0) || M == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor gu = at::empty({M, 2 * N}, x.options()), mid = at::empty({M, N}, x.options());
+  const int st = mvpa_gated_rows_bf16(x.data_ptr(), g.data_ptr(), u.data_ptr(), gu.data_ptr(), mid.data_ptr(), M, N, x.size(1), x.stride(0),
+                                      g.stride(0), current_stream());
+  if (st != MVPA_OK) return PyLong_FromLong(st);
+  PyObject* r = PyTuple_New(2);
+  PyTuple_SET_ITEM(r, 0, THPVariable_Wrap(gu));
+  PyTuple_SET_ITEM(r, 1, THPVariable_Wrap(mid));
+  return r;
+  END_HANDLE_TH_ERRORS
+}
+
+// gated_rows_backward(dy [M, K], down [K, N], gu [M, 2 N]) -> the gradient of gu | status
+PyObject* py_gated_rows_backward(PyObject*, PyObject* const* args, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  TORCH_CHECK(n == 3, "gated_rows_backward takes dy, the weight and the rows");
+  const Tensor &dy = tensor_of(args[0]), &w = tensor_of(args[1]), &gu = tensor_of(args[2]);
+  on_gpu(dy);
+  TORCH_CHECK(dy.dim() == 2 && w.dim() == 2 && gu.dim() == 2 && dy.size(1) == w.size(0) && gu.size(0) == dy.size(0) &&
+                  gu.size(1) == 2 * w.size(1) && gu.is_contiguous() && dy.scalar_type() == at::kBFloat16 &&
+                  w.scalar_type() == at::kBFloat16 && gu.scalar_type() == at::kBFloat16 && dy.device() == w.device() && dy.device() == gu.device(),
+              "gated_rows_backward: bf16 matrices on one GPU");
+  const int64_t M = dy.size(0);
+  if (dy.stride(1) != 1 || w.stride(1) != 1 || M == 0) return PyLong_FromLong(MVPA_ERR_UNSUPPORTED);
+  at::AutoDispatchBelowADInplaceOrView guard;
+  Tensor dgu = at::empty_like(gu);
+  const int st = mvpa_gated_rows_backward_bf16(dy.data_ptr(), w.data_ptr(), gu.data_ptr(), dgu.data_ptr(), M, w.size(1), dy.size(1),
+                                               dy.stride(0), w.stride(0), current_stream());
+  return st == MVPA_OK ? THPVariable_Wrap(dgu) : PyLong_FromLong(st);
+  END_HANDLE_TH_ERRORS
+}
+
 // as_operand, starting at a 16-byte boundary
 Tensor aligned_operand(const Tensor& t, at::ScalarType dt) {
   Tensor r = as_operand(t, dt);
@@ -916,6 +980,9 @@ PyMethodDef kMethods[] = {
     {"linear", (PyCFunction)(void*)py_linear, METH_FASTCALL, "x @ w^T in bf16"},
     {"linear_wgrad", (PyCFunction)(void*)py_linear_wgrad, METH_FASTCALL, "dy^T @ x in bf16"},
     {"linear_nn", (PyCFunction)(void*)py_linear_nn, METH_FASTCALL, "dy @ w in bf16"},
+    {"linear_nn2", (PyCFunction)(void*)py_linear_nn2, METH_FASTCALL, "dy @ [w0; w1] in bf16"},
+    {"gated_rows", (PyCFunction)(void*)py_gated_rows, METH_FASTCALL, "gate and up rows and silu(gate) * up"},
+    {"gated_rows_backward", (PyCFunction)(void*)py_gated_rows_backward, METH_FASTCALL, "the gradient of gate and up rows"},
     {"encode", (PyCFunction)(void*)py_encode, METH_FASTCALL, "db4 analysis + RMSNorm of signal rows"},
     {"mean_rows", (PyCFunction)py_mean_rows, METH_O, "means of groups of rows"},
     {"encode_saved", (PyCFunction)(void*)py_encode_saved, METH_FASTCALL, "encode, with what its backward needs"},

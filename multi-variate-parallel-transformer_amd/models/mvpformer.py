@@ -140,6 +140,9 @@ class GatedMLP(nn.Module):
     def forward(self, x):
         if torch.is_grad_enabled() and (x.requires_grad or self.training):
             wg, wu = self.gate_proj.weight, self.up_proj.weight
+            y = AG.gated_mlp(x, wg, wu, self.down_proj.weight)
+            if y is not None:
+                return y
             if x.is_cuda and x.dtype == torch.bfloat16 and wg.shape == wu.shape and wg.shape[0] % 8 == 0 and x.numel():
                 # frozen weights keep their stacked copy, others are stacked inside the graph
                 w = torch.cat([wg, wu], 0) if wg.requires_grad or wu.requires_grad else self._gate_up()

@@ -275,6 +275,61 @@ def gated_mid(x: torch.Tensor, w_gate_up: torch.Tensor) -> torch.Tensor:
     return _SiluGateFn.apply(linear(x, w_gate_up))
 
 
+class _GatedMLPFn(torch.autograd.Function):
+    """(silu(x @ wg^T) * (x @ wu^T)) @ wd^T for bf16 rows x [M, K]: the gate and up rows and their product come out of one
+    launch, and so do the gradients of gate and up with the product that the down projection's backward is."""
+
+    @staticmethod
+    def forward(ctx, x, wg, wu, wd):
+        gu, mid = mvpa_hip._taken(mvpa_hip.load_ext().gated_rows(x, wg, wu))
+        ctx.save_for_backward(x, wg, wu, wd, gu, mid)
+        return mvpa_hip.linear(mid, wd)
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, wg, wu, wd, gu, mid = ctx.saved_tensors
+        need_x, need_g, need_u, need_d = ctx.needs_input_grad
+        if torch.is_grad_enabled() or _mapped(dy):           # a backward that is differentiated itself, or mapped over
+            xf, g, u, d, df = x.float(), wg.float(), wu.float(), wd.float(), dy.float()
+            gate, up, dm = xf @ g.t().contiguous(), xf @ u.t().contiguous(), df @ d
+            s = torch.sigmoid(gate)
+            dg, du = dm * up * s * (1 + gate * (1 - s)), dm * gate * s
+            grads = (dg @ g + du @ u, dg.t().contiguous() @ xf, du.t().contiguous() @ xf, df.t().contiguous() @ (gate * s * up))
+            return tuple(a.to(b.dtype) if n else None for a, b, n in zip(grads, (x, wg, wu, wd), ctx.needs_input_grad))
+        ext, n = mvpa_hip.load_ext(), wg.shape[0]
+        dy = dy.contiguous()
+        dwd = _weight_gradient(dy, mid) if need_d else None
+        dx = dwg = dwu = None
+        if need_x or need_g or need_u:
+            if dy.data_ptr() % 16:
+                dy = dy.clone()
+            dgu = mvpa_hip._taken(ext.gated_rows_backward(dy, wd, gu))
+            if need_x:
+                if _dx_on_kernel(x.shape[0], x.shape[1], 2 * n):
+                    dx = mvpa_hip._taken(ext.linear_nn2(dgu, wg, wu))
+                else:
+                    dx = torch.matmul(dgu, torch.cat([wg, wu], 0))
+            if need_g or need_u:
+                dw = _weight_gradient(dgu, x)
+                dwg, dwu = dw[:n] if need_g else None, dw[n:] if need_u else None
+        return dx, dwg, dwu, dwd
+
+
+def gated_mlp(x: torch.Tensor, wg: torch.Tensor, wu: torch.Tensor, wd: torch.Tensor):
+    """wd applied to silu(x @ wg^T) * (x @ wu^T) with gradients, or None where the operands are not bf16 rows and weights in whole
+    blocks on the GPU, at least 512 rows of them."""
+    k, n, e = x.shape[-1], wg.shape[0], wd.shape[0]
+    if (not all(t.is_cuda and t.dtype == torch.bfloat16 and t.device == x.device for t in (x, wg, wu, wd)) or _mapped(x, wg, wu, wd)
+            or k % 64 or n % 64 or e % 64 or k < 128 or n < 128 or e < 128 or x.numel() < 512 * k
+            or max(k, n, e) > 1 << 20 or wg.shape != (n, k) or wu.shape != (n, k) or wd.shape != (e, n)
+            or not all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (wg, wu, wd))):
+        return None
+    rows = x.reshape(-1, k)
+    if not rows.is_contiguous() or rows.data_ptr() % 16:
+        rows = rows.clone(memory_format=torch.contiguous_format)
+    return _GatedMLPFn.apply(rows, wg, wu, wd).view(*x.shape[:-1], e)
+
+
 class _CosineStepsFn(torch.autograd.Function):
     """Cosine similarity of step t + 1 of nxt and step t of pred [B, T, C, E], one pass each way."""
 

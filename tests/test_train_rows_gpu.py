@@ -392,6 +392,60 @@ def test_operands_on_two_gpus_are_refused():
 
 # one wave a row and a workgroup a row, odd sizes of every level, rows at odd boundaries of 16 bytes (odd L); rows: one, fewer
 # than a wave's share, every group of rows and a remainder
+# tiles of 128 columns and 128, 192 and 256 rows, of 192 and 256 columns, whole and ragged each way; two blocks of a contraction and many
+@pytest.mark.parametrize("M,K,N,E", [(512, 128, 128, 128), (700, 192, 320, 192), (2600, 768, 1728, 768), (6400, 768, 1728, 768), (6001, 128, 832, 256),
+                                     (6300, 256, 704, 128), (16000, 128, 1728, 128), (13000, 128, 192, 1024), (20001, 192, 576, 192)])
+def test_gated_mlp(M, K, N, E):
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+
+    def rn(*s, std=1.0):
+        return (std * torch.randn(s, generator=g, device="cuda")).bfloat16()
+    x, wg, wu, wd = rn(M, K), rn(N, K, std=K ** -0.5), rn(N, K, std=K ** -0.5), rn(E, N, std=N ** -0.5)
+    x[0] *= 60                                                        # exp(-gate) overflows, underflows
+    dy, ext = rn(M, E), mvpa_hip.load_ext()
+    # the launches against the products by themselves, the same sums and roundings, and the gates in 64 bits
+    gu, mid = ext.gated_rows(x, wg, wu)
+    w = torch.cat([wg, wu], 0)
+    both = mvpa_hip.linear(x, w)
+    assert torch.equal(gu, both)
+    dgu = ext.gated_rows_backward(dy, wd, gu)
+    gate, up = (t.double() for t in gu.chunk(2, -1))
+    s, dm = torch.sigmoid(gate), ext.linear_nn(dy, wd).double()
+    _close(mid, gate * s * up)
+    _close(dgu, torch.cat([dm * up * s * (1 + gate * (1 - s)), dm * gate * s], -1))
+    # the passes by themselves round differently where the sigmoid's last bits decide
+    assert (mid != mvpa_hip.silu_gate(gu)).float().mean() <= 1e-3 and (dgu != mvpa_hip.silu_gate(gu, dm.bfloat16())).float().mean() <= 1e-3
+    assert torch.equal(ext.linear_nn2(dgu, wg, wu), ext.linear_nn(dgu, w))
+    # and the whole with its gradients against 64 bits, rounded where the pass rounds
+    leaves = [t.requires_grad_() for t in (x, wg, wu, wd)]
+    y = AG.gated_mlp(x.view(1, M, K), wg, wu, wd)
+    got = torch.autograd.grad(y, leaves, dy.view(1, M, E), retain_graph=True)
+    xd, gd, ud, dd = (t.detach().double() for t in leaves)
+    dm = dy.double() @ dd
+    dgate, dup = dm * up * s * (1 + gate * (1 - s)), dm * gate * s
+    want = dgate @ gd + dup @ ud, dgate.t() @ xd, dup.t() @ xd, dy.double().t() @ (gate * s * up)
+    assert (y[0].double() - (gate * s * up) @ dd.t()).norm() <= 4e-3 * y.double().norm()
+    for a, b in zip(got, want):
+        assert (a.double() - b).norm() <= 6e-3 * b.norm()             # one rounding of the operands, one of the result
+    if M < 3000:
+        again = torch.autograd.grad(y, leaves, dy.view(1, M, E), create_graph=True)
+        rows = torch.autograd.grad(y, leaves, torch.stack([dy, 2 * dy]).view(2, 1, M, E), is_grads_batched=True)
+        for a, r, b in zip(again, rows, want):
+            assert a.requires_grad and (a.double() - b).norm() <= 1e-2 * b.norm() and (r[1].double() - 2 * b).norm() <= 2e-2 * b.norm()
+    frozen = AG.gated_mlp(x.detach(), wg.detach(), wu, wd.detach())
+    assert torch.equal(torch.autograd.grad(frozen, wu, dy)[0], got[2])
+
+
+def test_gated_mlp_refuses():
+    def t(*s):
+        return torch.zeros(s, device="cuda", dtype=torch.bfloat16, requires_grad=True)
+    assert AG.gated_mlp(t(511, 128), t(128, 128), t(128, 128), t(128, 128)) is None
+    assert AG.gated_mlp(t(512, 96), t(128, 96), t(128, 96), t(128, 128)) is None
+    assert AG.gated_mlp(t(512, 128), t(136, 128), t(136, 128), t(128, 136)) is None
+    assert AG.gated_mlp(t(512, 128), t(128, 128), t(128, 128).float(), t(128, 128)) is None
+    assert AG.gated_mlp(t(512, 128), t(128, 256)[:, :128], t(128, 128), t(128, 128)) is None
+
+
 @pytest.mark.parametrize("L,M,wt", [(97, 1, torch.float32), (512, 131, torch.bfloat16), (1001, 33, torch.float32),
                                     (2560, 2051, torch.bfloat16), (4095, 65, torch.bfloat16),
                                     (16032, 3, torch.float32)])                  # (the longest in one pass)
