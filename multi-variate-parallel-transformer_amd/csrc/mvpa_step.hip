@@ -95,14 +95,17 @@ __global__ __launch_bounds__(512, 2) void mvpa_step_kernel(mvpa_fwd_args a, step
     koff[i] = (uint32_t)(rc * (int)a.k_stride_n + ((phys ^ swz_k<DH>(row)) << 3)) * 2;
     voff[i] = (uint32_t)(rc * (int)a.v_stride_n + ((phys ^ swz_v<DH>(row)) << 3)) * 2;
   }
-  auto issue = [&](int s, int stage) {
-    const bf16_t* ks = kbase + (int64_t)s * C_ * a.k_stride_n;
-    const bf16_t* vs = vbase + (int64_t)s * C_ * a.v_stride_n;
-    const uint32_t dst = lds0 + stage * G::STAGE;
-#pragma unroll
-    for (int i = 0; i < G::LPW; ++i) load_to_lds_16(ks, koff[i], dst + (wave + 8 * i) * 1024);
-#pragma unroll
-    for (int i = 0; i < G::LPW; ++i) load_to_lds_16(vs, voff[i], dst + G::TILE + (wave + 8 * i) * 1024);
+  const int64_t kstep = (int64_t)C_ * a.k_stride_n, vstep = (int64_t)C_ * a.v_stride_n;
+  const bf16_t *ks_next = kbase, *vs_next = vbase;               // of the step requested next
+  uint32_t dst = lds0 + (G::R - 1) * G::STAGE;
+  auto request = [&](int i) {                                     // 2 LPW of them are a step
+    if (i < G::LPW) load_to_lds_16(ks_next, koff[i < G::LPW ? i : 0], dst + (wave + 8 * i) * 1024);
+    else load_to_lds_16(vs_next, voff[i < G::LPW ? 0 : i - G::LPW], dst + G::TILE + (wave + 8 * (i - G::LPW)) * 1024);
+  };
+  auto next_step = [&]() {
+    ks_next += kstep;
+    vs_next += vstep;
+    dst = dst + G::STAGE == lds0 + G::RING ? lds0 : dst + G::STAGE;
   };
 
   // ---- tables
@@ -156,7 +159,9 @@ __global__ __launch_bounds__(512, 2) void mvpa_step_kernel(mvpa_fwd_args a, step
     kbits[t] = (uint32_t)__ballot(ok) >> (4 * hh);
   }
   lds_barrier();
-  issue(0, G::R - 1);                               // (everybody is done with the rows there)
+#pragma unroll
+  for (int i = 0; i < 2 * G::LPW; ++i) request(i);  // (everybody is done with the rows there)
+  next_step();
   f32x16 Bc[2];
 #pragma unroll
   for (int t = 0; t < 2; ++t)
@@ -190,16 +195,25 @@ __global__ __launch_bounds__(512, 2) void mvpa_step_kernel(mvpa_fwd_args a, step
     lds_barrier();
     const unsigned char* st_lds = sp_lds + stage * G::STAGE;
     stage = stage + 1 == G::R ? 0 : stage + 1;
-    if (s + 1 < steps) issue(s + 1, stage);
+    const bool more = s + 1 < steps;
     const float st = Stq[s * 32 + ln];
-    f32x16 S[2];
+    // The next step's requests go out one behind a product: together in front of them (64 KiB at the CU's one address unit, 1024
+    // cycles) every wave stood there first.  B1 H16 Hkv8 Dh128 with the merge, us: C100 T64 in 8 runs 28.4 -> 26.9, C128 T512 in 16
+    // 90.4 -> 86.5, T16 in 2 26.2 -> 24.5, T110 in 16 31.0 -> 30.6.
+    f32x16 S[2] = {Bc[0], Bc[1]};
+    x8 kf[4];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      S[t] = Bc[t];
+    for (int p = 0; p < 3; ++p) kf[p] = *(const x8*)(st_lds + k_lane[p >> 1] + (p & 1) * 32 * ROWB);
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        S[t] = E::mfma(*(const x8*)(st_lds + k_lane[ks] + t * 32 * ROWB), Qu[ks], S[t], 0, 0, 0);
+    for (int p = 0; p < 2 * KS; ++p) {
+      const int t = p & 1, ks = p >> 1;
+      if (p + 3 < 2 * KS) kf[(p + 3) & 3] = *(const x8*)(st_lds + k_lane[(p + 3) >> 1] + ((p + 3) & 1) * 32 * ROWB);
+      S[t] = E::mfma(kf[p & 3], Qu[ks], S[t], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more && p * 2 * G::LPW / (2 * KS) < (p + 1) * 2 * G::LPW / (2 * KS)) request(p * 2 * G::LPW / (2 * KS));
+      __builtin_amdgcn_sched_barrier(0);
     }
+    next_step();
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       float rmax = -INFINITY;
