@@ -34,6 +34,8 @@
 // the other sits at its barrier.
 #include "mvpa_mfma_tools.h"
 
+#include <type_traits>
+
 namespace mvpa {
 
 // NCT = key-channel tiles a WAVE handles per key step; KH = parts the keys of a step are split
@@ -891,7 +893,7 @@ __global__ __launch_bounds__(NW * 64, MINB) void mvpa_mfma_kernel(mvpa_fwd_args 
 
 // Combines the runs of a split last-step launch: out = sum_r 2^(lse_r - lse) o_r with
 // lse = log2 sum_r 2^lse_r.  DH/8 lanes per output row, 16 bytes each.
-template <int DH, typename E>
+template <int DH, typename E, int TOGETHER>
 __global__ __launch_bounds__(256) void mvpa_split_merge_kernel(mvpa_fwd_args a) {
   using x8 = typename E::x8;
   constexpr int LPR = DH / 8, RPB = 256 / LPR;         // lanes per row (8 elements each), rows per block
@@ -901,37 +903,42 @@ __global__ __launch_bounds__(256) void mvpa_split_merge_kernel(mvpa_fwd_args a) 
   if (row >= rows) return;
   const bf16_t* po = (const bf16_t*)a.split_ws;
   const float* plse = (const float*)(po + (int64_t)a.n_split * rows * DH);
-  // eight runs at a time, all of their loads in flight together (one run after the other: 16 runs took
-  // 10.5 us, the latency of 32 dependent round trips)
+  // TOGETHER runs at a time, all of their loads in flight together (one run after the other: 16 runs took
+  // 10.5 us, the latency of 32 dependent round trips; eight at a time 4.85)
   float m = -INFINITY, l = 0.f, acc[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) acc[i] = 0.f;
-  for (int r0 = 0; r0 < a.n_split; r0 += 8) {
-    float e[8];
-    x8 v[8];
+  for (int r0 = 0; r0 < a.n_split; r0 += TOGETHER) {
+    float e[TOGETHER];
+    x8 v[TOGETHER];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < TOGETHER; ++j) {
       const int64_t at = (int64_t)min(r0 + j, a.n_split - 1) * rows + row;
       e[j] = plse[at];
       v[j] = *(const x8*)(po + at * DH + 8 * sub);
     }
-    float mc = m;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (r0 + j >= a.n_split) e[j] = -INFINITY;
-      mc = fmaxf(mc, e[j]);
-    }
-    const float keep = fast_exp2(m - mc);
-    m = mc;
-    l *= keep;
+    for (int j0 = 0; j0 < TOGETHER; j0 += 8) {
+      if (j0 > 0 && r0 + j0 >= a.n_split) break;
+      float mc = m;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) acc[i] *= keep;
+      for (int j = j0; j < j0 + 8; ++j) {
+        if (r0 + j >= a.n_split) e[j] = -INFINITY;
+        mc = fmaxf(mc, e[j]);
+      }
+      const float keep = fast_exp2(m - mc);
+      m = mc;
+      l *= keep;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float w = fast_exp2(e[j] - m);
-      l += w;
+      for (int i = 0; i < 8; ++i) acc[i] *= keep;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] += w * (float)v[j][i];
+      for (int j = j0; j < j0 + 8; ++j) {
+        const float w = fast_exp2(e[j] - m);
+        l += w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) acc[i] += w * (float)v[j][i];
+      }
     }
   }
   const int bh = row / C_, cq = row % C_, b = bh / a.H, h = bh % a.H;
@@ -946,8 +953,11 @@ __global__ __launch_bounds__(256) void mvpa_split_merge_kernel(mvpa_fwd_args a) 
 template <typename E>
 static void launch_merge(const mvpa_fwd_args* a, hipStream_t stream) {
   const int rows = a->B * a->H * a->C, rpb = 2048 / a->Dh;
-  auto kern = a->Dh == 32 ? mvpa_split_merge_kernel<32, E> : a->Dh == 64 ? mvpa_split_merge_kernel<64, E>
-                                                                          : mvpa_split_merge_kernel<128, E>;
+  auto pick = [&](auto together) {
+    constexpr int N = decltype(together)::value;
+    return a->Dh == 32 ? mvpa_split_merge_kernel<32, E, N> : a->Dh == 64 ? mvpa_split_merge_kernel<64, E, N> : mvpa_split_merge_kernel<128, E, N>;
+  };
+  auto kern = a->n_split <= 8 ? pick(std::integral_constant<int, 8>()) : pick(std::integral_constant<int, 16>());
   MVPA_LAUNCH(kern, dim3((unsigned)((rows + rpb - 1) / rpb)), dim3(256), 0, stream, *a);
 }
 

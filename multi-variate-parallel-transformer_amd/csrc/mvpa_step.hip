@@ -12,11 +12,15 @@
 //   written over the other stages; step 0 goes into the last stage while the tables are gathered from.
 //   DH 128: two stages of 64 KB, DH 64: three of 32 KB.
 // Arithmetic, roundings and layouts as in mvpa_mfma.hip.
-// B1 H16 Hkv8 C128 T110 Dh128 in 16 runs: 43 -> 28 us without the merge; bound by the K and V rows on their
-// way from the L2 (115 MB: every query head reads its kv head's) and the set-up.
+// B1 H16 Hkv8 C128 T110 Dh128 in 16 runs: 43 -> 25 us without the merge, a chain: 2.5 to the rows, 6 of tables and the first step's way,
+// 1.8 a step (on 128 workgroups as on 256: products, exponentials and what lies between them, not memory), 4 of merge and stores.
 #include "mvpa_mfma_tools.h"
 
+#include <type_traits>
+
 namespace mvpa {
+
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 
 template <int DH>
 struct step_cfg {
@@ -26,7 +30,7 @@ struct step_cfg {
   static constexpr int R = TABLE / STAGE + 1;
   static constexpr int RING = R * STAGE;
   static constexpr int LPW = TILE / 1024 / 8;                     // 1 KiB loads per wave and tile
-  static_assert(4 * (2 + MT * 16) * 256 + 4 * 32 * (ROWB + 16) <= RING, "merge buffer and output rows");
+  static_assert(8 * (512 + MT * 2048 + 32 * (ROWB / 2 + 16)) <= RING, "merge buffer and output rows");
   static_assert(256 * ROWB <= STAGE, "q and channel-table rows fit a stage");
 };
 
@@ -251,44 +255,58 @@ __global__ __launch_bounds__(512, 2) void mvpa_step_kernel(mvpa_fwd_args a, step
     }
   }
 
-  // ---- the two halves of the keys
+  // ---- the two halves of the keys: each wave of a pair finishes half of the output columns (one of them all: 2.4 us)
+  constexpr int HALF = MT / 2;
   lds_barrier();
-  float* mb = (float*)sp_lds + qt * ((2 + MT * 16) * 64) + lane;
-  if (kp == 1) {
-    mb[0] = m_run;
-    mb[64] = l_run;
+  const int other = wave ^ 4;
+  float* ml = (float*)sp_lds + lane;                              // [wave][m | l][lane]
+  f32x4* give = (f32x4*)(sp_lds + 8 * 512) + lane;                // [wave][quad of the half][lane]
+  ml[wave * 128] = m_run;
+  ml[wave * 128 + 64] = l_run;
+  auto hand_over = [&](auto first) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) mb[(2 + mt * 16 + i) * 64] = acc[mt][i];
-  }
+    for (int q = 0; q < HALF * 4; ++q) {
+      const f32x16& v = acc[first() + q / 4];
+      give[(wave * HALF * 4 + q) * 64] = f32x4{v[q % 4 * 4], v[q % 4 * 4 + 1], v[q % 4 * 4 + 2], v[q % 4 * 4 + 3]};
+    }
+  };
+  if (kp == 0) hand_over(std::integral_constant<int, HALF>());
+  else hand_over(std::integral_constant<int, 0>());
   lds_barrier();
-  if (kp == 1) return;
-  const float m1 = mb[0], m = fmaxf(m_run, m1), a0 = fast_exp2(m_run - m), a1 = fast_exp2(m1 - m);
-  l_run = a0 * l_run + a1 * mb[64];
+  const float m1 = ml[other * 128], m = fmaxf(m_run, m1), a0 = fast_exp2(m_run - m), a1 = fast_exp2(m1 - m);
+  const float w0 = kp == 0 ? a0 : a1, w1 = kp == 0 ? a1 : a0;       // of the first half of the keys, of the second
+  const float l1 = ml[other * 128 + 64];
+  l_run = __builtin_fmaf(w0, kp == 0 ? l_run : l1, w1 * (kp == 0 ? l1 : l_run));
   const float ltot = l_run + __shfl_xor(l_run, 32);
   const float inv = 1.f / ltot;
-  // through LDS, so that whole rows leave
-  unsigned char* stg = sp_lds + 4 * (2 + MT * 16) * 256 + qt * (32 * (ROWB + 16));
+  // through LDS, so that whole halves of rows leave
+  constexpr int PITCH = HALF * 64 + 16, CPR = HALF * 4;
+  unsigned char* stg = sp_lds + 8 * (512 + HALF * 4 * 1024) + wave * (32 * PITCH);
+  auto finish = [&](auto first) {
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int a4 = 0; a4 < 4; ++a4) {
+    for (int q = 0; q < HALF * 4; ++q) {
+      const f32x16& v = acc[first() + q / 4];
+      const f32x4 o = give[(other * HALF * 4 + q) * 64];
       x4 w;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        w[r] = E::cvt((a0 * acc[mt][a4 * 4 + r] + a1 * mb[(2 + mt * 16 + a4 * 4 + r) * 64]) * inv);
-      *(x4*)(stg + ln * (ROWB + 16) + (mt * 32 + a4 * 8 + hh * 4) * 2) = w;
+      for (int r = 0; r < 4; ++r) {
+        const float own = v[q % 4 * 4 + r];
+        w[r] = E::cvt(__builtin_fmaf(w0, first() == 0 ? own : o[r], w1 * (first() == 0 ? o[r] : own)) * inv);
+      }
+      *(x4*)(stg + ln * PITCH + (q / 4 * 32 + q % 4 * 8 + hh * 4) * 2) = w;
     }
+  };
+  if (kp == 0) finish(std::integral_constant<int, 0>());
+  else finish(std::integral_constant<int, HALF>());
   wave_lds_sync();
   const int64_t prow0 = ((int64_t)run * nbh + bh) * C_;           // rows of the split workspace
 #pragma unroll
-  for (int i = 0; i < 32 * CHUNKS / 64; ++i) {
-    const int row = (i * 64 + lane) / CHUNKS, ch = (i * 64 + lane) % CHUNKS;
+  for (int i = 0; i < 32 * CPR / 64; ++i) {
+    const int row = (i * 64 + lane) / CPR, ch = (i * 64 + lane) % CPR;
     if (qt * 32 + row < C_)
-      *(u32x4*)((bf16_t*)a.split_ws + (prow0 + qt * 32 + row) * DH + ch * 8) = *(const u32x4*)(stg + row * (ROWB + 16) + ch * 16);
+      *(u32x4*)((bf16_t*)a.split_ws + (prow0 + qt * 32 + row) * DH + kp * HALF * 32 + ch * 8) = *(const u32x4*)(stg + row * PITCH + ch * 16);
   }
-  if (hh == 0 && cq < C_)
+  if (kp == 0 && hh == 0 && cq < C_)
     ((float*)((bf16_t*)a.split_ws + (int64_t)n_split * nbh * C_ * DH))[prow0 + cq] = m + log2f(ltot);
 }
 
