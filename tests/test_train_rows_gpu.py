@@ -323,6 +323,17 @@ def test_weight_gradient(m, n, k):
     _close(dw, dy.double().t() @ x.double(), m)
 
 
+# tiles of 256 x 128 and 128 x 256, one share and several; five blocks of rows a share, the last one whole, of one row, of all but one; ragged both ways
+@pytest.mark.parametrize("m,n,k", [(289, 2512, 1552), (290, 3400, 1512), (640, 2056, 1928), (1260, 3000, 272), (2623, 1392, 1576), (3009, 3456, 768),
+                                   (16001, 1280, 768)])
+def test_weight_gradient_on_wide_tiles(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    dy, x = (torch.randn((m, c + 8), generator=g, device="cuda").bfloat16()[:, :c] for c in (n, k))
+    want = dy.double().t() @ x.double()
+    for a, b in ((dy, x), (dy.contiguous(), x.contiguous())):
+        _close(mvpa_hip.load_ext().linear_wgrad(a, b), want, m)
+
+
 def test_weight_gradient_refuses_rows_off_16_bytes():
     x = torch.randn(64, 24, device="cuda").bfloat16()
     for dy in (x[:, 1:9], x[:, :12], x.t()):
@@ -390,8 +401,6 @@ def test_operands_on_two_gpus_are_refused():
         mvpa_hip.load_ext().linear_wgrad(here, there)
 
 
-# one wave a row and a workgroup a row, odd sizes of every level, rows at odd boundaries of 16 bytes (odd L); rows: one, fewer
-# than a wave's share, every group of rows and a remainder
 # tiles of 128 columns and 128, 192 and 256 rows, of 192 and 256 columns, whole and ragged each way; two blocks of a contraction and many
 @pytest.mark.parametrize("M,K,N,E", [(512, 128, 128, 128), (700, 192, 320, 192), (2600, 768, 1728, 768), (6400, 768, 1728, 768), (6001, 128, 832, 256),
                                      (6300, 256, 704, 128), (16000, 128, 1728, 128), (13000, 128, 192, 1024), (20001, 192, 576, 192)])
@@ -446,6 +455,8 @@ def test_gated_mlp_refuses():
     assert AG.gated_mlp(t(512, 128), t(128, 256)[:, :128], t(128, 128), t(128, 128)) is None
 
 
+# one wave a row and a workgroup a row, odd sizes of every level, rows at odd boundaries of 16 bytes (odd L); rows: one, fewer
+# than a wave's share, every group of rows and a remainder
 @pytest.mark.parametrize("L,M,wt", [(97, 1, torch.float32), (512, 131, torch.bfloat16), (1001, 33, torch.float32),
                                     (2560, 2051, torch.bfloat16), (4095, 65, torch.bfloat16),
                                     (16032, 3, torch.float32)])                  # (the longest in one pass)
