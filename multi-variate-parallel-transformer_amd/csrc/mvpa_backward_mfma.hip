@@ -796,13 +796,10 @@ __global__ __launch_bounds__((PHASE_WAVES<PHASE> * 64), (PHASE_OCC<DH, PHASE>)) 
     } else if (L < nbh) {
       bh = L;
       tile = nt - 1;
-    } else if ((nbh & 7) == 0) {
-      const int s = (L - nbh) >> 3;
-      bh = ((L - nbh) & 7) + 8 * (s / (nt - 1));
-      tile = nt - 2 - s % (nt - 1);
     } else {
-      bh = (L - nbh) / (nt - 1);
-      tile = nt - 2 - (L - nbh) % (nt - 1);
+      // (an XCD's first walk takes no turns; with / without: B1 H16/8 C64 T128 Dh128 1265 / 1247 us, B2 H16 C64 T64 Dh64 364 / 355)
+      deal_walks(L - nbh, nbh, nt - 1, DH == 64 ? 64 : 32, 1, bh, tile);
+      tile = nt - 2 - tile;
     }
   }
   if constexpr (LAST_APART<DH, NCT, PHASE>)
@@ -905,17 +902,7 @@ __global__ __launch_bounds__(KEY_WAVES * 64, DH == 64 ? 2 : 1) void mvpa_bwd_key
   // per_head: a workgroup takes one query head and dk, dv come per query head ([B,H,N,Dh])
   const int out_heads = per_head ? a.H : a.Hkv, nbg = a.B * out_heads, ntk = (T_ + KT - 1) / KT;
   int bg, tile;
-  {
-    const int L = blockIdx.x;
-    if ((nbg & 7) == 0) {
-      const int s = L >> 3;
-      bg = (L & 7) + 8 * (s / ntk);
-      tile = s % ntk;                             // early key steps (most queries) first
-    } else {
-      bg = L / ntk;
-      tile = L % ntk;
-    }
-  }
+  deal_walks(blockIdx.x, nbg, ntk, DH == 64 ? 64 : 32, 0, bg, tile);     // early key steps (most queries) first
   const int b = bg / out_heads, g = per_head ? bg % out_heads / (a.H / a.Hkv) : bg % out_heads;
   const int grp = per_head ? 1 : a.H / a.Hkv, h0 = per_head ? bg % out_heads : g * grp;
   const int tk0 = tile * KT;

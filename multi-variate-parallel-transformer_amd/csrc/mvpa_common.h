@@ -131,6 +131,26 @@ inline void want_dynamic_lds(const void* kern, int bytes) {
   (void)hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
 }
 
+// Workgroup L -> item i of walk w: n walks (the tiles of one (b, h), longest first) of nt items.  Ids equal mod 8 share an XCD and its L2: an XCD
+// takes whole walks, whose workgroups read the same rows at about the same time, one after the other; but the items of the last of them, as many
+// walks as fill the `slots` workgroups an XCD holds and one more, take turns, or a walk's longest would begin when all others end.  `alone`: of an XCD's
+// first walks, how many take no turns.  Walks that do not divide over the XCDs go first, longest items first, side by side: each stays on as few
+// XCDs as it can.  Forward and backward at Dh 64, us, walk by walk over all XCDs where they do not divide / this: B3 H12/4 C64 T64 622 / 439, T128
+// 1252 / 1078, B1 H12/4 C40 T200 1016 / 880, B3 H6 C64 T128 838 / 621; no turns / this: B4 H12/4 C64 T25 195 / 185, B4 H12/4 C100 T40 1191 / 1059.
+__host__ __device__ inline void deal_walks(int L, int n, int nt, int slots, int alone, int& w, int& i) {
+  const int rest = n & 7, spread = rest * nt;
+  if (L < spread) {
+    w = n - rest + L % rest;
+    i = L / rest;
+    return;
+  }
+  const int xcd = (L - spread) & 7, s = (L - spread) >> 3, per = n >> 3, most = min(1 + slots / nt, per - alone);
+  const int merged = max(most, 1), plain = (per - merged) * nt;
+  const int k = s < plain ? s / nt : per - merged + (s - plain) % merged;
+  i = s < plain ? s % nt : (s - plain) / merged;
+  w = xcd + 8 * k;
+}
+
 }  // namespace mvpa
 
 #define MVPA_LAUNCH(...) mvpa::note_launch(mvpa::launch(__VA_ARGS__))

@@ -258,8 +258,9 @@ template <int DH> __device__ inline int swz_v(int row) {
 //     stream the same K/V tiles at the same time;
 //   * the last two units are interleaved tile by tile, so that the grid does not end on the long
 //     tiles of a single unit.
-// Without XCD affinity to keep (the (b, h) do not divide over 8 XCDs): last tiles first, then
-// (b, h) by (b, h).
+// (b, h) that do not divide over the 8 XCDs come behind the last tiles, late tiles first, side by side, so that each stays on as few XCDs as
+// it can; the rest as above.  us, (b, h) by (b, h) over all XCDs / so: B3 H12/4 C64 T64 Dh64 118 / 85, C100
+// T128 860 / 750, B5 H4 C128 T16 Dh32 40.1 / 32.1.
 __host__ __device__ inline void map_block(int L, int nbh, int nt, int grp, int& bh, int& tile) {
   constexpr int TAIL_MERGE = 2;
   if (nt <= 1) {
@@ -267,24 +268,20 @@ __host__ __device__ inline void map_block(int L, int nbh, int nt, int grp, int& 
     tile = 0;
     return;
   }
-  if ((nbh & 7) != 0) {
-    if (L < nbh) {
-      bh = L;
-      tile = nt - 1;
-    } else {
-      bh = (L - nbh) / (nt - 1);
-      tile = nt - 2 - (L - nbh) % (nt - 1);
-    }
-    return;
-  }
-  const int per_xcd = nbh >> 3;
+  const int per_xcd = nbh >> 3, rest = nbh & 7, spread = rest * (nt - 1);
   if (L < nbh) {
-    bh = (L & 7) * per_xcd + (L >> 3);
+    bh = rest ? L : (L & 7) * per_xcd + (L >> 3);
     tile = nt - 1;
     return;
   }
-  const int L2 = L - nbh;
-  const int xcd = L2 & 7, s = L2 >> 3;
+  L -= nbh;
+  if (L < spread) {                              // (b, h) that do not divide over the XCDs
+    bh = nbh - rest + L % rest;
+    tile = nt - 2 - L / rest;
+    return;
+  }
+  L -= spread;
+  const int xcd = L & 7, s = L >> 3;
   const int u = (grp > 1 && per_xcd % grp == 0) ? grp : 1;      // heads per unit
   const int n_units = per_xcd / u, items = u * (nt - 1);
   const int merged = n_units < TAIL_MERGE ? n_units : TAIL_MERGE;

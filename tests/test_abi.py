@@ -229,6 +229,19 @@ def test_python_operator_errors():
         flashmvpa(q, b, b, b, kv, torch.zeros(1, 4, 4, 32), torch.zeros(1, 4, 3, 32), kv, True, 0.1)
 
 
+@pytest.mark.parametrize("nbh,grp,nt", [(36, 3, 33), (12, 3, 13), (9, 1, 2), (7, 1, 40), (4, 4, 26), (20, 1, 1), (15, 5, 64)])
+def test_block_order_of_pairs_that_do_not_divide_over_the_xcds(lib, nbh, grp, nt):
+    """Every (pair, tile) once, and behind the last tiles an XCD's share within two tiles and an eighth of the others'."""
+    import numpy as np
+    bh, tile = (np.full(nbh * nt, -1, dtype=np.int32) for _ in range(2))
+    assert lib.mvpa_debug_block_order(nbh, nt, grp, bh.ctypes.data, tile.ctypes.data) == 0
+    assert sorted(zip(bh.tolist(), tile.tolist())) == [(b, t) for b in range(nbh) for t in range(nt)]
+    if nt > 1:
+        assert set(tile[:nbh].tolist()) == {nt - 1}
+        late = [int((tile[nbh:][np.arange(nbh, nbh * nt) % 8 == x] + 1).sum()) for x in range(8)]
+        assert max(late) - min(late) <= max(late) / 8 + 2 * nt
+
+
 @pytest.mark.parametrize("status,falls_back", [(-5, True), (-7, True), (-8, True), (-1, False), (-10, False), (-12, False)])
 def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_back):
     """Operands the kernel does not take go to the general product; a launch that failed or a workspace that is too
