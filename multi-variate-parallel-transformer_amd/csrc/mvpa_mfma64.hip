@@ -465,12 +465,16 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
   const bf16_t* fv = vbase;
   int f_iss = 0;
   uint32_t iss_lds = ring_lds, cur_lds = ring_lds;       // (f0 = 0 unless the passes say otherwise)
-  auto issue_far = [&]() {
-#pragma unroll
-    for (int i = 0; i < LPW; ++i) load_to_lds_16(fv, v_off[i], iss_lds + (wave + NW * i) * 1024);
+  auto request_far = [&](int i) { load_to_lds_16(fv, v_off[i], iss_lds + (wave + NW * i) * 1024); };
+  auto next_far = [&]() {
     ++f_iss;
     fv = f_iss < n_far ? fv + vstep : fv;
     iss_lds = iss_lds + TILE_BYTES == ring_lds + RING_BYTES ? ring_lds : iss_lds + TILE_BYTES;
+  };
+  auto issue_far = [&]() {
+#pragma unroll
+    for (int i = 0; i < LPW; ++i) request_far(i);
+    next_far();
   };
   auto v_addr_at = [&](uint32_t base) {
     StageAddr sa;
@@ -575,7 +579,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
     for (int tk = tk0; tk < tk1; ++tk) {
       wait_vmcnt_imm<(FSLOTS - 2) * LPW>();
       lds_barrier();
-      issue_far();
+      if (tk > far_max) issue_far();
       const uint32_t now_lds = cur_lds;
       cur_lds = cur_lds + TILE_BYTES == ring_lds + RING_BYTES ? ring_lds : cur_lds + TILE_BYTES;
       if (tk <= far_max) {
@@ -586,6 +590,8 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
         // first and arrive under the previous step's accumulate for that tile; the fragments of
         // output tile 1 are requested next and arrive under the products of tile 0, between which
         // the accumulate for tile 1 is spread; the products of tile 1 close the step.
+        // The tile requests go out between those: behind the barrier a wave stood in line for the CU's address unit before its
+        // first fragment (B4 H16 C64 T128 375.6 -> 372.2 us, B4 H12 C50 T300 1081 -> 1075; four spilled registers gone).
         bf16x8 vf[MT][NCT * 2];
 #pragma unroll
         for (int t = 0; t < NCT; ++t)
@@ -618,14 +624,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
         for (int x = 0; x < 2; ++x)
 #pragma unroll
           for (int i = 0; i < 16; ++i) ptmp[x][1][i] = 0.f;
-#pragma unroll
-        for (int t = 0; t < NCT; ++t)
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-            for (int x = 0; x < 2; ++x)
-              ptmp[x][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][t * 2 + s2], qt[x].Ec[t][s2], ptmp[x][1], 0, 0, 0);
-        // 8 LDS reads, 32 FMAs, 8 LDS reads, then 8 x (1 MFMA + 4 FMAs), then 8 MFMAs
+        // 8 LDS reads, 32 FMAs, 8 LDS reads, then 8 x (1 MFMA + 4 FMAs), then 8 MFMAs and the requests
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 32, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
@@ -634,7 +633,18 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
           __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
         }
-        __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
+#pragma unroll
+        for (int c = 0; c < NCT * 2; ++c) {
+          if (c % (NCT * 2 / LPW) == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            request_far(c / (NCT * 2 / LPW));
+            __builtin_amdgcn_sched_barrier(0);
+          }
+#pragma unroll
+          for (int x = 0; x < 2; ++x)
+            ptmp[x][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][c], qt[x].Ec[c >> 1][c & 1], ptmp[x][1], 0, 0, 0);
+        }
+        next_far();
         pet[0] = fast_exp2(st0 + qt[0].mc - qt[0].m);
         qt[0].l += pet[0] * qt[0].sumEc;
         pet[1] = fast_exp2(st1 + qt[1].mc - qt[1].m);
