@@ -1465,10 +1465,9 @@ static void launch_key(const mvpa_bwd_args* a, const mvpa_kv_out& out, hipStream
 // gradients) and of disjoint query channels (to dk, dv) simply add up, so every (query part, key
 // part) pair is one query-pass launch followed by the key-pass launch that consumes its
 // workspace; later launches add to what earlier ones wrote (one stream, hence ordered).
-// At Dh 128 the key pass takes the (query part, key part) pair of a query-pass launch in quarters of 32 x 32
-// channels (the workspace is indexed by absolute channel, and its per-row maximum covers the whole key part).  That
-// was forced while a stage held two copies of each tile; with one, two channel tiles would fit as well (two stages 99 840
-// bytes, 195 .. 215 + 160 registers against 175 .. 181 + 160), which has not been measured.
+// A key-pass launch takes the (query part, key part) pair of a query-pass launch whole.  At Dh 128 it took quarters of 32 x 32 channels, a
+// launch each, whose waves had half the products between two barriers (forward and backward, H16/8, us, quarters / whole: B1 C64 T25 286 / 192,
+// B2 C64 T128 2228 / 2066, B1 C100 T40 1434 / 942, B1 C128 T128 4665 / 4195, T512 36.2 / 34.8 ms; three stages instead of two: the same).
 // far steps of the longest walk from which the two phases of the query pass are a launch each (Dh 128): the
 // set-up of a workgroup is paid twice.  Forward and backward, one launch / two, H16/8: B2 C128 T128 8.39 / 8.82 ms, B1
 // C128 T200 9.01 / 9.10, B2 C64 T256 6.40 / 6.37, B1 C128 T300 17.1 / 17.0, T 512 36.4 / 35.8.
@@ -1477,32 +1476,38 @@ template <int DH>
 static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per_head, const mvpa_kv_out* out) {
   using namespace mvpa::bwdq;
   const int C = a->C, T = a->T;
-  constexpr int KEY_CP = DH == 64 ? 64 : 32;      // channels per key-pass launch
   // Far query steps (outside the content window and not the last step) in a kernel of their own where its
-  // workgroups, of FAR_KT key steps (16 at Dh 64, 8 at Dh 128; 2 and 4 in the key pass), still fill the chip.  Forward and backward, far kernel / without:
+  // workgroups, of FAR_KT key steps (16 at Dh 64, 8 at Dh 128; 2 in the key pass), still fill the chip and its walks are long.  Forward and backward, far
+  // kernel / without:
   // Dh 64, C 64, T 128: 384 workgroups 1327 / 1495 us, 256: 962 / 1022, 192: 793 / 850, 128: 667 / 589; T 256 of 256:
   // 1480 / 1648; T 64, C 40 of 192: 495 / 495; T 64 of 48: 315 / 272;
-  // Dh 128, H16/8: B1 C64 T128, 256 workgroups, 1259 / 1453; C 128: T 128, 128 workgroups 5.77 / 6.15 ms.
+  // Dh 128, H16/8, C 64: T 64, 128 workgroups 502 / 453, T 72, 144: 613 / 571, T 80, 160: 688 / 660, T 90, 192: 766 / 780, T 64, 256: 840 / 876, T 128, 256:
+  // 1155 / 1289; walks of at most 13 steps (T 25), 256: 541 / 518, 18: 639 / 621, 22: 737 / 725, 28 (C 100): 3169 / 3242.
   constexpr int FAR_KT = FR * FAR_WAVES<DH> / 2;
   const int64_t far_groups = (int64_t)a->B * (per_head ? a->H : a->Hkv) * ((T + FAR_KT - 1) / FAR_KT);
-  const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= FAR_KT &&
-                   far_groups >= (DH == 64 ? 192 : 128);
+  const bool far = (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && C > 32 && T - 2 - a->window >= (DH == 64 ? 16 : 24) &&
+                   far_groups >= 192;
   const bool split_query = DH == 128 && (a->flags & MVPA_FLAG_CONTENT) && a->window > 0 && T - 2 - a->window >= SPLIT_STEPS;
-  auto key_launch = [&](auto near, int kk, int qq, int accum) {
+  auto key_launch = [&](auto near, auto tiles, int kk, int qq, int accum) {
     constexpr bool NEAR = decltype(near)::value;
-    const mvpa_kv_out to = out && qq + KEY_CP >= C ? *out : mvpa_kv_out{};        // the last query part rounds
-    const bool full = C - qq >= KEY_CP && C - kk >= KEY_CP;
-    if (full) launch_key<DH, KEY_CP / 32, false, NEAR>(a, to, stream, kk, qq, accum, per_head);
-    else launch_key<DH, KEY_CP / 32, true, NEAR>(a, to, stream, kk, qq, accum, per_head);
+    constexpr int NCT = decltype(tiles)::value, CP = NCT * 32;
+    const mvpa_kv_out to = out && qq + CP >= C ? *out : mvpa_kv_out{};        // the last query part rounds
+    const bool full = C - qq >= CP && C - kk >= CP;
+    if (full) launch_key<DH, NCT, false, NEAR>(a, to, stream, kk, qq, accum, per_head);
+    else launch_key<DH, NCT, true, NEAR>(a, to, stream, kk, qq, accum, per_head);
   };
-  auto key_launches = [&](int q0, int k0, int span, bool first_q) {
-    if (far) launch_far<DH>(a, stream, k0, q0, !first_q, per_head);
-    for (int kk = k0; kk < min(k0 + span, C); kk += KEY_CP)
-      for (int qq = q0; qq < min(q0 + span, C); qq += KEY_CP) {
-        const int accum = !(first_q && qq == q0);
-        if (far) key_launch(std::true_type{}, kk, qq, accum);
-        else key_launch(std::false_type{}, kk, qq, accum);
-      }
+  // Parts of up to 32 channels in tiles of 32, the existing ones alone; at Dh 64 where a launch on tiles of 64 is two rounds of two workgroups a CU.
+  // Tiles of 64 / of 32, us: Dh 128, H16/8 B3 C65 T77 5048 / 4708, B2 C96 T40 1574 / 1429, B1 C80 T25 556 / 578; Dh 64, 480 workgroups (B2 H12 C96
+  // T40) 684 / 698, 768 (B2 H12 C75 T64) 1009 / 1033, 960 (B4 H16 C65 T30) 805 / 772, 1200 (B1 H12 C90 T200) 3247 / 3074, 1404 (B3 H12 C65 T77) 1833 / 1645.
+  const bool by_32 = DH == 128 || (int64_t)a->B * (per_head ? a->H : a->Hkv) * ((T + 1) / 2) >= 900;
+  auto key_launches = [&](auto near, int q0, int k0, bool first_q) {
+    if (!by_32 || (C - q0 > 32 && C - k0 > 32)) {
+      key_launch(near, std::integral_constant<int, 2>{}, k0, q0, !first_q);
+      return;
+    }
+    for (int kk = k0; kk < min(k0 + 64, C); kk += 32)
+      for (int qq = q0; qq < min(q0 + 64, C); qq += 32)
+        key_launch(near, std::integral_constant<int, 1>{}, kk, qq, !(first_q && qq == q0));
   };
   if (C <= 32) {
     launch_query<DH, 1, ONE>(a, stream, 0, 0, 0);
@@ -1520,7 +1525,9 @@ static void launch_bwd_parts(const mvpa_bwd_args* a, hipStream_t stream, int per
           }
         }
         if (!split_query) launch_query<DH, 2, ONE>(a, stream, qp * 64, kp * 64, kp > 0);
-        key_launches(qp * 64, kp * 64, 64, qp == 0);
+        if (far) launch_far<DH>(a, stream, kp * 64, qp * 64, qp > 0, per_head);
+        if (far) key_launches(std::true_type{}, qp * 64, kp * 64, qp == 0);
+        else key_launches(std::false_type{}, qp * 64, kp * 64, qp == 0);
       }
   }
 }

@@ -597,12 +597,14 @@ static void row_split(const mvpa_bwd_args* b, int* n_split, int* len) {
 // as four key steps each) are less than two rounds of the chip, each query head gets its own, and finish_kv adds up their dk, dv.
 // Forward and backward without / with, us: B4 C64 T25 H12/4 (112 workgroups) 240 / 197, B1 C64 T64 (64) 405 / 275,
 // B4 C21 T100 (400) 490 / 425, B8 C32 T64 (512) 482 / 506, B32 C64 T25 (896) 1122 / 1215; Dh 128, H16/8: B1 C128 T128
-// (256) 5036 / 4582, B4 C128 T64 (512) 6245 / 6735, B1 C32 T192 (384) 952 / 972.
+// (256) 5036 / 4582, B1 C32 T192 (384) 952 / 972.
 // Long walks at Dh 64 gain up to twice as many, the far kernel's workgroups with them: B2 C64 T256 (512) 2331 / 2003,
 // B4 C40 T200 (800) 2845 / 2297, B4 C64 T256 (1024) 4670 / 3960, B8 C64 T128 (1024) 2800 / 2620, B16 C64 T64 (1024)
 // 2018 / 2008, B6 C64 T256 (1536) 5870 / 6010, B8 C64 T256 (2048) 7810 / 8200.
+// At Dh 128, H16/8, above 32 channels: B2 C64 T64 (256) 789 / 839, B8 C64 T25 (448) 873 / 954, B4 C40 T60 (480) 1296 / 1280; B2 C64 T100 (400) 1515 /
+// 1475, B2 C64 T128 (512) 2053 / 2002, B1 C64 T256 (512) 3446 / 3201, B3 C64 T128 (768) 2875 / 3007.
 static bool per_head(const mvpa_bwd_args* b) {
-  const int64_t full = b->Dh == 64 && b->C > 32 && b->T >= 64 ? 1280 : 512;
+  const int64_t full = b->C <= 32 ? 512 : b->Dh == 64 ? (b->T >= 64 ? 1280 : 512) : b->T >= 96 ? 640 : 256;
   return b->H > b->Hkv && (int64_t)b->B * b->Hkv * ((b->T + 3) / 4) < full;
 }
 

@@ -116,12 +116,12 @@ BF16_CASES = [
     dict(B=1, C=32, T=21, H=2, Hkv=1, Dh=64, window=3),       # one channel tile, four key steps per workgroup, GQA
     dict(B=2, C=20, T=40, H=2, Hkv=2, Dh=64, window=5),       # one ragged channel tile, two slabs
     dict(B=1, C=64, T=45, H=1, Hkv=1, Dh=64, window=2),       # odd T: the last key pair of a workgroup is half empty
-    # head dim 128: rows of 256 bytes in the LDS tiles, the key pass in quarters of 32 x 32 channels
+    # head dim 128: rows of 256 bytes in the LDS tiles
     dict(B=1, C=32, T=21, H=2, Hkv=1, Dh=128, window=3),      # one channel tile, GQA
     dict(B=2, C=20, T=40, H=2, Hkv=2, Dh=128, window=5),      # one ragged channel tile, two slabs
-    dict(B=1, C=64, T=12, H=2, Hkv=2, Dh=128, window=10),     # two channel tiles per query step, four key-pass launches
+    dict(B=1, C=64, T=12, H=2, Hkv=2, Dh=128, window=10),     # two channel tiles per query step
     dict(B=1, C=40, T=37, H=2, Hkv=1, Dh=128, window=10),     # ragged second tile, two slabs, GQA
-    dict(B=1, C=117, T=9, H=2, Hkv=1, Dh=128, window=2),      # two channel parts: 4 query-pass, 16 key-pass launches
+    dict(B=1, C=117, T=9, H=2, Hkv=1, Dh=128, window=2),      # two channel parts: 4 launches of either pass
     dict(B=1, C=128, T=6, H=1, Hkv=1, Dh=128, window=10),     # two full channel parts
     dict(B=2, C=65, T=35, H=2, Hkv=2, Dh=128, window=3),      # second part of one channel; two slabs
     dict(B=1, C=33, T=9, H=2, Hkv=2, Dh=128, window=0),       # content everywhere; odd C
@@ -458,7 +458,9 @@ def test_workgroups_per_query_head(B, C, T, H, Hkv):
 
 # (b, h) that do not divide over the XCDs, fewer than eight of them, just more, many; one tile, two, many; walks that take turns and ones that do not
 @pytest.mark.parametrize("B,C,T,H,Hkv,Dh", [(3, 40, 33, 3, 1, 64), (3, 64, 1, 5, 5, 64), (5, 20, 3, 2, 1, 64), (3, 33, 90, 12, 4, 64), (2, 20, 70, 9, 9, 64),
-                                            (3, 40, 20, 3, 3, 128), (6, 40, 26, 4, 4, 64), (5, 36, 140, 8, 8, 64)])
+                                            (3, 40, 20, 3, 3, 128), (6, 40, 26, 4, 4, 64), (5, 36, 140, 8, 8, 64),
+                                            # parts of up to 32 channels in tiles of 32 and (the samples alone) of 64, without the far kernel and with it
+                                            (6, 70, 24, 16, 16, 64), (8, 65, 60, 8, 8, 64), (2, 96, 52, 16, 8, 128), (2, 65, 20, 4, 2, 128)])
 def test_every_workgroup_of_a_batch(B, C, T, H, Hkv, Dh):
     """A batch against its samples one by one, which other kernels may serve, their workgroups dealt in another order.  Either rounds its
     probabilities to 8 bits at a reference of its own, so a (b, h) is compared by its norm, as the kernels are with the oracle; a tile of rows that no
