@@ -41,7 +41,8 @@ def _wgrad_on_kernel(m, n, k) -> bool:
     where many tiles meet many rows, earlier where rows do not start at lines of 128 bytes (rows times tiles in millions: [3456,768]
     10.6 410 / 541, [1536,2048] 25 1008 / 1024; [640,4000] 5.2 241 / 312, 10.5 478 / 428).  Long thin outputs are padding for the most
     part (25600 rows of [8,16000] 144 / 139).  The limits of tiles and of rows from 162 tiles on were drawn with a kernel that took up to a
-    fifth more (180 tiles 79 / 70, 225 80 / 73 over 6400 rows): they lie on the safe side."""
+    fifth more (180 tiles 79 / 70, 225 80 / 73 over 6400 rows): they lie on the safe side, and farther since tiles of 256 x 128 took the larger
+    problems ([3456,768] over 6400 rows 44, 25600 139; [768,1728] over 32768 111 -> 93)."""
     tiles = -(-n // 128) * -(-k // 128)
     if tiles > 170 or (min(n, k) < 64 and tiles > 96):
         return False
