@@ -77,6 +77,15 @@ template <> struct io<f16_t> {
 
 constexpr float kLog2e = 1.4426950408889634f;
 
+// silu(g) u and the gradients of g and u for the gradient d of that.  The passes by themselves and the products that end in them share these
+// lines and leave the same bits.
+__device__ inline float silu_gate(float g, float u) { return g / (1.f + expf(-g)) * u; }
+__device__ inline void silu_gate_gradients(float g, float u, float d, float& dg, float& du) {
+  const float s = 1.f / (1.f + expf(-g));
+  dg = d * u * (s * (1.f + g * (1.f - s)));
+  du = d * g * s;
+}
+
 }  // namespace mvpa
 
 // ---- launches ------------------------------------------------------------------------------

@@ -317,7 +317,7 @@ __global__ __launch_bounds__(256) void silu_gate_kernel(const bf16_t* __restrict
     load8(gu + row * 2 * n + c, g);
     load8(gu + row * 2 * n + n + c, u);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) g[j] = g[j] / (1.f + expf(-g[j])) * u[j];
+    for (int j = 0; j < 8; ++j) g[j] = silu_gate(g[j], u[j]);
     store8(out + row * n + c, g);
   }
 }
@@ -336,12 +336,7 @@ __global__ __launch_bounds__(256) void silu_gate_backward_kernel(const bf16_t* _
     load8(gu + row * 2 * n + n + c, u);
     load8(d + row * n + c, dv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float s = 1.f / (1.f + expf(-g[j]));
-      const float du = dv[j] * g[j] * s;
-      g[j] = dv[j] * u[j] * (s * (1.f + g[j] * (1.f - s)));
-      u[j] = du;
-    }
+    for (int j = 0; j < 8; ++j) silu_gate_gradients(g[j], u[j], dv[j], g[j], u[j]);
     store8(dgu + row * 2 * n + c, g);
     store8(dgu + row * 2 * n + n + c, u);
   }
