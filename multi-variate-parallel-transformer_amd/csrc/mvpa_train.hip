@@ -284,8 +284,9 @@ __global__ __launch_bounds__(256) void cosine_steps_backward_kernel(const bf16_t
   dot = wave_sum(dot);
   na = sqrtf(wave_sum(na));
   nb = sqrtf(wave_sum(nb));
-  const float ia = 1.f / fmaxf(na, eps), ib = 1.f / fmaxf(nb, eps), s = dot * ia * ib;
-  const float cross = g * ia * ib, ca = na > 0.f ? g * s * ia / na : 0.f, cb = nb > 0.f ? g * s * ib / nb : 0.f;
+  // comparisons that are false for a NaN, whose row's gradients are NaN throughout (fmaxf would give eps)
+  const float ia = 1.f / (na < eps ? eps : na), ib = 1.f / (nb < eps ? eps : nb), s = dot * ia * ib;
+  const float cross = g * ia * ib, ca = na == 0.f ? 0.f : g * s * ia / na, cb = nb == 0.f ? 0.f : g * s * ib / nb;
   for (int c = lane * 8; c < cols; c += 512) {
     float x[8], y[8], o[8];
     load8(ar + c, x);

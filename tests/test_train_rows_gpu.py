@@ -97,6 +97,26 @@ def test_generative_score_gradients(B, T, C, E):
     assert AG.cosine_steps(a[..., 4:], b[..., 4:]) is None and AG.cosine_steps(a[:, :1], b[:, :1]) is None
 
 
+@pytest.mark.parametrize("E", [8, 1032])
+def test_generative_score_gradients_of_rows_that_are_no_numbers(E):
+    """A NaN or an infinity in either row of a pair makes every gradient of both NaN, with a zero gradient of the score too, and
+    leaves the other pairs alone."""
+    g = torch.Generator(device="cuda").manual_seed(E)
+    a, b = (torch.randn((2, 4, 3, E), generator=g, device="cuda").bfloat16() for _ in range(2))
+    a[0, 1, 0, 5], b[0, 1, 1, E - 1], a[1, 3, 2, 0], b[1, 0, 0, 7] = float("nan"), float("nan"), float("inf"), -float("inf")
+    a[1, 2, 0, 3], a[0, 2, 2] = float("nan"), 0
+    a, b, d = a.requires_grad_(), b.requires_grad_(), torch.randn((2, 3, 3), generator=g, device="cuda")
+    d[1, 1, 0] = 0
+    ref = torch.cosine_similarity(a[:, 1:].float(), b[:, :-1].float(), dim=-1)
+    want = torch.autograd.grad(ref, (a, b), d)
+    s = AG.cosine_steps(a, b)
+    assert torch.equal(s.isnan(), ref.isnan()) and ref.isnan().sum() == 5
+    for graph in (False, True):
+        for x, w in zip(torch.autograd.grad(s, (a, b), d, retain_graph=True, create_graph=graph), want):
+            assert torch.equal(x.isnan(), w.isnan()) and w.isnan().sum() == 5 * E
+            assert ((x - w).float().nan_to_num().norm(dim=-1) <= 1e-2 * w.float().nan_to_num().norm(dim=-1)).all()
+
+
 @pytest.mark.parametrize("cols", [8, 768])
 def test_add3_norm_gradients(cols):
     """Gradients through both results, through one of them, and of a gradient (the tensor expressions)."""
