@@ -3,6 +3,7 @@ callers that cannot allocate device memory) against the same step through mvpa_f
 caller-allocated workspace: the same kernels on the same operands, so bit for bit - on two calls
 in a row, the second smaller, so that what the first left in the shared array is in the way."""
 import ctypes
+import gc
 
 import pytest
 import torch
@@ -92,10 +93,18 @@ def test_static_step_allocates_nothing_and_replays_in_a_graph():
     assert lib.mvpa_static_ws_init() == 0
     stream = torch.cuda.current_stream().cuda_stream
     torch.cuda.synchronize()
-    before = (torch.cuda.memory_allocated(), torch.cuda.memory_reserved())
-    assert lib.mvpa_forward_last_step_static(ctypes.byref(a), stream) == 0
-    torch.cuda.synchronize()
-    assert (torch.cuda.memory_allocated(), torch.cuda.memory_reserved()) == before
+    # the counters are the process's: tensors that earlier tests left in reference cycles (a module that holds a function that holds the
+    # module) go now, and none in between
+    gc.collect()
+    gc.disable()
+    try:
+        before = (torch.cuda.memory_allocated(), torch.cuda.memory_reserved())
+        status = lib.mvpa_forward_last_step_static(ctypes.byref(a), stream)
+        torch.cuda.synchronize()
+        after = (torch.cuda.memory_allocated(), torch.cuda.memory_reserved())
+    finally:
+        gc.enable()
+    assert status == 0 and after == before
     eager = out.clone()
 
     def caller_ws_step():
