@@ -291,6 +291,11 @@ int mvpa_select_kernel(const mvpa_fwd_args* args);
  * bh and tile hold n_bh * n_tiles entries.  Launches nothing. */
 int mvpa_debug_block_order(int32_t n_bh, int32_t n_tiles, int32_t heads_per_kv, int32_t* bh, int32_t* tile);
 
+/* Host-only: the same for the backward.  Workgroup L of n_walks walks of n_items each (the tiles of one (batch, head), longest
+ * first) takes item[L] of walk[L]; slots: workgroups an XCD holds at a time; alone: of an XCD's first walks, how many
+ * take no turns with others.  walk and item hold n_walks * n_items entries.  Launches nothing. */
+int mvpa_debug_walk_order(int32_t n_walks, int32_t n_items, int32_t slots, int32_t alone, int32_t* walk, int32_t* item);
+
 /*
  * Index/mask maps exactly as the kernels compute them, for bit-exact tests against
  * layers/mvpa.py:127-159 (shifts) and :230-264 (window and causal masks).

@@ -99,6 +99,19 @@ extern "C" int mvpa_debug_block_order(int32_t n_bh, int32_t n_tiles, int32_t hea
   return MVPA_OK;
 }
 
+extern "C" int mvpa_debug_walk_order(int32_t n_walks, int32_t n_items, int32_t slots, int32_t alone, int32_t* walk,
+                                     int32_t* item) {
+  if (!walk || !item) return MVPA_ERR_NULL;
+  if (n_walks <= 0 || n_items <= 0 || slots <= 0 || alone < 0) return MVPA_ERR_SHAPE;
+  for (int L = 0; L < n_walks * n_items; ++L) {
+    int w, i;
+    mvpa::deal_walks(L, n_walks, n_items, slots, alone, w, i);
+    walk[L] = w;
+    item[L] = i;
+  }
+  return MVPA_OK;
+}
+
 extern "C" int mvpa_select_kernel(const mvpa_fwd_args* a) {
   const int st = mvpa_validate(a);
   if (st != MVPA_OK) return st;

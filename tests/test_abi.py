@@ -242,6 +242,32 @@ def test_block_order_of_pairs_that_do_not_divide_over_the_xcds(lib, nbh, grp, nt
         assert max(late) - min(late) <= max(late) / 8 + 2 * nt
 
 
+@pytest.mark.parametrize("slots,alone", [(64, 0), (64, 1), (32, 0), (32, 1)])
+def test_walk_order_of_the_backward(lib, slots, alone):
+    """Every (walk, item) once; a walk that divides over the XCDs stays on one, its items in order, and so do those side by side
+    in front; an XCD's walks one after the other but for the last, which take turns; XCDs get alike."""
+    import numpy as np
+    for n in (*range(1, 26), 36, 64, 67, 100, 193):
+        for nt in (1, 2, 3, 13, 63, 64, 65, 150):
+            walk, item = (np.full(n * nt, -1, dtype=np.int32) for _ in range(2))
+            assert lib.mvpa_debug_walk_order(n, nt, slots, alone, walk.ctypes.data, item.ctypes.data) == 0
+            assert (np.sort(walk.astype(np.int64) * nt + item) == np.arange(n * nt)).all(), (n, nt)
+            rest, per = n % 8, n // 8
+            head = rest * nt
+            assert (walk[:head] >= n - rest).all() and (np.diff(item[:head]) >= 0).all()
+            merged = max(min(1 + slots // nt, per - alone), 1)
+            for x in range(8):
+                w, i = walk[head:][x::8], item[head:][x::8]
+                assert len(w) == per * nt and (w % 8 == x).all()
+                if per:
+                    plain = (per - merged) * nt
+                    assert (np.diff(w[:plain]) >= 0).all() and (np.diff(i[plain:]) >= 0).all()
+                    assert all((np.diff(i[w == k]) == 1).all() for k in np.unique(w))
+    out = np.zeros(8, dtype=np.int32)
+    assert lib.mvpa_debug_walk_order(8, 1, 64, 0, None, out.ctypes.data) == -1
+    assert lib.mvpa_debug_walk_order(0, 1, 64, 0, out.ctypes.data, out.ctypes.data) < 0
+
+
 @pytest.mark.parametrize("status,falls_back", [(-5, True), (-7, True), (-8, True), (-1, False), (-10, False), (-12, False)])
 def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_back):
     """Operands the kernel does not take go to the general product; a launch that failed or a workspace that is too
