@@ -384,7 +384,10 @@ static int tiles_of(int64_t N, int64_t K) { return (int)((N + TILE - 1) / TILE *
 // turn, us (vendor library): [3456,768] 53 (73), [768,1728] 32 (49), [1280,768] 26 (42), [768,768] 22 (39).  Pairs of groups
 // took 6 to 8 us off the last three.  ([3456,768] over 5120 rows 42.7 -> 46.5 us when blocks became 32 rows, 43.1 with these costs; 64 rows of
 // [768,768] 7.65 -> 8.8 -> 7.75.)  The wide tiles: 0.64 us a block of 64 rows and 1 a round more; of 65 shapes from 570 to 32768 rows
-// the plan chosen is 0.2 % behind the faster of the best plan on either tile (one 13 %: [240,2032] over 17880 rows, 37.5 / 33.0).
+// the plan chosen is 0.2 % behind the faster of the best plan on either tile (one 13 %: [240,2032] over 17880 rows, 37.5 / 33.0).  They are taken where
+// that is a hundredth less, and of fewer than 128 columns on either side, whose tile is padding for the most part and which it flatters, a sixth less.  us, tiles
+// of 128 x 128 / wide (what it says of them): [1728,8] over 33004 rows 28.3 / 31.0 (0.93), [24,3456] 15715 28.8 / 30.9 (0.87), [3456,32] 6150 15.3 / 16.1 (0.97),
+// [1280,136] 16951 21.9 / 22.6 (1.00), [2624,8] 26490 33.0 / 33.2 (0.85); [5632,16] 12564 34.9 / 32.9 (0.83), [4096,24] 36759 62.2 / 56.9 (0.79).
 struct plan {
   int groups, splits;
   int tn, tk;                                    // of the wide kernel; 0: tiles of 128 x 128
@@ -405,6 +408,7 @@ static plan plan_of(int64_t M, int64_t N, int64_t K) {
       }
     }
   const int64_t wblocks = (M + WKB - 1) / WKB;
+  best_us *= N < 128 || K < 128 ? 0.84 : 0.99;
   for (int t = 0; t < 2; ++t) {
     const int tn = t ? 128 : 256, tk = t ? 256 : 128;
     const int64_t wtiles = (N + tn - 1) / tn * ((K + tk - 1) / tk);

@@ -268,6 +268,13 @@ def test_walk_order_of_the_backward(lib, slots, alone):
     assert lib.mvpa_debug_walk_order(0, 1, 64, 0, out.ctypes.data, out.ctypes.data) < 0
 
 
+@pytest.mark.parametrize("M,N,K,splits", [(33004, 1728, 8, 18), (15715, 24, 3456, 18), (6150, 3456, 32, 9), (16951, 1280, 136, 12), (36807, 256, 2624, 12),
+                                          (37120, 512, 4032, 4)])
+def test_weight_gradients_of_few_columns_stay_on_small_tiles(lib, M, N, K, splits):
+    """The shares of the rows, by the workspace: those of the tiles of 128 x 128 for thin outputs, of the wide ones for the last two."""
+    assert lib.mvpa_linear_wgrad_ws_bytes(M, N, K) == splits * N * K * 4
+
+
 @pytest.mark.parametrize("status,falls_back", [(-5, True), (-7, True), (-8, True), (-1, False), (-10, False), (-12, False)])
 def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_back):
     """Operands the kernel does not take go to the general product; a launch that failed or a workspace that is too
