@@ -75,8 +75,14 @@ def _dx_on_kernel(m, n, k) -> bool:
                 [5632,.]   600 rows (220) 20.4 / 24.6, 1600 41.2 / 39.7, 6400 129 / 158
         k 3456  [768,.]    1024 rows (48) 23.7 / 19.9, 1600 (78) 23.8 / 23.6, 4096 29 / 41, 6400 39.9 / 40.7
         k 4096  [1024,.]   1024 rows (64) 27.4 / 23.3, 1600 (104) 27.7 / 32.0, 6400 57 / 61, 9000 83 / 80, 20000 166 / 156
-        k 11264 [2048,.]   600 rows (80) 79 / 90, 1024 (128) 91 / 87, 6400 250 / 361"""
-    return m >= 512 and (k <= 512 or -(-m // 128) * -(-n // 128) >= 72)
+        k 11264 [2048,.]   600 rows (80) 79 / 90, 1024 (128) 91 / 87, 6400 250 / 361
+    Up to 191 columns are a tile or two across, half empty: few rows of them, and long contractions, are the vendor library's ([16,.] k 192 6920 rows
+    5.2 / 4.5; [48,.] k 512 1330 6.9 / 5.7; [8,.] k 5632 13209 43 / 29, [152,.] k 3456 4517 23.9 / 19.7, 104 15888 37 / 32; taken: [160,.] k 384 10902
+    6.8 / 11.1, [104,.] k 1728 25571 23 / 39).  Of 240 shapes of 192 columns or more that the rule takes, 0.79 of the vendor's time on average, 11 are
+    slower, by 1 to 6 % and at no size in particular (k 2048 [512,.] 18785 rows 44.8 / 43.0, k 3456 [704,.] 1869 23.2 / 21.9): the vendor library picks
+    another tile there."""
+    tiles = -(-m // 128) * -(-n // 128)
+    return m >= 512 and (k <= 512 or tiles >= 72) and (n >= 192 or (tiles >= 72 and k <= 2048))
 
 
 def _input_gradient(dy, w):

@@ -275,6 +275,14 @@ def test_weight_gradients_of_few_columns_stay_on_small_tiles(lib, M, N, K, split
     assert lib.mvpa_linear_wgrad_ws_bytes(M, N, K) == splits * N * K * 4
 
 
+def test_input_gradients_of_few_columns_go_to_the_vendor_library():
+    from mvpa_hip import autograd as AG
+    for m, n, k in [(13209, 8, 5632), (4517, 152, 3456), (1330, 48, 512), (6920, 16, 192), (511, 768, 768), (1024, 768, 1280)]:
+        assert not AG._dx_on_kernel(m, n, k), (m, n, k)
+    for m, n, k in [(6400, 768, 3456), (10902, 160, 384), (25571, 104, 1728), (600, 640, 192), (600, 2048, 11264)]:
+        assert AG._dx_on_kernel(m, n, k), (m, n, k)
+
+
 @pytest.mark.parametrize("status,falls_back", [(-5, True), (-7, True), (-8, True), (-1, False), (-10, False), (-12, False)])
 def test_a_weight_gradient_that_fails_is_an_error(monkeypatch, status, falls_back):
     """Operands the kernel does not take go to the general product; a launch that failed or a workspace that is too
