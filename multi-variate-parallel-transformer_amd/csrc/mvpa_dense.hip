@@ -476,7 +476,7 @@ __device__ inline void tile_of_workgroup(int64_t L, int64_t mt64, int64_t nt64, 
 //   EPI 4  the product is the gradient of silu(gate) * up: the rows of gate and up that the forward stored are requested in front of
 //          the staging, and their gradients leave in its place.
 // The values are those of the passes by themselves (silu_gate_kernel, silu_gate_backward_kernel), which would read again what was just
-// written: expf and a division, of which the one wave of two on a SIMD has nobody to hide the forty instructions.  [3456,768] over 6400 rows 50 us, 44 with
+// written: expf and a division, of which the one wave of two on a SIMD has nobody to hide the forty instructions.  [3456,768] over 6400 rows 48 - 50 us, 44 with
 // the hardware's exponential and reciprocal alone, whose sigmoid is up to 60 ulp off where the gate is far below zero.
 struct gated_rows {
   const bf16_t* gu;        // [M][2 N], gate then up; what EPI 3 stores is y
@@ -1011,6 +1011,8 @@ static int launch_ring(const bf16_t* x, const bf16_t* w, bf16_t* y, int64_t M, i
 // waves send).  us, two stages and requests together / spread / by four waves / three stages of x: [3456,768] over 16384
 // rows 99 / 95 / 92 / 89, [768,2496] 62 / 62 / 59 / 52, [2048,2048] over 65536 486 / 470 / 446 / 433, [2048,7680] 1650 / 1605 / 1518 /
 // 1480, 8192^3 850 / 820 / 780 / 785; 128 columns, over 6400 rows [768,768] 14.3 / 12.0, [768,1728] 26.2 / 22.2, [768,3456] 46.3 / 36.
+// Another card, first / last: 97 / 93, 62 / 55, 487 / 443, 1662 / 1506, 860 / 788.  It is a wait that goes: of whole models, on cards whose clock follows
+// power, between nothing and 3.5 % is left of it.
 // Same tile order, roles, row mapping and epilogues as the other large-tile kernels.
 // Tiles of 128 columns have 256 rows or fewer (pair_tile_rows): waves of 64 x 64 outputs four by two, of 96 x 32 or 64 x 32 two by four.
 // -----------------------------------------------------------------------------------------

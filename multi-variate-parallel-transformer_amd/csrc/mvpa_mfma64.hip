@@ -591,7 +591,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mvpa_mfma64_kernel(mvpa_fwd_args a
         // output tile 1 are requested next and arrive under the products of tile 0, between which
         // the accumulate for tile 1 is spread; the products of tile 1 close the step.
         // The tile requests go out between those: behind the barrier a wave stood in line for the CU's address unit before its
-        // first fragment (B4 H16 C64 T128 375.6 -> 372.2 us, B4 H12 C50 T300 1081 -> 1075; four spilled registers gone).
+        // first fragment (B4 H16 C64 T128 375.6 -> 372.2 us, other cards 393 -> 390 and 395 -> 394, B4 H12 C50 T300 1081 -> 1075; four spilled registers gone).
         bf16x8 vf[MT][NCT * 2];
 #pragma unroll
         for (int t = 0; t < NCT; ++t)

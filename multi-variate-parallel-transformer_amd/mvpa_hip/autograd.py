@@ -79,7 +79,7 @@ def _dx_on_kernel(m, n, k) -> bool:
     Up to 191 columns are a tile or two across, half empty: few rows of them, and long contractions, are the vendor library's ([16,.] k 192 6920 rows
     5.2 / 4.5; [48,.] k 512 1330 6.9 / 5.7; [8,.] k 5632 13209 43 / 29, [152,.] k 3456 4517 23.9 / 19.7, 104 15888 37 / 32; taken: [160,.] k 384 10902
     6.8 / 11.1, [104,.] k 1728 25571 23 / 39).  Of 240 shapes of 192 columns or more that the rule takes, 0.79 of the vendor's time on average, 11 are
-    slower, by 1 to 6 % and at no size in particular (k 2048 [512,.] 18785 rows 44.8 / 43.0, k 3456 [704,.] 1869 23.2 / 21.9): the vendor library picks
+    slower, by 1 to 8 % and at no size in particular (k 2048 [512,.] 18785 rows 44.8 / 43.0, k 576 [320,.] 3010 7.6 / 7.0): the vendor library picks
     another tile there."""
     tiles = -(-m // 128) * -(-n // 128)
     return m >= 512 and (k <= 512 or tiles >= 72) and (n >= 192 or (tiles >= 72 and k <= 2048))
