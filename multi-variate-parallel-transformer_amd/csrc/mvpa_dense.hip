@@ -1573,9 +1573,22 @@ __global__ __launch_bounds__(256) void cosine_rows_bf16_kernel(const bf16_t* __r
     }
   }
   dot = wave_sum(dot);
-  na = wave_sum(na);
-  nb = wave_sum(nb);
-  if (lane == 0) out[row] = dot / (fmaxf(sqrtf(na), eps) * fmaxf(sqrtf(nb), eps));
+  na = sqrtf(wave_sum(na));
+  nb = sqrtf(wave_sum(nb));
+  float s = dot / (fmaxf(na, eps) * fmaxf(nb, eps));
+  if (na == INFINITY || nb == INFINITY) {       // squares past the type, a.b perhaps too: elements are divided first, infinite ones leave a NaN
+    const float ia = 1.f / fmaxf(na, eps), ib = 1.f / fmaxf(nb, eps);
+    s = 0.f;
+    for (int c = lane * 8; c < cols; c += 512) {
+      float x[8], y[8];
+      vec8<bf16_t>::load(ar + c, x);
+      vec8<bf16_t>::load(br + c, y);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += (x[i] * ia) * (y[i] * ib);
+    }
+    s = wave_sum(s);
+  }
+  if (lane == 0) out[row] = s;
 }
 
 // sum = bf16(a + b + c) and norm = RMSNorm(sum) * w in one pass over the three inputs: the

@@ -285,7 +285,19 @@ __global__ __launch_bounds__(256) void cosine_steps_backward_kernel(const bf16_t
   na = sqrtf(wave_sum(na));
   nb = sqrtf(wave_sum(nb));
   // comparisons that are false for a NaN, whose row's gradients are NaN throughout (fmaxf would give eps)
-  const float ia = 1.f / (na < eps ? eps : na), ib = 1.f / (nb < eps ? eps : nb), s = dot * ia * ib;
+  const float ia = 1.f / (na < eps ? eps : na), ib = 1.f / (nb < eps ? eps : nb);
+  float s = dot * ia * ib;
+  if (na == INFINITY || nb == INFINITY) {       // as the forward has it: the elements are divided first
+    s = 0.f;
+    for (int c = lane * 8; c < cols; c += 512) {
+      float x[8], y[8];
+      load8(ar + c, x);
+      load8(br + c, y);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s += (x[i] * ia) * (y[i] * ib);
+    }
+    s = wave_sum(s);
+  }
   const float cross = g * ia * ib, ca = na == 0.f ? 0.f : g * s * ia / na, cb = nb == 0.f ? 0.f : g * s * ib / nb;
   for (int c = lane * 8; c < cols; c += 512) {
     float x[8], y[8], o[8];

@@ -355,7 +355,7 @@ class _CosineStepsFn(torch.autograd.Function):
         a, b, d = nxt[:, 1:].float(), pred[:, :-1].float(), d[..., None]
         na, nb = a.norm(dim=-1, keepdim=True), b.norm(dim=-1, keepdim=True)
         ia, ib = 1 / na.clamp_min(ctx.eps), 1 / nb.clamp_min(ctx.eps)
-        s, tiny = (a * b).sum(-1, keepdim=True) * ia * ib, torch.finfo(torch.float32).tiny
+        s, tiny = ((a * ia) * (b * ib)).sum(-1, keepdim=True), torch.finfo(torch.float32).tiny
         da = d * (b * ia * ib - a * s * ia / na.clamp_min(tiny))
         db = d * (a * ia * ib - b * s * ib / nb.clamp_min(tiny))
         pad = torch.nn.functional.pad

@@ -99,18 +99,21 @@ def test_generative_score_gradients(B, T, C, E):
 
 @pytest.mark.parametrize("E", [8, 1032])
 def test_generative_score_gradients_of_rows_that_are_no_numbers(E):
-    """A NaN or an infinity in either row of a pair makes every gradient of both NaN, with a zero gradient of the score too, and
-    leaves the other pairs alone."""
+    """A NaN or an infinity in either row of a pair makes every gradient of both NaN, with a zero gradient of the score too; finite
+    elements whose squares are past the type give a score and gradients of zero; the other pairs are left alone."""
     g = torch.Generator(device="cuda").manual_seed(E)
     a, b = (torch.randn((2, 4, 3, E), generator=g, device="cuda").bfloat16() for _ in range(2))
     a[0, 1, 0, 5], b[0, 1, 1, E - 1], a[1, 3, 2, 0], b[1, 0, 0, 7] = float("nan"), float("nan"), float("inf"), -float("inf")
     a[1, 2, 0, 3], a[0, 2, 2] = float("nan"), 0
+    # squares past fp32, with a.b past it and within: no similarity and no gradients, but numbers
+    a[0, 3, 1, 4], b[0, 2, 1, 4], b[0, 2, 0, 6], a[1, 2, 1], b[1, 1, 1] = 3e38, 2, -2e19, 1e38, -1e30
     a, b, d = a.requires_grad_(), b.requires_grad_(), torch.randn((2, 3, 3), generator=g, device="cuda")
     d[1, 1, 0] = 0
     ref = torch.cosine_similarity(a[:, 1:].float(), b[:, :-1].float(), dim=-1)
     want = torch.autograd.grad(ref, (a, b), d)
     s = AG.cosine_steps(a, b)
     assert torch.equal(s.isnan(), ref.isnan()) and ref.isnan().sum() == 5
+    assert ((s - ref).abs() <= 1e-5).logical_or(ref.isnan()).all()
     for graph in (False, True):
         for x, w in zip(torch.autograd.grad(s, (a, b), d, retain_graph=True, create_graph=graph), want):
             assert torch.equal(x.isnan(), w.isnan()) and w.isnan().sum() == 5 * E
